@@ -118,6 +118,10 @@ int edge_sm_glu_gelu(const void* u, int ld, void* y, int rows, int ff, int f32, 
 int edge_sm_moe_route_grouped(const void* h, int W, const float* router, int E, int gate, const float* corr, int groups,
                               int keep, int top, float scale, float* z, int* idx, float* wts, float* gate_w, int rows, int f32,
                               hipStream_t st);
+int64_t edge_sm_moe_gemm_ints(int64_t R, int E);
+int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff);
+int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void* w_down, int* ints, void* y, void* out, int T,
+                     int top, int E, int W, int ff, int act, const float* row_w, float limit, hipStream_t st);
 int edge_sm_moe_experts_relu2(const void* h, int W, const int* idx, int top, const void* w_up, const void* w_down, int ff,
                               const void* su, const void* sd, int sff, void* y, void* ys, void* out, void* out_sh, int rows,
                               int E, int f32, hipStream_t st);
@@ -1044,6 +1048,40 @@ at::Tensor sm_glu_gelu(const at::Tensor& u, int64_t ff) {
   return y;
 }
 
+// Whether the MFMA form of prompt-sized expert steps takes these tensors: bf16, dense 16-byte aligned rows, whole
+// 64-wide k steps.
+bool sm_moe_gemm_ok(const at::Tensor& h, const at::Tensor& idx, const at::Tensor& w_gu, const at::Tensor& w_down, int64_t act,
+                    const std::optional<at::Tensor>& in_w) {
+  if (!h.is_cuda() || h.dim() != 2 || idx.dim() != 2 || w_gu.dim() != 3 || w_down.dim() != 3 || act < 1 || act > 3) return false;
+  for (const at::Tensor* t : {&h, &w_gu, &w_down})
+    if (t->scalar_type() != at::kBFloat16 || t->device() != h.device() || !t->is_contiguous() ||
+        reinterpret_cast<uintptr_t>(t->data_ptr()) % 16 != 0)
+      return false;
+  const int64_t T = h.size(0), W = h.size(1), E = w_gu.size(0), ff = w_down.size(2);
+  if (idx.scalar_type() != at::kInt || !idx.is_contiguous() || idx.device() != h.device() || idx.size(0) != T ||
+      w_gu.size(2) != W || w_gu.size(1) != (act == 3 ? ff : 2 * ff) || w_down.size(0) != E || w_down.size(1) != W)
+    return false;
+  if (in_w && (in_w->scalar_type() != at::kFloat || !in_w->is_contiguous() || in_w->device() != h.device() ||
+               in_w->numel() != idx.numel()))
+    return false;
+  return edge_sm_moe_gemm_ok(T, (int)idx.size(1), (int)E, (int)W, (int)ff) == 0;
+}
+
+// act 1: clamped gated unit, 2: silu-gated unit (in_w: a weight per choice on the unit's input), 3: squared ReLU
+at::Tensor sm_moe_gemm(const at::Tensor& h, const at::Tensor& idx, const at::Tensor& w_gu, const at::Tensor& w_down, int64_t act,
+                       double limit, const std::optional<at::Tensor>& in_w) {
+  TORCH_CHECK(sm_moe_gemm_ok(h, idx, w_gu, w_down, act, in_w), "sm_moe_gemm: shapes, types or layout not taken");
+  const int64_t T = h.size(0), W = h.size(1), E = w_gu.size(0), ff = w_down.size(2), top = idx.size(1);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(h.device());
+  auto ints = at::empty({edge_sm_moe_gemm_ints(T * top, (int)E)}, idx.options());
+  auto y = at::empty({T * top, ff}, h.options());
+  auto out = at::empty({T, top, W}, h.options());
+  check(edge_sm_moe_gemm(h.data_ptr(), idx.data_ptr<int>(), w_gu.data_ptr(), w_down.data_ptr(), ints.data_ptr<int>(), y.data_ptr(),
+                         out.data_ptr(), (int)T, (int)top, (int)E, (int)W, (int)ff, (int)act,
+                         in_w ? in_w->data_ptr<float>() : nullptr, (float)limit, stream()), "sm_moe_gemm");
+  return out;
+}
+
 std::tuple<at::Tensor, at::Tensor, at::Tensor> sm_moe_route_grouped(const at::Tensor& h, const at::Tensor& router,
                                                                     const std::optional<at::Tensor>& corr, int64_t top,
                                                                     double scale, int64_t groups, int64_t keep, bool gate) {
@@ -1285,6 +1323,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_delta_scan", &sm_delta_scan);
   m.def("sm_moe_route", &sm_moe_route);
   m.def("sm_moe_experts", &sm_moe_experts);
+  m.def("sm_moe_gemm_ok", &sm_moe_gemm_ok);
+  m.def("sm_moe_gemm", &sm_moe_gemm);
   m.def("sm_group_norm", &sm_group_norm);
   m.def("sm_group_norm_residual", &sm_group_norm_residual);
   m.def("sm_glu_silu", &sm_glu_silu);

@@ -1,0 +1,286 @@
+// Mixture of experts at prompt sizes (bf16, MFMA): the (token, choice) pairs are grouped by expert and every expert's
+// rows run through its gate | up weights (activation in the epilogue) and then its down weights, one launch for all
+// experts each.
+//
+//   moe_sort_kernel   one workgroup: counts per expert, rows[p] = the pair (t * top + k) at sorted position p, and
+//                     the list of row tiles (expert, first position, rows), a tile never spanning two experts
+//   moe_gemm_kernel   tile lists x column tiles; the activations' rows are gathered (first product: h[t]) or taken in
+//                     sorted order (second), and the second product's rows go straight back to their pair's row
+//
+// Nothing crosses to the host: the grid covers the largest possible tile count and workgroups past the real one leave.
+//
+// Measured (both products, sorting and activation; MI355X) against one library product per expert with the sort, the
+// gather, the activation and the scatter as launches of their own: 4096 tokens x 3 of 16 experts 1024 -> 1024,
+// 758 -> 129 us (600 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 790 us (734); 512 x 4 of 32, 2048 -> 2048,
+// 1369 -> 238 us, where the experts' 805 MB (3.4 TB/s) are the bound.  At 128-row tiles the bound is the operands' way
+// into the LDS (64 B per clock and CU at the full MFMA rate): 128 x 256 tiles gain 3-6 % from 2048 columns on and lose
+// below, deeper rings with one workgroup per CU lose 40 %.
+#include "seqmix_common.h"
+
+namespace {
+typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+constexpr int SORT_NT = 1024, SORT_E = 512;
+enum { ACT_NONE = 0, ACT_GLU_CLAMP = 1, ACT_GLU_SILU = 2, ACT_RELU2 = 3 };
+
+// tiles: [0] = their number, tile i at [4 + 4 i] = (expert, first sorted position, rows, 0).
+// Counting by LDS atomics, one table per wave (16 waves share a CU: the lanes of one wave meet on at most E
+// counters).  The order of an expert's rows follows the atomics; no result depends on it.
+__global__ void __launch_bounds__(SORT_NT) moe_sort_kernel(const int* __restrict__ idx, int R, int E, int BM,
+                                                           int* __restrict__ rows, int* __restrict__ tiles) {
+  constexpr int NW = SORT_NT / 64;
+  __shared__ int cnt[NW][SORT_E];
+  __shared__ int scan_r[SORT_E], scan_t[SORT_E];
+  const int tid = threadIdx.x, wave = tid >> 6;
+  for (int i = tid; i < NW * SORT_E; i += SORT_NT) (&cnt[0][0])[i] = 0;
+  __syncthreads();
+  for (int i = tid; i < R; i += SORT_NT) atomicAdd(&cnt[wave][min(max(idx[i], 0), E - 1)], 1);
+  __syncthreads();
+  int total = 0, nt = 0;
+  if (tid < E) {
+    for (int w = 0; w < NW; ++w) {                           // the wave tables become offsets inside the expert
+      const int c = cnt[w][tid];
+      cnt[w][tid] = total;
+      total += c;
+    }
+    nt = (total + BM - 1) / BM;
+  }
+  if (tid < SORT_E) {
+    scan_r[tid] = total;
+    scan_t[tid] = nt;
+  }
+  __syncthreads();
+  for (int d = 1; d < E; d <<= 1) {                          // inclusive sums over the experts
+    int a = 0, b = 0;
+    if (tid < E && tid >= d) { a = scan_r[tid - d]; b = scan_t[tid - d]; }
+    __syncthreads();
+    if (tid < E) { scan_r[tid] += a; scan_t[tid] += b; }
+    __syncthreads();
+  }
+  if (tid < E) {
+    const int r0 = scan_r[tid] - total, t0 = scan_t[tid] - nt;
+    for (int w = 0; w < NW; ++w) cnt[w][tid] += r0;
+    for (int i = 0; i < nt; ++i)
+      *reinterpret_cast<int4*>(tiles + 4 + 4 * (t0 + i)) = make_int4(tid, r0 + i * BM, min(BM, total - i * BM), 0);
+    if (tid == E - 1) tiles[0] = scan_t[tid];
+  }
+  __syncthreads();
+  for (int i = tid; i < R; i += SORT_NT) rows[atomicAdd(&cnt[wave][min(max(idx[i], 0), E - 1)], 1)] = i;
+}
+
+__device__ __forceinline__ void glds16(const void* g, void* lds_base) {
+  __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds_base, 16, 0, 0);
+}
+__device__ __forceinline__ uint32_t lds_off(const void* p) {
+  return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void*)p);
+}
+// N ds_read_b128 at addr + 2048 i, which the compiler does not track: callers wait and pin before use
+template <int I, int N>
+__device__ __forceinline__ void lds_frags(uint32_t addr, v4i (&f)[N]) {
+  if constexpr (I < N) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(f[I]) : "v"(addr), "n"(I * 2048));
+    lds_frags<I + 1, N>(addr, f);
+  }
+}
+template <int N>
+__device__ __forceinline__ void pin(v4i (&f)[N]) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) asm volatile("" : "+v"(f[i]));
+}
+
+// out[r] = act(A[row(r)] W_e^T) for the rows r of each tile's expert e.  A: K-contiguous rows, W [E, NW, K].
+//  * BM x BN block tile (BN weight rows), WM x WN waves, 64-k stages.  Both operands go global -> LDS by LDS-DMA in
+//    1 KiB pieces of 8 rows x 128 B (whole cache lines); the 16-byte chunk c of row r sits at slot c ^ (r & 7), so
+//    the 16 rows of a fragment read spread over the banks.  R stages ride ahead of the arithmetic (counted vmcnt, one
+//    bare barrier per stage, fragments double-buffered in registers and read by asm so that no read drains the ring).
+//  * The weights are the MFMA's first operand: a lane's accumulator holds four consecutive output columns of one row,
+//    stored as 8 bytes.  Gated units (NW = 2 ff): a wave's 64 (or 32) weight rows are half gate rows and half the
+//    up rows of the same features, so one lane holds both halves and the activation never leaves the registers
+//    (fp32; the unfused form rounds both halves to bf16 first).
+//  * blockIdx -> tile: each XCD takes a contiguous range of the (real) tiles, walked in groups of four row tiles
+//    column by column, so neighbours in an L2 share an expert's weights.
+template <int BM, int BN, int WM, int WN, int R, int ACT, bool GATHER>
+__global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                  const int* __restrict__ rows, const int* __restrict__ tiles,
+                                                                  bf16_t* __restrict__ out, int top, int N, int NW, int K,
+                                                                  int grid_n, const float* __restrict__ row_w, float limit) {
+  constexpr bool GLU = ACT == ACT_GLU_CLAMP || ACT == ACT_GLU_SILU;
+  constexpr int NWV = WM * WN, AP = BM / 8, BP = BN / 8, PIECES = AP + BP, PPW = PIECES / NWV, STAGE = PIECES * 1024;
+  constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;
+  static_assert(PIECES % NWV == 0 && (!GLU || NJ % 2 == 0) && R * STAGE <= 160 * 1024, "tile shape");
+  __shared__ __attribute__((aligned(1024))) int8_t ring[R * STAGE];
+
+  const int nwg = tiles[0] * grid_n, orig = blockIdx.x;
+  if (orig >= nwg) return;
+  const int xcd = orig & 7, q8 = nwg >> 3, r8 = nwg & 7;
+  const int wgid = (xcd < r8 ? xcd * (q8 + 1) : r8 * (q8 + 1) + (xcd - r8) * q8) + (orig >> 3);
+  constexpr int GM = 4;
+  const int per_group = GM * grid_n, grp = wgid / per_group, gsz = min(GM, tiles[0] - grp * GM);
+  const int inr = wgid - grp * per_group, bm = grp * GM + inr % gsz, bn = inr / gsz;
+  const int4 tile = *reinterpret_cast<const int4*>(tiles + 4 + 4 * bm);   // (expert, first position, rows)
+  const bf16_t* We = W + (size_t)tile.x * NW * K;
+
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = wave / WN, wn = wave % WN, KT = K / 64;
+  constexpr int FN = GLU ? BN / 2 : BN;                      // output columns of a block tile
+  // this wave's DMA pieces p = wave + NWV i: activation rows 8 p .. (p < AP), or weight rows
+  const char* src[PPW];
+#pragma unroll
+  for (int i = 0; i < PPW; ++i) {
+    const int p = wave + NWV * i, r = (p < AP ? p : p - AP) * 8 + (lane >> 3);
+    const int ck = ((lane & 7) ^ (r & 7)) * 16;
+    size_t row;
+    const bf16_t* base;
+    if (p < AP) {
+      const int pos = tile.y + min(r, tile.z - 1);
+      row = GATHER ? rows[pos] / top : pos;
+      base = A;
+    } else {
+      int f;
+      if constexpr (GLU) {
+        const int w = r / (16 * NJ), j = (r / 16) % NJ;
+        f = min(bn * FN + w * (8 * NJ) + (j % (NJ / 2)) * 16 + (r & 15), N - 1) + (j >= NJ / 2 ? N : 0);
+      } else {
+        f = min(bn * FN + r, N - 1);
+      }
+      row = f;
+      base = We;
+    }
+    src[i] = reinterpret_cast<const char*>(base + row * (size_t)K) + ck;
+  }
+  // stages past the last re-load the last one into a slot that is not read again: the counts stay constant
+  auto issue = [&](int st) {
+    const size_t ko = (size_t)min(st, KT - 1) * 128;
+    int8_t* slot = ring + (st % R) * STAGE + wave * 1024;
+#pragma unroll
+    for (int i = 0; i < PPW; ++i) glds16(src[i] + ko, slot + NWV * i * 1024);
+  };
+  // fragment (16 rows x 32 k of step ks): row lane & 15, chunk 4 ks + (lane >> 4)
+  const uint32_t fo = lds_off(ring) + (lane & 15) * 128 + (((lane >> 4) ^ (lane & 7)) << 4);
+  auto read = [&](int st, int ks, v4i (&fa)[MI], v4i (&fw)[NJ]) {
+    const uint32_t b = (fo ^ (ks << 6)) + (st % R) * STAGE;
+    lds_frags<0, MI>(b + wm * (MI * 2048), fa);
+    lds_frags<0, NJ>(b + AP * 1024 + wn * (NJ * 2048), fw);
+  };
+  v4f acc[MI][NJ];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+  auto mma = [&](v4i (&fa)[MI], v4i (&fw)[NJ]) {
+    pin(fa);
+    pin(fw);
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j)
+        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, fw[j]), __builtin_bit_cast(v8bf, fa[i]),
+                                                            acc[i][j], 0, 0, 0);
+  };
+  auto pin_acc = [&]() {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) asm volatile("" : "+v"(acc[i][j]));
+  };
+
+#pragma unroll
+  for (int st = 0; st < R; ++st) issue(st);
+  v4i a0[MI], w0[NJ], a1[MI], w1[NJ];
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * PPW) : "memory");
+  __builtin_amdgcn_s_barrier();
+  read(0, 0, a0, w0);
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  for (int s = 0; s < KT; ++s) {
+    read(s, 1, a1, w1);
+    mma(a0, w0);
+    pin_acc();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (s + 1 < KT) {
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * PPW) : "memory");   // own pieces of stage s + 1
+      __builtin_amdgcn_s_barrier();                          // stage s + 1 is there, stage s has been read by all
+      issue(s + R);
+      read(s + 1, 0, a0, w0);
+    }
+    mma(a1, w1);
+    pin_acc();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");           // the re-loads past the end
+
+  // lane: row i * 16 + (lane & 15), columns 4 (lane >> 4) + 0..3 of column tile j
+  const int c4 = 4 * (lane >> 4);
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int r = (wm * MI + i) * 16 + (lane & 15);
+    if (r >= tile.z) continue;
+    const int pos = tile.y + r;
+    const size_t orow = GATHER ? (size_t)pos : (size_t)rows[pos];
+    const float rw = (ACT == ACT_GLU_SILU && row_w != nullptr) ? row_w[rows[pos]] : 1.f;
+    constexpr int NO = GLU ? NJ / 2 : NJ;
+#pragma unroll
+    for (int j = 0; j < NO; ++j) {
+      const int col = bn * FN + (wn * NO + j) * 16 + c4;
+      if (col >= N) continue;                                // N % 16 == 0: a column tile is whole or absent
+      float v[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float x = acc[i][j][q];
+        if constexpr (ACT == ACT_GLU_CLAMP) v[q] = glu_clamp_f(x, acc[i][j + NO][q], limit);
+        else if constexpr (ACT == ACT_GLU_SILU) v[q] = siluf_(rw * x) * (rw * acc[i][j + NO][q]);
+        else if constexpr (ACT == ACT_RELU2) { const float m = fmaxf(x, 0.f); v[q] = m * m; }
+        else v[q] = x;
+      }
+      *reinterpret_cast<uint2*>(out + orow * (size_t)N + col) = make_uint2(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]));
+    }
+  }
+}
+
+template <int BM, int BN, int WM, int WN, int R>
+int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* rows, const int* tiles, void* y, void* out,
+                int max_tiles, int top, int W, int ff, int act, const float* row_w, float limit, hipStream_t st) {
+  const dim3 blk(64 * WM * WN);
+  const int up = act == ACT_RELU2 ? 1 : 2, fn = act == ACT_RELU2 ? BN : BN / 2;
+  const int g1 = (ff + fn - 1) / fn, g2 = (W + BN - 1) / BN;
+#define MOE_FIRST(ACT)                                                                                                     \
+  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, ACT, true>), dim3(max_tiles * g1), blk, 0, st, (const bf16_t*)h,  \
+                     (const bf16_t*)w_gu, rows, tiles, (bf16_t*)y, top, ff, up * ff, W, g1, row_w, limit)
+  if (act == ACT_GLU_CLAMP) MOE_FIRST(ACT_GLU_CLAMP);
+  else if (act == ACT_GLU_SILU) MOE_FIRST(ACT_GLU_SILU);
+  else MOE_FIRST(ACT_RELU2);
+#undef MOE_FIRST
+  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, ACT_NONE, false>), dim3(max_tiles * g2), blk, 0, st, (const bf16_t*)y,
+                     (const bf16_t*)w_down, rows, tiles, (bf16_t*)out, top, W, W, ff, g2, nullptr, 0.f);
+  return (int)hipGetLastError();
+}
+
+// Rows of a tile by the average rows per expert: a tile much taller than that multiplies padding, and below about 24
+// the weights' bytes are all that counts (32 rows: two fragments, the smallest ring).
+int tile_rows(int64_t R, int E) { return R > (int64_t)E * 80 ? 128 : R > (int64_t)E * 24 ? 64 : 32; }
+int max_tiles(int64_t R, int E, int BM) { return (int)((R + BM - 1) / BM + (R < E ? R : E)); }
+}  // namespace
+
+extern "C" {
+
+// int32 words of scratch: the sorted pairs and the tile list
+int64_t edge_sm_moe_gemm_ints(int64_t R, int E) { return ((R + 3) & ~3LL) + 4 + 4LL * max_tiles(R, E, tile_rows(R, E)); }
+
+// 0 when the kernels take these sizes
+int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff) {
+  const int64_t R = T * top;
+  return W % 64 == 0 && ff % 64 == 0 && W > 0 && ff > 0 && E >= 1 && E <= SORT_E && R >= 1 && R < (1LL << 24) ? 0 : -2;
+}
+
+// h [T, W] bf16, idx [T, top], w_gu [E, 2 ff | ff, W], w_down [E, W, ff]; y: scratch [T top, ff]; out [T, top, W].
+int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void* w_down, int* ints, void* y, void* out, int T,
+                     int top, int E, int W, int ff, int act, const float* row_w, float limit, hipStream_t st) {
+  if (edge_sm_moe_gemm_ok(T, top, E, W, ff) != 0 || act < ACT_GLU_CLAMP || act > ACT_RELU2) return -2;
+  const int R = T * top, BM = tile_rows(R, E), mt = max_tiles(R, E, BM);
+  int *rows = ints, *tiles = ints + ((R + 3) & ~3);
+  hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(SORT_NT), 0, st, idx, R, E, BM, rows, tiles);
+  if (BM == 128) return launch_pair<128, 128, 2, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, st);
+  if (BM == 64) return launch_pair<64, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, st);
+  return launch_pair<32, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, st);
+}
+
+}  // extern "C"

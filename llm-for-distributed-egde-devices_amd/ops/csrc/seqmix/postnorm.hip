@@ -188,13 +188,7 @@ __global__ void __launch_bounds__(64) head_norm_gate_kernel(const float* __restr
   }
 }
 
-// g sigmoid(1.702 g) (up + 1), g = min(gate, limit), up clamped to +-limit; u row = gate [ff] | up [ff]
-__device__ __forceinline__ float glu_clamp_f(float g, float up, float limit) {
-  g = fminf(g, limit);
-  up = fminf(fmaxf(up, -limit), limit);
-  return g * sigmoidf_(1.702f * g) * (up + 1.f);
-}
-
+// u row = gate [ff] | up [ff]
 template <typename T>
 __global__ void __launch_bounds__(NT) glu_clamp_kernel(const T* __restrict__ u, int ld, T* __restrict__ y, int ff,
                                                        float limit) {

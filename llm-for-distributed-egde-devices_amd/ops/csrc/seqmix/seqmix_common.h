@@ -32,6 +32,12 @@ template <> __device__ __forceinline__ void store8<bf16_t>(bf16_t* p, const floa
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float siluf_(float x) { return x * sigmoidf_(x); }
+// g sigmoid(1.702 g) (up + 1), g = min(gate, limit), up clamped to +-limit
+__device__ __forceinline__ float glu_clamp_f(float g, float up, float limit) {
+  g = fminf(g, limit);
+  up = fminf(fmaxf(up, -limit), limit);
+  return g * sigmoidf_(1.702f * g) * (up + 1.f);
+}
 
 __device__ __forceinline__ float ex2(float x) { return __builtin_amdgcn_exp2f(x); }
 __device__ __forceinline__ v4f mfma4(float a, float b, v4f c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }

@@ -872,6 +872,18 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, scale: float, mod
 
 
 MOE_GEMM_MIN = int(__import__("os").environ.get("EDGELLM_MOE_GEMM_MIN", "64"))
+# steps of this many tokens or more take the grouped MFMA kernels where they run (bf16, widths of whole 64s): they read
+# each chosen expert once, the per-pair kernels once per pair.  us per layer, per pair / grouped: 16 experts of 1024 x
+# 1024, 3 per token: 6 tokens 24.8 / 24.8, 12 tokens 42 / 25, 63 tokens 122 / 28; 32 of 2048 x 2048, 4 per token: 6
+# tokens 123 / 125, 12 tokens 186 / 166, 63 tokens 599 / 207; squared ReLU beside a shared expert a little later
+MOE_MFMA_MIN = int(__import__("os").environ.get("EDGELLM_MOE_MFMA_MIN", "10"))
+_MOE_ACT = {"glu_clamp": 1, "silu_glu": 2, "relu2": 3}
+
+
+def moe_grouped(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor, act: str,
+                in_w: Optional[torch.Tensor] = None) -> bool:
+    """Whether ``moe_experts`` runs this step through the grouped MFMA kernels (csrc/seqmix/moe_gemm.hip)."""
+    return _gpu(h) and h.shape[0] >= MOE_MFMA_MIN and bool(_ext().sm_moe_gemm_ok(h, idx, w_gu, w_down, _MOE_ACT[act], in_w))
 
 
 def moe_experts(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor, limit: float,
@@ -888,6 +900,9 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: 
     E, ff2, W = w_gu.shape
     assert act in ("glu_clamp", "silu_glu", "relu2") and (in_w is None or act == "silu_glu")
     if _gpu(h):
+        if moe_grouped(h, idx, w_gu, w_down, act, in_w):
+            out = _ext().sm_moe_gemm(h, idx, w_gu, w_down, _MOE_ACT[act], float(limit), in_w)
+            return (out, None) if sorted_rows else out
         if T >= MOE_GEMM_MIN:
             return _moe_experts_sorted(h, idx, w_gu, w_down, limit, act, in_w, sorted_rows)
         out = _ext().sm_moe_experts_relu2(h, idx, w_gu, w_down, None, None)[0] if act == "relu2" else \
@@ -914,9 +929,9 @@ def moe_experts_shared(h: torch.Tensor, idx: torch.Tensor, w_up: torch.Tensor, w
 
 
 def _moe_experts_sorted(h, idx, w_gu, w_down, limit, act="glu_clamp", in_w=None, sorted_rows=False):
-    """Prompt-sized steps: (token, choice) pairs sorted by expert; every expert's rows run through its
-    gate | up weights, one activation launch covers all rows, every expert's rows run through its down
-    weights, and the rows go back to (token, choice) order.  bf16 on the GPU: the library's grouped
+    """Prompt-sized steps that the grouped kernels do not take (fp32, odd widths): (token, choice) pairs sorted by
+    expert; every expert's rows run through its gate | up weights, one activation launch covers all rows, every
+    expert's rows run through its down weights, and the rows go back to (token, choice) order.  bf16 on the GPU: the library's grouped
     product over the sorted rows with the experts' end offsets on the device (nothing crosses to the
     host, so the step stays asynchronous); otherwise one GEMM per expert with the counts on the host."""
     T, top = idx.shape

@@ -1,0 +1,111 @@
+"""The grouped expert kernels of prompt-sized steps (csrc/seqmix/moe_gemm.hip) against the float64 form of the same
+experts, at the edges of their tiles and of the routing."""
+import pytest
+import torch
+
+import edgellm  # noqa: F401
+from edgellm.ops import seqmix
+
+gpu = pytest.mark.gpu
+
+
+def reference(h, idx, w_gu, w_down, act, limit, in_w):
+    T, top = idx.shape
+    out = torch.zeros(T, top, w_down.shape[1], dtype=torch.float64)
+    h, w_gu, w_down = (t.cpu().double() for t in (h, w_gu, w_down))
+    idx = idx.cpu().long()
+    ff = w_down.shape[2]
+    for e in idx.unique().tolist():
+        t, k = (idx == e).nonzero(as_tuple=True)
+        u = h[t] @ w_gu[e].T
+        if act == "relu2":
+            y = torch.relu(u) ** 2
+        elif act == "silu_glu":
+            u = u if in_w is None else u * in_w.cpu().double()[t, k][:, None]
+            y = torch.nn.functional.silu(u[:, :ff]) * u[:, ff:]
+        else:
+            g, up = u[:, :ff].clamp(max=limit), u[:, ff:].clamp(-limit, limit)
+            y = g * torch.sigmoid(1.702 * g) * (up + 1)
+        out[t, k] = y @ w_down[e].T
+    return out
+
+
+def inputs(T, top, E, W, ff, act, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    up = 1 if act == "relu2" else 2
+    h = torch.randn(T, W, generator=g).bfloat16()
+    w_gu = (torch.randn(E, up * ff, W, generator=g) * W ** -0.5).bfloat16()
+    w_down = (torch.randn(E, W, ff, generator=g) * ff ** -0.5).bfloat16()
+    idx = torch.rand(T, E, generator=g).topk(top, -1).indices.int()
+    in_w = torch.rand(T, top, generator=g) if act == "silu_glu" else None
+    return [t.cuda() if t is not None else None for t in (h, idx, w_gu, w_down, in_w)]
+
+
+# the hidden unit is stored in bf16 (relative rounding 2^-9 per term, random) and so is the result: 2-norm error about
+# 2^-9 sqrt(2 / 3) each = 2.3e-3 together; twice that is the bound
+TOL = 5e-3
+
+
+@gpu
+@pytest.mark.parametrize("act", ["glu_clamp", "silu_glu", "relu2"])
+@pytest.mark.parametrize("T,top,E,W,ff", [
+    (10, 2, 5, 64, 64),          # one k step, fewer rows than experts can fill
+    (33, 3, 4, 128, 192),        # rows per expert about one 32-row tile; columns past a whole 128
+    (100, 1, 2, 192, 64),        # 64-row tiles with a remainder
+    (257, 2, 3, 256, 320),       # 128-row tiles with a remainder
+    (1030, 4, 16, 320, 128),     # several tiles per expert
+    (70, 1, 512, 64, 128)])      # the most experts
+def test_grouped_experts_against_float64(T, top, E, W, ff, act):
+    h, idx, w_gu, w_down, in_w = inputs(T, top, E, W, ff, act)
+    assert seqmix.moe_grouped(h, idx, w_gu, w_down, act, in_w)
+    got = seqmix.moe_experts(h, idx, w_gu, w_down, 1.5, act, in_w).cpu().double()
+    want = reference(h, idx, w_gu, w_down, act, 1.5, in_w)
+    assert ((got - want).norm() / want.norm()) < TOL
+    assert ((got - want).norm(dim=-1) / want.norm(dim=-1).clamp_min(1e-3)).max() < 4 * TOL
+
+
+@gpu
+@pytest.mark.parametrize("case", ["one expert", "first and last", "idle neighbours"])
+def test_grouped_experts_with_skewed_routing(case):
+    T, E = 300, 9
+    h, idx, w_gu, w_down, _ = inputs(T, 2, E, 64, 128, "relu2", 3)
+    if case == "one expert":
+        idx.fill_(4)
+    elif case == "first and last":
+        idx[:, 0], idx[:, 1] = 0, E - 1
+    else:
+        idx[:, 0], idx[:, 1] = 2, 7
+    got, rows = seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "relu2", sorted_rows=True)
+    assert rows is None
+    want = reference(h, idx, w_gu, w_down, "relu2", 0.0, None)
+    assert ((got.cpu().double() - want).norm() / want.norm()) < TOL
+
+
+@gpu
+def test_grouped_experts_keep_nan_and_infinity_in_their_rows():
+    h, idx, w_gu, w_down, in_w = inputs(64, 2, 4, 128, 64, "silu_glu", 5)
+    clean = seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "silu_glu", in_w)
+    bad = h.clone()
+    bad[7], bad[40, 3] = float("nan"), float("inf")
+    got = seqmix.moe_experts(bad, idx, w_gu, w_down, 0.0, "silu_glu", in_w)
+    keep = torch.ones(64, dtype=torch.bool)
+    keep[[7, 40]] = False
+    assert torch.equal(got[keep.cuda()], clean[keep.cuda()])
+    assert got[7].isnan().all()
+
+
+@gpu
+def test_steps_that_the_grouped_kernels_do_not_take():
+    h, idx, w_gu, w_down, in_w = inputs(80, 2, 4, 128, 96, "silu_glu", 6)          # ff is no whole 64
+    assert not seqmix.moe_grouped(h, idx, w_gu, w_down, "silu_glu", in_w)
+    got = seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "silu_glu", in_w).cpu().double()
+    want = reference(h, idx, w_gu, w_down, "silu_glu", 0.0, in_w)
+    assert ((got - want).norm() / want.norm()) < 2 * TOL                            # both halves rounded to bf16 as well
+    h, idx, w_gu, w_down, in_w = inputs(80, 2, 4, 128, 64, "silu_glu", 7)
+    wide = torch.randn(80, 256, device="cuda").bfloat16()
+    wide[:, :128] = h
+    assert not seqmix.moe_grouped(wide[:, :128], idx, w_gu, w_down, "silu_glu", in_w)   # rows of a wider tensor
+    assert not seqmix.moe_grouped(h.float(), idx, w_gu.float(), w_down.float(), "silu_glu", in_w)
+    assert not seqmix.moe_grouped(h[:5], idx[:5], w_gu, w_down, "silu_glu", in_w[:5])
+    assert torch.allclose(seqmix.moe_experts(wide[:, :128], idx, w_gu, w_down, 0.0, "silu_glu", in_w).float(),
+                          seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "silu_glu", in_w).float(), atol=3e-2, rtol=3e-2)
