@@ -775,16 +775,27 @@ def delta_prepare_head(qkv: torch.Tensor, u: torch.Tensor, b0: int, a0: int, dt_
     return torch.cat([q.reshape(T, GN), k.reshape(T, GN), g, beta], -1)
 
 
+# bf16 steps whose longest portion has this many tokens run the delta rule over 64-token chunks (csrc/seqmix/delta_chunk.hip);
+# us, token by token / chunks, 16 heads: 64 x 64 states, 128 tokens 32 / 43, 1500 + 77 tokens 348 / 86, 4096 tokens 916 / 172;
+# 128 x 128 states, 96 tokens 38 / 49, two portions of 512 208 / 128, 4096 tokens 1521 / 378.  Against 64 bits the chunks
+# are 1.4e-7 to 2.8e-7 off (token by token 0.8e-7): nothing beside bf16 activations, but fp32 steps stay token by token
+DELTA_CHUNK_MIN = int(__import__("os").environ.get("EDGELLM_DELTA_CHUNK_MIN", "160"))
+
+
 def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, meta: RaggedMeta, heads: int,
                     kv_heads: int, N: int, P: int) -> torch.Tensor:
-    """The gated delta rule, token by token in fp32.  ``prep`` from ``delta_prepare`` (a decay per
+    """The gated delta rule in fp32.  ``prep`` from ``delta_prepare`` (a decay per
     head and key channel) or ``delta_prepare_head`` (one per head: the row is shorter); the values are
     columns [2 kv_heads N, ..) of ``qkv``.  Per head, with S [N, P]:  S <- g * S (rows) ;
     w = beta (v - S^T k) ;  S <- S + k w^T ;  o = S^T q.  state [slots, heads, N, P] fp32 is read
     (zero for a portion starting at 0) and left at the portion's end.  Returns o fp32 [T, heads P]."""
     if _gpu(prep):
+        chunks = max_chunks = 0                          # 0: one workgroup per (sequence, head, 16 value columns), token by token
+        if meta.max_len >= DELTA_CHUNK_MIN and N <= 256 and qkv.dtype == torch.bfloat16:
+            per = [(h[2] + 63) // 64 for h in meta.host]
+            chunks, max_chunks = sum(per), max(per)
         return _ext().sm_delta_scan(prep, qkv, state, meta.seq_slot, meta.seq_start, meta.seq_len, meta.seq_off,
-                                    int(meta.n), int(heads), int(kv_heads), int(N), int(P))
+                                    int(meta.n), int(heads), int(kv_heads), int(N), int(P), int(chunks), int(max_chunks))
     T, GN, rep = prep.shape[0], kv_heads * N, heads // kv_heads
     if prep.shape[1] == 2 * GN + 2 * heads and N != 1:           # per-head decays: one number for all key channels
         prep = torch.cat([prep[:, :2 * GN], prep[:, 2 * GN:2 * GN + heads].repeat_interleave(N, 1),

@@ -1,0 +1,88 @@
+"""The chunked form of the gated delta rule (csrc/seqmix/delta_chunk.hip) against the recurrence in float64."""
+import pytest
+import torch
+
+import edgellm  # noqa: F401
+from edgellm.ops import seqmix
+
+pytestmark = pytest.mark.gpu
+
+
+def recurrence(prep, v, S, G, H, N, channel):
+    """prep [L, q | k | decay | beta], v [L, H, P], S [H, N, P], all float64."""
+    GN, rep, D = G * N, H // G, H * (N if channel else 1)
+    q, k = (prep[:, i * GN:(i + 1) * GN].view(-1, G, N).repeat_interleave(rep, 1) for i in (0, 1))
+    g, beta = prep[:, 2 * GN:2 * GN + D].view(len(prep), H, -1), prep[:, 2 * GN + D:]
+    out = torch.empty_like(v)
+    for t in range(len(prep)):
+        S = S * g[t][:, :, None]
+        w = beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1))
+        S = S + k[t][:, :, None] * w[:, None, :]
+        out[t] = (S * q[t][:, :, None]).sum(1)
+    return out, S
+
+
+def inputs(lens, starts, H, G, N, P, channel, decay, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    T = sum(lens)
+    meta = seqmix.RaggedMeta.build([(len(lens) - 1 - i, st, L) for i, (st, L) in enumerate(zip(starts, lens))],
+                                   torch.zeros(len(lens), 4, dtype=torch.int32, device="cuda"), 64, "cuda")
+    qkv = torch.nn.functional.silu(torch.randn(T, 2 * G * N + H * P, generator=g)).bfloat16().cuda()
+    unit = torch.nn.functional.normalize(torch.randn(2, T, G, N, generator=g), dim=-1)
+    D = H * (N if channel else 1)
+    d = {"weak": 1.0 - 1e-4 * torch.rand(T, D, generator=g), "usual": torch.rand(T, D, generator=g) ** 0.1,
+         "strong": torch.rand(T, D, generator=g) * 1e-3, "mixed": torch.where(torch.rand(T, D, generator=g) < 0.1, 0.0, 0.99)}[decay]
+    prep = torch.cat([(unit[0] * N ** -0.5).reshape(T, -1), unit[1].reshape(T, -1), d, torch.rand(T, H, generator=g)], -1)
+    state = torch.randn(len(lens), H, N, P, generator=g)
+    return prep.cuda(), qkv, state.cuda(), meta
+
+
+# both forms sum in fp32 (2^-24 relative per operation); 64 terms a chunk and logs that add up to a few hundred leave about
+# 3e-7 of the output's size, and a token's own rounding the same: bound 2e-6
+TOL = 2e-6
+
+
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("decay", ["weak", "usual", "strong", "mixed"])
+@pytest.mark.parametrize("lens,starts,H,G,N,P", [
+    ((64, 63, 65), (0, 5, 0), 4, 4, 64, 64),          # about one chunk
+    ((200, 1, 16), (3, 7, 0), 4, 2, 24, 20),          # odd sizes, shared keys, a decode token and a short portion beside
+    ((321,), (0,), 2, 2, 128, 48),                    # 128 channels: two quarters
+    ((130, 17), (1, 0), 2, 1, 200, 70)])              # up to 256 channels: four quarters
+def test_chunks_against_the_recurrence(lens, starts, H, G, N, P, channel, decay, monkeypatch):
+    prep, qkv, state, meta = inputs(lens, starts, H, G, N, P, channel, decay)
+    before = state.double().cpu()
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1)
+    y = seqmix.delta_rule_scan(prep, qkv, state, meta, H, G, N, P).double().cpu()
+    p, v = prep.double().cpu(), qkv[:, 2 * G * N:].double().cpu().view(len(prep), H, P)
+    for slot, start, n, off in meta.host:
+        S0 = before[slot] if start > 0 else torch.zeros(H, N, P, dtype=torch.float64)
+        want, S = recurrence(p[off:off + n], v[off:off + n], S0, G, H, N, channel)
+        got = y[off:off + n].view(n, H, P)
+        assert (got - want).norm() < TOL * want.norm() and (got - want).abs().max() < 20 * TOL * want.abs().max()
+        assert (state[slot].double().cpu() - S).norm() < TOL * S.norm().clamp_min(1e-3)
+
+
+def test_the_longest_portion_decides_and_fp32_steps_stay_token_by_token(monkeypatch):
+    prep, qkv, state, meta = inputs((200, 40), (0, 9), 2, 2, 64, 32, True, "usual", 1)
+    a, b = state.clone(), state.clone()
+    chunks = seqmix.delta_rule_scan(prep, qkv, a, meta, 2, 2, 64, 32)
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1 << 30)
+    steps = seqmix.delta_rule_scan(prep, qkv, b, meta, 2, 2, 64, 32)
+    assert not torch.equal(chunks, steps) and torch.allclose(chunks, steps, atol=1e-5) and torch.allclose(a, b, atol=1e-5)
+    monkeypatch.undo()
+    c, d = state.clone(), state.clone()
+    y = seqmix.delta_rule_scan(prep, qkv.float(), c, meta, 2, 2, 64, 32)
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1 << 30)
+    assert torch.equal(y, seqmix.delta_rule_scan(prep, qkv.float(), d, meta, 2, 2, 64, 32)) and torch.equal(c, d)
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_value_that_is_not_finite_reaches_no_earlier_token(bad, monkeypatch):
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1)
+    prep, qkv, state, meta = inputs((100, 70), (0, 0), 2, 2, 64, 32, True, "usual", 2)
+    clean = seqmix.delta_rule_scan(prep, qkv, state.clone(), meta, 2, 2, 64, 32)
+    qkv[75, -3] = bad                                  # a value of head 1, in the middle of a block
+    y = seqmix.delta_rule_scan(prep, qkv, state.clone(), meta, 2, 2, 64, 32)
+    assert torch.allclose(y[:75], clean[:75], atol=1e-6) and torch.allclose(y[100:], clean[100:], atol=1e-6)
+    assert torch.allclose(y[75:100, :32], clean[75:100, :32], atol=1e-6) and not y[75, -3].isfinite()
