@@ -1,3 +1,4 @@
+import pytest
 import torch
 
 from edgellm.engine import Generator, KVCache, SamplingParams
@@ -108,3 +109,18 @@ def test_sample_advance_is_sample_then_decode_advance():
         assert torch.equal(nb, nxt)
     for k in a:
         assert torch.equal(a[k], b[k]), k
+
+
+def test_start_marks_every_prompt_token_and_refuses_ids_outside_the_vocabulary():
+    """The repetition-penalty flags after ``start``: one per (row, prompt token), for unequal prompts and repeats."""
+    model = build_model(tiny("llama2"), dtype=torch.float32, device="cpu", seed=0)
+    V = model.cfg.vocab_size
+    gen = Generator(model, max_batch=3, max_seq=64)
+    prompts = [[5, 5, V - 1], [0], [7, 3, 2, 1]]
+    gen.start(prompts, SamplingParams(max_new_tokens=2, do_sample=False, repetition_penalty=1.0))
+    first = gen._state.out[:, 0].tolist()
+    for b, p in enumerate(prompts):
+        assert set(gen._state.seen[b].nonzero().flatten().tolist()) - {first[b]} == set(p) - {first[b]}
+    for bad in (V, -1):
+        with pytest.raises(IndexError):
+            gen.start([[1, 2, bad], [3], [4]], SamplingParams(max_new_tokens=2))
