@@ -93,7 +93,7 @@ int edge_llmint8_prep(const void* x, int M, int K, float thr, int cmax, void* q,
 int edge_llmint8_outlier(void* out, const float* xo, const int* cols, const int* count, const void* wt,
                          const float* scb, int M, int N, int cmax, hipStream_t st);
 int edge_llmint8_gemv(const void* x, float thr, const void* Wp, const float* sw, const void* bias, const void* wt,
-                      const float* scb, void* out, int N, int K, hipStream_t st, int act);
+                      const float* scb, void* out, int N, int K, hipStream_t st, int act, const void* add);
 int edge_llmint8_gemv_norm(const void* x, const void* res, const void* gamma, const void* beta, float eps, int ln,
                            void* res_out, void* y_out, float thr, const void* Wp, const float* sw, const void* bias,
                            const void* wt, const float* scb, void* out, int N, int K, hipStream_t st, int glu,
@@ -814,10 +814,11 @@ void llmint8_outlier(at::Tensor& out, const at::Tensor& xo, const at::Tensor& co
 }
 
 // LLM.int8 projection of one bf16 row [1, K] in one launch (gemm_i8.hip l8_prologue: outlier
-// columns, int8 quant, GEMV, outlier part): bf16 [1, N], or None when the shape is not taken.
+// columns, int8 quant, GEMV, outlier part): bf16 [1, N] (+ add, bf16 [1, N]), or None when the shape is not taken.
 std::optional<at::Tensor> llmint8_gemv(const at::Tensor& x, double thr, const at::Tensor& wp, const at::Tensor& sw,
                                        const std::optional<at::Tensor>& bias, const at::Tensor& wt,
-                                       const at::Tensor& scb, int64_t N, int64_t act) {
+                                       const at::Tensor& scb, int64_t N, int64_t act,
+                                       const std::optional<at::Tensor>& add) {
   DEVICE_GUARD(x);
   need(x, at::kBFloat16, "x");
   need(wt, at::kChar, "weight_t");
@@ -827,10 +828,14 @@ std::optional<at::Tensor> llmint8_gemv(const at::Tensor& x, double thr, const at
   check_w8a8_operands(wp, sw, bias, N, K);
   TORCH_CHECK(wt.dim() == 2 && wt.size(0) == K && wt.size(1) == N && wt.is_contiguous() && scb.numel() == N,
               "weight_t [K, N], SCB [N]");
+  if (add) {
+    need(*add, at::kBFloat16, "add");
+    TORCH_CHECK(add->numel() == N && add->is_contiguous() && act == 0, "add: dense bf16 [1, N], no activation");
+  }
   auto out = at::empty({1, N}, x.options());
   const int r = edge_llmint8_gemv(x.data_ptr(), (float)thr, wp.data_ptr(), sw.data_ptr<float>(),
                                   bias ? bias->data_ptr() : nullptr, wt.data_ptr(), scb.data_ptr<float>(),
-                                  out.data_ptr(), (int)N, (int)K, stream(), (int)act);
+                                  out.data_ptr(), (int)N, (int)K, stream(), (int)act, add ? add->data_ptr() : nullptr);
   if (r == -2) return std::nullopt;
   check(r, "llmint8_gemv");
   return out;

@@ -296,9 +296,11 @@ struct NormIn {
   float thr = 0.f;                // LLM.int8 (NRM >= 128): outlier threshold on |x|
   const int8_t* wt = nullptr;     // LLM.int8: int8 W^T [K][N] (an outlier column is one row)
   const float* scb = nullptr;     // LLM.int8: per-row weight absmax SCB [N]
+  const bf16_t* add = nullptr;    // LLM.int8: a row added to the (bf16) result (may be null)
   bf16_t* y_out = nullptr;        // LLM.int8 of a normed row: the normalised row too (may be null)
 };
 constexpr int NRM_ROWS = 4;
+constexpr int L8_COUNT = 24;      // where l8_prologue leaves the outlier count (after 4 wave totals for each of 6 chunks)
 constexpr int L8_CMAX = 256;      // LLM.int8 outlier columns per row held in LDS (llmint8.hip's cap)
 
 // The prologue's global loads (slices, residual, gamma) are issued by norm_load BEFORE the
@@ -683,8 +685,9 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, int H, int8_t* aq,
       }
     }
   }
+  // outliers per thread and chunk, ranked in column order: wave totals of every chunk meet in LDS at one barrier
   uint32_t take[NCH];
-  int base = 0;                                           // outliers in the chunks before c
+  int incl[NCH];
 #pragma unroll
   for (int c = 0; c < NCH; ++c) {
     const int e = (c * 256 + (act ? t : 0)) * 8;
@@ -695,24 +698,25 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, int H, int8_t* aq,
         for (int j = 0; j < 8; ++j) bits |= (fabsf(v[c][j]) > na.thr ? 1u : 0u) << j;
       }
     }
-    const int pc = __popc(bits);
-    int incl = pc;
+    take[c] = bits;
+    incl[c] = __popc(bits);
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
-      const int tt = __shfl_up(incl, o, 64);
-      if (lane >= o) incl += tt;
+      const int tt = __shfl_up(incl[c], o, 64);
+      if (lane >= o) incl[c] += tt;
     }
-    if (act && lane == 63) scr[w] = incl;                 // wave totals of this chunk
-    __syncthreads();
-    int wb = base;
-    if (act) {
-      for (int i = 0; i < w; ++i) wb += scr[i];
-    }
-    const int tot = scr[0] + scr[1] + scr[2] + scr[3];
-    __syncthreads();                                      // scr reused by the next chunk
+    if (act && lane == 63) scr[c * 4 + w] = incl[c];
+  }
+  __syncthreads();
+  int base = 0;                                           // outliers in the chunks before c
+#pragma unroll
+  for (int c = 0; c < NCH; ++c) {
+    const int e = (c * 256 + (act ? t : 0)) * 8;
+    const int n0 = scr[c * 4], n1 = scr[c * 4 + 1], n2 = scr[c * 4 + 2], n3 = scr[c * 4 + 3];
+    const uint32_t bits = take[c];
     uint32_t tk = 0;
-    if (act) {
-      int slot = wb + incl - pc;
+    if (bits) {
+      int slot = base + (w > 0 ? n0 : 0) + (w > 1 ? n1 : 0) + (w > 2 ? n2 : 0) + incl[c] - __popc(bits);
 #pragma unroll
       for (int j = 0; j < 8; ++j) {                       // (static indices: v stays in registers)
         if ((bits >> j) & 1u) {
@@ -726,9 +730,9 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, int H, int8_t* aq,
       }
     }
     take[c] = tk;
-    base += tot;
+    base += n0 + n1 + n2 + n3;
   }
-  if (t == 0) scr[8] = min(base, L8_CMAX);
+  if (t == 0) scr[L8_COUNT] = min(base, L8_CMAX);
   float am = 0.f;
   if (act) {
 #pragma unroll
@@ -788,7 +792,7 @@ __global__ void __launch_bounds__(TG * KW * 64) w8a8_gemv_kernel(const int8_t* _
   static_assert(!L8_N || (EPI == EPI_OUT && MB == 1), "LLM.int8 prologue: one row, plain output");
   __shared__ int l8_cols[L8_N ? L8_CMAX : 1];
   __shared__ float l8_xo[L8_N ? L8_CMAX : 1];
-  __shared__ int l8_scr[16];
+  __shared__ int l8_scr[L8_COUNT + 1];
   __shared__ int8_t aq_l[NRM > 0 ? NRM_ROWS * NCH_N * 2048 : 16];
   __shared__ float nsa[16], nred[16];
   constexpr bool GELUQ = EPI == EPI_GELUQT || EPI == EPI_GELUQE;
@@ -1017,7 +1021,7 @@ __global__ void __launch_bounds__(TG * KW * 64) w8a8_gemv_kernel(const int8_t* _
         const int col = (jj == 0 ? nt0 : nt0 + NTt / 2) * 16 + lane;
         float y = (float)tot * nsa[0];
         y = y * sw[col] + (bias != nullptr ? bf2f(bias[col]) : 0.f);
-        const int nt = l8_scr[8];
+        const int nt = l8_scr[L8_COUNT];
         if (nt > 0) {
           float a = 0.f;
           for (int j = 0; j < nt; ++j) a += l8_xo[j] * (float)na.wt[(size_t)l8_cols[j] * N + col];
@@ -1041,7 +1045,7 @@ __global__ void __launch_bounds__(TG * KW * 64) w8a8_gemv_kernel(const int8_t* _
       if (col < N) {
         float y = (float)tot * nsa[0];
         y = y * pre.s0[0] + pre.b0[0];
-        const int nt = l8_scr[8];
+        const int nt = l8_scr[L8_COUNT];
         if (nt > 0) {
           float a = 0.f;
           for (int j = 0; j < nt; ++j) a += l8_xo[j] * (float)na.wt[(size_t)l8_cols[j] * N + col];
@@ -1053,6 +1057,7 @@ __global__ void __launch_bounds__(TG * KW * 64) w8a8_gemv_kernel(const int8_t* _
           if constexpr (L8ACT_N == 1) y = 0.5f * a * (1.f + tanhf(0.7978845608028654f * (a + 0.044715f * a * a * a)));
           else y = 0.5f * a * (1.f + erff(a * 0.7071067811865476f));
         }
+        if (na.add != nullptr) y = bf2f(f2bf(y)) + bf2f(na.add[col]);   // the other branch's row
         reinterpret_cast<bf16_t*>(outv)[col] = f2bf(y);
       }
     }
@@ -1801,6 +1806,20 @@ int launch_norm(const NormIn& na, const void* Wp, const float* sw, const void* b
   return (int)hipGetLastError();
 }
 
+// One row over plain outputs: as many 16-column tiles per workgroup as keep the launch to about one round of the 256
+// CUs: with fewer, the launch waits on a few CUs' own read rate.  LLM.int8 at batch 1, us per launch, three tiles always
+// / this rule with the ranking at one barrier: N x K 2560 x 10240 18.8 / 11.2, 2560 x 2560 8.5 / 6.2, 7680 x 2560 10.4 /
+// 9.1; 10240 x 2560 (three tiles either way) 10.2 / 9.3.  W8A8 behind LayerNorm 2048 x 2048 5.7 / 4.7, 6144 x 2048 6.3 /
+// 5.5, 7680 x 2560 8.3 / 7.7; behind RMSNorm 4096 x 4096 8.0 / 6.1, 6144 x 4096 8.4 / 7.3, 12288 x 4096 11.5 / 11.5.
+template <int NRM>
+int launch_norm_out(const NormIn& na, const void* Wp, const float* sw, const void* bias, void* out, int M, int N, int K,
+                    hipStream_t st) {
+  const int NTt = (N + 15) / 16;
+  if (NTt <= 256) return launch_norm<1, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+  if (NTt <= 512) return launch_norm<2, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+  return launch_norm<3, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+}
+
 // 65-128 decode rows (two 64-row micro-batches, or one 128-row one) on the ring2 kernel (geometries
 // measured with tools/bench_ops.py --only ring):
 //  * split-K (o / down): 8 compute waves (two per SIMD: the grouped-scale per-k-tile fold issues
@@ -2030,7 +2049,11 @@ extern "C" int edge_w8a8_gemv_norm(const float* part, int S, const void* res, co
                              : launch_norm<NTW, TG, KW, EP, 20>(na, Wp, sw, bias, out, OS, M, N, K, st))    \
                    : (S <= 2 ? launch_norm<NTW, TG, KW, EP, 10>(na, Wp, sw, bias, out, OS, M, N, K, st)     \
                              : launch_norm<NTW, TG, KW, EP, 12>(na, Wp, sw, bias, out, OS, M, N, K, st))
-  if (epi == EPI_OUT) NRM_L(3, 1, 16, EPI_OUT, nullptr);
+  if (epi == EPI_OUT)
+    return K == 4096 ? (S <= 2 ? launch_norm_out<18>(na, Wp, sw, bias, out, M, N, K, st)
+                               : launch_norm_out<20>(na, Wp, sw, bias, out, M, N, K, st))
+                     : (S <= 2 ? launch_norm_out<10>(na, Wp, sw, bias, out, M, N, K, st)
+                               : launch_norm_out<12>(na, Wp, sw, bias, out, M, N, K, st));
   if (epi == EPI_GLUQ) {
     if (N % 128 != 0 || os == nullptr) return -2;
     NRM_L(8, 2, 8, EPI_GLUQ, os);
@@ -2056,7 +2079,9 @@ extern "C" int edge_w8a8_gemv_ln(const void* x, const void* res, const void* gam
 #define LN_L(NTW, TG, KW, EP, OS)                                                                   \
   return K <= 2048 ? launch_norm<NTW, TG, KW, EP, 64 + 8>(na, Wp, sw, bias, out, OS, M, N, K, st)  \
                    : launch_norm<NTW, TG, KW, EP, 64 + 16>(na, Wp, sw, bias, out, OS, M, N, K, st)
-  if (epi == EPI_OUT) LN_L(3, 1, 16, EPI_OUT, nullptr);
+  if (epi == EPI_OUT)
+    return K <= 2048 ? launch_norm_out<64 + 8>(na, Wp, sw, bias, out, M, N, K, st)
+                     : launch_norm_out<64 + 16>(na, Wp, sw, bias, out, M, N, K, st);
   if (epi == EPI_GELUQT || epi == EPI_GELUQE) {
     if (N % 64 != 0 || os == nullptr) return -2;
     if (epi == EPI_GELUQT) LN_L(4, 1, 16, EPI_GELUQT, os);
@@ -2069,29 +2094,31 @@ extern "C" int edge_w8a8_gemv_ln(const void* x, const void* res, const void* gam
 // LLM.int8 projection of one bf16 row in one launch (l8_prologue): out bf16 [1, N] = int8 GEMV of x
 // with its outlier columns (|x| > thr, the first 256 in column order) zeroed, per-token scale, sw =
 // SCB / 127 (+ bias), plus the outlier columns' part from wt = int8 W^T [K, N].  K % 64 == 0,
-// K <= 12288.  -2: not taken.
+// K <= 12288.  add (may be null): a bf16 row added to the rounded result.  -2: not taken.
 extern "C" int edge_llmint8_gemv(const void* x, float thr, const void* Wp, const float* sw, const void* bias,
-                                 const void* wt, const float* scb, void* out, int N, int K, hipStream_t st, int act) {
+                                 const void* wt, const float* scb, void* out, int N, int K, hipStream_t st, int act,
+                                 const void* add) {
   if (K % 64 != 0 || K > 12288 || K < 64 || N % 16 != 0) return -2;
   NormIn na{nullptr, nullptr, nullptr, nullptr, 0.f, 0};
   na.x = (const bf16_t*)x;
   na.thr = thr;
   na.wt = (const int8_t*)wt;
   na.scb = scb;
+  na.add = (const bf16_t*)add;
   if (act == 1 || act == 2) {                            // + gelu (tanh / erf) of the output, K <= 4096
     if (K > 4096) return -2;
-    if (act == 1) return K <= 2048 ? launch_norm<3, 1, 16, EPI_OUT, 256 + 8>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-                                   : launch_norm<3, 1, 16, EPI_OUT, 256 + 16>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    return K <= 2048 ? launch_norm<3, 1, 16, EPI_OUT, 320 + 8>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-                     : launch_norm<3, 1, 16, EPI_OUT, 320 + 16>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
+    if (act == 1) return K <= 2048 ? launch_norm_out<256 + 8>(na, Wp, sw, bias, out, 1, N, K, st)
+                                   : launch_norm_out<256 + 16>(na, Wp, sw, bias, out, 1, N, K, st);
+    return K <= 2048 ? launch_norm_out<320 + 8>(na, Wp, sw, bias, out, 1, N, K, st)
+                     : launch_norm_out<320 + 16>(na, Wp, sw, bias, out, 1, N, K, st);
   }
   switch ((K + 2047) / 2048) {                            // row chunks of 2048 per 256 threads
-    case 1: return launch_norm<3, 1, 16, EPI_OUT, 128 + 8>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    case 2: return launch_norm<3, 1, 16, EPI_OUT, 128 + 16>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    case 3: return launch_norm<3, 1, 16, EPI_OUT, 128 + 24>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    case 4: return launch_norm<3, 1, 16, EPI_OUT, 128 + 32>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    case 5: return launch_norm<3, 1, 16, EPI_OUT, 128 + 40>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    default: return launch_norm<3, 1, 16, EPI_OUT, 128 + 48>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
+    case 1: return launch_norm_out<128 + 8>(na, Wp, sw, bias, out, 1, N, K, st);
+    case 2: return launch_norm_out<128 + 16>(na, Wp, sw, bias, out, 1, N, K, st);
+    case 3: return launch_norm_out<128 + 24>(na, Wp, sw, bias, out, 1, N, K, st);
+    case 4: return launch_norm_out<128 + 32>(na, Wp, sw, bias, out, 1, N, K, st);
+    case 5: return launch_norm_out<128 + 40>(na, Wp, sw, bias, out, 1, N, K, st);
+    default: return launch_norm_out<128 + 48>(na, Wp, sw, bias, out, 1, N, K, st);
   }
 }
 
@@ -2114,24 +2141,24 @@ extern "C" int edge_llmint8_gemv_norm(const void* x, const void* res, const void
   if (act == 1 || act == 2) {              // + gelu (tanh / erf) of the output
     if (glu) return -2;
     if (act == 1) {
-      if (K <= 2048) return ln ? launch_norm<3, 1, 16, EPI_OUT, 256 + 8 + 2>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-                               : launch_norm<3, 1, 16, EPI_OUT, 256 + 8 + 1>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-      return ln ? launch_norm<3, 1, 16, EPI_OUT, 256 + 16 + 2>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-                : launch_norm<3, 1, 16, EPI_OUT, 256 + 16 + 1>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
+      if (K <= 2048) return ln ? launch_norm_out<256 + 8 + 2>(na, Wp, sw, bias, out, 1, N, K, st)
+                               : launch_norm_out<256 + 8 + 1>(na, Wp, sw, bias, out, 1, N, K, st);
+      return ln ? launch_norm_out<256 + 16 + 2>(na, Wp, sw, bias, out, 1, N, K, st)
+                : launch_norm_out<256 + 16 + 1>(na, Wp, sw, bias, out, 1, N, K, st);
     }
-    if (K <= 2048) return ln ? launch_norm<3, 1, 16, EPI_OUT, 320 + 8 + 2>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-                             : launch_norm<3, 1, 16, EPI_OUT, 320 + 8 + 1>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-    return ln ? launch_norm<3, 1, 16, EPI_OUT, 320 + 16 + 2>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-              : launch_norm<3, 1, 16, EPI_OUT, 320 + 16 + 1>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
+    if (K <= 2048) return ln ? launch_norm_out<320 + 8 + 2>(na, Wp, sw, bias, out, 1, N, K, st)
+                             : launch_norm_out<320 + 8 + 1>(na, Wp, sw, bias, out, 1, N, K, st);
+    return ln ? launch_norm_out<320 + 16 + 2>(na, Wp, sw, bias, out, 1, N, K, st)
+              : launch_norm_out<320 + 16 + 1>(na, Wp, sw, bias, out, 1, N, K, st);
   }
   if (glu)                                  // SwiGLU of [gate | up] (N = 2F): out [1, N / 2]
     return K <= 2048 ? launch_norm<2, 1, 16, EPI_OUT, 192 + 8 + 5>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
                      : launch_norm<2, 1, 16, EPI_OUT, 192 + 16 + 5>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
   if (K <= 2048)
-    return ln ? launch_norm<3, 1, 16, EPI_OUT, 192 + 8 + 2>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-              : launch_norm<3, 1, 16, EPI_OUT, 192 + 8 + 1>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
-  return ln ? launch_norm<3, 1, 16, EPI_OUT, 192 + 16 + 2>(na, Wp, sw, bias, out, nullptr, 1, N, K, st)
-            : launch_norm<3, 1, 16, EPI_OUT, 192 + 16 + 1>(na, Wp, sw, bias, out, nullptr, 1, N, K, st);
+    return ln ? launch_norm_out<192 + 8 + 2>(na, Wp, sw, bias, out, 1, N, K, st)
+              : launch_norm_out<192 + 8 + 1>(na, Wp, sw, bias, out, 1, N, K, st);
+  return ln ? launch_norm_out<192 + 16 + 2>(na, Wp, sw, bias, out, 1, N, K, st)
+            : launch_norm_out<192 + 16 + 1>(na, Wp, sw, bias, out, 1, N, K, st);
 }
 
 // sa: per-token [M] (a_mode 0) or per-group [KT][Mpad] (a_mode 1, M <= 64).

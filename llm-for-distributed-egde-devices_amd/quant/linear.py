@@ -295,8 +295,7 @@ class LLMInt8Linear(nn.Module):
             self.bias.copy_(bias)
 
     def forward(self, x, add=None):
-        out = self._forward(x)
-        return out if add is None else out + add.view_as(out)
+        return self._forward(x, add=add)
 
     def glu_norm(self, x: PendingLN):
         """Batch 1, [gate | up] rows: silu(gate) * up of the projection of RMSNorm(x + residual), one
@@ -318,7 +317,7 @@ class LLMInt8Linear(nn.Module):
             return self._forward(x, act=self._ACT[act])
         return None
 
-    def _forward(self, x, glu: bool = False, act: int = 0):
+    def _forward(self, x, glu: bool = False, act: int = 0, add: Optional[torch.Tensor] = None):
         if isinstance(x, PendingLN):
             y = None
             K, N = self.in_features, self.out_features
@@ -332,12 +331,13 @@ class LLMInt8Linear(nn.Module):
                                         x.weight, x.bias, x.eps, not x.rms, x.h, x.y, self.threshold, self.w_packed,
                                         self._w_deq, self.bias, self._weight_t, self.SCB, N, glu, act)
             if y is not None or glu or act:
-                return y
+                return y if add is None else y + add.view_as(y)
             x = x.materialize()
         if isinstance(x, QAct):
             x = (x.q.float() * x.scale[..., None]).to(torch.bfloat16)
         K, N = self.in_features, self.out_features
         shp = x.shape[:-1]
+        plus = lambda out: out if add is None else out + add.view_as(out)
         x2 = x.reshape(-1, K)
         if x2.is_cuda and ops.gpu_path(x2) and x2.dtype == torch.bfloat16 and self._device_ok():
             # outlier columns found on the device (llmint8.hip), no host sync at any row count
@@ -348,10 +348,12 @@ class LLMInt8Linear(nn.Module):
             x2 = x2.contiguous()
             if x2.shape[0] == 1 and K <= 12288 and K % 64 == 0 and self.ONE_LAUNCH:
                 # batch 1: outlier discovery, quantisation and the outlier part inside the GEMV
+                fuse = add is not None and not act and add.dtype == torch.bfloat16 and add.device == x2.device and \
+                    add.is_contiguous()                     # the other branch's row joins in the epilogue
                 out = C.llmint8_gemv(x2, self.threshold, self.w_packed, self._w_deq, self.bias, self._weight_t,
-                                     self.SCB, N, act)
+                                     self.SCB, N, act, add if fuse else None)
                 if out is not None:
-                    return out.view(*shp, N)
+                    return out.view(*shp, N) if fuse else plus(out.view(*shp, N))
                 if act:
                     return None
             if x2.shape[0] <= self.DECODE_ROWS:
@@ -362,7 +364,7 @@ class LLMInt8Linear(nn.Module):
                 q, sa, cols, count = C.llmint8_prep_rows(x2, self.threshold)
                 out = ops.w8a8_linear(q, sa, self.w_packed, self._w_deq, self.bias, N, K)
                 C.llmint8_outlier_rows(out, x2, cols, count, self._weight_t, self.SCB)
-            return out.view(*shp, N)
+            return plus(out.view(*shp, N))
         cols = (x2.abs() > self.threshold).any(0).nonzero().flatten()
         w_scale = self.SCB / 127.0
         if cols.numel() > 0:
@@ -377,7 +379,7 @@ class LLMInt8Linear(nn.Module):
                               w_ref=None if q.is_cuda else self.weight_i8, out_dtype=x.dtype)
         if out_o is not None:
             out = (out.float() + out_o.float()).to(out.dtype)
-        return out.view(*shp, N)
+        return plus(out.view(*shp, N))
 
     def extra_repr(self):
         return f"{self.in_features}->{self.out_features}, LLM.int8 threshold={self.threshold}"
