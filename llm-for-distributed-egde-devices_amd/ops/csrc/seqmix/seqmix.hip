@@ -1108,6 +1108,11 @@ int edge_sm_attention_mfma_rel(const void* q, const void* gate, int gate_ld, con
                                const float* sink, int keep_first, const float* rel, int rel_n, int out_ld, float out_scale, int rh,
                                hipStream_t st);
 
+int edge_sm_attention_latent(const void* q, const void* gate, int gate_ld, const void* kp, const int* seq_slot,
+                             const int* seq_start, const int* seq_len, const int* seq_off, const int* ptab, int ptab_ld,
+                             void* out, int n, int qtiles, int H, int G, int D, int Dv, float scale_log2, int window, int kld,
+                             int out_ld, float out_scale, hipStream_t st);
+
 // bf16 prompt portions on the matrix cores; returns 1 when no instantiation takes (D, Dv): the caller
 // then runs the general kernel
 int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp,
@@ -1186,28 +1191,18 @@ int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const v
   dim3(NT), 0, st, (const bf16_t*)q, (const bf16_t*)gate, gate_ld, (const bf16_t*)kp, (const bf16_t*)vp, kb, vb,     \
       seq_slot, seq_start, seq_len, seq_off, ptab, ptab_ld, (bf16_t*)out, n, H, G, PB, sl2, window, pool, kld, vld,  \
       out_ld, out_scale
-#define SM_MF_R(DK, DV, RH, KVS) \
-  hipLaunchKernelGGL((attn_mfma_kernel<DK, DV, RH, KVS>), dim3(qtiles, H / RH), SM_MF_ARGS)
-#define SM_MF(DK, DV)                             \
-  do {                                            \
-    if (rh == 4) SM_MF_R(DK, DV, 4, false);       \
-    else if (rh == 2) SM_MF_R(DK, DV, 2, false);  \
-    else SM_MF_R(DK, DV, 1, false);               \
+#define SM_MF_R(DK, DV, RH) \
+  hipLaunchKernelGGL((attn_mfma_kernel<DK, DV, RH, false>), dim3(qtiles, H / RH), SM_MF_ARGS)
+#define SM_MF(DK, DV)                    \
+  do {                                   \
+    if (rh == 4) SM_MF_R(DK, DV, 4);     \
+    else if (rh == 2) SM_MF_R(DK, DV, 2);\
+    else SM_MF_R(DK, DV, 1);             \
   } while (0)
-#define SM_MFK(DK, DV)                            \
-  do {                                            \
-    if (rh == 4) SM_MF_R(DK, DV, 4, true);        \
-    else if (rh == 2) SM_MF_R(DK, DV, 2, true);   \
-    else SM_MF_R(DK, DV, 1, true);                \
-  } while (0)
-  if (kvs) {                                                 // latent rows: latent | shared key part, value = the latent
-    if (D == 128 && Dv == 96) SM_MFK(4, 6);
-    else if (D == 160 && Dv == 128) SM_MFK(5, 8);
-    else if (D == 192 && Dv == 128) SM_MFK(6, 8);
-    else if (D == 320 && Dv == 256) SM_MF_R(10, 16, 1, true);   // one head per workgroup: its output tile fills the registers
-    else return 1;
-  }
-  else if (D == 64 && Dv == 64) SM_MF(2, 4);
+  if (kvs)                                                   // latent rows: latent | shared key part, value = the latent
+    return edge_sm_attention_latent(q, gate, gate_ld, kp, seq_slot, seq_start, seq_len, seq_off, ptab, ptab_ld, out, n, qtiles,
+                                    H, G, D, Dv, sl2, window, kld, out_ld, out_scale, st);
+  if (D == 64 && Dv == 64) SM_MF(2, 4);
   else if (D == 96 && Dv == 96) SM_MF(3, 6);
   else if (D == 128 && Dv == 128) SM_MF(4, 8);
   else if (D == 128 && Dv == 64) SM_MF(4, 4);
@@ -1215,7 +1210,6 @@ int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const v
   else if (D == 32 && Dv == 32) SM_MF(1, 2);
   else return 1;
 #undef SM_MF
-#undef SM_MFK
 #undef SM_MF_R
 #undef SM_MF_ARGS
   return (int)hipGetLastError();
