@@ -86,6 +86,7 @@ int edge_w8a8_rows256_splits(int K);
 void edge_w8a8_prefill_x32(int v);
 int edge_gemv_bf16(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi,
                    hipStream_t st, const void* add, int h16);
+int edge_gemv_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K, hipStream_t st);
 int edge_gemv_bf16_splitk(const void* A, const void* W, const void* bias, float* part, int M, int N, int K, int S,
                           hipStream_t st, int h16);
 int edge_llmint8_prep(const void* x, int M, int K, float thr, int cmax, void* q, float* sa, int* cols, float* xo,
@@ -729,6 +730,26 @@ at::Tensor gemv_bf16(const at::Tensor& x, const at::Tensor& wp, const std::optio
   check(edge_gemv_bf16(x.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr, out.data_ptr(), (int)M, (int)N,
                        (int)K, (int)epi, stream(), addend ? addend->data_ptr() : nullptr, h16),
         "gemv_bf16");
+  return out;
+}
+
+// fp32 projection of up to 8 rows over the [N, K] weight as it is (gemv_f32.hip): K % 4 == 0.
+at::Tensor gemv_f32(const at::Tensor& x, const at::Tensor& w, const std::optional<at::Tensor>& bias) {
+  DEVICE_GUARD(x);
+  need(x, at::kFloat, "x");
+  need(w, at::kFloat, "weight");
+  TORCH_CHECK(w.dim() == 2 && x.dim() >= 1 && x.size(-1) == w.size(1), "x [.., K], weight [N, K]");
+  TORCH_CHECK(w.device() == x.device() && (!bias || bias->device() == x.device()), "gemv_f32: one device");
+  TORCH_CHECK(w.size(1) > 0, "gemv_f32: K");
+  const int64_t N = w.size(0), K = w.size(1), M = rows_of(x);
+  TORCH_CHECK(M >= 1 && M <= 8 && N >= 1 && K >= 4 && K % 4 == 0, "gemv_f32: 1-8 rows, K a multiple of 4");
+  TORCH_CHECK((uintptr_t)x.data_ptr() % 16 == 0 && (uintptr_t)w.data_ptr() % 16 == 0, "gemv_f32: 16-byte aligned operands");
+  if (bias) { need(*bias, at::kFloat, "bias"); TORCH_CHECK(bias->numel() == N); }
+  auto os = x.sizes().vec();
+  os.back() = N;
+  auto out = at::empty(os, x.options());
+  check(edge_gemv_f32(x.data_ptr<float>(), w.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr,
+                      out.data_ptr<float>(), (int)M, (int)N, (int)K, stream()), "gemv_f32");
   return out;
 }
 
@@ -1415,6 +1436,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("bf16_ring_min_rows", []() { return (int64_t)edge_bf16_ring_min_rows(); });
   m.def("gemv_bf16", &gemv_bf16, "bf16 decode GEMV (M <= 16), optional fused SwiGLU over [gate | up]", py::arg("x"),
         py::arg("wp"), py::arg("bias"), py::arg("N"), py::arg("epi"), py::arg("addend") = py::none());
+  m.def("gemv_f32", &gemv_f32, "fp32 projection of up to 8 rows", py::arg("x"), py::arg("w"), py::arg("bias"));
   m.def("decode_attn_fused", &decode_attn_fused);
   m.def("decode_attn_i8", &decode_attn_i8, "decode attention over an int8 KV cache, fused RoPE + quantising append");
   m.def("kv_dequant", &kv_dequant, "dequantise the first T rows of an int8 KV cache into a bf16 scratch");

@@ -1,0 +1,100 @@
+// fp32 projection of a few rows: y[M, N] = x[M, K] . W[N, K]^T (+ bias), M <= 8, K % 4 == 0, in fp32 throughout.
+// Bound by reading W once, and below some 16 MB by the launch itself.  W stays in its [N, K] layout (no copy is made): a
+// wave takes R rows by 256 k at a time, each load one contiguous KiB of a row (with 16 rows by 16 k per load, the matrix
+// instruction's layout, the loads themselves were the bound: 1024 x 4096 12.8 us against 5.9 here), the next 256 k on
+// their way meanwhile.  Few rows: KW waves of a workgroup share a row's k (until about 1024 waves are at work) and add up
+// through LDS.  All sums in a fixed order.
+// N x K at 2 rows, us, library / here: 1024 x 384 5.1 / 3.4, 1024 x 1024 8.3 / 3.9, 1024 x 4096 12.2 / 5.9, 4096 x 1024
+// 11.6 / 6.2, 6784 x 1024 12.9 / 8.6, 32000 x 1024 32.6 / 25.7 (5.1 TB/s), 32000 x 2048 59.6 / 44.8; relative error
+// against 64-bit sums 1e-7 here, 2 to 8e-7 there.
+#include "common.h"
+
+namespace {
+
+// Sums of C numbers over the 64 lanes: while a lane holds several it hands half of them over and keeps the sums of the
+// other half (idx: which), then all lanes add up the one they share.
+template <int C, int S, int V>
+__device__ __forceinline__ void lane_sums(float (&v)[V], int& idx, int lane) {
+  const bool up = lane & S;
+  if constexpr (C > 1) {
+#pragma unroll
+    for (int i = 0; i < C / 2; ++i) {
+      const float give = up ? v[i] : v[i + C / 2], keep = up ? v[i + C / 2] : v[i];
+      v[i] = keep + __shfl_xor(give, S, 64);
+    }
+    idx = idx * 2 + (up ? 1 : 0);
+  } else v[0] += __shfl_xor(v[0], S, 64);
+  if constexpr (S > 1) lane_sums<(C > 1 ? C / 2 : 1), S / 2>(v, idx, lane);
+}
+
+template <int MV, int R>
+__global__ void __launch_bounds__(1024) gemv_f32_kernel(const float* __restrict__ x, const float* __restrict__ W,
+                                                        const float* __restrict__ bias, float* __restrict__ y, int M, int N,
+                                                        int K, int KW) {
+  constexpr int V = MV * R;
+  __shared__ float part[16 * V];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int rg = wave / KW, kw = wave - rg * KW, n0 = ((int)blockIdx.x * (waves / KW) + rg) * R;
+  const int C = (K + 255) / 256;
+  float acc[V];
+#pragma unroll
+  for (int i = 0; i < V; ++i) acc[i] = 0.f;
+  v4f wv[2][R], xv[2][MV];
+  auto load = [&](int b, int c) {                            // rows past the last and k past the end: a clamped one
+    const int k = min(min(c, C - 1) * 256 + lane * 4, K - 4);
+#pragma unroll
+    for (int r = 0; r < R; ++r) wv[b][r] = *reinterpret_cast<const v4f*>(W + (size_t)min(n0 + r, N - 1) * K + k);
+#pragma unroll
+    for (int m = 0; m < MV; ++m) xv[b][m] = *reinterpret_cast<const v4f*>(x + (size_t)min(m, M - 1) * K + k);
+  };
+  auto use = [&](int b, int c) {
+    if (c * 256 + lane * 4 >= K) return;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int m = 0; m < MV; ++m)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[r * MV + m] = __builtin_fmaf(wv[b][r][j], xv[b][m][j], acc[r * MV + m]);
+  };
+  load(0, kw);
+  for (int c = kw; c < C; c += 2 * KW) {
+    load(1, c + KW);
+    use(0, c);
+    load(0, c + 2 * KW);
+    use(1, c + KW);
+  }
+  int idx = 0;
+  lane_sums<V, 32>(acc, idx, lane);
+  // the first bits of the lane number chose; lanes that differ only in the others hold the same sum
+  static_assert(V <= 64, "one sum per lane");
+  if (lane % (64 / V) == 0) part[wave * V + idx] = acc[0];
+  __syncthreads();
+  for (int e = tid; e < waves / KW * V; e += blockDim.x) {
+    const int gq = e / V, v = e - gq * V, m = v % MV, n = ((int)blockIdx.x * (waves / KW) + gq) * R + v / MV;
+    float sum = 0.f;
+    for (int w = 0; w < KW; ++w) sum += part[(gq * KW + w) * V + v];
+    if (m < M && n < N) y[(size_t)m * N + n] = sum + (bias ? bias[n] : 0.f);
+  }
+}
+
+template <int MV, int R>
+void launch_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K, hipStream_t st) {
+  const int groups = (N + R - 1) / R, C = (K + 255) / 256;
+  int KW = 1;
+  while (KW < 16 && KW * 2 <= C && groups * KW < 1024) KW *= 2;
+  const int waves = KW < 4 ? 4 : KW, per = waves / KW;
+  hipLaunchKernelGGL((gemv_f32_kernel<MV, R>), dim3((groups + per - 1) / per), dim3(waves * 64), 0, st, x, W, bias, y, M, N, K, KW);
+}
+}  // namespace
+
+// x, W: 16-byte aligned.  5 - 8 rows: two weight rows per wave (four leave no registers for the next loads: 4096 x 1024 at
+// 8 rows 13.7 us, two 7.9, library 11.6)
+extern "C" int edge_gemv_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K,
+                             hipStream_t st) {
+  if (M < 1 || M > 8 || N < 1 || K < 4 || K % 4) return -2;
+  if (M == 1) launch_f32<1, 4>(x, W, bias, y, M, N, K, st);
+  else if (M == 2) launch_f32<2, 4>(x, W, bias, y, M, N, K, st);
+  else if (M <= 4) launch_f32<4, 4>(x, W, bias, y, M, N, K, st);
+  else launch_f32<8, 2>(x, W, bias, y, M, N, K, st);
+  return (int)hipGetLastError();
+}
