@@ -9,24 +9,6 @@
 
 namespace {
 
-// 4 consecutive elements (16 or 8 bytes)
-template <typename T> __device__ __forceinline__ void load4(const T* p, float* f);
-template <> __device__ __forceinline__ void load4<float>(const float* p, float* f) {
-  const float4 a = *reinterpret_cast<const float4*>(p);
-  f[0] = a.x; f[1] = a.y; f[2] = a.z; f[3] = a.w;
-}
-template <> __device__ __forceinline__ void load4<bf16_t>(const bf16_t* p, float* f) {
-  const uint2 a = *reinterpret_cast<const uint2*>(p);
-  f[0] = __uint_as_float(a.x << 16); f[1] = __uint_as_float(a.x & 0xffff0000u);
-  f[2] = __uint_as_float(a.y << 16); f[3] = __uint_as_float(a.y & 0xffff0000u);
-}
-template <typename T> __device__ __forceinline__ void store4(T* p, const float* f);
-template <> __device__ __forceinline__ void store4<float>(float* p, const float* f) {
-  *reinterpret_cast<float4*>(p) = make_float4(f[0], f[1], f[2], f[3]);
-}
-template <> __device__ __forceinline__ void store4<bf16_t>(bf16_t* p, const float* f) {
-  *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf2(f[0], f[1]), pack_bf2(f[2], f[3]));
-}
 // C elements: 4 with wide accesses or 1
 template <typename T, int C> __device__ __forceinline__ void loadc(const T* p, float* f) {
   if constexpr (C == 4) load4<T>(p, f);

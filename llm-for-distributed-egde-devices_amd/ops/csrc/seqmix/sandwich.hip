@@ -7,6 +7,7 @@
 // Storage is fp32 or bf16 (template T); the norms, the router weights, decays and beta are fp32 in both.
 #include "common.h"
 #include "seqmix/seqmix_common.h"
+#include "seqmix/delta_prep.h"
 
 namespace {
 
@@ -214,6 +215,10 @@ int edge_sm_delta_prep_head(const void* qkv, int Cq, const void* u, int ld, int 
                             const float* A_log, float* prep, int rows, int H, int G, int N, int f32, hipStream_t st) {
   if (rows == 0) return 0;
   if (G <= 0 || H % G) return -2;
+  bool took;
+  SM_T(f32, (took = launch_delta_prep16<T, true>((const T*)qkv, Cq, (const T*)u, ld, b0, a0, nullptr, dt_bias, A_log, prep, rows,
+                                                 H, G, N, st)));
+  if (took) return (int)hipGetLastError();
   SM_T(f32, hipLaunchKernelGGL(delta_prep_head_kernel<T>, dim3(rows), dim3(NT), 0, st, (const T*)qkv, Cq, (const T*)u, ld,
                                b0, a0, dt_bias, A_log, prep, H, G, N));
   return (int)hipGetLastError();
