@@ -11,22 +11,6 @@
 
 namespace {
 
-// Sums of C numbers over the 64 lanes: while a lane holds several it hands half of them over and keeps the sums of the
-// other half (idx: which), then all lanes add up the one they share.
-template <int C, int S, int V>
-__device__ __forceinline__ void lane_sums(float (&v)[V], int& idx, int lane) {
-  const bool up = lane & S;
-  if constexpr (C > 1) {
-#pragma unroll
-    for (int i = 0; i < C / 2; ++i) {
-      const float give = up ? v[i] : v[i + C / 2], keep = up ? v[i + C / 2] : v[i];
-      v[i] = keep + __shfl_xor(give, S, 64);
-    }
-    idx = idx * 2 + (up ? 1 : 0);
-  } else v[0] += __shfl_xor(v[0], S, 64);
-  if constexpr (S > 1) lane_sums<(C > 1 ? C / 2 : 1), S / 2>(v, idx, lane);
-}
-
 template <int MV, int R>
 __global__ void __launch_bounds__(1024) gemv_f32_kernel(const float* __restrict__ x, const float* __restrict__ W,
                                                         const float* __restrict__ bias, float* __restrict__ y, int M, int N,

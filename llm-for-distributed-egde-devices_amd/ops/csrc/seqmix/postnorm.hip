@@ -15,6 +15,7 @@
 #include "common.h"
 #include "seqmix/seqmix_common.h"
 #include "seqmix/delta_prep.h"
+#include "seqmix/moe_rows.h"
 #include "seqmix/tap4.h"
 
 namespace {
@@ -1025,6 +1026,13 @@ int edge_sm_moe_experts(const void* h, int W, const int* idx, int top, const voi
                         hipStream_t st) {
   if (rows == 0) return 0;
   if ((size_t)W * 4 > 60 * 1024 || (size_t)ff * 4 > 60 * 1024) return -3;
+  if ((!f32 || rows == 1) && moe_rows_ok(W, ff, {h, w_gu, w_down, y, out})) {
+    SM_T(f32, (launch_moe_rows<T, MR_GLU>((const T*)h, nullptr, idx, rows * top, rows * top, top, (const T*)w_gu, nullptr, W, ff, 0,
+                                          0, E, limit, silu, in_w, (T*)y, nullptr, st),
+               launch_moe_rows<T, MR_PLAIN>((const T*)y, nullptr, idx, rows * top, rows * top, top, (const T*)w_down, nullptr, ff,
+                                            W, 0, 0, E, 0.f, 0, nullptr, (T*)out, nullptr, st)));
+    return (int)hipGetLastError();
+  }
   const int rpw = 16;
   SM_T(f32, hipLaunchKernelGGL(moe_gate_up_kernel<T>, dim3(rows * top, (ff + rpw - 1) / rpw), dim3(NT), (size_t)W * 4, st,
                                (const T*)h, W, idx, top, (const T*)w_gu, ff, limit, (T*)y, rpw, E, silu, in_w));
@@ -1058,6 +1066,13 @@ int edge_sm_moe_experts_relu2(const void* h, int W, const int* idx, int top, con
   const int big = sff > ff ? sff : ff;
   if ((size_t)W * 4 > 60 * 1024 || (size_t)big * 4 > 60 * 1024) return -3;
   const int rpw = 16, routed = rows * top, pairs = routed + (sff > 0 ? rows : 0);
+  if ((!f32 || rows == 1) && ff % 8 == 0 && moe_rows_ok(W, sff, {h, w_up, w_down, su, sd, y, ys, out, out_sh})) {
+    SM_T(f32, (launch_moe_rows<T, MR_RELU2>((const T*)h, (const T*)h, idx, routed, pairs, top, (const T*)w_up, (const T*)su, W, ff,
+                                            W, sff, E, 0.f, 0, nullptr, (T*)y, (T*)ys, st),
+               launch_moe_rows<T, MR_PLAIN>((const T*)y, (const T*)ys, idx, routed, pairs, top, (const T*)w_down, (const T*)sd, ff,
+                                            W, sff, W, E, 0.f, 0, nullptr, (T*)out, (T*)out_sh, st)));
+    return (int)hipGetLastError();
+  }
   SM_T(f32, hipLaunchKernelGGL((relu2_experts_kernel<T, true>), dim3(pairs, (big + rpw - 1) / rpw), dim3(NT), (size_t)W * 4, st,
                                (const T*)h, (const T*)h, idx, routed, top, (const T*)w_up, (const T*)su, W, ff, sff, (T*)y,
                                (T*)ys, rpw, E));

@@ -1,0 +1,53 @@
+"""Experts of decode-sized steps (moe_rows.h) against the same op in fp32 on the CPU: every count of tokens per expert that
+the shared readings distinguish (1, 2, 3, 4, 5 and all), widths beside a wave's 512 and 1024 numbers and a workgroup's rows,
+repeated and out-of-range choices, more pairs than one ballot names, the shared expert, widths of the general kernels."""
+import pytest
+import torch
+
+import edgellm.ops.seqmix as S
+
+pytestmark = pytest.mark.gpu
+
+CHOICES = {
+    "one": [[2, 0]],
+    "apart": [[0, 1], [2, 3], [4, 5]],
+    "pairs": [[0, 1], [1, 2], [2, 0]],
+    "three": [[3, 0], [3, 1], [0, 3]],
+    "five": [[1, 0], [1, 2], [3, 1], [1, 4], [5, 1]],
+    "all": [[4, 4], [4, 4], [4, 4], [4, 4], [4, -7], [99, 4]],
+    "many": [[i % 6, (i * 5 + 1) % 6] for i in range(40)],
+}
+
+
+def _operands(dt, W, ff, top, T, act, seed):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(dt)
+    return r(T, W), r(6, ff if act == "relu2" else 2 * ff, W), r(6, W, ff), torch.rand(T, top, generator=g) + 0.5, r(ff + 8, W), r(W, ff + 8)
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("name", list(CHOICES))
+@pytest.mark.parametrize("W,ff,act", [(8, 8, "glu_clamp"), (520, 24, "silu_glu"), (1024, 520, "silu_w"), (1032, 16, "glu_clamp"),
+                                      (2056, 40, "silu_glu"), (512, 1032, "relu2"), (1024, 20, "silu_glu"), (20, 64, "relu2")])
+def test_decode_sized_experts(dt, name, W, ff, act):
+    T = len(CHOICES[name])
+    if dt == torch.bfloat16 and S.MOE_MFMA_MIN <= T:
+        pytest.skip("the grouped kernels' size")
+    h, w_gu, w_down, in_w, su, sd = _operands(dt, W, ff, 2, T, act, T + W)
+    idx = torch.tensor(CHOICES[name], dtype=torch.int32)
+    op, in_w = ("silu_glu", in_w) if act == "silu_w" else (act, None)
+    cuda = lambda x: None if x is None else x.cuda()
+    got = S.moe_experts(h.cuda(), idx.cuda(), w_gu.cuda(), w_down.cuda(), 1.5, op, cuda(in_w)).float().cpu()
+    f = lambda x: x.float()
+    ref = S.moe_experts(f(h), idx.clamp(0, 5), f(w_gu), f(w_down), 1.5, op, in_w)
+    # the inner row is rounded to dt before the second product: ff terms of at most 2^-8 (2^-24) of their size each
+    u = torch.stack([torch.stack([f(w_down)[e].abs() @ torch.ones(ff) for e in row.clamp(0, 5)]) for row in idx])
+    inner = S.moe_experts(f(h), idx.clamp(0, 5), f(w_gu), torch.eye(ff).repeat(6, 1, 1), 1.5, op, in_w).abs().amax(-1, keepdim=True)
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20
+    assert ((got - ref).abs() <= eps * (ref.abs() + u * inner) + 1e-6).all()
+    if act == "relu2":
+        o, o_sh = S.moe_experts_shared(h.cuda(), idx.cuda(), w_gu.cuda(), w_down.cuda(), su.cuda(), sd.cuda())
+        y = S.relu2(f(h) @ f(su).t())
+        sh = y @ f(sd).t()
+        assert torch.equal(o.float().cpu(), got)
+        assert ((o_sh.float().cpu() - sh).abs() <= eps * (sh.abs() + f(sd).abs().sum(1) * y.amax(-1, keepdim=True)) + 1e-6).all()
