@@ -700,10 +700,14 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, int H, int8_t* aq,
     }
     take[c] = bits;
     incl[c] = __popc(bits);
+    // outliers are few: most waves' runs have none to rank (a plain row of two chunks is faster without the branch: 2560 x
+    // 2560 11.7 us with it, 6.0 without; 2560 x 10240 10.1 with it, 11.1 without)
+    if ((SRC == 0 && NCH <= 2) || __any(bits != 0)) {
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-      const int tt = __shfl_up(incl[c], o, 64);
-      if (lane >= o) incl[c] += tt;
+      for (int o = 1; o < 64; o <<= 1) {
+        const int tt = __shfl_up(incl[c], o, 64);
+        if (lane >= o) incl[c] += tt;
+      }
     }
     if (act && lane == 63) scr[c * 4 + w] = incl[c];
   }
@@ -1796,26 +1800,39 @@ int launch_one(const void* A, const float* sa, const void* Wp, const float* sw, 
   return (int)hipGetLastError();
 }
 
-template <int NTW, int TG, int KW, int EP, int NRM>
+template <int NTW, int TG, int KW, int EP, int NRM, int U = 2>
 int launch_norm(const NormIn& na, const void* Wp, const float* sw, const void* bias, void* out, float* os, int M,
                 int N, int K, hipStream_t st) {
   const int NTt = (N + 15) / 16;
-  hipLaunchKernelGGL((w8a8_gemv_kernel<1, NTW, TG, KW, 2, A_TOKEN, EP, NRM>), dim3((NTt + NTW - 1) / NTW),
+  hipLaunchKernelGGL((w8a8_gemv_kernel<1, NTW, TG, KW, U, A_TOKEN, EP, NRM>), dim3((NTt + NTW - 1) / NTW),
                      dim3(TG * KW * 64), 0, st, (const int8_t*)nullptr, (const float*)nullptr, (const int8_t*)Wp, sw,
                      (const bf16_t*)bias, out, os, M, N, K, K / 64, NTt, 16, 1, na);   // Mpad 16: scales [N/128][16]
   return (int)hipGetLastError();
 }
 
 // One row over plain outputs: as many 16-column tiles per workgroup as keep the launch to about one round of the 256
-// CUs: with fewer, the launch waits on a few CUs' own read rate.  LLM.int8 at batch 1, us per launch, three tiles always
-// / this rule with the ranking at one barrier: N x K 2560 x 10240 18.8 / 11.2, 2560 x 2560 8.5 / 6.2, 7680 x 2560 10.4 /
-// 9.1; 10240 x 2560 (three tiles either way) 10.2 / 9.3.  W8A8 behind LayerNorm 2048 x 2048 5.7 / 4.7, 6144 x 2048 6.3 /
-// 5.5, 7680 x 2560 8.3 / 7.7; behind RMSNorm 4096 x 4096 8.0 / 6.1, 6144 x 4096 8.4 / 7.3, 12288 x 4096 11.5 / 11.5.
+// CUs (with fewer, the launch waits on a few CUs' own read rate), and as many k-tiles in flight per wave (U) as leave one
+// or two rounds of loads: K = 2560 has 2.5 k-tiles a wave, K > 4096 more than four.  us per launch, three tiles and two
+// k-tiles always / this rule, LLM.int8 with the ranking at one barrier: N x K 2560 x 10240 18.8 / 10.2, 2560 x 2560 8.5 /
+// 6.0, 7680 x 2560 10.4 / 8.8, 10240 x 2560 10.2 / 9.1.  W8A8 behind LayerNorm 2048 x 2048 5.7 / 4.7, 6144 x 2048 6.3 / 5.5,
+// 2560 x 2560 7.4 / 5.5, 7680 x 2560 8.3 / 7.2; behind RMSNorm 4096 x 4096 8.0 / 6.1, 6144 x 4096 8.4 / 7.3, 12288 x 4096
+// 11.5 / 11.5.
 template <int NRM>
 int launch_norm_out(const NormIn& na, const void* Wp, const float* sw, const void* bias, void* out, int M, int N, int K,
                     hipStream_t st) {
   const int NTt = (N + 15) / 16;
-  if (NTt <= 256) return launch_norm<1, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+  constexpr int NCH = NRM % 64 / 8;
+  if (NTt <= 256) {
+    if constexpr (NCH >= 3) return launch_norm<1, 1, 16, EPI_OUT, NRM, 5>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+    else if constexpr (NCH == 2) {
+      if (K <= 3072) return launch_norm<1, 1, 16, EPI_OUT, NRM, 3>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+    }
+    return launch_norm<1, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+  }
+  if constexpr (NCH == 2) {
+    if (K <= 3072 && NTt <= 512) return launch_norm<2, 1, 16, EPI_OUT, NRM, 3>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+    if (K <= 3072) return launch_norm<3, 1, 16, EPI_OUT, NRM, 3>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
+  }
   if (NTt <= 512) return launch_norm<2, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
   return launch_norm<3, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
 }
