@@ -631,6 +631,47 @@ __global__ void __launch_bounds__(NT) moe_logits_kernel(const T* __restrict__ h,
   if (lane == 0) z[t * E + e] = acc + (bias ? bias[e] : 0.f);
 }
 
+// The same for prompt-sized steps, four tokens by four experts per wave: the router's rows are read once per four tokens
+// (they were the bound: E x W fp32 numbers a token) and the sums are those of one wave per pair, bit for bit (the same chain
+// per lane, the same pairs of lanes).  us: 32 experts, 7680 tokens of 2048 103 / 46; 16 experts, 4096 of 1024 16.2 / 8.5; below 64 tokens one wave per pair is as
+// fast and has the shorter chain.
+template <typename T>
+__global__ void __launch_bounds__(NT) moe_logits16_kernel(const T* __restrict__ h, int W, const float* __restrict__ router,
+                                                          int E, float* __restrict__ z, const float* __restrict__ bias,
+                                                          int rows) {
+  const int lane = threadIdx.x & 63, t0 = blockIdx.x * 4, e0 = (blockIdx.y * (NT / 64) + (threadIdx.x >> 6)) * 4;
+  if (e0 >= E) return;
+  float acc[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i) acc[i] = 0.f;
+  for (int c = lane * 8; c < W; c += 64 * 8) {
+    float a[4][8], r[4][8];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      load8<T>(h + (size_t)min(t0 + i, rows - 1) * W + c, a[i]);
+      load8<float>(router + (size_t)min(e0 + i, E - 1) * W + c, r[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc[i * 4 + j] += a[i][k] * r[j][k];
+  }
+  int id = 0;
+  lane_sums<16, 32>(acc, id, lane);
+  const int t = t0 + id / 4, e = e0 + id % 4;
+  if (lane % 4 == 0 && t < rows && e < E) z[(size_t)t * E + e] = acc[0] + (bias ? bias[e] : 0.f);
+}
+
+template <typename T>
+void launch_moe_logits(const T* h, int W, const float* router, int E, float* z, const float* bias, int rows, hipStream_t st) {
+  if (rows >= 64 && W % 8 == 0)
+    hipLaunchKernelGGL(moe_logits16_kernel<T>, dim3((rows + 3) / 4, (E + 15) / 16), dim3(NT), 0, st, h, W, router, E, z, bias, rows);
+  else
+    hipLaunchKernelGGL(moe_logits_kernel<T>, dim3(rows, (E + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st, h, W, router, E, z, bias);
+}
+
 // One wave per token: softmax over the experts' scores, then the `top` largest (lowest index on a tie),
 // divided by their sum (+ 1e-20) and multiplied by scale.  sigm: the scores are sigmoid(z) and the `top`
 // largest keep their own value (times scale); they are picked by z itself (the same order), so scores that
@@ -1014,8 +1055,7 @@ int edge_sm_moe_route(const void* h, int W, const float* router, const float* bi
                       int* idx, float* wts, int rows, int sigm, int f32, hipStream_t st) {
   if (rows == 0) return 0;
   if (top < 1 || top > E || top > 64 || E > 8192) return -2;
-  SM_T(f32, hipLaunchKernelGGL(moe_logits_kernel<T>, dim3(rows, (E + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st, (const T*)h,
-                               W, router, E, z, bias));
+  SM_T(f32, launch_moe_logits<T>((const T*)h, W, router, E, z, bias, rows, st));
   hipLaunchKernelGGL(moe_topk_kernel, dim3(rows), dim3(64), (size_t)E * 4, st, (const float*)z, E, top, scale, idx, wts, sigm);
   return (int)hipGetLastError();
 }
@@ -1049,8 +1089,7 @@ int edge_sm_moe_route_grouped(const void* h, int W, const float* router, int E, 
   if (E < 1 || groups < 1 || E % groups || keep < 1 || keep > groups || top < 1 || top > 64 || top > E / groups * keep ||
       E > 4096 || (gate && !gate_w))
     return -2;
-  SM_T(f32, hipLaunchKernelGGL(moe_logits_kernel<T>, dim3(rows, (E + gate + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st,
-                               (const T*)h, W, router, E + gate, z, (const float*)nullptr));
+  SM_T(f32, launch_moe_logits<T>((const T*)h, W, router, E + gate, z, nullptr, rows, st));
   hipLaunchKernelGGL(route_grouped_kernel, dim3(rows), dim3(64), (size_t)(2 * E + groups) * 4, st, (const float*)z, E, gate,
                      corr, groups, keep, top, scale, idx, wts, gate_w);
   return (int)hipGetLastError();

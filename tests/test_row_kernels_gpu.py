@@ -90,3 +90,16 @@ def test_latent_write(dt, H, D, R, kvr, rot):
         res.append((qc.reshape(10, -1), pages))
     _near(res[0][0], res[1][0].cpu(), dt)
     _near(res[0][1], res[1][1].cpu(), dt)
+
+
+@pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("T,E,W,bias", [(64, 16, 1024, False), (67, 5, 520, True), (130, 33, 2048, False), (65, 1, 8, True), (66, 16, 1030, False)])
+def test_router_scores_of_prompts(dt, T, E, W, bias):
+    """From 64 tokens on four tokens share the router's rows: the same choices and weights, bit for bit, as in small steps."""
+    g = torch.Generator().manual_seed(E)
+    h, router = _rand(g, T, W).to(dt).cuda(), _rand(g, E, W).cuda()
+    b = _rand(g, E).cuda() if bias else None
+    top = min(3, E)
+    idx, wts = S.moe_route(h, router, top, 1.5, "softmax", b)
+    small = [S.moe_route(h[a:a + 63].contiguous(), router, top, 1.5, "softmax", b) for a in range(0, T, 63)]
+    assert torch.equal(idx, torch.cat([s[0] for s in small])) and torch.equal(wts, torch.cat([s[1] for s in small]))
