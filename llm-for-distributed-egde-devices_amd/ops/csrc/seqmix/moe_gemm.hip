@@ -12,7 +12,7 @@
 // Measured (both products, sorting and activation; MI355X) against one library product per expert with the sort, the
 // gather, the activation and the scatter as launches of their own: 4096 tokens x 3 of 16 experts 1024 -> 1024,
 // 758 -> 129 us (600 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 790 us (734); 512 x 4 of 32, 2048 -> 2048,
-// 1369 -> 238 us, where the experts' 805 MB (3.4 TB/s) are the bound.  At 128-row tiles the bound is the operands' way
+// 1369 -> 212 us, where the experts' 805 MB (3.8 TB/s) are the bound.  At 128-row tiles the bound is the operands' way
 // into the LDS (64 B per clock and CU at the full MFMA rate): 128 x 256 tiles gain 3-6 % from 2048 columns on and lose
 // below, deeper rings with one workgroup per CU lose 40 %.
 #include "seqmix_common.h"
@@ -103,7 +103,7 @@ template <int BM, int BN, int WM, int WN, int R, int ACT, bool GATHER>
 __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                                   const int* __restrict__ rows, const int* __restrict__ tiles,
                                                                   bf16_t* __restrict__ out, int top, int N, int NW, int K,
-                                                                  int grid_n, const float* __restrict__ row_w, float limit) {
+                                                                  int grid_n, const float* __restrict__ row_w, float limit, int spread) {
   constexpr bool GLU = ACT == ACT_GLU_CLAMP || ACT == ACT_GLU_SILU;
   constexpr int NWV = WM * WN, AP = BM / 8, BP = BN / 8, PIECES = AP + BP, PPW = PIECES / NWV, STAGE = PIECES * 1024;
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;
@@ -149,8 +149,12 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
     src[i] = reinterpret_cast<const char*>(base + row * (size_t)K) + ck;
   }
   // stages past the last re-load the last one into a slot that is not read again: the counts stay constant
+  // spread: column blocks and experts start at different k and go round.  In step, every workgroup reads the same 128 bytes
+  // of rows 2 K bytes apart, which lie in few memory channels
+  const int k0 = spread ? (tile.x * 7 + bn * 5) % KT : 0;
   auto issue = [&](int st) {
-    const size_t ko = (size_t)min(st, KT - 1) * 128;
+    const int kt = min(st, KT - 1) + k0;
+    const size_t ko = (size_t)(kt < KT ? kt : kt - KT) * 128;
     int8_t* slot = ring + (st % R) * STAGE + wave * 1024;
 #pragma unroll
     for (int i = 0; i < PPW; ++i) glds16(src[i] + ko, slot + NWV * i * 1024);
@@ -238,19 +242,19 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
 
 template <int BM, int BN, int WM, int WN, int R>
 int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* rows, const int* tiles, void* y, void* out,
-                int max_tiles, int top, int W, int ff, int act, const float* row_w, float limit, hipStream_t st) {
+                int max_tiles, int top, int W, int ff, int act, const float* row_w, float limit, int spread, hipStream_t st) {
   const dim3 blk(64 * WM * WN);
   const int up = act == ACT_RELU2 ? 1 : 2, fn = act == ACT_RELU2 ? BN : BN / 2;
   const int g1 = (ff + fn - 1) / fn, g2 = (W + BN - 1) / BN;
 #define MOE_FIRST(ACT)                                                                                                     \
   hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, ACT, true>), dim3(max_tiles * g1), blk, 0, st, (const bf16_t*)h,  \
-                     (const bf16_t*)w_gu, rows, tiles, (bf16_t*)y, top, ff, up * ff, W, g1, row_w, limit)
+                     (const bf16_t*)w_gu, rows, tiles, (bf16_t*)y, top, ff, up * ff, W, g1, row_w, limit, spread)
   if (act == ACT_GLU_CLAMP) MOE_FIRST(ACT_GLU_CLAMP);
   else if (act == ACT_GLU_SILU) MOE_FIRST(ACT_GLU_SILU);
   else MOE_FIRST(ACT_RELU2);
 #undef MOE_FIRST
   hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, ACT_NONE, false>), dim3(max_tiles * g2), blk, 0, st, (const bf16_t*)y,
-                     (const bf16_t*)w_down, rows, tiles, (bf16_t*)out, top, W, W, ff, g2, nullptr, 0.f);
+                     (const bf16_t*)w_down, rows, tiles, (bf16_t*)out, top, W, W, ff, g2, nullptr, 0.f, spread);
   return (int)hipGetLastError();
 }
 
@@ -277,10 +281,14 @@ int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void
   if (edge_sm_moe_gemm_ok(T, top, E, W, ff) != 0 || act < ACT_GLU_CLAMP || act > ACT_RELU2) return -2;
   const int R = T * top, BM = tile_rows(R, E), mt = max_tiles(R, E, BM);
   int *rows = ints, *tiles = ints + ((R + 3) & ~3);
+  // while the weights' bytes are the bound (up to some 500 rows an expert) the workgroups' k starts are spread: us for both
+  // products, 32 experts of 2048 x 2048, 4 each: 24 tokens 194 / 139, 128 209 / 147 (5.5 TB/s), 384 210 / 158, 800 224 / 179,
+  // 3000 476 / 474; with more rows it costs 2 % (7680 tokens of 3, ff 3072: 779 / 798)
+  const int spread = R <= E * 512;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(SORT_NT), 0, st, idx, R, E, BM, rows, tiles);
-  if (BM == 128) return launch_pair<128, 128, 2, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, st);
-  if (BM == 64) return launch_pair<64, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, st);
-  return launch_pair<32, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, st);
+  if (BM == 128) return launch_pair<128, 128, 2, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  if (BM == 64) return launch_pair<64, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  return launch_pair<32, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
 }
 
 }  // extern "C"

@@ -883,10 +883,10 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, scale: float, mod
 
 
 MOE_GEMM_MIN = int(__import__("os").environ.get("EDGELLM_MOE_GEMM_MIN", "64"))
-# steps of this many tokens or more take the grouped MFMA kernels where they run (bf16, widths of whole 64s): they read
-# each chosen expert once, the per-pair kernels once per pair.  us per layer, per pair / grouped: 16 experts of 1024 x
-# 1024, 3 per token: 6 tokens 24.8 / 24.8, 12 tokens 42 / 25, 63 tokens 122 / 28; 32 of 2048 x 2048, 4 per token: 6
-# tokens 123 / 125, 12 tokens 186 / 166, 63 tokens 599 / 207; squared ReLU beside a shared expert a little later
+# steps of this many tokens or more take the grouped MFMA kernels where they run (bf16, widths of whole 64s); below, the
+# pairs of one expert share its rows in moe_rows.h, up to four at a reading.  us per layer, by rows / grouped: 16 experts of
+# 1024 x 1024, 3 per token: 6 tokens 21.5 / 25.8, 9 tokens 25.2 / 29.6, 12 tokens 31.3 / 29.9, 16 tokens 50 / 31; 32 of 2048 x
+# 2048, 4 per token: 6 tokens 92 / 96, 9 tokens 114 / 115, 10 tokens 128 / 119, 16 tokens 227 / 133
 MOE_MFMA_MIN = int(__import__("os").environ.get("EDGELLM_MOE_MFMA_MIN", "10"))
 _MOE_ACT = {"glu_clamp": 1, "silu_glu": 2, "relu2": 3}
 
