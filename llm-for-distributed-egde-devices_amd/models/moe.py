@@ -6,12 +6,12 @@ alone (``ops.seqmix.moe_route``), or softmax scores that are corrected and limit
 choice only (``ops.seqmix.moe_route_grouped``).  Experts: clamped or plain silu
 gated-linear units or squared-ReLU units without a gate (then ``w_gu`` is [E, ff, W]), the router's weight on their output or on their input, weights stacked per layer as
 ``w_gu`` [E, 2 ff, W] (gate rows, then up rows) and ``w_down`` [E, W, ff]; decode-sized steps read
-only the chosen experts' rows, prompt-sized steps sort (token, choice) pairs by expert
-(``ops.seqmix.moe_experts``).  The shared expert is a dense unit of the same form.  ``forward``
+only the chosen experts' rows, once for all pairs of an expert; prompt-sized steps sort (token, choice) pairs by
+expert, in bf16 on the device beside two grouped products that leave the rows in order (``ops.seqmix.moe_experts``).  The shared expert is a dense unit of the same form.  ``forward``
 returns the shared expert's output and the chosen experts' outputs with their weights apart: the
 layer's output norm adds them up in fp32 in one kernel with the residual add.  ``run`` also returns the
-shared expert's weight per token and leaves prompt-sized steps' rows sorted by expert, for a residual kernel
-that takes both.
+shared expert's weight per token; where the grouped kernels do not run (fp32, odd widths) it leaves prompt-sized
+steps' rows sorted by expert, for a residual kernel that takes both.
 """
 from __future__ import annotations
 
