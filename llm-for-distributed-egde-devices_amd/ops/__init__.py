@@ -453,27 +453,40 @@ _GEMV_EPI = {None: 0, "silu_glu": 1, "gelu_tanh": 2, "gelu": 3}
 
 
 def _wrapped(t: torch.Tensor) -> bool:
-    """A tensor without memory of its own to read: a function transform's wrapper or a subclass."""
-    return type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t)
+    """A tensor without plain memory of its own to read: a function transform's wrapper, a subclass, a sparse or a lazily
+    negated one."""
+    return type(t) not in (torch.Tensor, torch.nn.Parameter) or torch._C._functorch.is_functorch_wrapped_tensor(t) or \
+        t.layout is not torch.strided or t.is_neg()
+
+
+def raw_call(*ts: torch.Tensor) -> bool:
+    """Whether a kernel that reads these tensors' memory itself may stand in for PyTorch ops that follow autograd, tracing and
+    function transforms: nothing records, rewrites or watches the ops of this call (autograd, forward mode, autocast,
+    ``torch.jit.trace``, ``make_fx`` / export / compile, any dispatch or function mode), and every tensor has memory to read."""
+    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
+        return False
+    if torch.is_autocast_enabled() or _fwd_ad._current_level >= 0:
+        return False
+    if torch.jit.is_tracing() or torch.compiler.is_compiling() or torch._C._len_torch_dispatch_stack() or \
+            torch._C._len_torch_function_stack():
+        return False
+    return not any(_wrapped(t) for t in ts)
 
 
 def f32_rows_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """Whether ``linear_bf16`` runs ``gemv_f32.hip`` for this call: dense 16-byte-aligned fp32 operands of one GPU, K % 4 == 0,
     up to 4 rows, or up to 8 rows and 8192 columns (measured at 8 rows: 6784 x 1024 12.1 us against the library's 12.9,
-    32000 x 1024 38 against 33), outside autograd, autocast, forward-mode and function transforms (the library product
-    serves those)."""
+    32000 x 1024 38 against 33), in a ``raw_call`` (the library product serves the others)."""
     if not (_gpu(x) and x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
+        return False
+    ts = (x, weight) if bias is None else (x, weight, bias)
+    if not raw_call(*ts):                                  # (before any size is looked at: those may be symbols)
         return False
     N, K = weight.shape
     if not (K >= 4 and K % 4 == 0 and N >= 1 and x.shape[-1] == K):
         return False
     M = x.numel() // K
     if not (1 <= M <= 4 or (4 < M <= 8 and N <= 8192)):
-        return False
-    ts = (x, weight) if bias is None else (x, weight, bias)
-    if torch.is_grad_enabled() and any(t.requires_grad for t in ts):
-        return False
-    if torch.is_autocast_enabled() or _fwd_ad._current_level >= 0 or any(_wrapped(t) for t in ts):
         return False
     if bias is not None and (bias.dtype != torch.float32 or bias.numel() != N):
         return False

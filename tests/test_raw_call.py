@@ -1,0 +1,89 @@
+"""Calls whose ops are recorded, rewritten or watched keep PyTorch ops; only the others reach kernels that read memory."""
+import ctypes
+
+import pytest
+import torch
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+from torch.utils.flop_counter import FlopCounterMode
+
+import edgellm  # noqa: F401
+from edgellm import ops
+
+
+class _Raw:
+    """The extension's fp32 product, its result written past PyTorch."""
+
+    calls = 0
+
+    def gemv_f32(self, x, w, bias):
+        self.calls += 1
+        y = torch.empty(*x.shape[:-1], w.shape[0])
+        ref = (x.detach().double() @ w.detach().double().t()).float().contiguous()
+        ctypes.memmove(y.data_ptr(), ref.data_ptr(), ref.numel() * 4)
+        return y
+
+
+@pytest.fixture
+def raw(monkeypatch):
+    r = _Raw()
+    monkeypatch.setattr(ops, "_gpu", lambda t: True)
+    monkeypatch.setattr(ops, "available", lambda: True)
+    monkeypatch.setattr(ops, "ext", lambda: r)
+    monkeypatch.setattr(ops, "bf16_decode_mode", lambda *a, **k: 0)
+    return r
+
+
+def _xw(seed=0):
+    g = torch.Generator().manual_seed(seed)
+    return torch.randn(2, 64, generator=g), torch.randn(32, 64, generator=g)
+
+
+@pytest.mark.parametrize("kw", [{}, {"pre_dispatch": True}, {"tracing_mode": "fake"}, {"tracing_mode": "symbolic"}])
+def test_make_fx_records_the_product(raw, kw):
+    x, w = _xw()
+    graph = make_fx(lambda a, b: ops.linear_bf16(a, b), **kw)(x, w)
+    x2, w2 = _xw(1)
+    assert raw.calls == 0 and torch.allclose(graph(x2, w2), torch.nn.functional.linear(x2, w2), atol=1e-4)
+
+
+def test_jit_trace_records_the_product(raw):
+    x, w = _xw()
+    traced = torch.jit.trace(lambda a, b: ops.linear_bf16(a, b), (x, w), check_trace=False)
+    x2, w2 = _xw(1)
+    assert raw.calls == 0 and torch.allclose(traced(x2, w2), torch.nn.functional.linear(x2, w2), atol=1e-4)
+
+
+def test_modes_and_transforms_keep_the_library_product(raw):
+    x, w = _xw()
+    ref = torch.nn.functional.linear(x, w)
+    with FlopCounterMode(display=False) as flops:
+        ops.linear_bf16(x, w)
+    assert flops.get_total_flops() == 2 * 2 * 64 * 32
+
+    class Seen(TorchFunctionMode):
+        linear = 0
+
+        def __torch_function__(self, f, types, args=(), kwargs=None):
+            self.linear += f is torch.nn.functional.linear or f is torch._C._nn.linear
+            return f(*args, **(kwargs or {}))
+
+    with Seen() as seen:
+        ops.linear_bf16(x, w)
+    assert seen.linear
+    assert torch.allclose(torch.func.functionalize(ops.linear_bf16)(x, w), ref, atol=1e-4)
+    assert torch.allclose(torch.func.vmap(lambda r: ops.linear_bf16(r, w))(x), ref, atol=1e-4)
+    assert torch.allclose(ops.linear_bf16(torch._neg_view(x), w), -ref, atol=1e-4)
+    assert torch.allclose(ops.linear_bf16(x, w.to_sparse_csr()), ref, atol=1e-4)
+    y = ops.linear_bf16(x.clone().requires_grad_(), w)
+    assert y.requires_grad and raw.calls == 0
+
+
+def test_a_plain_call_reaches_the_kernel(raw):
+    x, w = _xw()
+    assert torch.allclose(ops.linear_bf16(x, w), torch.nn.functional.linear(x, w), atol=1e-4)
+    with torch.no_grad():
+        ops.linear_bf16(x, torch.nn.Parameter(w))
+    with torch.inference_mode():
+        ops.linear_bf16(x, w)
+    assert raw.calls == 3
