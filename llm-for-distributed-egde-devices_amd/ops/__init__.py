@@ -488,7 +488,7 @@ def f32_rows_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     M = x.numel() // K
     if not (1 <= M <= 4 or (4 < M <= 8 and N <= 8192)):
         return False
-    if bias is not None and (bias.dtype != torch.float32 or bias.numel() != N):
+    if bias is not None and (bias.dtype != torch.float32 or tuple(bias.shape) != (N,)):   # others broadcast
         return False
     if any(t.device != x.device or not t.is_contiguous() for t in ts) or (x.data_ptr() | weight.data_ptr()) % 16:
         return False

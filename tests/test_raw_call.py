@@ -87,3 +87,12 @@ def test_a_plain_call_reaches_the_kernel(raw):
     with torch.inference_mode():
         ops.linear_bf16(x, w)
     assert raw.calls == 3
+
+
+def test_a_bias_that_broadcasts_is_the_librarys(raw):
+    x, w = _xw()
+    col, w2 = torch.tensor([[1.0], [2.0]]), w[:2].contiguous()
+    assert torch.allclose(ops.linear_bf16(x, w2, col), x @ w2.t() + col, atol=1e-4)
+    with pytest.raises(RuntimeError):
+        ops.linear_bf16(x[:1].expand(3, 64).contiguous(), w2, col)
+    assert raw.calls == 0
