@@ -231,6 +231,12 @@ class W8A8Linear(nn.Module):
         return f"{self.in_features}->{self.out_features}, bias={self.bias is not None}, W8A8 int8"
 
 
+def _epilogue_row(add: torch.Tensor, x: torch.Tensor) -> bool:
+    """Whether the other branch's row may join in the epilogue: dense bf16 beside ``x``, and no gradient, trace or transform
+    that the sum has to be an op for."""
+    return ops.raw_call(add) and add.dtype == torch.bfloat16 and add.device == x.device and add.is_contiguous()
+
+
 class LLMInt8Linear(nn.Module):
     takes_quantized_input = False
     graph_safe = False   # outlier-column discovery is data dependent (host sync on CPU), like bnb ...
@@ -348,8 +354,7 @@ class LLMInt8Linear(nn.Module):
             x2 = x2.contiguous()
             if x2.shape[0] == 1 and K <= 12288 and K % 64 == 0 and self.ONE_LAUNCH:
                 # batch 1: outlier discovery, quantisation and the outlier part inside the GEMV
-                fuse = add is not None and not act and add.dtype == torch.bfloat16 and add.device == x2.device and \
-                    add.is_contiguous()                     # the other branch's row joins in the epilogue
+                fuse = add is not None and not act and _epilogue_row(add, x2)
                 out = C.llmint8_gemv(x2, self.threshold, self.w_packed, self._w_deq, self.bias, self._weight_t,
                                      self.SCB, N, act, add if fuse else None)
                 if out is not None:

@@ -96,3 +96,41 @@ def test_a_bias_that_broadcasts_is_the_librarys(raw):
     with pytest.raises(RuntimeError):
         ops.linear_bf16(x[:1].expand(3, 64).contiguous(), w2, col)
     assert raw.calls == 0
+
+
+@pytest.mark.gpu
+def test_llmint8_added_row_keeps_its_gradient_and_transforms():
+    """One row, the sum where autograd, forward mode, vmap and dispatch modes see it: add's own gradient, tangent and batch."""
+    from edgellm.models.layers import Linear
+    from edgellm.quant import LLMInt8Linear
+    lin = Linear(128, 96, bias=False, device="cuda:0")
+    lin.weight.data.copy_(torch.randn(96, 128) * 0.05)
+    m = LLMInt8Linear.from_float(lin)
+    x, add = torch.randn(1, 128).bfloat16().cuda(), torch.randn(1, 96).bfloat16().cuda()
+    with torch.no_grad():
+        ref = m(x, add=add)                                # in the epilogue
+    leaf, up = add.clone().requires_grad_(), torch.randn(1, 96).bfloat16().cuda()
+    y = m(x, add=leaf)
+    (grad,) = torch.autograd.grad(y + leaf, leaf, up)      # add reaches the result another way as well
+    assert torch.equal(y, ref) and torch.equal(grad, 2 * up)
+    _, tangent = torch.func.jvp(lambda a: m(x, add=a), (add,), (up,))
+    assert torch.equal(tangent, up)
+    rows = torch.stack([add, add * 2])
+    assert torch.equal(torch.func.vmap(lambda a: m(x, add=a))(rows), torch.stack([ref, m(x) + add * 2]))
+    with FlopCounterMode(display=False):
+        assert torch.equal(m(x, add=add), ref)
+
+
+def test_a_row_joins_an_epilogue_only_as_plain_memory():
+    from edgellm.quant.linear import _epilogue_row
+    x, add = torch.zeros(1, 8, dtype=torch.bfloat16), torch.zeros(1, 8, dtype=torch.bfloat16)
+    leaf = add.clone().requires_grad_()
+    assert _epilogue_row(add, x) and not _epilogue_row(leaf, x) and not _epilogue_row(add.float(), x)
+    assert not _epilogue_row(torch.zeros(1, 16, dtype=torch.bfloat16)[:, ::2], x)
+    with torch.no_grad():
+        assert _epilogue_row(leaf, x)
+    seen = []
+    torch.func.vmap(lambda a: (seen.append(_epilogue_row(a, x)), a * 1)[1])(add)
+    torch.func.jvp(lambda a: (seen.append(_epilogue_row(a, x)), a * 1)[1], (add,), (add,))
+    make_fx(lambda a: (seen.append(_epilogue_row(a, x)), a * 1)[1])(add)
+    assert seen == [False] * 3
