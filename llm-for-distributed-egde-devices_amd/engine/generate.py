@@ -15,7 +15,6 @@ import time
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence
 
-import numpy as np
 import torch
 
 from .. import ops
@@ -193,6 +192,13 @@ class Generator:
         max_new = sampling.max_new_tokens
         assert max(plens) + max_new <= self.max_seq, "prompt + max_new_tokens exceeds max_seq"
         assert self.attn_hook is None or len(set(plens)) == 1, "HeadInfer offload batches equal-length prompts"
+        # the prompts' tokens count for the repetition penalty: one copy and one launch for the whole batch (a copy and
+        # a launch per prompt were 11 of the 129 ms that 256 prompts of 128 tokens with 32 new ones took).  Ids are looked
+        # at before any state is touched; negative ones count from the vocabulary's end here, as in an index
+        flat = torch.cat([torch.as_tensor(p, dtype=torch.long, device="cpu") for p in prompts])
+        if ((flat < -V) | (flat >= V)).any():
+            raise IndexError(f"token ids outside the vocabulary of {V}")
+        flat = torch.where(flat < 0, flat + V, flat) + torch.repeat_interleave(torch.arange(B) * V, torch.tensor(plens))
         st = self._state
         if st is None or st.tok.shape[0] != B or st.out.shape[1] < max_new:
             self.reset_graphs()
@@ -217,13 +223,7 @@ class Generator:
         else:
             logits = torch.cat([self.prefill(torch.tensor([p], dtype=torch.long, device=self.device), b, 0)
                                 for b, p in enumerate(prompts)], 0)
-        # the prompts' tokens count for the repetition penalty: one copy and one launch for the whole batch (a copy and
-        # a launch per prompt were 11 of the 129 ms that 256 prompts of 128 tokens with 32 new ones took)
-        flat = np.concatenate([np.asarray(p, dtype=np.int64) for p in prompts])
-        if flat.size and (flat.min() < 0 or flat.max() >= V):
-            raise IndexError(f"token ids outside the vocabulary of {V}")
-        flat += np.repeat(np.arange(B, dtype=np.int64) * V, plens)
-        st.seen.view(-1).index_fill_(0, torch.from_numpy(flat).to(self.device), 1)
+        st.seen.view(-1).index_fill_(0, flat.to(self.device), 1)
         st.pos.copy_(torch.tensor(plens, dtype=torch.int32, device=self.device))
         st.seq_lens.copy_(st.pos + 1)
         nxt = ops.sample(logits, st.seen, sampling.temperature, sampling.top_k, sampling.top_p,

@@ -121,6 +121,37 @@ def test_start_marks_every_prompt_token_and_refuses_ids_outside_the_vocabulary()
     first = gen._state.out[:, 0].tolist()
     for b, p in enumerate(prompts):
         assert set(gen._state.seen[b].nonzero().flatten().tolist()) - {first[b]} == set(p) - {first[b]}
-    for bad in (V, -1):
-        with pytest.raises(IndexError):
+    seen, out = gen._state.seen.clone(), gen._state.out.clone()
+    for bad in (V, -V - 1):                                # refused before any state is touched
+        with pytest.raises(IndexError, match="outside the vocabulary"):
             gen.start([[1, 2, bad], [3], [4]], SamplingParams(max_new_tokens=2))
+    assert torch.equal(gen._state.seen, seen) and torch.equal(gen._state.out, out)
+    with pytest.raises(IndexError):                        # (the CPU's embedding has no row for it)
+        gen.start([[1, 2, -1], [3], [4]], SamplingParams(max_new_tokens=2))
+
+
+def _start_forms(device):
+    model = build_model(tiny("llama2"), dtype=torch.float32, device=device, seed=0)
+    gen = Generator(model, max_batch=2, max_seq=64)
+    sp = SamplingParams(max_new_tokens=2, do_sample=False)
+    for rows in ([[5, 1, 9], [4, 4, 2]], [[5, 1, 9], [7]]):
+        forms = [rows, [torch.tensor(r, device=device).unbind() for r in rows], [tuple(r) for r in rows]]
+        forms += [torch.tensor(rows, device=device)] if len(rows[0]) == len(rows[1]) else [[torch.tensor(r, device=device) for r in rows]]
+        for f in forms:
+            gen.start(f, sp)
+            first = gen._state.out[:, 0].tolist()
+            for b in (0, 1):
+                assert set(gen._state.seen[b].nonzero().flatten().tolist()) - {first[b]} == set(rows[b]) - {first[b]}
+    return gen
+
+
+def test_start_takes_prompts_of_every_sequence_type():
+    _start_forms("cpu")
+
+
+@pytest.mark.gpu
+def test_start_takes_prompts_on_the_device_and_negative_ids():
+    """Device tensors as prompts; the device's embedding clamps ids, so a negative one is an index from the end, as it was."""
+    gen = _start_forms("cuda:0")
+    gen.start([[3, -1], [6, 2]], SamplingParams(max_new_tokens=2, do_sample=False))
+    assert gen._state.seen[0, gen.cfg.vocab_size - 1] == 1 and gen._state.seen[0, 3] == 1
