@@ -131,7 +131,7 @@ def test_start_marks_every_prompt_token_and_refuses_ids_outside_the_vocabulary()
 
 
 def _start_forms(device):
-    model = build_model(tiny("llama2"), dtype=torch.float32, device=device, seed=0)
+    model = build_model(tiny("llama2"), dtype=torch.float32 if device == "cpu" else torch.bfloat16, device=device, seed=0)
     gen = Generator(model, max_batch=2, max_seq=64)
     sp = SamplingParams(max_new_tokens=2, do_sample=False)
     for rows in ([[5, 1, 9], [4, 4, 2]], [[5, 1, 9], [7]]):

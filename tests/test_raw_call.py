@@ -113,8 +113,9 @@ def test_llmint8_added_row_keeps_its_gradient_and_transforms():
     y = m(x, add=leaf)
     (grad,) = torch.autograd.grad(y + leaf, leaf, up)      # add reaches the result another way as well
     assert torch.equal(y, ref) and torch.equal(grad, 2 * up)
-    _, tangent = torch.func.jvp(lambda a: m(x, add=a), (add,), (up,))
-    assert torch.equal(tangent, up)
+    with torch.autograd.forward_ad.dual_level():
+        dual = m(x, add=torch.autograd.forward_ad.make_dual(add, up))
+        assert torch.equal(torch.autograd.forward_ad.unpack_dual(dual).tangent, up)
     rows = torch.stack([add, add * 2])
     assert torch.equal(torch.func.vmap(lambda a: m(x, add=a))(rows), torch.stack([ref, m(x) + add * 2]))
     with FlopCounterMode(display=False):
