@@ -71,7 +71,7 @@ class MoEFeedForward(nn.Module):
         assert s.router == "softmax" and s.weight_on == "output" and (s.act == "relu2" or (s.act == "silu_glu" and not s.shared_ff))
         idx, wts, shared_w = seqmix.moe_route_grouped(h, self.router, s.top, s.scale, self.correction, s.groups, s.groups_keep,
                                                       s.shared_gate)
-        if s.shared_ff and h.shape[0] < seqmix.MOE_GEMM_MIN and not seqmix.moe_grouped(h, idx, self.w_gu, self.w_down, s.act):
+        if s.shared_ff and h.shape[0] < seqmix.MOE_GEMM_MIN:
             parts, shared = seqmix.moe_experts_shared(h, idx, self.w_gu, self.w_down, self.shared_gu.weight,
                                                       self.shared_down.weight)
             return MoEOut(shared, shared_w, parts, wts, None)

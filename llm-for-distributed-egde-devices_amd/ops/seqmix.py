@@ -931,10 +931,15 @@ def moe_experts(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: 
 
 def moe_experts_shared(h: torch.Tensor, idx: torch.Tensor, w_up: torch.Tensor, w_down: torch.Tensor, shared_up: torch.Tensor,
                        shared_down: torch.Tensor):
-    """Squared-ReLU experts and the shared expert of the same form in one go, for decode-sized steps: w_up
+    """Squared-ReLU experts and the shared expert of the same form in one go, for steps below MOE_GEMM_MIN tokens: w_up
     [E, ff, W], w_down [E, W, ff], shared_up [sff, W], shared_down [W, sff] -> (the chosen experts' outputs
-    [T, top, W], the shared expert's [T, W])."""
+    [T, top, W], the shared expert's [T, W]).  Both square max(u, 0) in fp32 before anything is rounded: where the
+    grouped kernels run, the shared expert is a single group of its own."""
     if _gpu(h):
+        if moe_grouped(h, idx, w_up, w_down, "relu2"):
+            one, up, down = torch.zeros(h.shape[0], 1, dtype=torch.int32, device=h.device), shared_up[None], shared_down[None]
+            if _ext().sm_moe_gemm_ok(h, one, up, down, 3, None):
+                return moe_experts(h, idx, w_up, w_down, 0.0, "relu2"), _ext().sm_moe_gemm(h, one, up, down, 3, 0.0, None)[:, 0]
         return _ext().sm_moe_experts_relu2(h, idx, w_up, w_down, shared_up, shared_down)
     return moe_experts(h, idx, w_up, w_down, 0.0, "relu2"), F.linear(relu2(F.linear(h, shared_up)), shared_down)
 

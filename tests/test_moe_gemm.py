@@ -65,6 +65,29 @@ def test_grouped_experts_against_float64(T, top, E, W, ff, act):
 
 
 @gpu
+@pytest.mark.parametrize("T,W,ff,sff", [(9, 1024, 512, 1024), (10, 1024, 512, 1024), (33, 512, 1024, 512), (63, 1024, 512, 576),
+                                        (12, 1024, 512, 1032), (40, 256, 128, 192)])
+def test_shared_expert_of_small_steps_squares_in_fp32(T, W, ff, sff):
+    """Steps below MOE_GEMM_MIN tokens: u is squared before it is rounded.  The unit and the result are rounded to bf16 (rms
+    2^-9 each at most, random): 2.8e-3 together; a u rounded first would add 2 x 1.6e-3 to the unit (4e-3 measured)."""
+    from edgellm.models.configs import MoESpec
+    from edgellm.models.moe import MoEFeedForward
+    g = torch.Generator().manual_seed(T)
+    m = MoEFeedForward(MoESpec(8, 3, 1.0, ff, shared_ff=sff, router="softmax", act="relu2", correction=True, groups=4, groups_keep=2,
+                               shared_gate=True), W, torch.bfloat16, torch.device("cuda:0"))
+    for p in m.parameters():
+        p.data.copy_(torch.randn(p.shape, generator=g) * p.shape[-1] ** -0.5)
+    h = torch.randn(T, W, generator=g).bfloat16().cuda()
+    f = m.run(h)
+    d = lambda t: t.cpu().double()
+    want = torch.relu(d(h) @ d(m.shared_gu.weight).T) ** 2 @ d(m.shared_down.weight).T
+    assert (d(f.shared) - want).norm() < 2.8e-3 * want.norm()
+    idx = seqmix.moe_route_grouped(h, m.router, 3, 1.0, m.correction, 4, 2, True)[0]
+    want = reference(h, idx, m.w_gu, m.w_down, "relu2", 0.0, None)
+    assert f.rows is None and (d(f.parts) - want).norm() < 2.8e-3 * want.norm()
+
+
+@gpu
 @pytest.mark.parametrize("case", ["one expert", "first and last", "idle neighbours"])
 def test_grouped_experts_with_skewed_routing(case):
     T, E = 300, 9
