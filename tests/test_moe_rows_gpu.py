@@ -1,6 +1,7 @@
 """Experts of decode-sized steps (moe_rows.h) against the same op in fp32 on the CPU: every count of tokens per expert that
 the shared readings distinguish (1, 2, 3, 4, 5 and all), widths beside a wave's 512 and 1024 numbers and a workgroup's rows,
-repeated and out-of-range choices, more pairs than one ballot names, the shared expert, widths of the general kernels."""
+experts on both sides of the size from which readings are shared, repeated and out-of-range choices, more pairs than one
+ballot names (by tokens and by choices), the shared expert, widths of the general kernels."""
 import pytest
 import torch
 
@@ -16,6 +17,7 @@ CHOICES = {
     "five": [[1, 0], [1, 2], [3, 1], [1, 4], [5, 1]],
     "all": [[4, 4], [4, 4], [4, 4], [4, 4], [4, -7], [99, 4]],
     "many": [[i % 6, (i * 5 + 1) % 6] for i in range(40)],
+    "wide": [[(i + k) % 6 for k in range(8)] for i in range(9)],
 }
 
 
@@ -28,15 +30,16 @@ def _operands(dt, W, ff, top, T, act, seed):
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("name", list(CHOICES))
 @pytest.mark.parametrize("W,ff,act", [(8, 8, "glu_clamp"), (520, 24, "silu_glu"), (1024, 520, "silu_w"), (1032, 16, "glu_clamp"),
-                                      (2056, 40, "silu_glu"), (512, 1032, "relu2"), (1024, 20, "silu_glu"), (20, 64, "relu2")])
+                                      (2056, 40, "silu_glu"), (512, 1032, "relu2"), (1024, 20, "silu_glu"), (20, 64, "relu2"),
+                                      (1032, 1032, "silu_glu"), (1032, 1048, "relu2")])
 def test_decode_sized_experts(dt, name, W, ff, act):
-    T = len(CHOICES[name])
-    if dt == torch.bfloat16 and S.MOE_MFMA_MIN <= T:
-        pytest.skip("the grouped kernels' size")
-    h, w_gu, w_down, in_w, su, sd = _operands(dt, W, ff, 2, T, act, T + W)
+    """No case has both widths whole 64s: none is the grouped kernels', of whatever length."""
+    T, top = len(CHOICES[name]), len(CHOICES[name][0])
+    h, w_gu, w_down, in_w, su, sd = _operands(dt, W, ff, top, T, act, T + W)
     idx = torch.tensor(CHOICES[name], dtype=torch.int32)
     op, in_w = ("silu_glu", in_w) if act == "silu_w" else (act, None)
     cuda = lambda x: None if x is None else x.cuda()
+    assert not S.moe_grouped(h.cuda(), idx.cuda(), w_gu.cuda(), w_down.cuda(), op, cuda(in_w))
     got = S.moe_experts(h.cuda(), idx.cuda(), w_gu.cuda(), w_down.cuda(), 1.5, op, cuda(in_w)).float().cpu()
     f = lambda x: x.float()
     ref = S.moe_experts(f(h), idx.clamp(0, 5), f(w_gu), f(w_down), 1.5, op, in_w)
