@@ -11,13 +11,13 @@ constexpr int MR_GLU = 0, MR_PLAIN = 1, MR_RELU2 = 2;
 // weights w_sh, widths K_sh -> R_sh).  MR_GLU: out = act(gate . x, up . x), weights [E, 2 R, K], rows of x per token; act =
 // silu(rw g) (rw u) (silu, rw = in_w[pair] or 1) or the clamped form.  MR_RELU2: out = max(W x, 0)^2, rows of x per token.
 // MR_PLAIN: out = W x, rows of x per pair.
-// Bound by the chosen experts' weights.  A workgroup is (pair, 4 waves of 4 weight rows); pairs of one expert belong to the
-// first of them (`share`: at most 64 routed pairs, so one ballot names them), which runs them together, up to four per
-// reading of the rows; the others leave at once.  A wave has its four rows' next 1024 numbers (2048 for one pair) in flight
-// as contiguous KiBs and the inputs beside them in registers; the sums over lanes end with one sum per lane.
-// us for both launches, one wave per row and pair / this, bf16: 3 of 16 experts of 1024 x 1024, 1 token 16.8 / 10.3, 4 tokens
-// 22.7 / 19.0, 9 31.5 / 25.3; 4 of 32 of 2048 x 2048 35.4 / 25.8, 82.6 / 66.7, 160 / 114 (5.0 TB/s).  fp32 only for one
-// token (19.5 / 14.0): rows shared by several pairs need more registers than they save there (4 of 16 of 1024 x 1024,
+// Bound by the chosen experts' weights.  A workgroup is (pair, 4 waves of 4 weight rows).  `share` (launch_moe_rows): pairs
+// of one expert belong to the first of them (at most 64 routed pairs, so one ballot names them), which runs them together,
+// up to four per reading of the rows; the others leave at once.  A wave has its four rows' next 1024 numbers (2048 for one
+// pair) in flight as contiguous KiBs and the inputs beside them in registers; the sums over lanes end with one sum per lane.
+// us for both launches, one wave per row and pair / this, bf16: 3 of 16 experts of 1024 x 1024, 1 token 11.1 / 7.4, 4 tokens
+// 18.8 / 17.4, 9 29.4 / 23.0; 4 of 32 of 2048 x 2048 26.5 / 20.9, 74 / 69, 159 / 113 (5.0 TB/s).  fp32 only for one
+// token (15.1 / 9.6): rows shared by several pairs need more registers than they save there (4 of 16 of 1024 x 1024,
 // 6 tokens 48.6 / 54.7, 16 tokens 102 / 141).
 template <typename T, int MODE, int MT, int CH>
 __device__ __forceinline__ void moe_rows_run(const T* const (&wr)[4], const T* const (&xr)[MT], int K, float (&acc)[4 * MT]) {
@@ -141,7 +141,12 @@ void launch_moe_rows(const T* in, const T* in_sh, const int* idx, int routed, in
                      hipStream_t st) {
   constexpr int FW = (MODE == MR_GLU ? 2 : 4) * (NT / 64);
   const int big = pairs > routed && R_sh > R ? R_sh : R;
-  const int share = sizeof(T) == 2 && routed <= 64 && pairs - routed <= 64;
+  // Sharing pays where rows come from memory: an expert of a million numbers or more, and few tokens, for the expert's
+  // pairs then run one group after another.  us for both launches, each pair for itself / shared: 2 of 8 experts of 512 x
+  // 520, 16 tokens 9.9 / 17.8; 2 of 4 of 64 x 64, 9 tokens 6.5 / 12.8; 3 of 16 of 1024 x 1536, 9 tokens 27.8 / 20.8;
+  // with a shared expert of 1024 x 1536 beside them, 9 tokens 42 / 36, 10 40.0 / 39.5, 16 49 / 92
+  const int share = sizeof(T) == 2 && routed <= 64 && routed <= 12 * top && pairs - routed <= 12 &&
+                    (int64_t)K * R * (MODE == MR_GLU ? 2 : 1) >= 1 << 20;
   hipLaunchKernelGGL((moe_rows_kernel<T, MODE>), dim3(pairs, (big + FW - 1) / FW), dim3(NT), 0, st, in, in_sh, idx, routed, pairs,
                      top, w, w_sh, K, R, K_sh, R_sh, E, limit, silu, in_w, out, out_sh, share);
 }
