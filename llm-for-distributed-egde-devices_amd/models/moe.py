@@ -6,7 +6,7 @@ alone (``ops.seqmix.moe_route``), or softmax scores that are corrected and limit
 choice only (``ops.seqmix.moe_route_grouped``).  Experts: clamped or plain silu
 gated-linear units or squared-ReLU units without a gate (then ``w_gu`` is [E, ff, W]), the router's weight on their output or on their input, weights stacked per layer as
 ``w_gu`` [E, 2 ff, W] (gate rows, then up rows) and ``w_down`` [E, W, ff]; decode-sized steps read
-only the chosen experts' rows, once for all pairs of an expert; prompt-sized steps sort (token, choice) pairs by
+only the chosen experts' rows, a large expert's once for all its pairs; prompt-sized steps sort (token, choice) pairs by
 expert, in bf16 on the device beside two grouped products that leave the rows in order (``ops.seqmix.moe_experts``).  The shared expert is a dense unit of the same form.  ``forward``
 returns the shared expert's output and the chosen experts' outputs with their weights apart: the
 layer's output norm adds them up in fp32 in one kernel with the residual add.  ``run`` also returns the

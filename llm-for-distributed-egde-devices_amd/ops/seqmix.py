@@ -883,18 +883,30 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, scale: float, mod
 
 
 MOE_GEMM_MIN = int(__import__("os").environ.get("EDGELLM_MOE_GEMM_MIN", "64"))
-# steps of this many tokens or more take the grouped MFMA kernels where they run (bf16, widths of whole 64s); below, the
-# pairs of one expert share its rows in moe_rows.h, up to four at a reading.  us per layer, by rows / grouped: 16 experts of
-# 1024 x 1024, 3 per token: 6 tokens 21.5 / 25.8, 9 tokens 25.2 / 29.6, 12 tokens 31.3 / 29.9, 16 tokens 50 / 31; 32 of 2048 x
-# 2048, 4 per token: 6 tokens 92 / 96, 9 tokens 114 / 115, 10 tokens 128 / 119, 16 tokens 227 / 133
+# steps of this many tokens or more take the grouped MFMA kernels where they run (bf16, widths of whole 64s), those below
+# MOE_GEMM_MIN only for MOE_MFMA_WORK pairs times numbers of an expert or more; otherwise the rows of moe_rows.h.  us per
+# layer, by rows / grouped: 3 of 16 experts of 1024 x 1024: 9 tokens 25.2 / 29.6, 12 tokens 31.3 / 29.9, 16 tokens 50 / 31; 4 of
+# 32 of 2048 x 2048, 9 tokens 114 / 115, 10 tokens 128 / 119, 16 tokens 227 / 133; small experts are bound by the launches,
+# three against two: 2 of 8 of 256 x 128 (98 thousand numbers), 12 tokens 6.6 / 10.6, 40 tokens 10.0 / 10.3, 63 tokens 12.7 /
+# 10.6; 2 of 4 of 64 x 64, 63 tokens 7.6 / 10.6
 MOE_MFMA_MIN = int(__import__("os").environ.get("EDGELLM_MOE_MFMA_MIN", "10"))
+MOE_MFMA_WORK = 1 << 23
+# the same where a shared expert runs beside them (its pairs counted; three launches more): by rows / grouped, 3 of 8 experts of
+# 256 x 128, 63 tokens 24 / 31; of 512 x 520 or 512 x 512, 24 tokens 28 / 28; 3 of 16 of 1024 x 1536, 10 tokens 40 / 43, 16 tokens
+# 49 / 44
+MOE_SHARED_WORK = 50 << 20
 _MOE_ACT = {"glu_clamp": 1, "silu_glu": 2, "relu2": 3}
 
 
 def moe_grouped(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor, act: str,
                 in_w: Optional[torch.Tensor] = None) -> bool:
     """Whether ``moe_experts`` runs this step through the grouped MFMA kernels (csrc/seqmix/moe_gemm.hip)."""
-    return _gpu(h) and h.shape[0] >= MOE_MFMA_MIN and bool(_ext().sm_moe_gemm_ok(h, idx, w_gu, w_down, _MOE_ACT[act], in_w))
+    T = h.shape[0]
+    if not _gpu(h) or T < MOE_MFMA_MIN:
+        return False
+    if T < MOE_GEMM_MIN and idx.numel() * ((w_gu.numel() + w_down.numel()) // max(w_gu.shape[0], 1)) < MOE_MFMA_WORK:
+        return False
+    return bool(_ext().sm_moe_gemm_ok(h, idx, w_gu, w_down, _MOE_ACT[act], in_w))
 
 
 def moe_experts(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor, limit: float,
@@ -936,7 +948,8 @@ def moe_experts_shared(h: torch.Tensor, idx: torch.Tensor, w_up: torch.Tensor, w
     [T, top, W], the shared expert's [T, W]).  Both square max(u, 0) in fp32 before anything is rounded: where the
     grouped kernels run, the shared expert is a single group of its own."""
     if _gpu(h):
-        if moe_grouped(h, idx, w_up, w_down, "relu2"):
+        work = (idx.numel() + h.shape[0]) * ((w_up.numel() + w_down.numel()) // max(w_up.shape[0], 1))
+        if work >= MOE_SHARED_WORK and moe_grouped(h, idx, w_up, w_down, "relu2"):
             one, up, down = torch.zeros(h.shape[0], 1, dtype=torch.int32, device=h.device), shared_up[None], shared_down[None]
             if _ext().sm_moe_gemm_ok(h, one, up, down, 3, None):
                 return moe_experts(h, idx, w_up, w_down, 0.0, "relu2"), _ext().sm_moe_gemm(h, one, up, down, 3, 0.0, None)[:, 0]

@@ -46,6 +46,12 @@ def inputs(T, top, E, W, ff, act, seed=0):
 TOL = 5e-3
 
 
+@pytest.fixture
+def every_size(monkeypatch):
+    """Small experts too, which steps below MOE_GEMM_MIN tokens otherwise run by rows."""
+    monkeypatch.setattr(seqmix, "MOE_MFMA_WORK", 0)
+
+
 @gpu
 @pytest.mark.parametrize("act", ["glu_clamp", "silu_glu", "relu2"])
 @pytest.mark.parametrize("T,top,E,W,ff", [
@@ -55,13 +61,24 @@ TOL = 5e-3
     (257, 2, 3, 256, 320),       # 128-row tiles with a remainder
     (1030, 4, 16, 320, 128),     # several tiles per expert
     (70, 1, 512, 64, 128)])      # the most experts
-def test_grouped_experts_against_float64(T, top, E, W, ff, act):
+def test_grouped_experts_against_float64(T, top, E, W, ff, act, every_size):
     h, idx, w_gu, w_down, in_w = inputs(T, top, E, W, ff, act)
     assert seqmix.moe_grouped(h, idx, w_gu, w_down, act, in_w)
     got = seqmix.moe_experts(h, idx, w_gu, w_down, 1.5, act, in_w).cpu().double()
     want = reference(h, idx, w_gu, w_down, act, 1.5, in_w)
     assert ((got - want).norm() / want.norm()) < TOL
     assert ((got - want).norm(dim=-1) / want.norm(dim=-1).clamp_min(1e-3)).max() < 4 * TOL
+
+
+@gpu
+def test_small_experts_of_small_steps_run_by_rows():
+    """Pairs times an expert's numbers on both sides of MOE_MFMA_WORK, and a step of MOE_GEMM_MIN tokens: the same result."""
+    for T, W, ff, grouped in ((12, 256, 128, False), (42, 256, 128, False), (43, 256, 128, True), (64, 64, 64, True), (63, 64, 64, False)):
+        h, idx, w_gu, w_down, in_w = inputs(T, 2, 8, W, ff, "silu_glu", T)
+        assert seqmix.moe_grouped(h, idx, w_gu, w_down, "silu_glu", in_w) == grouped
+        got = seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "silu_glu", in_w).cpu().double()
+        want = reference(h, idx, w_gu, w_down, "silu_glu", 0.0, in_w)
+        assert (got - want).norm() < TOL * want.norm()
 
 
 @gpu
