@@ -631,10 +631,9 @@ __global__ void __launch_bounds__(NT) moe_logits_kernel(const T* __restrict__ h,
   if (lane == 0) z[t * E + e] = acc + (bias ? bias[e] : 0.f);
 }
 
-// The same for prompt-sized steps, four tokens by four experts per wave: the router's rows are read once per four tokens
+// The same for long prompts, four tokens by four experts per wave: the router's rows are read once per four tokens
 // (they were the bound: E x W fp32 numbers a token) and the sums are those of one wave per pair, bit for bit (the same chain
-// per lane, the same pairs of lanes).  us: 32 experts, 7680 tokens of 2048 103 / 46; 16 experts, 4096 of 1024 16.2 / 8.5; below 64 tokens one wave per pair is as
-// fast and has the shorter chain.
+// per lane, the same pairs of lanes).
 template <typename T>
 __global__ void __launch_bounds__(NT) moe_logits16_kernel(const T* __restrict__ h, int W, const float* __restrict__ router,
                                                           int E, float* __restrict__ z, const float* __restrict__ bias,
@@ -666,7 +665,11 @@ __global__ void __launch_bounds__(NT) moe_logits16_kernel(const T* __restrict__ 
 
 template <typename T>
 void launch_moe_logits(const T* h, int W, const float* router, int E, float* z, const float* bias, int rows, hipStream_t st) {
-  if (rows >= 64 && W % 8 == 0)
+  // sixteen times fewer waves with a chain four times as long: it pays once one wave per pair takes more than about one round
+  // of the chip.  us with the choice behind it, a wave per pair / four by four: 32 experts of 2048, 256 tokens 8.8 / 10.0, 511
+  // 12.3 / 10.3, 4096 51 / 27; 16 of 1024, 256 6.8 / 8.2, 700 8.2 / 8.4, 1000 9.1 / 8.6, 4096 19.3 / 11.4; 8 of 256, 1000 7.0 /
+  // 7.3, 1500 7.6 / 7.5, 4096 10.7 / 8.6
+  if ((int64_t)rows * E >= 12288 && W % 8 == 0)
     hipLaunchKernelGGL(moe_logits16_kernel<T>, dim3((rows + 3) / 4, (E + 15) / 16), dim3(NT), 0, st, h, W, router, E, z, bias, rows);
   else
     hipLaunchKernelGGL(moe_logits_kernel<T>, dim3(rows, (E + NT / 64 - 1) / (NT / 64)), dim3(NT), 0, st, h, W, router, E, z, bias);

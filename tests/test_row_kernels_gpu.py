@@ -93,9 +93,10 @@ def test_latent_write(dt, H, D, R, kvr, rot):
 
 
 @pytest.mark.parametrize("dt", DT)
-@pytest.mark.parametrize("T,E,W,bias", [(64, 16, 1024, False), (67, 5, 520, True), (130, 33, 2048, False), (65, 1, 8, True), (66, 16, 1030, False)])
+@pytest.mark.parametrize("T,E,W,bias", [(64, 16, 1024, False), (768, 16, 1024, False), (2459, 5, 520, True), (374, 33, 2048, False),
+                                        (12289, 1, 8, True), (770, 16, 1030, False)])
 def test_router_scores_of_prompts(dt, T, E, W, bias):
-    """From 64 tokens on four tokens share the router's rows: the same choices and weights, bit for bit, as in small steps."""
+    """From 12288 scores on four tokens share the router's rows: the same choices and weights, bit for bit, as in small steps."""
     g = torch.Generator().manual_seed(E)
     h, router = _rand(g, T, W).to(dt).cuda(), _rand(g, E, W).cuda()
     b = _rand(g, E).cuda() if bias else None
