@@ -260,7 +260,9 @@ __global__ void __launch_bounds__(64) head_norm_gate_kernel(const float* __restr
 }
 
 // The same with 16 lanes per head and four numbers per access (P % 4 == 0, P <= 256): 16 heads per workgroup instead of one
-// per wave of its own.  16 heads of 64, us: 4096 tokens 18.2 / 9.5, 4 tokens 3.9 / 2.6.
+// per wave of its own.  16 heads of 64, us: 4096 tokens 17.6 / 8.5, 4 tokens 2.4 / 2.4; of 128: 4096 tokens 22.7 / 15.9, 128
+// tokens 3.2 / 3.1, 16 tokens 2.7 / 3.0: heads of more than one run per lane (P > 64) take it from 2048 of them on.  Up to 2^28
+// heads (a launch has at most 2^32 threads).
 template <typename T>
 __global__ void __launch_bounds__(NT) head_norm_gate16_kernel(const float* __restrict__ y, const T* __restrict__ z, int z_ld,
                                                               const float* __restrict__ w, T* __restrict__ out, int H, int P,
@@ -989,7 +991,7 @@ int edge_sm_head_norm_gate(const float* y, const void* z, int z_ld, const float*
   if (rows == 0) return 0;
   const long items = (long)rows * H;
   if (P % 4 == 0 && P >= 4 && P <= 256 && z_ld % 4 == 0 && (((uintptr_t)y | (uintptr_t)w | (uintptr_t)out) & 15) == 0 &&
-      (uintptr_t)z % (f32 ? 16 : 8) == 0 && items <= (1l << 33)) {
+      (uintptr_t)z % (f32 ? 16 : 8) == 0 && (P <= 64 || items >= 2048) && items < (1l << 28)) {
     SM_T(f32, hipLaunchKernelGGL(head_norm_gate16_kernel<T>, dim3((unsigned)((items + 15) / 16)), dim3(NT), 0, st, y, (const T*)z,
                                  z_ld, w, (T*)out, H, P, eps, silu, items));
     return (int)hipGetLastError();

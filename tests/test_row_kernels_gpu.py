@@ -40,7 +40,7 @@ def test_layer_norm_residual(dt, W, T, K, with_y):
 @pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("heads,P,act", [(1, 4, "silu"), (16, 64, "sigmoid"), (5, 68, "silu"), (3, 128, "sigmoid"), (2, 256, "silu"),
                                          (2, 260, "sigmoid"), (3, 62, "silu")])
-@pytest.mark.parametrize("T,pad", [(1, 0), (7, 4), (7, 3)])
+@pytest.mark.parametrize("T,pad", [(1, 0), (7, 4), (7, 3), (1025, 4)])
 def test_head_norm_gate(dt, heads, P, act, T, pad):
     g = torch.Generator().manual_seed(P)
     y, w = _rand(g, T, heads * P), _rand(g, P)
