@@ -166,7 +166,9 @@ __global__ void __launch_bounds__(NT) ln_residual_kernel(float* __restrict__ x, 
 
 // The same with the row in registers: four numbers per access, CH accesses per thread (W <= 4 NT CH), every row's loads
 // (the stream's and the weights' too) before the first sum, four parts at a time.  us, LDS row / this, W 1024: 4096 tokens
-// 17.8 / 10.7 (half the calls with three parts), 4 tokens 6.5 / 3.0.  W % 4 == 0 and 16-byte (y, parts: 4 numbers) aligned.
+// 17.8 / 10.7 (half the calls with three parts), 4 tokens 6.5 / 3.0.  W % 4 == 0 and 16-byte (y, parts: 4 numbers) aligned;
+// from 256 numbers on (with a copy of x and three parts: 260 numbers, 4096 tokens 12.9 / 12.0, 4 tokens 5.4 / 4.9; 64, where most
+// threads have no run, 8.2 / 9.8 and 4.8 / 4.5).
 template <typename T, int CH>
 __global__ void __launch_bounds__(NT) ln_residual4_kernel(float* __restrict__ x, const T* __restrict__ y,
                                                           const T* __restrict__ parts, const float* __restrict__ pw, int K,
@@ -963,7 +965,7 @@ int edge_sm_ln_residual(float* x, const void* y, const void* parts, const float*
                         int rows, int W, float eps, int f32, hipStream_t st) {
   if (rows == 0) return 0;
   if ((size_t)W * 4 > 60 * 1024) return -3;
-  if (W % 4 == 0 && W <= 16 * NT && W > 0 &&
+  if (W % 4 == 0 && W <= 16 * NT && W >= 256 &&
       (((uintptr_t)x | (uintptr_t)w | (uintptr_t)b | (uintptr_t)y | (uintptr_t)parts) & 15) == 0) {
 #define SM_LNR(CH)                                                                                                 \
   SM_T(f32, hipLaunchKernelGGL((ln_residual4_kernel<T, CH>), dim3(rows), dim3(NT), 0, st, x, (const T*)y,           \

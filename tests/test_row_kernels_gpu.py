@@ -25,7 +25,7 @@ def _near(got, ref, dt, scale=1.0):
 
 
 @pytest.mark.parametrize("dt", DT)
-@pytest.mark.parametrize("W", [4, 1020, 1024, 1028, 2048, 4096, 4100, 1022])
+@pytest.mark.parametrize("W", [4, 252, 256, 1020, 1024, 1028, 2048, 4096, 4100, 1022])
 @pytest.mark.parametrize("T,K,with_y", [(3, 0, True), (1, 1, False), (5, 3, True), (2, 4, False), (2, 5, True), (2, 9, False)])
 def test_layer_norm_residual(dt, W, T, K, with_y):
     g = torch.Generator().manual_seed(W + K)
