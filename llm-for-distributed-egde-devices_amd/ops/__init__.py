@@ -475,8 +475,8 @@ def raw_call(*ts: torch.Tensor) -> bool:
 
 def f32_rows_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """Whether ``linear_bf16`` runs ``gemv_f32.hip`` for this call: dense 16-byte-aligned fp32 operands of one GPU, K % 4 == 0,
-    up to 4 rows, or up to 8 rows and 8192 columns (measured at 8 rows: 6784 x 1024 12.1 us against the library's 12.9,
-    32000 x 1024 38 against 33), in a ``raw_call`` (the library product serves the others)."""
+    up to 4 rows, or up to 8 rows of at most 2^22 weights (in a graph, us at 8 rows, here / library: 1024 x 4096 6.2 / 10.0,
+    4096 x 1024 5.9 / 6.0, 6784 x 1024 8.7 / 7.3, 3000 x 12288 36 / 27; at 4 rows 5.6 / 7.3 and 24.9 / 26.4), in a ``raw_call`` (the library product serves the others)."""
     if not (_gpu(x) and x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
         return False
     ts = (x, weight) if bias is None else (x, weight, bias)
@@ -486,7 +486,7 @@ def f32_rows_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tens
     if not (K >= 4 and K % 4 == 0 and N >= 1 and x.shape[-1] == K):
         return False
     M = x.numel() // K
-    if not (1 <= M <= 4 or (4 < M <= 8 and N <= 8192)):
+    if not (1 <= M <= 4 or (4 < M <= 8 and N * K <= 1 << 22)):
         return False
     if bias is not None and (bias.dtype != torch.float32 or tuple(bias.shape) != (N,)):   # others broadcast
         return False

@@ -1,12 +1,12 @@
 // fp32 projection of a few rows: y[M, N] = x[M, K] . W[N, K]^T (+ bias), M <= 8, K % 4 == 0, in fp32 throughout.
 // Bound by reading W once, and below some 16 MB by the launch itself.  W stays in its [N, K] layout (no copy is made): a
 // wave takes R rows by 256 k at a time, each load one contiguous KiB of a row (with 16 rows by 16 k per load, the matrix
-// instruction's layout, the loads themselves were the bound: 1024 x 4096 12.8 us against 5.9 here), the next 256 k on
+// instruction's layout, the loads themselves were the bound: 1024 x 4096, launched one by one, 12.8 us against 5.9 here), the next 256 k on
 // their way meanwhile.  Few rows: KW waves of a workgroup share a row's k (until about 1024 waves are at work) and add up
 // through LDS.  All sums in a fixed order.
-// N x K at 2 rows, us, library / here: 1024 x 384 5.1 / 3.4, 1024 x 1024 8.3 / 3.9, 1024 x 4096 12.2 / 5.9, 4096 x 1024
-// 11.6 / 6.2, 6784 x 1024 12.9 / 8.6, 32000 x 1024 32.6 / 25.7 (5.1 TB/s), 32000 x 2048 59.6 / 44.8; relative error
-// against 64-bit sums 1e-7 here, 2 to 8e-7 there.
+// N x K at 2 rows in a graph, us, library / here: 384 x 1024 5.7 / 3.3, 1024 x 4096 9.9 / 4.1, 4096 x 1024 5.9 / 4.1, 6784 x
+// 1024 7.3 / 4.8, 8192 x 2048 13.1 / 12.2, 32000 x 2048 46 / 40 (6.6 TB/s), 128256 x 2048 187 / 167; relative error against
+// 64-bit sums 1e-7 here, 2 to 8e-7 there.
 #include "common.h"
 
 namespace {
@@ -72,7 +72,7 @@ void launch_f32(const float* x, const float* W, const float* bias, float* y, int
 }  // namespace
 
 // x, W: 16-byte aligned.  5 - 8 rows: two weight rows per wave (four leave no registers for the next loads: 4096 x 1024 at
-// 8 rows 13.7 us, two 7.9, library 11.6)
+// 8 rows, launched one by one, 13.7 us, two 7.9, library 11.6)
 extern "C" int edge_gemv_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K,
                              hipStream_t st) {
   if (M < 1 || M > 8 || N < 1 || K < 4 || K % 4) return -2;

@@ -14,11 +14,11 @@ def _operands(M, N, K, seed=0):
 
 
 @pytest.mark.parametrize("M", [1, 2, 3, 4, 5, 8])
-@pytest.mark.parametrize("N,K", [(1, 4), (3, 252), (4, 256), (5, 260), (33, 1024), (1023, 1028), (1025, 4096), (4097, 516),
-                                 (8192, 768)])
+@pytest.mark.parametrize("N,K", [(1, 4), (3, 252), (4, 256), (5, 260), (33, 1024), (1023, 1028), (1024, 4096), (1025, 4096),
+                                 (4097, 516), (8192, 768)])
 def test_f32_rows(M, N, K):
     x, w, b = _operands(M, N, K, M)
-    assert ops.f32_rows_ok(x, w, b)
+    assert ops.f32_rows_ok(x, w, b) == (M <= 4 or N * K <= 1 << 22)
     for bias in (None, b):
         got = ops.linear_bf16(x, w, bias).double().cpu()
         ref = x.double().cpu() @ w.double().cpu().t() + (0 if bias is None else bias.double().cpu())
