@@ -56,12 +56,14 @@ def test_latent_prompt(D, Dv, H, step, window):
 
 
 @pytest.mark.parametrize("D,Dv", DIMS)
-@pytest.mark.parametrize("pad", [0, 4, 8, 3])
-def test_latent_prompt_rows(D, Dv, pad):
-    """Wide cache rows, no gate, result rows in a wider matrix (whole-line and number-by-number stores)."""
+@pytest.mark.parametrize("pad,first,lines", [(0, 0, True), (8, 0, True), (16, 8, True), (24, 16, True), (8, 4, False), (4, 0, False),
+                                             (3, 1, False), (9, 8, False)])
+def test_latent_prompt_rows(D, Dv, pad, first, lines):
+    """Wide cache rows, no gate, result rows in a wider matrix: whole-line stores where its rows and its start are whole 16
+    bytes (also with room on either side), number by number elsewhere; the columns beside the slice stay."""
     H, T = 8, sum(n for _, _, n in STEPS["edges"])
-    wide = torch.full((T, H * Dv + pad + 1), 7.0, device="cuda:0").bfloat16()
-    for first in (0, 1) if pad else (0,):
-        out = wide[:, first:first + H * Dv] if pad else torch.empty(T, H * Dv, device="cuda:0").bfloat16()
-        _check(STEPS["edges"], H, D, Dv, 50, wide=40, gated=False, out=out, out_scale=0.5)
-    assert (wide[:, H * Dv + 1:] == 7).all()
+    wide = torch.full((T, H * Dv + pad), 7.0, device="cuda:0").bfloat16()
+    out = wide[:, first:first + H * Dv]
+    assert (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0) == lines
+    _check(STEPS["edges"], H, D, Dv, 50, wide=40, gated=False, out=out, out_scale=0.5)
+    assert (wide[:, :first] == 7).all() and (wide[:, first + H * Dv:] == 7).all()
