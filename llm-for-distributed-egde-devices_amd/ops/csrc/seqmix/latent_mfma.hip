@@ -108,7 +108,9 @@ __global__ void __launch_bounds__(LNT) latent_attn_kernel(
   static_assert(D % 32 == 0 && DV % 32 == 0 && DV <= D && L::PIECES % 4 == 0, "panels");
   __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
   const int TM = 32 * (LW / hw);
-  int qt = (int)(gridDim.y - 1 - blockIdx.y), s = 0;         // late query tiles see the most keys: they go first
+  // neighbours share a query tile and differ in heads; late query tiles see the most keys: they go first
+  const int hgs = H / hw, hg = blockIdx.x % hgs;
+  int qt = (int)((gridDim.x - 1 - blockIdx.x) / hgs), s = 0;
   for (; s < n; ++s) {
     const int nq = (seq_len[s] + TM - 1) / TM;
     if (qt < nq) break;
@@ -116,7 +118,7 @@ __global__ void __launch_bounds__(LNT) latent_attn_kernel(
   }
   if (s == n) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 31, g2 = lane >> 5;
-  const int h = blockIdx.x * hw + wave % hw, g = blockIdx.x * hw / (H / G);
+  const int h = hg * hw + wave % hw, g = hg * hw / (H / G);
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
   const int* pt = ptab + (size_t)seq_slot[s] * ptab_ld;
   const int wq0 = qt * TM + wave / hw * 32, tq = wq0 + c, qpos = start + tq;
@@ -299,7 +301,7 @@ int launch_latent(const void* q, const void* gate, int gate_ld, const void* kp, 
                   const int* seq_len, const int* seq_off, const int* ptab, int ptab_ld, void* out, int n, int qtiles, int H,
                   int G, int hw, float sl2, int window, int kld, int out_ld, float out_scale, hipStream_t st) {
   const int vec_out = out_ld % 8 == 0 && (uintptr_t)out % 16 == 0;
-  hipLaunchKernelGGL((latent_attn_kernel<D, DV>), dim3(H / hw, hw == 8 ? 2 * qtiles : qtiles), dim3(LNT), 0, st,
+  hipLaunchKernelGGL((latent_attn_kernel<D, DV>), dim3((H / hw) * (hw == 8 ? 2 * qtiles : qtiles)), dim3(LNT), 0, st,
                      (const bf16_t*)q, (const bf16_t*)gate, gate_ld, (const bf16_t*)kp, seq_slot, seq_start, seq_len, seq_off,
                      ptab, ptab_ld, (bf16_t*)out, n, H, G, hw, sl2, window, kld, out_ld, out_scale, vec_out);
   return (int)hipGetLastError();

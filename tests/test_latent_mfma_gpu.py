@@ -67,3 +67,16 @@ def test_latent_prompt_rows(D, Dv, pad, first, lines):
     assert (out.stride(0) % 8 == 0 and out.data_ptr() % 16 == 0) == lines
     _check(STEPS["edges"], H, D, Dv, 50, wide=40, gated=False, out=out, out_scale=0.5)
     assert (wide[:, :first] == 7).all() and (wide[:, first + H * Dv:] == 7).all()
+
+
+def test_latent_prompt_of_two_million_tokens():
+    """More query tiles than a grid's second dimension may hold; with a window of one token the result is the token's value."""
+    H, D, Dv, T = 8, 128, 96, (1 << 21) + 77
+    g = torch.Generator(device="cuda:0").manual_seed(0)
+    rows = torch.randn((T + 63) // 64, 64, 1, D, generator=g, device="cuda:0", dtype=torch.bfloat16)
+    q = torch.randn(T, H, D, generator=g, device="cuda:0", dtype=torch.bfloat16)
+    meta = S.RaggedMeta.build([(0, 0, T)], torch.arange(rows.shape[0], dtype=torch.int32, device="cuda:0")[None], 64, "cuda:0")
+    out = S.window_pool_attention(q, None, rows, rows[..., :Dv], None, None, meta, D ** -0.5, 1, None)
+    want = rows.view(-1, D)[:T, :Dv]
+    for h in range(H):
+        assert torch.equal(out.view(T, H, Dv)[:, h], want)
