@@ -107,21 +107,23 @@ __global__ void __launch_bounds__(LNT) latent_attn_kernel(
   constexpr int KK = D / 16, DB = DV / 32, NB = L::NB, WC = L::WC;
   static_assert(D % 32 == 0 && DV % 32 == 0 && DV <= D && L::PIECES % 4 == 0, "panels");
   __shared__ __attribute__((aligned(1024))) char smem[L::LDS];
-  const int TM = 32 * (LW / hw);
+  // (hw is a power of two: a step of 100 short sequences walks up to 100 lengths here, and a division each cost 5 us)
+  const int lhw = __ffs(hw) - 1, ltm = 8 - lhw, TM = 1 << ltm;
+  static_assert(LW == 8, "32 queries by 8 waves");
   // neighbours share a query tile and differ in heads; late query tiles see the most keys: they go first
   const int hgs = H / hw, hg = blockIdx.x % hgs;
   int qt = (int)((gridDim.x - 1 - blockIdx.x) / hgs), s = 0;
   for (; s < n; ++s) {
-    const int nq = (seq_len[s] + TM - 1) / TM;
+    const int nq = (seq_len[s] + TM - 1) >> ltm;
     if (qt < nq) break;
     qt -= nq;
   }
   if (s == n) return;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), c = lane & 31, g2 = lane >> 5;
-  const int h = hg * hw + wave % hw, g = hg * hw / (H / G);
+  const int h = hg * hw + (wave & (hw - 1)), g = hg * hw / (H / G);
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
   const int* pt = ptab + (size_t)seq_slot[s] * ptab_ld;
-  const int wq0 = qt * TM + wave / hw * 32, tq = wq0 + c, qpos = start + tq;
+  const int wq0 = qt * TM + (wave >> lhw) * 32, tq = wq0 + c, qpos = start + tq;
   const int imin = start + qt * TM, imax = start + min(len, qt * TM + TM) - 1;
   const int t0 = window > 0 ? max(0, imin - window + 1) / LKT : 0, ntiles = imax / LKT - t0 + 1;
 
