@@ -319,7 +319,8 @@ int edge_sm_attention_latent(const void* q, const void* gate, int gate_ld, const
                              const int* seq_start, const int* seq_len, const int* seq_off, const int* ptab, int ptab_ld,
                              void* out, int n, int qtiles, int H, int G, int D, int Dv, float scale_log2, int window, int kld,
                              int out_ld, float out_scale, hipStream_t st) {
-  const int R = H / G, hw = R % 8 == 0 ? 8 : R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
+  // eight heads a workgroup once that gives one for every CU: on short steps eight waves of 320-wide rows only wait longer
+  const int R = H / G, hw = R % 8 == 0 && 2 * qtiles * (H / 8) >= 256 ? 8 : R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
   if (!(scale_log2 > 0.f) || (int64_t)LKT * kld * 2 > INT_MAX) return 1;   // the maximum is taken before the scale
 #define LAT(DD, DDV)                                                                                                       \
   return launch_latent<DD, DDV>(q, gate, gate_ld, kp, seq_slot, seq_start, seq_len, seq_off, ptab, ptab_ld, out, n, qtiles, \
