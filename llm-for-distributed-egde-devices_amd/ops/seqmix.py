@@ -775,11 +775,11 @@ def delta_prepare_head(qkv: torch.Tensor, u: torch.Tensor, b0: int, a0: int, dt_
     return torch.cat([q.reshape(T, GN), k.reshape(T, GN), g, beta], -1)
 
 
-# bf16 steps whose longest portion has this many tokens run the delta rule over 64-token chunks (csrc/seqmix/delta_chunk.hip);
-# us, token by token / chunks, 16 heads: 64 x 64 states, 128 tokens 32 / 43, 1500 + 77 tokens 348 / 86, 4096 tokens 916 / 172;
-# 128 x 128 states, 96 tokens 38 / 49, two portions of 512 208 / 128, 4096 tokens 1521 / 378.  Against 64 bits the chunks
-# are 1.4e-7 to 2.8e-7 off (token by token 0.8e-7): nothing beside bf16 activations, but fp32 steps stay token by token
-DELTA_CHUNK_MIN = int(__import__("os").environ.get("EDGELLM_DELTA_CHUNK_MIN", "160"))
+# bf16 steps whose longest portion has this many tokens run the delta rule over 64-token chunks (csrc/seqmix/delta_chunk.hip,
+# fp64 inside); us, token by token / chunks, 16 heads: 64 x 64 states, 160 tokens 39 / 53, 256 tokens 60 / 55, 4096 tokens 916 /
+# 257; 128 x 128 states, 256 tokens 94 / 92, two portions of 512 194 / 118, 4096 tokens 1512 / 527.  Against 64 bits the chunks
+# are 0.3e-7 to 0.5e-7 off, token by token 0.8e-7 to 3.2e-7
+DELTA_CHUNK_MIN = int(__import__("os").environ.get("EDGELLM_DELTA_CHUNK_MIN", "256"))
 
 
 def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, meta: RaggedMeta, heads: int,

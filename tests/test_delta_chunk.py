@@ -22,24 +22,27 @@ def recurrence(prep, v, S, G, H, N, channel):
     return out, S
 
 
-def inputs(lens, starts, H, G, N, P, channel, decay, seed=0):
+def inputs(lens, starts, H, G, N, P, channel, decay, seed=0, keys="random"):
     g = torch.Generator().manual_seed(seed)
     T = sum(lens)
     meta = seqmix.RaggedMeta.build([(len(lens) - 1 - i, st, L) for i, (st, L) in enumerate(zip(starts, lens))],
                                    torch.zeros(len(lens), 4, dtype=torch.int32, device="cuda"), 64, "cuda")
     qkv = torch.nn.functional.silu(torch.randn(T, 2 * G * N + H * P, generator=g)).bfloat16().cuda()
-    unit = torch.nn.functional.normalize(torch.randn(2, T, G, N, generator=g), dim=-1)
+    unit = torch.randn(2, T, G, N, generator=g)
+    if keys == "alike":                                # about 0.98 of each other's direction
+        unit = torch.nn.functional.normalize(unit, dim=-1) * 0.14 + torch.nn.functional.normalize(torch.randn(G, N, generator=g), dim=-1)
+    unit = torch.nn.functional.normalize(unit, dim=-1)
     D = H * (N if channel else 1)
     d = {"weak": 1.0 - 1e-4 * torch.rand(T, D, generator=g), "usual": torch.rand(T, D, generator=g) ** 0.1,
-         "strong": torch.rand(T, D, generator=g) * 1e-3, "mixed": torch.where(torch.rand(T, D, generator=g) < 0.1, 0.0, 0.99)}[decay]
-    prep = torch.cat([(unit[0] * N ** -0.5).reshape(T, -1), unit[1].reshape(T, -1), d, torch.rand(T, H, generator=g)], -1)
+         "none": torch.ones(T, D), "strong": torch.rand(T, D, generator=g) * 1e-3, "mixed": torch.where(torch.rand(T, D, generator=g) < 0.1, 0.0, 0.99)}[decay]
+    prep = torch.cat([(unit[0] * N ** -0.5).reshape(T, -1), unit[1].reshape(T, -1), d,
+                      (0.97 + 0.03 * torch.rand(T, H, generator=g)) if keys == "alike" else torch.rand(T, H, generator=g)], -1)
     state = torch.randn(len(lens), H, N, P, generator=g)
     return prep.cuda(), qkv, state.cuda(), meta
 
 
-# both forms sum in fp32 (2^-24 relative per operation); 64 terms a chunk and logs that add up to a few hundred leave about
-# 3e-7 of the output's size, and a token's own rounding the same: bound 2e-6
-TOL = 2e-6
+# fp64 inside; inputs of the outputs' products and the states rounded to fp32 (2^-25 rms 3e-8 each): bound 2e-7
+TOL = 2e-7
 
 
 @pytest.mark.parametrize("channel", [True, False])
@@ -63,8 +66,27 @@ def test_chunks_against_the_recurrence(lens, starts, H, G, N, P, channel, decay,
         assert (state[slot].double().cpu() - S).norm() < TOL * S.norm().clamp_min(1e-3)
 
 
+@pytest.mark.parametrize("channel", [True, False])
+@pytest.mark.parametrize("keys,decay", [("random", "usual"), ("random", "weak"), ("random", "strong"), ("alike", "none"), ("alike", "weak")])
+@pytest.mark.parametrize("H,G,N,P", [(4, 2, 64, 64), (2, 2, 128, 64), (2, 1, 200, 70)])
+def test_chunks_are_no_further_off_than_the_recurrence_in_fp32(H, G, N, P, channel, keys, decay, monkeypatch):
+    """Outputs and states, also with keys that resemble each other, where a chunk's terms cancel."""
+    prep, qkv, state, meta = inputs((321, 70), (0, 9), H, G, N, P, channel, decay, 3, keys)
+    p, v, off = prep.double().cpu(), qkv[:, 2 * G * N:].double().cpu().view(len(prep), H, P), [(m[3], m[2], m[0], m[1]) for m in meta.host]
+    want = [recurrence(p[o:o + n], v[o:o + n], state[s].double().cpu() * (st > 0), G, H, N, channel) for o, n, s, st in off]
+    err = []
+    for least in (1 << 30, 1):
+        monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", least)
+        S = state.clone()
+        y = seqmix.delta_rule_scan(prep, qkv, S, meta, H, G, N, P).double().cpu()
+        err.append([(((y[o:o + n].view(n, H, P) - w[0]).norm() / w[0].norm()).item(), ((S[s].double().cpu() - w[1]).norm() / w[1].norm()).item())
+                    for (o, n, s, _), w in zip(off, want)])
+    steps, chunks = torch.tensor(err[0]), torch.tensor(err[1])
+    assert (chunks <= steps).all(), (chunks, steps)
+
+
 def test_the_longest_portion_decides_and_fp32_steps_stay_token_by_token(monkeypatch):
-    prep, qkv, state, meta = inputs((200, 40), (0, 9), 2, 2, 64, 32, True, "usual", 1)
+    prep, qkv, state, meta = inputs((300, 40), (0, 9), 2, 2, 64, 32, True, "usual", 1)
     a, b = state.clone(), state.clone()
     chunks = seqmix.delta_rule_scan(prep, qkv, a, meta, 2, 2, 64, 32)
     monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1 << 30)
