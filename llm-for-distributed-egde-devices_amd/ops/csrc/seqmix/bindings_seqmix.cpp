@@ -81,11 +81,11 @@ int edge_sm_delta_prep(const void* qkv, int Cq, const void* u, int ld, int b0, c
                        const float* A_log, float* prep, int rows, int H, int G, int N, int f32, hipStream_t st);
 int edge_sm_delta_scan(const float* prep, int prep_ld, const void* qkv, int Cq, float* state, const int* seq_slot,
                        const int* seq_start, const int* seq_len, const int* seq_off, float* y, int n, int H, int G, int N,
-                       int P, int GD, int f32, hipStream_t st);
+                       int P, int GD, int below, int f32, hipStream_t st);
 int64_t edge_sm_delta_chunk_floats(int64_t chunks, int64_t H, int64_t N, int64_t P);
 int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int Cq, float* state, const int* seq_slot,
                           const int* seq_start, const int* seq_len, const int* seq_off, float* scratch, float* y, int rows, int n,
-                          int chunks, int max_chunks, int H, int G, int N, int P, int GD, int f32, hipStream_t st);
+                          int chunks, int max_chunks, int least, int H, int G, int N, int P, int GD, int f32, hipStream_t st);
 int edge_sm_moe_route(const void* h, int W, const float* router, const float* bias, int E, int top, float scale, float* z,
                       int* idx, float* wts, int rows, int sigm, int f32, hipStream_t st);
 int edge_sm_hyper_read_norm(const float* X, const float* in_w, const float* w, void* y, int rows, int S, int W, float eps,
@@ -672,7 +672,7 @@ at::Tensor sm_delta_prep(const at::Tensor& qkv, const at::Tensor& u, int64_t b0,
 
 at::Tensor sm_delta_scan(const at::Tensor& prep, const at::Tensor& qkv, at::Tensor& state, const at::Tensor& seq_slot,
                          const at::Tensor& seq_start, const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n,
-                         int64_t H, int64_t G, int64_t N, int64_t P, int64_t chunks, int64_t max_chunks) {
+                         int64_t H, int64_t G, int64_t N, int64_t P, int64_t chunks, int64_t max_chunks, int64_t least) {
   chk_f32(prep, "prep");
   chk_f32(state, "state");
   chk_act2(qkv, "qkv");
@@ -689,19 +689,22 @@ at::Tensor sm_delta_scan(const at::Tensor& prep, const at::Tensor& qkv, at::Tens
               "sequence metadata: [n]");
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
   auto y = at::empty({T, H * P}, prep.options());
-  if (max_chunks > 0) {                                      // long portions: 64-token chunks in parallel
+  // portions of `least` tokens or more (`chunks` 64-token chunks in all, `max_chunks` the longest) over chunks, the others
+  // token by token
+  if (max_chunks > 0) {
     auto scratch = at::empty({edge_sm_delta_chunk_floats(chunks, H, N, P)}, prep.options());
     check(edge_sm_delta_chunked(prep.data_ptr<float>(), (int)prep.size(1), qkv.data_ptr(), (int)qkv.size(1), state.data_ptr<float>(),
                                 seq_slot.data_ptr<int>(), seq_start.data_ptr<int>(), seq_len.data_ptr<int>(),
                                 seq_off.data_ptr<int>(), scratch.data_ptr<float>(), y.data_ptr<float>(), (int)T, (int)n,
-                                (int)chunks, (int)max_chunks, (int)H, (int)G, (int)N, (int)P, GD, f32(qkv), stream()),
+                                (int)chunks, (int)max_chunks, (int)least, (int)H, (int)G, (int)N, (int)P, GD, f32(qkv), stream()),
           "sm_delta_scan (chunks)");
-    return y;
   }
-  check(edge_sm_delta_scan(prep.data_ptr<float>(), (int)prep.size(1), qkv.data_ptr(), (int)qkv.size(1), state.data_ptr<float>(),
-                           seq_slot.data_ptr<int>(), seq_start.data_ptr<int>(), seq_len.data_ptr<int>(),
-                           seq_off.data_ptr<int>(), y.data_ptr<float>(), (int)n, (int)H, (int)G, (int)N, (int)P, GD,
-                           f32(qkv), stream()), "sm_delta_scan");
+  if (least > 1)
+    check(edge_sm_delta_scan(prep.data_ptr<float>(), (int)prep.size(1), qkv.data_ptr(), (int)qkv.size(1), state.data_ptr<float>(),
+                             seq_slot.data_ptr<int>(), seq_start.data_ptr<int>(), seq_len.data_ptr<int>(),
+                             seq_off.data_ptr<int>(), y.data_ptr<float>(), (int)n, (int)H, (int)G, (int)N, (int)P, GD,
+                             (int)least, f32(qkv), stream()),
+          "sm_delta_scan");
   return y;
 }
 

@@ -41,6 +41,14 @@ __device__ __forceinline__ bool finite4(const v4d& x) {
   return d[0] == 0. && d[1] == 0. && d[2] == 0. && d[3] == 0.;
 }
 
+// chunks of a portion: none below `least` tokens (those run token by token), and a portion's first among all of the step
+__device__ __forceinline__ int chunks_of(int len, int least) { return len < least ? 0 : (len + CL - 1) / CL; }
+__device__ __forceinline__ size_t first_chunk(const int* __restrict__ seq_len, int s, int least) {
+  size_t b = 0;
+  for (int i = 0; i < s; ++i) b += chunks_of(seq_len[i], least);
+  return b;
+}
+
 // Scratch per (chunk, head), NP = 64, 128 or 256 channels (zero past N) and PP = P rounded up to 16:
 //   fp64  M [4 token blocks][NP / 16][token][PERM channel]  U (later W) [64][PP]  Cs [4][4][token][PERM earlier token]
 //         cdec [NP / 16][PERM channel]
@@ -55,7 +63,7 @@ template <typename T, bool VEC, bool ONE>
 __global__ void __launch_bounds__(NT, 2) delta_chunk_solve_kernel(const float* __restrict__ prep, int prep_ld,
                                                                   const T* __restrict__ qkv, int Cq,
                                                                   const int* __restrict__ seq_len, const int* __restrict__ seq_off,
-                                                                  DeltaScratch sc, int H, int G, int N, int NP, int P, int PP) {
+                                                                  DeltaScratch sc, int least, int H, int G, int N, int NP, int P, int PP) {
   constexpr int NK = 32, LQ = NK + 4, LA = CL + 4, LG = ONE ? 1 : CL;
   __shared__ __attribute__((aligned(16))) float Q_s[CL][LQ], K_s[CL][LQ], G_s[LG][LQ];
   // decays of a token's 16-token block up to and with it / after it; A takes their place
@@ -66,9 +74,9 @@ __global__ void __launch_bounds__(NT, 2) delta_chunk_solve_kernel(const float* _
   auto E_s = reinterpret_cast<double(*)[LQ]>(be_s + CL * LQ);
   auto A_s = reinterpret_cast<double(*)[LA]>(be_s);
   const int c = blockIdx.x, s = blockIdx.y, h = blockIdx.z, len = seq_len[s];
-  if (c * CL >= len) return;
+  if (c >= chunks_of(len, least)) return;
   const int tc = min(CL, len - c * CL), GN = G * N, GD = ONE ? 1 : N;
-  const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL, cb = ((size_t)chunk_base(seq_len, s) + c) * H + h;
+  const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL, cb = (first_chunk(seq_len, s, least) + c) * H + h;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
   const float* pr = prep + row0 * prep_ld;
   const float *qb = pr + (h / (H / G)) * N, *kb = qb + GN, *gb = pr + 2 * GN + h * GD, *bb = pr + 2 * GN + H * GD + h;
@@ -365,14 +373,15 @@ template <int KS, int D>
 __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch sc, float* __restrict__ state,
                                                                    const int* __restrict__ seq_slot,
                                                                    const int* __restrict__ seq_start,
-                                                                   const int* __restrict__ seq_len, int H, int N, int P, int PP) {
+                                                                   const int* __restrict__ seq_len, int least, int H, int N, int P,
+                                                                   int PP) {
   constexpr int NP = 64 * KS, UE = 4 / KS;                   // rows of 16 numbers: four rows take each bank twice, the least
   __shared__ double S_s[NP][16], W_s[CL][16], P_s[KS > 1 ? KS : 1][KS > 1 ? CL : 1][16];
-  const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * 16, tid = threadIdx.x;
+  const int p0 = blockIdx.x * 16, h = blockIdx.y, s = blockIdx.z, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4, p = p0 + l16;
-  const int tb = wave & 3, kq = wave >> 2, n0 = 16 * wave, len = seq_len[s], nc = (len + CL - 1) / CL;
+  const int tb = wave & 3, kq = wave >> 2, n0 = 16 * wave, nc = chunks_of(seq_len[s], least);
   if (nc == 0) return;
-  const size_t cb0 = (size_t)chunk_base(seq_len, s);
+  const size_t cb0 = first_chunk(seq_len, s, least);
   float* st = state + ((size_t)seq_slot[s] * H + h) * N * P;
   const bool cont = seq_start[s] > 0;
   v4d S;
@@ -471,13 +480,13 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
 // workgroup share the state and W tiles, nothing else is read twice.
 template <int PT>
 __global__ void __launch_bounds__(NT) delta_chunk_out_kernel(DeltaScratch sc, const int* __restrict__ seq_len,
-                                                             const int* __restrict__ seq_off, float* __restrict__ y, int H, int NP,
-                                                             int P, int PP, int ntp) {
+                                                             const int* __restrict__ seq_off, float* __restrict__ y, int least, int H,
+                                                             int NP, int P, int PP, int ntp) {
   const int c = blockIdx.x / ntp, t0 = (blockIdx.x % ntp) * PT, s = blockIdx.y, h = blockIdx.z, len = seq_len[s];
-  if (c * CL >= len) return;
+  if (c >= chunks_of(len, least)) return;
   const int tc = min(CL, len - c * CL), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
   if (16 * wave >= tc) return;
-  const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL, cb = ((size_t)chunk_base(seq_len, s) + c) * H + h;
+  const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL, cb = (first_chunk(seq_len, s, least) + c) * H + h;
   const int at = l16 * 16 + 4 * g4;
   const float *qp = sc.Qe + cb * CL * NP + (size_t)wave * NP * 16 + at, *sp = sc.sin + cb * NP * PP + at;
   const double *cp = sc.Cs + cb * CL * CL + wave * 4 * 256, *wp = sc.U + cb * CL * PP + l16;
@@ -539,7 +548,7 @@ int64_t edge_sm_delta_chunk_floats(int64_t chunks, int64_t H, int64_t N, int64_t
 
 int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int Cq, float* state, const int* seq_slot,
                           const int* seq_start, const int* seq_len, const int* seq_off, float* scratch, float* y, int rows, int n,
-                          int chunks, int max_chunks, int H, int G, int N, int P, int GD, int f32, hipStream_t st) {
+                          int chunks, int max_chunks, int least, int H, int G, int N, int P, int GD, int f32, hipStream_t st) {
   if (n == 0 || rows == 0 || max_chunks <= 0) return 0;
   if (f32 || G <= 0 || H % G || N < 1 || N > 256 || P < 1 || (GD != N && GD != 1)) return -2;
   const int NP = channels(N), PP = (P + 15) & ~15;
@@ -556,24 +565,24 @@ int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int C
   const bool vec = N % 4 == 0 && prep_ld % 4 == 0 && ((uintptr_t)prep & 15) == 0;
 #define SM_DSOLVE(V, ONE)                                                                                           \
   hipLaunchKernelGGL((delta_chunk_solve_kernel<bf16_t, V, ONE>), dim3(max_chunks, n, H), dim3(NT), 0, st, prep, prep_ld, \
-                     (const bf16_t*)qkv, Cq, seq_len, seq_off, sc, H, G, N, NP, P, PP)
+                     (const bf16_t*)qkv, Cq, seq_len, seq_off, sc, least, H, G, N, NP, P, PP)
   if (GD == 1) {
     if (vec) SM_DSOLVE(true, true);
     else SM_DSOLVE(false, true);
   } else if (vec) SM_DSOLVE(true, false);
   else SM_DSOLVE(false, false);
 #undef SM_DSOLVE
-  const dim3 grid(n, H, PP / 16);
+  const dim3 grid(PP / 16, H, n);                            // (a sequence's workgroups are neighbours: on all XCDs)
 #define SM_DSCAN(KS, D)                                                                                                       \
-  hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, D>), grid, dim3(256 * KS), 0, st, sc, state, seq_slot, seq_start, seq_len, H, \
-                     N, P, PP)
+  hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, D>), grid, dim3(256 * KS), 0, st, sc, state, seq_slot, seq_start, seq_len, \
+                     least, H, N, P, PP)
   if (NP == 64) SM_DSCAN(1, 3);
   else if (NP == 128) SM_DSCAN(2, 2);
   else SM_DSCAN(4, 1);
 #undef SM_DSCAN
   const int ntp = (PP + 63) / 64;
-  hipLaunchKernelGGL((delta_chunk_out_kernel<4>), dim3(max_chunks * ntp, n, H), dim3(NT), 0, st, sc, seq_len, seq_off, y, H, NP, P,
-                     PP, ntp);
+  hipLaunchKernelGGL((delta_chunk_out_kernel<4>), dim3(max_chunks * ntp, n, H), dim3(NT), 0, st, sc, seq_len, seq_off, y, least, H,
+                     NP, P, PP, ntp);
   return (int)hipGetLastError();
 }
 

@@ -519,7 +519,7 @@ __global__ void __launch_bounds__(NT) delta_scan_kernel(const float* __restrict_
                                                         int Cq, float* __restrict__ state, const int* __restrict__ seq_slot,
                                                         const int* __restrict__ seq_start, const int* __restrict__ seq_len,
                                                         const int* __restrict__ seq_off, float* __restrict__ y, int H, int G,
-                                                        int N, int P, int GD) {
+                                                        int N, int P, int GD, int below) {
   constexpr int NP = 16 * NR, TC = NR >= 16 ? 4 : (NR >= 8 ? 8 : 16), EL = TC * 3 * NP / NT;   // EL = 12
   constexpr int CW = 16;                                     // value columns per workgroup
   __shared__ __attribute__((aligned(16))) float rows_s[2][TC][3][NP];   // q | k | decay
@@ -527,6 +527,7 @@ __global__ void __launch_bounds__(NT) delta_scan_kernel(const float* __restrict_
   const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * CW, tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6, rg = lane & 15, col = wave * 4 + (lane >> 4), p = p0 + col;
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
+  if (len >= below) return;                                  // (run over chunks)
   const int g = h / (H / G), GN = G * N, HN = H * GD;
   float* st = state + ((size_t)seq_slot[s] * H + h) * N * P;
   float S[NR];
@@ -1043,13 +1044,13 @@ int edge_sm_delta_prep(const void* qkv, int Cq, const void* u, int ld, int b0, c
 
 int edge_sm_delta_scan(const float* prep, int prep_ld, const void* qkv, int Cq, float* state, const int* seq_slot,
                        const int* seq_start, const int* seq_len, const int* seq_off, float* y, int n, int H, int G, int N,
-                       int P, int GD, int f32, hipStream_t st) {
+                       int P, int GD, int below, int f32, hipStream_t st) {
   if (n == 0) return 0;
   if (G <= 0 || H % G || N > 256 || (GD != N && GD != 1)) return -2;
   const dim3 grid(n, H, (P + 15) / 16);
 #define SM_DS(NR)                                                                                                  \
   SM_T(f32, hipLaunchKernelGGL((delta_scan_kernel<T, NR>), grid, dim3(NT), 0, st, prep, prep_ld, (const T*)qkv, Cq, \
-                               state, seq_slot, seq_start, seq_len, seq_off, y, H, G, N, P, GD))
+                               state, seq_slot, seq_start, seq_len, seq_off, y, H, G, N, P, GD, below))
   if (N <= 64) SM_DS(4);
   else if (N <= 128) SM_DS(8);
   else SM_DS(16);

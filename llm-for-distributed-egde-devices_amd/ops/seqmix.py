@@ -775,11 +775,38 @@ def delta_prepare_head(qkv: torch.Tensor, u: torch.Tensor, b0: int, a0: int, dt_
     return torch.cat([q.reshape(T, GN), k.reshape(T, GN), g, beta], -1)
 
 
-# bf16 steps whose longest portion has this many tokens run the delta rule over 64-token chunks (csrc/seqmix/delta_chunk.hip,
-# fp64 inside); us, token by token / chunks, 16 heads: 64 x 64 states, 160 tokens 39 / 53, 256 tokens 60 / 55, 4096 tokens 916 /
-# 257; 128 x 128 states, 256 tokens 94 / 92, two portions of 512 194 / 118, 4096 tokens 1512 / 527.  Against 64 bits the chunks
-# are 0.3e-7 to 0.5e-7 off, token by token 0.8e-7 to 3.2e-7
-DELTA_CHUNK_MIN = int(__import__("os").environ.get("EDGELLM_DELTA_CHUNK_MIN", "256"))
+# bf16 portions run the delta rule token by token or over 64-token chunks (csrc/seqmix/delta_chunk.hip, fp64 inside): those of
+# DELTA_LONG tokens or more over chunks where these estimates call that shorter for the step.  Token by token a step waits for
+# its longest portion, or for all tokens together; the chunks have a start (longer with many sequences), a serial part per
+# chunk of the longest portion and a parallel one per chunk and head, and they lose where many portions fill the chip anyway.
+# us measured, 16 heads, all token by token / as chosen, then in brackets what the chunks would have taken: 64 x 64 states, 160
+# tokens 39 (53), 256 60 / 57, 4096 922 / 256, 8 portions of 512 121 (167), 512 beside 15 decode tokens 158 / 88, beside 63
+# 320 / 113; 128 x 128, 300 tokens 106 / 95, two of 512 191 / 128, 4096 1480 / 531, 32 of 512 1102 (1698), 1000 + 300 + 100 362 /
+# 234; 256 x 256, 160 tokens 112 (144), 300 204 / 168, 4096 2945 / 1111, 32 of 512 6339 / 4524.  Against 64 bits the chunks are
+# 0.3e-7 to 0.5e-7 off, token by token 0.8e-7 to 3.2e-7
+# channels: us per token of the longest portion, per token and head | start, per chunk of the longest, per chunk and head
+_DELTA_US = {64: (0.223, 1.2e-3, 35.0, 1.7, 0.13), 128: (0.37, 4.1e-3, 55.0, 2.1, 0.33), 256: (0.68, 24e-3, 90.0, 5.8, 1.0)}
+DELTA_LONG = 128
+# > 0: portions of this many tokens or more run over chunks, whatever the estimates say
+DELTA_CHUNK_MIN = int(__import__("os").environ.get("EDGELLM_DELTA_CHUNK_MIN", "0"))
+
+
+def delta_chunks_from(lens, heads: int, N: int, P: int) -> int:
+    """The length from which on the portions (``lens`` tokens each) of a bf16 step run the delta rule over chunks; 0: none."""
+    least = DELTA_CHUNK_MIN if DELTA_CHUNK_MIN > 0 else DELTA_LONG
+    long, short = [n for n in lens if n >= least], [n for n in lens if 0 < n < least]
+    if not long or N > 256:
+        return 0
+    if DELTA_CHUNK_MIN == 0:
+        NP = 64 if N <= 64 else 128 if N <= 128 else 256
+        a, b, start, serial, each = _DELTA_US[NP]
+        wide = heads * P / NP
+        steps = lambda ls: max(a * max(ls), b * sum(ls) * wide, 5.0) if ls else 0.0
+        chunks = sum((n + 63) // 64 for n in long)
+        over = start * (1 + len(lens) / 64) + serial * ((max(long) + 63) // 64) + each * chunks * wide
+        if over + steps(short) >= steps(long + short):
+            return 0
+    return least if short else 1
 
 
 def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, meta: RaggedMeta, heads: int,
@@ -790,12 +817,12 @@ def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, 
     w = beta (v - S^T k) ;  S <- S + k w^T ;  o = S^T q.  state [slots, heads, N, P] fp32 is read
     (zero for a portion starting at 0) and left at the portion's end.  Returns o fp32 [T, heads P]."""
     if _gpu(prep):
-        chunks = max_chunks = 0                          # 0: one workgroup per (sequence, head, 16 value columns), token by token
-        if meta.max_len >= DELTA_CHUNK_MIN and N <= 256 and qkv.dtype == torch.bfloat16:
-            per = [(h[2] + 63) // 64 for h in meta.host]
-            chunks, max_chunks = sum(per), max(per)
+        # portions below `least` tokens: one workgroup per (sequence, head, 16 value columns), token by token
+        least = delta_chunks_from([h[2] for h in meta.host], heads, N, P) if qkv.dtype == torch.bfloat16 else 0
+        per = [(h[2] + 63) // 64 for h in meta.host if h[2] >= least] if least else []
         return _ext().sm_delta_scan(prep, qkv, state, meta.seq_slot, meta.seq_start, meta.seq_len, meta.seq_off,
-                                    int(meta.n), int(heads), int(kv_heads), int(N), int(P), int(chunks), int(max_chunks))
+                                    int(meta.n), int(heads), int(kv_heads), int(N), int(P), sum(per), max(per, default=0),
+                                    int(least) or 2 ** 31 - 1)
     T, GN, rep = prep.shape[0], kv_heads * N, heads // kv_heads
     if prep.shape[1] == 2 * GN + 2 * heads and N != 1:           # per-head decays: one number for all key channels
         prep = torch.cat([prep[:, :2 * GN], prep[:, 2 * GN:2 * GN + heads].repeat_interleave(N, 1),

@@ -5,7 +5,7 @@ import torch
 import edgellm  # noqa: F401
 from edgellm.ops import seqmix
 
-pytestmark = pytest.mark.gpu
+gpu = pytest.mark.gpu
 
 
 def recurrence(prep, v, S, G, H, N, channel):
@@ -45,6 +45,7 @@ def inputs(lens, starts, H, G, N, P, channel, decay, seed=0, keys="random"):
 TOL = 2e-7
 
 
+@gpu
 @pytest.mark.parametrize("channel", [True, False])
 @pytest.mark.parametrize("decay", ["weak", "usual", "strong", "mixed"])
 @pytest.mark.parametrize("lens,starts,H,G,N,P", [
@@ -66,6 +67,7 @@ def test_chunks_against_the_recurrence(lens, starts, H, G, N, P, channel, decay,
         assert (state[slot].double().cpu() - S).norm() < TOL * S.norm().clamp_min(1e-3)
 
 
+@gpu
 @pytest.mark.parametrize("channel", [True, False])
 @pytest.mark.parametrize("keys,decay", [("random", "usual"), ("random", "weak"), ("random", "strong"), ("alike", "none"), ("alike", "weak")])
 @pytest.mark.parametrize("H,G,N,P", [(4, 2, 64, 64), (2, 2, 128, 64), (2, 1, 200, 70)])
@@ -85,7 +87,35 @@ def test_chunks_are_no_further_off_than_the_recurrence_in_fp32(H, G, N, P, chann
     assert (chunks <= steps).all(), (chunks, steps)
 
 
-def test_the_longest_portion_decides_and_fp32_steps_stay_token_by_token(monkeypatch):
+@pytest.mark.parametrize("lens,H,N,least", [
+    ((160,), 16, 64, 0), ((300,), 16, 64, 1), ((4096,), 4, 64, 1), ((512,) + (1,) * 5, 16, 64, 128), ((512,) + (1,) * 63, 16, 64, 128),
+    ((256,) + (1,) * 255, 16, 64, 0), ((512,) * 8, 16, 64, 0), ((512,) * 8, 4, 64, 1), ((1,) * 40, 16, 64, 0), ((512, 512), 16, 128, 1),
+    ((512,) * 32, 16, 128, 0), ((1000, 300, 0, 100), 16, 128, 128), ((160,), 4, 256, 0), ((512,) * 32, 16, 256, 1),
+    ((4096,), 16, 257, 0), ((), 16, 64, 0)])
+def test_portions_take_the_shorter_form(lens, H, N, least):
+    """The length from which on portions run over chunks (1: all of them do)."""
+    assert seqmix.delta_chunks_from(lens, H, N, N) == least
+
+
+@gpu
+@pytest.mark.parametrize("channel", [True, False])
+def test_long_and_short_portions_of_one_step(channel, monkeypatch):
+    """Long ones over chunks, the others token by token, each with its own slot; portions at the line itself."""
+    lens, starts, H, G, N, P = (130, 1, 64, 16, 63, 200), (3, 700, 0, 0, 9, 1), 4, 2, 64, 48
+    prep, qkv, state, meta = inputs(lens, starts, H, G, N, P, channel, "usual", 4)
+    res = []
+    for least in (64, 1, 1 << 30):
+        monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", least)
+        S = state.clone()
+        res.append((seqmix.delta_rule_scan(prep, qkv, S, meta, H, G, N, P), S))
+    (y, S), (yc, Sc), (yt, St) = res
+    for slot, _, n, off in meta.host:
+        w, Sw = (yc, Sc) if n >= 64 else (yt, St)
+        assert torch.equal(y[off:off + n], w[off:off + n]) and torch.equal(S[slot], Sw[slot])
+
+
+@gpu
+def test_long_portions_run_over_chunks_and_fp32_steps_stay_token_by_token(monkeypatch):
     prep, qkv, state, meta = inputs((300, 40), (0, 9), 2, 2, 64, 32, True, "usual", 1)
     a, b = state.clone(), state.clone()
     chunks = seqmix.delta_rule_scan(prep, qkv, a, meta, 2, 2, 64, 32)
@@ -99,6 +129,7 @@ def test_the_longest_portion_decides_and_fp32_steps_stay_token_by_token(monkeypa
     assert torch.equal(y, seqmix.delta_rule_scan(prep, qkv.float(), d, meta, 2, 2, 64, 32)) and torch.equal(c, d)
 
 
+@gpu
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
 def test_a_value_that_is_not_finite_reaches_no_earlier_token(bad, monkeypatch):
     monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1)
