@@ -85,7 +85,7 @@ int edge_sm_delta_scan(const float* prep, int prep_ld, const void* qkv, int Cq, 
 int64_t edge_sm_delta_chunk_floats(int64_t chunks, int64_t H, int64_t N, int64_t P);
 int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int Cq, float* state, const int* seq_slot,
                           const int* seq_start, const int* seq_len, const int* seq_off, float* scratch, float* y, int rows, int n,
-                          int chunks, int max_chunks, int least, int H, int G, int N, int P, int GD, int f32, hipStream_t st);
+                          int room, int most, int max_chunks, int least, int H, int G, int N, int P, int GD, int f32, hipStream_t st);
 int edge_sm_moe_route(const void* h, int W, const float* router, const float* bias, int E, int top, float scale, float* z,
                       int* idx, float* wts, int rows, int sigm, int f32, hipStream_t st);
 int edge_sm_hyper_read_norm(const float* X, const float* in_w, const float* w, void* y, int rows, int S, int W, float eps,
@@ -672,7 +672,7 @@ at::Tensor sm_delta_prep(const at::Tensor& qkv, const at::Tensor& u, int64_t b0,
 
 at::Tensor sm_delta_scan(const at::Tensor& prep, const at::Tensor& qkv, at::Tensor& state, const at::Tensor& seq_slot,
                          const at::Tensor& seq_start, const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n,
-                         int64_t H, int64_t G, int64_t N, int64_t P, int64_t chunks, int64_t max_chunks, int64_t least) {
+                         int64_t H, int64_t G, int64_t N, int64_t P, int64_t room, int64_t most, int64_t max_chunks, int64_t least) {
   chk_f32(prep, "prep");
   chk_f32(state, "state");
   chk_act2(qkv, "qkv");
@@ -689,14 +689,17 @@ at::Tensor sm_delta_scan(const at::Tensor& prep, const at::Tensor& qkv, at::Tens
               "sequence metadata: [n]");
   c10::hip::HIPGuardMasqueradingAsCUDA guard(qkv.device());
   auto y = at::empty({T, H * P}, prep.options());
-  // portions of `least` tokens or more (`chunks` 64-token chunks in all, `max_chunks` the longest) over chunks, the others
-  // token by token
+  // portions of `least` tokens or more over 64-token chunks (`max_chunks`: the longest's), `most` of each portion's at a time,
+  // scratch for `room` chunks; the others token by token
+  TORCH_CHECK(max_chunks >= 0 && (max_chunks == 0 || (room >= 1 && most >= 1 && most <= max_chunks)) &&
+                  ((max_chunks > 0 && least >= 1) || least > T) && (least > 1 || most < max_chunks || room * 64 >= T),
+              "delta rule: chunk counts");
   if (max_chunks > 0) {
-    auto scratch = at::empty({edge_sm_delta_chunk_floats(chunks, H, N, P)}, prep.options());
+    auto scratch = at::empty({edge_sm_delta_chunk_floats(room, H, N, P)}, prep.options());
     check(edge_sm_delta_chunked(prep.data_ptr<float>(), (int)prep.size(1), qkv.data_ptr(), (int)qkv.size(1), state.data_ptr<float>(),
                                 seq_slot.data_ptr<int>(), seq_start.data_ptr<int>(), seq_len.data_ptr<int>(),
                                 seq_off.data_ptr<int>(), scratch.data_ptr<float>(), y.data_ptr<float>(), (int)T, (int)n,
-                                (int)chunks, (int)max_chunks, (int)least, (int)H, (int)G, (int)N, (int)P, GD, f32(qkv), stream()),
+                                (int)room, (int)most, (int)max_chunks, (int)least, (int)H, (int)G, (int)N, (int)P, GD, f32(qkv), stream()),
           "sm_delta_scan (chunks)");
   }
   if (least > 1)
@@ -1337,6 +1340,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_latent_write", &sm_latent_write);
   m.def("sm_delta_prep", &sm_delta_prep);
   m.def("sm_delta_scan", &sm_delta_scan);
+  m.def("sm_delta_chunk_floats", &edge_sm_delta_chunk_floats);
   m.def("sm_moe_route", &sm_moe_route);
   m.def("sm_moe_experts", &sm_moe_experts);
   m.def("sm_moe_gemm_ok", &sm_moe_gemm_ok);

@@ -21,7 +21,8 @@
 //
 // Bound: token by token, every token costs a chain of two row sums (about 530 clocks); here the chain is two products
 // and two barriers per 64 tokens, in fp64 at half the rate of fp32.  16 heads, 4096 tokens, us, token by token / this: 64 x 64
-// states 916 / 257 (170 in fp32), 128 x 128 states 1512 / 527 (373 in fp32); 512 tokens 114 / 67 and 181 / 107.
+// states 916 / 257 ((1) 115, (2) 140, (3) 37; 170 in fp32), 128 x 128 states 1512 / 527 ((2) 267, (3) 102; 373 in fp32); 512 tokens
+// 114 / 67 and 181 / 107.
 #include "seqmix_common.h"
 
 namespace {
@@ -41,12 +42,19 @@ __device__ __forceinline__ bool finite4(const v4d& x) {
   return d[0] == 0. && d[1] == 0. && d[2] == 0. && d[3] == 0.;
 }
 
-// chunks of a portion: none below `least` tokens (those run token by token), and a portion's first among all of the step
-__device__ __forceinline__ int chunks_of(int len, int least) { return len < least ? 0 : (len + CL - 1) / CL; }
-__device__ __forceinline__ size_t first_chunk(const int* __restrict__ seq_len, int s, int least) {
-  size_t b = 0;
-  for (int i = 0; i < s; ++i) b += chunks_of(seq_len[i], least);
-  return b;
+// What one launch covers: of every portion of `least` tokens or more (shorter ones run token by token) the chunks c0 .. c0 + most
+// - 1, for at most `room` chunks of scratch in all
+struct DeltaPart {
+  int least, c0, most, room;
+};
+__device__ __forceinline__ int chunks_of(int len, const DeltaPart& dp) {
+  return len < dp.least ? 0 : min(max((len + CL - 1) / CL - dp.c0, 0), dp.most);
+}
+// a portion's first chunk among those of the launch, and whether all of its chunks have room (the host counted them)
+__device__ __forceinline__ bool first_chunk(const int* __restrict__ seq_len, int s, const DeltaPart& dp, size_t& b) {
+  b = 0;
+  for (int i = 0; i < s; ++i) b += chunks_of(seq_len[i], dp);
+  return b + chunks_of(seq_len[s], dp) <= (size_t)dp.room;
 }
 
 // Scratch per (chunk, head), NP = 64, 128 or 256 channels (zero past N) and PP = P rounded up to 16:
@@ -63,7 +71,7 @@ template <typename T, bool VEC, bool ONE>
 __global__ void __launch_bounds__(NT, 2) delta_chunk_solve_kernel(const float* __restrict__ prep, int prep_ld,
                                                                   const T* __restrict__ qkv, int Cq,
                                                                   const int* __restrict__ seq_len, const int* __restrict__ seq_off,
-                                                                  DeltaScratch sc, int least, int H, int G, int N, int NP, int P, int PP) {
+                                                                  DeltaScratch sc, DeltaPart dp, int H, int G, int N, int NP, int P, int PP) {
   constexpr int NK = 32, LQ = NK + 4, LA = CL + 4, LG = ONE ? 1 : CL;
   __shared__ __attribute__((aligned(16))) float Q_s[CL][LQ], K_s[CL][LQ], G_s[LG][LQ];
   // decays of a token's 16-token block up to and with it / after it; A takes their place
@@ -74,9 +82,11 @@ __global__ void __launch_bounds__(NT, 2) delta_chunk_solve_kernel(const float* _
   auto E_s = reinterpret_cast<double(*)[LQ]>(be_s + CL * LQ);
   auto A_s = reinterpret_cast<double(*)[LA]>(be_s);
   const int c = blockIdx.x, s = blockIdx.y, h = blockIdx.z, len = seq_len[s];
-  if (c >= chunks_of(len, least)) return;
-  const int tc = min(CL, len - c * CL), GN = G * N, GD = ONE ? 1 : N;
-  const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL, cb = (first_chunk(seq_len, s, least) + c) * H + h;
+  size_t cb;
+  if (c >= chunks_of(len, dp) || !first_chunk(seq_len, s, dp, cb)) return;
+  const int t0 = (dp.c0 + c) * CL, tc = min(CL, len - t0), GN = G * N, GD = ONE ? 1 : N;
+  const size_t row0 = (size_t)seq_off[s] + t0;
+  cb = (cb + c) * H + h;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
   const float* pr = prep + row0 * prep_ld;
   const float *qb = pr + (h / (H / G)) * N, *kb = qb + GN, *gb = pr + 2 * GN + h * GD, *bb = pr + 2 * GN + H * GD + h;
@@ -373,17 +383,17 @@ template <int KS, int D>
 __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch sc, float* __restrict__ state,
                                                                    const int* __restrict__ seq_slot,
                                                                    const int* __restrict__ seq_start,
-                                                                   const int* __restrict__ seq_len, int least, int H, int N, int P,
+                                                                   const int* __restrict__ seq_len, DeltaPart dp, int H, int N, int P,
                                                                    int PP) {
   constexpr int NP = 64 * KS, UE = 4 / KS;                   // rows of 16 numbers: four rows take each bank twice, the least
   __shared__ double S_s[NP][16], W_s[CL][16], P_s[KS > 1 ? KS : 1][KS > 1 ? CL : 1][16];
   const int p0 = blockIdx.x * 16, h = blockIdx.y, s = blockIdx.z, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4, p = p0 + l16;
-  const int tb = wave & 3, kq = wave >> 2, n0 = 16 * wave, nc = chunks_of(seq_len[s], least);
-  if (nc == 0) return;
-  const size_t cb0 = first_chunk(seq_len, s, least);
+  const int tb = wave & 3, kq = wave >> 2, n0 = 16 * wave, nc = chunks_of(seq_len[s], dp);
+  size_t cb0;
+  if (nc == 0 || !first_chunk(seq_len, s, dp, cb0)) return;
   float* st = state + ((size_t)seq_slot[s] * H + h) * N * P;
-  const bool cont = seq_start[s] > 0;
+  const bool cont = seq_start[s] > 0 || dp.c0 > 0;
   v4d S;
 #pragma unroll
   for (int r = 0; r < 4; ++r) S[r] = (cont && n0 + 4 * r + g4 < N && p < P) ? (double)st[(size_t)(n0 + 4 * r + g4) * P + p] : 0.;
@@ -480,13 +490,15 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
 // workgroup share the state and W tiles, nothing else is read twice.
 template <int PT>
 __global__ void __launch_bounds__(NT) delta_chunk_out_kernel(DeltaScratch sc, const int* __restrict__ seq_len,
-                                                             const int* __restrict__ seq_off, float* __restrict__ y, int least, int H,
+                                                             const int* __restrict__ seq_off, float* __restrict__ y, DeltaPart dp, int H,
                                                              int NP, int P, int PP, int ntp) {
   const int c = blockIdx.x / ntp, t0 = (blockIdx.x % ntp) * PT, s = blockIdx.y, h = blockIdx.z, len = seq_len[s];
-  if (c >= chunks_of(len, least)) return;
-  const int tc = min(CL, len - c * CL), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
+  size_t cb;
+  if (c >= chunks_of(len, dp) || !first_chunk(seq_len, s, dp, cb)) return;
+  const int first = (dp.c0 + c) * CL, tc = min(CL, len - first), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
   if (16 * wave >= tc) return;
-  const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL, cb = (first_chunk(seq_len, s, least) + c) * H + h;
+  const size_t row0 = (size_t)seq_off[s] + first;
+  cb = (cb + c) * H + h;
   const int at = l16 * 16 + 4 * g4;
   const float *qp = sc.Qe + cb * CL * NP + (size_t)wave * NP * 16 + at, *sp = sc.sin + cb * NP * PP + at;
   const double *cp = sc.Cs + cb * CL * CL + wave * 4 * 256, *wp = sc.U + cb * CL * PP + l16;
@@ -546,13 +558,16 @@ int64_t edge_sm_delta_chunk_floats(int64_t chunks, int64_t H, int64_t N, int64_t
   return chunks * H * (2 * (CL * NP + CL * PP + CL * CL + NP) + 2 * CL * NP + NP * PP);
 }
 
+// Portions of `least` tokens or more, `most` of their chunks at a time (what the scratch of `room` chunks holds), the state
+// carried from one run of the kernels to the next; max_chunks: the longest portion's.
 int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int Cq, float* state, const int* seq_slot,
                           const int* seq_start, const int* seq_len, const int* seq_off, float* scratch, float* y, int rows, int n,
-                          int chunks, int max_chunks, int least, int H, int G, int N, int P, int GD, int f32, hipStream_t st) {
+                          int room, int most, int max_chunks, int least, int H, int G, int N, int P, int GD, int f32,
+                          hipStream_t st) {
   if (n == 0 || rows == 0 || max_chunks <= 0) return 0;
-  if (f32 || G <= 0 || H % G || N < 1 || N > 256 || P < 1 || (GD != N && GD != 1)) return -2;
+  if (f32 || G <= 0 || H % G || N < 1 || N > 256 || P < 1 || (GD != N && GD != 1) || most < 1 || room < 1) return -2;
   const int NP = channels(N), PP = (P + 15) & ~15;
-  const int64_t CH = (int64_t)chunks * H;
+  const int64_t CH = (int64_t)room * H;
   if (((uintptr_t)scratch & 31) != 0) return -3;
   DeltaScratch sc;
   sc.M = reinterpret_cast<double*>(scratch);
@@ -563,26 +578,30 @@ int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int C
   sc.Kd = sc.Qe + CH * CL * NP;
   sc.sin = sc.Kd + CH * CL * NP;
   const bool vec = N % 4 == 0 && prep_ld % 4 == 0 && ((uintptr_t)prep & 15) == 0;
-#define SM_DSOLVE(V, ONE)                                                                                           \
-  hipLaunchKernelGGL((delta_chunk_solve_kernel<bf16_t, V, ONE>), dim3(max_chunks, n, H), dim3(NT), 0, st, prep, prep_ld, \
-                     (const bf16_t*)qkv, Cq, seq_len, seq_off, sc, least, H, G, N, NP, P, PP)
-  if (GD == 1) {
-    if (vec) SM_DSOLVE(true, true);
-    else SM_DSOLVE(false, true);
-  } else if (vec) SM_DSOLVE(true, false);
-  else SM_DSOLVE(false, false);
-#undef SM_DSOLVE
   const dim3 grid(PP / 16, H, n);                            // (a sequence's workgroups are neighbours: on all XCDs)
-#define SM_DSCAN(KS, D)                                                                                                       \
-  hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, D>), grid, dim3(256 * KS), 0, st, sc, state, seq_slot, seq_start, seq_len, \
-                     least, H, N, P, PP)
-  if (NP == 64) SM_DSCAN(1, 3);
-  else if (NP == 128) SM_DSCAN(2, 2);
-  else SM_DSCAN(4, 1);
-#undef SM_DSCAN
   const int ntp = (PP + 63) / 64;
-  hipLaunchKernelGGL((delta_chunk_out_kernel<4>), dim3(max_chunks * ntp, n, H), dim3(NT), 0, st, sc, seq_len, seq_off, y, least, H,
-                     NP, P, PP, ntp);
+  for (int c0 = 0; c0 < max_chunks; c0 += most) {
+    const DeltaPart dp{least, c0, most, room};
+    const int mc = max_chunks - c0 < most ? max_chunks - c0 : most;
+#define SM_DSOLVE(V, ONE)                                                                                           \
+  hipLaunchKernelGGL((delta_chunk_solve_kernel<bf16_t, V, ONE>), dim3(mc, n, H), dim3(NT), 0, st, prep, prep_ld,    \
+                     (const bf16_t*)qkv, Cq, seq_len, seq_off, sc, dp, H, G, N, NP, P, PP)
+    if (GD == 1) {
+      if (vec) SM_DSOLVE(true, true);
+      else SM_DSOLVE(false, true);
+    } else if (vec) SM_DSOLVE(true, false);
+    else SM_DSOLVE(false, false);
+#undef SM_DSOLVE
+#define SM_DSCAN(KS, D)                                                                                                    \
+  hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, D>), grid, dim3(256 * KS), 0, st, sc, state, seq_slot, seq_start, seq_len, \
+                     dp, H, N, P, PP)
+    if (NP == 64) SM_DSCAN(1, 3);
+    else if (NP == 128) SM_DSCAN(2, 2);
+    else SM_DSCAN(4, 1);
+#undef SM_DSCAN
+    hipLaunchKernelGGL((delta_chunk_out_kernel<4>), dim3(mc * ntp, n, H), dim3(NT), 0, st, sc, seq_len, seq_off, y, dp, H, NP, P,
+                       PP, ntp);
+  }
   return (int)hipGetLastError();
 }
 

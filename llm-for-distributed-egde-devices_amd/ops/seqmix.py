@@ -809,6 +809,20 @@ def delta_chunks_from(lens, heads: int, N: int, P: int) -> int:
     return least if short else 1
 
 
+# scratch of the chunks at one time: portions run in parts of as many chunks as fit, the state carried on.  16 heads of 128 x 128
+# states hold 296 KB a chunk and head
+DELTA_SCRATCH_BYTES = 256 << 20
+
+
+def delta_parts(chunks, room: int) -> Tuple[int, int]:
+    """How portions of ``chunks`` 64-token chunks run through scratch for ``room``: (chunks of each portion at a time, chunks of
+    all portions in the fullest part); (0, 0) when not one of each fits."""
+    most = max(chunks, default=0)
+    while most > 0 and sum(min(c, most) for c in chunks) > room:
+        most = most // 2 if most > 1 else 0
+    return most, sum(min(c, most) for c in chunks)
+
+
 def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, meta: RaggedMeta, heads: int,
                     kv_heads: int, N: int, P: int) -> torch.Tensor:
     """The gated delta rule in fp32.  ``prep`` from ``delta_prepare`` (a decay per
@@ -820,9 +834,11 @@ def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, 
         # portions below `least` tokens: one workgroup per (sequence, head, 16 value columns), token by token
         least = delta_chunks_from([h[2] for h in meta.host], heads, N, P) if qkv.dtype == torch.bfloat16 else 0
         per = [(h[2] + 63) // 64 for h in meta.host if h[2] >= least] if least else []
+        most, room = delta_parts(per, DELTA_SCRATCH_BYTES // (4 * _ext().sm_delta_chunk_floats(1, heads, N, P))) if per else (0, 0)
+        if most == 0:
+            least, per = 2 ** 31 - 1, []
         return _ext().sm_delta_scan(prep, qkv, state, meta.seq_slot, meta.seq_start, meta.seq_len, meta.seq_off,
-                                    int(meta.n), int(heads), int(kv_heads), int(N), int(P), sum(per), max(per, default=0),
-                                    int(least) or 2 ** 31 - 1)
+                                    int(meta.n), int(heads), int(kv_heads), int(N), int(P), room, most, max(per, default=0), least)
     T, GN, rep = prep.shape[0], kv_heads * N, heads // kv_heads
     if prep.shape[1] == 2 * GN + 2 * heads and N != 1:           # per-head decays: one number for all key channels
         prep = torch.cat([prep[:, :2 * GN], prep[:, 2 * GN:2 * GN + heads].repeat_interleave(N, 1),

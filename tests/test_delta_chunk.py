@@ -97,6 +97,30 @@ def test_portions_take_the_shorter_form(lens, H, N, least):
     assert seqmix.delta_chunks_from(lens, H, N, N) == least
 
 
+@pytest.mark.parametrize("chunks,room,parts", [
+    ([64], 64, (64, 64)), ([64], 63, (32, 32)), ([9], 1, (1, 1)), ([8, 3], 9, (4, 7)), ([8, 3], 11, (8, 11)), ([2, 2, 2], 2, (0, 0)),
+    ([1, 1, 1], 3, (1, 3)), ([], 5, (0, 0)), ([7], 0, (0, 0))])
+def test_portions_run_in_parts_that_fit_the_scratch(chunks, room, parts):
+    assert seqmix.delta_parts(chunks, room) == parts
+
+
+@gpu
+@pytest.mark.parametrize("channel,H,N,P", [(True, 4, 64, 48), (False, 2, 128, 64), (True, 2, 200, 70)])
+@pytest.mark.parametrize("room", [3, 5, 7, 0])
+def test_parts_carry_the_state(channel, H, N, P, room, monkeypatch):
+    """Portions of several lengths in parts of one, two and four chunks each, and in none (token by token)."""
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 100)
+    prep, qkv, state, meta = inputs((330, 20, 130, 500), (0, 3, 5, 64), H, 2, N, P, channel, "usual", 5)
+    S, Sw = state.clone(), state.clone()
+    whole = seqmix.delta_rule_scan(prep, qkv, Sw, meta, H, 2, N, P)
+    monkeypatch.setattr(seqmix, "DELTA_SCRATCH_BYTES", room * 4 * seqmix._ext().sm_delta_chunk_floats(1, H, N, P))
+    y = seqmix.delta_rule_scan(prep, qkv, S, meta, H, 2, N, P)
+    # the state is rounded to fp32 between parts (2^-25 rms 3e-8 of its size each time); room 0: the recurrence in fp32
+    tol = 2e-7 if room else 6e-7
+    assert (y - whole).norm() < tol * whole.norm() and (S - Sw).norm() < tol * Sw.norm()
+    assert not torch.equal(y, whole) and torch.equal(y[330:350], whole[330:350])
+
+
 @gpu
 @pytest.mark.parametrize("channel", [True, False])
 def test_long_and_short_portions_of_one_step(channel, monkeypatch):
