@@ -1822,14 +1822,15 @@ int launch_norm_out(const NormIn& na, const void* Wp, const float* sw, const voi
                     hipStream_t st) {
   const int NTt = (N + 15) / 16;
   constexpr int NCH = NRM % 64 / 8;
+  constexpr bool SHORT_K = NCH == 2 && NRM >= 64;            // (W8A8 rows behind RMSNorm of two chunks: K = 4096 only)
   if (NTt <= 256) {
     if constexpr (NCH >= 3) return launch_norm<1, 1, 16, EPI_OUT, NRM, 5>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
-    else if constexpr (NCH == 2) {
+    else if constexpr (SHORT_K) {
       if (K <= 3072) return launch_norm<1, 1, 16, EPI_OUT, NRM, 3>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
     }
     return launch_norm<1, 1, 16, EPI_OUT, NRM>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
   }
-  if constexpr (NCH == 2) {
+  if constexpr (SHORT_K) {
     if (K <= 3072 && NTt <= 512) return launch_norm<2, 1, 16, EPI_OUT, NRM, 3>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
     if (K <= 3072) return launch_norm<3, 1, 16, EPI_OUT, NRM, 3>(na, Wp, sw, bias, out, nullptr, M, N, K, st);
   }
