@@ -17,8 +17,8 @@ constexpr int MQ = 64, MK = 64;
 // RH query heads of one kv head per workgroup: a staged key / value tile serves all of them
 // (second launch bound: workgroups per CU the register budget must allow - four for 64-wide heads, so the
 // 1024 workgroups of a 4096-token, 16-head prompt are resident at once)
-// KVS: the value of a cached row is its first Dv numbers (a latent cache, or values that are the keys): the
-// staged key tile serves as the value tile, nothing is loaded twice
+// KVS (with EXT; plain attention over latent rows is latent_mfma.hip's): the value of a cached row is its first Dv numbers
+// (values that are the keys): the staged key tile serves as the value tile, nothing is loaded twice
 // EXT: scores are capped (cap tanh(s / cap), cap > 0) and lose slopes[head] * distance; chunked: `window` is a
 // chunk size (a query sees its own chunk's start .. itself), else a sliding window beside the sequence's first
 // keep_first tokens; sink[head] joins the softmax denominator; the gate is [T, H * Dv], one per output coordinate
@@ -43,6 +43,7 @@ __global__ void __launch_bounds__(NT, (DV * RH <= 4 ? (REL && DK > 2 ? 2 : 4) : 
     const int* __restrict__ seq_off, const int* __restrict__ ptab, int ptab_ld, bf16_t* __restrict__ out, int n, int H,
     int G, int PB, float scale_log2, int window, int pool, int kld, int vld, int out_ld, float out_scale,
     AttnExt ext = AttnExt{}) {
+  static_assert(!KVS || EXT, "values that are the keys come with the EXT form");
   static_assert(!REL || (EXT && !KVS), "the distance bias extends the EXT form over separate key and value pages");
   constexpr int DP = 32 * DK, DvP = 16 * DV;                 // what the tiles hold
   const int D = REL ? ext.dim : DP, Dv = REL ? ext.vdim : DvP;

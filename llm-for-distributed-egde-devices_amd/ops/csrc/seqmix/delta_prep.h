@@ -10,7 +10,8 @@ namespace {
 // A unit (q or k of one head) belongs to 16 lanes, four numbers per access; a workgroup of a token takes 16 units or 1024
 // decays, so one token's chain is one load, one sum over 16 lanes, one store.  (One workgroup per token walked 2 G units, a
 // wave each, and then the decays.)  us, G = H = 16, N = 64, one workgroup per token / this: 4096 tokens 38 / 24.9, 4 tokens
-// 10.5 / 3.6; HEAD, N = 128, 6 tokens 12.3 / 5.2.  N % 4 == 0, N <= 256, H % 4 == 0, Cq % 4 == 0 and 16-byte rows (delta_prep_ok).
+// 10.5 / 3.6; HEAD, N = 128, 6 tokens 12.3 / 5.2.  N % 4 == 0, N <= 256, H % 4 == 0, Cq % 4 == 0 and 16-byte rows (launch_delta_prep16
+// asks).
 template <typename T, bool HEAD>
 __global__ void __launch_bounds__(NT) delta_prep16_kernel(const T* __restrict__ qkv, int Cq, const T* __restrict__ u, int ld,
                                                           int b0, int a0, const float* __restrict__ a,
