@@ -15,6 +15,7 @@ import time
 from dataclasses import dataclass, field
 from typing import Dict, List, Optional, Sequence
 
+import numpy as np
 import torch
 
 from .. import ops
@@ -95,6 +96,16 @@ class _DecodeState:
         self.out = torch.zeros(B, max_new, dtype=torch.long, device=device)
         self.seen = torch.zeros(B, V, dtype=torch.uint8, device=device)
         self.ctr = torch.zeros(1, dtype=torch.int32, device=device)       # sampler arrival counter
+
+
+def _host_ids(prompt) -> np.ndarray:
+    """A prompt's ids as int64 on the host: a sequence of numbers, an array, or a tensor of any device."""
+    if not isinstance(prompt, torch.Tensor):
+        try:
+            return np.asarray(prompt, dtype=np.int64)
+        except (TypeError, ValueError):                    # a sequence of device scalars
+            pass
+    return torch.as_tensor(prompt, dtype=torch.long, device="cpu").numpy()
 
 
 class Generator:
@@ -192,13 +203,12 @@ class Generator:
         max_new = sampling.max_new_tokens
         assert max(plens) + max_new <= self.max_seq, "prompt + max_new_tokens exceeds max_seq"
         assert self.attn_hook is None or len(set(plens)) == 1, "HeadInfer offload batches equal-length prompts"
-        # the prompts' tokens count for the repetition penalty: one copy and one launch for the whole batch (a copy and
-        # a launch per prompt were 11 of the 129 ms that 256 prompts of 128 tokens with 32 new ones took).  Ids are looked
-        # at before any state is touched; negative ones count from the vocabulary's end here, as in an index
-        flat = torch.cat([torch.as_tensor(p, dtype=torch.long, device="cpu") for p in prompts])
-        if ((flat < -V) | (flat >= V)).any():
+        t_ids = time.perf_counter()
+        rows = [_host_ids(p) for p in prompts]             # read once: for the pass and for the penalty's flags
+        flat = np.concatenate(rows)
+        if flat.size and (flat.min() < -V or flat.max() >= V):
             raise IndexError(f"token ids outside the vocabulary of {V}")
-        flat = torch.where(flat < 0, flat + V, flat) + torch.repeat_interleave(torch.arange(B) * V, torch.tensor(plens))
+        t_ids = time.perf_counter() - t_ids
         st = self._state
         if st is None or st.tok.shape[0] != B or st.out.shape[1] < max_new:
             self.reset_graphs()
@@ -211,19 +221,23 @@ class Generator:
         cuda = self.device.type == "cuda"
         if cuda:
             torch.cuda.synchronize()
-        t0 = time.perf_counter()
+        t0 = time.perf_counter() - t_ids                   # (the prompts' reading counts)
         # one batched pass; ragged prompts are right-padded to the longest (AttnCtx.last_pos), except
         # under HeadInfer's chunked prefill, which takes one pass per sequence (own cache row)
         if len(set(plens)) == 1:
-            logits = self.prefill(torch.tensor(prompts, dtype=torch.long, device=self.device), 0, 0)
+            logits = self.prefill(torch.from_numpy(flat.reshape(B, -1)).to(self.device), 0, 0)
         elif not self.prefill_chunk:
-            T = max(plens)
-            pad = [list(p) + [0] * (T - len(p)) for p in prompts]
-            logits = self.prefill(torch.tensor(pad, dtype=torch.long, device=self.device), 0, 0, lens=plens)
+            pad = np.zeros((B, max(plens)), dtype=np.int64)
+            for b, r in enumerate(rows):
+                pad[b, :len(r)] = r
+            logits = self.prefill(torch.from_numpy(pad).to(self.device), 0, 0, lens=plens)
         else:
-            logits = torch.cat([self.prefill(torch.tensor([p], dtype=torch.long, device=self.device), b, 0)
-                                for b, p in enumerate(prompts)], 0)
-        st.seen.view(-1).index_fill_(0, flat.to(self.device), 1)
+            logits = torch.cat([self.prefill(torch.from_numpy(r[None]).to(self.device), b, 0) for b, r in enumerate(rows)], 0)
+        # the prompts' tokens count for the repetition penalty: one copy and one launch for the whole batch (a copy and
+        # a launch per prompt were 11 of the 129 ms that 256 prompts of 128 tokens with 32 new ones took), formed while the
+        # pass runs; negative ids count from the vocabulary's end, as in an index
+        flags = np.where(flat < 0, flat + V, flat) + np.repeat(np.arange(B, dtype=np.int64) * V, plens)
+        st.seen.view(-1).index_fill_(0, torch.from_numpy(flags).to(self.device), 1)
         st.pos.copy_(torch.tensor(plens, dtype=torch.int32, device=self.device))
         st.seq_lens.copy_(st.pos + 1)
         nxt = ops.sample(logits, st.seen, sampling.temperature, sampling.top_k, sampling.top_p,
