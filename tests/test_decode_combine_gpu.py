@@ -1,5 +1,6 @@
-"""Decode attention over many key splits (attn_decode.hip decode_combine_kernel): split counts around the 32 that are read
-together and the 128 whose weights meet in LDS at once, rows whose later splits hold no keys."""
+"""Decode attention over key splits (attn_decode.hip decode_combine_few_kernel up to 4 and 8 splits, decode_combine_kernel):
+split counts around those, around the 32 that are read together and the 128 whose weights meet in LDS at once, rows whose
+later splits hold no keys."""
 import math
 
 import pytest
@@ -12,7 +13,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("D,Hq,Hkv", [(64, 4, 1), (128, 2, 2), (80, 2, 1), (256, 2, 1)])
-@pytest.mark.parametrize("splits", [2, 31, 32, 33, 64, 65, 128, 129])
+@pytest.mark.parametrize("splits", [2, 3, 4, 5, 8, 9, 31, 32, 33, 64, 65, 128, 129])
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
 def test_split_counts(D, Hq, Hkv, splits, dt):
     S = splits * 256                                         # 256 keys per split for so few heads
