@@ -71,7 +71,7 @@ def test_delta_prepare(dt, per_head, heads, kv, N):
 
 
 @pytest.mark.parametrize("dt", DT)
-@pytest.mark.parametrize("H,D,R,kvr,rot", [(16, 64, 32, 128, 32), (3, 8, 8, 8, 0), (5, 16, 16, 24, 8), (2, 128, 64, 256, 64), (3, 12, 8, 16, 8),
+@pytest.mark.parametrize("H,D,R,kvr,rot", [(16, 64, 32, 128, 32), (3, 8, 8, 8, 0), (33, 8, 8, 8, 0), (5, 16, 16, 24, 8), (13, 16, 16, 24, 8), (2, 128, 64, 256, 64), (3, 12, 8, 16, 8), (33, 12, 8, 16, 8),
                                            (2, 8, 6, 10, 4), (2, 8, 8, 16, 4)])
 def test_latent_write(dt, H, D, R, kvr, rot):
     g = torch.Generator().manual_seed(H)
