@@ -832,7 +832,9 @@ def delta_rule_scan(prep: torch.Tensor, qkv: torch.Tensor, state: torch.Tensor, 
     (zero for a portion starting at 0) and left at the portion's end.  Returns o fp32 [T, heads P]."""
     if _gpu(prep):
         # portions below `least` tokens: one workgroup per (sequence, head, 16 value columns), token by token
-        least = delta_chunks_from([h[2] for h in meta.host], heads, N, P) if qkv.dtype == torch.bfloat16 else 0
+        least = 0
+        if qkv.dtype == torch.bfloat16 and meta.max_len >= (DELTA_CHUNK_MIN or DELTA_LONG):
+            least = delta_chunks_from([h[2] for h in meta.host], heads, N, P)
         per = [(h[2] + 63) // 64 for h in meta.host if h[2] >= least] if least else []
         most, room = delta_parts(per, DELTA_SCRATCH_BYTES // (4 * _ext().sm_delta_chunk_floats(1, heads, N, P))) if per else (0, 0)
         if most == 0:
