@@ -99,13 +99,18 @@ class _DecodeState:
 
 
 def _host_ids(prompt) -> np.ndarray:
-    """A prompt's ids as int64 on the host: a sequence of numbers, an array, or a tensor of any device."""
+    """A prompt's ids as int64 on the host: a flat sequence of numbers, an array, or a tensor of any device."""
+    ids = None
     if not isinstance(prompt, torch.Tensor):
         try:
-            return np.asarray(prompt, dtype=np.int64)
+            ids = np.asarray(prompt)
         except (TypeError, ValueError):                    # a sequence of device scalars
             pass
-    return torch.as_tensor(prompt, dtype=torch.long, device="cpu").numpy()
+    if ids is None or ids.dtype in (object, np.uint64):    # (numbers past int64 are refused, not wrapped)
+        ids = torch.as_tensor(prompt, dtype=torch.long, device="cpu").numpy()
+    if ids.ndim != 1 or ids.dtype.kind not in "biuf":      # (a cast alone would parse texts and drop imaginary parts)
+        raise ValueError(f"a prompt is a flat sequence of token ids, not {ids.ndim}-dimensional {ids.dtype}")
+    return ids.astype(np.int64, copy=False)
 
 
 class Generator:

@@ -1,3 +1,4 @@
+import numpy as np
 import pytest
 import torch
 
@@ -147,6 +148,16 @@ def _start_forms(device):
 
 def test_start_takes_prompts_of_every_sequence_type():
     _start_forms("cpu")
+
+
+@pytest.mark.parametrize("prompts", [[["1", "2"]], [["1", "2"], ["3"]], ["12"], [[[1, 2, 3]]], [torch.tensor([[1, 2, 3]])],
+                                     [np.array([1 + 2j, 3])], [[2 ** 64 - 1]]], ids=str)
+def test_start_refuses_what_is_no_flat_sequence_of_numbers(prompts):
+    """Texts, nested sequences, complex numbers and numbers past int64 are refused before any state is touched."""
+    gen = Generator(build_model(tiny("llama2"), dtype=torch.float32, device="cpu", seed=0), max_batch=2, max_seq=64)
+    with pytest.raises((ValueError, RuntimeError), match="flat sequence|[Oo]verflow"):
+        gen.start(prompts, SamplingParams(max_new_tokens=2))
+    assert gen._state is None
 
 
 @pytest.mark.gpu
