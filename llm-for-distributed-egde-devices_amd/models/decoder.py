@@ -30,7 +30,7 @@ import torch.nn as nn
 from .. import ops
 from ..utils import tracing
 from .configs import ModelConfig
-from .layers import Linear, Norm, PartialSum, PendingLN, PendingNorm, QAct, act_fn, quant_if
+from .layers import BranchRows, Linear, Norm, PartialSum, PendingLN, PendingNorm, QAct, act_fn, quant_if
 
 # split-K slices of the bf16 o / down decode GEMVs (0 = off); N = 2048-4096 outputs have only
 # 128-256 tiles, so two slices put every CU to work
@@ -292,6 +292,34 @@ class DecoderLayer(nn.Module):
                 and getattr(self.mlp.up, "pending_ln_ok", lambda **k: False)(geluq=True)
                 and getattr(self.mlp.down, "group_scales_ok", lambda m: False)(x.shape[0]))
 
+    def _pair_ok(self, x, ctx: AttnCtx) -> bool:
+        """Rows that ``_ln_deferred`` takes whose independent parts can share launches (``_pair``): a plain decode step over a
+        16-bit cache, plain 16-bit projections, and nobody who watches a module's own call."""
+        o, down = self.attn.o, self.mlp.down
+        return (ctx.mode == "decode" and ctx.T == 1 and ctx.B == x.shape[0] and ctx.attn_hook is None
+                and self.cfg.head_dim in ops.DECODE_ATTN_DIMS and self.cfg.rotary_dim % 16 == 0
+                and not getattr(ctx.kv, "quantized", False) and type(o) is Linear and type(down) is Linear
+                and o.pair_ok() and down.pair_ok() and self.norm1.eps == (self.norm2 or self.norm1).eps
+                and not any(m._forward_hooks or m._forward_pre_hooks
+                            for m in (self.attn, self.mlp, self.attn.qkv, o, self.mlp.up, down)))
+
+    def _pair(self, x, residual, ctx: AttnCtx):
+        """A parallel-residual decode step in three launches (decode_pair.hip): qkv with the norm(s) in its prologue,
+        attention beside up, o beside down."""
+        cfg, n1 = self.cfg, self.norm1
+        n2 = n1 if self.norm2 is None else self.norm2
+        x, x2 = (x.mlp, x.attn) if isinstance(x, BranchRows) else (x, None)
+        qkv, o, up, down = self.attn.qkv, self.attn.o, self.mlp.up, self.mlp.down
+        h, y = torch.empty_like(x), torch.empty_like(x)
+        q = qkv.forward_ln(PendingLN(x, residual, n1.weight, n1.bias, n1.eps, h, y, x2=x2, y_weight=n2.weight, y_bias=n2.bias))
+        k_cache, v_cache = ctx.kv.layer(self.idx)
+        rot = cfg.rotary_dim if cfg.pos_emb == "rope" else 0
+        a, m = ops.decode_attn_up(q.view(ctx.B, -1), ctx.start_pos, ctx.rope if rot else None, k_cache, v_cache, ctx.seq_lens,
+                                  cfg.num_heads, self.attn.scale, ctx.max_len, rot, y, up.packed_weight(), up.bias,
+                                  up.out_features, cfg.act)
+        return BranchRows(*ops.ext().decode_o_down(a, o.packed_weight(), o.bias, m, down.packed_weight(), down.bias,
+                                                   cfg.hidden_size)), h
+
     def forward(self, x, residual, ctx: AttnCtx):
         cfg = self.cfg
         if not cfg.parallel_residual:
@@ -312,6 +340,11 @@ class DecoderLayer(nn.Module):
             return self.mlp(n2), h2
         qa = self.attn.qkv.takes_quantized_input
         qm = self.mlp.up.takes_quantized_input
+        rows = x.mlp if isinstance(x, BranchRows) else x
+        if self._ln_deferred(rows, qa, qm) and self._pair_ok(rows, ctx):
+            return self._pair(x, residual, ctx)
+        if isinstance(x, BranchRows):
+            x = x.materialize()
         if self._ln_deferred_w8a8(x, qa, qm):
             # W8A8 decode at batch 1 (GPT-NeoX): LayerNorm + int8 quant in the qkv / up GEMV prologues
             n1, n2, h = self.norm1, self.norm2, torch.empty_like(x)
@@ -469,7 +502,7 @@ class DecoderLM(nn.Module):
         final-normed last rows only, for an LM head split by vocabulary over pipeline ranks
         (parallel/vocab_head.py)."""
         last = logits in ("last", "hidden")
-        if isinstance(x, PartialSum) and last and ctx.T > 1:
+        if isinstance(x, (BranchRows, PartialSum)) and last and ctx.T > 1:
             x = x.materialize()
         if last and ctx.T > 1:
             idx = ctx.last_rows(x.device)
@@ -521,7 +554,7 @@ class DecoderLM(nn.Module):
         x, residual = self.forward_layers(x, ctx, None)
         if self.has_head:
             return self.head(x, residual, ctx, logits)
-        if isinstance(x, PartialSum):
+        if isinstance(x, (BranchRows, PartialSum)):
             x = x.materialize()
         return x + residual if residual is not None else x
 

@@ -61,13 +61,28 @@ class PendingNorm(NamedTuple):
         return QAct(y, s) if self.quant else y
 
 
+class BranchRows(NamedTuple):
+    """Output of a parallel-residual block whose o and down projections ran in one launch: the two
+    branches' 16-bit rows, whose rounded sum is the block's output.  The next block's norm adds them
+    (PendingLN.x2); anything else calls ``materialize()``."""
+    attn: torch.Tensor
+    mlp: torch.Tensor
+
+    @property
+    def device(self):
+        return self.mlp.device
+
+    def materialize(self) -> torch.Tensor:
+        return self.mlp + self.attn
+
+
 class PendingLN(NamedTuple):
-    """LayerNorm of 16-bit decode rows x (+ residual, M <= 4), deferred into the prologue of the
-    16-bit GEMV(s) that consume it (ops.gemv_bf16_ln; parallel-residual blocks, where the qkv and
+    """LayerNorm of 16-bit decode rows x (+ x2, rounded) (+ residual, M <= 4), deferred into the prologue
+    of the 16-bit GEMV(s) that consume it (ops.gemv_bf16_ln; parallel-residual blocks, where the qkv and
     the MLP up projection both read a norm of the same rows): no norm launch.  ``h`` = x + residual,
     written by the consumer (every consumer writes the same bits); ``y`` (optional): the consumer
-    also writes the normalised rows there, for a second consumer that reads them as a plain input.
-    ``materialize()`` runs the norm kernel instead."""
+    also writes the normalised rows there (under ``y_weight`` / ``y_bias`` where given), for a second
+    consumer that reads them as a plain input.  ``materialize()`` runs the norm kernel instead."""
     x: torch.Tensor
     residual: Optional[torch.Tensor]
     weight: torch.Tensor
@@ -77,8 +92,13 @@ class PendingLN(NamedTuple):
     y: Optional[torch.Tensor] = None
     quant: bool = False              # the consumers are W8A8: int8 rows per token (QAct)
     rms: bool = False                # RMSNorm (no bias) instead of LayerNorm (LLM.int8 consumers only)
+    x2: Optional[torch.Tensor] = None
+    y_weight: Optional[torch.Tensor] = None
+    y_bias: Optional[torch.Tensor] = None
 
     def materialize(self):
+        if self.x2 is not None:
+            return self._replace(x=self.x + self.x2, x2=None).materialize()
         if self.rms:
             y, r = ops.rms_norm(self.x, self.weight, self.eps, self.residual)
             self.h.copy_(r.view_as(self.h))
@@ -92,7 +112,8 @@ class PendingLN(NamedTuple):
         y, r = ops.layer_norm(self.x, self.weight, self.bias, self.eps, self.residual)
         self.h.copy_(r.view_as(self.h))
         if self.y is not None:
-            self.y.copy_(y.view_as(self.y))
+            z = y if self.y_weight is None else ops.layer_norm(self.h, self.y_weight, self.y_bias, self.eps, None)[0]
+            self.y.copy_(z.view_as(self.y))
         return y
 
 
@@ -150,12 +171,19 @@ class Linear(nn.Module):
                 and self.in_features <= 4096 and self.in_features % 64 == 0 and self.out_features % 16 == 0
                 and not self.split_k_out and ops.gpu_path(w))
 
+    def pair_ok(self) -> bool:
+        """Whether this 16-bit projection of decode rows can share a launch with another part of its block
+        (decode_pair.hip)."""
+        w = self.weight
+        return (w.is_cuda and w.dtype in (torch.bfloat16, torch.float16) and ops.available() and not self.split_k_out
+                and self.in_features % 64 == 0 and self.out_features % 16 == 0 and ops.gpu_path(w))
+
     def forward_ln(self, x: "PendingLN", act: Optional[str] = None):
         """The decode GEMV over a PendingLN (LayerNorm in the prologue); act: its GELU epilogue."""
         y = None
         if self.pending_ln_ok() and x.x.dtype == self.weight.dtype and not x.rms:
             y = ops.gemv_bf16_ln(x.x, x.residual, x.weight, x.bias, x.eps, x.h, self.packed_weight(), self.bias,
-                                 self.out_features, act, y_out=x.y)
+                                 self.out_features, act, y_out=x.y, x2=x.x2, gamma2=x.y_weight, beta2=x.y_bias)
         if y is not None:
             return y
         xm = x.materialize()
@@ -240,6 +268,8 @@ class Norm(nn.Module):
             # consumer (not quant) takes the normalised rows in its own dtype
             h = torch.empty(x.parts.shape[1], x.parts.shape[2], dtype=self.weight.dtype, device=x.parts.device)
             return PendingNorm(x.parts, residual, self.weight, self.eps, h, quant), h
+        if isinstance(x, BranchRows):
+            x = x.materialize()
         if isinstance(x, PartialSum):
             if self.kind == "rms" and x.parts.is_cuda and ops.gpu_path(x.parts):
                 y, s, r = ops.rms_norm_parts(x.parts, residual, self.weight, self.eps, quant)

@@ -147,13 +147,24 @@ _LN_EPI = {None: 0, "gelu_tanh": 2, "gelu": 3}
 
 
 def gemv_bf16_ln(x, residual, gamma, beta, eps: float, res_out, packed, bias, N: int, act: Optional[str] = None,
-                 y_out=None):
-    """16-bit decode GEMV (M <= 4 rows) over LayerNorm(x + residual (None: none)) with the norm in
-    its prologue (bit-identical to the norm kernel); x + residual goes to ``res_out``, the
-    normalised rows to ``y_out`` when given (a second consumer's input); ``act``: None /
-    "gelu_tanh" / "gelu" epilogue.  None when no kernel takes the shape."""
+                 y_out=None, x2=None, gamma2=None, beta2=None):
+    """16-bit decode GEMV (M <= 4 rows) over LayerNorm(x (+ x2, rounded) + residual (None: none)) with the
+    norm in its prologue (bit-identical to the norm kernel); the sum goes to ``res_out``, the normalised
+    rows to ``y_out`` when given (a second consumer's input; under ``gamma2`` / ``beta2`` where given);
+    ``act``: None / "gelu_tanh" / "gelu" epilogue.  None when no kernel takes the shape."""
     return ext().gemv_bf16_ln(x, residual.contiguous() if residual is not None else None, gamma, beta, eps, res_out,
-                              packed, bias, N, _LN_EPI[act], y_out)
+                              packed, bias, N, _LN_EPI[act], y_out, x2, gamma2, beta2)
+
+
+DECODE_ATTN_DIMS = (64, 80, 128, 256)      # head sizes of the decode attention kernels (attn_decode.hip)
+
+
+def decode_attn_up(qkv, start_pos, rope, k_cache, v_cache, seq_lens, num_heads: int, scale: float, max_len_hint: int,
+                   rotary_dim: int, y, packed, bias, N: int, act: str):
+    """``decode_attention_fused`` beside act(y Wup^T + bias), up to 4 rows, one launch (decode_pair.hip):
+    ``(attention rows [B, Hq*D], h [B, N])``; None when no kernel takes the shapes."""
+    return ext().decode_attn_up(qkv, start_pos, rope if rotary_dim else None, k_cache, v_cache, seq_lens, num_heads, scale,
+                                int(max_len_hint), rotary_dim, y, packed, bias, N, _LN_EPI[act])
 
 
 def w8a8_gemv_ln(x, residual, gamma, beta, eps: float, res_out, w_packed, w_scale, bias, N: int, K: int,

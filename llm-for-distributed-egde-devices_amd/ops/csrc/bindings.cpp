@@ -27,9 +27,15 @@ int edge_w8a8_gemv_ln(const void* x, const void* res, const void* gamma, const v
 int edge_gemv_bf16_norm(const float* part, int S, const void* res, const void* gamma, float eps, void* res_out,
                         const void* W, const void* bias, void* out, int M, int N, int K, int epi, hipStream_t st,
                         int h16);
-int edge_gemv_bf16_ln(const void* x, const void* res, const void* gamma, const void* beta, float eps, void* res_out,
-                      const void* W, const void* bias, void* out, int M, int N, int K, int epi, hipStream_t st,
-                      int h16, void* y_out);
+int edge_gemv_bf16_ln(const void* x, const void* x2, const void* res, const void* gamma, const void* beta, float eps,
+                      void* res_out, const void* W, const void* bias, void* out, int M, int N, int K, int epi,
+                      hipStream_t st, int h16, void* y_out, const void* gamma2, const void* beta2);
+int edge_attn_up(const void* qkv, int64_t q_sb, void* kc, void* vc, int64_t c_sb, int64_t c_sh, const int* seq_lens, int B,
+                 int Hq, int Hkv, int D, float scale, int ch, int nsplit, void* out, int64_t o_sb, float* part_acc,
+                 float* part_ml, const int* pos, const float* cs, int rot, const void* y, const void* w, const void* bias,
+                 void* h, int N, int K, int act, int h16, hipStream_t st);
+int edge_o_down(const void* x, const void* wo, const void* bo, void* a, int Ko, const void* h, const void* wd,
+                const void* bd, void* y, int Kd, int M, int N, int h16, hipStream_t st);
 int edge_w8a8_gemv_norm_on();
 int edge_w8a8_gemm_splitk(const void* A, const float* sa, const void* Wp, const float* sw, const void* bias,
                           float* part, int M, int N, int K, int KT, int a_mode, int Mpad, int S, hipStream_t st);
@@ -407,16 +413,10 @@ at::Tensor decode_attn(const at::Tensor& q, const at::Tensor& k_cache, const at:
   return out;
 }
 
-// Decode step straight from the QKV projection: rotates q, appends the new k/v at start_pos[b]
-// and attends over [0, seq_lens[b]).  quant_out: returns (int8 [B, Hq*D], scales [Hq*D/64, Mpad])
-// for a W8A8 consumer; else (bf16 [B, Hq, D], None).
-std::tuple<at::Tensor, std::optional<at::Tensor>> decode_attn_fused(
-    const at::Tensor& qkv, const at::Tensor& start_pos, const std::optional<at::Tensor>& rope, at::Tensor& k_cache,
-    at::Tensor& v_cache, const at::Tensor& seq_lens, int64_t Hq, double scale, int64_t max_len_hint, int64_t rot,
-    bool quant_out) {
-  DEVICE_GUARD(qkv);
-  const int h16 = need16(qkv, "qkv");
-  TORCH_CHECK(!(h16 && quant_out), "int8 attention output from fp16 rows is not supported");
+// Operands of a decode step straight from the QKV projection; returns the rope table (null: no rotation).
+const float* check_fused_attn(const at::Tensor& qkv, const at::Tensor& start_pos, const std::optional<at::Tensor>& rope,
+                              const at::Tensor& k_cache, const at::Tensor& v_cache, const at::Tensor& seq_lens, int64_t Hq,
+                              int64_t max_len_hint, int64_t rot) {
   TORCH_CHECK(qkv.dim() == 2, "qkv must be [B, (Hq + 2 Hkv) * D]");
   const int64_t B = qkv.size(0), D = k_cache.size(3), Hkv = k_cache.size(1);
   TORCH_CHECK(qkv.size(1) == (Hq + 2 * Hkv) * D, "qkv width does not match the cache geometry");
@@ -434,6 +434,21 @@ std::tuple<at::Tensor, std::optional<at::Tensor>> decode_attn_fused(
     TORCH_CHECK(rope->size(-2) * 2 == rot, "rope table width must be rot/2");
     cs = rope->data_ptr<float>();
   }
+  return cs;
+}
+
+// Decode step straight from the QKV projection: rotates q, appends the new k/v at start_pos[b]
+// and attends over [0, seq_lens[b]).  quant_out: returns (int8 [B, Hq*D], scales [Hq*D/64, Mpad])
+// for a W8A8 consumer; else (bf16 [B, Hq, D], None).
+std::tuple<at::Tensor, std::optional<at::Tensor>> decode_attn_fused(
+    const at::Tensor& qkv, const at::Tensor& start_pos, const std::optional<at::Tensor>& rope, at::Tensor& k_cache,
+    at::Tensor& v_cache, const at::Tensor& seq_lens, int64_t Hq, double scale, int64_t max_len_hint, int64_t rot,
+    bool quant_out) {
+  DEVICE_GUARD(qkv);
+  const int h16 = need16(qkv, "qkv");
+  TORCH_CHECK(!(h16 && quant_out), "int8 attention output from fp16 rows is not supported");
+  const float* cs = check_fused_attn(qkv, start_pos, rope, k_cache, v_cache, seq_lens, Hq, max_len_hint, rot);
+  const int64_t B = qkv.size(0), D = k_cache.size(3), Hkv = k_cache.size(1);
   int ch = 0, nsplit = 0;
   edge_decode_attn_plan((int)B, (int)Hkv, (int)max_len_hint, (int)D, &ch, &nsplit);
   at::Tensor pacc, pml, out, oq;
@@ -459,6 +474,62 @@ std::tuple<at::Tensor, std::optional<at::Tensor>> decode_attn_fused(
         "decode_attn_fused");
   if (quant_out) return {oq, os};
   return {out, std::nullopt};
+}
+
+// Parallel-residual decode step of up to 4 rows (decode_pair.hip): decode_attn_fused (16-bit output) beside
+// h = gelu(y Wup^T + bias) (act 2 tanh, 3 erf) in one launch.  None where no kernel takes the shapes.
+std::optional<std::tuple<at::Tensor, at::Tensor>> decode_attn_up(
+    const at::Tensor& qkv, const at::Tensor& start_pos, const std::optional<at::Tensor>& rope, at::Tensor& k_cache,
+    at::Tensor& v_cache, const at::Tensor& seq_lens, int64_t Hq, double scale, int64_t max_len_hint, int64_t rot,
+    const at::Tensor& y, const at::Tensor& wp, const std::optional<at::Tensor>& bias, int64_t N, int64_t act) {
+  DEVICE_GUARD(qkv);
+  const int h16 = need16(qkv, "qkv");
+  const float* cs = check_fused_attn(qkv, start_pos, rope, k_cache, v_cache, seq_lens, Hq, max_len_hint, rot);
+  const int64_t B = qkv.size(0), D = k_cache.size(3), Hkv = k_cache.size(1), K = y.size(-1);
+  need_same(y, qkv, "y");
+  need_same(wp, qkv, "weight (packed)");
+  TORCH_CHECK(y.dim() == 2 && y.size(0) == B && wp.numel() == N * K, "y [B, K], packed weight N * K");
+  if (bias) { need_same(*bias, qkv, "bias"); TORCH_CHECK(bias->numel() == N, "bias [N]"); }
+  TORCH_CHECK(act == 2 || act == 3, "act 2 (gelu tanh), 3 (gelu erf)");
+  if (B < 1 || B > 4 || Hq % Hkv != 0 || (D != 64 && D != 80 && D != 128 && D != 256) || N % 16 != 0 || K % 64 != 0 || K == 0 ||
+      rot % 16 != 0 || rot > D)
+    return std::nullopt;
+  int ch = 0, nsplit = 0;
+  edge_decode_attn_plan((int)B, (int)Hkv, (int)max_len_hint, (int)D, &ch, &nsplit);
+  at::Tensor pacc, pml;
+  if (nsplit > 1) {
+    pacc = at::empty({B, Hq, nsplit, D}, qkv.options().dtype(at::kFloat));
+    pml = at::empty({B, Hq, nsplit, 2}, qkv.options().dtype(at::kFloat));
+  }
+  auto out = at::empty({B, Hq * D}, qkv.options()), h = at::empty({B, N}, qkv.options());
+  check(edge_attn_up(qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0), k_cache.stride(1),
+                     seq_lens.data_ptr<int>(), (int)B, (int)Hq, (int)Hkv, (int)D, (float)scale, ch, nsplit, out.data_ptr(),
+                     out.stride(0), nsplit > 1 ? pacc.data_ptr<float>() : nullptr, nsplit > 1 ? pml.data_ptr<float>() : nullptr,
+                     start_pos.data_ptr<int>(), cs, (int)rot, y.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr,
+                     h.data_ptr(), (int)N, (int)K, act == 2 ? 1 : 0, h16, stream()),
+        "decode_attn_up");
+  return std::make_tuple(out, h);
+}
+
+// The o and down projections of a parallel-residual block in one launch, each into rows of its own (up to 4 rows).
+std::tuple<at::Tensor, at::Tensor> decode_o_down(const at::Tensor& x, const at::Tensor& wo, const std::optional<at::Tensor>& bo,
+                                                 const at::Tensor& h, const at::Tensor& wd, const std::optional<at::Tensor>& bd,
+                                                 int64_t N) {
+  DEVICE_GUARD(x);
+  const int h16 = need16(x, "x");
+  need_same(wo, x, "o weight (packed)");
+  need_same(h, x, "h");
+  need_same(wd, x, "down weight (packed)");
+  TORCH_CHECK(x.dim() == 2 && h.dim() == 2 && h.size(0) == x.size(0), "x [M, Ko], h [M, Kd]");
+  const int64_t M = x.size(0), Ko = x.size(1), Kd = h.size(1);
+  TORCH_CHECK(wo.numel() == N * Ko && wd.numel() == N * Kd, "packed weights must hold N * K elements");
+  if (bo) { need_same(*bo, x, "o bias"); TORCH_CHECK(bo->numel() == N); }
+  if (bd) { need_same(*bd, x, "down bias"); TORCH_CHECK(bd->numel() == N); }
+  auto a = at::empty({M, N}, x.options()), y = at::empty({M, N}, x.options());
+  check(edge_o_down(x.data_ptr(), wo.data_ptr(), bo ? bo->data_ptr() : nullptr, a.data_ptr(), (int)Ko, h.data_ptr(),
+                    wd.data_ptr(), bd ? bd->data_ptr() : nullptr, y.data_ptr(), (int)Kd, (int)M, (int)N, h16, stream()),
+        "decode_o_down");
+  return {a, y};
 }
 
 // ---------------------------------------------------------------------------- int8 KV cache
@@ -1044,7 +1115,8 @@ std::optional<at::Tensor> gemv_bf16_ln(const at::Tensor& x, const std::optional<
                                        const at::Tensor& gamma, const std::optional<at::Tensor>& beta, double eps,
                                        const at::Tensor& res_out, const at::Tensor& wp,
                                        const std::optional<at::Tensor>& bias, int64_t N, int64_t epi,
-                                       const std::optional<at::Tensor>& y_out) {
+                                       const std::optional<at::Tensor>& y_out, const std::optional<at::Tensor>& x2,
+                                       const std::optional<at::Tensor>& gamma2, const std::optional<at::Tensor>& beta2) {
   DEVICE_GUARD(x);
   const bool h16 = gamma.scalar_type() == at::kHalf;
   const auto dt = h16 ? at::kHalf : at::kBFloat16;
@@ -1066,13 +1138,21 @@ std::optional<at::Tensor> gemv_bf16_ln(const at::Tensor& x, const std::optional<
     need(*y_out, dt, "y_out");
     TORCH_CHECK(y_out->numel() == M * K && y_out->data_ptr() != res_out.data_ptr(), "y_out [M, K]");
   }
+  if (x2) {
+    need(*x2, dt, "x2");
+    TORCH_CHECK(x2->numel() == M * K && x2->data_ptr() != res_out.data_ptr(), "x2 [M, K], not aliasing res_out");
+  }
+  TORCH_CHECK(!gamma2 || y_out, "gamma2: the weights of y_out");
+  if (gamma2) { need(*gamma2, dt, "gamma2"); TORCH_CHECK(gamma2->numel() == K, "gamma2 [K]"); }
+  if (beta2) { need(*beta2, dt, "beta2"); TORCH_CHECK(gamma2 && beta2->numel() == K, "beta2 [K], beside gamma2"); }
   TORCH_CHECK(epi == 0 || epi == 2 || epi == 3, "epi 0 (out), 2 (gelu tanh), 3 (gelu erf)");
   if (M < 1 || M > 4 || K > 4096 || K % 64 != 0 || N % 16 != 0) return std::nullopt;
   auto y = at::empty({M, N}, res_out.options());
-  const int r = edge_gemv_bf16_ln(x.data_ptr(), residual ? residual->data_ptr() : nullptr, gamma.data_ptr(),
+  const int r = edge_gemv_bf16_ln(x.data_ptr(), x2 ? x2->data_ptr() : nullptr, residual ? residual->data_ptr() : nullptr, gamma.data_ptr(),
                                   beta ? beta->data_ptr() : nullptr, (float)eps, res_out.data_ptr(), wp.data_ptr(),
                                   bias ? bias->data_ptr() : nullptr, y.data_ptr(), (int)M, (int)N, (int)K, (int)epi,
-                                  stream(), h16 ? 1 : 0, y_out ? y_out->data_ptr() : nullptr);
+                                  stream(), h16 ? 1 : 0, y_out ? y_out->data_ptr() : nullptr,
+                                  gamma2 ? gamma2->data_ptr() : nullptr, beta2 ? beta2->data_ptr() : nullptr);
   if (r == -2) return std::nullopt;
   check(r, "gemv_bf16_ln");
   return y;
@@ -1425,6 +1505,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("llmint8_outlier", &llmint8_outlier, "LLM.int8 decode outlier part, added in place");
   m.def("gemv_bf16_norm", &gemv_bf16_norm, "16-bit decode GEMV with the RMSNorm in its prologue (M <= 4)");
   m.def("gemv_bf16_ln", &gemv_bf16_ln, "16-bit decode GEMV with the LayerNorm in its prologue (M <= 4)");
+  m.def("decode_attn_up", &decode_attn_up, "decode attention beside the up projection of a parallel-residual block (M <= 4)");
+  m.def("decode_o_down", &decode_o_down, "o beside the down projection of a parallel-residual block (M <= 4)");
   m.def("w8a8_gemv_ln", &w8a8_gemv_ln, "W8A8 decode GEMV with the LayerNorm + int8 quant in its prologue (M <= 4)");
   m.def("llmint8_gemv", &llmint8_gemv, "LLM.int8 projection of one row in one launch (prep in the GEMV prologue)");
   m.def("llmint8_gemv_norm", &llmint8_gemv_norm, "LLM.int8 projection of RMSNorm / LayerNorm(x + residual), one launch");

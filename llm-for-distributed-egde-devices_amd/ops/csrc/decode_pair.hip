@@ -1,0 +1,121 @@
+// Two independent parts of a parallel-residual block (GPT-NeoX, Phi) in one launch of a 16-bit decode step, up to 4 rows:
+//   * attention beside the MLP's up projection (both need only the qkv launch's results);
+//   * the o projection beside the down projection, each into rows of its own (the next layer's norm adds them up).
+// What bounds a step of such a layer is not its bytes but the launches: each costs some 3.3 us of ramp, first loads and
+// reduction beside the time of its weights, and the attention's 5 us leave the memory idle.  Five launches a layer are
+// three this way.  The workgroups are the parts' own (attn_decode.h, gemv_bf16.h) with 8 waves instead of 16, one tile of 16
+// columns each: two to a CU under 128 VGPRs, so that the attention's workgroups take no CU away from the projection.
+// The attention's come first in the grid: they are the longest chains.  us a layer of Pythia-1B, fp16, one row: attention 5.3
+// and up 8.3 are 10.3 together, o 5.0 and down 10.4 are 10.9; whole answers, one row: Pythia-1B 48 tokens 33.9 -> 28.2 ms
+// (4 rows, 32 tokens 27.6 -> 22.3), Phi-2 32 tokens 57.8 -> 47.0, 64 tokens behind 200 116.6 -> 90.5.
+#include "attn_decode.h"
+#include "gemv_bf16.h"
+
+namespace {
+constexpr int PW = 8;                      // waves a workgroup
+
+struct Proj {
+  const bf16_t *x, *w, *bias;              // rows [M, K], packed weights, bias [N] or null
+  bf16_t* out;
+  int N, K;
+};
+
+// One workgroup of a projection: as many k-pairs in flight per wave as divide its rounds evenly (8, 5 or 4: a round that runs
+// over the end loads its last k-pair again), else 2.
+template <int EPI, bool HF>
+__device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act) {
+  const int KP = p.K / 64;
+  const NormIn16 none{};
+  if (KP % (8 * PW) == 0) gemv_bf16_body<PW, 1, 1, 8, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
+  else if (KP % (5 * PW) == 0) gemv_bf16_body<PW, 1, 1, 5, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
+  else if (KP % (4 * PW) == 0) gemv_bf16_body<PW, 1, 1, 4, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
+  else gemv_bf16_body<PW, 1, 1, 2, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
+}
+
+struct AttnArgs {
+  const bf16_t* q;
+  int64_t q_sb;
+  bf16_t *kc, *vc;
+  int64_t c_sb, c_sh;
+  const int* seq_lens;
+  float scale_log2;
+  int ch, nsplit, ny;                      // ny: query heads (each a workgroup of its own)
+  bf16_t* out;
+  int64_t o_sb;
+  float *part_acc, *part_ml;
+  Fuse fz;
+};
+
+template <int D, bool DIRECT, bool HF>
+__global__ void __launch_bounds__(PW * 64, 4) attn_up_kernel(AttnArgs a, Proj p, int M, int act, int na) {
+  __shared__ __attribute__((aligned(16))) float smem[PW * D + 2 * PW + 2];
+  const int bid = blockIdx.x;
+  if (bid < na) {
+    const int s = bid % a.nsplit, r = bid / a.nsplit;
+    decode_attn_body<D, 1, DIRECT, true, false, 4, HF, PW, UNROLL_DEF>(smem, s, r % a.ny, a.ny, r / a.ny, a.q, a.q_sb, a.kc, a.vc,
+                                                                      a.c_sb, a.c_sh, a.seq_lens, a.scale_log2, a.ch, a.nsplit,
+                                                                      a.out, a.o_sb, a.part_acc, a.part_ml, a.fz);
+  } else {
+    proj_body<EPI_GELU_ANY, HF>(bid - na, p, M, act);
+  }
+}
+
+// The down projection's workgroups first: their chains are the longer ones.
+template <bool HF>
+__global__ void __launch_bounds__(PW * 64, 4) o_down_kernel(Proj o, Proj d, int M) {
+  const int nd = d.N / 16, bid = blockIdx.x;
+  const bool down = bid < nd;
+  proj_body<EPI_OUT, HF>(down ? bid : bid - nd, down ? d : o, M, 0);
+}
+
+template <bool HF>
+int run_attn_up(const AttnArgs& a, const Proj& p, int B, int D, int act, hipStream_t st) {
+  const int na = a.nsplit * a.ny * B;
+  const dim3 grid(na + p.N / 16), block(PW * 64);
+#define AU(DD)                                                                                                   \
+  if (a.nsplit == 1) hipLaunchKernelGGL((attn_up_kernel<DD, true, HF>), grid, block, 0, st, a, p, B, act, na);    \
+  else hipLaunchKernelGGL((attn_up_kernel<DD, false, HF>), grid, block, 0, st, a, p, B, act, na);                 \
+  break
+  switch (D) {
+    case 64: AU(64);
+    case 80: AU(80);
+    case 128: AU(128);
+    case 256: AU(256);
+    default: return -2;
+  }
+#undef AU
+  return (int)hipGetLastError();
+}
+}  // namespace
+
+extern "C" int edge_decode_attn_combine(const float* part_acc, const float* part_ml, int nsplit, int B, int Hq, int D, void* out,
+                                        int64_t o_sb, int h16, hipStream_t st);
+
+// edge_decode_attn's FUSED form (B <= 4 rows, 16-bit output, every query head a workgroup of its own) beside
+// h = gelu(y . Wup^T + bias) of the B rows y [B, K]: act 1 tanh, 0 erf.  -2: not taken.
+extern "C" int edge_attn_up(const void* qkv, int64_t q_sb, void* kc, void* vc, int64_t c_sb, int64_t c_sh, const int* seq_lens,
+                            int B, int Hq, int Hkv, int D, float scale, int ch, int nsplit, void* out, int64_t o_sb,
+                            float* part_acc, float* part_ml, const int* pos, const float* cs, int rot, const void* y,
+                            const void* w, const void* bias, void* h, int N, int K, int act, int h16, hipStream_t st) {
+  if (B < 1 || B > 4 || Hkv < 1 || Hq % Hkv != 0 || N <= 0 || N % 16 != 0 || K <= 0 || K % 64 != 0 || nsplit < 1) return -2;
+  if (pos == nullptr || (rot > 0 && (cs == nullptr || rot % 16 != 0 || rot > D))) return -2;
+  const AttnArgs a{(const bf16_t*)qkv, q_sb, (bf16_t*)kc, (bf16_t*)vc, c_sb, c_sh, seq_lens, scale * 1.4426950408889634f,
+                   ch, nsplit, Hq, (bf16_t*)out, o_sb, part_acc, part_ml,
+                   Fuse{pos, cs, rot, q_sb, nullptr, nullptr, 0, Hq / Hkv, 1}};
+  const Proj p{(const bf16_t*)y, (const bf16_t*)w, (const bf16_t*)bias, (bf16_t*)h, N, K};
+  const int r = h16 ? run_attn_up<true>(a, p, B, D, act, st) : run_attn_up<false>(a, p, B, D, act, st);
+  if (r != 0 || nsplit == 1) return r;
+  return edge_decode_attn_combine(part_acc, part_ml, nsplit, B, Hq, D, out, o_sb, h16, st);
+}
+
+// a = x . Wo^T + bo (x [M, Ko]) beside y = h . Wd^T + bd (h [M, Kd]), M <= 4 rows of N numbers each.  -2: not taken.
+extern "C" int edge_o_down(const void* x, const void* wo, const void* bo, void* a, int Ko, const void* h, const void* wd,
+                           const void* bd, void* y, int Kd, int M, int N, int h16, hipStream_t st) {
+  if (M < 1 || M > 4 || N <= 0 || N % 16 != 0 || Ko <= 0 || Ko % 64 != 0 || Kd <= 0 || Kd % 64 != 0) return -2;
+  const Proj o{(const bf16_t*)x, (const bf16_t*)wo, (const bf16_t*)bo, (bf16_t*)a, N, Ko};
+  const Proj d{(const bf16_t*)h, (const bf16_t*)wd, (const bf16_t*)bd, (bf16_t*)y, N, Kd};
+  const dim3 grid(2 * (N / 16)), block(PW * 64);
+  if (h16) hipLaunchKernelGGL(o_down_kernel<true>, grid, block, 0, st, o, d, M);
+  else hipLaunchKernelGGL(o_down_kernel<false>, grid, block, 0, st, o, d, M);
+  return (int)hipGetLastError();
+}

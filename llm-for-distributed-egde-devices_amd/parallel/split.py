@@ -24,7 +24,7 @@ import torch.nn as nn
 
 from ..engine.kv_cache import KVCache
 from ..models.decoder import AttnCtx, DecoderLM
-from ..models.layers import PartialSum
+from ..models.layers import BranchRows, PartialSum
 from .partition import partition_model
 
 
@@ -136,7 +136,7 @@ class SplitLM(nn.Module):
             c = self._ctx_on(ctx, dev)
             xd = x.parts.device if isinstance(x, PartialSum) else x.device   # split-K slices (o / down)
             if xd != dev:                                    # the inter-stage hop (xGMI peer copy)
-                if isinstance(x, PartialSum):
+                if isinstance(x, (BranchRows, PartialSum)):
                     x = x.materialize()
                 x = x.to(dev, non_blocking=True)
                 residual = residual.to(dev, non_blocking=True) if residual is not None else None
@@ -144,7 +144,7 @@ class SplitLM(nn.Module):
                 x, residual = layer(x, residual, c)
         c = self._ctx_on(ctx, self.devices[-1])
         if self._head_embed is not None:
-            if isinstance(x, PartialSum):
+            if isinstance(x, (BranchRows, PartialSum)):
                 x = x.materialize()
             if logits == "last" and c.T > 1:
                 idx = c.last_rows(x.device)

@@ -1,0 +1,103 @@
+"""Independent parts of a parallel-residual decode step in one launch (decode_pair.hip) against float64 and the separate ops."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+EPS = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}
+
+
+def _rows(g, *shape, dtype, scale=1.0):
+    return (torch.randn(*shape, generator=g) * scale).to(dtype).cuda()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,Ko,Kd", [(1, 16, 64, 64), (2, 2048, 2048, 8192), (4, 2560, 2560, 10240), (3, 48, 320, 192), (1, 272, 2112, 512)])
+def test_o_down(cuda, dtype, M, N, Ko, Kd):
+    from edgellm import ops
+    g = torch.Generator().manual_seed(N + Ko + Kd + M)
+    for with_bias in (False, True):
+        xs, ws, bs = [], [], []
+        for K in (Ko, Kd):
+            xs.append(_rows(g, M, K, dtype=dtype))
+            ws.append(_rows(g, N, K, dtype=dtype, scale=K ** -0.5))
+            bs.append(_rows(g, N, dtype=dtype) if with_bias else None)
+        out = ops.ext().decode_o_down(xs[0], ops.pack_bf16_weight(ws[0]), bs[0], xs[1], ops.pack_bf16_weight(ws[1]), bs[1], N)
+        for y, x, w, b, K in zip(out, xs, ws, bs, (Ko, Kd)):
+            ref = x.double() @ w.double().T + (0 if b is None else b.double())
+            # one rounding of the result and fp32 sums of K products
+            bound = EPS[dtype] * ref.abs() + 2.0 ** -24 * K * (x.double().abs() @ w.double().abs().T)
+            assert ((y.double() - ref).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("act", ["gelu", "gelu_tanh"])
+@pytest.mark.parametrize("B,D,Hq,Hkv,S,lens,N,K", [
+    (1, 256, 8, 8, 128, [1], 8192, 2048), (1, 80, 32, 32, 320, [300], 10240, 2560), (4, 64, 12, 12, 700, [3, 700, 257, 64], 64, 768),
+    (2, 128, 8, 2, 256, [255, 256], 16, 64), (3, 256, 4, 1, 1100, [1100, 900, 5], 400, 320)])
+def test_attn_up(cuda, dtype, act, B, D, Hq, Hkv, S, lens, N, K):
+    from edgellm import ops
+    g = torch.Generator().manual_seed(B * D + S + N)
+    rot = 16 * (D // 32)
+    qkv = _rows(g, B, (Hq + 2 * Hkv) * D, dtype=dtype)
+    k1, v1 = (_rows(g, B, Hkv, S, D, dtype=dtype) for _ in range(2))
+    k2, v2 = k1.clone(), v1.clone()
+    seq = torch.tensor(lens, dtype=torch.int32).cuda()
+    pos = seq - 1
+    rope = ops.rope_tables(rot, S, 10000.0, None, device="cuda")
+    y, w, b = _rows(g, B, K, dtype=dtype), _rows(g, N, K, dtype=dtype, scale=K ** -0.5), _rows(g, N, dtype=dtype)
+    ref, _ = ops.decode_attention_fused(qkv, pos, rope, k1, v1, seq, Hq, D ** -0.5, max(lens), rot)
+    a, h = ops.decode_attn_up(qkv, pos, rope, k2, v2, seq, Hq, D ** -0.5, max(lens), rot, y, ops.pack_bf16_weight(w), b, N, act)
+    assert torch.equal(k1, k2) and torch.equal(v1, v2)
+    # the same products and weights; the fp32 sums meet in another order: at most the last rounding differs
+    assert ((a.view(B, Hq, D).float() - ref.float()).abs() <= 2 * EPS[dtype] * ref.float().abs() + 1e-5).all()
+    z = y.double() @ w.double().T + b.double()
+    e = EPS[dtype] * z.abs() + 2.0 ** -24 * K * (y.double().abs() @ w.double().abs().T)
+    gelu = lambda t: torch.nn.functional.gelu(t, approximate="tanh" if act == "gelu_tanh" else "none")  # noqa: E731
+    # gelu's slope is at most 1.13; then the result's own rounding and fp32 function error
+    assert ((h.double() - gelu(z)).abs() <= 1.13 * e + EPS[dtype] * gelu(z).abs() + 2.0 ** -22 * (1 + z.abs())).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,K", [(1, 2048), (4, 2560), (3, 768)])
+@pytest.mark.parametrize("two", [False, True])
+def test_norm_of_both_branches_is_the_norm_kernels(cuda, dtype, M, K, two):
+    from edgellm import ops
+    g = torch.Generator().manual_seed(M * K)
+    x, x2, res = (_rows(g, M, K, dtype=dtype) for _ in range(3))
+    g1, b1, g2, b2 = (_rows(g, K, dtype=dtype) for _ in range(4))
+    w = _rows(g, 64, K, dtype=dtype, scale=K ** -0.5)
+    h, y = torch.empty_like(x), torch.empty_like(x)
+    out = ops.gemv_bf16_ln(x, res, g1, b1, 1e-5, h, ops.pack_bf16_weight(w), None, 64, None, y_out=y, x2=x2,
+                           gamma2=g2 if two else None, beta2=b2 if two else None)
+    n1, r = ops.layer_norm(x + x2, g1, b1, 1e-5, res)
+    n2, _ = ops.layer_norm(r, g2 if two else g1, b2 if two else b1, 1e-5, None)
+    assert torch.equal(h, r) and torch.equal(y, n2)
+    assert torch.equal(out, ops.linear_bf16(n1, w, None, packed=ops.pack_bf16_weight(w)))
+
+
+@pytest.mark.parametrize("family,dtype", [("gpt_neox", torch.float16), ("phi", torch.bfloat16)])
+def test_decode_steps_agree_with_the_separate_launches(cuda, family, dtype, monkeypatch):
+    from edgellm.engine import Generator, SamplingParams
+    from edgellm.models import build_model, tiny
+    from edgellm.models.decoder import DecoderLayer
+    cfg = tiny(family, num_layers=3, hidden_size=256, num_heads=4, num_kv_heads=4, intermediate_size=512, rotary_dim=32)
+    model = build_model(cfg, dtype=dtype, device="cuda", seed=3)
+    sp = SamplingParams(max_new_tokens=5, temperature=0.0, do_sample=False) if "do_sample" in SamplingParams.__dataclass_fields__ \
+        else SamplingParams(max_new_tokens=5, top_k=1)
+    prompts = [[5, 9, 2, 7, 1], [3, 8, 8, 4, 6]]
+    used = []
+    real = DecoderLayer._pair
+    monkeypatch.setattr(DecoderLayer, "_pair", lambda self, *a: used.append(1) or real(self, *a))
+    one = Generator(model, max_batch=2, max_seq=32)
+    one.generate(prompts, sp, seed=1)
+    k1, v1 = one.kv.k.clone(), one.kv.v.clone()
+    assert used
+    monkeypatch.setattr(DecoderLayer, "_pair_ok", lambda self, *a: False)
+    two = Generator(model, max_batch=2, max_seq=32)
+    two.generate(prompts, sp, seed=1)
+    for a, b in ((k1, two.kv.k), (v1, two.kv.v)):
+        d = (a.float() - b.float()).norm() / b.float().norm()
+        assert d < 4 * EPS[dtype], d                     # three layers of differing last roundings
+    assert math.isfinite(float(k1.float().abs().max()))
