@@ -292,33 +292,37 @@ class DecoderLayer(nn.Module):
                 and getattr(self.mlp.up, "pending_ln_ok", lambda **k: False)(geluq=True)
                 and getattr(self.mlp.down, "group_scales_ok", lambda m: False)(x.shape[0]))
 
-    def _pair_ok(self, x, ctx: AttnCtx) -> bool:
-        """Rows that ``_ln_deferred`` takes whose independent parts can share launches (``_pair``): a plain decode step over a
-        16-bit cache, plain 16-bit projections, and nobody who watches a module's own call."""
-        o, down = self.attn.o, self.mlp.down
+    def _pair_ok(self, x, ctx: AttnCtx, kind) -> bool:
+        """Rows that ``_ln_deferred`` / ``_ln_deferred_l8`` take whose independent parts can share launches (``_pair``): a plain
+        decode step over a 16-bit cache, projections of one ``kind``, and nobody who watches a module's own call."""
+        qkv, o, up, down = self.attn.qkv, self.attn.o, self.mlp.up, self.mlp.down
         return (ctx.mode == "decode" and ctx.T == 1 and ctx.B == x.shape[0] and ctx.attn_hook is None
                 and self.cfg.head_dim in ops.DECODE_ATTN_DIMS and self.cfg.rotary_dim % 16 == 0
-                and not getattr(ctx.kv, "quantized", False) and type(o) is Linear and type(down) is Linear
-                and o.pair_ok() and down.pair_ok() and self.norm1.eps == (self.norm2 or self.norm1).eps
-                and not any(m._forward_hooks or m._forward_pre_hooks
-                            for m in (self.attn, self.mlp, self.attn.qkv, o, self.mlp.up, down)))
+                and self.cfg.act in ("gelu_tanh", "gelu") and not getattr(ctx.kv, "quantized", False)
+                and all(type(m) is kind for m in (qkv, o, up, down)) and up.pair_ok(up=True) and o.pair_ok() and down.pair_ok()
+                and (kind is Linear or o.in_features <= 4096 < down.in_features)
+                and self.norm1.eps == (self.norm2 or self.norm1).eps
+                and not any(m._forward_hooks or m._forward_pre_hooks for m in (self.attn, self.mlp, qkv, o, up, down)))
 
     def _pair(self, x, residual, ctx: AttnCtx):
-        """A parallel-residual decode step in three launches (decode_pair.hip): qkv with the norm(s) in its prologue,
-        attention beside up, o beside down."""
+        """A parallel-residual decode step in three launches (decode_pair.hip, decode_pair_i8.hip): qkv with the norm(s) in its
+        prologue, attention beside up, o beside down."""
         cfg, n1 = self.cfg, self.norm1
         n2 = n1 if self.norm2 is None else self.norm2
         x, x2 = (x.mlp, x.attn) if isinstance(x, BranchRows) else (x, None)
         qkv, o, up, down = self.attn.qkv, self.attn.o, self.mlp.up, self.mlp.down
         h, y = torch.empty_like(x), torch.empty_like(x)
-        q = qkv.forward_ln(PendingLN(x, residual, n1.weight, n1.bias, n1.eps, h, y, x2=x2, y_weight=n2.weight, y_bias=n2.bias))
+        q = qkv(PendingLN(x, residual, n1.weight, n1.bias, n1.eps, h, y, x2=x2, y_weight=n2.weight, y_bias=n2.bias))
         k_cache, v_cache = ctx.kv.layer(self.idx)
         rot = cfg.rotary_dim if cfg.pos_emb == "rope" else 0
-        a, m = ops.decode_attn_up(q.view(ctx.B, -1), ctx.start_pos, ctx.rope if rot else None, k_cache, v_cache, ctx.seq_lens,
-                                  cfg.num_heads, self.attn.scale, ctx.max_len, rot, y, up.packed_weight(), up.bias,
-                                  up.out_features, cfg.act)
-        return BranchRows(*ops.ext().decode_o_down(a, o.packed_weight(), o.bias, m, down.packed_weight(), down.bias,
-                                                   cfg.hidden_size)), h
+        step = (q.view(ctx.B, -1), ctx.start_pos, ctx.rope if rot else None, k_cache, v_cache, ctx.seq_lens, cfg.num_heads,
+                self.attn.scale, int(ctx.max_len), rot, y)
+        C, W = ops.ext(), cfg.hidden_size
+        if type(o) is Linear:
+            a, m = ops.decode_attn_up(*step, up.packed_weight(), up.bias, up.out_features, cfg.act)
+            return BranchRows(*C.decode_o_down(a, o.packed_weight(), o.bias, m, down.packed_weight(), down.bias, W)), h
+        a, m = C.llmint8_attn_up(*step, *up.pair_args(), up.out_features, up._ACT[cfg.act])
+        return BranchRows(*C.llmint8_o_down(a, *o.pair_args(), m, *down.pair_args(), W)), h
 
     def forward(self, x, residual, ctx: AttnCtx):
         cfg = self.cfg
@@ -341,7 +345,8 @@ class DecoderLayer(nn.Module):
         qa = self.attn.qkv.takes_quantized_input
         qm = self.mlp.up.takes_quantized_input
         rows = x.mlp if isinstance(x, BranchRows) else x
-        if self._ln_deferred(rows, qa, qm) and self._pair_ok(rows, ctx):
+        if self._ln_deferred(rows, qa, qm) and self._pair_ok(rows, ctx, Linear) or \
+                self._ln_deferred_l8(rows, qa, qm) and self._pair_ok(rows, ctx, type(self.attn.qkv)):
             return self._pair(x, residual, ctx)
         if isinstance(x, BranchRows):
             x = x.materialize()

@@ -171,7 +171,7 @@ class Linear(nn.Module):
                 and self.in_features <= 4096 and self.in_features % 64 == 0 and self.out_features % 16 == 0
                 and not self.split_k_out and ops.gpu_path(w))
 
-    def pair_ok(self) -> bool:
+    def pair_ok(self, up: bool = False) -> bool:
         """Whether this 16-bit projection of decode rows can share a launch with another part of its block
         (decode_pair.hip)."""
         w = self.weight

@@ -101,10 +101,18 @@ int edge_llmint8_outlier(void* out, const float* xo, const int* cols, const int*
                          const float* scb, int M, int N, int cmax, hipStream_t st);
 int edge_llmint8_gemv(const void* x, float thr, const void* Wp, const float* sw, const void* bias, const void* wt,
                       const float* scb, void* out, int N, int K, hipStream_t st, int act, const void* add);
-int edge_llmint8_gemv_norm(const void* x, const void* res, const void* gamma, const void* beta, float eps, int ln,
+int edge_llmint8_gemv_norm(const void* x, const void* x2, const void* res, const void* gamma, const void* beta, float eps, int ln,
                            void* res_out, void* y_out, float thr, const void* Wp, const float* sw, const void* bias,
                            const void* wt, const float* scb, void* out, int N, int K, hipStream_t st, int glu,
-                           int act);
+                           int act,
+                           const void* gamma2, const void* beta2);
+int edge_llmint8_attn_up(const void* qkv, int64_t q_sb, void* kc, void* vc, int64_t c_sb, int64_t c_sh, const int* seq_lens, int Hq,
+                         int Hkv, int D, float scale, int ch, int nsplit, void* out, float* part_acc, float* part_ml,
+                         const int* pos, const float* cs, int rot, const void* y, float thr, const void* w, const float* sw,
+                         const void* bias, const void* wt, const float* scb, void* h, int N, int K, int act, hipStream_t st);
+int edge_llmint8_o_down(const void* x, float thr_o, const void* wo, const float* swo, const void* bo, const void* wto,
+                        const float* scbo, void* a, int Ko, const void* h, float thr_d, const void* wd, const float* swd,
+                        const void* bd, const void* wtd, const float* scbd, void* y, int Kd, int N, hipStream_t st);
 int edge_llmint8_prep_rows(const void* x, int M, int K, float thr, void* q, float* sa, int* cols, int* count,
                            uint32_t* flags, uint32_t* take, hipStream_t st);
 int edge_llmint8_outlier_rows(void* out, const void* x, const int* cols, const int* count, const void* wt,
@@ -941,7 +949,8 @@ std::optional<at::Tensor> llmint8_gemv_norm(const at::Tensor& x, const std::opti
                                             const std::optional<at::Tensor>& y_out, double thr, const at::Tensor& wp,
                                             const at::Tensor& sw, const std::optional<at::Tensor>& bias,
                                             const at::Tensor& wt, const at::Tensor& scb, int64_t N, bool glu,
-                                            int64_t act) {
+                                            int64_t act, const std::optional<at::Tensor>& x2,
+                                            const std::optional<at::Tensor>& gamma2, const std::optional<at::Tensor>& beta2) {
   DEVICE_GUARD(x);
   need(x, at::kBFloat16, "x");
   need(gamma, at::kBFloat16, "gamma");
@@ -960,16 +969,88 @@ std::optional<at::Tensor> llmint8_gemv_norm(const at::Tensor& x, const std::opti
     TORCH_CHECK(residual->numel() == K && residual->data_ptr() != res_out.data_ptr(), "residual [1, K]");
   }
   if (y_out) { need(*y_out, at::kBFloat16, "y_out"); TORCH_CHECK(y_out->numel() == K, "y_out [1, K]"); }
+  if (x2) { need(*x2, at::kBFloat16, "x2"); TORCH_CHECK(x2->numel() == K && ln, "x2 [1, K], LayerNorm only"); }
+  if (gamma2) { need(*gamma2, at::kBFloat16, "gamma2"); TORCH_CHECK(gamma2->numel() == K && y_out && ln, "gamma2 [K]: y_out's"); }
+  if (beta2) { need(*beta2, at::kBFloat16, "beta2"); TORCH_CHECK(beta2->numel() == K && gamma2, "beta2 [K], beside gamma2"); }
   auto out = at::empty({1, glu ? N / 2 : N}, x.options());
-  const int r = edge_llmint8_gemv_norm(x.data_ptr(), residual ? residual->data_ptr() : nullptr, gamma.data_ptr(),
+  const int r = edge_llmint8_gemv_norm(x.data_ptr(), x2 ? x2->data_ptr() : nullptr, residual ? residual->data_ptr() : nullptr, gamma.data_ptr(),
                                        beta ? beta->data_ptr() : nullptr, (float)eps, ln ? 1 : 0, res_out.data_ptr(),
                                        y_out ? y_out->data_ptr() : nullptr, (float)thr, wp.data_ptr(),
                                        sw.data_ptr<float>(), bias ? bias->data_ptr() : nullptr, wt.data_ptr(),
                                        scb.data_ptr<float>(), out.data_ptr(), (int)N, (int)K, stream(), glu ? 1 : 0,
-                                       (int)act);
+                                       (int)act,
+                                       gamma2 ? gamma2->data_ptr() : nullptr, beta2 ? beta2->data_ptr() : nullptr);
   if (r == -2) return std::nullopt;
   check(r, "llmint8_gemv_norm");
   return out;
+}
+
+// One LLM.int8 projection of a two-part launch: packed int8 weight, its scales SCB / 127, bias, int8 W^T, SCB.
+void check_l8(const at::Tensor& wp, const at::Tensor& sw, const std::optional<at::Tensor>& bias, const at::Tensor& wt,
+              const at::Tensor& scb, int64_t N, int64_t K) {
+  check_w8a8_operands(wp, sw, bias, N, K);
+  need(wt, at::kChar, "weight_t");
+  need(scb, at::kFloat, "SCB");
+  TORCH_CHECK(wt.dim() == 2 && wt.size(0) == K && wt.size(1) == N && wt.is_contiguous() && scb.numel() == N,
+              "weight_t [K, N], SCB [N]");
+}
+
+// LLM.int8 decode step of one row (decode_pair_i8.hip): decode_attn_fused beside h = gelu(up(y)) (act 1 tanh, 2 erf), one launch.
+// None where no kernel takes the shapes.
+std::optional<std::tuple<at::Tensor, at::Tensor>> llmint8_attn_up(
+    const at::Tensor& qkv, const at::Tensor& start_pos, const std::optional<at::Tensor>& rope, at::Tensor& k_cache,
+    at::Tensor& v_cache, const at::Tensor& seq_lens, int64_t Hq, double scale, int64_t max_len_hint, int64_t rot,
+    const at::Tensor& y, double thr, const at::Tensor& wp, const at::Tensor& sw, const std::optional<at::Tensor>& bias,
+    const at::Tensor& wt, const at::Tensor& scb, int64_t N, int64_t act) {
+  DEVICE_GUARD(qkv);
+  need(qkv, at::kBFloat16, "qkv");
+  need(y, at::kBFloat16, "y");
+  const float* cs = check_fused_attn(qkv, start_pos, rope, k_cache, v_cache, seq_lens, Hq, max_len_hint, rot);
+  TORCH_CHECK(qkv.size(0) == 1 && y.dim() == 2 && y.size(0) == 1 && y.is_contiguous(), "one row");
+  const int64_t D = k_cache.size(3), Hkv = k_cache.size(1), K = y.size(1);
+  check_l8(wp, sw, bias, wt, scb, N, K);
+  TORCH_CHECK(act == 1 || act == 2, "act 1 (gelu tanh), 2 (gelu erf)");
+  if (Hq % Hkv != 0 || (D != 64 && D != 80 && D != 128 && D != 256) || N % 16 != 0 || K % 64 != 0 || K < 64 || K > 4096 ||
+      rot % 16 != 0 || rot > D)
+    return std::nullopt;
+  int ch = 0, nsplit = 0;
+  edge_decode_attn_plan(1, (int)Hkv, (int)max_len_hint, (int)D, &ch, &nsplit);
+  at::Tensor pacc, pml;
+  if (nsplit > 1) {
+    pacc = at::empty({Hq, nsplit, D}, qkv.options().dtype(at::kFloat));
+    pml = at::empty({Hq, nsplit, 2}, qkv.options().dtype(at::kFloat));
+  }
+  auto out = at::empty({1, Hq * D}, qkv.options()), h = at::empty({1, N}, qkv.options());
+  check(edge_llmint8_attn_up(qkv.data_ptr(), qkv.stride(0), k_cache.data_ptr(), v_cache.data_ptr(), k_cache.stride(0),
+                             k_cache.stride(1), seq_lens.data_ptr<int>(), (int)Hq, (int)Hkv, (int)D, (float)scale, ch, nsplit,
+                             out.data_ptr(), nsplit > 1 ? pacc.data_ptr<float>() : nullptr,
+                             nsplit > 1 ? pml.data_ptr<float>() : nullptr, start_pos.data_ptr<int>(), cs, (int)rot, y.data_ptr(),
+                             (float)thr, wp.data_ptr(), sw.data_ptr<float>(), bias ? bias->data_ptr() : nullptr, wt.data_ptr(),
+                             scb.data_ptr<float>(), h.data_ptr(), (int)N, (int)K, (int)act, stream()),
+        "llmint8_attn_up");
+  return std::make_tuple(out, h);
+}
+
+// The o and down projections of one LLM.int8 row in one launch, each into a row of its own; None where not taken.
+std::optional<std::tuple<at::Tensor, at::Tensor>> llmint8_o_down(
+    const at::Tensor& x, double thr_o, const at::Tensor& wo, const at::Tensor& swo, const std::optional<at::Tensor>& bo,
+    const at::Tensor& wto, const at::Tensor& scbo, const at::Tensor& h, double thr_d, const at::Tensor& wd, const at::Tensor& swd,
+    const std::optional<at::Tensor>& bd, const at::Tensor& wtd, const at::Tensor& scbd, int64_t N) {
+  DEVICE_GUARD(x);
+  need(x, at::kBFloat16, "x");
+  need(h, at::kBFloat16, "h");
+  TORCH_CHECK(x.dim() == 2 && x.size(0) == 1 && h.dim() == 2 && h.size(0) == 1, "one row");
+  const int64_t Ko = x.size(1), Kd = h.size(1);
+  check_l8(wo, swo, bo, wto, scbo, N, Ko);
+  check_l8(wd, swd, bd, wtd, scbd, N, Kd);
+  auto a = at::empty({1, N}, x.options()), y = at::empty({1, N}, x.options());
+  const int r = edge_llmint8_o_down(x.data_ptr(), (float)thr_o, wo.data_ptr(), swo.data_ptr<float>(), bo ? bo->data_ptr() : nullptr,
+                                    wto.data_ptr(), scbo.data_ptr<float>(), a.data_ptr(), (int)Ko, h.data_ptr(), (float)thr_d,
+                                    wd.data_ptr(), swd.data_ptr<float>(), bd ? bd->data_ptr() : nullptr, wtd.data_ptr(),
+                                    scbd.data_ptr<float>(), y.data_ptr(), (int)Kd, (int)N, stream());
+  if (r == -2) return std::nullopt;
+  check(r, "llmint8_o_down");
+  return std::make_tuple(a, y);
 }
 
 // LLM.int8 preparation for any number of rows, uncapped (every outlier column to the 16-bit part):
@@ -1504,12 +1585,20 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("llmint8_prep", &llmint8_prep, "LLM.int8 decode preparation (outlier columns on the device)");
   m.def("llmint8_outlier", &llmint8_outlier, "LLM.int8 decode outlier part, added in place");
   m.def("gemv_bf16_norm", &gemv_bf16_norm, "16-bit decode GEMV with the RMSNorm in its prologue (M <= 4)");
-  m.def("gemv_bf16_ln", &gemv_bf16_ln, "16-bit decode GEMV with the LayerNorm in its prologue (M <= 4)");
+  m.def("gemv_bf16_ln", &gemv_bf16_ln, "16-bit decode GEMV with the LayerNorm in its prologue (M <= 4)", py::arg("x"),
+        py::arg("residual"), py::arg("gamma"), py::arg("beta"), py::arg("eps"), py::arg("res_out"), py::arg("wp"), py::arg("bias"),
+        py::arg("N"), py::arg("epi"), py::arg("y_out"), py::arg("x2") = py::none(), py::arg("gamma2") = py::none(),
+        py::arg("beta2") = py::none());
   m.def("decode_attn_up", &decode_attn_up, "decode attention beside the up projection of a parallel-residual block (M <= 4)");
   m.def("decode_o_down", &decode_o_down, "o beside the down projection of a parallel-residual block (M <= 4)");
   m.def("w8a8_gemv_ln", &w8a8_gemv_ln, "W8A8 decode GEMV with the LayerNorm + int8 quant in its prologue (M <= 4)");
   m.def("llmint8_gemv", &llmint8_gemv, "LLM.int8 projection of one row in one launch (prep in the GEMV prologue)");
-  m.def("llmint8_gemv_norm", &llmint8_gemv_norm, "LLM.int8 projection of RMSNorm / LayerNorm(x + residual), one launch");
+  m.def("llmint8_gemv_norm", &llmint8_gemv_norm, "LLM.int8 projection of RMSNorm / LayerNorm(x + residual), one launch",
+        py::arg("x"), py::arg("residual"), py::arg("gamma"), py::arg("beta"), py::arg("eps"), py::arg("ln"), py::arg("res_out"),
+        py::arg("y_out"), py::arg("thr"), py::arg("wp"), py::arg("sw"), py::arg("bias"), py::arg("wt"), py::arg("scb"), py::arg("N"),
+        py::arg("glu"), py::arg("act"), py::arg("x2") = py::none(), py::arg("gamma2") = py::none(), py::arg("beta2") = py::none());
+  m.def("llmint8_attn_up", &llmint8_attn_up, "decode attention beside the LLM.int8 up projection of one row");
+  m.def("llmint8_o_down", &llmint8_o_down, "o beside the down projection of one LLM.int8 row");
   m.def("llmint8_prep_rows", &llmint8_prep_rows, "LLM.int8 preparation for any rows (uncapped, on the device)");
   m.def("llmint8_outlier_rows", &llmint8_outlier_rows, "LLM.int8 outlier part for any rows, added in place");
   m.def("gemv_bf16_splitk", &gemv_bf16_splitk, "bf16 decode GEMV, split-K fp32 partial slices");

@@ -8,12 +8,10 @@
 // The attention's come first in the grid: they are the longest chains.  us a layer of Pythia-1B, fp16, one row: attention 5.3
 // and up 8.3 are 10.3 together, o 5.0 and down 10.4 are 10.9; whole answers, one row: Pythia-1B 48 tokens 33.9 -> 28.2 ms
 // (4 rows, 32 tokens 27.6 -> 22.3), Phi-2 32 tokens 57.8 -> 47.0, 64 tokens behind 200 116.6 -> 90.5.
-#include "attn_decode.h"
+#include "decode_pair.h"
 #include "gemv_bf16.h"
 
 namespace {
-constexpr int PW = 8;                      // waves a workgroup
-
 struct Proj {
   const bf16_t *x, *w, *bias;              // rows [M, K], packed weights, bias [N] or null
   bf16_t* out;
@@ -32,29 +30,12 @@ __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act
   else gemv_bf16_body<PW, 1, 1, 2, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
 }
 
-struct AttnArgs {
-  const bf16_t* q;
-  int64_t q_sb;
-  bf16_t *kc, *vc;
-  int64_t c_sb, c_sh;
-  const int* seq_lens;
-  float scale_log2;
-  int ch, nsplit, ny;                      // ny: query heads (each a workgroup of its own)
-  bf16_t* out;
-  int64_t o_sb;
-  float *part_acc, *part_ml;
-  Fuse fz;
-};
-
 template <int D, bool DIRECT, bool HF>
 __global__ void __launch_bounds__(PW * 64, 4) attn_up_kernel(AttnArgs a, Proj p, int M, int act, int na) {
-  __shared__ __attribute__((aligned(16))) float smem[PW * D + 2 * PW + 2];
+  __shared__ __attribute__((aligned(16))) float smem[attn_part_lds<D>()];
   const int bid = blockIdx.x;
   if (bid < na) {
-    const int s = bid % a.nsplit, r = bid / a.nsplit;
-    decode_attn_body<D, 1, DIRECT, true, false, 4, HF, PW, UNROLL_DEF>(smem, s, r % a.ny, a.ny, r / a.ny, a.q, a.q_sb, a.kc, a.vc,
-                                                                      a.c_sb, a.c_sh, a.seq_lens, a.scale_log2, a.ch, a.nsplit,
-                                                                      a.out, a.o_sb, a.part_acc, a.part_ml, a.fz);
+    attn_part<D, DIRECT, HF>(smem, bid, a);
   } else {
     proj_body<EPI_GELU_ANY, HF>(bid - na, p, M, act);
   }
@@ -87,9 +68,6 @@ int run_attn_up(const AttnArgs& a, const Proj& p, int B, int D, int act, hipStre
   return (int)hipGetLastError();
 }
 }  // namespace
-
-extern "C" int edge_decode_attn_combine(const float* part_acc, const float* part_ml, int nsplit, int B, int Hq, int D, void* out,
-                                        int64_t o_sb, int h16, hipStream_t st);
 
 // edge_decode_attn's FUSED form (B <= 4 rows, 16-bit output, every query head a workgroup of its own) beside
 // h = gelu(y . Wup^T + bias) of the B rows y [B, K]: act 1 tanh, 0 erf.  -2: not taken.

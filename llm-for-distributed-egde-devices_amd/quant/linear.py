@@ -323,6 +323,23 @@ class LLMInt8Linear(nn.Module):
             return self._forward(x, act=self._ACT[act])
         return None
 
+    def pair_ok(self, up: bool = False) -> bool:
+        """Whether this projection of one row can share a launch with another part of its block (decode_pair_i8.hip); up: as
+        the projection beside attention."""
+        K, N = self.in_features, self.out_features
+        return (self._device_ok() and self.ONE_LAUNCH and K % 64 == 0 and N % 16 == 0 and K <= (4096 if up else 12288)
+                and ops.gpu_path(self.w_packed))
+
+    def pair_args(self):
+        """Operands of a one-row launch: threshold, packed weight, scales, bias, W^T, SCB."""
+        self._transposed(self.w_packed.device)
+        return self.threshold, self.w_packed, self._w_deq, self.bias, self._weight_t, self.SCB
+
+    def _transposed(self, device):
+        if self._weight_t is None or self._weight_t.device != device:
+            self._weight_t = self.weight_i8.t().contiguous()          # W^T: outlier columns as rows
+            self._w_deq = self.SCB / 127.0
+
     def _forward(self, x, glu: bool = False, act: int = 0, add: Optional[torch.Tensor] = None):
         if isinstance(x, PendingLN):
             y = None
@@ -330,12 +347,10 @@ class LLMInt8Linear(nn.Module):
             if (x.x.shape[0] == 1 and x.x.is_cuda and ops.gpu_path(x.x) and x.x.dtype == torch.bfloat16
                     and self._device_ok() and self.ONE_LAUNCH and K <= 4096):
                 C = ops.ext()
-                if self._weight_t is None or self._weight_t.device != x.x.device:
-                    self._weight_t = self.weight_i8.t().contiguous()
-                    self._w_deq = self.SCB / 127.0
+                self._transposed(x.x.device)
                 y = C.llmint8_gemv_norm(x.x.contiguous(), x.residual.contiguous() if x.residual is not None else None,
                                         x.weight, x.bias, x.eps, not x.rms, x.h, x.y, self.threshold, self.w_packed,
-                                        self._w_deq, self.bias, self._weight_t, self.SCB, N, glu, act)
+                                        self._w_deq, self.bias, self._weight_t, self.SCB, N, glu, act, x.x2, x.y_weight, x.y_bias)
             if y is not None or glu or act:
                 return y if add is None else y + add.view_as(y)
             x = x.materialize()
@@ -348,9 +363,7 @@ class LLMInt8Linear(nn.Module):
         if x2.is_cuda and ops.gpu_path(x2) and x2.dtype == torch.bfloat16 and self._device_ok():
             # outlier columns found on the device (llmint8.hip), no host sync at any row count
             C = ops.ext()
-            if self._weight_t is None or self._weight_t.device != x2.device:
-                self._weight_t = self.weight_i8.t().contiguous()          # W^T: outlier columns as rows
-                self._w_deq = self.SCB / 127.0
+            self._transposed(x2.device)
             x2 = x2.contiguous()
             if x2.shape[0] == 1 and K <= 12288 and K % 64 == 0 and self.ONE_LAUNCH:
                 # batch 1: outlier discovery, quantisation and the outlier part inside the GEMV

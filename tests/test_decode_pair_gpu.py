@@ -101,3 +101,66 @@ def test_decode_steps_agree_with_the_separate_launches(cuda, family, dtype, monk
         d = (a.float() - b.float()).norm() / b.float().norm()
         assert d < 4 * EPS[dtype], d                     # three layers of differing last roundings
     assert math.isfinite(float(k1.float().abs().max()))
+
+
+def _l8(g, N, K, bias=True):
+    from edgellm.models.layers import Linear
+    from edgellm.quant.linear import LLMInt8Linear
+    lin = Linear(K, N, bias, torch.bfloat16, "cuda")
+    lin.weight.data.copy_(torch.randn(N, K, generator=g) * K ** -0.5)
+    if bias:
+        lin.bias.data.copy_(torch.randn(N, generator=g))
+    return LLMInt8Linear.from_float(lin)
+
+
+def _row(g, K, outliers):
+    x = torch.randn(1, K, generator=g)
+    at = torch.randperm(K, generator=g)[:outliers]
+    x[0, at] = 6.5 + 3 * torch.rand(outliers, generator=g)
+    return x.to(torch.bfloat16).cuda()
+
+
+@pytest.mark.parametrize("N,Ko,Kd,out", [(2560, 2560, 10240, 7), (16, 64, 4160, 0), (2048, 2048, 8192, 300), (272, 4096, 12288, 64)])
+def test_llmint8_o_down_is_each_projections_own(cuda, N, Ko, Kd, out):
+    from edgellm import ops
+    g = torch.Generator().manual_seed(N + Kd)
+    o, d = _l8(g, N, Ko), _l8(g, N, Kd, bias=False)
+    x, h = _row(g, Ko, min(out, Ko)), _row(g, Kd, out)
+    a, y = ops.ext().llmint8_o_down(x, *o.pair_args(), h, *d.pair_args(), N)
+    assert torch.equal(a, o(x)) and torch.equal(y, d(h))
+
+
+@pytest.mark.parametrize("act", ["gelu", "gelu_tanh"])
+@pytest.mark.parametrize("D,Hq,Hkv,S,n,N,K", [(80, 32, 32, 128, 77, 10240, 2560), (256, 8, 8, 64, 1, 8192, 2048),
+                                              (64, 4, 2, 700, 700, 48, 64), (128, 16, 16, 300, 290, 4112, 4096)])
+def test_llmint8_attn_up(cuda, act, D, Hq, Hkv, S, n, N, K):
+    from edgellm import ops
+    g = torch.Generator().manual_seed(D + S + N)
+    up = _l8(g, N, K)
+    y = _row(g, K, 3)
+    rot = 16 * (D // 32)
+    qkv = _rows(g, 1, (Hq + 2 * Hkv) * D, dtype=torch.bfloat16)
+    k1, v1 = (_rows(g, 1, Hkv, S, D, dtype=torch.bfloat16) for _ in range(2))
+    k2, v2 = k1.clone(), v1.clone()
+    seq = torch.tensor([n], dtype=torch.int32).cuda()
+    rope = ops.rope_tables(rot, S, 10000.0, None, device="cuda")
+    ref, _ = ops.decode_attention_fused(qkv, seq - 1, rope, k1, v1, seq, Hq, D ** -0.5, n, rot)
+    a, h = ops.ext().llmint8_attn_up(qkv, seq - 1, rope, k2, v2, seq, Hq, D ** -0.5, n, rot, y, *up.pair_args(), N, up._ACT[act])
+    assert torch.equal(k1, k2) and torch.equal(v1, v2)
+    assert ((a.view(1, Hq, D).float() - ref.float()).abs() <= 2 ** -7 * ref.float().abs() + 1e-5).all()
+    assert torch.equal(h, up.gelu_fused(y, act))
+
+
+@pytest.mark.parametrize("K", [64, 2048, 2560, 4096])
+def test_llmint8_norm_of_both_branches(cuda, K):
+    from edgellm import ops
+    from edgellm.models.layers import PendingLN
+    g = torch.Generator().manual_seed(K)
+    x, x2, res = (_rows(g, 1, K, dtype=torch.bfloat16) for _ in range(3))
+    g1, b1, g2, b2 = (_rows(g, K, dtype=torch.bfloat16) for _ in range(4))
+    m = _l8(g, 272, K)
+    h, y = torch.empty_like(x), torch.empty_like(x)
+    out = m(PendingLN(x, res, g1, b1, 1e-5, h, y, x2=x2, y_weight=g2, y_bias=b2))
+    n1, r = ops.layer_norm(x + x2, g1, b1, 1e-5, res)
+    n2, _ = ops.layer_norm(r, g2, b2, 1e-5, None)
+    assert torch.equal(h, r) and torch.equal(y, n2) and torch.equal(out, m(n1))
