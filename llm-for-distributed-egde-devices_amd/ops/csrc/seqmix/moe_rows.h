@@ -9,16 +9,19 @@ constexpr int MR_GLU = 0, MR_PLAIN = 1, MR_RELU2 = 2;
 
 // Pairs p < routed are (token, choice) of the routed experts, pairs after them one per token of the shared expert (own
 // weights w_sh, widths K_sh -> R_sh).  MR_GLU: out = act(gate . x, up . x), weights [E, 2 R, K], rows of x per token; act =
-// silu(rw g) (rw u) (silu, rw = in_w[pair] or 1) or the clamped form.  MR_RELU2: out = max(W x, 0)^2, rows of x per token.
-// MR_PLAIN: out = W x, rows of x per pair.
+// silu(rw g) (rw u) (silu, rw = in_w[pair] or 1) or the clamped form.  MR_RELU2:
+// out = max(W x, 0)^2, rows of x per token.  MR_PLAIN: out = W x, rows of x per pair.
 // Bound by the chosen experts' weights.  A workgroup is (pair, 4 waves of 4 weight rows).  `share` (launch_moe_rows): pairs
 // of one expert belong to the first of them (at most 64 routed pairs, so one ballot names them), which runs them together,
 // up to four per reading of the rows; the others leave at once.  A wave has its four rows' next 1024 numbers (2048 for one
 // pair) in flight as contiguous KiBs and the inputs beside them in registers; the sums over lanes end with one sum per lane.
 // us for both launches, one wave per row and pair / this, bf16: 3 of 16 experts of 1024 x 1024, 1 token 11.1 / 7.4, 4 tokens
-// 18.8 / 17.4, 9 29.4 / 23.0; 4 of 32 of 2048 x 2048 26.5 / 20.9, 74 / 69, 159 / 113 (5.0 TB/s).  fp32 only for one
+// 18.8 / 17.2, 9 29.4 / 24.1; 4 of 32 of 2048 x 2048 26.5 / 20.9, 74 / 62, 159 / 107 (5.4 TB/s).  fp32 only for one
 // token (15.1 / 9.6): rows shared by several pairs need more registers than they save there (4 of 16 of 1024 x 1024,
 // 6 tokens 48.6 / 54.7, 16 tokens 102 / 141).
+// A grid's x dimension is the features: consecutive workgroups go to the eight dies in turn, and with the pairs there a count of 8,
+// 16 or 24 pairs gave every expert to one die's 32 CUs (us, pairs first / features first: 4 of 32 experts of 2048 x 2048, 4 tokens
+// 65.7 / 61.9, 6 88.0 / 74.9, 8 114 / 92.5 (5.4 TB/s); 4 of 16 of 1024 x 1024, 8 tokens 44.6 / 25.9; 2 of 8 of 512 x 520, 8 11.8 / 11.1).
 template <typename T, int MODE, int MT, int CH>
 __device__ __forceinline__ void moe_rows_run(const T* const (&wr)[4], const T* const (&xr)[MT], int K, float (&acc)[4 * MT]) {
   constexpr int Q = sizeof(T) / 2;                           // 16-byte loads per 8 numbers
@@ -64,9 +67,9 @@ __global__ void __launch_bounds__(NT) moe_rows_kernel(const T* __restrict__ in, 
                                                       int R_sh, int E, float limit, int silu, const float* __restrict__ in_w,
                                                       T* __restrict__ out, T* __restrict__ out_sh, int share) {
   constexpr int NF = MODE == MR_GLU ? 2 : 4;                 // output features of a wave
-  const int pair = blockIdx.x, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int pair = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool sh = pair >= routed;
-  const int k = sh ? K_sh : K, n = sh ? R_sh : R, f0 = (blockIdx.y * (NT / 64) + wave) * NF;
+  const int k = sh ? K_sh : K, n = sh ? R_sh : R, f0 = (blockIdx.x * (NT / 64) + wave) * NF;
   uint64_t mine = 1;                                         // pairs of this expert, from `first` on
   int first = pair;
   const T* we = w_sh;
@@ -147,7 +150,7 @@ void launch_moe_rows(const T* in, const T* in_sh, const int* idx, int routed, in
   // with a shared expert of 1024 x 1536 beside them, 9 tokens 42 / 36, 10 40.0 / 39.5, 16 49 / 92
   const int share = sizeof(T) == 2 && routed <= 64 && routed <= 12 * top && pairs - routed <= 12 &&
                     (int64_t)K * R * (MODE == MR_GLU ? 2 : 1) >= 1 << 20;
-  hipLaunchKernelGGL((moe_rows_kernel<T, MODE>), dim3(pairs, (big + FW - 1) / FW), dim3(NT), 0, st, in, in_sh, idx, routed, pairs,
+  hipLaunchKernelGGL((moe_rows_kernel<T, MODE>), dim3((big + FW - 1) / FW, pairs), dim3(NT), 0, st, in, in_sh, idx, routed, pairs,
                      top, w, w_sh, K, R, K_sh, R_sh, E, limit, silu, in_w, out, out_sh, share);
 }
 
