@@ -33,6 +33,11 @@ class MoEOut(NamedTuple):
     rows: Optional[torch.Tensor]        # int32 [T, top]: each choice's row of parts viewed [-1, W] (None: in order)
 
 
+def _plain(m: nn.Module) -> bool:
+    """A bias-free 16- or 32-bit projection whose own call nobody watches: its weight says all."""
+    return type(m) is Linear and m.bias is None and not (m._forward_hooks or m._forward_pre_hooks)
+
+
 class MoEFeedForward(nn.Module):
     def __init__(self, spec: MoESpec, width: int, dtype, device):
         super().__init__()
@@ -57,6 +62,11 @@ class MoEFeedForward(nn.Module):
         s = self.spec
         idx, wts = seqmix.moe_route(h, self.router, s.top, s.scale, s.router, self.router_b)
         on_input = s.weight_on == "input"
+        if s.shared_ff and s.act == "glu_clamp" and not on_input and _plain(self.shared_gu) and _plain(self.shared_down):
+            both = seqmix.moe_experts_glu_shared(h, idx, self.w_gu, self.w_down, s.limit, self.shared_gu.weight,
+                                                 self.shared_down.weight, s.shared_limit)
+            if both is not None:
+                return both[1], both[0], wts
         parts = seqmix.moe_experts(h, idx, self.w_gu, self.w_down, s.limit, s.act, wts if on_input else None)
         if on_input:
             wts = None

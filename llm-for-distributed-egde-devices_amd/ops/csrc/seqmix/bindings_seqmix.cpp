@@ -126,6 +126,9 @@ int64_t edge_sm_moe_gemm_ints(int64_t R, int E);
 int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff);
 int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void* w_down, int* ints, void* y, void* out, int T,
                      int top, int E, int W, int ff, int act, const float* row_w, float limit, hipStream_t st);
+int edge_sm_moe_experts_glu_shared(const void* h, int W, const int* idx, int top, const void* w_gu, const void* w_down, int ff,
+                                   float limit, const void* su, const void* sd, int sff, float limit_sh, void* y, void* ys,
+                                   void* out, void* out_sh, int rows, int E, int f32, hipStream_t st);
 int edge_sm_moe_experts_relu2(const void* h, int W, const int* idx, int top, const void* w_up, const void* w_down, int ff,
                               const void* su, const void* sd, int sff, void* y, void* ys, void* out, void* out_sh, int rows,
                               int E, int f32, hipStream_t st);
@@ -1124,6 +1127,37 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> sm_moe_route_grouped(const at::Te
   return {idx, wts, gw};
 }
 
+// (chosen experts' outputs [T, top, W], the shared expert's [T, W]) of clamped gated units, or nothing where the rows kernel
+// does not take these widths, types or addresses
+std::optional<std::tuple<at::Tensor, at::Tensor>> sm_moe_experts_glu_shared(const at::Tensor& h, const at::Tensor& idx,
+                                                                            const at::Tensor& w_gu, const at::Tensor& w_down,
+                                                                            double limit, const at::Tensor& su,
+                                                                            const at::Tensor& sd, double limit_sh) {
+  chk_act2(h, "h");
+  chk_i32(idx, "idx");
+  const int64_t T = h.size(0), W = h.size(1);
+  TORCH_CHECK(idx.dim() == 2 && idx.size(0) == T, "idx: int32 [T, top]");
+  TORCH_CHECK(w_gu.is_cuda() && w_gu.is_contiguous() && w_gu.dim() == 3 && w_gu.size(2) == W && w_gu.size(1) % 2 == 0 &&
+                  w_down.is_cuda() && w_down.is_contiguous() && w_down.dim() == 3 && w_down.size(0) == w_gu.size(0) &&
+                  w_down.size(1) == W && w_down.size(2) == w_gu.size(1) / 2 && w_gu.scalar_type() == h.scalar_type() &&
+                  w_down.scalar_type() == h.scalar_type(), "experts: w_gu [E, 2 ff, W], w_down [E, W, ff]");
+  if (!(su.device() == h.device() && su.is_contiguous() && su.dim() == 2 && su.size(1) == W && su.size(0) % 2 == 0 &&
+        sd.device() == h.device() && sd.is_contiguous() && sd.dim() == 2 && sd.size(0) == W && sd.size(1) == su.size(0) / 2 &&
+        su.scalar_type() == h.scalar_type() && sd.scalar_type() == h.scalar_type()))
+    return std::nullopt;
+  const int64_t top = idx.size(1), ff = w_gu.size(1) / 2, sff = sd.size(1);
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(h.device());
+  auto y = at::empty({T * top, ff}, h.options()), ys = at::empty({T, sff}, h.options());
+  auto out = at::empty({T, top, W}, h.options()), out_sh = at::empty({T, W}, h.options());
+  const int rc = edge_sm_moe_experts_glu_shared(h.data_ptr(), (int)W, idx.data_ptr<int>(), (int)top, w_gu.data_ptr(),
+                                                w_down.data_ptr(), (int)ff, (float)limit, su.data_ptr(), sd.data_ptr(), (int)sff,
+                                                (float)limit_sh, y.data_ptr(), ys.data_ptr(), out.data_ptr(), out_sh.data_ptr(),
+                                                (int)T, (int)w_gu.size(0), f32(h), stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_moe_experts_glu_shared");
+  return std::make_tuple(out, out_sh);
+}
+
 std::tuple<at::Tensor, at::Tensor> sm_moe_experts_relu2(const at::Tensor& h, const at::Tensor& idx, const at::Tensor& w_up,
                                                         const at::Tensor& w_down, const std::optional<at::Tensor>& su,
                                                         const std::optional<at::Tensor>& sd) {
@@ -1358,6 +1392,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_parallel_update", &sm_parallel_update);
   m.def("sm_glu_gelu", &sm_glu_gelu);
   m.def("sm_moe_route_grouped", &sm_moe_route_grouped);
+  m.def("sm_moe_experts_glu_shared", &sm_moe_experts_glu_shared);
   m.def("sm_moe_experts_relu2", &sm_moe_experts_relu2);
   m.def("sm_latent_expand_write", &sm_latent_expand_write);
   m.def("sm_head_expand_gate", &sm_head_expand_gate);

@@ -6,10 +6,11 @@
 namespace {
 
 constexpr int MR_GLU = 0, MR_PLAIN = 1, MR_RELU2 = 2;
+constexpr int MR_MAX_PAIRS = 65535;                          // a grid's second dimension
 
 // Pairs p < routed are (token, choice) of the routed experts, pairs after them one per token of the shared expert (own
 // weights w_sh, widths K_sh -> R_sh).  MR_GLU: out = act(gate . x, up . x), weights [E, 2 R, K], rows of x per token; act =
-// silu(rw g) (rw u) (silu, rw = in_w[pair] or 1) or the clamped form.  MR_RELU2:
+// silu(rw g) (rw u) (silu, rw = in_w[pair] or 1) or the clamped form (limit; limit_sh for the shared expert).  MR_RELU2:
 // out = max(W x, 0)^2, rows of x per token.  MR_PLAIN: out = W x, rows of x per pair.
 // Bound by the chosen experts' weights.  A workgroup is (pair, 4 waves of 4 weight rows).  `share` (launch_moe_rows): pairs
 // of one expert belong to the first of them (at most 64 routed pairs, so one ballot names them), which runs them together,
@@ -64,8 +65,9 @@ template <typename T, int MODE>
 __global__ void __launch_bounds__(NT) moe_rows_kernel(const T* __restrict__ in, const T* __restrict__ in_sh,
                                                       const int* __restrict__ idx, int routed, int pairs, int top,
                                                       const T* __restrict__ w, const T* __restrict__ w_sh, int K, int R, int K_sh,
-                                                      int R_sh, int E, float limit, int silu, const float* __restrict__ in_w,
-                                                      T* __restrict__ out, T* __restrict__ out_sh, int share) {
+                                                      int R_sh, int E, float limit, float limit_sh, int silu,
+                                                      const float* __restrict__ in_w, T* __restrict__ out, T* __restrict__ out_sh,
+                                                      int share) {
   constexpr int NF = MODE == MR_GLU ? 2 : 4;                 // output features of a wave
   const int pair = blockIdx.y, lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bool sh = pair >= routed;
@@ -113,8 +115,8 @@ __global__ void __launch_bounds__(NT) moe_rows_kernel(const T* __restrict__ in, 
     if (lane % (64 / V) == 0 && id / MT < NF && f < n) {
       float y = acc[0];
       if constexpr (MODE == MR_GLU) {
-        const float rw = in_w ? in_w[pm] : 1.f;
-        y = silu ? siluf_(rw * y) * (rw * up) : glu_clamp_f(y, up, limit);
+        const float rw = in_w && !sh ? in_w[pm] : 1.f;
+        y = silu ? siluf_(rw * y) * (rw * up) : glu_clamp_f(y, up, sh ? limit_sh : limit);
       }
       if constexpr (MODE == MR_RELU2) { y = fmaxf(y, 0.f); y *= y; }
       stf<T>((sh ? out_sh + (size_t)(pm - routed) * n : out + (size_t)pm * n) + f, y);
@@ -140,7 +142,7 @@ inline bool moe_rows_ok(int K, int K_sh, std::initializer_list<const void*> ps) 
 
 template <typename T, int MODE>
 void launch_moe_rows(const T* in, const T* in_sh, const int* idx, int routed, int pairs, int top, const T* w, const T* w_sh, int K,
-                     int R, int K_sh, int R_sh, int E, float limit, int silu, const float* in_w, T* out, T* out_sh,
+                     int R, int K_sh, int R_sh, int E, float limit, float limit_sh, int silu, const float* in_w, T* out, T* out_sh,
                      hipStream_t st) {
   constexpr int FW = (MODE == MR_GLU ? 2 : 4) * (NT / 64);
   const int big = pairs > routed && R_sh > R ? R_sh : R;
@@ -151,7 +153,7 @@ void launch_moe_rows(const T* in, const T* in_sh, const int* idx, int routed, in
   const int share = sizeof(T) == 2 && routed <= 64 && routed <= 12 * top && pairs - routed <= 12 &&
                     (int64_t)K * R * (MODE == MR_GLU ? 2 : 1) >= 1 << 20;
   hipLaunchKernelGGL((moe_rows_kernel<T, MODE>), dim3((big + FW - 1) / FW, pairs), dim3(NT), 0, st, in, in_sh, idx, routed, pairs,
-                     top, w, w_sh, K, R, K_sh, R_sh, E, limit, silu, in_w, out, out_sh, share);
+                     top, w, w_sh, K, R, K_sh, R_sh, E, limit, limit_sh, silu, in_w, out, out_sh, share);
 }
 
 }  // namespace

@@ -1075,11 +1075,11 @@ int edge_sm_moe_experts(const void* h, int W, const int* idx, int top, const voi
                         hipStream_t st) {
   if (rows == 0) return 0;
   if ((size_t)W * 4 > 60 * 1024 || (size_t)ff * 4 > 60 * 1024) return -3;
-  if ((!f32 || rows == 1) && moe_rows_ok(W, ff, {h, w_gu, w_down, y, out})) {
+  if ((!f32 || rows == 1) && (long)rows * top <= MR_MAX_PAIRS && moe_rows_ok(W, ff, {h, w_gu, w_down, y, out})) {
     SM_T(f32, (launch_moe_rows<T, MR_GLU>((const T*)h, nullptr, idx, rows * top, rows * top, top, (const T*)w_gu, nullptr, W, ff, 0,
-                                          0, E, limit, silu, in_w, (T*)y, nullptr, st),
+                                          0, E, limit, 0.f, silu, in_w, (T*)y, nullptr, st),
                launch_moe_rows<T, MR_PLAIN>((const T*)y, nullptr, idx, rows * top, rows * top, top, (const T*)w_down, nullptr, ff,
-                                            W, 0, 0, E, 0.f, 0, nullptr, (T*)out, nullptr, st)));
+                                            W, 0, 0, E, 0.f, 0.f, 0, nullptr, (T*)out, nullptr, st)));
     return (int)hipGetLastError();
   }
   const int rpw = 16;
@@ -1087,6 +1087,25 @@ int edge_sm_moe_experts(const void* h, int W, const int* idx, int top, const voi
                                (const T*)h, W, idx, top, (const T*)w_gu, ff, limit, (T*)y, rpw, E, silu, in_w));
   SM_T(f32, hipLaunchKernelGGL(moe_down_kernel<T>, dim3(rows * top, (W + rpw - 1) / rpw), dim3(NT), (size_t)ff * 4, st,
                                (const T*)y, ff, idx, (const T*)w_down, W, (T*)out, rpw, E));
+  return (int)hipGetLastError();
+}
+
+// The same (clamped gated units) with a shared expert su [2 sff, W], sd [W, sff] in the same two launches, where moe_rows.h takes
+// the rows; out_sh [rows, W], scratch ys [rows, sff].  By themselves its three launches cost some 4.5 us each, whatever their
+// bytes (ops.seqmix.MOE_GLU_SHARED_MAX has both sides).  -2: not taken.
+int edge_sm_moe_experts_glu_shared(const void* h, int W, const int* idx, int top, const void* w_gu, const void* w_down, int ff,
+                                   float limit, const void* su, const void* sd, int sff, float limit_sh, void* y, void* ys,
+                                   void* out, void* out_sh, int rows, int E, int f32, hipStream_t st) {
+  if (rows == 0) return 0;
+  if (ff < 1 || sff < 1 || (size_t)W * 4 > 60 * 1024 || (size_t)ff * 4 > 60 * 1024 || (f32 && rows > 1) || ff % 8 != 0 ||
+      (long)rows * (top + 1) > MR_MAX_PAIRS ||
+      !moe_rows_ok(W, sff, {h, w_gu, w_down, su, sd, y, ys, out, out_sh}))
+    return -2;
+  const int routed = rows * top, pairs = routed + rows;
+  SM_T(f32, (launch_moe_rows<T, MR_GLU>((const T*)h, (const T*)h, idx, routed, pairs, top, (const T*)w_gu, (const T*)su, W, ff, W, sff,
+                                        E, limit, limit_sh, 0, nullptr, (T*)y, (T*)ys, st),
+             launch_moe_rows<T, MR_PLAIN>((const T*)y, (const T*)ys, idx, routed, pairs, top, (const T*)w_down, (const T*)sd, ff, W,
+                                          sff, W, E, 0.f, 0.f, 0, nullptr, (T*)out, (T*)out_sh, st)));
   return (int)hipGetLastError();
 }
 
@@ -1114,11 +1133,11 @@ int edge_sm_moe_experts_relu2(const void* h, int W, const int* idx, int top, con
   const int big = sff > ff ? sff : ff;
   if ((size_t)W * 4 > 60 * 1024 || (size_t)big * 4 > 60 * 1024) return -3;
   const int rpw = 16, routed = rows * top, pairs = routed + (sff > 0 ? rows : 0);
-  if ((!f32 || rows == 1) && ff % 8 == 0 && moe_rows_ok(W, sff, {h, w_up, w_down, su, sd, y, ys, out, out_sh})) {
+  if ((!f32 || rows == 1) && ff % 8 == 0 && pairs <= MR_MAX_PAIRS && moe_rows_ok(W, sff, {h, w_up, w_down, su, sd, y, ys, out, out_sh})) {
     SM_T(f32, (launch_moe_rows<T, MR_RELU2>((const T*)h, (const T*)h, idx, routed, pairs, top, (const T*)w_up, (const T*)su, W, ff,
-                                            W, sff, E, 0.f, 0, nullptr, (T*)y, (T*)ys, st),
+                                            W, sff, E, 0.f, 0.f, 0, nullptr, (T*)y, (T*)ys, st),
                launch_moe_rows<T, MR_PLAIN>((const T*)y, (const T*)ys, idx, routed, pairs, top, (const T*)w_down, (const T*)sd, ff,
-                                            W, sff, W, E, 0.f, 0, nullptr, (T*)out, (T*)out_sh, st)));
+                                            W, sff, W, E, 0.f, 0.f, 0, nullptr, (T*)out, (T*)out_sh, st)));
     return (int)hipGetLastError();
   }
   SM_T(f32, hipLaunchKernelGGL((relu2_experts_kernel<T, true>), dim3(pairs, (big + rpw - 1) / rpw), dim3(NT), (size_t)W * 4, st,

@@ -54,3 +54,26 @@ def test_decode_sized_experts(dt, name, W, ff, act):
         sh = y @ f(sd).t()
         assert torch.equal(o.float().cpu(), got)
         assert ((o_sh.float().cpu() - sh).abs() <= eps * (sh.abs() + f(sd).abs().sum(1) * y.amax(-1, keepdim=True)) + 1e-6).all()
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("W,ff,sff", [(8, 8, 16), (1032, 24, 1048), (512, 1032, 8), (64, 512, 72)])
+@pytest.mark.parametrize("T", [1, 3, 4, 5, 8, 12])
+def test_clamped_shared_expert(dt, T, W, ff, sff):
+    """The shared expert beside the routed ones: the routed results keep their bits, its own are those of a float64 product."""
+    g = torch.Generator().manual_seed(T + W + sff)
+    r = lambda *s: (torch.randn(*s, generator=g) * 0.3).to(dt)
+    h, w_gu, w_down, su, sd = r(T, W), r(6, 2 * ff, W), r(6, W, ff), r(2 * sff, W), r(W, sff)
+    idx = torch.randint(0, 6, (T, 2), generator=g, dtype=torch.int32)
+    D = lambda x: x.cuda()
+    both = S.moe_experts_glu_shared(D(h), D(idx), D(w_gu), D(w_down), 1.5, D(su), D(sd), 0.8)
+    if dt == torch.float32 and T > 1:
+        assert both is None
+        return
+    assert torch.equal(both[0], S.moe_experts(D(h), D(idx), D(w_gu), D(w_down), 1.5))
+    y = S.glu_clamp(h.double() @ su.double().t(), sff, 0.8)
+    ref = y @ sd.double().t()
+    eps = 2.0 ** -8 if dt == torch.bfloat16 else 2.0 ** -20    # one rounding of the inner row and one of the result
+    bound = eps * (ref.abs() + sd.double().abs().sum(1) * y.abs().amax(-1, keepdim=True)) + 1e-6
+    assert ((both[1].cpu().double() - ref).abs() <= bound).all()
+    assert S.moe_experts_glu_shared(D(h.repeat(13, 1)), D(idx.repeat(13, 1)), D(w_gu), D(w_down), 1.5, D(su), D(sd), 0.8) is None
