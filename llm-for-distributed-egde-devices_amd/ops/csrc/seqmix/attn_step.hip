@@ -1,0 +1,359 @@
+// Windowed attention with pooled blocks over a paged cache for steps of few queries (decode steps): attn_kernel's rule
+// (seqmix.hip) of what a query sees and how its scores are formed, fp32 or bf16 rows.
+//
+// Bound by latency: a handful of queries, each over some hundred keys that lie in caches, so what counts is the length of the
+// chain of dependent loads.  attn_kernel lets one thread walk a whole key row, 16 bytes a trip.  Here a wave owns 16 keys at a time:
+// four lanes hold a key's row (all of it in flight at once, and the 16 value rows beside it), the scores of the SH heads come from
+// the matrix cores (bf16 rows 16x16x32, fp32 rows 16x16x4; the heads are repeated over the 16 rows, so that every group of 16
+// lanes holds all of them), and each wave keeps its own running maximum, sum and weighted values, fp32 and without a barrier;
+// the waves meet once, in LDS, at the end.  A workgroup's time is its vector instructions then (some 1.5 us for 128 keys and four
+// heads, 0.7 for one), so few queries run one head a workgroup; reading the next rows ahead took registers and gained nothing, and
+// an unrolled end cost 30 KB of code that every launch has to fetch (6.0 -> 18 us).
+// us, attn_kernel with its sum over key splits / this (bf16 but for the first): fp32, 16 heads of 64 in 4 groups, 2 tokens behind
+// 777 (window 512, 16 blocks) 15.3 / 9.9; latent rows of 160, 16 heads, 4 tokens behind 97 19.4 / 5.2; of 320, 6 behind 1100 (window 1024)
+// 35.1 / 27.0, 1 behind 7600 56 / 21; 16 heads of 128 in 4 groups, 6 in chunks of 1000 20.7 / 13.3.
+#include "common.h"
+#include "seqmix/seqmix_common.h"
+
+namespace {
+
+__device__ __forceinline__ float row16_max(float v) {
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xF, 0xF, false)));
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xF, 0xF, false)));
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xF, 0xF, false)));
+  v = fmaxf(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xF, 0xF, false)));
+  return v;
+}
+
+struct StepArgs {
+  const void *q, *gate, *kp, *vp;
+  const float *kb, *vb;
+  const int *tok_seq, *tok_pos, *seq_slot, *ptab;
+  void* out;
+  float* part;
+  const float *slopes, *sink, *rel;
+  int rows, gate_ld, ptab_ld, H, G, D, Dv, page, page_sh, PB, window, pool_sh, nsp, nsplit, kld, vld, chunked, gate_elem, keep_first, rel_n, out_ld;
+  float scale, cap, out_scale;
+};
+
+// 16 keys' rows of one wave: lane (key = lane & 15, 16-byte parts 4 c + (lane >> 4) of its row) and values (LPK lanes a key)
+template <typename KT, int NC, int DVL>
+struct Tile {
+  static constexpr int Q = sizeof(KT) / 2, VP = 2 * DVL;
+  uint4 k[NC][Q], v[VP][Q];
+};
+
+template <typename KT, int NC, int DVL>
+__device__ __forceinline__ void tile_load(Tile<KT, NC, DVL>& t, const KT* kb, const KT* vb, int row, int kld, int vld, int D, int Dv) {
+  constexpr int LPK = 8 * DVL, KPR = 64 / LPK;
+  const int lane = threadIdx.x & 63, grp = lane >> 4, dp = min(lane % LPK * 8, Dv - 8);
+  const KT* kr = kb + (size_t)row * kld;
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int q = 0; q < Tile<KT, NC, DVL>::Q; ++q) t.k[c][q] = reinterpret_cast<const uint4*>(kr + min(32 * c + 8 * grp, D - 8))[q];
+#pragma unroll
+  for (int p = 0; p < Tile<KT, NC, DVL>::VP; ++p) {
+    const KT* vr = vb + (size_t)__shfl(row, p * KPR + lane / LPK, 64) * vld + dp;
+#pragma unroll
+    for (int q = 0; q < Tile<KT, NC, DVL>::Q; ++q) t.v[p][q] = reinterpret_cast<const uint4*>(vr)[q];
+  }
+}
+
+// halves the V numbers of a lane between partners S apart, down to partners S0 apart; off: the first number it is left with
+template <int V, int S, int S0, int N>
+__device__ __forceinline__ void halve(float (&v)[N], int& off, int lane) {
+  if constexpr (S >= S0) {
+    const bool hi = lane & S;
+#pragma unroll
+    for (int j = 0; j < V / 2; ++j) {
+      const float give = hi ? v[j] : v[j + V / 2], keep = hi ? v[j + V / 2] : v[j];
+      v[j] = keep + __shfl_xor(give, S, 64);
+    }
+    off += hi ? V / 2 : 0;
+    halve<V / 2, S / 2, S0>(v, off, lane);
+  }
+}
+
+constexpr int STEP_NW = 8;                                  // waves of a workgroup
+
+// e^x for x <= 0 (or NaN) to about one rounding: x log2(e) in two parts, the small one to first order
+__device__ __forceinline__ float exp_neg(float x) {
+  constexpr float L = 1.44269502e+00f, L2 = 1.92596299e-08f, LN2 = 6.93147182e-01f;     // log2(e) = L + L2
+  x = x < -200.f ? -200.f : x;
+  const float t = x * L, lo = fmaf(x, L2, fmaf(x, L, -t)), p = ex2(t);
+  return fmaf(p * lo, LN2, p);
+}
+
+template <typename T, int NC, int DVL, int SH, bool POOL>
+__global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
+  constexpr int NW = STEP_NW, LPK = 8 * DVL, KPR = 64 / LPK, VP = 2 * DVL, RK = 16 * NW, DR = 64 * DVL;
+  __shared__ __attribute__((aligned(16))) float p_s[NW][16][SH];
+  __shared__ __attribute__((aligned(16))) float red[NW][SH][DR];
+  __shared__ float m_s[NW][SH], l_s[NW][SH], tot_s[2][SH];
+  // consecutive workgroups go to the eight dies in turn: those of one (token, kv head, part of its keys) stay on one die, where they
+  // read the same rows
+  const int unit = blockIdx.x % 8 + 8 * (blockIdx.x / 8 / a.nsp), sub = blockIdx.x / 8 % a.nsp;
+  if (unit >= a.rows * a.G * a.nsplit) return;
+  const int z = unit % a.nsplit, g = unit / a.nsplit % a.G, t = unit / a.nsplit / a.G, r0 = sub * SH, D = a.D, Dv = a.Dv;
+  const int R = min(SH, a.H / a.G - r0), hq0 = g * (a.H / a.G) + r0;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int key = lane & 15, grp = lane >> 4;
+  const int i = a.tok_pos[t];
+  const int* pt = a.ptab + (size_t)a.seq_slot[a.tok_seq[t]] * a.ptab_ld;
+  // the queries as the matrix cores' rows: row = lane & 15 is head row % SH; numbers past D (or heads past R) are zero
+  const T* qp = reinterpret_cast<const T*>(a.q) + ((size_t)t * a.H + hq0 + min(key % SH, R - 1)) * D;
+  uint4 qr[NC][Tile<T, NC, DVL>::Q];
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int e = 0; e < Tile<T, NC, DVL>::Q; ++e) {
+      const int d = 32 * c + 8 * grp;
+      qr[c][e] = reinterpret_cast<const uint4*>(qp + min(d, D - 8))[e];
+      if (d >= D || (key % SH) >= R) qr[c][e] = uint4{0u, 0u, 0u, 0u};
+    }
+  float m[SH], l[SH], acc[SH * 8];
+#pragma unroll
+  for (int r = 0; r < SH; ++r) { m[r] = -INFINITY; l[r] = 0.f; }
+#pragma unroll
+  for (int e = 0; e < SH * 8; ++e) acc[e] = 0.f;
+  const int win = a.window;
+  const int jlo = win > 0 ? (a.chunked ? i - i % win : max(0, i - win + 1)) : 0;
+  const int kf = !a.chunked && win > 0 ? min(a.keep_first, jlo) : 0;
+  const int nk = kf + i - jlo + 1;                           // tokens this query sees, the kept first ones in front
+  const int nb = POOL && i - win + 1 > 0 ? (i - win + 1) >> a.pool_sh : 0;
+  const int rounds_k = (nk + RK - 1) / RK, rounds = rounds_k + (nb + RK - 1) / RK;
+  int first = 0, last = rounds;
+  if (a.nsplit > 1) {
+    const int per = (rounds + a.nsplit - 1) / a.nsplit;
+    first = z * per;
+    last = min(rounds, first + per);
+  }
+
+  // rounds [b, e) over n keys; row(x) the cached row of key x
+  auto walk = [&](auto kt, const auto* kbase, const auto* vbase, int kld, int vld, int n, int b, int e, auto&& row, auto&& shape) {
+    using KT = decltype(kt);
+    using TL = Tile<KT, NC, DVL>;
+    const int end = min(n, e * RK);
+    int x0 = b * RK + wave * 16;
+    if (x0 >= end) return;
+    auto row_of = [&](int x) { return row(min(x + key, n - 1)); };
+    int rw = row_of(x0);
+#pragma unroll 1
+    for (; x0 < end; x0 += RK) {
+      TL tl;
+      tile_load<KT, NC, DVL>(tl, kbase, vbase, rw, kld, vld, D, Dv);
+      rw = row_of(x0 + RK);                                  // (past the end: the last key's, not used)
+      v4f s2[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};     // (two sums: half the chain)
+#pragma unroll
+      for (int c = 0; c < NC; ++c) {
+        v4f& s = s2[c & 1];
+        const bool in = 32 * c + 8 * grp < D;
+        if constexpr (TL::Q == 1) {
+          uint4 kv = tl.k[c][0];
+          if (!in) kv = uint4{0u, 0u, 0u, 0u};
+          s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8s, qr[c][0]), __builtin_bit_cast(v8s, kv), s, 0, 0, 0);
+        } else {
+          float qf[8], kf8[8];
+          load8<T>(reinterpret_cast<const T*>(&qr[c][0]), qf);
+          load8<float>(reinterpret_cast<const float*>(&tl.k[c][0]), kf8);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) s = mfma4(qf[j], in ? kf8[j] : 0.f, s);
+        }
+      }
+      v4f s = (s2[0] + s2[1]) * a.scale;
+      shape(s, x0 + key);                                    // (s[r], r < SH: head r's score of this lane's key)
+      const bool ok = x0 + key < n;
+      float p[SH], mn[SH];
+      bool grows = false;
+#pragma unroll
+      for (int r = 0; r < SH; ++r) {
+        if (!ok) s[r] = -INFINITY;
+        mn[r] = fmaxf(m[r], row16_max(s[r]));
+        grows |= mn[r] != m[r];
+      }
+      if (__builtin_amdgcn_readfirstlane(grows)) {           // (every lane holds the same maxima)
+#pragma unroll
+        for (int r = 0; r < SH; ++r) {
+          const float al = m[r] == -INFINITY ? 0.f : exp_neg(m[r] - mn[r]);
+          l[r] *= al;
+          m[r] = mn[r];
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[r * 8 + j] *= al;
+        }
+      }
+#pragma unroll
+      for (int r = 0; r < SH; ++r) {
+        p[r] = exp_neg(s[r] - (mn[r] == -INFINITY ? 0.f : mn[r]));
+        l[r] += row16_sum(p[r]);
+      }
+      if (grp == 0) {
+        if constexpr (SH == 4) *reinterpret_cast<float4*>(&p_s[wave][key][0]) = make_float4(p[0], p[1], p[2], p[3]);
+        else p_s[wave][key][0] = p[0];
+      }
+      __builtin_amdgcn_wave_barrier();                       // (a wave's own LDS accesses stay in order)
+      const bool full = x0 + 16 <= n;
+#pragma unroll
+      for (int ps = 0; ps < VP; ++ps) {
+        const int kx = ps * KPR + lane / LPK;
+        float w[SH], vf[8];
+        if constexpr (SH == 4) {
+          const float4 w4 = *reinterpret_cast<const float4*>(&p_s[wave][kx][0]);
+          w[0] = w4.x; w[1] = w4.y; w[2] = w4.z; w[3] = w4.w;
+        } else w[0] = p_s[wave][kx][0];
+        load8<KT>(reinterpret_cast<const KT*>(&tl.v[ps][0]), vf);
+        if (!full && x0 + kx >= n) {                         // a key past the end: its weight is 0, its row some other key's
+#pragma unroll
+          for (int j = 0; j < 8; ++j) vf[j] = 0.f;
+        }
+#pragma unroll
+        for (int r = 0; r < SH; ++r)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) acc[r * 8 + j] += w[r] * vf[j];
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+  };
+  auto token = [&](int x) { return x < kf ? x : jlo + x - kf; };
+  walk(T{}, reinterpret_cast<const T*>(a.kp) + g * D, reinterpret_cast<const T*>(a.vp) + g * Dv, a.kld, a.vld, nk, first,
+       min(last, rounds_k), [&](int x) { const int j = token(x); return (pt[j >> a.page_sh] << a.page_sh) + (j & (a.page - 1)); },
+       [&](v4f& s, int x) {
+         if (a.cap > 0.f || a.slopes || a.rel) {             // uniform: nothing of this for plain scores
+           const int dist = i - token(x);
+#pragma unroll
+           for (int r = 0; r < SH; ++r) {
+             const int h = hq0 + min(r, R - 1);
+             if (a.cap > 0.f) s[r] = a.cap * tanhf(s[r] / a.cap);
+             if (a.slopes) s[r] -= a.slopes[h] * (float)dist;
+             if (a.rel) s[r] += a.rel[(size_t)h * a.rel_n + min(max(dist, 0), a.rel_n - 1)];
+           }
+         }
+       });
+  if constexpr (POOL)
+    walk(float{}, a.kb + g * D, a.vb + g * Dv, a.G * D, a.G * Dv, nb, max(first - rounds_k, 0), last - rounds_k,
+         [&](int x) {
+           const int p0 = x << a.pool_sh;
+           return pt[p0 >> a.page_sh] * a.PB + ((p0 & (a.page - 1)) >> a.pool_sh);
+         },
+         [&](v4f&, int) {});
+
+  // add up the lanes that walked different keys, then the waves
+  int off = 0;
+  halve<SH * 8, 32, LPK>(acc, off, lane);
+  constexpr int VN = SH * 8 / KPR;                           // numbers a lane is left with, from off on
+  const int d0 = lane % LPK * 8;
+#pragma unroll
+  for (int j = 0; j < VN; ++j) red[wave][(off + j) / 8][d0 + (off + j) % 8] = acc[j];
+  if (lane == 0) {
+#pragma unroll
+    for (int r = 0; r < SH; ++r) { m_s[wave][r] = m[r]; l_s[wave][r] = l[r]; }
+  }
+  __syncthreads();
+  if (wave == 0) {                                           // lane = (wave, head): the waves' weights
+    const int w = min(lane / SH, NW - 1), r = lane % SH;
+    const bool sk = a.sink && z == 0;
+    const float sv = sk ? a.sink[hq0 + min(r, R - 1)] : -INFINITY, mw = m_s[w][r];
+    float M = fmaxf(mw, sv);
+#pragma unroll
+    for (int o = SH; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+    const float x = mw == -INFINITY ? 0.f : exp_neg(mw - M);
+    float ls = lane < NW * SH ? x * l_s[w][r] : 0.f;
+#pragma unroll
+    for (int o = SH; o < 64; o <<= 1) ls += __shfl_xor(ls, o, 64);
+    if (sk) ls += exp_neg(sv - M);
+    if (lane < NW * SH) m_s[w][r] = x;
+    if (lane < SH) { tot_s[0][r] = M; tot_s[1][r] = ls; }
+  }
+  __syncthreads();
+  const int d = tid % DR;
+#pragma unroll 1
+  for (int r = tid / DR; r < R; r += NW / DVL) {
+    float o = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) o += m_s[w][r] * red[w][r][d];
+    if (d >= Dv) continue;
+    if (a.nsplit > 1) {                                      // unnormalised sums, maximum and sum per head (attn_merge_kernel's rows)
+      float* dst = a.part + (((size_t)t * a.G * a.nsp + g * a.nsp + sub) * a.nsplit + z) * (SH * (Dv + 2));
+      dst[r * Dv + d] = o;
+      if (d == 0) { dst[SH * Dv + r] = tot_s[0][r]; dst[SH * Dv + SH + r] = tot_s[1][r]; }
+    } else {
+      const int h = hq0 + r;
+      float y = o / tot_s[1][r];
+      if (a.gate) y *= sigmoidf_(ldf<T>(reinterpret_cast<const T*>(a.gate) + (size_t)t * a.gate_ld + (a.gate_elem ? h * Dv + d : h)));
+      stf<T>(reinterpret_cast<T*>(a.out) + (size_t)t * a.out_ld + h * Dv + d, y * a.out_scale);
+    }
+  }
+}
+
+template <typename T, int SH>
+int run_step(const StepArgs& a, hipStream_t st) {
+  const dim3 grid((a.rows * a.G * a.nsplit + 7) / 8 * 8 * a.nsp), block(STEP_NW * 64);
+  const bool pool = a.pool_sh >= 0;
+#define STEP(NC, DL, P) hipLaunchKernelGGL((attn_step_kernel<T, NC, DL, SH, P>), grid, block, 0, st, a)
+  if (a.D <= 64 && a.Dv <= 64) { if (pool) STEP(2, 1, true); else STEP(2, 1, false); }
+  else if (a.D <= 128 && a.Dv <= 128) { if (pool) STEP(4, 2, true); else STEP(4, 2, false); }
+  else if (pool) return -2;
+  else if (a.D <= 192 && a.Dv <= 128) STEP(6, 2, false);
+  else STEP(10, 4, false);
+#undef STEP
+  return (int)hipGetLastError();
+}
+
+}  // namespace
+
+extern "C" int edge_sm_attn_merge(const float* part, const void* gate, int gate_ld, void* out, int rows, int H, int G, int Dv, int nsp,
+                                  int nsplit, int rmax, int gate_elem, int out_ld, float out_scale, int f32, hipStream_t st);
+
+extern "C" {
+
+// query heads of a workgroup in the low bits, workgroups that share one query's keys (vis: the most a query may see) above; 0: the
+// step is not this kernel's.
+int edge_sm_attention_step_plan(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis,
+                                int f32, uintptr_t addresses) {
+  if (rows < 1 || G < 1 || H % G || D < 8 || Dv < 8 || D > 320 || Dv > 256 || D % 8 || Dv % 8 || kld % 8 || vld % 8 || addresses % 16 ||
+      page < 1 || (page & (page - 1)) || pool < 0 || (pool & (pool - 1)) || pool > page || (pool > 0 && (D > 128 || Dv > 128)))
+    return 0;
+  // One head a workgroup while that leaves no CU more than one, four (one reading of the keys, one product for their scores) for more
+  // queries; not for one or two heads a kv head, of which three or two places would stay empty, nor for long fp32 rows, whose
+  // products on the matrix cores cost more than attn_kernel's.  us, attn_kernel / one / four: fp32, 16 heads of 64 in 4 groups, 16
+  // tokens behind 100 14.2 / 6.0 / 7.2, 1024 behind 300 174 / 364 / 149; bf16 of 128, 16 behind 300 24.2 / 8.4 / 10.4, 128 behind 300 43.5 /
+  // 39.7 / 24.0; fp32 rows of 160, 4 behind 900 21.2 / 22.6 / 32, 200 behind 200 46.7 / 142 / 69
+  const int sh = (long)rows * H <= 256 ? 1 : 4;
+  if (sh == 4 && (H / G < 3 || (f32 && D > 128))) return 0;
+  const long groups = (long)rows * G * ((H / G + sh - 1) / sh);
+  // Keys are split where one workgroup would walk more than 1536 (512 of long fp32 rows): the sum over the splits is a launch more,
+  // which a captured step pays however short its sequences are.  us, 6 tokens behind 1100, window 1024 and 34 blocks, whole / split:
+  // 14.3 / 17.9, 2 behind 300 6.6 / 8.9; without a window, 2 behind 8000, 44 (attn_kernel) / 22.6
+  const long each = f32 && D > 128 ? 512 : 1536, want = vis <= each ? 1 : (vis + 511) / 512, room = groups >= 1024 ? 1 : 1024 / groups;
+  return sh + 8 * (int)(want < room ? (want < 16 ? want : 16) : (room < 16 ? room : 16));
+}
+
+size_t edge_sm_attention_step_floats(int rows, int H, int G, int Dv, int plan) {
+  const int sh = plan % 8, nsplit = plan / 8;
+  return nsplit > 1 ? (size_t)rows * G * ((H / G + sh - 1) / sh) * nsplit * sh * (Dv + 2) : 0;
+}
+
+// plan as edge_sm_attention_step_plan says, part edge_sm_attention_step_floats numbers; the rest as edge_sm_attention's
+int edge_sm_attention_step(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb,
+                           const float* vb, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
+                           int ptab_ld, void* out, int rows, int H, int G, int D, int Dv, int page, int PB, float scale,
+                           int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
+                           const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
+                           int out_ld, float out_scale, hipStream_t st) {
+  if (rows == 0) return 0;
+  const int sh = plan % 8, nsplit = plan / 8;
+  if (G <= 0 || H % G || (chunked && pool > 0) || keep_first < 0 || (rel && (rel_n < 1 || pool > 0)) || out_ld < H * Dv ||
+      (sh != 1 && sh != 4) || nsplit < 1 || nsplit > 16 || (nsplit > 1 && !part) || D > 320 || Dv > 256 || page < 1 ||
+      (page & (page - 1)) || (pool & (pool - 1)))
+    return -2;
+  const int nsp = (H / G + sh - 1) / sh, page_sh = __builtin_ctz(page), pool_sh = window > 0 && pool > 0 ? __builtin_ctz(pool) : -1;
+  const StepArgs a{q, gate, kp, vp, kb, vb, tok_seq, tok_pos, seq_slot, ptab, out, part, slopes, sink, rel, rows, gate_ld, ptab_ld, H, G, D,
+                   Dv, page, page_sh, PB, window, pool_sh, nsp, nsplit, kld, vld, chunked, gate_elem, keep_first, rel_n, out_ld, scale,
+                   cap, out_scale};
+  const int r = sh == 1 ? (f32 ? run_step<float, 1>(a, st) : run_step<bf16_t, 1>(a, st))
+                        : (f32 ? run_step<float, 4>(a, st) : run_step<bf16_t, 4>(a, st));
+  if (r != 0 || nsplit == 1) return r;
+  return edge_sm_attn_merge(part, gate, gate_ld, out, rows, H, G, Dv, nsp, nsplit, sh, gate_elem, out_ld, out_scale, f32, st);
+}
+
+}  // extern "C"

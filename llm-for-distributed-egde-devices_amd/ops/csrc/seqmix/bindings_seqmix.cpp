@@ -37,6 +37,15 @@ int edge_sm_attention(const void* q, const void* gate, int gate_ld, const void* 
                       int window, int pool, int f32, int nsplit, float* part, int kld, int vld, int chunked, float cap,
                       const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
                       int out_ld, float out_scale, hipStream_t st);
+int edge_sm_attention_step_plan(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis,
+                                int f32, uintptr_t addresses);
+size_t edge_sm_attention_step_floats(int rows, int H, int G, int Dv, int plan);
+int edge_sm_attention_step(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb,
+                           const float* vb, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
+                           int ptab_ld, void* out, int rows, int H, int G, int D, int Dv, int page, int PB, float scale,
+                           int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
+                           const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
+                           int out_ld, float out_scale, hipStream_t st);
 int edge_sm_attention_splits(int rows, int G, int chunks);
 size_t edge_sm_attention_part_floats(int rows, int H, int G, int D, int Dv, int nsplit);
 int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp,
@@ -399,23 +408,25 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
       return out;
     }
   }
-  // few queries over many keys (decode steps): split every query's keys over several workgroups
-  int nsplit = 1;
-  {
-    const int64_t vis = (window > 0 ? std::min<int64_t>(window + keep_first, max_keys) : max_keys) + (PB ? max_keys / pool : 0);
-    nsplit = edge_sm_attention_splits((int)T, (int)G, (int)((vis + 255) / 256));
-  }
+  const int64_t vis = (window > 0 ? std::min<int64_t>(window + keep_first, max_keys) : max_keys) + (PB ? max_keys / pool : 0);
+  const uintptr_t addresses = (uintptr_t)q.data_ptr() | (uintptr_t)kp.data_ptr() | (uintptr_t)vp.data_ptr() |
+                              (uintptr_t)(PB ? kb->data_ptr<float>() : nullptr) | (uintptr_t)(PB ? vb->data_ptr<float>() : nullptr);
+  // few queries over many keys (decode steps): several workgroups may share a query's keys
+  int plan = edge_sm_attention_step_plan((int)T, (int)H, (int)G, (int)D, (int)Dv, (int)kld, (int)vld, (int)page,
+                                         PB ? (int)pool : 0, vis, f32(q), addresses);
+  const bool step = plan > 0;
+  if (!step) plan = edge_sm_attention_splits((int)T, (int)G, (int)((vis + 255) / 256));
+  const int64_t floats = step ? edge_sm_attention_step_floats((int)T, (int)H, (int)G, (int)Dv, plan)
+                              : plan > 1 ? edge_sm_attention_part_floats((int)T, (int)H, (int)G, (int)D, (int)Dv, plan) : 0;
   at::Tensor part;
-  if (nsplit > 1)
-    part = at::empty({(int64_t)edge_sm_attention_part_floats((int)T, (int)H, (int)G, (int)D, (int)Dv, nsplit)},
-                     q.options().dtype(at::kFloat));
-  check(edge_sm_attention(q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(), vp.data_ptr(),
-                          PB ? kb->data_ptr<float>() : nullptr, PB ? vb->data_ptr<float>() : nullptr,
-                          tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(),
-                          ptab.data_ptr<int>(), (int)ptab.stride(0), out.data_ptr(), (int)T, (int)H, (int)G, (int)D, (int)Dv,
-                          (int)page, PB, (float)scale, (int)window, PB ? (int)pool : 0, f32(q), nsplit,
-                          nsplit > 1 ? part.data_ptr<float>() : nullptr, (int)kld, (int)vld, chunked ? 1 : 0, (float)softcap,
-                          slopes_p, sink_p, gate_elem, (int)keep_first, rel_p, rel_n, out_ld, (float)out_scale, stream()),
+  if (floats) part = at::empty({floats}, q.options().dtype(at::kFloat));
+  const auto run = step ? edge_sm_attention_step : edge_sm_attention;
+  check(run(q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(), vp.data_ptr(),
+            PB ? kb->data_ptr<float>() : nullptr, PB ? vb->data_ptr<float>() : nullptr, tok_seq.data_ptr<int>(),
+            tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(), ptab.data_ptr<int>(), (int)ptab.stride(0), out.data_ptr(), (int)T,
+            (int)H, (int)G, (int)D, (int)Dv, (int)page, PB, (float)scale, (int)window, PB ? (int)pool : 0, f32(q), plan,
+            floats ? part.data_ptr<float>() : nullptr, (int)kld, (int)vld, chunked ? 1 : 0, (float)softcap, slopes_p, sink_p,
+            gate_elem, (int)keep_first, rel_p, rel_n, out_ld, (float)out_scale, stream()),
         "sm_attention");
   return out;
 }

@@ -995,6 +995,13 @@ size_t edge_sm_attention_part_floats(int rows, int H, int G, int D, int Dv, int 
   return (size_t)rows * G * nsp * nsplit * rmax * (Dv + 2);
 }
 
+int edge_sm_attn_merge(const float* part, const void* gate, int gate_ld, void* out, int rows, int H, int G, int Dv, int nsp,
+                       int nsplit, int rmax, int gate_elem, int out_ld, float out_scale, int f32, hipStream_t st) {
+  SM_T(f32, hipLaunchKernelGGL(attn_merge_kernel<T>, dim3(rows, G * nsp), dim3(NT), 0, st, part, (const T*)gate, gate_ld, (T*)out, H,
+                               G, Dv, nsp, nsplit, rmax, gate_elem, out_ld, out_scale));
+  return (int)hipGetLastError();
+}
+
 int edge_sm_attention(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb,
                       const float* vb, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
                       int ptab_ld, void* out, int rows, int H, int G, int D, int Dv, int page, int PB, float scale,
@@ -1037,8 +1044,7 @@ int edge_sm_attention(const void* q, const void* gate, int gate_ld, const void* 
 #undef SM_ATT
 #undef SM_ATT_V
   if (nsplit > 1)
-    SM_T(f32, hipLaunchKernelGGL(attn_merge_kernel<T>, dim3(rows, G * nsp), dim3(NT), 0, st, part, (const T*)gate, gate_ld,
-                                 (T*)out, H, G, Dv, nsp, nsplit, rmax, gate_elem, out_ld, out_scale));
+    return edge_sm_attn_merge(part, gate, gate_ld, out, rows, H, G, Dv, nsp, nsplit, rmax, gate_elem, out_ld, out_scale, f32, st);
   return (int)hipGetLastError();
 }
 
