@@ -798,6 +798,143 @@ __global__ void __launch_bounds__(64) route_grouped_kernel(const float* __restri
   if (gate && lane == 0) gate_w[t] = sigmoidf_(zr[E]);
 }
 
+// Scores and choice of few tokens in one launch, a workgroup a token: 16 waves form the scores of EPW experts each (moe_logits_kernel's
+// chain per lane), the first wave chooses with one expert a lane by moe_topk_kernel's rule (GROUPED: route_grouped_kernel's): a
+// maximum over lanes, then the lowest lane that holds it.  The two launches were each a chain of a few memory round trips.  Up to 512
+// tokens, which is two workgroups a CU, and three scores a wave: us, two launches / one, 16 experts of 1024, 4 tokens 6.8 / 4.0, 64
+// 6.9 / 4.1, 512 8.4 / 5.1; 32 of 2048 7.5 / 5.6, 7.8 / 5.8, 13.2 / 10.3; grouped with a gate, 16 of 1024 7.9 / 5.3, 8.5 / 5.5, 10.1 / 7.8, 32
+// of 2048 8.6 / 7.5, 9.3 / 7.8, 14.5 / 13.5; not 64 of 4096, 4 tokens 12.1 / 22.7.
+constexpr int RF_WAVES = 16, RF_SCORES = 48;
+struct RouteFew {
+  const float *router, *bias;                                // bias: GROUPED the correction of the choice
+  int W, E, gate, groups, keep, top, sigm;
+  float scale;
+  int* idx;
+  float *wts, *gate_w;
+};
+
+// what the whole wave holds most of among lanes with v > floor: its lowest lane, -1 for none
+__device__ __forceinline__ int best_lane(float v, float floor, float& best) {
+  const bool in = v > floor;
+  float m = in ? v : -INFINITY;
+  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0xB1, 0xF, 0xF, false)));
+  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x4E, 0xF, 0xF, false)));
+  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x124, 0xF, 0xF, false)));
+  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x128, 0xF, 0xF, false)));
+  auto row = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), l)); };
+  best = fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
+  return __ffsll((unsigned long long)__ballot(in && v == best)) - 1;
+}
+
+template <typename T, int EPW, bool GROUPED>
+__global__ void __launch_bounds__(RF_WAVES * 64) route_few_kernel(const T* __restrict__ h, RouteFew a) {
+  __shared__ float z_s[RF_SCORES], c_s[64], g_s[64];
+  const size_t t = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = a.E + a.gate;
+  const T* hr = h + t * a.W;
+  float acc[EPW];
+#pragma unroll
+  for (int k = 0; k < EPW; ++k) acc[k] = 0.f;
+#pragma unroll 4
+  for (int c = lane * 8; c < a.W; c += 64 * 8) {
+    float x[8];
+    load8<T>(hr + c, x);
+#pragma unroll
+    for (int k = 0; k < EPW; ++k) {
+      float r[8];
+      load8<float>(a.router + (size_t)min(wave + RF_WAVES * k, n - 1) * a.W + c, r);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) acc[k] += x[j] * r[j];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < EPW; ++k) {
+    const int e = wave + RF_WAVES * k;
+    const float s = wave_sum(acc[k]);
+    if (lane == 0 && e < n) z_s[e] = s + (!GROUPED && a.bias ? a.bias[e] : 0.f);
+  }
+  __syncthreads();
+  if (wave != 0) return;
+  const int E = a.E, top = a.top;
+  const bool live = lane < E;
+  const float z = live ? z_s[lane] : -INFINITY;
+  auto softmax = [&]() {
+    const float mx = wave_max(z), ex = live ? expf(z - mx) : 0.f;
+    return ex / wave_sum(ex);
+  };
+  float tot = 0.f, my_w = 0.f;
+  int my_i = 0;                                              // lane k keeps the k-th choice
+  if constexpr (GROUPED) {
+    const float s = softmax();
+    float c = live ? s + (a.bias ? a.bias[lane] : 0.f) : -INFINITY;
+    if (a.groups > 1) {
+      const int size = E / a.groups, g = min(lane / size, a.groups - 1);
+      c_s[lane] = c;
+      __builtin_amdgcn_wave_barrier();                       // (one wave: its LDS accesses keep their order)
+      float b = -INFINITY;
+      for (int e = g * size; e < (g + 1) * size; ++e) b = fmaxf(b, c_s[e]);
+      g_s[g] = b;
+      __builtin_amdgcn_wave_barrier();
+      int better = 0;
+      for (int o = 0; o < a.groups; ++o) better += g_s[o] > b || (g_s[o] == b && o < g);
+      if (better >= a.keep) c = -INFINITY;
+    }
+    for (int k = 0; k < top; ++k) {
+      float best;
+      int bi = best_lane(c, -INFINITY, best);
+      if (bi < 0) bi = k;                                    // scores that compare with nothing (NaN): keep the ids in range
+      const float w = __shfl(s, bi, 64);
+      if (lane == k) { my_w = w; my_i = bi; }
+      tot += w;
+      if (lane == bi) c = -INFINITY;
+    }
+    if (a.gate && lane == 0) a.gate_w[t] = sigmoidf_(z_s[E]);
+  } else {
+    float v = z;
+    if (!a.sigm) {                                           // (every lane takes part in its sums)
+      v = softmax();
+      if (!live) v = -2.f;
+    }
+    const float floor = a.sigm ? -INFINITY : -1.f, gone = a.sigm ? -INFINITY : -2.f;
+    for (int k = 0; k < top; ++k) {
+      float best;
+      int bi = best_lane(v, floor, best);
+      if (bi < 0) {
+        bi = k;
+        best = 0.f;
+      }
+      if (lane == k) { my_w = best; my_i = bi; }
+      if (lane == bi) v = gone;
+      tot += best;
+    }
+  }
+  float soft = 0.f;
+  if (!GROUPED && a.sigm == 2) {
+    const float ex = lane < top ? expf(my_w - __shfl(my_w, 0, 64)) : 0.f;
+    soft = ex / wave_sum(ex);
+  }
+  if (lane < top) {
+    a.idx[t * top + lane] = my_i;
+    a.wts[t * top + lane] = (!GROUPED && a.sigm == 2) ? soft * a.scale : (!GROUPED && a.sigm) ? sigmoidf_(my_w) * a.scale
+                                                                                             : my_w / (tot + 1e-20f) * a.scale;
+  }
+}
+
+// whether one launch takes the step
+inline bool route_few_ok(int rows, int W, int E, int gate) {
+  return rows <= 512 && E + gate <= RF_SCORES && W % 8 == 0 && W <= 2048;
+}
+
+template <typename T, bool GROUPED>
+void launch_route_few(const T* h, const RouteFew& a, int rows, hipStream_t st) {
+  const int n = (a.E + a.gate + RF_WAVES - 1) / RF_WAVES;
+#define RF(K) hipLaunchKernelGGL((route_few_kernel<T, K, GROUPED>), dim3(rows), dim3(RF_WAVES * 64), 0, st, h, a)
+  if (n == 1) RF(1);
+  else if (n == 2) RF(2);
+  else RF(3);
+#undef RF
+}
+
 // decode-sized steps: out row r of pair (token, choice) = act(gate_r . h, up_r . h); one wave per row at a time,
 // lanes stride the width with 8-element loads, the token's row sits in LDS as fp32.  silu: the activation is
 // silu(w gate) (w up) with w = in_w[pair] (null: 1), the unit of an input scaled by the router's weight.
@@ -1064,6 +1201,11 @@ int edge_sm_moe_route(const void* h, int W, const float* router, const float* bi
                       int* idx, float* wts, int rows, int sigm, int f32, hipStream_t st) {
   if (rows == 0) return 0;
   if (top < 1 || top > E || top > 64 || E > 8192) return -2;
+  if (route_few_ok(rows, W, E, 0)) {
+    const RouteFew a{router, bias, W, E, 0, 1, 1, top, sigm, scale, idx, wts, nullptr};
+    SM_T(f32, (launch_route_few<T, false>((const T*)h, a, rows, st)));
+    return (int)hipGetLastError();
+  }
   SM_T(f32, launch_moe_logits<T>((const T*)h, W, router, E, z, bias, rows, st));
   hipLaunchKernelGGL(moe_topk_kernel, dim3(rows), dim3(64), (size_t)E * 4, st, (const float*)z, E, top, scale, idx, wts, sigm);
   return (int)hipGetLastError();
@@ -1117,6 +1259,11 @@ int edge_sm_moe_route_grouped(const void* h, int W, const float* router, int E, 
   if (E < 1 || groups < 1 || E % groups || keep < 1 || keep > groups || top < 1 || top > 64 || top > E / groups * keep ||
       E > 4096 || (gate && !gate_w))
     return -2;
+  if (route_few_ok(rows, W, E, gate)) {
+    const RouteFew a{router, corr, W, E, gate, groups, keep, top, 0, scale, idx, wts, gate_w};
+    SM_T(f32, (launch_route_few<T, true>((const T*)h, a, rows, st)));
+    return (int)hipGetLastError();
+  }
   SM_T(f32, launch_moe_logits<T>((const T*)h, W, router, E + gate, z, nullptr, rows, st));
   hipLaunchKernelGGL(route_grouped_kernel, dim3(rows), dim3(64), (size_t)(2 * E + groups) * 4, st, (const float*)z, E, gate,
                      corr, groups, keep, top, scale, idx, wts, gate_w);
