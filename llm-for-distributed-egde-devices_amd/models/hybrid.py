@@ -59,6 +59,11 @@ from .mixers import (AttentionRetention, ChannelDeltaMixer, ChunkAttention, Deca
 from .moe import MoEFeedForward, MoEOut
 
 
+def _unwatched(m: nn.Module) -> bool:
+    """Nobody has asked to see or change this module's calls."""
+    return not (m._forward_hooks or m._forward_pre_hooks)
+
+
 class HybridLayer(nn.Module):
     def __init__(self, cfg: ModelConfig, spec: LayerSpec, idx: int, dtype, device):
         super().__init__()
@@ -72,11 +77,20 @@ class HybridLayer(nn.Module):
         self.proj_in = Linear(W, self.mix.in_rows + self.ff, False, dtype, device)
         self.down = Linear(self.ff, W, False, dtype, device) if self.ff else None
 
-    def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
-        h = self.norm1(x, self.proj_in.weight.dtype)
+    def first_read(self, run):
+        """What forms this layer's first input from the stream: the layer before may do it with its residual sum."""
+        return self.norm1 if _unwatched(self.norm1) else None
+
+    def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run, h: Optional[torch.Tensor] = None, nxt=None):
+        """``h``: this layer's first input when the layer before already formed it; ``nxt``: the next layer's ``first_read()``.
+        Returns x (updated in place), with ``nxt`` (x, the next layer's first input)."""
+        if h is None:
+            h = self.norm1(x, self.proj_in.weight.dtype)
         u = self.proj_in(h)
         m = self.down(seqmix.relu2(u, self.mix.in_rows, self.ff)) if self.ff else None
-        return self.mix(x, u, meta, run, m)
+        if nxt is None:
+            return self.mix(x, u, meta, run, m)
+        return x, self.mix(x, u, meta, run, m, nxt)
 
 
 class PostNormLayer(nn.Module):
@@ -102,15 +116,28 @@ class PostNormLayer(nn.Module):
             self.canon2 = P() if taps else None
             self.norm2 = RowLayerNorm(W, eps, device)
 
-    def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
-        h = seqmix.canon_conv(x, self.canon1, run.canon1, meta, self.dtype) if self.canon1 is not None else x.to(self.dtype)
-        self.norm1.add_to(x, self.mix(h, meta, run))
-        if self.ff is not None:
-            h = seqmix.canon_conv(x, self.canon2, run.canon2, meta, self.dtype) if self.canon2 is not None \
-                else x.to(self.dtype)
-            shared, parts, wts = self.ff(h)
-            self.norm2.add_to(x, shared, parts, wts)
-        return x
+    def first_read(self, run):
+        """What forms this layer's first input from the stream (``HybridLayer.first_read``): taps and their state."""
+        return (self.canon1, run.canon1) if self.canon1 is not None else None
+
+    def _join(self, norm, x, meta, nxt, y, parts=None, wts=None):
+        """x += the normed result; the next sublayer's convolved rows where ``nxt`` names its taps and state."""
+        if nxt is None:
+            norm.add_to(x, y, parts, wts)
+            return None
+        return seqmix.layer_norm_residual_canon(x, y, norm.weight, norm.bias, norm.eps, parts, wts, *nxt, meta, self.dtype)
+
+    def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run, h: Optional[torch.Tensor] = None, nxt=None):
+        """``h``, ``nxt`` and the result: as ``HybridLayer.forward``."""
+        if h is None:
+            h = seqmix.canon_conv(x, self.canon1, run.canon1, meta, self.dtype) if self.canon1 is not None else x.to(self.dtype)
+        last = self.ff is None
+        h2 = self._join(self.norm1, x, meta, nxt if last else (self.canon2, run.canon2) if self.canon2 is not None else None,
+                        self.mix(h, meta, run))
+        if not last:
+            shared, parts, wts = self.ff(x.to(self.dtype) if h2 is None else h2)
+            h2 = self._join(self.norm2, x, meta, nxt, shared, parts, wts)
+        return x if nxt is None else (x, h2)
 
 
 class SandwichLayer(nn.Module):
@@ -134,12 +161,27 @@ class SandwichLayer(nn.Module):
         if self.ff is not None:
             self.norm2, self.norm2b = N(), N()
 
-    def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
-        self.norm1b.add_to(x, self.mix(self.norm1(x, self.dtype), meta, run), self.mult)
-        if self.ff is not None:
-            shared, parts, wts = self.ff(self.norm2(x, self.dtype))
-            self.norm2b.add_to(x, shared, self.mult, parts, wts)
-        return x
+    def first_read(self, run):
+        """What forms this layer's first input from the stream (``HybridLayer.first_read``)."""
+        return self.norm1 if _unwatched(self.norm1) else None
+
+    def _join(self, norm, x, nxt, y, parts=None, wts=None):
+        """x += the normed result; the rows of the norm that reads x next, where one is given."""
+        if nxt is None:
+            norm.add_to(x, y, self.mult, parts, wts)
+            return None
+        return seqmix.group_norm_residual_norm(x, y, norm.weight, norm.groups, norm.eps, self.mult, parts, wts, nxt.weight, nxt.groups,
+                                               nxt.eps, self.dtype)
+
+    def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run, h: Optional[torch.Tensor] = None, nxt=None):
+        """``h``, ``nxt`` and the result: as ``HybridLayer.forward``."""
+        last = self.ff is None
+        inner = None if last or not _unwatched(self.norm2) else self.norm2
+        h = self._join(self.norm1b, x, nxt if last else inner, self.mix(self.norm1(x, self.dtype) if h is None else h, meta, run))
+        if not last:
+            shared, parts, wts = self.ff(self.norm2(x, self.dtype) if h is None else h)
+            h = self._join(self.norm2b, x, nxt, shared, parts, wts)
+        return x if nxt is None else (x, h)
 
 
 class StreamNorm(nn.Module):
@@ -369,6 +411,19 @@ class HybridLM(nn.Module):
         """The LayerSpec of every run, in order (sizes the paged cache)."""
         return [self.cfg.layer_specs[i] for i, _ in self.runs]
 
+    def _next_read(self, r: int, cache):
+        """``first_read()`` of run r + 1 where nothing comes between run r and it: both layers of one kind, nobody watching their
+        calls, no pass of a looped span that starts by changing the stream."""
+        if r + 1 >= len(self.runs):
+            return None
+        i, t = self.runs[r + 1]
+        loop, here, there = self.cfg.loop, self.layers[self.runs[r][0]], self.layers[i]
+        if t is not None and i == loop.start and (loop.entry == "project" or (loop.entry == "add_embed" and t > 0)):
+            return None
+        if type(here) is not type(there) or not (_unwatched(here) and _unwatched(there)):
+            return None
+        return there.first_read(cache.run(r + 1))
+
     def forward(self, ids: torch.Tensor, meta: seqmix.RaggedMeta, cache, rows: Optional[torch.Tensor] = None,
                 taps: Optional[list] = None) -> torch.Tensor:
         """ids [T] (flat step) -> fp32 logits of ``rows`` (flat row indices; None: every row).
@@ -399,8 +454,12 @@ class HybridLM(nn.Module):
             elif cfg.streams:                            # the next layer's read + norm rides on this layer's last rebuild
                 nxt = self.layers[self.runs[r + 1][0]].first_read() if r + 1 < len(self.runs) and cfg.loop is None else None
                 x, h_next = self.layers[i](x, meta, cache.run(r), h_next, nxt)
-            else:
-                x = self.layers[i](x, meta, cache.run(r))
+            else:                                        # the next layer's first input rides on this layer's residual sum
+                nxt = self._next_read(r, cache)
+                if nxt is None:
+                    x, h_next = self.layers[i](x, meta, cache.run(r), h_next), None
+                else:
+                    x, h_next = self.layers[i](x, meta, cache.run(r), h_next, nxt)
             if taps is not None:
                 taps.append(x.sum(1) if cfg.streams else x.clone())
         if rows is not None:

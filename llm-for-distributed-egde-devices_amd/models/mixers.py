@@ -114,10 +114,13 @@ class ParallelMixer(nn.Module):
     def in_rows(self) -> int:
         return sum(self.left.spec.proj_sizes) + self.right.spec.in_size
 
-    def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None):
-        """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra."""
+    def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None):
+        """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra.  ``nxt``: the norm that reads x next; its rows
+        (of u's dtype) come back in x's place."""
         a = self.left(u, 0, meta, run)
         r = self.right(u, sum(self.left.spec.proj_sizes), meta, run)
+        if nxt is not None:
+            return seqmix.combine_residual_norm(x, a, r, self.left_out, self.right_out, self.eps, extra, nxt.weight, nxt.eps, u.dtype)
         return seqmix.combine_residual(x, a, r, self.left_out, self.right_out, self.eps, extra)
 
 

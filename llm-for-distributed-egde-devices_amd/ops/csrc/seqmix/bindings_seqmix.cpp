@@ -21,6 +21,14 @@ int edge_sm_gated_norm(const float* y, const void* z, int z_ld, const float* w, 
 int edge_sm_rope_write(const void* proj, int ld, const int* tok_seq, const int* tok_pos, const int* seq_slot,
                        const int* ptab, int ptab_ld, const float* cs, void* q_out, void* kp, void* vp, int rows,
                        int H, int G, int D, int Dv, int rot, int page, int f32, hipStream_t st);
+int edge_sm_ln_residual_taps(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b,
+                             const float* cw, float* state, const int* tok_seq, const int* tok_pos, const int* seq_slot, void* out,
+                             int rows, int W, float eps, int f32, hipStream_t st);
+int edge_sm_group_residual_norm(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, int groups,
+                                float eps, float mult, const float* w2, int groups2, float eps2, void* out, int rows, int W, int f32,
+                                hipStream_t st);
+int edge_sm_combine_norm(float* x, const void* l, const void* r, const float* wl, const float* wr, const void* extra, float eps,
+                         const float* gain, float eps2, void* out, int rows, int W, int f32, hipStream_t st);
 int edge_sm_group_norm(const float* x, const float* w, void* y, int rows, int W, int groups, float eps, int f32,
                        hipStream_t st);
 int edge_sm_group_norm_residual(float* x, const void* y, const void* parts, const float* pw, int K, const float* w,
@@ -584,6 +592,101 @@ void sm_ln_residual(at::Tensor& x, const std::optional<at::Tensor>& y, const at:
   check(edge_sm_ln_residual(x.data_ptr<float>(), y ? y->data_ptr() : nullptr, parts ? parts->data_ptr() : nullptr,
                             parts ? part_w->data_ptr<float>() : nullptr, K, w.data_ptr<float>(), b.data_ptr<float>(), (int)T,
                             (int)W, (float)eps, is_f32, stream()), "sm_ln_residual");
+}
+
+// The residual sums with the next sublayer's row (residual_next.hip); nothing comes back, and nothing was done, where the row
+// does not fit.
+struct Results {
+  const void *y = nullptr, *parts = nullptr;
+  const float* pw = nullptr;
+  int K = 0, is_f32 = 0;
+};
+Results results_of(const at::Tensor& x, const std::optional<at::Tensor>& y, const std::optional<at::Tensor>& parts,
+                   const std::optional<at::Tensor>& part_w) {
+  const int64_t T = x.size(0), W = x.size(1);
+  TORCH_CHECK(y || parts, "nothing to norm");
+  Results r;
+  if (y) {
+    chk_act2(*y, "y");
+    TORCH_CHECK(y->size(0) == T && y->size(1) == W, "y: [T, W]");
+    r.is_f32 = f32(*y);
+    r.y = y->data_ptr();
+  }
+  if (parts) {
+    TORCH_CHECK(parts->is_cuda() && parts->is_contiguous() && is_act(*parts) && parts->dim() == 3 && parts->size(0) == T &&
+                    parts->size(2) == W && (!y || parts->scalar_type() == y->scalar_type()), "parts: [T, K, W]");
+    r.K = (int)parts->size(1);
+    r.is_f32 = f32(*parts);
+    r.parts = parts->data_ptr();
+    if (part_w) {
+      chk_f32(*part_w, "part_w");
+      TORCH_CHECK(part_w->numel() == T * r.K, "part_w: fp32 [T, K]");
+      r.pw = part_w->data_ptr<float>();
+    }
+  }
+  return r;
+}
+
+std::optional<at::Tensor> sm_ln_residual_taps(at::Tensor& x, const std::optional<at::Tensor>& y, const at::Tensor& w,
+                                              const at::Tensor& b, double eps, const std::optional<at::Tensor>& parts,
+                                              const std::optional<at::Tensor>& part_w, const at::Tensor& cw, at::Tensor& state,
+                                              const at::Tensor& tok_seq, const at::Tensor& tok_pos, const at::Tensor& seq_slot,
+                                              bool out_f32) {
+  for (const at::Tensor* f : {(const at::Tensor*)&x, &w, &b, &cw, (const at::Tensor*)&state}) chk_f32(*f, "x, weights, state");
+  for (const at::Tensor* t : {&tok_seq, &tok_pos, &seq_slot}) chk_i32(*t, "metadata");
+  const int64_t T = x.size(0), W = x.size(1);
+  TORCH_CHECK(x.dim() == 2 && w.numel() == W && b.numel() == W && cw.dim() == 2 && cw.size(0) == W, "x [T, W], weights [W], taps [W, n]");
+  TORCH_CHECK(tok_seq.numel() == T && tok_pos.numel() == T, "one token per sequence");
+  const Results r = results_of(x, y, parts, part_w);
+  if (cw.size(1) != 4 || (r.is_f32 != 0) != out_f32) return std::nullopt;
+  TORCH_CHECK(state.dim() == 3 && state.size(1) == 3 && state.size(2) == W, "state: fp32 [slots, 3, W]");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  auto out = at::empty({T, W}, x.options().dtype(act_type(out_f32)));
+  const int rc = edge_sm_ln_residual_taps(x.data_ptr<float>(), r.y, r.parts, r.pw, r.K, w.data_ptr<float>(), b.data_ptr<float>(),
+                                          cw.data_ptr<float>(), state.data_ptr<float>(), tok_seq.data_ptr<int>(),
+                                          tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(), out.data_ptr(), (int)T, (int)W,
+                                          (float)eps, r.is_f32, stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_ln_residual_taps");
+  return out;
+}
+
+std::optional<at::Tensor> sm_group_residual_norm(at::Tensor& x, const std::optional<at::Tensor>& y, const at::Tensor& w,
+                                                 int64_t groups, double eps, double mult, const std::optional<at::Tensor>& parts,
+                                                 const std::optional<at::Tensor>& part_w, const at::Tensor& w2, int64_t groups2,
+                                                 double eps2, bool out_f32) {
+  for (const at::Tensor* f : {(const at::Tensor*)&x, &w, &w2}) chk_f32(*f, "x, weights");
+  TORCH_CHECK(x.dim() == 2 && w.numel() == x.size(1) && w2.numel() == x.size(1), "x fp32 [T, W], weights [W]");
+  const Results r = results_of(x, y, parts, part_w);
+  if ((r.is_f32 != 0) != out_f32) return std::nullopt;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  auto out = at::empty({x.size(0), x.size(1)}, x.options().dtype(act_type(out_f32)));
+  const int rc = edge_sm_group_residual_norm(x.data_ptr<float>(), r.y, r.parts, r.pw, r.K, w.data_ptr<float>(), (int)groups,
+                                             (float)eps, (float)mult, w2.data_ptr<float>(), (int)groups2, (float)eps2,
+                                             out.data_ptr(), (int)x.size(0), (int)x.size(1), r.is_f32, stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_group_residual_norm");
+  return out;
+}
+
+std::optional<at::Tensor> sm_combine_norm(at::Tensor& x, const at::Tensor& l, const at::Tensor& r, const at::Tensor& wl,
+                                          const at::Tensor& wr, double eps, const std::optional<at::Tensor>& extra,
+                                          const at::Tensor& gain, double eps2, bool out_f32) {
+  for (const at::Tensor* f : {(const at::Tensor*)&x, &wl, &wr, &gain}) chk_f32(*f, "x, weights, gain");
+  TORCH_CHECK(x.dim() == 2 && l.sizes() == x.sizes() && r.sizes() == x.sizes() && l.is_contiguous() && r.is_contiguous() && is_act(l) &&
+                  r.scalar_type() == l.scalar_type() && l.is_cuda() && r.is_cuda(), "left / right: [T, W] like x");
+  TORCH_CHECK(wl.numel() == x.size(1) && wr.numel() == x.size(1) && gain.numel() == 1, "weights: [W], gain: one number");
+  if (extra) TORCH_CHECK(extra->sizes() == x.sizes() && extra->is_contiguous() && extra->is_cuda() &&
+                             extra->scalar_type() == l.scalar_type(), "extra: [T, W] like left");
+  if ((f32(l) != 0) != out_f32) return std::nullopt;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  auto out = at::empty({x.size(0), x.size(1)}, x.options().dtype(act_type(out_f32)));
+  const int rc = edge_sm_combine_norm(x.data_ptr<float>(), l.data_ptr(), r.data_ptr(), wl.data_ptr<float>(), wr.data_ptr<float>(),
+                                      extra ? extra->data_ptr() : nullptr, (float)eps, gain.data_ptr<float>(), (float)eps2,
+                                      out.data_ptr(), (int)x.size(0), (int)x.size(1), f32(l), stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_combine_norm");
+  return out;
 }
 
 at::Tensor sm_rms_cols(const at::Tensor& u, int64_t c0, int64_t C, const at::Tensor& w, double eps, bool out_f32) {
@@ -1377,6 +1480,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_ssd_scan", &sm_ssd_scan);
   m.def("sm_embed_bigram", &sm_embed_bigram);
   m.def("sm_canon", &sm_canon);
+  m.def("sm_ln_residual_taps", &sm_ln_residual_taps);
+  m.def("sm_group_residual_norm", &sm_group_residual_norm);
+  m.def("sm_combine_norm", &sm_combine_norm);
   m.def("sm_layer_norm", &sm_layer_norm);
   m.def("sm_ln_residual", &sm_ln_residual);
   m.def("sm_rms_cols", &sm_rms_cols);

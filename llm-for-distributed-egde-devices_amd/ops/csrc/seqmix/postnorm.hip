@@ -16,6 +16,7 @@
 #include "seqmix/seqmix_common.h"
 #include "seqmix/delta_prep.h"
 #include "seqmix/moe_rows.h"
+#include "seqmix/row_parts.h"
 #include "seqmix/tap4.h"
 
 namespace {
@@ -187,42 +188,18 @@ __global__ void __launch_bounds__(NT) ln_residual4_kernel(float* __restrict__ x,
     load4<float>(w + c, wv[i]);
     load4<float>(b + c, bv[i]);
   }
-  for (int k0 = 0; k0 < K; k0 += 4) {
-    float p[4][CH][4], pk[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      pk[k] = pw[t * K + min(k0 + k, K - 1)];
-#pragma unroll
-      for (int i = 0; i < CH; ++i)
-        load4<T>(parts + (t * K + min(k0 + k, K - 1)) * W + min(((int)threadIdx.x + i * NT) * 4, W - 4), p[k][i]);
-    }
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int i = 0; i < CH; ++i)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[i][e] = k0 + k < K ? v[i][e] + pk[k] * p[k][i][e] : v[i][e];
-  }
-  auto total = [&](float s, float* r) {
-    s = wave_sum(s);
-    if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = s;
-    __syncthreads();
-    float o = 0.f;
-#pragma unroll
-    for (int i = 0; i < NT / 64; ++i) o += r[i];
-    return o;
-  };
+  add_parts<T, CH>(v, parts, pw, K, t, W);
 #pragma unroll
   for (int i = 0; i < CH; ++i)
     if (((int)threadIdx.x + i * NT) * 4 < W) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-  const float mean = total(sum, red[0]) / (float)W;
+  const float mean = row_total(sum, red[0]) / (float)W;
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < CH; ++i)
     if (((int)threadIdx.x + i * NT) * 4 < W)
 #pragma unroll
       for (int e = 0; e < 4; ++e) { const float d = v[i][e] - mean; ss += d * d; }
-  const float r = 1.f / sqrtf(total(ss, red[1]) / (float)W + eps);
+  const float r = 1.f / sqrtf(row_total(ss, red[1]) / (float)W + eps);
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     const int c = ((int)threadIdx.x + i * NT) * 4;

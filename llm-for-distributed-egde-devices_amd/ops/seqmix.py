@@ -167,6 +167,17 @@ def combine_residual(x: torch.Tensor, left: torch.Tensor, right: torch.Tensor, w
     return x
 
 
+def combine_residual_norm(x: torch.Tensor, left: torch.Tensor, right: torch.Tensor, wl: torch.Tensor, wr: torch.Tensor, eps: float,
+                          extra: Optional[torch.Tensor], gain: torch.Tensor, gain_eps: float, out_dtype) -> torch.Tensor:
+    """``combine_residual``, then ``scalar_rms_norm`` of the new x (one launch where the row fits): returns the normed rows."""
+    if _gpu(x):
+        h = _ext().sm_combine_norm(x, left, right, wl, wr, float(eps), extra, gain, float(gain_eps), out_dtype == torch.float32)
+        if h is not None:
+            return h
+    combine_residual(x, left, right, wl, wr, eps, extra)
+    return scalar_rms_norm(x, gain, gain_eps, out_dtype)
+
+
 def gated_group_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, groups: int, eps: float,
                      out_dtype) -> torch.Tensor:
     """rms-norm in ``groups`` equal parts of (y * silu(z)) times weight.  y fp32 [T, C]; z [T, C] a
@@ -507,6 +518,20 @@ def layer_norm_residual(x: torch.Tensor, y: Optional[torch.Tensor], weight: torc
     return x
 
 
+def layer_norm_residual_canon(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor, eps: float,
+                              parts: Optional[torch.Tensor], part_w: Optional[torch.Tensor], canon: torch.Tensor, state: torch.Tensor,
+                              meta: RaggedMeta, out_dtype) -> torch.Tensor:
+    """``layer_norm_residual``, then ``canon_conv`` of the new x (one launch in steps in which every sequence brings one token,
+    where the row fits): returns the convolved rows."""
+    if _gpu(x) and meta.max_len == 1:
+        h = _ext().sm_ln_residual_taps(x, y, weight, bias, float(eps), parts, part_w, canon, state, meta.tok_seq, meta.tok_pos,
+                                       meta.seq_slot, out_dtype == torch.float32)
+        if h is not None:
+            return h
+    layer_norm_residual(x, y, weight, bias, eps, parts, part_w)
+    return canon_conv(x, canon, state, meta, out_dtype)
+
+
 def _group_rms(v: torch.Tensor, groups: int, eps: float) -> torch.Tensor:
     T, W = v.shape
     g = v.view(T, groups, W // groups)
@@ -535,6 +560,19 @@ def group_norm_residual(x: torch.Tensor, y: Optional[torch.Tensor], weight: torc
             v = v + (parts[:, k].float() if part_w is None else part_w[:, k:k + 1] * parts[:, k].float())
     x.add_(_group_rms(v, groups, eps) * weight.float(), alpha=mult)
     return x
+
+
+def group_norm_residual_norm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, groups: int, eps: float, mult: float,
+                             parts: Optional[torch.Tensor], part_w: Optional[torch.Tensor], next_weight: torch.Tensor,
+                             next_groups: int, next_eps: float, out_dtype) -> torch.Tensor:
+    """``group_norm_residual``, then ``group_rms_norm`` of the new x (one launch where the row fits): returns the normed rows."""
+    if _gpu(x):
+        h = _ext().sm_group_residual_norm(x, y, weight, int(groups), float(eps), float(mult), parts, part_w, next_weight,
+                                          int(next_groups), float(next_eps), out_dtype == torch.float32)
+        if h is not None:
+            return h
+    group_norm_residual(x, y, weight, groups, eps, mult, parts, part_w)
+    return group_rms_norm(x, next_weight, next_groups, next_eps, out_dtype)
 
 
 def rms_norm_cols(u: torch.Tensor, c0: int, C: int, weight: torch.Tensor, eps: float, out_dtype) -> torch.Tensor:
