@@ -286,6 +286,11 @@ class Norm(nn.Module):
         return ops.layer_norm(x, self.weight, self.bias, self.eps, residual)
 
 
+def plain_linear(m: nn.Module) -> bool:
+    """A bias-free 16- or 32-bit projection whose own call nobody watches: its weight says all."""
+    return type(m) is Linear and m.bias is None and not (m._forward_hooks or m._forward_pre_hooks)
+
+
 class ScalarNorm(nn.Module):
     """RMS norm whose gain is one number for all coordinates: fp32 rows in (the residual stream of
     the layer-spec models), rows of the consumer's dtype out."""

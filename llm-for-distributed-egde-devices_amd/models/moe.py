@@ -22,7 +22,7 @@ import torch.nn as nn
 
 from ..ops import seqmix
 from .configs import MoESpec
-from .layers import Linear
+from .layers import Linear, plain_linear
 
 
 class MoEOut(NamedTuple):
@@ -31,11 +31,6 @@ class MoEOut(NamedTuple):
     parts: torch.Tensor                 # the chosen experts' outputs [T, top, W]
     wts: Optional[torch.Tensor]         # their weights fp32 [T, top]
     rows: Optional[torch.Tensor]        # int32 [T, top]: each choice's row of parts viewed [-1, W] (None: in order)
-
-
-def _plain(m: nn.Module) -> bool:
-    """A bias-free 16- or 32-bit projection whose own call nobody watches: its weight says all."""
-    return type(m) is Linear and m.bias is None and not (m._forward_hooks or m._forward_pre_hooks)
 
 
 class MoEFeedForward(nn.Module):
@@ -62,7 +57,7 @@ class MoEFeedForward(nn.Module):
         s = self.spec
         idx, wts = seqmix.moe_route(h, self.router, s.top, s.scale, s.router, self.router_b)
         on_input = s.weight_on == "input"
-        if s.shared_ff and s.act == "glu_clamp" and not on_input and _plain(self.shared_gu) and _plain(self.shared_down):
+        if s.shared_ff and s.act == "glu_clamp" and not on_input and plain_linear(self.shared_gu) and plain_linear(self.shared_down):
             both = seqmix.moe_experts_glu_shared(h, idx, self.w_gu, self.w_down, s.limit, self.shared_gu.weight,
                                                  self.shared_down.weight, s.shared_limit)
             if both is not None:

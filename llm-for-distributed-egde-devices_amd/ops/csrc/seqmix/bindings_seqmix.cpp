@@ -29,6 +29,10 @@ int edge_sm_group_residual_norm(float* x, const void* y, const void* parts, cons
                                 hipStream_t st);
 int edge_sm_combine_norm(float* x, const void* l, const void* r, const float* wl, const float* wr, const void* extra, float eps,
                          const float* gain, float eps2, void* out, int rows, int W, int f32, hipStream_t st);
+int edge_sm_delta_step(const void* u, int ld, int b0, int a0, int z0, const void* a2, int ra, const void* g2, int rg,
+                       const float* conv_w, const float* conv_b, void* tail, float* state, const float* dt_bias, const float* A_log,
+                       const float* norm_w, const int* seq_slot, const int* seq_start, const int* seq_off, void* out, int n, int H, int N,
+                       int P, float eps, int f32, hipStream_t st);
 int edge_sm_group_norm(const float* x, const float* w, void* y, int rows, int W, int groups, float eps, int f32,
                        hipStream_t st);
 int edge_sm_group_norm_residual(float* x, const void* y, const void* parts, const float* pw, int K, const float* w,
@@ -787,6 +791,48 @@ at::Tensor sm_delta_prep(const at::Tensor& qkv, const at::Tensor& u, int64_t b0,
   return prep;
 }
 
+// One token per sequence through a whole gated delta rule between its projections (delta_step.hip); nothing comes back, and nothing
+// was done, where the kernel does not take the sizes, types or addresses.  a2 / g2: low-rank products over columns a0.. / z0.. of u, or
+// neither (one decay per head at column a0, gates at column z0)
+std::optional<at::Tensor> sm_delta_step(const at::Tensor& u, int64_t b0, int64_t a0, int64_t z0, const std::optional<at::Tensor>& a2,
+                                        const std::optional<at::Tensor>& g2, const at::Tensor& conv_w, const at::Tensor& conv_b,
+                                        at::Tensor& tail, at::Tensor& state, const at::Tensor& dt_bias, const at::Tensor& A_log,
+                                        const at::Tensor& norm_w, const at::Tensor& seq_slot, const at::Tensor& seq_start,
+                                        const at::Tensor& seq_off, int64_t n, double eps) {
+  const int ld = row_ld(u, "u");
+  TORCH_CHECK(is_act(u) && u.size(0) == n, "u: one row per sequence");
+  for (const at::Tensor* t : {&seq_slot, &seq_start, &seq_off}) chk_i32(*t, "metadata");
+  TORCH_CHECK(seq_slot.numel() >= n && seq_start.numel() >= n && seq_off.numel() >= n, "sequence metadata: [n]");
+  for (const at::Tensor* t : {&conv_w, &conv_b, (const at::Tensor*)&state, &dt_bias, &A_log, &norm_w}) chk_f32(*t, "weights, state");
+  TORCH_CHECK(state.dim() == 4, "state: fp32 [slots, heads, N, P]");
+  const int64_t H = state.size(1), N = state.size(2), P = state.size(3), C = 2 * H * N + H * P;
+  if (conv_w.dim() != 2 || conv_w.size(0) != C || conv_w.size(1) != 4 || bool(a2) != bool(g2)) return std::nullopt;
+  TORCH_CHECK(tail.is_cuda() && tail.is_contiguous() && tail.scalar_type() == u.scalar_type() && tail.dim() == 3 && tail.size(1) == 3 &&
+                  tail.size(2) == C && tail.size(0) == state.size(0), "tail: [slots, 3, C]");
+  TORCH_CHECK(conv_b.numel() == C && A_log.numel() == H && norm_w.numel() == P && dt_bias.numel() == (a2 ? H * N : H) && b0 >= C &&
+                  a0 >= C && z0 >= C && b0 + H <= u.size(1), "delta step: weights");
+  int64_t ra = 0, rg = 0;
+  if (a2) {
+    for (const at::Tensor* t : {&*a2, &*g2})
+      if (!t->is_cuda() || !t->is_contiguous() || t->dim() != 2 || t->scalar_type() != u.scalar_type()) return std::nullopt;
+    ra = a2->size(1);
+    rg = g2->size(1);
+    TORCH_CHECK(a2->size(0) == H * N && g2->size(0) == H * P, "low-rank products: [H N, rank], [H P, rank]");
+  }
+  TORCH_CHECK(a0 + (a2 ? ra : H) <= u.size(1) && z0 + (a2 ? rg : H * P) <= u.size(1), "delta step: columns of u");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(u.device());
+  auto out = at::empty({n, H * P}, u.options());
+  const int rc = edge_sm_delta_step(u.data_ptr(), ld, (int)b0, (int)a0, (int)z0, a2 ? a2->data_ptr() : nullptr, (int)ra,
+                                    g2 ? g2->data_ptr() : nullptr, (int)rg, conv_w.data_ptr<float>(), conv_b.data_ptr<float>(),
+                                    tail.data_ptr(), state.data_ptr<float>(), dt_bias.data_ptr<float>(), A_log.data_ptr<float>(),
+                                    norm_w.data_ptr<float>(), seq_slot.data_ptr<int>(), seq_start.data_ptr<int>(),
+                                    seq_off.data_ptr<int>(), out.data_ptr(), (int)n, (int)H, (int)N, (int)P, (float)eps, f32(u),
+                                    stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_delta_step");
+  return out;
+}
+
 at::Tensor sm_delta_scan(const at::Tensor& prep, const at::Tensor& qkv, at::Tensor& state, const at::Tensor& seq_slot,
                          const at::Tensor& seq_start, const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n,
                          int64_t H, int64_t G, int64_t N, int64_t P, int64_t room, int64_t most, int64_t max_chunks, int64_t least) {
@@ -1490,6 +1536,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_glu_clamp", &sm_glu_clamp);
   m.def("sm_latent_write", &sm_latent_write);
   m.def("sm_delta_prep", &sm_delta_prep);
+  m.def("sm_delta_step", &sm_delta_step);
   m.def("sm_delta_scan", &sm_delta_scan);
   m.def("sm_delta_chunk_floats", &edge_sm_delta_chunk_floats);
   m.def("sm_moe_route", &sm_moe_route);

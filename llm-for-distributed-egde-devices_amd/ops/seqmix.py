@@ -914,6 +914,20 @@ def head_norm_gate(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, heads
     return (g.view(T, C) * gate).to(out_dtype)
 
 
+def delta_step(u: torch.Tensor, b0: int, a0: int, z0: int, a2: Optional[torch.Tensor], g2: Optional[torch.Tensor],
+               conv_w: torch.Tensor, conv_b: torch.Tensor, tail: torch.Tensor, state: torch.Tensor, dt_bias: torch.Tensor,
+               A_log: torch.Tensor, norm_w: torch.Tensor, eps: float, meta: RaggedMeta, kv_heads: int) -> Optional[torch.Tensor]:
+    """A gated delta rule between its two projections in one launch, for steps in which every sequence brings one token and no two
+    heads share q and k: ``conv_silu`` of u's first columns, ``delta_prepare`` (a2 [heads N, rank], g2 [heads P, rank]: products over
+    u's columns from a0 and z0) or ``delta_prepare_head`` (neither: the decay at column a0 + head, the gates from z0 on),
+    ``delta_rule_scan`` and ``head_norm_gate`` (sigmoid; per-head decays: silu).  ``tail`` and ``state`` move on.  None where it is
+    not one launch: nothing has been done then."""
+    if not _gpu(u) or meta.max_len != 1 or meta.T != meta.n or kv_heads != state.shape[1]:
+        return None
+    return _ext().sm_delta_step(u, int(b0), int(a0), int(z0), a2, g2, conv_w, conv_b, tail, state, dt_bias, A_log, norm_w,
+                                meta.seq_slot, meta.seq_start, meta.seq_off, int(meta.n), float(eps))
+
+
 # --------------------------------------------------------------------------- mixture of experts
 def moe_route_grouped(h: torch.Tensor, router: torch.Tensor, top: int, scale: float, correction: Optional[torch.Tensor],
                       groups: int = 1, keep: int = 1, gate: bool = False):
