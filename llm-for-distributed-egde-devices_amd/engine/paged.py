@@ -125,7 +125,10 @@ class PagedCache:
         if need > 0:
             first = len(own)
             own.extend(self.free_pages.pop() for _ in range(need))
-            self.page_table[slot, first:len(own)] = torch.tensor(own[first:], dtype=torch.int32)
+            ids = torch.tensor(own[first:], dtype=torch.int32)
+            if self.page_table.is_cuda:                     # from pinned memory: a copy in stream order that nobody waits for
+                ids = ids.pin_memory()
+            self.page_table[slot, first:len(own)].copy_(ids, non_blocking=True)
         self.lens[slot] = max(self.lens[slot], new_len)
 
     def release(self, slot: int) -> None:

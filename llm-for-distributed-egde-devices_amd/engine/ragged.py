@@ -39,36 +39,43 @@ class _DecodeGraph:
     def __init__(self, eng: "RaggedEngine", n: int):
         dev = eng.device
         self.eng, self.n = eng, n
-        self.buf = torch.zeros(6 * n, dtype=torch.int32, device=dev)
-        self.ids = torch.zeros(n, dtype=torch.long, device=dev)
-        self.host = [(torch.zeros(6 * n, dtype=torch.int32).pin_memory(), torch.zeros(n, dtype=torch.long).pin_memory(),
-                      torch.cuda.Event()) for _ in range(self.RING)]
+        # one buffer, one copy a step: the ids (8 bytes each) in front of the metadata (4 bytes each)
+        parts = lambda raw: (raw[:8 * n].view(torch.long), raw[8 * n:].view(torch.int32))
+        self.raw = torch.zeros(32 * n, dtype=torch.uint8, device=dev)
+        self.ids, self.buf = parts(self.raw)
+        raws = [torch.zeros(32 * n, dtype=torch.uint8).pin_memory() for _ in range(self.RING)]
+        self.host = [(raw, *(t.numpy() for t in parts(raw)), torch.cuda.Event()) for raw in raws]
+        fixed = np.concatenate([np.ones(n), np.arange(n), np.arange(n)]).astype(np.int32)    # lengths, offsets, tokens' sequences
+        for _, _, hb, _ in self.host:
+            hb[2 * n:5 * n] = fixed
         self.turn = 0
         b = self.buf
         cap = eng.cache.num_pages * eng.page
         self.meta = RaggedMeta(n, n, b[0:n], b[n:2 * n], b[2 * n:3 * n], b[3 * n:4 * n], b[4 * n:5 * n], b[5 * n:6 * n],
                                eng.cache.page_table, eng.page, [(0, 1, 1, i) for i in range(n)], 1, cap)
-        self.rows = torch.arange(n, dtype=torch.long, device=dev)
         self.graph: Optional[torch.cuda.CUDAGraph] = None
         self.out: Optional[torch.Tensor] = None
+        self.raw_out = False
         self.warm = False
 
     def run(self, seqs, ids) -> torch.Tensor:
+        """fp32 logits of every sequence, in memory of their own."""
         n = self.n
-        hb, hi, ev = self.host[self.turn]
+        hraw, hi, hb, ev = self.host[self.turn]
         self.turn = (self.turn + 1) % self.RING
         ev.synchronize()                           # the copy that last read this pinned row is done
-        flat = [s[0] for s in seqs] + [s[1] for s in seqs] + [1] * n + list(range(n)) + list(range(n)) + \
-            [s[1] for s in seqs]
-        hb.copy_(torch.tensor(flat, dtype=torch.int32))
-        hi.copy_(torch.tensor(ids, dtype=torch.long))
-        self.buf.copy_(hb, non_blocking=True)
-        self.ids.copy_(hi, non_blocking=True)
+        hb[:n] = [s[0] for s in seqs]
+        hb[n:2 * n] = hb[5 * n:] = [s[1] for s in seqs]     # a token's position is its portion's start
+        hi[:] = torch.tensor(ids, dtype=torch.long).numpy()
+        self.raw.copy_(hraw, non_blocking=True)
         ev.record()
         eng = self.eng
+        # a model that nobody watches is captured up to its output projection's rows: making logits of them also takes them out of
+        # the graph's memory, and every row is wanted
+        watched = bool(eng.model._forward_hooks or eng.model._forward_pre_hooks) or not hasattr(eng.model, "scores")
         if not self.warm:
             self.warm = True
-            return eng.model(self.ids, self.meta, eng.cache, self.rows)
+            return eng.model(self.ids, self.meta, eng.cache)
         if self.graph is None:
             # no cyclic garbage collection while the stream captures: a collected engine of an earlier
             # request frees pinned buffers and graphs, which the runtime refuses during a capture; what
@@ -81,13 +88,15 @@ class _DecodeGraph:
             gc.disable()
             try:
                 with torch.cuda.graph(g, pool=eng._pool):
-                    self.out = eng.model(self.ids, self.meta, eng.cache, self.rows)
+                    self.out = eng.model(self.ids, self.meta, eng.cache) if watched else \
+                        eng.model.scores(self.ids, self.meta, eng.cache)
+                self.raw_out = not watched
             except Exception as e:  # noqa: BLE001 - an op that cannot be captured: this engine steps eagerly
                 from ..utils.log import get_logger
                 get_logger("ragged").warning(f"decode step not graph-capturable ({e!r}): running eagerly")
                 torch.cuda.synchronize()
                 eng.use_graphs = False
-                return eng.model(self.ids, self.meta, eng.cache, self.rows)
+                return eng.model(self.ids, self.meta, eng.cache)
             finally:
                 if gc_was_on:
                     gc.enable()
@@ -95,7 +104,7 @@ class _DecodeGraph:
                 eng._pool = g.pool()
             self.graph = g
         self.graph.replay()
-        return self.out
+        return eng.model.finish(self.out) if self.raw_out else self.out.clone()
 
 
 class RaggedEngine:
@@ -164,7 +173,7 @@ class RaggedEngine:
                 out = dg.run(seqs, ids)
             self.graphs_used = self.graphs_used or dg.graph is not None
             if rows == list(range(len(seqs))):
-                return out.clone()
+                return out
             return out.index_select(0, torch.tensor(rows, dtype=torch.long, device=self.device))
         meta = RaggedMeta.build(seqs, self.cache.page_table, self.page, self.device)
         ids_t = torch.from_numpy(np.asarray(ids, dtype=np.int64))

@@ -428,6 +428,23 @@ class HybridLM(nn.Module):
                 taps: Optional[list] = None) -> torch.Tensor:
         """ids [T] (flat step) -> fp32 logits of ``rows`` (flat row indices; None: every row).
         ``taps`` (a list) receives the residual stream after every run."""
+        return self.finish(self.scores(ids, meta, cache, rows, taps), ours=True)
+
+    def finish(self, z: torch.Tensor, ours: bool = False) -> torch.Tensor:
+        """fp32 logits from the output projection's rows, in memory of their own unless z is ``ours`` to reuse."""
+        cfg = self.cfg
+        if z.numel() == 0:
+            return torch.empty(0, cfg.vocab_size, dtype=torch.float32, device=z.device)
+        if cfg.logit_softcap is not None:
+            return seqmix.softcap(z, cfg.logit_softcap)
+        if z.dtype != torch.float32 or ours:
+            z = z.float()
+            return z if cfg.logit_scale == 1.0 else z.mul_(cfg.logit_scale)
+        return z.clone() if cfg.logit_scale == 1.0 else z * cfg.logit_scale
+
+    def scores(self, ids: torch.Tensor, meta: seqmix.RaggedMeta, cache, rows: Optional[torch.Tensor] = None,
+               taps: Optional[list] = None) -> torch.Tensor:
+        """``forward`` up to the output projection's rows in the model's own type (``finish`` makes logits of them)."""
         cfg = self.cfg
         if cfg.bigram:
             b = cfg.bigram
@@ -466,12 +483,7 @@ class HybridLM(nn.Module):
             if rows.numel() == 0:                        # nothing asked for: the step only fed the cache
                 return torch.empty(0, cfg.vocab_size, dtype=torch.float32, device=x.device)
             x = x.index_select(0, rows)
-        h = self.final_norm(x, None, self.dtype) if cfg.streams else self.final_norm(x, self.dtype)
-        logits = self.lm_head(h)
-        if cfg.logit_softcap is not None:
-            return seqmix.softcap(logits, cfg.logit_softcap)
-        logits = logits.float()
-        return logits if cfg.logit_scale == 1.0 else logits.mul_(cfg.logit_scale)
+        return self.lm_head(self.final_norm(x, None, self.dtype) if cfg.streams else self.final_norm(x, self.dtype))
 
 
 # --------------------------------------------------------------------------- weights
