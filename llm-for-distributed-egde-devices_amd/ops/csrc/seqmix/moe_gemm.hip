@@ -11,10 +11,10 @@
 //
 // Measured (both products, sorting and activation; MI355X) against one library product per expert with the sort, the
 // gather, the activation and the scatter as launches of their own: 4096 tokens x 3 of 16 experts 1024 -> 1024,
-// 758 -> 129 us (600 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 790 us (734); 512 x 4 of 32, 2048 -> 2048,
-// 1369 -> 212 us, where the experts' 805 MB (3.8 TB/s) are the bound.  At 128-row tiles the bound is the operands' way
-// into the LDS (64 B per clock and CU at the full MFMA rate): 128 x 256 tiles gain 3-6 % from 2048 columns on and lose
-// below, deeper rings with one workgroup per CU lose 40 %.
+// 758 -> 127 us (610 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 664 us (874); 512 x 4 of 32, 2048 -> 2048,
+// 1369 -> 200 us, where the experts' 805 MB (4.0 TB/s) are the bound.  At 128-row tiles the bound is the LDS: 64 B per clock and
+// CU come in and 128 are read at the full MFMA rate (tall_tiles says what 256-row tiles change); 128 x 256 tiles gained 3-6 %
+// from 2048 columns on and lost below, deeper rings with one workgroup of 128 x 128 per CU lose 40 %.
 #include "seqmix_common.h"
 
 namespace {
@@ -261,6 +261,19 @@ int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* 
 // Rows of a tile by the average rows per expert: a tile much taller than that multiplies padding, and below about 24
 // the weights' bytes are all that counts (32 rows: two fragments, the smallest ring).
 int tile_rows(int64_t R, int E) { return R > (int64_t)E * 80 ? 128 : R > (int64_t)E * 24 ? 64 : 32; }
+// 256 x 256 tiles (one workgroup of 8 waves a CU, 128 x 64 a wave) halve what 128 x 128 ones (two workgroups of 4 waves, 64 x 64)
+// read from and bring into the LDS per product, which is their bound, but fill the chip in whole rounds of 256 workgroups and
+// multiply more padding.  So both times are estimated, from us a 64-k stage and us a workgroup's start and end fitted to both
+// sides, half a tile of padding an expert.  us for both products, 128 / 256: 3 of 32 experts of 2048 -> 3072 (relu2), 1000 tokens
+// 204 / 223, 4096 534 / 400, 7680 760 / 664 (874 TFLOP/s); 4 of 32 of 2048 -> 2048, 7600 976 / 781 (980 TFLOP/s); 3 of 16 of 1024
+// -> 1024, 2048 82 / 85, 4096 134 / 127; 4 of 16, 4096 171 / 195, 7600 280 / 256
+bool tall_tiles(int64_t R, int E, int W, int ff, int up) {
+  auto tiles = [&](int64_t BM) { const int64_t t = R / BM + E / 2; return t > E ? t : E; };
+  const int fn = up == 2 ? 2 : 1;                            // gated units: half a tile's weight rows are features
+  auto tall = [&](int N, int K) { return (double)((tiles(256) * ((N + 255) / 256) + 255) / 256) * (1.5 * K / 64 + 12.8); };
+  auto low = [&](int N, int K) { return tiles(128) * ((N + 127) / 128) / 512.0 * (0.94 * K / 64 + 10.2); };
+  return tall(ff * fn, W) + tall(W, ff) < low(ff * fn, W) + low(W, ff);
+}
 int max_tiles(int64_t R, int E, int BM) { return (int)((R + BM - 1) / BM + (R < E ? R : E)); }
 }  // namespace
 
@@ -279,13 +292,16 @@ int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff) {
 int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void* w_down, int* ints, void* y, void* out, int T,
                      int top, int E, int W, int ff, int act, const float* row_w, float limit, hipStream_t st) {
   if (edge_sm_moe_gemm_ok(T, top, E, W, ff) != 0 || act < ACT_GLU_CLAMP || act > ACT_RELU2) return -2;
-  const int R = T * top, BM = tile_rows(R, E), mt = max_tiles(R, E, BM);
+  // (the tile list of 256-row tiles is the shorter one: edge_sm_moe_gemm_ints serves both)
+  const int R = T * top, low = tile_rows(R, E), BM = low == 128 && tall_tiles(R, E, W, ff, act == ACT_RELU2 ? 1 : 2) ? 256 : low,
+            mt = max_tiles(R, E, BM);
   int *rows = ints, *tiles = ints + ((R + 3) & ~3);
   // while the weights' bytes are the bound (up to some 500 rows an expert) the workgroups' k starts are spread: us for both
   // products, 32 experts of 2048 x 2048, 4 each: 24 tokens 194 / 139, 128 209 / 147 (5.5 TB/s), 384 210 / 158, 800 224 / 179,
   // 3000 476 / 474; with more rows it costs 2 % (7680 tokens of 3, ff 3072: 779 / 798)
   const int spread = R <= E * 512;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(SORT_NT), 0, st, idx, R, E, BM, rows, tiles);
+  if (BM == 256) return launch_pair<256, 256, 2, 4, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
   if (BM == 128) return launch_pair<128, 128, 2, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
   if (BM == 64) return launch_pair<64, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
   return launch_pair<32, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);

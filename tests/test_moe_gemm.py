@@ -149,3 +149,35 @@ def test_steps_that_the_grouped_kernels_do_not_take():
     assert not seqmix.moe_grouped(h[:5], idx[:5], w_gu, w_down, "silu_glu", in_w[:5])
     assert torch.allclose(seqmix.moe_experts(wide[:, :128], idx, w_gu, w_down, 0.0, "silu_glu", in_w).float(),
                           seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "silu_glu", in_w).float(), atol=3e-2, rtol=3e-2)
+
+
+@gpu
+@pytest.mark.parametrize("act,T,top,E,W,ff", [("glu_clamp", 5200, 3, 7, 960, 1088), ("silu_glu", 5200, 3, 7, 960, 1088),
+                                              ("relu2", 10200, 2, 5, 2048, 2048)])
+def test_tall_tiles(act, T, top, E, W, ff):
+    """Sizes whose estimate chooses 256 x 256 tiles, with remainders of rows and columns (960 = 3 x 256 + 192)."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    h, w_gu = r(T, W).bfloat16(), (r(E, ff if act == "relu2" else 2 * ff, W) * W ** -0.5).bfloat16()
+    w_down, in_w = (r(E, W, ff) * ff ** -0.5).bfloat16(), torch.rand(T, top, generator=g, device="cuda") if act == "silu_glu" else None
+    idx = torch.rand(T, E, generator=g, device="cuda").topk(top, 1)[1].int()
+    assert seqmix.moe_grouped(h, idx, w_gu, w_down, act, in_w)
+    got = seqmix.moe_experts(h, idx, w_gu, w_down, 1.5, act, in_w)
+    err = norm = 0.0
+    for e in range(E):
+        t, k = (idx == e).nonzero(as_tuple=True)
+        u = h[t].double() @ w_gu[e].double().t()
+        gate, up = u[:, :ff], u[:, ff:]
+        if act == "relu2":
+            y = torch.relu(u) ** 2
+        elif act == "glu_clamp":
+            gate = gate.clamp(max=1.5)
+            y = gate * torch.sigmoid(1.702 * gate) * (up.clamp(-1.5, 1.5) + 1)
+        else:
+            rw = in_w[t, k].double()[:, None]
+            y = torch.nn.functional.silu(rw * gate) * (rw * up)
+        want = y @ w_down[e].double().t()
+        d = got[t, k].double() - want
+        assert (d.norm(dim=-1) / want.norm(dim=-1).clamp_min(1e-3)).max() < 4 * TOL
+        err, norm = err + d.norm().item() ** 2, norm + want.norm().item() ** 2
+    assert err ** 0.5 < TOL * norm ** 0.5
