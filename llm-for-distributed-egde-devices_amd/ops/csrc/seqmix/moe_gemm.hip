@@ -12,7 +12,7 @@
 // Measured (both products, sorting and activation; MI355X) against one library product per expert with the sort, the
 // gather, the activation and the scatter as launches of their own: 4096 tokens x 3 of 16 experts 1024 -> 1024,
 // 758 -> 127 us (610 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 664 us (874); 512 x 4 of 32, 2048 -> 2048,
-// 1369 -> 200 us, where the experts' 805 MB (4.0 TB/s) are the bound.  At 128-row tiles the bound is the LDS: 64 B per clock and
+// 1369 -> 169 us, where the experts' 805 MB (4.8 TB/s) are the bound.  At 128-row tiles the bound is the LDS: 64 B per clock and
 // CU come in and 128 are read at the full MFMA rate (tall_tiles says what 256-row tiles change); 128 x 256 tiles gained 3-6 %
 // from 2048 columns on and lost below, deeper rings with one workgroup of 128 x 128 per CU lose 40 %.
 #include "seqmix_common.h"
@@ -259,8 +259,14 @@ int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* 
 }
 
 // Rows of a tile by the average rows per expert: a tile much taller than that multiplies padding, and below about 24
-// the weights' bytes are all that counts (32 rows: two fragments, the smallest ring).
-int tile_rows(int64_t R, int E) { return R > (int64_t)E * 80 ? 128 : R > (int64_t)E * 24 ? 64 : 32; }
+// the weights' bytes are all that counts (32 rows: two fragments, the smallest ring).  From some 50 rows on about half of the
+// experts need a second 64-row tile, which reads their weights once more for a few rows: with experts of 2^26 numbers or more
+// together 128 rows pay from there (us for both products, 64 / 128: 4 of 32 of 2048 x 2048, 49 rows an expert 161 / 164, 52 173 / 166,
+// 65 196 / 169, 73 241 / 172), with fewer, which leave CUs without a tile, only from 128 on (3 or 4 of 16 of 1024 x 1024, 75 rows
+// 35 / 38, 100 34 / 40, 131 46 / 46, 188 51 / 47)
+int tile_rows(int64_t R, int E, int W, int ff) {
+  return R > (int64_t)E * ((int64_t)E * W * ff >= 1 << 26 ? 50 : 128) ? 128 : R > (int64_t)E * 24 ? 64 : 32;
+}
 // 256 x 256 tiles (one workgroup of 8 waves a CU, 128 x 64 a wave) halve what 128 x 128 ones (two workgroups of 4 waves, 64 x 64)
 // read from and bring into the LDS per product, which is their bound, but fill the chip in whole rounds of 256 workgroups and
 // multiply more padding.  So both times are estimated, from us a 64-k stage and us a workgroup's start and end fitted to both
@@ -279,8 +285,8 @@ int max_tiles(int64_t R, int E, int BM) { return (int)((R + BM - 1) / BM + (R < 
 
 extern "C" {
 
-// int32 words of scratch: the sorted pairs and the tile list
-int64_t edge_sm_moe_gemm_ints(int64_t R, int E) { return ((R + 3) & ~3LL) + 4 + 4LL * max_tiles(R, E, tile_rows(R, E)); }
+// int32 words of scratch: the sorted pairs and the tile list (its longest: taller tiles are fewer)
+int64_t edge_sm_moe_gemm_ints(int64_t R, int E) { return ((R + 3) & ~3LL) + 4 + 4LL * max_tiles(R, E, R > (int64_t)E * 24 ? 64 : 32); }
 
 // 0 when the kernels take these sizes
 int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff) {
@@ -292,8 +298,7 @@ int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff) {
 int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void* w_down, int* ints, void* y, void* out, int T,
                      int top, int E, int W, int ff, int act, const float* row_w, float limit, hipStream_t st) {
   if (edge_sm_moe_gemm_ok(T, top, E, W, ff) != 0 || act < ACT_GLU_CLAMP || act > ACT_RELU2) return -2;
-  // (the tile list of 256-row tiles is the shorter one: edge_sm_moe_gemm_ints serves both)
-  const int R = T * top, low = tile_rows(R, E), BM = low == 128 && tall_tiles(R, E, W, ff, act == ACT_RELU2 ? 1 : 2) ? 256 : low,
+  const int R = T * top, low = tile_rows(R, E, W, ff), BM = low == 128 && tall_tiles(R, E, W, ff, act == ACT_RELU2 ? 1 : 2) ? 256 : low,
             mt = max_tiles(R, E, BM);
   int *rows = ints, *tiles = ints + ((R + 3) & ~3);
   // while the weights' bytes are the bound (up to some 500 rows an expert) the workgroups' k starts are spread: us for both

@@ -152,6 +152,23 @@ def test_steps_that_the_grouped_kernels_do_not_take():
 
 
 @gpu
+@pytest.mark.parametrize("E,W,ff,T,top", [(32, 1024, 2048, 400, 4), (32, 1024, 2048, 401, 4), (32, 1024, 1984, 401, 4), (4, 64, 64, 256, 2),
+                                          (4, 64, 64, 257, 2)])
+def test_lines_between_tile_heights(E, W, ff, T, top, every_size):
+    """Rows per expert on both sides of 50 (experts of 2^26 numbers together) and of 128, numbers on both sides of 2^26."""
+    g = torch.Generator(device="cuda").manual_seed(T + ff)
+    r = lambda *s: torch.randn(*s, generator=g, device="cuda")
+    h, w_gu, w_down = r(T, W).bfloat16(), (r(E, ff, W) * W ** -0.5).bfloat16(), (r(E, W, ff) * ff ** -0.5).bfloat16()
+    idx = torch.rand(T, E, generator=g, device="cuda").topk(top, 1)[1].int()
+    assert seqmix.moe_grouped(h, idx, w_gu, w_down, "relu2", None)
+    got = seqmix.moe_experts(h, idx, w_gu, w_down, 0.0, "relu2")
+    for e in range(E):
+        t, k = (idx == e).nonzero(as_tuple=True)
+        want = torch.relu(h[t].double() @ w_gu[e].double().t()) ** 2 @ w_down[e].double().t()
+        assert (got[t, k].double() - want).norm() < TOL * want.norm()
+
+
+@gpu
 @pytest.mark.parametrize("act,T,top,E,W,ff", [("glu_clamp", 5200, 3, 7, 960, 1088), ("silu_glu", 5200, 3, 7, 960, 1088),
                                               ("relu2", 10200, 2, 5, 2048, 2048)])
 def test_tall_tiles(act, T, top, E, W, ff):
