@@ -125,10 +125,14 @@ class PagedCache:
         if need > 0:
             first = len(own)
             own.extend(self.free_pages.pop() for _ in range(need))
-            ids = torch.tensor(own[first:], dtype=torch.int32)
-            if self.page_table.is_cuda:                     # from pinned memory: a copy in stream order that nobody waits for
-                ids = ids.pin_memory()
-            self.page_table[slot, first:len(own)].copy_(ids, non_blocking=True)
+            # every run of consecutive ids is one launch that carries its numbers itself: nobody waits for a copy, and no pinned
+            # memory is asked for.  A scattered list goes as a copy
+            cuts = [first] + [i for i in range(first + 1, len(own)) if own[i] != own[i - 1] + 1] + [len(own)]
+            if len(cuts) <= 5:
+                for i, j in zip(cuts, cuts[1:]):
+                    torch.arange(own[i], own[i] + j - i, out=self.page_table[slot, i:j])
+            else:
+                self.page_table[slot, first:len(own)] = torch.tensor(own[first:], dtype=torch.int32)
         self.lens[slot] = max(self.lens[slot], new_len)
 
     def release(self, slot: int) -> None:
