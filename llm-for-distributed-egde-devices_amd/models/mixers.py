@@ -56,13 +56,16 @@ class WindowPoolAttention(nn.Module):
             self._rope = tab
         return self._rope
 
-    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
-        """``u`` columns [c0, ..) hold q | k | v | gate.  Returns the o-projection's output [T, W]."""
+    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, q: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """``u`` columns [c0, ..) hold q | k | v | gate; ``q``: the rotated queries, when they and the cached rows and block means
+        are there already.  Returns the o-projection's output [T, W]."""
         s = self.spec
         nq, nk, nv, ng = s.proj_sizes
-        proj = u[:, c0:c0 + nq + nk + nv]
-        q = seqmix.rope_paged_write(proj, meta, self.rope(meta.max_keys, u.device), run.k, run.v, s.heads, s.rot_dims)
-        if s.window is not None and s.pool:
+        written = q is not None
+        if not written:
+            proj = u[:, c0:c0 + nq + nk + nv]
+            q = seqmix.rope_paged_write(proj, meta, self.rope(meta.max_keys, u.device), run.k, run.v, s.heads, s.rot_dims)
+        if s.window is not None and s.pool and not written:
             seqmix.pool_blocks(run.k, run.v, run.k_pool, run.v_pool, meta, s.pool)
         gate = u[:, c0 + nq + nk + nv:c0 + nq + nk + nv + ng] if ng else None
         a = seqmix.window_pool_attention(q, gate, run.k, run.v, run.k_pool, run.v_pool, meta, s.scale, s.window,
@@ -86,11 +89,12 @@ class SSDMixer(nn.Module):
         self.norm_w = P(spec.inner)
         self.o = Linear(spec.inner, width, False, dtype, device)
 
-    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
-        """``u`` columns [c0, ..) hold z | x | B | C | dt."""
+    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, xbc: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """``u`` columns [c0, ..) hold z | x | B | C | dt; ``xbc``: the convolved x | B | C rows, when they are there already."""
         s = self.spec
         inner, C = s.inner, s.conv_channels
-        xbc = seqmix.conv_silu(u, c0 + inner, C, self.conv_w, self.conv_b, run.conv, meta)
+        if xbc is None:
+            xbc = seqmix.conv_silu(u, c0 + inner, C, self.conv_w, self.conv_b, run.conv, meta)
         y = seqmix.ssd_scan(xbc, u, c0 + inner + C, self.dt_bias, self.A_log, self.D, run.ssm, meta, s.heads, s.vdim,
                             s.state, s.groups)
         g = seqmix.gated_group_norm(y, u[:, c0:c0 + inner], self.norm_w, s.norm_groups, self.eps, u.dtype)
@@ -114,11 +118,18 @@ class ParallelMixer(nn.Module):
     def in_rows(self) -> int:
         return sum(self.left.spec.proj_sizes) + self.right.spec.in_size
 
-    def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None):
+    def step_in(self, u: torch.Tensor, meta, run, f0: int, ff: int):
+        """(rotated queries, x | B | C rows, squared ReLU of ff columns from f0) of a decode step, formed in one launch; or None."""
+        a, s = self.left.spec, self.right.spec
+        return seqmix.parallel_step_in(u, meta, self.left.rope(meta.max_keys, u.device), run.k, run.v, run.k_pool, run.v_pool, a.heads,
+                                       a.rot_dims, a.pool if a.window is not None and a.pool else 0, sum(a.proj_sizes) + s.inner,
+                                       self.right.conv_w, self.right.conv_b, run.conv, f0, ff)
+
+    def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None, pre=(None, None)):
         """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra.  ``nxt``: the norm that reads x next; its rows
-        (of u's dtype) come back in x's place."""
-        a = self.left(u, 0, meta, run)
-        r = self.right(u, sum(self.left.spec.proj_sizes), meta, run)
+        (of u's dtype) come back in x's place.  ``pre``: ``step_in``'s first two results."""
+        a = self.left(u, 0, meta, run, pre[0])
+        r = self.right(u, sum(self.left.spec.proj_sizes), meta, run, pre[1])
         if nxt is not None:
             return seqmix.combine_residual_norm(x, a, r, self.left_out, self.right_out, self.eps, extra, nxt.weight, nxt.eps, u.dtype)
         return seqmix.combine_residual(x, a, r, self.left_out, self.right_out, self.eps, extra)

@@ -33,6 +33,10 @@ int edge_sm_delta_step(const void* u, int ld, int b0, int a0, int z0, const void
                        const float* conv_w, const float* conv_b, void* tail, float* state, const float* dt_bias, const float* A_log,
                        const float* norm_w, const int* seq_slot, const int* seq_start, const int* seq_off, void* out, int n, int H, int N,
                        int P, float eps, int f32, hipStream_t st);
+int edge_sm_parallel_in(const void* u, int ld, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
+                        int ptab_ld, const float* cs, void* q, void* kp, void* vp, float* kb, float* vb, int H, int G, int D, int Dv,
+                        int rot, int page, int PB, int pool, int c0, int C, const float* conv_w, const float* conv_b, void* tail,
+                        void* xbc, int f0, int F, void* act, int rows, int f32, hipStream_t st);
 int edge_sm_group_norm(const float* x, const float* w, void* y, int rows, int W, int groups, float eps, int f32,
                        hipStream_t st);
 int edge_sm_group_norm_residual(float* x, const void* y, const void* parts, const float* pw, int K, const float* w,
@@ -306,6 +310,55 @@ at::Tensor sm_rope_write(const at::Tensor& proj, const at::Tensor& tok_seq, cons
                            vpo ? vpo->data_ptr() : nullptr, (int)T,
                            (int)H, (int)G, (int)D, (int)Dv, (int)rot, (int)page, f32(proj), stream()), "sm_rope_write");
   return q;
+}
+
+// A parallel layer's parts between its input projection and its attention and recurrence (parallel_step.hip): (rotated q, x | B | C
+// rows, squared ReLU of F columns), one token per sequence; nothing comes back, and nothing was done, where the row does not fit
+std::optional<std::tuple<at::Tensor, at::Tensor, at::Tensor>> sm_parallel_in(
+    const at::Tensor& u, const at::Tensor& tok_seq, const at::Tensor& tok_pos, const at::Tensor& seq_slot, const at::Tensor& ptab,
+    const std::optional<at::Tensor>& rope, at::Tensor& kp, at::Tensor& vp, const std::optional<at::Tensor>& kb,
+    const std::optional<at::Tensor>& vb, int64_t H, int64_t rot, int64_t pool, int64_t c0, const at::Tensor& conv_w,
+    const at::Tensor& conv_b, at::Tensor& tail, int64_t f0, int64_t F) {
+  const int ld = row_ld(u, "u");
+  for (const at::Tensor* t : {&tok_seq, &tok_pos, &seq_slot}) chk_i32(*t, "metadata");
+  chk_table(ptab);
+  chk_f32(conv_w, "conv weight");
+  chk_f32(conv_b, "conv bias");
+  TORCH_CHECK(is_act(u) && kp.is_cuda() && kp.is_contiguous() && kp.dim() == 4 && kp.scalar_type() == u.scalar_type() && vp.is_cuda() &&
+                  vp.is_contiguous() && vp.dim() == 4 && vp.scalar_type() == u.scalar_type() && vp.size(0) == kp.size(0) &&
+                  vp.size(1) == kp.size(1) && vp.size(2) == kp.size(2), "pages: [pages, page, G, D] in u's dtype");
+  const int64_t T = u.size(0), page = kp.size(1), G = kp.size(2), D = kp.size(3), Dv = vp.size(3), C = conv_w.size(0);
+  TORCH_CHECK(tok_seq.numel() == T && tok_pos.numel() == T, "one token per sequence");
+  TORCH_CHECK(H * D + G * (D + Dv) <= c0 && c0 + C <= f0 && f0 + F <= u.size(1) && conv_b.numel() == C, "columns of u");
+  int PB = 0;
+  if (pool > 0) {
+    TORCH_CHECK(kb && vb, "pooled entries missing");
+    chk_f32(*kb, "k_pool");
+    chk_f32(*vb, "v_pool");
+    PB = (int)kb->size(1);
+    TORCH_CHECK(kb->dim() == 4 && vb->dim() == 4 && kb->size(0) == kp.size(0) && PB == (page + pool - 1) / pool && kb->size(2) == G &&
+                    kb->size(3) == D && vb->size(0) == kp.size(0) && vb->size(1) == PB && vb->size(2) == G && vb->size(3) == Dv,
+                "pooled entries: [pages, ceil(page / pool), G, D]");
+  }
+  if (rot > 0) {
+    TORCH_CHECK(rope, "rotary table missing");
+    chk_f32(*rope, "rope");
+    TORCH_CHECK(rope->dim() == 3 && rope->size(1) * 2 == rot && rope->size(2) == 2, "rope: fp32 [positions, rot / 2, 2]");
+  }
+  if (conv_w.dim() != 2 || conv_w.size(1) != 4) return std::nullopt;
+  TORCH_CHECK(tail.is_cuda() && tail.is_contiguous() && tail.scalar_type() == u.scalar_type() && tail.dim() == 3 && tail.size(1) == 3 &&
+                  tail.size(2) == C, "tail: [slots, 3, C]");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(u.device());
+  auto q = at::empty({T, H, D}, u.options()), xbc = at::empty({T, C}, u.options()), act = at::empty({T, F}, u.options());
+  const int rc = edge_sm_parallel_in(u.data_ptr(), ld, tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(),
+                                     ptab.data_ptr<int>(), (int)ptab.stride(0), rot > 0 ? rope->data_ptr<float>() : nullptr,
+                                     q.data_ptr(), kp.data_ptr(), vp.data_ptr(), PB ? kb->data_ptr<float>() : nullptr,
+                                     PB ? vb->data_ptr<float>() : nullptr, (int)H, (int)G, (int)D, (int)Dv, (int)rot, (int)page, PB,
+                                     PB ? (int)pool : 0, (int)c0, (int)C, conv_w.data_ptr<float>(), conv_b.data_ptr<float>(),
+                                     tail.data_ptr(), xbc.data_ptr(), (int)f0, (int)F, act.data_ptr(), (int)T, f32(u), stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_parallel_in");
+  return std::make_tuple(q, xbc, act);
 }
 
 void sm_pool_blocks(const at::Tensor& kp, const at::Tensor& vp, at::Tensor& kb, at::Tensor& vb,
@@ -1520,6 +1573,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_combine", &sm_combine);
   m.def("sm_gated_norm", &sm_gated_norm);
   m.def("sm_rope_write", &sm_rope_write);
+  m.def("sm_parallel_in", &sm_parallel_in);
   m.def("sm_pool_blocks", &sm_pool_blocks);
   m.def("sm_attention", &sm_attention);
   m.def("sm_conv_silu", &sm_conv_silu);

@@ -246,6 +246,19 @@ def pool_blocks(k_pages, v_pages, k_pool, v_pool, meta: RaggedMeta, pool: int) -
             b += 1
 
 
+def parallel_step_in(u: torch.Tensor, meta: RaggedMeta, rope: Optional[torch.Tensor], k_pages, v_pages, k_pool, v_pool, heads: int,
+                     rot_dims: int, pool: int, c0: int, conv_w: torch.Tensor, conv_b: torch.Tensor, tail: torch.Tensor, f0: int, F_: int):
+    """What a parallel layer forms from its input projection's rows u in steps in which every sequence brings one token, in one
+    launch: ``rope_paged_write`` of the first columns (and ``pool_blocks`` where ``pool``), ``conv_silu`` of the columns from c0
+    and ``relu2`` of F_ columns from f0 -> (q, x | B | C rows, squared ReLU).  None where it is not one launch: nothing has been
+    done then."""
+    if not _gpu(u) or meta.max_len != 1 or meta.T != meta.n:
+        return None
+    return _ext().sm_parallel_in(u, meta.tok_seq, meta.tok_pos, meta.seq_slot, meta.page_table, rope if rot_dims else None, k_pages,
+                                 v_pages, k_pool if pool else None, v_pool if pool else None, int(heads), int(rot_dims), int(pool), int(c0),
+                                 conv_w, conv_b, tail, int(f0), int(F_))
+
+
 ATTN_MFMA_MIN = int(__import__("os").environ.get("EDGELLM_ATTN_MFMA_MIN", "16"))
 
 
