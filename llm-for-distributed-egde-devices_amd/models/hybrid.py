@@ -88,14 +88,9 @@ class HybridLayer(nn.Module):
             h = self.norm1(x, self.proj_in.weight.dtype)
         u = self.proj_in(h)
         pre = self.mix.step_in(u, meta, run, self.mix.in_rows, self.ff)
-        if pre is None:
-            m = self.down(seqmix.relu2(u, self.mix.in_rows, self.ff)) if self.ff else None
-            pre = (None, None)
-        else:
-            m = self.down(pre[2]) if self.ff else None
-        if nxt is None:
-            return self.mix(x, u, meta, run, m, None, pre)
-        return x, self.mix(x, u, meta, run, m, nxt, pre)
+        m = self.down(seqmix.relu2(u, self.mix.in_rows, self.ff)) if self.ff and pre is None else None
+        y = self.mix(x, u, meta, run, m, nxt, pre, self.down)
+        return y if nxt is None else (x, y)
 
 
 class PostNormLayer(nn.Module):

@@ -291,6 +291,19 @@ def plain_linear(m: nn.Module) -> bool:
     return type(m) is Linear and m.bias is None and not (m._forward_hooks or m._forward_pre_hooks)
 
 
+def rows_together(xs, mods):
+    """The three projections ``mods[j](xs[j])`` of the same few rows in one launch, or each by itself."""
+    if all(plain_linear(m) and not m.split_k_out for m in mods) and all(x.dim() == 2 and x.is_contiguous() for x in xs):
+        ws = [m.weight for m in mods]
+        if all(ops.f32_rows_ok(x, w) for x, w in zip(xs, ws)):
+            return ops.ext().gemv_rows3(xs[0], ws[0], xs[1], ws[1], xs[2], ws[2], *(m.out_features for m in mods))
+        if xs[0].shape[0] <= 4 and all(ops.bf16_decode_mode(x, w) == 1 and w.dtype == xs[0].dtype and m.in_features % 64 == 0
+                                       and m.out_features % 16 == 0 for x, w, m in zip(xs, ws, mods)):
+            p = [m.packed_weight() for m in mods]
+            return ops.ext().gemv_rows3(xs[0], p[0], xs[1], p[1], xs[2], p[2], *(m.out_features for m in mods))
+    return tuple(m(x) for m, x in zip(mods, xs))
+
+
 class ScalarNorm(nn.Module):
     """RMS norm whose gain is one number for all coordinates: fp32 rows in (the residual stream of
     the layer-spec models), rows of the consumer's dtype out."""

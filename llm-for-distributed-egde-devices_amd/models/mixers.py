@@ -17,7 +17,7 @@ import torch.nn as nn
 
 from ..ops import seqmix
 from .configs import ChunkAttnSpec, DecayAttnSpec, DeltaSpec, GatedAttnSpec, GLASpec, LayerSpec, SSDSpec, WindowAttnSpec
-from .layers import Linear, plain_linear
+from .layers import Linear, plain_linear, rows_together
 
 
 _ROPE_TABLES: dict = {}
@@ -57,8 +57,11 @@ class WindowPoolAttention(nn.Module):
         return self._rope
 
     def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, q: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """``u`` columns [c0, ..) hold q | k | v | gate; ``q``: the rotated queries, when they and the cached rows and block means
-        are there already.  Returns the o-projection's output [T, W]."""
+        """``u`` columns [c0, ..) hold q | k | v | gate.  Returns the o-projection's output [T, W]."""
+        return self.o(self.heads(u, c0, meta, run, q))
+
+    def heads(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, q: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """The o-projection's input; ``q``: the rotated queries, when they and the cached rows and block means are there already."""
         s = self.spec
         nq, nk, nv, ng = s.proj_sizes
         written = q is not None
@@ -68,9 +71,8 @@ class WindowPoolAttention(nn.Module):
         if s.window is not None and s.pool and not written:
             seqmix.pool_blocks(run.k, run.v, run.k_pool, run.v_pool, meta, s.pool)
         gate = u[:, c0 + nq + nk + nv:c0 + nq + nk + nv + ng] if ng else None
-        a = seqmix.window_pool_attention(q, gate, run.k, run.v, run.k_pool, run.v_pool, meta, s.scale, s.window,
-                                         s.pool if s.window is not None else None)
-        return self.o(a)
+        return seqmix.window_pool_attention(q, gate, run.k, run.v, run.k_pool, run.v_pool, meta, s.scale, s.window,
+                                            s.pool if s.window is not None else None)
 
 
 class SSDMixer(nn.Module):
@@ -90,15 +92,18 @@ class SSDMixer(nn.Module):
         self.o = Linear(spec.inner, width, False, dtype, device)
 
     def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, xbc: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """``u`` columns [c0, ..) hold z | x | B | C | dt; ``xbc``: the convolved x | B | C rows, when they are there already."""
+        """``u`` columns [c0, ..) hold z | x | B | C | dt.  Returns the o-projection's output [T, W]."""
+        return self.o(self.rows(u, c0, meta, run, xbc))
+
+    def rows(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, xbc: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """The o-projection's input; ``xbc``: the convolved x | B | C rows, when they are there already."""
         s = self.spec
         inner, C = s.inner, s.conv_channels
         if xbc is None:
             xbc = seqmix.conv_silu(u, c0 + inner, C, self.conv_w, self.conv_b, run.conv, meta)
         y = seqmix.ssd_scan(xbc, u, c0 + inner + C, self.dt_bias, self.A_log, self.D, run.ssm, meta, s.heads, s.vdim,
                             s.state, s.groups)
-        g = seqmix.gated_group_norm(y, u[:, c0:c0 + inner], self.norm_w, s.norm_groups, self.eps, u.dtype)
-        return self.o(g)
+        return seqmix.gated_group_norm(y, u[:, c0:c0 + inner], self.norm_w, s.norm_groups, self.eps, u.dtype)
 
 
 class ParallelMixer(nn.Module):
@@ -125,11 +130,20 @@ class ParallelMixer(nn.Module):
                                        a.rot_dims, a.pool if a.window is not None and a.pool else 0, sum(a.proj_sizes) + s.inner,
                                        self.right.conv_w, self.right.conv_b, run.conv, f0, ff)
 
-    def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None, pre=(None, None)):
+    def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None, pre=None,
+                down: Optional[nn.Module] = None):
         """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra.  ``nxt``: the norm that reads x next; its rows
-        (of u's dtype) come back in x's place.  ``pre``: ``step_in``'s first two results."""
-        a = self.left(u, 0, meta, run, pre[0])
-        r = self.right(u, sum(self.left.spec.proj_sizes), meta, run, pre[1])
+        (of u's dtype) come back in x's place.  ``pre``: ``step_in``'s results; with ``down``, extra is its output on the last."""
+        c0, watched = sum(self.left.spec.proj_sizes), any(m._forward_hooks or m._forward_pre_hooks for m in (self.left, self.right))
+        if pre is not None and down is not None and not watched:
+            extra, a, r = rows_together((pre[2], self.left.heads(u, 0, meta, run, pre[0]), self.right.rows(u, c0, meta, run, pre[1])),
+                                        (down, self.left.o, self.right.o))
+        else:
+            q, xbc, act = pre if pre is not None else (None, None, None)
+            if down is not None and pre is not None:
+                extra = down(act)
+            a = self.left(u, 0, meta, run, q)
+            r = self.right(u, c0, meta, run, xbc)
         if nxt is not None:
             return seqmix.combine_residual_norm(x, a, r, self.left_out, self.right_out, self.eps, extra, nxt.weight, nxt.eps, u.dtype)
         return seqmix.combine_residual(x, a, r, self.left_out, self.right_out, self.eps, extra)

@@ -92,6 +92,8 @@ int edge_w8a8_rows256_splits(int K);
 void edge_w8a8_prefill_x32(int v);
 int edge_gemv_bf16(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi,
                    hipStream_t st, const void* add, int h16);
+int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K, hipStream_t st);
+int edge_rows3(const void* const* x, const void* const* w, void* const* y, const int* N, const int* K, int M, int h16, hipStream_t st);
 int edge_gemv_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K, hipStream_t st);
 int edge_gemv_bf16_splitk(const void* A, const void* W, const void* bias, float* part, int M, int N, int K, int S,
                           hipStream_t st, int h16);
@@ -830,6 +832,45 @@ at::Tensor gemv_f32(const at::Tensor& x, const at::Tensor& w, const std::optiona
   check(edge_gemv_f32(x.data_ptr<float>(), w.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr,
                       out.data_ptr<float>(), (int)M, (int)N, (int)K, stream()), "gemv_f32");
   return out;
+}
+
+// Three projections of the same rows in one launch: fp32 x_j [M <= 8, K_j] over weights [N_j, K_j] as they are, or 16 bits, M <= 4,
+// over packed weights of N_j K_j numbers.
+std::tuple<at::Tensor, at::Tensor, at::Tensor> gemv_rows3(const at::Tensor& x0, const at::Tensor& w0, const at::Tensor& x1,
+                                                          const at::Tensor& w1, const at::Tensor& x2, const at::Tensor& w2,
+                                                          int64_t n0, int64_t n1, int64_t n2) {
+  DEVICE_GUARD(x0);
+  const at::Tensor *x[3] = {&x0, &x1, &x2}, *w[3] = {&w0, &w1, &w2};
+  const int64_t nn[3] = {n0, n1, n2}, M = x0.size(0);
+  const bool f = x0.scalar_type() == at::kFloat;
+  const int h16 = f ? 0 : need16(x0, "x");
+  at::Tensor y[3];
+  int N[3], K[3];
+  for (int j = 0; j < 3; ++j) {
+    if (f) need(*x[j], at::kFloat, "x");
+    else need_same(*x[j], x0, "x");
+    if (f) need(*w[j], at::kFloat, "weight");
+    else need_same(*w[j], x0, "weight (packed)");
+    TORCH_CHECK(x[j]->dim() == 2 && x[j]->size(0) == M && w[j]->device() == x0.device() && x[j]->device() == x0.device(),
+                "x_j [M, K_j], one device");
+    N[j] = (int)nn[j];
+    K[j] = (int)x[j]->size(1);
+    TORCH_CHECK(N[j] > 0 && K[j] > 0 && w[j]->numel() == nn[j] * K[j] && (uintptr_t)x[j]->data_ptr() % 16 == 0 &&
+                    (uintptr_t)w[j]->data_ptr() % 16 == 0, "weights of N_j K_j numbers, 16-byte aligned operands");
+    y[j] = at::empty({M, nn[j]}, x0.options());
+  }
+  if (f) {
+    const float *xp[3], *wp[3];
+    float* yp[3];
+    for (int j = 0; j < 3; ++j) { xp[j] = x[j]->data_ptr<float>(); wp[j] = w[j]->data_ptr<float>(); yp[j] = y[j].data_ptr<float>(); }
+    check(edge_gemv_f32x3(xp, wp, yp, (int)M, N, K, stream()), "gemv_rows3");
+  } else {
+    const void *xp[3], *wp[3];
+    void* yp[3];
+    for (int j = 0; j < 3; ++j) { xp[j] = x[j]->data_ptr(); wp[j] = w[j]->data_ptr(); yp[j] = y[j].data_ptr(); }
+    check(edge_rows3(xp, wp, yp, N, K, (int)M, h16, stream()), "gemv_rows3");
+  }
+  return {y[0], y[1], y[2]};
 }
 
 // Split-K bf16 decode GEMV: fp32 partial slices [S, M, N] (bias in slice 0) for rms_norm_parts.
@@ -1590,6 +1631,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("N"), py::arg("epi"), py::arg("y_out"), py::arg("x2") = py::none(), py::arg("gamma2") = py::none(),
         py::arg("beta2") = py::none());
   m.def("decode_attn_up", &decode_attn_up, "decode attention beside the up projection of a parallel-residual block (M <= 4)");
+  m.def("gemv_rows3", &gemv_rows3, "three projections of the same rows in one launch (fp32 M <= 8, 16 bits M <= 4)");
   m.def("decode_o_down", &decode_o_down, "o beside the down projection of a parallel-residual block (M <= 4)");
   m.def("w8a8_gemv_ln", &w8a8_gemv_ln, "W8A8 decode GEMV with the LayerNorm + int8 quant in its prologue (M <= 4)");
   m.def("llmint8_gemv", &llmint8_gemv, "LLM.int8 projection of one row in one launch (prep in the GEMV prologue)");

@@ -30,6 +30,15 @@ __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act
   else gemv_bf16_body<PW, 1, 1, 2, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
 }
 
+// Three projections of the same rows (a parallel layer of attention, recurrence and feed-forward); d first, its chains are the
+// longest.  us in a graph, bf16, three launches / one, 1024 x 4096 and twice 1024 x 1024: 1 row 13.1 / 6.5, 4 rows 14.1 / 7.1; 2048 x
+// 8192 and twice 2048 x 2048 19.8 / 12.3, 22.7 / 14.7.
+template <bool HF>
+__global__ void __launch_bounds__(PW * 64, 4) rows3_kernel(Proj d, Proj o, Proj r, int M) {
+  const int nd = d.N / 16, no = nd + o.N / 16, bid = blockIdx.x;
+  proj_body<EPI_OUT, HF>(bid < nd ? bid : bid < no ? bid - nd : bid - no, bid < nd ? d : bid < no ? o : r, M, 0);
+}
+
 template <int D, bool DIRECT, bool HF>
 __global__ void __launch_bounds__(PW * 64, 4) attn_up_kernel(AttnArgs a, Proj p, int M, int act, int na) {
   __shared__ __attribute__((aligned(16))) float smem[attn_part_lds<D>()];
@@ -95,5 +104,21 @@ extern "C" int edge_o_down(const void* x, const void* wo, const void* bo, void* 
   const dim3 grid(2 * (N / 16)), block(PW * 64);
   if (h16) hipLaunchKernelGGL(o_down_kernel<true>, grid, block, 0, st, o, d, M);
   else hipLaunchKernelGGL(o_down_kernel<false>, grid, block, 0, st, o, d, M);
+  return (int)hipGetLastError();
+}
+
+// y_j = x_j . W_j^T (x_j [M, K_j], packed weights), M <= 4 rows of N_j numbers, j = 0 .. 2.  -2: not taken.
+extern "C" int edge_rows3(const void* const* x, const void* const* w, void* const* y, const int* N, const int* K, int M, int h16,
+                          hipStream_t st) {
+  Proj p[3];
+  int blocks = 0;
+  for (int j = 0; j < 3; ++j) {
+    if (N[j] <= 0 || N[j] % 16 != 0 || K[j] <= 0 || K[j] % 64 != 0) return -2;
+    p[j] = Proj{(const bf16_t*)x[j], (const bf16_t*)w[j], nullptr, (bf16_t*)y[j], N[j], K[j]};
+    blocks += N[j] / 16;
+  }
+  if (M < 1 || M > 4) return -2;
+  if (h16) hipLaunchKernelGGL(rows3_kernel<true>, dim3(blocks), dim3(PW * 64), 0, st, p[0], p[1], p[2], M);
+  else hipLaunchKernelGGL(rows3_kernel<false>, dim3(blocks), dim3(PW * 64), 0, st, p[0], p[1], p[2], M);
   return (int)hipGetLastError();
 }

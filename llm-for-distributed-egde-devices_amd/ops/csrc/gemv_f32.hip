@@ -12,13 +12,12 @@
 namespace {
 
 template <int MV, int R>
-__global__ void __launch_bounds__(1024) gemv_f32_kernel(const float* __restrict__ x, const float* __restrict__ W,
-                                                        const float* __restrict__ bias, float* __restrict__ y, int M, int N,
-                                                        int K, int KW) {
+__device__ __forceinline__ void gemv_f32_body(int bid, const float* __restrict__ x, const float* __restrict__ W,
+                                              const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K, int KW) {
   constexpr int V = MV * R;
   __shared__ float part[16 * V];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
-  const int rg = wave / KW, kw = wave - rg * KW, n0 = ((int)blockIdx.x * (waves / KW) + rg) * R;
+  const int rg = wave / KW, kw = wave - rg * KW, n0 = (bid * (waves / KW) + rg) * R;
   const int C = (K + 255) / 256;
   float acc[V];
 #pragma unroll
@@ -54,7 +53,7 @@ __global__ void __launch_bounds__(1024) gemv_f32_kernel(const float* __restrict_
   if (lane % (64 / V) == 0) part[wave * V + idx] = acc[0];
   __syncthreads();
   for (int e = tid; e < waves / KW * V; e += blockDim.x) {
-    const int gq = e / V, v = e - gq * V, m = v % MV, n = ((int)blockIdx.x * (waves / KW) + gq) * R + v / MV;
+    const int gq = e / V, v = e - gq * V, m = v % MV, n = (bid * (waves / KW) + gq) * R + v / MV;
     float sum = 0.f;
     for (int w = 0; w < KW; ++w) sum += part[(gq * KW + w) * V + v];
     if (m < M && n < N) y[(size_t)m * N + n] = sum + (bias ? bias[n] : 0.f);
@@ -62,14 +61,72 @@ __global__ void __launch_bounds__(1024) gemv_f32_kernel(const float* __restrict_
 }
 
 template <int MV, int R>
-void launch_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K, hipStream_t st) {
-  const int groups = (N + R - 1) / R, C = (K + 255) / 256;
+__global__ void __launch_bounds__(1024) gemv_f32_kernel(const float* __restrict__ x, const float* __restrict__ W,
+                                                        const float* __restrict__ bias, float* __restrict__ y, int M, int N,
+                                                        int K, int KW) {
+  gemv_f32_body<MV, R>(blockIdx.x, x, W, bias, y, M, N, K, KW);
+}
+
+// three projections of M rows each, workgroups [0, n[0]), [n[0], n[1]), [n[1], ..) of the grid
+struct Jobs3 {
+  const float *x[3], *W[3];
+  float* y[3];
+  int N[3], K[3], KW[3], n[2];
+};
+template <int MV, int R>
+__global__ void __launch_bounds__(1024) gemv_f32x3_kernel(Jobs3 a, int M) {
+  const int bid = blockIdx.x, j = bid < a.n[0] ? 0 : bid < a.n[1] ? 1 : 2;
+  gemv_f32_body<MV, R>(bid - (j == 0 ? 0 : a.n[j - 1]), a.x[j], a.W[j], nullptr, a.y[j], M, a.N[j], a.K[j], a.KW[j]);
+}
+
+// waves of a workgroup that share a row's k
+int share_k(int groups, int K) {
+  const int C = (K + 255) / 256;
   int KW = 1;
   while (KW < 16 && KW * 2 <= C && groups * KW < 1024) KW *= 2;
+  return KW;
+}
+
+template <int MV, int R>
+void launch_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K, hipStream_t st) {
+  const int groups = (N + R - 1) / R, KW = share_k(groups, K);
   const int waves = KW < 4 ? 4 : KW, per = waves / KW;
   hipLaunchKernelGGL((gemv_f32_kernel<MV, R>), dim3((groups + per - 1) / per), dim3(waves * 64), 0, st, x, W, bias, y, M, N, K, KW);
 }
+
+template <int MV, int R>
+void launch_f32x3(Jobs3 a, int M, hipStream_t st) {
+  int waves = 4, blocks = 0;
+  for (int j = 0; j < 3; ++j) {
+    a.KW[j] = share_k((a.N[j] + R - 1) / R, a.K[j]);
+    waves = a.KW[j] > waves ? a.KW[j] : waves;
+  }
+  for (int j = 0; j < 3; ++j) {
+    const int per = waves / a.KW[j];
+    blocks += ((a.N[j] + R - 1) / R + per - 1) / per;
+    if (j < 2) a.n[j] = blocks;
+  }
+  hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R>), dim3(blocks), dim3(waves * 64), 0, st, a, M);
+}
 }  // namespace
+
+// y_j = x_j W_j^T for three projections of the same M rows' inputs, each as edge_gemv_f32 forms it: a parallel layer's three output
+// projections, whose launches' ramps and ends then overlap.  us in a graph, three launches / one, 1024 x 4096 and twice 1024 x
+// 1024: 1 row 11.9 / 7.1, 2 12.6 / 7.5, 8 14.8 / 9.5; 2048 x 8192 and twice 2048 x 2048, 2 rows 27.0 / 22.1
+extern "C" int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K,
+                               hipStream_t st) {
+  Jobs3 a{};
+  for (int j = 0; j < 3; ++j) {
+    if (N[j] < 1 || K[j] < 4 || K[j] % 4) return -2;
+    a.x[j] = x[j]; a.W[j] = W[j]; a.y[j] = y[j]; a.N[j] = N[j]; a.K[j] = K[j];
+  }
+  if (M < 1 || M > 8) return -2;
+  if (M == 1) launch_f32x3<1, 4>(a, M, st);
+  else if (M == 2) launch_f32x3<2, 4>(a, M, st);
+  else if (M <= 4) launch_f32x3<4, 4>(a, M, st);
+  else launch_f32x3<8, 2>(a, M, st);
+  return (int)hipGetLastError();
+}
 
 // x, W: 16-byte aligned.  5 - 8 rows: two weight rows per wave (four leave no registers for the next loads: 4096 x 1024 at
 // 8 rows, launched one by one, 13.7 us, two 7.9, library 11.6)
