@@ -37,6 +37,9 @@ int edge_sm_parallel_in(const void* u, int ld, const int* tok_seq, const int* to
                         int ptab_ld, const float* cs, void* q, void* kp, void* vp, float* kb, float* vb, int H, int G, int D, int Dv,
                         int rot, int page, int PB, int pool, int c0, int C, const float* conv_w, const float* conv_b, void* tail,
                         void* xbc, int f0, int F, void* act, int rows, int f32, hipStream_t st);
+int edge_sm_ssd_step(const void* xbc, int Cx, const void* u, int ld, int dt0, const float* dt_bias, const float* A_log, const float* D,
+                     float* state, const int* seq_slot, const int* seq_start, const int* seq_off, float* y, int n, int H, int P, int N,
+                     int groups, int f32, hipStream_t st);
 int edge_sm_group_norm(const float* x, const float* w, void* y, int rows, int W, int groups, float eps, int f32,
                        hipStream_t st);
 int edge_sm_group_norm_residual(float* x, const void* y, const void* parts, const float* pw, int K, const float* w,
@@ -522,7 +525,7 @@ at::Tensor sm_conv_silu(const at::Tensor& u, int64_t c0, int64_t C, const at::Te
 at::Tensor sm_ssd_scan(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, const at::Tensor& dt_bias,
                        const at::Tensor& A_log, const at::Tensor& D, at::Tensor& state, const at::Tensor& seq_slot,
                        const at::Tensor& seq_start, const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n,
-                       int64_t Hs, int64_t P, int64_t N, int64_t groups, int64_t chunks, int64_t max_chunks) {
+                       int64_t Hs, int64_t P, int64_t N, int64_t groups, int64_t chunks, int64_t max_chunks, bool one) {
   const int ld = row_ld(u, "u");
   chk_f32(dt_bias, "dt_bias");
   chk_f32(A_log, "A_log");
@@ -552,6 +555,17 @@ at::Tensor sm_ssd_scan(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, 
                               (int)n, (int)max_chunks, (int)Hs, (int)P, (int)N, (int)groups, f32(xbc), stream()),
           "sm_ssd_chunked");
     return y;
+  }
+  if (one) {                                                 // every sequence brings one token
+    TORCH_CHECK(xbc.size(0) == n, "one row per sequence");
+    const int rc = edge_sm_ssd_step(xbc.data_ptr(), (int)xbc.size(1), u.data_ptr(), ld, (int)dt0, dt_bias.data_ptr<float>(),
+                                    A_log.data_ptr<float>(), D.data_ptr<float>(), state.data_ptr<float>(), seq_slot.data_ptr<int>(),
+                                    seq_start.data_ptr<int>(), seq_off.data_ptr<int>(), y.data_ptr<float>(), (int)n, (int)Hs, (int)P,
+                                    (int)N, (int)groups, f32(xbc), stream());
+    if (rc != -2) {
+      check(rc, "sm_ssd_step");
+      return y;
+    }
   }
   check(edge_sm_ssd_scan(xbc.data_ptr(), (int)xbc.size(1), u.data_ptr(), ld, (int)dt0, dt_bias.data_ptr<float>(),
                          A_log.data_ptr<float>(), D.data_ptr<float>(), state.data_ptr<float>(), seq_slot.data_ptr<int>(),

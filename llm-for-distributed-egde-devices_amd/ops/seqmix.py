@@ -437,14 +437,14 @@ def ssd_scan(xbc: torch.Tensor, u: torch.Tensor, dt0: int, dt_bias, A_log, D, st
     inner = heads * vdim
     if _gpu(xbc):
         # portions of SSD_CHUNK_MIN tokens or more: the chunked (state-space duality) kernels, parallel
-        # over chunks of 64 tokens; shorter steps (decode): one wave per (sequence, head) token by token
+        # over chunks of 64 tokens; one token per sequence: four waves per (sequence, head); other short steps: one wave, token by token
         chunks = max_chunks = 0
         if meta.max_len >= SSD_CHUNK_MIN:
             per = [(h[2] + 63) // 64 for h in meta.host]
             chunks, max_chunks = sum(per), max(per)
         return _ext().sm_ssd_scan(xbc, u, int(dt0), dt_bias, A_log, D, state, meta.seq_slot, meta.seq_start,
                                   meta.seq_len, meta.seq_off, int(meta.n), int(heads), int(vdim), int(N), int(groups),
-                                  int(chunks), int(max_chunks))
+                                  int(chunks), int(max_chunks), meta.max_len == 1 and meta.T == meta.n)
     T = xbc.shape[0]
     y = torch.empty(T, inner, dtype=torch.float32, device=xbc.device)
     a = torch.exp(A_log.float())

@@ -65,3 +65,26 @@ def test_what_stays_apart():
     assert call(u, one, 3) is None                                            # three taps
     assert call(u, S.RaggedMeta.build([(0, 0, 2)], table, PAGE, "cuda")) is None
     assert call(torch.randn(2, 105, device="cuda")[:, 1:], one) is None       # rows that do not lie on 16 bytes
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,P,N,groups", [(4, 64, 64, 1), (6, 64, 128, 3), (2, 128, 64, 2), (3, 128, 128, 1), (2, 32, 64, 1), (4, 64, 60, 2)])
+def test_recurrence_of_one_token(dt, H, P, N, groups):
+    """ssd_step.hip's state sizes and others, three steps in a row, positions 0 and later, step sizes on both sides of 20."""
+    g = torch.Generator().manual_seed(H + P + N)
+    n, inner = 5, H * P
+    r = lambda *s: torch.randn(*s, generator=g)
+    bias, A_log, D = r(H), r(H) * 0.3, r(H)
+    bias[0] = 21.0
+    state = r(n + 1, H, N, P)
+    dev_state, ref_state = state.cuda(), state.clone()
+    table = torch.zeros(n + 1, 1, dtype=torch.int32)
+    slots = torch.randperm(n + 1, generator=g)[:n].tolist()
+    for i in range(3):
+        xbc, u = r(n, inner + 2 * groups * N).to(dt), r(n, H + 3).to(dt)
+        seqs = [(s, j * 3 + i, 1) for j, s in enumerate(slots)]
+        got = S.ssd_scan(xbc.cuda(), u.cuda(), 3, bias.cuda(), A_log.cuda(), D.cuda(), dev_state, S.RaggedMeta.build(seqs, table.cuda(), PAGE, "cuda"), H, P, N, groups)
+        ref = S.ssd_scan(xbc, u, 3, bias, A_log, D, ref_state, S.RaggedMeta.build(seqs, table, PAGE, "cpu"), H, P, N, groups)
+        # fp32 on both sides: sums of N products in another order, device exponentials
+        assert (got.cpu() - ref).abs().max() <= 2e-5 * ref.abs().max()
+        assert (dev_state.cpu() - ref_state).abs().max() <= 2e-5 * ref_state.abs().max()
