@@ -121,10 +121,14 @@ class PostNormLayer(nn.Module):
         return (self.canon1, run.canon1) if self.canon1 is not None else None
 
     def _join(self, norm, x, meta, nxt, y, parts=None, wts=None):
-        """x += the normed result; the next sublayer's convolved rows where ``nxt`` names its taps and state."""
+        """x += the normed result; the next sublayer's convolved rows where ``nxt`` names its taps and state, or the rows of the
+        norm that reads x next."""
         if nxt is None:
             norm.add_to(x, y, parts, wts)
             return None
+        if isinstance(nxt, RowLayerNorm):
+            return seqmix.layer_norm_residual_norm(x, y, norm.weight, norm.bias, norm.eps, parts, wts, nxt.weight, nxt.bias, nxt.eps,
+                                                   self.dtype)
         return seqmix.layer_norm_residual_canon(x, y, norm.weight, norm.bias, norm.eps, parts, wts, *nxt, meta, self.dtype)
 
     def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run, h: Optional[torch.Tensor] = None, nxt=None):
@@ -411,11 +415,16 @@ class HybridLM(nn.Module):
         """The LayerSpec of every run, in order (sizes the paged cache)."""
         return [self.cfg.layer_specs[i] for i, _ in self.runs]
 
-    def _next_read(self, r: int, cache):
+    # the final norm that a layer of each kind may form with its last residual sum
+    _LAST_READ = {HybridLayer: ScalarNorm, PostNormLayer: RowLayerNorm, SandwichLayer: GroupRMSNorm}
+
+    def _next_read(self, r: int, cache, last: bool):
         """``first_read()`` of run r + 1 where nothing comes between run r and it: both layers of one kind, nobody watching their
-        calls, no pass of a looped span that starts by changing the stream."""
+        calls, no pass of a looped span that starts by changing the stream.  ``last``: the final norm follows the last run."""
         if r + 1 >= len(self.runs):
-            return None
+            here = self.layers[self.runs[r][0]]
+            ok = last and type(self.final_norm) is self._LAST_READ.get(type(here)) and _unwatched(here) and _unwatched(self.final_norm)
+            return self.final_norm if ok else None
         i, t = self.runs[r + 1]
         loop, here, there = self.cfg.loop, self.layers[self.runs[r][0]], self.layers[i]
         if t is not None and i == loop.start and (loop.entry == "project" or (loop.entry == "add_embed" and t > 0)):
@@ -472,7 +481,7 @@ class HybridLM(nn.Module):
                 nxt = self.layers[self.runs[r + 1][0]].first_read() if r + 1 < len(self.runs) and cfg.loop is None else None
                 x, h_next = self.layers[i](x, meta, cache.run(r), h_next, nxt)
             else:                                        # the next layer's first input rides on this layer's residual sum
-                nxt = self._next_read(r, cache)
+                nxt = self._next_read(r, cache, rows is None and taps is None)
                 if nxt is None:
                     x, h_next = self.layers[i](x, meta, cache.run(r), h_next), None
                 else:
@@ -483,6 +492,8 @@ class HybridLM(nn.Module):
             if rows.numel() == 0:                        # nothing asked for: the step only fed the cache
                 return torch.empty(0, cfg.vocab_size, dtype=torch.float32, device=x.device)
             x = x.index_select(0, rows)
+        if h_next is not None:                           # the last layer formed the final norm with its residual sum
+            return self.lm_head(h_next)
         return self.lm_head(self.final_norm(x, None, self.dtype) if cfg.streams else self.final_norm(x, self.dtype))
 
 

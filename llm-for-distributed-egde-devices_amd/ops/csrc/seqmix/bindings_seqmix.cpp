@@ -24,6 +24,8 @@ int edge_sm_rope_write(const void* proj, int ld, const int* tok_seq, const int* 
 int edge_sm_ln_residual_taps(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b,
                              const float* cw, float* state, const int* tok_seq, const int* tok_pos, const int* seq_slot, void* out,
                              int rows, int W, float eps, int f32, hipStream_t st);
+int edge_sm_ln_residual_ln(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b, float eps,
+                           const float* w2, const float* b2, float eps2, void* out, int rows, int W, int f32, hipStream_t st);
 int edge_sm_group_residual_norm(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, int groups,
                                 float eps, float mult, const float* w2, int groups2, float eps2, void* out, int rows, int W, int f32,
                                 hipStream_t st);
@@ -719,6 +721,25 @@ std::optional<at::Tensor> sm_ln_residual_taps(at::Tensor& x, const std::optional
                                           (float)eps, r.is_f32, stream());
   if (rc == -2) return std::nullopt;
   check(rc, "sm_ln_residual_taps");
+  return out;
+}
+
+std::optional<at::Tensor> sm_ln_residual_ln(at::Tensor& x, const std::optional<at::Tensor>& y, const at::Tensor& w, const at::Tensor& b,
+                                            double eps, const std::optional<at::Tensor>& parts,
+                                            const std::optional<at::Tensor>& part_w, const at::Tensor& w2, const at::Tensor& b2,
+                                            double eps2, bool out_f32) {
+  for (const at::Tensor* f : {(const at::Tensor*)&x, &w, &b, &w2, &b2}) chk_f32(*f, "x, weights");
+  TORCH_CHECK(x.dim() == 2 && w.numel() == x.size(1) && b.numel() == x.size(1) && w2.numel() == x.size(1) && b2.numel() == x.size(1),
+              "x fp32 [T, W], weights [W]");
+  const Results r = results_of(x, y, parts, part_w);
+  if ((r.is_f32 != 0) != out_f32) return std::nullopt;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  auto out = at::empty({x.size(0), x.size(1)}, x.options().dtype(act_type(out_f32)));
+  const int rc = edge_sm_ln_residual_ln(x.data_ptr<float>(), r.y, r.parts, r.pw, r.K, w.data_ptr<float>(), b.data_ptr<float>(), (float)eps,
+                                        w2.data_ptr<float>(), b2.data_ptr<float>(), (float)eps2, out.data_ptr(), (int)x.size(0),
+                                        (int)x.size(1), r.is_f32, stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_ln_residual_ln");
   return out;
 }
 
@@ -1595,6 +1616,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_embed_bigram", &sm_embed_bigram);
   m.def("sm_canon", &sm_canon);
   m.def("sm_ln_residual_taps", &sm_ln_residual_taps);
+  m.def("sm_ln_residual_ln", &sm_ln_residual_ln);
   m.def("sm_group_residual_norm", &sm_group_residual_norm);
   m.def("sm_combine_norm", &sm_combine_norm);
   m.def("sm_layer_norm", &sm_layer_norm);

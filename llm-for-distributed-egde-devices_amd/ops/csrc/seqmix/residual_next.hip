@@ -1,7 +1,7 @@
-// A sublayer's result joins the fp32 residual stream and the row that the next sublayer reads is formed in the same launch, for the
-// three kinds of layers that do the two in a row: LayerNorm of the result, then the stream's four-tap convolution (steps in which
-// every sequence brings one token); group RMS norm of the result, then the next group RMS norm; the two branches of a parallel
-// mixer, then the next RMS norm.  (ops/seqmix.py has the rules; widths, types and addresses that do not fit run the separate
+// A sublayer's result joins the fp32 residual stream and the row that the next sublayer (or the output projection) reads is formed in
+// the same launch, for the three kinds of layers that do the two in a row: LayerNorm of the result, then the stream's four-tap
+// convolution (steps in which every sequence brings one token) or, behind the last layer, its LayerNorm; group RMS norm of the
+// result, then the next group RMS norm; the two branches of a parallel mixer, then the next RMS norm.  (ops/seqmix.py has the rules; widths, types and addresses that do not fit run the separate
 // kernels.)
 //
 // Bound by latency on decode-sized steps: each of the two launches was one chain of loads, a reduction over the row and a store, and
@@ -87,6 +87,60 @@ __global__ void __launch_bounds__(NT) ln_residual_taps_kernel(float* __restrict_
     store4<float>(st + c, tail[i][1]);
     store4<float>(st + W + c, tail[i][2]);
     store4<float>(st + 2 * (size_t)W + c, xv[i]);
+  }
+}
+
+// x += LayerNorm(y + sum_k pw[k] parts[k]) w + b;  out = LayerNorm(x) w2 + b2
+template <typename T, int CH>
+__global__ void __launch_bounds__(NT) ln_residual_ln_kernel(float* __restrict__ x, const T* __restrict__ y,
+                                                            const T* __restrict__ parts, const float* __restrict__ pw, int K,
+                                                            const float* __restrict__ w, const float* __restrict__ b, int W, float eps,
+                                                            const float* __restrict__ w2, const float* __restrict__ b2, float eps2,
+                                                            T* __restrict__ out) {
+  __shared__ float red[4][NT / 64];
+  const size_t t = blockIdx.x;
+  float v[CH][4], xv[CH][4], wv[CH][4], bv[CH][4], w2v[CH][4], b2v[CH][4];
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    const int c = col(i, W);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[i][e] = 0.f;
+    if (y) load4<T>(y + t * W + c, v[i]);
+    load4<float>(x + t * W + c, xv[i]);
+    load4<float>(w + c, wv[i]);
+    load4<float>(b + c, bv[i]);
+    load4<float>(w2 + c, w2v[i]);
+    load4<float>(b2 + c, b2v[i]);
+  }
+  add_parts<T, CH>(v, parts, pw, K, t, W);
+  auto norm = [&](float (&z)[CH][4], float* r0, float* r1, float e0, float& mean) {   // 1 / deviation
+    float sum = 0.f, ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+      if (in_row(i, W)) sum += (z[i][0] + z[i][1]) + (z[i][2] + z[i][3]);
+    mean = row_total(sum, r0) / (float)W;
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+      if (in_row(i, W))
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { const float d = z[i][e] - mean; ss += d * d; }
+    return 1.f / sqrtf(row_total(ss, r1) / (float)W + e0);
+  };
+  float mean;
+  const float r = norm(v, red[0], red[1], eps, mean);
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xv[i][e] += (v[i][e] - mean) * r * wv[i][e] + bv[i][e];
+    if (in_row(i, W)) store4<float>(x + t * W + col(i, W), xv[i]);
+  }
+  const float r2 = norm(xv, red[2], red[3], eps2, mean);
+#pragma unroll
+  for (int i = 0; i < CH; ++i) {
+    if (!in_row(i, W)) continue;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) xv[i][e] = (xv[i][e] - mean) * r2 * w2v[i][e] + b2v[i][e];
+    store4<T>(out + t * W + col(i, W), xv[i]);
   }
 }
 
@@ -222,7 +276,16 @@ bool row_ok(int W, std::initializer_list<const void*> ps) {
 
 extern "C" {
 
-// all three: -2 where the row does not fit
+// all of them: -2 where the row does not fit
+
+int edge_sm_ln_residual_ln(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b, float eps,
+                           const float* w2, const float* b2, float eps2, void* out, int rows, int W, int f32, hipStream_t st) {
+  if (!row_ok(W, {x, y, parts, w, b, w2, b2, out})) return -2;
+  if (rows == 0) return 0;
+  if (f32) RN_CH(ln_residual_ln_kernel, float, x, (const float*)y, (const float*)parts, pw, K, w, b, W, eps, w2, b2, eps2, (float*)out);
+  else RN_CH(ln_residual_ln_kernel, bf16_t, x, (const bf16_t*)y, (const bf16_t*)parts, pw, K, w, b, W, eps, w2, b2, eps2, (bf16_t*)out);
+  return (int)hipGetLastError();
+}
 
 int edge_sm_ln_residual_taps(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b,
                              const float* cw, float* state, const int* tok_seq, const int* tok_pos, const int* seq_slot, void* out,

@@ -545,6 +545,19 @@ def layer_norm_residual_canon(x: torch.Tensor, y: Optional[torch.Tensor], weight
     return canon_conv(x, canon, state, meta, out_dtype)
 
 
+def layer_norm_residual_norm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor, eps: float,
+                             parts: Optional[torch.Tensor], part_w: Optional[torch.Tensor], next_weight: torch.Tensor,
+                             next_bias: torch.Tensor, next_eps: float, out_dtype) -> torch.Tensor:
+    """``layer_norm_residual``, then ``layer_norm_rows`` of the new x (one launch where the row fits): returns the normed rows."""
+    if _gpu(x):
+        h = _ext().sm_ln_residual_ln(x, y, weight, bias, float(eps), parts, part_w, next_weight, next_bias, float(next_eps),
+                                     out_dtype == torch.float32)
+        if h is not None:
+            return h
+    layer_norm_residual(x, y, weight, bias, eps, parts, part_w)
+    return layer_norm_rows(x, next_weight, next_bias, next_eps, out_dtype)
+
+
 def _group_rms(v: torch.Tensor, groups: int, eps: float) -> torch.Tensor:
     T, W = v.shape
     g = v.view(T, groups, W // groups)

@@ -55,6 +55,20 @@ def test_layer_norm_then_taps(dt, W, T, K, with_y):
 
 
 @pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("W", [64, 256, 1020, 1028, 2048, 4096, 4100, 1022])
+@pytest.mark.parametrize("T,K,with_y", [(1, 0, True), (5, 3, True), (4, 5, False)])
+def test_layer_norm_then_layer_norm(dt, W, T, K, with_y):
+    g = torch.Generator().manual_seed(W + K)
+    x, w, b, w2, b2 = _rand(g, T, W), _rand(g, W), _rand(g, W), _rand(g, W), _rand(g, W)
+    y, parts, pw = _results(g, T, K, W, dt, with_y)
+    a, xa = x.cuda(), x.clone()
+    h = S.layer_norm_residual_norm(a, cuda(y), cuda(w), cuda(b), 1e-6, cuda(parts), cuda(pw), cuda(w2), cuda(b2), 1e-5, dt)
+    ref = S.layer_norm_residual_norm(xa, cpu(y), w, b, 1e-6, cpu(parts), pw, w2, b2, 1e-5, torch.float32)
+    _near(a, xa, torch.float32)
+    _near(h, ref, dt)
+
+
+@pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("W,groups,groups2", [(256, 1, 1), (1024, 4, 2), (1280, 1, 5), (2048, 2, 8), (2304, 3, 1), (4096, 16, 1), (1024, 8, 2), (96, 2, 3),
                                               (4352, 1, 17)])
 @pytest.mark.parametrize("T,K,with_y,with_w", [(1, 0, True, True), (7, 3, False, False), (3, 5, True, True)])
@@ -103,7 +117,7 @@ def test_watched_layers_give_the_same_logits(family, loop):
     res = []
     for watched in (False, True):
         hooks = [m.register_forward_hook(lambda *a: None) for m in model.modules() if m is not model] if watched else []
-        eng = RaggedEngine(model, 256, slots=2, page=16, use_graphs=False)
+        eng = RaggedEngine(model, 256, slots=2, page=16, use_graphs=not watched)     # (captured steps want every row)
         out = [eng.step([(0, list(range(5, 25)), [19]), (1, [7, 9], [1])])]
         for t in range(4):
             out.append(eng.step([(0, [t + 1], [0]), (1, [t + 3], [0])]))
