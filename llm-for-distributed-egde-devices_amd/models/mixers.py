@@ -215,9 +215,8 @@ class LatentAttention(nn.Module):
         else:
             q_lat = torch.bmm(q[:, :, :s.dim].transpose(0, 1), self.uk).transpose(0, 1)  # [T, H, kv_rank]
             qc = seqmix.latent_write(None, s.q_rank, None, self.eps, q, q_lat, meta, rope, run.lat, s.kv_rank, s.rot_dims)
-        a = seqmix.window_pool_attention(qc, None, run.lat, run.lat[..., :s.kv_rank], None, None, meta, s.scale,
-                                         s.window, None, self.sink)                     # [T, H * kv_rank]
-        return self.o(seqmix.head_expand_gate(a, self.uv, u[:, u.shape[1] - self.ng:] if self.ng else None, meta))
+        return self.o(seqmix.latent_attention(qc, run.lat, self.uv, u[:, u.shape[1] - self.ng:] if self.ng else None, meta, s.scale,
+                                              s.window, self.sink))
 
 
 class GatedAttention(nn.Module):

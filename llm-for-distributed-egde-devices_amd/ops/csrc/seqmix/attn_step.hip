@@ -32,7 +32,8 @@ struct StepArgs {
   void* out;
   float* part;
   const float *slopes, *sink, *rel;
-  int rows, gate_ld, ptab_ld, H, G, D, Dv, page, page_sh, PB, window, pool_sh, nsp, nsplit, kld, vld, chunked, gate_elem, keep_first, rel_n, out_ld;
+  const void* uv;                                            // [H, Dv, vdim]: each head's result times its matrix (null: as it is)
+  int vdim, rows, gate_ld, ptab_ld, H, G, D, Dv, page, page_sh, PB, window, pool_sh, nsp, nsplit, kld, vld, chunked, gate_elem, keep_first, rel_n, out_ld;
   float scale, cap, out_scale;
 };
 
@@ -75,6 +76,7 @@ __device__ __forceinline__ void halve(float (&v)[N], int& off, int lane) {
   }
 }
 
+constexpr int MAX_VDIM = 128;                               // columns of a head's matrix
 constexpr int STEP_NW = 8;                                  // waves of a workgroup
 
 // e^x for x <= 0 (or NaN) to about one rounding: x log2(e) in two parts, the small one to first order
@@ -85,12 +87,13 @@ __device__ __forceinline__ float exp_neg(float x) {
   return fmaf(p * lo, LN2, p);
 }
 
-template <typename T, int NC, int DVL, int SH, bool POOL>
+template <typename T, int NC, int DVL, int SH, bool POOL, bool EX>
 __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
   constexpr int NW = STEP_NW, LPK = 8 * DVL, KPR = 64 / LPK, VP = 2 * DVL, RK = 16 * NW, DR = 64 * DVL;
   __shared__ __attribute__((aligned(16))) float p_s[NW][16][SH];
   __shared__ __attribute__((aligned(16))) float red[NW][SH][DR];
   __shared__ float m_s[NW][SH], l_s[NW][SH], tot_s[2][SH];
+  __shared__ __attribute__((aligned(16))) float y_s[EX ? DR : 1], e_s[EX ? NW : 1][EX ? MAX_VDIM : 1];
   // consecutive workgroups go to the eight dies in turn: those of one (token, kv head, part of its keys) stay on one die, where they
   // read the same rows
   const int unit = blockIdx.x % 8 + 8 * (blockIdx.x / 8 / a.nsp), sub = blockIdx.x / 8 % a.nsp;
@@ -237,6 +240,18 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
          },
          [&](v4f&, int) {});
 
+  // uv: eight columns a thread, rows rg, rg + EG, .. (a matrix of 64 DVL x 128: 8 DVL or 16 DVL registers, on its way from here)
+  constexpr int UR = EX ? 2 * DVL : 1, TQ = sizeof(T) / 2;
+  uint4 uvr[UR][TQ];
+  const int vl = EX ? a.vdim / 8 : 64, uc = tid % vl * 8, rg = tid / vl, EG = NW * 64 / vl;
+  if constexpr (EX) {
+#pragma unroll
+    for (int k = 0; k < UR; ++k)
+#pragma unroll
+      for (int q = 0; q < TQ; ++q)
+        uvr[k][q] = reinterpret_cast<const uint4*>(reinterpret_cast<const T*>(a.uv) +
+                                                   ((size_t)hq0 * Dv + min(rg + EG * k, Dv - 1)) * a.vdim + uc)[q];
+  }
   // add up the lanes that walked different keys, then the waves
   int off = 0;
   halve<SH * 8, 32, LPK>(acc, off, lane);
@@ -279,17 +294,55 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
     } else {
       const int h = hq0 + r;
       float y = o / tot_s[1][r];
+      if constexpr (EX) {
+        y_s[d] = y;
+        continue;
+      }
       if (a.gate) y *= sigmoidf_(ldf<T>(reinterpret_cast<const T*>(a.gate) + (size_t)t * a.gate_ld + (a.gate_elem ? h * Dv + d : h)));
       stf<T>(reinterpret_cast<T*>(a.out) + (size_t)t * a.out_ld + h * Dv + d, y * a.out_scale);
     }
   }
+  if constexpr (EX) {
+    __syncthreads();
+    float e8[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < UR; ++k) {
+      const int r = rg + EG * k;
+      float uf[8];
+      load8<T>(reinterpret_cast<const T*>(&uvr[k][0]), uf);
+      const float y = r < Dv ? y_s[min(r, DR - 1)] : 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) e8[e] += r < Dv ? y * uf[e] : 0.f;
+    }
+    for (int o = vl; o < 64; o <<= 1)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) e8[e] += __shfl_xor(e8[e], o, 64);
+    if (lane < vl)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) e_s[wave][uc + e] = e8[e];
+    __syncthreads();
+    if (tid < a.vdim) {
+      float y = 0.f;
+#pragma unroll
+      for (int w = 0; w < NW; ++w) y += e_s[w][tid];
+      if (a.gate) y *= sigmoidf_(ldf<T>(reinterpret_cast<const T*>(a.gate) + (size_t)t * a.gate_ld + hq0 * a.vdim + tid));
+      stf<T>(reinterpret_cast<T*>(a.out) + (size_t)t * a.out_ld + hq0 * a.vdim + tid, y);
+    }
+  }
 }
 
-template <typename T, int SH>
+template <typename T, int SH, bool EX>
 int run_step(const StepArgs& a, hipStream_t st) {
   const dim3 grid((a.rows * a.G * a.nsplit + 7) / 8 * 8 * a.nsp), block(STEP_NW * 64);
   const bool pool = a.pool_sh >= 0;
-#define STEP(NC, DL, P) hipLaunchKernelGGL((attn_step_kernel<T, NC, DL, SH, P>), grid, block, 0, st, a)
+#define STEP(NC, DL, P) hipLaunchKernelGGL((attn_step_kernel<T, NC, DL, SH, P, EX>), grid, block, 0, st, a)
+  if constexpr (EX) {
+    if (pool) return -2;
+    if (a.D <= 128 && a.Dv <= 128) STEP(4, 2, false);
+    else if (a.D <= 192 && a.Dv <= 128) STEP(6, 2, false);
+    else STEP(10, 4, false);
+    return (int)hipGetLastError();
+  }
   if (a.D <= 64 && a.Dv <= 64) { if (pool) STEP(2, 1, true); else STEP(2, 1, false); }
   else if (a.D <= 128 && a.Dv <= 128) { if (pool) STEP(4, 2, true); else STEP(4, 2, false); }
   else if (pool) return -2;
@@ -333,6 +386,35 @@ size_t edge_sm_attention_step_floats(int rows, int H, int G, int Dv, int plan) {
   return nsplit > 1 ? (size_t)rows * G * ((H / G + sh - 1) / sh) * nsplit * sh * (Dv + 2) : 0;
 }
 
+// The general form: with uv [H, Dv, vdim] every head's result is multiplied by its matrix (and gated behind it: gate [rows, H vdim]);
+// for plans of one head a workgroup and whole keys (elsewhere a workgroup does not hold a finished head), vdim 64 or 128: 8 or 16
+// lanes a row, up to 256 rows.  The matrix is on its way while the waves' shares are added up, the head stays fp32 in between, and a
+// launch of latency is gone: 4 tokens a step, 63 steps, 16.67 -> 16.33 ms against the product in a launch of its own (runs of one
+// side differ by 0.3%).
+int edge_sm_attention_expand(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb,
+                             const float* vb, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
+                             int ptab_ld, void* out, int rows, int H, int G, int D, int Dv, int page, int PB, float scale,
+                             int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
+                             const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
+                             int out_ld, float out_scale, const void* uv, int vdim, hipStream_t st) {
+  if (rows == 0) return 0;
+  const int sh = plan % 8, nsplit = plan / 8;
+  if (uv && (sh != 1 || nsplit != 1 || (vdim != 64 && vdim != MAX_VDIM) || (uintptr_t)uv % 16 || out_scale != 1.f)) return -2;
+  if (G <= 0 || H % G || (chunked && pool > 0) || keep_first < 0 || (rel && (rel_n < 1 || pool > 0)) || out_ld < H * (uv ? vdim : Dv) ||
+      (sh != 1 && sh != 4) || nsplit < 1 || nsplit > 16 || (nsplit > 1 && !part) || D > 320 || Dv > 256 || page < 1 ||
+      (page & (page - 1)) || (pool & (pool - 1)))
+    return -2;
+  const int nsp = (H / G + sh - 1) / sh, page_sh = __builtin_ctz(page), pool_sh = window > 0 && pool > 0 ? __builtin_ctz(pool) : -1;
+  const StepArgs a{q, gate, kp, vp, kb, vb, tok_seq, tok_pos, seq_slot, ptab, out, part, slopes, sink, rel, uv, vdim, rows, gate_ld, ptab_ld, H, G, D,
+                   Dv, page, page_sh, PB, window, pool_sh, nsp, nsplit, kld, vld, chunked, gate_elem, keep_first, rel_n, out_ld, scale,
+                   cap, out_scale};
+  if (uv) return f32 ? run_step<float, 1, true>(a, st) : run_step<bf16_t, 1, true>(a, st);
+  const int r = sh == 1 ? (f32 ? run_step<float, 1, false>(a, st) : run_step<bf16_t, 1, false>(a, st))
+                        : (f32 ? run_step<float, 4, false>(a, st) : run_step<bf16_t, 4, false>(a, st));
+  if (r != 0 || nsplit == 1) return r;
+  return edge_sm_attn_merge(part, gate, gate_ld, out, rows, H, G, Dv, nsp, nsplit, sh, gate_elem, out_ld, out_scale, f32, st);
+}
+
 // plan as edge_sm_attention_step_plan says, part edge_sm_attention_step_floats numbers; the rest as edge_sm_attention's
 int edge_sm_attention_step(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb,
                            const float* vb, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
@@ -340,20 +422,9 @@ int edge_sm_attention_step(const void* q, const void* gate, int gate_ld, const v
                            int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
                            const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
                            int out_ld, float out_scale, hipStream_t st) {
-  if (rows == 0) return 0;
-  const int sh = plan % 8, nsplit = plan / 8;
-  if (G <= 0 || H % G || (chunked && pool > 0) || keep_first < 0 || (rel && (rel_n < 1 || pool > 0)) || out_ld < H * Dv ||
-      (sh != 1 && sh != 4) || nsplit < 1 || nsplit > 16 || (nsplit > 1 && !part) || D > 320 || Dv > 256 || page < 1 ||
-      (page & (page - 1)) || (pool & (pool - 1)))
-    return -2;
-  const int nsp = (H / G + sh - 1) / sh, page_sh = __builtin_ctz(page), pool_sh = window > 0 && pool > 0 ? __builtin_ctz(pool) : -1;
-  const StepArgs a{q, gate, kp, vp, kb, vb, tok_seq, tok_pos, seq_slot, ptab, out, part, slopes, sink, rel, rows, gate_ld, ptab_ld, H, G, D,
-                   Dv, page, page_sh, PB, window, pool_sh, nsp, nsplit, kld, vld, chunked, gate_elem, keep_first, rel_n, out_ld, scale,
-                   cap, out_scale};
-  const int r = sh == 1 ? (f32 ? run_step<float, 1>(a, st) : run_step<bf16_t, 1>(a, st))
-                        : (f32 ? run_step<float, 4>(a, st) : run_step<bf16_t, 4>(a, st));
-  if (r != 0 || nsplit == 1) return r;
-  return edge_sm_attn_merge(part, gate, gate_ld, out, rows, H, G, Dv, nsp, nsplit, sh, gate_elem, out_ld, out_scale, f32, st);
+  return edge_sm_attention_expand(q, gate, gate_ld, kp, vp, kb, vb, tok_seq, tok_pos, seq_slot, ptab, ptab_ld, out, rows, H, G, D, Dv, page,
+                                  PB, scale, window, pool, f32, plan, part, kld, vld, chunked, cap, slopes, sink, gate_elem, keep_first,
+                                  rel, rel_n, out_ld, out_scale, nullptr, 0, st);
 }
 
 }  // extern "C"

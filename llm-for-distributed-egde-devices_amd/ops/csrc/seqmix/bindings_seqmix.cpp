@@ -67,6 +67,12 @@ int edge_sm_attention_step(const void* q, const void* gate, int gate_ld, const v
                            int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
                            const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
                            int out_ld, float out_scale, hipStream_t st);
+int edge_sm_attention_expand(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb,
+                             const float* vb, const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab,
+                             int ptab_ld, void* out, int rows, int H, int G, int D, int Dv, int page, int PB, float scale,
+                             int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
+                             const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
+                             int out_ld, float out_scale, const void* uv, int vdim, hipStream_t st);
 int edge_sm_attention_splits(int rows, int G, int chunks);
 size_t edge_sm_attention_part_floats(int rows, int H, int G, int D, int Dv, int nsplit);
 int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp,
@@ -498,6 +504,49 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
             floats ? part.data_ptr<float>() : nullptr, (int)kld, (int)vld, chunked ? 1 : 0, (float)softcap, slopes_p, sink_p,
             gate_elem, (int)keep_first, rel_p, rel_n, out_ld, (float)out_scale, stream()),
         "sm_attention");
+  return out;
+}
+
+// the attention of latent rows with each head's result times uv[h] (and sigmoid of the gate); nothing where the step is not
+// attn_step_kernel's with one head a workgroup and whole keys, or the matrix has other columns than 64 or 128
+std::optional<at::Tensor> sm_attention_expand(const at::Tensor& q, const at::Tensor& lat, int64_t R, const at::Tensor& tok_seq,
+                                              const at::Tensor& tok_pos, const at::Tensor& seq_slot, const at::Tensor& ptab, double scale,
+                                              int64_t window, int64_t max_keys, const std::optional<at::Tensor>& sink,
+                                              const at::Tensor& uv, const std::optional<at::Tensor>& gate) {
+  chk_i32(tok_seq, "tok_seq");
+  chk_i32(tok_pos, "tok_pos");
+  chk_i32(seq_slot, "seq_slot");
+  chk_table(ptab);
+  TORCH_CHECK(q.is_cuda() && q.dim() == 3 && q.is_contiguous() && is_act(q), "q: [T, H, D]");
+  const int64_t T = q.size(0), H = q.size(1), D = q.size(2);
+  TORCH_CHECK(lat.is_cuda() && lat.dim() == 4 && lat.scalar_type() == q.scalar_type() && lat.size(2) == 1 &&
+                  lat.size(3) == D && R >= 1 && R <= D, "latent rows: [pages, page, 1, D]");
+  TORCH_CHECK(uv.is_cuda() && uv.dim() == 3 && uv.is_contiguous() && uv.scalar_type() == q.scalar_type() && uv.size(0) == H &&
+                  uv.size(1) == R, "uv [H, R, vdim]");
+  TORCH_CHECK(tok_seq.numel() == T && tok_pos.numel() == T, "metadata sizes");
+  const int64_t page = lat.size(1), vdim = uv.size(2);
+  TORCH_CHECK(max_keys <= ptab.size(1) * page, "page table too short for the step");
+  int gate_ld = 0;
+  if (gate) {
+    gate_ld = row_ld(*gate, "gate");
+    TORCH_CHECK(gate->size(0) == T && gate->size(1) == H * vdim && gate->scalar_type() == q.scalar_type(), "gate: [T, H vdim]");
+  }
+  if (sink) {
+    chk_f32(*sink, "sink");
+    TORCH_CHECK(sink->numel() == H, "sink: fp32 [H]");
+  }
+  const int64_t vis = window > 0 ? std::min<int64_t>(window, max_keys) : max_keys;
+  const int plan = edge_sm_attention_step_plan((int)T, (int)H, 1, (int)D, (int)R, (int)D, (int)D, (int)page, 0, vis, f32(q),
+                                               (uintptr_t)q.data_ptr() | (uintptr_t)lat.data_ptr());
+  if (plan != 1 + 8 || !lat.is_contiguous() || (vdim != 64 && vdim != 128) || (uintptr_t)uv.data_ptr() % 16) return std::nullopt;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+  auto out = at::empty({T, H * vdim}, q.options());
+  check(edge_sm_attention_expand(q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, lat.data_ptr(), lat.data_ptr(), nullptr,
+                                 nullptr, tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(),
+                                 ptab.data_ptr<int>(), (int)ptab.stride(0), out.data_ptr(), (int)T, (int)H, 1, (int)D, (int)R, (int)page,
+                                 0, (float)scale, (int)window, 0, f32(q), plan, nullptr, (int)D, (int)D, 0, 0.f, nullptr,
+                                 sink ? sink->data_ptr<float>() : nullptr, gate ? 1 : 0, 0, nullptr, 0, (int)(H * vdim), 1.f,
+                                 uv.data_ptr(), (int)vdim, stream()), "sm_attention_expand");
   return out;
 }
 
@@ -1649,6 +1698,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_moe_experts_glu_shared", &sm_moe_experts_glu_shared);
   m.def("sm_moe_experts_relu2", &sm_moe_experts_relu2);
   m.def("sm_latent_expand_write", &sm_latent_expand_write);
+  m.def("sm_attention_expand", &sm_attention_expand);
   m.def("sm_head_expand_gate", &sm_head_expand_gate);
   m.def("sm_heads_gate", &sm_heads_gate);
   m.def("sm_gla", &sm_gla);

@@ -278,7 +278,7 @@ def window_pool_attention(q: torch.Tensor, gate: Optional[torch.Tensor], k_pages
     assert rel is None or not pool, "pooled blocks have no distance"
     if _gpu(q):
         # bf16 steps with a portion of ATTN_MFMA_MIN tokens or more: the MFMA kernel (64 query rows per
-        # workgroup); decode-sized steps and fp32: one workgroup per (token, kv head)
+        # workgroup); decode-sized steps: attn_step.hip where its plan takes the sizes; else one workgroup per (token, kv head)
         qtiles = 0
         if q.dtype == torch.bfloat16 and meta.max_len >= ATTN_MFMA_MIN:
             qtiles = sum((h[2] + 63) // 64 for h in meta.host)
@@ -703,6 +703,20 @@ def head_expand_gate(a: torch.Tensor, uv: torch.Tensor, gate: Optional[torch.Ten
     if _gpu(a):
         return _ext().sm_heads_gate(v, gate)
     return (v.transpose(0, 1).reshape(T, H * Dv).float() * torch.sigmoid(gate.float())).to(a.dtype)
+
+
+def latent_attention(q: torch.Tensor, lat: torch.Tensor, uv: torch.Tensor, gate: Optional[torch.Tensor], meta: RaggedMeta,
+                     scale: float, window: Optional[int], sink: Optional[torch.Tensor]) -> torch.Tensor:
+    """``window_pool_attention`` of q [T, H, D] over the cached rows ``lat`` [pages, page, 1, D], their first kv_rank numbers the
+    values, then ``head_expand_gate``: [T, H * Dv]; one launch at decode steps where each head is a workgroup."""
+    R = uv.shape[1]
+    if _gpu(q) and q.shape[0] <= HEAD_FUSE_MAX and (q.dtype != torch.bfloat16 or meta.max_len < ATTN_MFMA_MIN):
+        out = _ext().sm_attention_expand(q, lat, R, meta.tok_seq, meta.tok_pos, meta.seq_slot, meta.page_table, float(scale),
+                                         int(window) if window is not None else 0, int(meta.max_keys), sink, uv, gate)
+        if out is not None:
+            return out
+    a = window_pool_attention(q, None, lat, lat[..., :R], None, None, meta, scale, window, None, sink)
+    return head_expand_gate(a, uv, gate, meta)
 
 
 # --------------------------------------------------------------------------- gated linear attention

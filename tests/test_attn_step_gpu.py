@@ -93,3 +93,28 @@ def test_scores_of_minus_infinity_and_page_sizes():
         assert s[:, 3].isneginf().all()
         ref = (torch.softmax(s, -1) @ v.view(-1, 64)[:60].double()).view(1, -1)
         assert (got.double() - ref).abs().max() < 1e-5
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,D,R,vdim", [(4, 320, 256, 128), (16, 288, 256, 64), (5, 160, 128, 64), (3, 72, 64, 128), (2, 200, 136, 64),
+                                        (4, 64, 48, 40)])
+@pytest.mark.parametrize("lens", [[1], [127, 300, 16, 129], [2000, 3]])
+@pytest.mark.parametrize("gated", [False, True])
+def test_latent_heads(dt, H, D, R, vdim, lens, gated):
+    """Each head's result times its matrix: columns and ranks beside the thread layout, keys split, other columns than the fused ones."""
+    g = torch.Generator().manual_seed(4)
+    uv = (torch.randn(H, R, vdim, generator=g) * R ** -0.5).to(dt)
+    wide = torch.randn(len(lens), 24 + H * vdim, generator=g).to(dt)
+    sink = torch.linspace(-1, 3, H)
+    table = torch.randperm(len(lens) * 125, generator=g).view(len(lens), 125).int()
+    lat = torch.randn(len(lens) * 125, PAGE, 1, D, generator=g).to(dt)
+    q = torch.randn(len(lens), H, D, generator=g).to(dt)
+
+    def on(dev, f):
+        c = lambda t: t.to(dev).to(f)
+        return S.latent_attention(c(q), c(lat), c(uv), c(wide)[:, 24:] if gated else None, _meta(lens, dev, table), D ** -0.5, 100,
+                                  sink.to(dev))
+    got, ref = on("cuda", dt).float().cpu(), on("cpu", torch.float32)
+    # one rounding of the result and, where the launches are two, one of each of the R numbers behind it (weights of norm about 1)
+    eps = 2.0 ** -6 if dt == torch.bfloat16 else 2.0 ** -16
+    assert torch.isfinite(got).all() and ((got - ref).abs() <= eps * (1 + ref.abs())).all(), (got - ref).abs().max()
