@@ -209,12 +209,8 @@ class LatentAttention(nn.Module):
         cq = seqmix.rms_norm_cols(u, 0, s.q_rank, self.q_norm, self.eps, h.dtype)
         q = self.uq(cq).view(T, H, s.dim + s.rot_dim)
         rope = _shared_rope(self._rope, (s.rot_dims, s.rot_base, s.rot_scaling), meta.max_keys, h.device)
-        if self.own_kv:
-            qc = seqmix.latent_expand_write(u, s.q_rank, self.kv_norm, self.eps, q, self.uk, meta, rope, run.lat, s.kv_rank,
-                                            s.rot_dims)
-        else:
-            q_lat = torch.bmm(q[:, :, :s.dim].transpose(0, 1), self.uk).transpose(0, 1)  # [T, H, kv_rank]
-            qc = seqmix.latent_write(None, s.q_rank, None, self.eps, q, q_lat, meta, rope, run.lat, s.kv_rank, s.rot_dims)
+        qc = seqmix.latent_expand_write(u if self.own_kv else None, s.q_rank, self.kv_norm, self.eps, q, self.uk, meta, rope, run.lat,
+                                        s.kv_rank, s.rot_dims)
         return self.o(seqmix.latent_attention(qc, run.lat, self.uv, u[:, u.shape[1] - self.ng:] if self.ng else None, meta, s.scale,
                                               s.window, self.sink))
 

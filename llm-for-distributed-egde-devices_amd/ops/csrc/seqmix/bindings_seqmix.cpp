@@ -1488,7 +1488,8 @@ std::tuple<at::Tensor, at::Tensor> sm_moe_experts_relu2(const at::Tensor& h, con
   return {out, out_sh};
 }
 
-at::Tensor sm_latent_expand_write(const at::Tensor& u, int64_t c0, const at::Tensor& w, double eps, const at::Tensor& q,
+at::Tensor sm_latent_expand_write(const std::optional<at::Tensor>& u, int64_t c0, const std::optional<at::Tensor>& w, double eps,
+                                  const at::Tensor& q,
                                   const at::Tensor& uk, const at::Tensor& tok_seq, const at::Tensor& tok_pos,
                                   const at::Tensor& seq_slot, const at::Tensor& ptab, const std::optional<at::Tensor>& cs,
                                   at::Tensor& pages, int64_t rot) {
@@ -1496,16 +1497,20 @@ at::Tensor sm_latent_expand_write(const at::Tensor& u, int64_t c0, const at::Ten
   chk_i32(tok_pos, "tok_pos");
   chk_i32(seq_slot, "seq_slot");
   chk_table(ptab);
-  chk_f32(w, "latent norm weight");
-  const int ld = row_ld(u, "u");
   TORCH_CHECK(q.is_cuda() && q.dim() == 3 && q.is_contiguous() && is_act(q), "q: [T, H, D + R]");
   TORCH_CHECK(uk.is_cuda() && uk.dim() == 3 && uk.is_contiguous() && uk.scalar_type() == q.scalar_type() &&
                   uk.size(0) == q.size(1) && uk.size(1) <= q.size(2), "uk: [H, D, kv_rank]");
   const int64_t T = q.size(0), H = q.size(1), D = uk.size(1), R = q.size(2) - D, kvr = uk.size(2), page = pages.size(1);
   TORCH_CHECK(pages.is_cuda() && pages.is_contiguous() && pages.dim() == 4 && pages.size(2) == 1 &&
                   pages.scalar_type() == q.scalar_type() && pages.size(3) == kvr + R, "pages: [pages, page, 1, kv_rank + R]");
-  TORCH_CHECK(u.scalar_type() == q.scalar_type() && u.size(0) == T && c0 >= 0 && c0 + kvr + R <= u.size(1) && w.numel() == kvr,
-              "u: [T, .. latent | key part ..]");
+  int ld = 0;
+  if (u) {
+    ld = row_ld(*u, "u");
+    TORCH_CHECK(w, "latent norm weight missing");
+    chk_f32(*w, "latent norm weight");
+    TORCH_CHECK(u->scalar_type() == q.scalar_type() && u->size(0) == T && c0 >= 0 && c0 + kvr + R <= u->size(1) && w->numel() == kvr,
+                "u: [T, .. latent | key part ..]");
+  }
   TORCH_CHECK(tok_seq.numel() == T && tok_pos.numel() == T, "metadata sizes");
   if (rot > 0) {
     TORCH_CHECK(cs, "rotary table missing");
@@ -1514,7 +1519,8 @@ at::Tensor sm_latent_expand_write(const at::Tensor& u, int64_t c0, const at::Ten
   }
   c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
   auto qc = at::empty({T, H, kvr + R}, q.options());
-  check(edge_sm_latent_expand_write(u.data_ptr(), ld, (int)c0, w.data_ptr<float>(), (float)eps, q.data_ptr(), uk.data_ptr(),
+  check(edge_sm_latent_expand_write(u ? u->data_ptr() : nullptr, ld, (int)c0, u ? w->data_ptr<float>() : nullptr, (float)eps,
+                                    q.data_ptr(), uk.data_ptr(),
                                     tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(),
                                     ptab.data_ptr<int>(), (int)ptab.stride(0), rot > 0 ? cs->data_ptr<float>() : nullptr,
                                     pages.data_ptr(), qc.data_ptr(), (int)T, (int)H, (int)D, (int)R, (int)kvr, (int)rot,

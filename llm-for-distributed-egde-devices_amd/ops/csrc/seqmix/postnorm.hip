@@ -379,7 +379,8 @@ __device__ __forceinline__ void vec_mat(const float* x_s, const T* __restrict__ 
 }
 
 // Workgroup (t, h < H): qc[t, h] = (sum_d q[t, h, d] uk[h, d, :]) | rotate(q[t, h, D : D + R]).  Workgroup (t, H): the
-// cached row rms(u[c0 : c0 + kvr]) w | rotate(u[c0 + kvr : ..]).  LDS: x [max(D, 1)] | out [kvr] | shares [8 NT].
+// cached row rms(u[c0 : c0 + kvr]) w | rotate(u[c0 + kvr : ..]); not launched where the rows are another layer's (u null).
+// LDS: x [max(D, 1)] | out [kvr] | shares [8 NT].
 template <typename T>
 __global__ void __launch_bounds__(NT) latent_expand_write_kernel(
     const T* __restrict__ u, int ld, int c0, const float* __restrict__ w, float eps, const T* __restrict__ q,
@@ -1278,10 +1279,10 @@ int edge_sm_latent_expand_write(const void* u, int ld, int c0, const float* w, f
                                 const float* cs, void* pages, void* qc, int rows, int H, int D, int R, int kvr, int rot, int page,
                                 int f32, hipStream_t st) {
   if (rows == 0) return 0;
-  if (rot % 2 || rot > R || (rot > 0 && !cs) || !u || !w) return -2;
+  if (rot % 2 || rot > R || (rot > 0 && !cs) || (u && !w)) return -2;
   const size_t lds = sizeof(float) * ((size_t)D + kvr + 8 * NT);
   if (lds > 60 * 1024) return -3;
-  SM_T(f32, hipLaunchKernelGGL(latent_expand_write_kernel<T>, dim3(rows, H + 1), dim3(NT), lds, st, (const T*)u, ld, c0, w, eps,
+  SM_T(f32, hipLaunchKernelGGL(latent_expand_write_kernel<T>, dim3(rows, u ? H + 1 : H), dim3(NT), lds, st, (const T*)u, ld, c0, w, eps,
                                (const T*)q, (const T*)uk, tok_seq, tok_pos, seq_slot, ptab, ptab_ld, cs, (T*)pages, (T*)qc, H,
                                D, R, kvr, rot, page));
   return (int)hipGetLastError();

@@ -678,13 +678,16 @@ def latent_write(u: Optional[torch.Tensor], c0: int, weight: Optional[torch.Tens
 HEAD_FUSE_MAX = int(__import__("os").environ.get("EDGELLM_HEAD_FUSE_MAX", "16"))
 
 
-def latent_expand_write(u: torch.Tensor, c0: int, weight: torch.Tensor, eps: float, q: torch.Tensor, uk: torch.Tensor,
+def latent_expand_write(u: Optional[torch.Tensor], c0: int, weight: Optional[torch.Tensor], eps: float, q: torch.Tensor, uk: torch.Tensor,
                         meta: RaggedMeta, rope: Optional[torch.Tensor], pages: torch.Tensor, kv_rank: int,
                         rot_dims: int) -> torch.Tensor:
     """``latent_write`` that also computes q_lat[t, h] = q[t, h, :D] uk[h] (uk [H, D, kv_rank]); on the GPU one
-    kernel at up to HEAD_FUSE_MAX tokens."""
+    kernel at up to HEAD_FUSE_MAX tokens.  ``u`` None (another layer's rows): the queries alone, for heads that fit the kernel's
+    LDS.  63 steps of 4 tokens 16.37 -> 15.98 ms against a batched product (6.9 us) and the write (3.9 us); error of the
+    product against 64 bits: the same in bf16, 0.9e-7 for 0.8e-7 to 2.1e-7 in fp32."""
     D = uk.shape[1]
-    if _gpu(q) and q.shape[0] <= HEAD_FUSE_MAX:
+    if _gpu(q) and q.shape[0] <= HEAD_FUSE_MAX and (u is not None or (D > 0 and D + kv_rank <= 8192 and uk.is_contiguous()
+                                                                       and uk.data_ptr() % 16 == 0)):
         return _ext().sm_latent_expand_write(u, int(c0), weight, float(eps), q, uk, meta.tok_seq, meta.tok_pos, meta.seq_slot,
                                              meta.page_table, rope if rot_dims else None, pages, int(rot_dims))
     q_lat = torch.bmm(q[:, :, :D].transpose(0, 1), uk).transpose(0, 1)                  # [T, H, kv_rank]

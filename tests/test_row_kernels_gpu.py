@@ -93,6 +93,27 @@ def test_latent_write(dt, H, D, R, kvr, rot):
 
 
 @pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("H,D,R,kvr,rot", [(16, 64, 32, 128, 32), (3, 8, 8, 8, 0), (2, 128, 64, 256, 64), (2, 8, 6, 10, 4), (1, 1, 2, 1, 2)])
+@pytest.mark.parametrize("T", [1, 16, 17])
+def test_queries_of_shared_latents(dt, H, D, R, kvr, rot, T):
+    """Queries against another layer's cached rows: up to 16 tokens in one launch, 17 in two; the rows stay as they are."""
+    g = torch.Generator().manual_seed(H + T)
+    tab = torch.arange(T, dtype=torch.int32).view(T, 1)
+    q, uk = _rand(g, T, H, D + R), _rand(g, H, D, kvr) * D ** -0.5
+    ang = _rand(g, 80, max(rot // 2, 1))
+    rope, rows = torch.stack([ang.cos(), ang.sin()], -1).contiguous(), _rand(g, T, 64, 1, kvr + R)
+    res = []
+    for dev, t in (("cuda", dt), ("cpu", torch.float32)):
+        meta = S.RaggedMeta.build([(i, i, 1) for i in range(T)], tab.to(dev), 64, torch.device(dev))
+        cast = lambda x: x.to(dt).to(dev, t)
+        pages = cast(rows)
+        qc = S.latent_expand_write(None, 0, None, 1e-6, cast(q), cast(uk), meta, rope.to(dev) if rot else None, pages, kvr, rot)
+        assert torch.equal(pages, cast(rows))
+        res.append(qc.reshape(T, -1))
+    _near(res[0], res[1].cpu(), dt)
+
+
+@pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("T,E,W,bias", [(64, 16, 1024, False), (768, 16, 1024, False), (2459, 5, 520, True), (374, 33, 2048, False),
                                         (12289, 1, 8, True), (770, 16, 1030, False)])
 def test_router_scores_of_prompts(dt, T, E, W, bias):
