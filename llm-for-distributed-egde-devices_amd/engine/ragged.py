@@ -24,6 +24,8 @@ import numpy as np
 import torch
 
 from .. import ops
+from ..models.hybrid import HybridLM
+from ..models.layers import unwatched
 from ..ops.seqmix import RaggedMeta
 from ..utils.tracing import trace_range
 from .generate import GenerationResult, SamplingParams
@@ -72,7 +74,7 @@ class _DecodeGraph:
         eng = self.eng
         # a model that nobody watches is captured up to its output projection's rows: making logits of them also takes them out of
         # the graph's memory, and every row is wanted
-        watched = bool(eng.model._forward_hooks or eng.model._forward_pre_hooks) or not hasattr(eng.model, "scores")
+        watched = type(eng.model).forward is not HybridLM.forward or not unwatched(eng.model)
         if not self.warm:
             self.warm = True
             return eng.model(self.ids, self.meta, eng.cache)

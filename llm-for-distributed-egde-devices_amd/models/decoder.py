@@ -30,7 +30,7 @@ import torch.nn as nn
 from .. import ops
 from ..utils import tracing
 from .configs import ModelConfig
-from .layers import BranchRows, Linear, Norm, PartialSum, PendingLN, PendingNorm, QAct, act_fn, quant_if
+from .layers import BranchRows, Linear, Norm, PartialSum, PendingLN, PendingNorm, QAct, act_fn, quant_if, unwatched
 
 # split-K slices of the bf16 o / down decode GEMVs (0 = off); N = 2048-4096 outputs have only
 # 128-256 tiles, so two slices put every CU to work
@@ -302,7 +302,7 @@ class DecoderLayer(nn.Module):
                 and all(type(m) is kind for m in (qkv, o, up, down)) and up.pair_ok(up=True) and o.pair_ok() and down.pair_ok()
                 and (kind is Linear or o.in_features <= 4096 < down.in_features)
                 and self.norm1.eps == (self.norm2 or self.norm1).eps
-                and not any(m._forward_hooks or m._forward_pre_hooks for m in (self.attn, self.mlp, qkv, o, up, down)))
+                and unwatched(self.attn, self.mlp, qkv, o, up, down))
 
     def _pair(self, x, residual, ctx: AttnCtx):
         """A parallel-residual decode step in three launches (decode_pair.hip, decode_pair_i8.hip): qkv with the norm(s) in its

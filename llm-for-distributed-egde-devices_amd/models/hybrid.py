@@ -53,15 +53,10 @@ import torch.nn as nn
 
 from ..ops import seqmix
 from .configs import LayerSpec, ModelConfig
-from .layers import DynamicTanh, GroupRMSNorm, Linear, RowLayerNorm, ScalarNorm
+from .layers import DynamicTanh, GroupRMSNorm, Linear, RowLayerNorm, ScalarNorm, unwatched
 from .mixers import (AttentionRetention, ChannelDeltaMixer, ChunkAttention, DecayLinearAttention, GatedAttention,
                      GatedLinearAttention, HeadDeltaMixer, LatentAttention, ParallelMixer)
 from .moe import MoEFeedForward, MoEOut
-
-
-def _unwatched(m: nn.Module) -> bool:
-    """Nobody has asked to see or change this module's calls."""
-    return not (m._forward_hooks or m._forward_pre_hooks)
 
 
 class HybridLayer(nn.Module):
@@ -79,7 +74,7 @@ class HybridLayer(nn.Module):
 
     def first_read(self, run):
         """What forms this layer's first input from the stream: the layer before may do it with its residual sum."""
-        return self.norm1 if _unwatched(self.norm1) else None
+        return self.norm1 if unwatched(self.norm1) else None
 
     def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run, h: Optional[torch.Tensor] = None, nxt=None):
         """``h``: this layer's first input when the layer before already formed it; ``nxt``: the next layer's ``first_read()``.
@@ -167,7 +162,7 @@ class SandwichLayer(nn.Module):
 
     def first_read(self, run):
         """What forms this layer's first input from the stream (``HybridLayer.first_read``)."""
-        return self.norm1 if _unwatched(self.norm1) else None
+        return self.norm1 if unwatched(self.norm1) else None
 
     def _join(self, norm, x, nxt, y, parts=None, wts=None):
         """x += the normed result; the rows of the norm that reads x next, where one is given."""
@@ -180,7 +175,7 @@ class SandwichLayer(nn.Module):
     def forward(self, x: torch.Tensor, meta: seqmix.RaggedMeta, run, h: Optional[torch.Tensor] = None, nxt=None):
         """``h``, ``nxt`` and the result: as ``HybridLayer.forward``."""
         last = self.ff is None
-        inner = None if last or not _unwatched(self.norm2) else self.norm2
+        inner = None if last or not unwatched(self.norm2) else self.norm2
         h = self._join(self.norm1b, x, nxt if last else inner, self.mix(self.norm1(x, self.dtype) if h is None else h, meta, run))
         if not last:
             shared, parts, wts = self.ff(self.norm2(x, self.dtype) if h is None else h)
@@ -423,13 +418,13 @@ class HybridLM(nn.Module):
         calls, no pass of a looped span that starts by changing the stream.  ``last``: the final norm follows the last run."""
         if r + 1 >= len(self.runs):
             here = self.layers[self.runs[r][0]]
-            ok = last and type(self.final_norm) is self._LAST_READ.get(type(here)) and _unwatched(here) and _unwatched(self.final_norm)
+            ok = last and type(self.final_norm) is self._LAST_READ.get(type(here)) and unwatched(here, self.final_norm)
             return self.final_norm if ok else None
         i, t = self.runs[r + 1]
         loop, here, there = self.cfg.loop, self.layers[self.runs[r][0]], self.layers[i]
         if t is not None and i == loop.start and (loop.entry == "project" or (loop.entry == "add_embed" and t > 0)):
             return None
-        if type(here) is not type(there) or not (_unwatched(here) and _unwatched(there)):
+        if type(here) is not type(there) or not unwatched(here, there):
             return None
         return there.first_read(cache.run(r + 1))
 

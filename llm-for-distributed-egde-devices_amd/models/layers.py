@@ -286,9 +286,16 @@ class Norm(nn.Module):
         return ops.layer_norm(x, self.weight, self.bias, self.eps, residual)
 
 
+def unwatched(*mods: nn.Module) -> bool:
+    """Nobody sees or changes these modules' own calls: no hook of theirs or for all modules, no ``forward`` set on one of them."""
+    hooks = nn.modules.module
+    return not (hooks._global_forward_hooks or hooks._global_forward_pre_hooks
+                or any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in mods))
+
+
 def plain_linear(m: nn.Module) -> bool:
     """A bias-free 16- or 32-bit projection whose own call nobody watches: its weight says all."""
-    return type(m) is Linear and m.bias is None and not (m._forward_hooks or m._forward_pre_hooks)
+    return type(m) is Linear and m.bias is None and unwatched(m)
 
 
 def rows_together(xs, mods):

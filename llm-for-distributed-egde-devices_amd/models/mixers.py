@@ -17,7 +17,7 @@ import torch.nn as nn
 
 from ..ops import seqmix
 from .configs import ChunkAttnSpec, DecayAttnSpec, DeltaSpec, GatedAttnSpec, GLASpec, LayerSpec, SSDSpec, WindowAttnSpec
-from .layers import Linear, plain_linear, rows_together
+from .layers import Linear, plain_linear, rows_together, unwatched
 
 
 _ROPE_TABLES: dict = {}
@@ -134,8 +134,8 @@ class ParallelMixer(nn.Module):
                 down: Optional[nn.Module] = None):
         """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra.  ``nxt``: the norm that reads x next; its rows
         (of u's dtype) come back in x's place.  ``pre``: ``step_in``'s results; with ``down``, extra is its output on the last."""
-        c0, watched = sum(self.left.spec.proj_sizes), any(m._forward_hooks or m._forward_pre_hooks for m in (self.left, self.right))
-        if pre is not None and down is not None and not watched:
+        c0 = sum(self.left.spec.proj_sizes)
+        if pre is not None and down is not None and unwatched(self.left, self.right):
             extra, a, r = rows_together((pre[2], self.left.heads(u, 0, meta, run, pre[0]), self.right.rows(u, c0, meta, run, pre[1])),
                                         (down, self.left.o, self.right.o))
         else:
