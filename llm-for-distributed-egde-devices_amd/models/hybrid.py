@@ -82,9 +82,10 @@ class HybridLayer(nn.Module):
         if h is None:
             h = self.norm1(x, self.proj_in.weight.dtype)
         u = self.proj_in(h)
-        pre = self.mix.step_in(u, meta, run, self.mix.in_rows, self.ff)
+        ours = unwatched(self.mix)                         # else its call and result are the plain ones
+        pre = self.mix.step_in(u, meta, run, self.mix.in_rows, self.ff) if ours and unwatched(self.mix.left, self.mix.right) else None
         m = self.down(seqmix.relu2(u, self.mix.in_rows, self.ff)) if self.ff and pre is None else None
-        y = self.mix(x, u, meta, run, m, nxt, pre, self.down)
+        y = self.mix(x, u, meta, run, m, nxt, pre, self.down) if ours else self.mix(x, u, meta, run, m)
         return y if nxt is None else (x, y)
 
 
@@ -416,12 +417,14 @@ class HybridLM(nn.Module):
     def _next_read(self, r: int, cache, last: bool):
         """``first_read()`` of run r + 1 where nothing comes between run r and it: both layers of one kind, nobody watching their
         calls, no pass of a looped span that starts by changing the stream.  ``last``: the final norm follows the last run."""
+        here = self.layers[self.runs[r][0]]
+        if type(here) is HybridLayer and not unwatched(here.mix):      # (its result would be the next rows)
+            return None
         if r + 1 >= len(self.runs):
-            here = self.layers[self.runs[r][0]]
             ok = last and type(self.final_norm) is self._LAST_READ.get(type(here)) and unwatched(here, self.final_norm)
             return self.final_norm if ok else None
         i, t = self.runs[r + 1]
-        loop, here, there = self.cfg.loop, self.layers[self.runs[r][0]], self.layers[i]
+        loop, there = self.cfg.loop, self.layers[i]
         if t is not None and i == loop.start and (loop.entry == "project" or (loop.entry == "add_embed" and t > 0)):
             return None
         if type(here) is not type(there) or not unwatched(here, there):

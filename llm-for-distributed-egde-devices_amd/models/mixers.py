@@ -17,7 +17,7 @@ import torch.nn as nn
 
 from ..ops import seqmix
 from .configs import ChunkAttnSpec, DecayAttnSpec, DeltaSpec, GatedAttnSpec, GLASpec, LayerSpec, SSDSpec, WindowAttnSpec
-from .layers import Linear, plain_linear, rows_together, unwatched
+from .layers import Linear, plain_linear, rows_together
 
 
 _ROPE_TABLES: dict = {}
@@ -56,9 +56,9 @@ class WindowPoolAttention(nn.Module):
             self._rope = tab
         return self._rope
 
-    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, q: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
         """``u`` columns [c0, ..) hold q | k | v | gate.  Returns the o-projection's output [T, W]."""
-        return self.o(self.heads(u, c0, meta, run, q))
+        return self.o(self.heads(u, c0, meta, run))
 
     def heads(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, q: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The o-projection's input; ``q``: the rotated queries, when they and the cached rows and block means are there already."""
@@ -91,9 +91,9 @@ class SSDMixer(nn.Module):
         self.norm_w = P(spec.inner)
         self.o = Linear(spec.inner, width, False, dtype, device)
 
-    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, xbc: Optional[torch.Tensor] = None) -> torch.Tensor:
+    def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
         """``u`` columns [c0, ..) hold z | x | B | C | dt.  Returns the o-projection's output [T, W]."""
-        return self.o(self.rows(u, c0, meta, run, xbc))
+        return self.o(self.rows(u, c0, meta, run))
 
     def rows(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, xbc: Optional[torch.Tensor] = None) -> torch.Tensor:
         """The o-projection's input; ``xbc``: the convolved x | B | C rows, when they are there already."""
@@ -135,15 +135,14 @@ class ParallelMixer(nn.Module):
         """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra.  ``nxt``: the norm that reads x next; its rows
         (of u's dtype) come back in x's place.  ``pre``: ``step_in``'s results; with ``down``, extra is its output on the last."""
         c0 = sum(self.left.spec.proj_sizes)
-        if pre is not None and down is not None and unwatched(self.left, self.right):
-            extra, a, r = rows_together((pre[2], self.left.heads(u, 0, meta, run, pre[0]), self.right.rows(u, c0, meta, run, pre[1])),
-                                        (down, self.left.o, self.right.o))
+        if pre is None:
+            a, r = self.left(u, 0, meta, run), self.right(u, c0, meta, run)
         else:
-            q, xbc, act = pre if pre is not None else (None, None, None)
-            if down is not None and pre is not None:
-                extra = down(act)
-            a = self.left(u, 0, meta, run, q)
-            r = self.right(u, c0, meta, run, xbc)
+            ins = self.left.heads(u, 0, meta, run, pre[0]), self.right.rows(u, c0, meta, run, pre[1])
+            if down is not None:
+                extra, a, r = rows_together((pre[2], *ins), (down, self.left.o, self.right.o))
+            else:
+                a, r = self.left.o(ins[0]), self.right.o(ins[1])
         if nxt is not None:
             return seqmix.combine_residual_norm(x, a, r, self.left_out, self.right_out, self.eps, extra, nxt.weight, nxt.eps, u.dtype)
         return seqmix.combine_residual(x, a, r, self.left_out, self.right_out, self.eps, extra)

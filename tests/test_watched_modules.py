@@ -12,18 +12,21 @@ FAMILIES = {"nudadra": (rb.SIZES, rb.hybrid_config), "pagonex": (rb.PAGONEX_SIZE
             "vetevik": (rb.VETEVIK_SIZES, rb.vetevik_config)}
 
 
-def _model(family):
+DEVICES = ["cpu", pytest.param("cuda", marks=pytest.mark.gpu)]
+
+
+def _model(family, device="cpu"):
     sizes, make = FAMILIES[family]
     model = HybridLM(make(dict(sizes["w1024"], layers=3, vocab=64)), torch.float32, "cpu")
     g = torch.Generator().manual_seed(0)
     for p in model.parameters():
         if p.dim() > 1:
             p.data.normal_(0, 0.02, generator=g)
-    return model
+    return model.to(device)
 
 
 def _step(model):
-    eng = RaggedEngine(model, 64, slots=1, page=16)
+    eng = RaggedEngine(model, 64, slots=1, page=16, use_graphs=False)
     return torch.cat([eng.step([(0, [5, 6, 7], [0, 1, 2])]), eng.step([(0, [8], [0])])])
 
 
@@ -57,6 +60,33 @@ def test_a_forward_set_on_a_norm_runs(family):
         _step(model)
         del m.forward
         assert len(seen) == 2, type(m)
+
+
+@pytest.mark.parametrize("device", DEVICES)
+def test_a_hook_on_a_parallel_mixer_alone_sees_the_stream(device):
+    model, seen = _model("nudadra", device), []
+    ref = _step(model)
+    layer = model.layers[1]
+    with torch.no_grad():
+        h = layer.mix.register_forward_hook(lambda m, a, y: seen.append((a, y)) and None)
+        out = _step(model)
+        h.remove()
+    assert len(seen) == 2
+    for a, y in seen:                                        # stream, projected rows, step, state, feed-forward's output -> stream
+        assert len(a) == 5 and y is a[0] and a[4].shape == a[0].shape
+    assert (out - ref).abs().max() <= 1e-5 * ref.abs().max()
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("half", ["left", "right"])
+def test_a_hook_on_one_half_of_a_parallel_mixer_sees_its_own_arguments(device, half):
+    model, seen = _model("nudadra", device), []
+    ref = _step(model)
+    h = getattr(model.layers[1].mix, half).register_forward_pre_hook(lambda m, a: seen.append(len(a)) and None)
+    out = _step(model)
+    h.remove()
+    assert seen == [4, 4]                                    # projected rows, first column, step, state
+    assert (out - ref).abs().max() <= 1e-5 * ref.abs().max()
 
 
 def test_who_counts_as_watched():
