@@ -480,8 +480,8 @@ class HybridLM(nn.Module):
                 x, h_next = self.layers[i](x, meta, cache.run(r), h_next, nxt)
             else:                                        # the next layer's first input rides on this layer's residual sum
                 nxt = self._next_read(r, cache, rows is None and taps is None)
-                if nxt is None:
-                    x, h_next = self.layers[i](x, meta, cache.run(r), h_next), None
+                if nxt is None:                          # (a watched layer's call: the stream alone, and the stream comes back)
+                    x, h_next = self.layers[i](x, meta, cache.run(r), *(() if h_next is None else (h_next,))), None
                 else:
                     x, h_next = self.layers[i](x, meta, cache.run(r), h_next, nxt)
             if taps is not None:

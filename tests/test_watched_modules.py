@@ -89,6 +89,15 @@ def test_a_hook_on_one_half_of_a_parallel_mixer_sees_its_own_arguments(device, h
     assert (out - ref).abs().max() <= 1e-5 * ref.abs().max()
 
 
+@pytest.mark.parametrize("family", FAMILIES)
+def test_a_hook_on_one_layer_sees_the_stream_alone(family):
+    model, seen = _model(family), []
+    h = model.layers[1].register_forward_hook(lambda m, a, y: seen.append((len(a), y is a[0])) and None)
+    _step(model)
+    h.remove()
+    assert seen == [(3, True)] * 2                           # stream, step, state -> stream
+
+
 def test_who_counts_as_watched():
     m = Linear(8, 8, False, torch.float32, "cpu")
     assert unwatched(m) and plain_linear(m)
