@@ -324,7 +324,8 @@ class DecoderLayer(nn.Module):
         a, m = C.llmint8_attn_up(*step, *up.pair_args(), up.out_features, up._ACT[cfg.act])
         return BranchRows(*C.llmint8_o_down(a, *o.pair_args(), m, *down.pair_args(), W)), h
 
-    def forward(self, x, residual, ctx: AttnCtx):
+    def forward(self, x, residual, ctx: AttnCtx, branches: bool = False):
+        """-> (the block's output, the stream that it joins).  ``branches``: the output may be BranchRows (``hands_branches``)."""
         cfg = self.cfg
         if not cfg.parallel_residual:
             # <= 4 rows: each norm of a split-K sum runs in the prologue of the W8A8 GEMV after it
@@ -345,8 +346,8 @@ class DecoderLayer(nn.Module):
         qa = self.attn.qkv.takes_quantized_input
         qm = self.mlp.up.takes_quantized_input
         rows = x.mlp if isinstance(x, BranchRows) else x
-        if self._ln_deferred(rows, qa, qm) and self._pair_ok(rows, ctx, Linear) or \
-                self._ln_deferred_l8(rows, qa, qm) and self._pair_ok(rows, ctx, type(self.attn.qkv)):
+        if branches and (self._ln_deferred(rows, qa, qm) and self._pair_ok(rows, ctx, Linear) or
+                         self._ln_deferred_l8(rows, qa, qm) and self._pair_ok(rows, ctx, type(self.attn.qkv))):
             return self._pair(x, residual, ctx)
         if isinstance(x, BranchRows):
             x = x.materialize()
@@ -394,6 +395,12 @@ class DecoderLayer(nn.Module):
         n1, h = self.norm1(x, residual, quant=qa)      # gpt_neox
         n2, _ = self.norm2(h, None, quant=qm)
         return self.mlp(n2, add=self.attn(n1, ctx)), h
+
+
+def hands_branches(layer: nn.Module, nxt: Optional[nn.Module]) -> bool:
+    """Whether ``layer`` may leave its two branches to ``nxt`` (the next layer or the final norm) to add: nobody watches either's
+    call, so nobody sees them."""
+    return type(layer) is DecoderLayer and type(nxt) in (DecoderLayer, Norm) and layer.cfg.parallel_residual and unwatched(layer, nxt)
 
 
 def _ln_consumer_ok(lin) -> bool:
@@ -492,13 +499,18 @@ class DecoderLM(nn.Module):
 
     # ------------------------------------------------------------------ forward
     def forward_layers(self, x: torch.Tensor, ctx: AttnCtx, residual: Optional[torch.Tensor] = None):
-        if tracing.TRACE:                      # roctx range per layer (rocprofv3 --marker-trace)
-            for layer in self.layers:
+        return self._run_layers(x, ctx, residual, None)
+
+    def _run_layers(self, x, ctx: AttnCtx, residual: Optional[torch.Tensor], nxt: Optional[nn.Module]):
+        """``nxt``: what reads the last layer's output next, where that is a module of this model."""
+        layers = list(self.layers)
+        for layer, follows in zip(layers, layers[1:] + [nxt]):
+            kw = {"branches": True} if hands_branches(layer, follows) else {}
+            if tracing.TRACE:                  # roctx range per layer (rocprofv3 --marker-trace)
                 with tracing.trace_range(f"{ctx.mode}.layer{layer.idx}"):
-                    x, residual = layer(x, residual, ctx)
-            return x, residual
-        for layer in self.layers:
-            x, residual = layer(x, residual, ctx)
+                    x, residual = layer(x, residual, ctx, **kw)
+            else:
+                x, residual = layer(x, residual, ctx, **kw)
         return x, residual
 
     def head(self, x: torch.Tensor, residual: Optional[torch.Tensor], ctx: AttnCtx,
@@ -556,10 +568,10 @@ class DecoderLM(nn.Module):
                 h = eng.run(ops.embedding(ids.reshape(-1), self.embed), ctx.start_pos)
                 return self.head(h, None, ctx, logits)
         x = self.embed_tokens(ids, ctx.start_pos, decode=ctx.mode == "decode") if self.has_embed else hidden
-        x, residual = self.forward_layers(x, ctx, None)
+        x, residual = self._run_layers(x, ctx, None, self.final_norm if self.has_head else None)
         if self.has_head:
             return self.head(x, residual, ctx, logits)
-        if isinstance(x, (BranchRows, PartialSum)):
+        if isinstance(x, PartialSum):
             x = x.materialize()
         return x + residual if residual is not None else x
 

@@ -23,8 +23,8 @@ import torch
 import torch.nn as nn
 
 from ..engine.kv_cache import KVCache
-from ..models.decoder import AttnCtx, DecoderLM
-from ..models.layers import BranchRows, PartialSum
+from ..models.decoder import AttnCtx, DecoderLM, hands_branches
+from ..models.layers import PartialSum
 from .partition import partition_model
 
 
@@ -136,15 +136,17 @@ class SplitLM(nn.Module):
             c = self._ctx_on(ctx, dev)
             xd = x.parts.device if isinstance(x, PartialSum) else x.device   # split-K slices (o / down)
             if xd != dev:                                    # the inter-stage hop (xGMI peer copy)
-                if isinstance(x, (BranchRows, PartialSum)):
+                if isinstance(x, PartialSum):
                     x = x.materialize()
                 x = x.to(dev, non_blocking=True)
                 residual = residual.to(dev, non_blocking=True) if residual is not None else None
-            for layer in m.layers[self.bounds[s]:self.bounds[s + 1]]:
-                x, residual = layer(x, residual, c)
+            layers = list(m.layers)[self.bounds[s]:self.bounds[s + 1]]
+            last = m.final_norm if s + 1 == len(self.devices) and self._head_embed is None else None
+            for layer, nxt in zip(layers, layers[1:] + [last]):
+                x, residual = layer(x, residual, c, **({"branches": True} if hands_branches(layer, nxt) else {}))
         c = self._ctx_on(ctx, self.devices[-1])
         if self._head_embed is not None:
-            if isinstance(x, (BranchRows, PartialSum)):
+            if isinstance(x, PartialSum):
                 x = x.materialize()
             if logits == "last" and c.T > 1:
                 idx = c.last_rows(x.device)

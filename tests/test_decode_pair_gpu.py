@@ -103,6 +103,61 @@ def test_decode_steps_agree_with_the_separate_launches(cuda, family, dtype, monk
     assert math.isfinite(float(k1.float().abs().max()))
 
 
+def _stepped(model, steps=2):
+    """Logits of a two-token prompt and some decode steps of one sequence, through the model's own call."""
+    from edgellm.engine import KVCache
+    from edgellm.models import AttnCtx
+    kv, rope = KVCache(model.cfg, 1, 16, dtype=model.dtype, device="cuda"), model.rope_table()
+    at = lambda n: torch.tensor([n], dtype=torch.int32, device="cuda")
+    ids = torch.tensor([[5, 9, 3, 7]], device="cuda")
+    with torch.no_grad():
+        out = [model(ids[:, :2], AttnCtx("prefill", 1, 2, at(0), at(2), 2, kv.rows(0, 1), rope), logits="last")]
+        for t in range(steps):
+            out.append(model(ids[:, 2 + t:3 + t], AttnCtx("decode", 1, 1, at(2 + t), at(3 + t), 3 + t, kv.rows(0, 1), rope)))
+    return torch.cat(out).float()
+
+
+@pytest.mark.parametrize("where", ["layer", "final_norm"])
+@pytest.mark.parametrize("kind", ["hook", "pre_hook", "forward"])
+def test_a_watched_layer_or_final_norm_sees_rows(cuda, where, kind, monkeypatch):
+    from edgellm.models import build_model, tiny
+    from edgellm.models.decoder import DecoderLayer
+    cfg = tiny("gpt_neox", num_layers=4, hidden_size=256, num_heads=4, num_kv_heads=4, intermediate_size=512, rotary_dim=32)
+    model, used, seen = build_model(cfg, dtype=torch.float16, device="cuda", seed=3), [], []
+    real = DecoderLayer._pair
+    monkeypatch.setattr(DecoderLayer, "_pair", lambda self, *a: used.append(self.idx) or real(self, *a))
+    ref = _stepped(model)
+    assert used == [0, 1, 2, 3] * 2
+    m = model.layers[1] if where == "layer" else model.final_norm
+    used.clear()
+    if kind == "hook":
+        h = m.register_forward_hook(lambda m, a, y: seen.append(a[:2] + y) and None)
+    elif kind == "pre_hook":
+        h = m.register_forward_pre_hook(lambda m, a: seen.append(a[:2]) and None)
+    else:
+        fwd = m.forward
+        m.forward = lambda *a, **k: seen.append(a[:2]) or fwd(*a, **k)
+    out = _stepped(model)
+    assert len(seen) == 3 and all(isinstance(t, (torch.Tensor, type(None))) for s in seen for t in s)
+    assert used == ([2, 3] if where == "layer" else [0, 1, 2]) * 2
+    assert (out - ref).norm() <= 4 * EPS[torch.float16] * ref.norm()     # four layers of differing last roundings
+
+
+def test_layers_that_a_program_steps_itself_give_rows(cuda):
+    from edgellm.engine import KVCache
+    from edgellm.models import AttnCtx, build_model, tiny
+    cfg = tiny("phi", num_layers=2, hidden_size=256, num_heads=4, num_kv_heads=4, intermediate_size=512, rotary_dim=32)
+    model = build_model(cfg, dtype=torch.bfloat16, device="cuda", seed=3)
+    kv, at = KVCache(cfg, 1, 8, dtype=model.dtype, device="cuda"), lambda n: torch.tensor([n], dtype=torch.int32, device="cuda")
+    ctx = AttnCtx("decode", 1, 1, at(0), at(1), 1, kv.rows(0, 1), model.rope_table())
+    x = torch.randn(1, 256, generator=torch.Generator().manual_seed(0)).bfloat16().cuda()
+    with torch.no_grad():
+        a, h = model.layers[0](x, None, ctx)
+        assert isinstance(a, torch.Tensor) and (a + h).shape == x.shape
+        y, r = model.forward_layers(x, ctx)
+    assert isinstance(y, torch.Tensor) and (y + r).shape == x.shape
+
+
 def _l8(g, N, K, bias=True):
     from edgellm.models.layers import Linear
     from edgellm.quant.linear import LLMInt8Linear
