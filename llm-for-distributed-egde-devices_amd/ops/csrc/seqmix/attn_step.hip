@@ -15,6 +15,9 @@
 #include "common.h"
 #include "seqmix/seqmix_common.h"
 
+extern "C" int edge_sm_attention_rmax(int rows, int H, int G, int D, int Dv);
+extern "C" int edge_sm_attention_splits(int rows, int G, int chunks);
+
 namespace {
 
 __device__ __forceinline__ float row16_max(float v) {
@@ -352,6 +355,34 @@ int run_step(const StepArgs& a, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// Estimates in us, fitted to both kernels' times at 936 points (13 shapes of 8 to 64 heads of 32 to 320 numbers, both types, 1 to 400 rows
+// behind 17 to 8000 keys; half of them are within 7 %): a launch, then the longer of one workgroup's chain and the chip's work per CU,
+// then the sum over key splits.
+constexpr double LAUNCH_US = 4.5, MERGE_US = 4.5;
+
+// groups workgroups of sh heads, each over its part of vis keys, 128 a round; a round's numbers count as the kernel pads them
+double step_us(int f32, int sh, int D, int Dv, long groups, long vis, int ns) {
+  static const double fit[2][2][5] = {{{0.57, 0.0043, 0.0017, 0.21, 0.0037}, {1.8, 0.0063, 0.0071, 0.73, 0.0053}},
+                                      {{0.28, 0.0096, 0.002, 0.13, 0.01}, {1.4, 0.014, 0.0068, 0.5, 0.016}}};
+  const double* p = fit[f32 ? 1 : 0][sh == 4];
+  const int w = D <= 64 && Dv <= 64 ? 128 : D <= 128 && Dv <= 128 ? 256 : D <= 192 && Dv <= 128 ? 320 : 576;
+  const double rounds = (double)(((vis + 127) / 128 + ns - 1) / ns), chain = p[0] + rounds * p[1] * w;
+  const double work = groups / 256.0 * (p[2] * w + rounds * (p[3] + p[4] * w));
+  return LAUNCH_US + (chain > work ? chain : work) + (ns > 1 ? MERGE_US : 0.);
+}
+
+// attn_kernel on fp32 rows, with the heads and splits that its own rules give it
+double attn_kernel_us(int rows, int H, int G, int D, int Dv, long vis) {
+  const int R = H / G, rm = edge_sm_attention_rmax(rows, H, G, D, Dv);
+  if (rm == 0) return 1e30;
+  const int ns = edge_sm_attention_splits(rows, G, (int)((vis + 255) / 256));
+  const double chunks = (double)(((vis + 255) / 256 + ns - 1) / ns), keys = (double)vis / ns;
+  const double chain = chunks * (2.6 + 0.0099 * D * rm) + keys * (0.0019 + 2.3e-5 * Dv * rm);
+  const double work = rows * (double)G * ((R + rm - 1) / rm) * ns / 256.0 *
+                      (0.99 + keys * 1.5e-4 * (D + Dv) + chunks * 0.0068 * D * rm);
+  return LAUNCH_US + (chain > work ? chain : work) + (ns > 1 ? MERGE_US : 0.);
+}
+
 }  // namespace
 
 extern "C" int edge_sm_attn_merge(const float* part, const void* gate, int gate_ld, void* out, int rows, int H, int G, int Dv, int nsp,
@@ -366,19 +397,39 @@ int edge_sm_attention_step_plan(int rows, int H, int G, int D, int Dv, int kld, 
   if (rows < 1 || G < 1 || H % G || D < 8 || Dv < 8 || D > 320 || Dv > 256 || D % 8 || Dv % 8 || kld % 8 || vld % 8 || addresses % 16 ||
       page < 1 || (page & (page - 1)) || pool < 0 || (pool & (pool - 1)) || pool > page || (pool > 0 && (D > 128 || Dv > 128)))
     return 0;
-  // One head a workgroup while that leaves no CU more than one, four (one reading of the keys, one product for their scores) for more
-  // queries; not for one or two heads a kv head, of which three or two places would stay empty, nor for long fp32 rows, whose
-  // products on the matrix cores cost more than attn_kernel's.  us, attn_kernel / one / four: fp32, 16 heads of 64 in 4 groups, 16
-  // tokens behind 100 14.2 / 6.0 / 7.2, 1024 behind 300 174 / 364 / 149; bf16 of 128, 16 behind 300 24.2 / 8.4 / 10.4, 128 behind 300 43.5 /
-  // 39.7 / 24.0; fp32 rows of 160, 4 behind 900 21.2 / 22.6 / 32, 200 behind 200 46.7 / 142 / 69
-  const int sh = (long)rows * H <= 256 ? 1 : 4;
-  if (sh == 4 && (H / G < 3 || (f32 && D > 128))) return 0;
-  const long groups = (long)rows * G * ((H / G + sh - 1) / sh);
-  // Keys are split where one workgroup would walk more than 1536 (512 of long fp32 rows): the sum over the splits is a launch more,
-  // which a captured step pays however short its sequences are.  us, 6 tokens behind 1100, window 1024 and 34 blocks, whole / split:
-  // 14.3 / 17.9, 2 behind 300 6.6 / 8.9; without a window, 2 behind 8000, 44 (attn_kernel) / 22.6
-  const long each = f32 && D > 128 ? 512 : 1536, want = vis <= each ? 1 : (vis + 511) / 512, room = groups >= 1024 ? 1 : 1024 / groups;
-  return sh + 8 * (int)(want < room ? (want < 16 ? want : 16) : (room < 16 ? room : 16));
+  // One head a workgroup for few heads altogether; with more, four (one reading of the keys, one product for their scores), but not
+  // for one or two heads a kv head, of which three or two places would stay empty.
+  const int R = H / G, per4 = (R + 3) / 4;
+  const bool few = (long)rows * H <= 256;
+  const long groups4 = (long)rows * G * per4;
+  if (!few) {
+    if (R < 3) return 0;
+    // fp32 rows: attn_kernel multiplies without the matrix cores' idle rows and is ahead once its workgroups fill the chip (us,
+    // attn_kernel / four heads: 16 heads of 64 in 4 groups, 64 rows behind 400 19.8 / 15.6, a portion of 150 behind 1000 42 / 49; of 128, 64
+    // behind 700 43 / 37, 400 behind 17 37 / 49; rows of 160, 256 behind 200 45 / 61) or splits long keys (64 heads of 128 in 8, 8
+    // behind 8000 135 / 153)
+    if (f32 && (D > 128 || groups4 * 4 * per4 * 64 > (D <= 64 ? 512L * D : 256L * 64) * R || (vis > 2500 && (long)rows * G <= 64)))
+      return 0;
+    // one chunk of attn_kernel's with all heads of a group in it (bf16, 64 heads of 128 in 8 groups, 256 rows behind 200 109 / 125)
+    if (!f32 && per4 > 1 && groups4 >= 2048 && vis <= 256 && D >= 128) return 0;
+  }
+  // Of what is left the quickest by estimate: heads a workgroup, and workgroups for a query's keys.  For few heads of fp32 rows
+  // attn_kernel is one of the choices; four heads a workgroup or long walks are not.  Keys are split from 1536 on (512 of fp32 rows): the
+  // sum is a launch more, which a step whose sequences are far shorter than vis pays too.  us, attn_kernel / these forms' choice: fp32,
+  // 16 heads of 64 in 4 groups, 1 row behind 700 14.8 / 11.5, 8 rows behind 8000 37 (attn_kernel's), of 128, 1 behind 2000 20.4 / 18.5; rows
+  // of 160, 8 behind 200 14.8 / 11.8, 16 behind 4000 53 (attn_kernel's); bf16 rows of 320, 4 behind 700 34 / 21, 16 behind 8000 159 / 64
+  double best = few && f32 ? attn_kernel_us(rows, H, G, D, Dv, vis) / 1.04 : 1e30;
+  int plan = 0;
+  for (int sh = 1; sh <= 4; sh += 3) {
+    if (sh == 1 ? !few : R < 3 || (few && f32)) continue;
+    const long groups = (long)rows * G * ((R + sh - 1) / sh);
+    for (int ns = 1; ns <= 16; ns *= 2) {
+      if ((ns > 1 && (vis <= (f32 ? 512 : 1536) || vis < 256 * ns || groups * ns > 1024)) || (few && f32 && vis > 1100L * ns)) continue;
+      const double us = step_us(f32, sh, D, Dv, groups * ns, vis, ns);
+      if (us < best) { best = us; plan = sh + 8 * ns; }
+    }
+  }
+  return plan;
 }
 
 size_t edge_sm_attention_step_floats(int rows, int H, int G, int Dv, int plan) {

@@ -79,6 +79,18 @@ def test_splits_bias_and_view(dt):
     _check(dt, [3000, 1, 1700], 8, 2, 96, 96, run)
 
 
+@pytest.mark.parametrize("dt,H,G,D,Dv,lens", [
+    (torch.bfloat16, 16, 1, 320, 256, [2600, 900, 2599, 1] * 2),   # four heads a workgroup, split
+    (torch.bfloat16, 8, 8, 64, 64, [2100]),                         # one head, split
+    (torch.bfloat16, 16, 4, 64, 64, [1600] * 17),                   # more than 256 heads, split
+    (torch.float32, 16, 4, 128, 128, [2000, 3]),                    # one head, split
+    (torch.float32, 16, 1, 160, 128, [1300] * 12),                  # the general kernel's, split
+    (torch.float32, 12, 3, 64, 64, [70] * 30)])                     # four heads a workgroup, whole
+def test_every_form_of_the_plan(dt, H, G, D, Dv, lens):
+    _check(dt, lens, H, G, D, Dv, lambda q, k, v, kb, vb, m, on: S.window_pool_attention(
+        q, None, k, v, None, None, m, D ** -0.5, None, None), latent=G == 1)
+
+
 def test_scores_of_minus_infinity_and_page_sizes():
     """A key whose score is -inf has no weight; pages that are no power of two stay with the general kernel."""
     for page in (16, 24):
