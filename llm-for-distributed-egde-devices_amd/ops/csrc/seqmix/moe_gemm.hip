@@ -13,7 +13,7 @@
 // gather, the activation and the scatter as launches of their own: 4096 tokens x 3 of 16 experts 1024 -> 1024,
 // 758 -> 127 us (610 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 664 us (874); 512 x 4 of 32, 2048 -> 2048,
 // 1369 -> 169 us, where the experts' 805 MB (4.8 TB/s) are the bound.  At 128-row tiles the bound is the LDS: 64 B per clock and
-// CU come in and 128 are read at the full MFMA rate (tall_tiles says what 256-row tiles change); 128 x 256 tiles gained 3-6 %
+// CU come in and 128 are read at the full MFMA rate (tile_rows says what 256-row tiles change); 128 x 256 tiles gained 3-6 %
 // from 2048 columns on and lost below, deeper rings with one workgroup of 128 x 128 per CU lose 40 %.
 #include "seqmix_common.h"
 
@@ -258,27 +258,46 @@ int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* 
   return (int)hipGetLastError();
 }
 
-// Rows of a tile by the average rows per expert: a tile much taller than that multiplies padding, and below about 24
-// the weights' bytes are all that counts (32 rows: two fragments, the smallest ring).  From some 50 rows on about half of the
-// experts need a second 64-row tile, which reads their weights once more for a few rows: with experts of 2^26 numbers or more
-// together 128 rows pay from there (us for both products, 64 / 128: 4 of 32 of 2048 x 2048, 49 rows an expert 161 / 164, 52 173 / 166,
-// 65 196 / 169, 73 241 / 172), with fewer, which leave CUs without a tile, only from 128 on (3 or 4 of 16 of 1024 x 1024, 75 rows
-// 35 / 38, 100 34 / 40, 131 46 / 46, 188 51 / 47)
-int tile_rows(int64_t R, int E, int W, int ff) {
-  return R > (int64_t)E * ((int64_t)E * W * ff >= 1 << 26 ? 50 : 128) ? 128 : R > (int64_t)E * 24 ? 64 : 32;
+// Row tiles of E experts that R pairs fall on at random: a normal count an expert, sum over k of P(count > k BM), the first always
+// (an expert without rows costs its launch slot too)
+double expected_tiles(double R, int E, int BM) {
+  const double m = R / E, s = sqrt(m > 1. ? m : 1.);
+  double n = 1.;
+  for (int k = 1; k * BM < m + 5. * s; ++k) n += 0.5 * (1. + erf((m - k * BM) / (s * 1.4142135623730951)));
+  return E * n;
 }
-// 256 x 256 tiles (one workgroup of 8 waves a CU, 128 x 64 a wave) halve what 128 x 128 ones (two workgroups of 4 waves, 64 x 64)
-// read from and bring into the LDS per product, which is their bound, but fill the chip in whole rounds of 256 workgroups and
-// multiply more padding.  So both times are estimated, from us a 64-k stage and us a workgroup's start and end fitted to both
-// sides, half a tile of padding an expert.  us for both products, 128 / 256: 3 of 32 experts of 2048 -> 3072 (relu2), 1000 tokens
-// 204 / 223, 4096 534 / 400, 7680 760 / 664 (874 TFLOP/s); 4 of 32 of 2048 -> 2048, 7600 976 / 781 (980 TFLOP/s); 3 of 16 of 1024
-// -> 1024, 2048 82 / 85, 4096 134 / 127; 4 of 16, 4096 171 / 195, 7600 280 / 256
-bool tall_tiles(int64_t R, int E, int W, int ff, int up) {
-  auto tiles = [&](int64_t BM) { const int64_t t = R / BM + E / 2; return t > E ? t : E; };
-  const int fn = up == 2 ? 2 : 1;                            // gated units: half a tile's weight rows are features
-  auto tall = [&](int N, int K) { return (double)((tiles(256) * ((N + 255) / 256) + 255) / 256) * (1.5 * K / 64 + 12.8); };
-  auto low = [&](int N, int K) { return tiles(128) * ((N + 127) / 128) / 512.0 * (0.94 * K / 64 + 10.2); };
-  return tall(ff * fn, W) + tall(W, ff) < low(ff * fn, W) + low(W, ff);
+// us of both products with tiles of BM rows, fitted to 525 points (15 sets of 8 to 64 experts of 512 to 4096 x 512 to 4096, 26 to 1300 rows
+// an expert; half of the estimates are within 5 %): workgroups come in rounds of 512 (two to a CU; 256 of the 256-row tiles), a round
+// costs its 64-k stages and its start and end, and a partly filled last round more than its share; the experts' bytes are partly
+// hidden behind that, or (256 rows) bound it from below.
+double tile_us(int BM, double R, int E, int W, int ff, int up) {
+  //                              us a stage, a start, both launches, TB/s, whole rounds' part
+  static const double fit[3][5] = {{0.621, 4.35, 5.4, 9.36, 0.266}, {0.991, 7.2, 3.53, 13.3, 0.429}, {1.64, 16.1, 5.69, 4.04, 0.585}};
+  const double* p = fit[BM == 64 ? 0 : BM == 128 ? 1 : 2];
+  const int BN = BM == 256 ? 256 : 128, slots = BM == 256 ? 256 : 512;
+  const double tiles = expected_tiles(R, E, BM);
+  double us = p[2];
+  for (int j = 0; j < 2; ++j) {
+    const int N = j ? W : ff * up, K = j ? ff : W;
+    const double x = tiles * ((N + BN - 1) / BN) / slots, rounds = p[4] * ceil(x - 0.02) + (1. - p[4]) * x;
+    const double work = rounds * (p[0] * K / 64 + p[1]), bytes = 2e-6 * E * N * K / p[3];
+    us += BM == 256 ? (work > bytes ? work : bytes) : work + bytes;
+  }
+  return us;
+}
+// Rows of a tile: up to 24 an expert the weights' bytes are all that counts (32 rows: two fragments, the smallest ring); above, the
+// quickest by estimate.  A tile much taller than an expert's rows multiplies padding, a lower one reads the weights once more for an
+// expert's second tile, and 256 x 256 tiles (one workgroup of 8 waves a CU, 128 x 64 a wave) halve what 128 x 128 ones read from and
+// bring into the LDS per product, which is their bound, but fill the chip in whole rounds of 256 workgroups.  us for both products, 64 /
+// 128 / 256 rows: 32 experts of 2048 -> 3072 (relu2), 48 rows an expert 162 / 172, 60 195 / 178 / 218, 135 323 / 299 / 232, 720 760 (128) / 664
+// (874 TFLOP/s); 32 of 1024 -> 1024 (gated), 48 53 / 58, 94 72 / 62 / 77, 410 160 (128) / 133, 510 188 (128) / 201; 8 of 2048 -> 4096
+// (gated), 54 102 / 120, 150 159 / 147 / 167, 600 358 (128) / 299; 24 of 1536 -> 1536 (relu2), 250 141 / 139 / 116, 330 168 / 141 / 193.
+int tile_rows(int64_t R, int E, int W, int ff, int up) {
+  if (R <= (int64_t)E * 24) return 32;
+  const int widest = ff * up > W ? ff * up : W;              // up to half a tile a CU: the lowest (4 of 256 -> 512, 72 rows an expert 16 / 19)
+  if (expected_tiles((double)R, E, 64) * ((widest + 127) / 128) <= 128.) return 64;
+  const double low = tile_us(64, (double)R, E, W, ff, up), mid = tile_us(128, (double)R, E, W, ff, up);
+  return tile_us(256, (double)R, E, W, ff, up) < 0.97 * (low < mid ? low : mid) ? 256 : low < mid ? 64 : 128;
 }
 int max_tiles(int64_t R, int E, int BM) { return (int)((R + BM - 1) / BM + (R < E ? R : E)); }
 }  // namespace
@@ -298,8 +317,7 @@ int edge_sm_moe_gemm_ok(int64_t T, int top, int E, int W, int ff) {
 int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void* w_down, int* ints, void* y, void* out, int T,
                      int top, int E, int W, int ff, int act, const float* row_w, float limit, hipStream_t st) {
   if (edge_sm_moe_gemm_ok(T, top, E, W, ff) != 0 || act < ACT_GLU_CLAMP || act > ACT_RELU2) return -2;
-  const int R = T * top, low = tile_rows(R, E, W, ff), BM = low == 128 && tall_tiles(R, E, W, ff, act == ACT_RELU2 ? 1 : 2) ? 256 : low,
-            mt = max_tiles(R, E, BM);
+  const int R = T * top, BM = tile_rows(R, E, W, ff, act == ACT_RELU2 ? 1 : 2), mt = max_tiles(R, E, BM);
   int *rows = ints, *tiles = ints + ((R + 3) & ~3);
   // while the weights' bytes are the bound (up to some 500 rows an expert) the workgroups' k starts are spread: us for both
   // products, 32 experts of 2048 x 2048, 4 each: 24 tokens 194 / 139, 128 209 / 147 (5.5 TB/s), 384 210 / 158, 800 224 / 179,

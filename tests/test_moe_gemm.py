@@ -153,9 +153,9 @@ def test_steps_that_the_grouped_kernels_do_not_take():
 
 @gpu
 @pytest.mark.parametrize("E,W,ff,T,top", [(32, 1024, 2048, 400, 4), (32, 1024, 2048, 401, 4), (32, 1024, 1984, 401, 4), (4, 64, 64, 256, 2),
-                                          (4, 64, 64, 257, 2)])
+                                          (4, 64, 64, 257, 2), (32, 1024, 2048, 488, 4), (32, 1024, 2048, 492, 4)])
 def test_lines_between_tile_heights(E, W, ff, T, top, every_size):
-    """Rows per expert on both sides of 50 (experts of 2^26 numbers together) and of 128, numbers on both sides of 2^26."""
+    """Rows per expert around 50, 60 and 128: 488 tokens run 64-row tiles by estimate, 492 run 128-row ones."""
     g = torch.Generator(device="cuda").manual_seed(T + ff)
     r = lambda *s: torch.randn(*s, generator=g, device="cuda")
     h, w_gu, w_down = r(T, W).bfloat16(), (r(E, ff, W) * W ** -0.5).bfloat16(), (r(E, W, ff) * ff ** -0.5).bfloat16()
@@ -170,9 +170,11 @@ def test_lines_between_tile_heights(E, W, ff, T, top, every_size):
 
 @gpu
 @pytest.mark.parametrize("act,T,top,E,W,ff", [("glu_clamp", 5200, 3, 7, 960, 1088), ("silu_glu", 5200, 3, 7, 960, 1088),
-                                              ("relu2", 10200, 2, 5, 2048, 2048)])
+                                              ("relu2", 10200, 2, 5, 2048, 2048), ("glu_clamp", 4600, 3, 7, 960, 1088),
+                                              ("silu_glu", 4600, 3, 7, 960, 1088)])
 def test_tall_tiles(act, T, top, E, W, ff):
-    """Sizes whose estimate chooses 256 x 256 tiles, with remainders of rows and columns (960 = 3 x 256 + 192)."""
+    """Sizes whose estimates choose 256 x 256 tiles (10200 and 4600 tokens) or nearly do, with remainders of rows and columns (960 = 3 x 256
+    + 192)."""
     g = torch.Generator(device="cuda").manual_seed(T)
     r = lambda *s: torch.randn(*s, generator=g, device="cuda")
     h, w_gu = r(T, W).bfloat16(), (r(E, ff if act == "relu2" else 2 * ff, W) * W ** -0.5).bfloat16()
