@@ -1,8 +1,8 @@
 // A sublayer's result joins the fp32 residual stream and the row that the next sublayer (or the output projection) reads is formed in
 // the same launch, for the three kinds of layers that do the two in a row: LayerNorm of the result, then the stream's four-tap
 // convolution (steps in which every sequence brings one token) or, behind the last layer, its LayerNorm; group RMS norm of the
-// result, then the next group RMS norm; the two branches of a parallel mixer, then the next RMS norm.  (ops/seqmix.py has the rules; widths, types and addresses that do not fit run the separate
-// kernels.)
+// result, then the next group RMS norm; the two branches of a parallel mixer, then the next RMS norm.  (ops/seqmix.py has the rules;
+// widths, types and addresses that do not fit run the separate kernels.)
 //
 // Bound by latency on decode-sized steps: each of the two launches was one chain of loads, a reduction over the row and a store, and
 // the second began by reading back what the first had written.  A workgroup holds a row in registers, four numbers per access, and
@@ -307,6 +307,9 @@ int edge_sm_group_residual_norm(float* x, const void* y, const void* parts, cons
   if (groups < 1 || groups2 < 1 || W % groups || W % groups2 || W / groups % 256 || W / groups2 % 256 ||
       !row_ok(W, {x, y, parts, w, w2, out}))
     return -2;
+  // long rows and many: a thread's four runs with both norms' weights leave too few wavefronts in flight (us, two launches / one, bf16 rows
+  // of 3072: 256 rows 10.9 / 10.5, 1024 17.5 / 21.9, 8192 81 / 110)
+  if (W > 8 * NT && rows > 512) return -2;
   if (rows == 0) return 0;
   const int gs = W / groups, gs2 = W / groups2;
   if (f32) RN_CH(group_residual_norm_kernel, float, x, (const float*)y, (const float*)parts, pw, K, w, W, gs, eps, mult, w2, gs2,

@@ -84,6 +84,20 @@ def test_group_norm_then_group_norm(dt, W, groups, groups2, T, K, with_y, with_w
 
 
 @pytest.mark.parametrize("dt", DT)
+@pytest.mark.parametrize("T,W", [(512, 2304), (513, 2304), (513, 2048)])
+def test_group_norms_of_many_rows(dt, T, W):
+    """Both sides of the line from which long rows run two launches."""
+    g = torch.Generator().manual_seed(T)
+    x, w, w2 = _rand(g, T, W), _rand(g, W), _rand(g, W)
+    y, parts, pw = _results(g, T, 2, W, dt, True, True)
+    a, xa = x.cuda(), x.clone()
+    h = S.group_norm_residual_norm(a, cuda(y), cuda(w), 1, 1e-6, 0.3, cuda(parts), cuda(pw), cuda(w2), 1, 1e-5, dt)
+    ref = S.group_norm_residual_norm(xa, cpu(y), w, 1, 1e-6, 0.3, cpu(parts), pw, w2, 1, 1e-5, torch.float32)
+    _near(a, xa, torch.float32)
+    _near(h, ref, dt)
+
+
+@pytest.mark.parametrize("dt", DT)
 @pytest.mark.parametrize("W", [64, 256, 1020, 1024, 2052, 4096, 4100, 1022])
 @pytest.mark.parametrize("T,extra", [(1, True), (6, False)])
 def test_combine_then_norm(dt, W, T, extra):
