@@ -235,6 +235,15 @@ class MLP(nn.Module):
         return self.down(h, add=add)
 
 
+# The launch with the up projection gives every query head a workgroup of its own, which reads a key once per head of its group; the
+# attention's own launch shares those readings once it has workgroups enough.  So grouped heads stay together up to so many rows x
+# keys.  us a layer in a graph, separate / together, bf16: 16 heads of 256 in 4 groups (4096 x 8192), 4 rows behind 4000 88.3 / 80.9,
+# 8000 95.8 / 106.9, 2 behind 8000 83.9 / 78.3; 32 of 80 in 8 (2560 x 10240), 4 behind 4000 70.0 / 69.6, 8000 80.3 / 83.6, 2 behind 8000
+# 67.0 / 67.5; without groups together at any length (32 of 80, 4 behind 8000 109.9 / 98.5; 8 of 256, fp16, 85.2 / 78.6; LLM.int8 1 behind
+# 8000 55.3 / 47.1)
+PAIR_GROUPED_KEYS = 1 << 14
+
+
 class DecoderLayer(nn.Module):
     """One decoder block.  ``has_attn`` / ``has_mlp`` False builds half a block (sequential-residual
     architectures only): a pipeline stage boundary may then fall between the attention half
@@ -302,6 +311,7 @@ class DecoderLayer(nn.Module):
                 and all(type(m) is kind for m in (qkv, o, up, down)) and up.pair_ok(up=True) and o.pair_ok() and down.pair_ok()
                 and (kind is Linear or o.in_features <= 4096 < down.in_features)
                 and self.norm1.eps == (self.norm2 or self.norm1).eps
+                and (self.cfg.num_heads == self.cfg.num_kv_heads or ctx.B * ctx.max_len <= PAIR_GROUPED_KEYS)
                 and unwatched(self.attn, self.mlp, qkv, o, up, down))
 
     def _pair(self, x, residual, ctx: AttnCtx):

@@ -158,6 +158,24 @@ def test_layers_that_a_program_steps_itself_give_rows(cuda):
     assert isinstance(y, torch.Tensor) and (y + r).shape == x.shape
 
 
+@pytest.mark.parametrize("kv_heads,B,keys,together", [(2, 4, 4096, True), (2, 4, 4097, False), (4, 4, 4097, True)])
+def test_long_caches_of_grouped_heads_run_apart(cuda, kv_heads, B, keys, together, monkeypatch):
+    from edgellm.engine import KVCache
+    from edgellm.models import AttnCtx, build_model, tiny
+    from edgellm.models.decoder import DecoderLayer
+    cfg = tiny("phi", num_layers=2, hidden_size=256, num_heads=4, num_kv_heads=kv_heads, intermediate_size=512, rotary_dim=32,
+               max_position_embeddings=8192)
+    model, used = build_model(cfg, dtype=torch.bfloat16, device="cuda", seed=3), []
+    real = DecoderLayer._pair
+    monkeypatch.setattr(DecoderLayer, "_pair", lambda self, *a: used.append(1) or real(self, *a))
+    kv = KVCache(cfg, B, 4100, dtype=model.dtype, device="cuda")
+    pos = torch.full((B,), keys - 1, dtype=torch.int32, device="cuda")
+    with torch.no_grad():
+        out = model(torch.ones(B, 1, dtype=torch.long, device="cuda"),
+                    AttnCtx("decode", B, 1, pos, pos + 1, keys, kv.rows(0, B), model.rope_table()))
+    assert bool(used) == together and torch.isfinite(out).all()
+
+
 def _l8(g, N, K, bias=True):
     from edgellm.models.layers import Linear
     from edgellm.quant.linear import LLMInt8Linear
