@@ -831,7 +831,11 @@ __device__ __forceinline__ void w8a8_gemv_body(int bid, const int8_t* __restrict
 #pragma unroll
   for (int j = 0; j < TPW; ++j) {
     const int nt = L8G_N ? (j == 0 ? nt0 : nt0 + NTt / 2) : min(nt0 + t0 + j, NTt - 1);
-    wp[j] = reinterpret_cast<const v4i*>(Wp + ((size_t)nt * KT) * 1024) + lane;
+    // (the offset stays a scalar product: added to the lane's address in one go it is three vector multiplications in front of the first
+    // weights; one row behind RMSNorm, us, so / scalar: 12288 x 4096 11.30 / 11.12, 22016 x 4096 18.99 / 18.68)
+    size_t panel = (size_t)nt * KT * 1024;
+    asm("" : "+s"(panel));
+    wp[j] = reinterpret_cast<const v4i*>(Wp + panel) + lane;
   }
   const int8_t* ap[MB];
 #pragma unroll
