@@ -900,7 +900,8 @@ __global__ void __launch_bounds__(RF_WAVES * 64) route_few_kernel(const T* __res
 
 // whether one launch takes the step
 inline bool route_few_ok(int rows, int W, int E, int gate) {
-  return rows <= 512 && E + gate <= RF_SCORES && W % 8 == 0 && W <= 2048;
+  // (three scores a wave over long rows: one workgroup a CU; 47 of 2048, bf16, 256 rows 12.1 / 8.8, 300 12.0 / 12.5, 512 12.9 / 13.8)
+  return rows <= (E + gate > 32 && W > 1536 ? 256 : 512) && E + gate <= RF_SCORES && W % 8 == 0 && W <= 2048;
 }
 
 template <typename T, bool GROUPED>

@@ -1100,8 +1100,8 @@ def moe_experts_shared(h: torch.Tensor, idx: torch.Tensor, w_up: torch.Tensor, w
 # Steps of up to so many tokens run a clamped gated shared expert beside the routed ones (moe_rows.h: two launches instead of five,
 # the shared rows read once for four tokens), up to 12 where it is small.  us, apart / together, 3 of 16 experts of 1024 x 1024 and a
 # shared one: 1 token 20.4 / 10.7, 4 28.2 / 19.6, 8 34.1 / 29.4, 9 35.6 / 32.7; 3 of 32 of 2048 x 2048: 1 35.5 / 23.9, 4 64.5 / 56.5,
-# 8 91.5 / 90.4, 9 102.8 / 106.8; 2 of 8 of 256 x 128, 12 15.2 / 9.0
-MOE_GLU_SHARED_MAX, MOE_GLU_SHARED_SMALL = 8, 1 << 23
+# 8 91.5 / 90.4, 9 102.8 / 106.8; with a shared one of 1024 x 2048, 8 40.5 / 35.3, 9 38.7 / 41.2; 2 of 8 of 256 x 128, 12 15.2 / 9.0
+MOE_GLU_SHARED_MAX, MOE_GLU_SHARED_SMALL = 8, 1 << 22
 
 
 def moe_experts_glu_shared(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor, limit: float,
