@@ -103,8 +103,8 @@ def test_decode_steps_agree_with_the_separate_launches(cuda, family, dtype, monk
     assert math.isfinite(float(k1.float().abs().max()))
 
 
-def _stepped(model, steps=2):
-    """Logits of a two-token prompt and some decode steps of one sequence, through the model's own call."""
+def _stepped(model, steps=2, caches=False):
+    """Logits (and caches) of a two-token prompt and some decode steps of one sequence, through the model's own call."""
     from edgellm.engine import KVCache
     from edgellm.models import AttnCtx
     kv, rope = KVCache(model.cfg, 1, 16, dtype=model.dtype, device="cuda"), model.rope_table()
@@ -114,7 +114,7 @@ def _stepped(model, steps=2):
         out = [model(ids[:, :2], AttnCtx("prefill", 1, 2, at(0), at(2), 2, kv.rows(0, 1), rope), logits="last")]
         for t in range(steps):
             out.append(model(ids[:, 2 + t:3 + t], AttnCtx("decode", 1, 1, at(2 + t), at(3 + t), 3 + t, kv.rows(0, 1), rope)))
-    return torch.cat(out).float()
+    return (torch.cat(out).float(), kv.k, kv.v) if caches else torch.cat(out).float()
 
 
 @pytest.mark.parametrize("where", ["layer", "final_norm"])
@@ -237,3 +237,30 @@ def test_llmint8_norm_of_both_branches(cuda, K):
     n1, r = ops.layer_norm(x + x2, g1, b1, 1e-5, res)
     n2, _ = ops.layer_norm(r, g2, b2, 1e-5, None)
     assert torch.equal(h, r) and torch.equal(y, n2) and torch.equal(out, m(n1))
+
+
+@pytest.mark.parametrize("family", ["gpt_neox", "phi"])                  # two norms of the same row; one
+def test_llmint8_decode_steps_agree_with_the_separate_launches(cuda, family, monkeypatch):
+    """The layer's wiring around the int8 launches: branches into the next norm and the final norm, the second norm's weights, caches."""
+    from edgellm.models import build_model, tiny
+    from edgellm.models.decoder import DecoderLayer
+    from edgellm.quant import quantize_model
+    cfg = tiny(family, num_layers=3, hidden_size=256, num_heads=4, num_kv_heads=4, intermediate_size=4160, rotary_dim=32)
+    model, g = build_model(cfg, dtype=torch.bfloat16, device="cuda", seed=3), torch.Generator().manual_seed(4)
+    norms = [n for layer in model.layers for n in (layer.norm1, layer.norm2) if n is not None] + [model.final_norm]
+    for n in norms:                                                      # (weights of one would hide a norm in another's place)
+        n.weight.data.copy_(0.5 + torch.rand(256, generator=g))
+        n.bias.data.copy_(0.5 * torch.randn(256, generator=g))
+    model, used = quantize_model(model, "llm_int8"), []
+    real = DecoderLayer._pair
+    monkeypatch.setattr(DecoderLayer, "_pair", lambda self, *a: used.append(self.idx) or real(self, *a))
+    one, k1, v1 = _stepped(model, caches=True)
+    assert used == [0, 1, 2] * 2
+    monkeypatch.setattr(DecoderLayer, "_pair_ok", lambda self, *a: False)
+    two, k2, v2 = _stepped(model, caches=True)
+    assert used == [0, 1, 2] * 2
+    # only the attention's last bf16 rounding differs (2^-9 of a number).  o quantises those rows in steps of some 3 sigma / 127 = 0.024
+    # sigma, so about 2^-9 / 0.024 = 8 % of the numbers may move by a step: sqrt(0.08) 0.024 = 0.7 % of a branch a layer, three layers
+    for a, b in ((one, two), (k1, k2), (v1, v2)):
+        assert (a.float() - b.float()).norm() <= 0.03 * b.float().norm()
+    assert two.std() > 0 and torch.isfinite(two).all()

@@ -54,9 +54,6 @@ def test_steps(dt, H, N, P, ra, rg, n):
         wide[:, :u.shape[1]] = u.cuda()
         got = S.delta_step(wide[:, :u.shape[1]], *cols, cu(w["a2"]), cu(w["g2"]), cu(w["conv_w"]), cu(w["conv_b"]), tail_d, state_d,
                            cu(w["dt_bias"]), cu(w["A_log"]), cu(w["norm_w"]), 1e-6, S.RaggedMeta.build(seqs, table.cuda(), 16, "cuda"), H)
-        if u.shape[1] % 8 and ra:                          # the low-rank rows do not lie on 16 bytes
-            assert got is None
-            return
         ref = _apart(u, *cols, w["a2"], w["g2"], w["conv_w"], w["conv_b"], tail_c, state_c, w["dt_bias"], w["A_log"], w["norm_w"], 1e-6,
                      S.RaggedMeta.build(seqs, table, 16, "cpu"), H)
         # fp32 sums of up to 136 and 128 terms in another order; bf16: silu's rounding may fall to the neighbour in q | k | v
@@ -77,3 +74,19 @@ def test_what_stays_apart():
     assert args(us[0].cuda(), d(state), one, 4) is not None
     assert args(us[0].cuda(), d(state), one, 2) is None                       # shared q and k
     assert args(us[0].cuda(), d(state), two, 4) is None                       # a portion of two tokens
+
+
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("H,pad", [(3, 8), (8, 4)])          # the decay's rows start off eight numbers; rows lie off eight numbers apart
+def test_low_rank_rows_off_16_bytes_stay_apart(dt, H, pad):
+    us, w, tail, state, C, slots = _case(dt, H, 64, 64, 32, 32, 2, 7)
+    u = us[0]
+    wide = torch.zeros(2, (u.shape[1] + 7) // 8 * 8 + pad, dtype=dt, device="cuda")
+    wide[:, :u.shape[1]] = u.cuda()
+    d = {k: v.cuda() for k, v in w.items()}
+    tail_d, state_d = tail.cuda(), state.cuda()
+    m = S.RaggedMeta.build([(s, 5, 1) for s in slots], torch.zeros(4, 1, dtype=torch.int32, device="cuda"), 16, "cuda")
+    assert (C + H) % 8 != 0 or wide.stride(0) % 8 != 0
+    assert S.delta_step(wide[:, :u.shape[1]], C, C + H, C + H + 32, d["a2"], d["g2"], d["conv_w"], d["conv_b"], tail_d, state_d, d["dt_bias"],
+                        d["A_log"], d["norm_w"], 1e-6, m, H) is None
+    assert torch.equal(tail_d.cpu(), tail) and torch.equal(state_d.cpu(), state)             # nothing was done
