@@ -258,20 +258,26 @@ def bench_hybrid(s: dict, prompt: int, batch: int, steps: int, device, cfg: Mode
     return out
 
 
+# what the layers call in ops.seqmix, each of which a breakdown names
+STEP_OPS = ["embedding_scaled", "scalar_rms_norm", "relu2", "cat_cast", "combine_residual", "gated_group_norm",
+            "rope_paged_write", "pool_blocks", "window_pool_attention", "conv_silu", "ssd_scan", "linear_f32",
+            "embedding_bigram", "canon_conv", "layer_norm_rows", "layer_norm_residual", "rms_norm_cols", "glu_clamp",
+            "latent_write", "delta_prepare", "delta_rule_scan", "head_norm_gate", "moe_route", "moe_experts",
+            "group_rms_norm", "group_norm_residual", "chunk_attention", "delta_prepare_head", "glu_silu",
+            "hyper_read_norm", "hyper_update", "poly_norm", "qk_norm_rope_write", "unrotate_gate",
+            "embedding_learned", "parallel_update", "glu_gelu", "moe_route_grouped", "moe_experts_shared",
+            "latent_expand_write", "head_expand_gate", "gated_linear_attention", "decay_linear_attention", "softcap",
+            "parallel_step_in", "combine_residual_norm", "layer_norm_residual_canon", "layer_norm_residual_norm",
+            "group_norm_residual_norm", "delta_step", "latent_attention", "moe_experts_glu_shared"]
+
+
 def op_times(eng: RaggedEngine, entries, close=()) -> Dict[str, float]:
     """Device time per op kind over one step (sum over layers), from events around every
     ``ops.seqmix`` call and every projection (eager step: no graph)."""
     from ..ops import seqmix
     import torch.nn.functional as F
     marks: List[tuple] = []
-    names = ["embedding_scaled", "scalar_rms_norm", "relu2", "cat_cast", "combine_residual", "gated_group_norm",
-             "rope_paged_write", "pool_blocks", "window_pool_attention", "conv_silu", "ssd_scan", "linear_f32",
-             "embedding_bigram", "canon_conv", "layer_norm_rows", "layer_norm_residual", "rms_norm_cols", "glu_clamp",
-             "latent_write", "delta_prepare", "delta_rule_scan", "head_norm_gate", "moe_route", "moe_experts",
-             "group_rms_norm", "group_norm_residual", "chunk_attention", "delta_prepare_head", "glu_silu",
-             "hyper_read_norm", "hyper_update", "poly_norm", "qk_norm_rope_write", "unrotate_gate",
-             "embedding_learned", "parallel_update", "glu_gelu", "moe_route_grouped", "moe_experts_shared",
-             "latent_expand_write", "head_expand_gate", "gated_linear_attention", "decay_linear_attention", "softcap"]
+    names = STEP_OPS
     saved = {n: getattr(seqmix, n) for n in names}
     lin = F.linear
 
@@ -298,9 +304,9 @@ def op_times(eng: RaggedEngine, entries, close=()) -> Dict[str, float]:
             eng.use_graphs = False
         for n in names:
             setattr(seqmix, n, wrap(n, saved[n]))
-        from ..models import layers as L
-        orig_fwd = L.Linear.forward
-        L.Linear.forward = wrap("projections", orig_fwd)
+        from ..models import layers as L, mixers as M
+        orig_fwd, together = L.Linear.forward, M.rows_together
+        L.Linear.forward, M.rows_together = wrap("projections", orig_fwd), wrap("projections", together)
         bmm = torch.bmm
         torch.bmm = wrap("head_expansions_bmm", bmm)
         eng.step(entries)
@@ -308,7 +314,7 @@ def op_times(eng: RaggedEngine, entries, close=()) -> Dict[str, float]:
     finally:
         for n in names:
             setattr(seqmix, n, saved[n])
-        L.Linear.forward = orig_fwd
+        L.Linear.forward, M.rows_together = orig_fwd, together
         torch.bmm = bmm
         if graphs is not None:
             eng.use_graphs = graphs

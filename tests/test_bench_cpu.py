@@ -126,3 +126,17 @@ def test_bench_headinfer_cpu(n):
     assert r.returncode == 0, r.stderr[-3000:]
     d = _last_json(r.stdout)
     assert d["config"]["headinfer_heads"] == 1 and d["value"] > 0
+
+
+def test_a_step_breakdown_names_every_op_that_layers_call():
+    import os
+    import re
+    from edgellm import models
+    from edgellm.engine.ragged_bench import STEP_OPS
+    from edgellm.ops import seqmix
+    called, here = set(), os.path.dirname(models.__file__)
+    for name in ("hybrid", "layers", "mixers", "moe"):
+        with open(os.path.join(here, name + ".py")) as f:
+            called |= set(re.findall(r"seqmix\.([a-z]\w+)\(", f.read()))
+    tables = {"decay_table", "distance_bias_table", "distance_slopes"}      # laid out once, with the weights
+    assert called - tables <= set(STEP_OPS) and all(callable(getattr(seqmix, n)) for n in STEP_OPS)
