@@ -262,8 +262,9 @@ int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* 
 // (an expert without rows costs its launch slot too)
 double expected_tiles(double R, int E, int BM) {
   const double m = R / E, s = sqrt(m > 1. ? m : 1.);
-  double n = 1.;
-  for (int k = 1; k * BM < m + 5. * s; ++k) n += 0.5 * (1. + erf((m - k * BM) / (s * 1.4142135623730951)));
+  const int sure = m > 5. * s + BM ? (int)((m - 5. * s) / BM) : 0;       // (tiles that every such count fills)
+  double n = 1. + sure;
+  for (int k = sure + 1; k * BM < m + 5. * s; ++k) n += 0.5 * (1. + erf((m - k * BM) / (s * 1.4142135623730951)));
   return E * n;
 }
 // us of both products with tiles of BM rows, fitted to 525 points (15 sets of 8 to 64 experts of 512 to 4096 x 512 to 4096, 26 to 1300 rows

@@ -4,7 +4,7 @@
 // Bound by latency and, with many sequences, by the states' bytes.  ssd_kernel gives a head to one wave, a column a lane: N loads of 256
 // bytes each in a row and 64 to 128 registers of state.  Here a workgroup of four waves takes a head, a thread four columns of N P
 // / 1024 rows through 16-byte accesses, all in flight at once, and the sums over rows meet by shuffles and once in LDS.
-// us, one wave / this: 16 heads of 64 x 64, bf16, 2 tokens 12.8 / 4.0, 64 17.7 / 8.6 (7.9 TB/s out of the caches), fp32, 2 tokens 7.8 / 4.0; 32
+// us, one wave / this: 16 heads of 64 x 64, bf16, 2 tokens 12.8 / 4.0, 64 17.7 / 8.6 (3.9 TB/s, read and written), fp32, 2 tokens 7.8 / 4.0; 32
 // heads of 128 x 64, bf16, 2 tokens 25.9 / 4.3, 64 80 / 30.
 #include "common.h"
 #include "seqmix/seqmix_common.h"
