@@ -15,6 +15,7 @@ from typing import NamedTuple, Optional
 
 import torch
 import torch.nn as nn
+from torch.nn.modules import module as _hooks
 
 from .. import ops
 
@@ -288,9 +289,13 @@ class Norm(nn.Module):
 
 def unwatched(*mods: nn.Module) -> bool:
     """Nobody sees or changes these modules' own calls: no hook of theirs or for all modules, no ``forward`` set on one of them."""
-    hooks = nn.modules.module
-    return not (hooks._global_forward_hooks or hooks._global_forward_pre_hooks
-                or any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in mods))
+    if _hooks._global_forward_hooks or _hooks._global_forward_pre_hooks:
+        return False
+    for m in mods:
+        own = m.__dict__
+        if own["_forward_hooks"] or own["_forward_pre_hooks"] or "forward" in own:
+            return False
+    return True
 
 
 def plain_linear(m: nn.Module) -> bool:
