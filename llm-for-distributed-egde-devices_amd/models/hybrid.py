@@ -83,7 +83,9 @@ class HybridLayer(nn.Module):
             h = self.norm1(x, self.proj_in.weight.dtype)
         u = self.proj_in(h)
         ours = unwatched(self.mix)                         # else its call and result are the plain ones
-        pre = self.mix.step_in(u, meta, run, self.mix.in_rows, self.ff) if ours and unwatched(self.mix.left, self.mix.right) else None
+        pre = None
+        if meta.max_len == 1 and ours and unwatched(self.mix.left, self.mix.right):
+            pre = self.mix.step_in(u, meta, run, self.mix.in_rows, self.ff)
         m = self.down(seqmix.relu2(u, self.mix.in_rows, self.ff)) if self.ff and pre is None else None
         y = self.mix(x, u, meta, run, m, nxt, pre, self.down) if ours else self.mix(x, u, meta, run, m)
         return y if nxt is None else (x, y)

@@ -371,7 +371,7 @@ class ChannelDeltaMixer(nn.Module):
         nq, nk, nv, nb, na, ng = s.in_sizes
         u = self.proj_in(h)
         C = s.conv_channels
-        if plain_linear(self.a2) and plain_linear(self.g2):
+        if meta.max_len == 1 and plain_linear(self.a2) and plain_linear(self.g2):
             y = seqmix.delta_step(u, C, C + nb, C + nb + na, self.a2.weight, self.g2.weight, self.conv_w, self.conv_b, run.conv, run.ssm,
                                   self.dt_bias, self.A_log, self.norm_w, self.eps, meta, s.kv_heads)
             if y is not None:
@@ -434,10 +434,11 @@ class HeadDeltaMixer(nn.Module):
         s = self.spec
         H, C = s.heads, s.conv_channels
         u = self.proj_in(h)
-        y = seqmix.delta_step(u, C, C + H, C + 2 * H, None, None, self.conv_w, self.conv_b, run.conv, run.ssm, self.dt_bias, self.A_log,
-                              self.norm_w, self.eps, meta, s.kv_heads)
-        if y is not None:
-            return self.o(y)
+        if meta.max_len == 1:
+            y = seqmix.delta_step(u, C, C + H, C + 2 * H, None, None, self.conv_w, self.conv_b, run.conv, run.ssm, self.dt_bias,
+                                  self.A_log, self.norm_w, self.eps, meta, s.kv_heads)
+            if y is not None:
+                return self.o(y)
         qkv = seqmix.conv_silu(u, 0, C, self.conv_w, self.conv_b, run.conv, meta)
         prep = seqmix.delta_prepare_head(qkv, u, C, C + H, self.dt_bias, self.A_log, H, s.kv_heads, s.dim)
         y = seqmix.delta_rule_scan(prep, qkv, run.ssm, meta, H, s.kv_heads, s.dim, s.vdim)

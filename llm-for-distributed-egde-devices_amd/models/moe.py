@@ -57,7 +57,8 @@ class MoEFeedForward(nn.Module):
         s = self.spec
         idx, wts = seqmix.moe_route(h, self.router, s.top, s.scale, s.router, self.router_b)
         on_input = s.weight_on == "input"
-        if s.shared_ff and s.act == "glu_clamp" and not on_input and plain_linear(self.shared_gu) and plain_linear(self.shared_down):
+        if s.shared_ff and h.shape[0] <= seqmix.MOE_GLU_SHARED_MOST and s.act == "glu_clamp" and not on_input \
+                and plain_linear(self.shared_gu) and plain_linear(self.shared_down):
             both = seqmix.moe_experts_glu_shared(h, idx, self.w_gu, self.w_down, s.limit, self.shared_gu.weight,
                                                  self.shared_down.weight, s.shared_limit)
             if both is not None:

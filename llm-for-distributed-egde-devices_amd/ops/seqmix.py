@@ -1101,7 +1101,7 @@ def moe_experts_shared(h: torch.Tensor, idx: torch.Tensor, w_up: torch.Tensor, w
 # the shared rows read once for four tokens), up to 12 where it is small.  us, apart / together, 3 of 16 experts of 1024 x 1024 and a
 # shared one: 1 token 20.4 / 10.7, 4 28.2 / 19.6, 8 34.1 / 29.4, 9 35.6 / 32.7; 3 of 32 of 2048 x 2048: 1 35.5 / 23.9, 4 64.5 / 56.5,
 # 8 91.5 / 90.4, 9 102.8 / 106.8; with a shared one of 1024 x 2048, 8 40.5 / 35.3, 9 38.7 / 41.2; 2 of 8 of 256 x 128, 12 15.2 / 9.0
-MOE_GLU_SHARED_MAX, MOE_GLU_SHARED_SMALL = 8, 1 << 22
+MOE_GLU_SHARED_MAX, MOE_GLU_SHARED_MOST, MOE_GLU_SHARED_SMALL = 8, 12, 1 << 22
 
 
 def moe_experts_glu_shared(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tensor, w_down: torch.Tensor, limit: float,
@@ -1109,7 +1109,7 @@ def moe_experts_glu_shared(h: torch.Tensor, idx: torch.Tensor, w_gu: torch.Tenso
     """Clamped gated experts and the shared expert of the same form in one go, for few tokens: shared_gu [2 sff, W] (gate
     rows, then up rows), shared_down [W, sff] -> (the chosen experts' outputs [T, top, W], the shared expert's [T, W]);
     None where they do not run together."""
-    most = 12 if shared_gu.numel() + shared_down.numel() < MOE_GLU_SHARED_SMALL else MOE_GLU_SHARED_MAX
+    most = MOE_GLU_SHARED_MOST if shared_gu.numel() + shared_down.numel() < MOE_GLU_SHARED_SMALL else MOE_GLU_SHARED_MAX
     if not _gpu(h) or not 0 < h.shape[0] <= most or moe_grouped(h, idx, w_gu, w_down, "glu_clamp"):
         return None
     return _ext().sm_moe_experts_glu_shared(h, idx, w_gu, w_down, float(limit), shared_gu, shared_down, float(shared_limit))
