@@ -1,6 +1,7 @@
-"""Attention of steps of few queries (attn_step.hip) against the same op on the CPU, in fp32 over the operands' exact values: head sizes beside the four row
-layouts, one head a workgroup and four, keys beside a wave's 16, a round's 128 and a split, windows, kept first tokens, pooled
-blocks, chunks, caps, slopes, sinks, distance biases, gates and result views, and calls that stay with the general kernel."""
+"""Attention of steps of few queries (attn_step.hip) against the same op on the CPU, in fp32 over the operands' exact values:
+head sizes beside the four row layouts, one head a workgroup and four, keys beside a wave's 16, a round's 128 and a split,
+windows, kept first tokens, pooled blocks, chunks, caps, slopes, sinks, distance biases, gates and result views, and calls
+that stay with the general kernel."""
 import pytest
 import torch
 

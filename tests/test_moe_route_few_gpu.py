@@ -25,7 +25,8 @@ def _same(got, ref, z):
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("T,W,E,top", [(1, 8, 1, 1), (4, 64, 4, 2), (3, 520, 16, 3), (5, 1024, 17, 4), (9, 2048, 32, 4), (2, 2040, 33, 33),
-                                       (512, 256, 8, 2), (513, 256, 8, 2), (256, 2048, 47, 4), (257, 2048, 47, 4), (6, 512, 48, 8), (6, 512, 49, 8), (3, 2056, 16, 2)])
+                                       (512, 256, 8, 2), (513, 256, 8, 2), (256, 2048, 47, 4), (257, 2048, 47, 4),
+                                       (6, 512, 48, 8), (6, 512, 49, 8), (3, 2056, 16, 2)])
 @pytest.mark.parametrize("mode", ["softmax", "sigmoid", "top_softmax"])
 def test_plain(dt, T, W, E, top, mode):
     h, r, b = _operands(dt, T, W, E, T + W + E)
