@@ -232,7 +232,7 @@ __device__ __forceinline__ void decode_attn_body(
 #pragma unroll
       for (int u = 0; u < UNROLL; ++u)
 #pragma unroll
-        for (int h = 0; h < G; ++h) s[u][h] += __shfl_xor(s[u][h], o, 64);
+        for (int h = 0; h < G; ++h) s[u][h] = xor_sum(s[u][h], o);
 #pragma unroll
     for (int u = 0; u < UNROLL; ++u)
       if (base + kl + u * KPB >= nl) {
@@ -245,7 +245,7 @@ __device__ __forceinline__ void decode_attn_body(
 #pragma unroll
       for (int u = 1; u < UNROLL; ++u) cm = fmaxf(cm, s[u][h]);
 #pragma unroll
-      for (int o = LPK; o < 64; o <<= 1) cm = fmaxf(cm, __shfl_xor(cm, o, 64));
+      for (int o = LPK; o < 64; o <<= 1) cm = xor_max(cm, o);
       // cm is finite: key `base` (kl = 0, u = 0) is in range whenever a chunk is consumed
       const float mn = fmaxf(m[h], cm);
       const float alpha = __builtin_amdgcn_exp2f(m[h] - mn);        // 0 on the first chunk (m = -inf)
@@ -277,7 +277,7 @@ __device__ __forceinline__ void decode_attn_body(
           for (int j = 0; j < 8; ++j) sp += qf[h][j] * knew[j];
         }
 #pragma unroll
-        for (int o = LPK / 2; o > 0; o >>= 1) sp += __shfl_xor(sp, o, 64);
+        for (int o = LPK / 2; o > 0; o >>= 1) sp = xor_sum(sp, o);
         m[h] = __shfl(sp, dl, 64);                   // lane dl holds the kl = 0 group's sum
         if (kl == 1) {
           l[h] = 1.f;
@@ -312,9 +312,9 @@ __device__ __forceinline__ void decode_attn_body(
   for (int o = LPK; o < 64; o <<= 1)
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      l[h] += __shfl_xor(l[h], o, 64);
+      l[h] = xor_sum(l[h], o);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) acc[h][j] += __shfl_xor(acc[h][j], o, 64);
+      for (int j = 0; j < 8; ++j) acc[h][j] = xor_sum(acc[h][j], o);
     }
   // merge the waves: rescale each to the workgroup max
   if (lane == 0) {

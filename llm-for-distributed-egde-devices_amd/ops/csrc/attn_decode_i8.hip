@@ -75,13 +75,13 @@ __device__ __forceinline__ void unpack16u(const uint4& u, float* f) {
 template <int LPK>
 __device__ __forceinline__ float group_sum(float v) {
 #pragma unroll
-  for (int o = LPK / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+  for (int o = LPK / 2; o > 0; o >>= 1) v = xor_sum(v, o);
   return v;
 }
 template <int LPK>
 __device__ __forceinline__ float group_max(float v) {
 #pragma unroll
-  for (int o = LPK / 2; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+  for (int o = LPK / 2; o > 0; o >>= 1) v = xor_max(v, o);
   return v;
 }
 
@@ -290,7 +290,7 @@ __global__ void __launch_bounds__(NT, OCC) decode_attn_i8_kernel(
 #pragma unroll
       for (int u = 1; u < UNROLL; ++u) cm = fmaxf(cm, s[u][h]);
 #pragma unroll
-      for (int o = LPK; o < 64; o <<= 1) cm = fmaxf(cm, __shfl_xor(cm, o, 64));
+      for (int o = LPK; o < 64; o <<= 1) cm = xor_max(cm, o);
       const float mn = fmaxf(m[h], cm);            // finite: key `base` is in range
       const float alpha = __builtin_amdgcn_exp2f(m[h] - mn);
       m[h] = mn;
@@ -323,9 +323,9 @@ __global__ void __launch_bounds__(NT, OCC) decode_attn_i8_kernel(
   for (int o = LPK; o < 64; o <<= 1)
 #pragma unroll
     for (int h = 0; h < G; ++h) {
-      l[h] += __shfl_xor(l[h], o, 64);
+      l[h] = xor_sum(l[h], o);
 #pragma unroll
-      for (int j = 0; j < 16; ++j) acc[h][j] += __shfl_xor(acc[h][j], o, 64);
+      for (int j = 0; j < 16; ++j) acc[h][j] = xor_sum(acc[h][j], o);
     }
   // l was accumulated per lane group (every lane of a group holds the same l): no dim reduction
   if (lane == 0) {
@@ -496,7 +496,7 @@ __global__ void __launch_bounds__(NT, 4) decode_attn_i8_wave_kernel(
 #pragma unroll
     for (int u = 1; u < U; ++u) cm = fmaxf(cm, s[u]);
 #pragma unroll
-    for (int o = LPK; o < 64; o <<= 1) cm = fmaxf(cm, __shfl_xor(cm, o, 64));
+    for (int o = LPK; o < 64; o <<= 1) cm = xor_max(cm, o);
     const float mn = fmaxf(m, cm);
     const float alpha = __builtin_amdgcn_exp2f(m - mn);
     m = mn;
@@ -521,9 +521,9 @@ __global__ void __launch_bounds__(NT, 4) decode_attn_i8_wave_kernel(
   for (int j = 0; j < 16; ++j) acc[j] -= 128.f * vbias;
 #pragma unroll
   for (int o = LPK; o < 64; o <<= 1) {
-    l += __shfl_xor(l, o, 64);
+    l = xor_sum(l, o);
 #pragma unroll
-    for (int j = 0; j < 16; ++j) acc[j] += __shfl_xor(acc[j], o, 64);
+    for (int j = 0; j < 16; ++j) acc[j] = xor_sum(acc[j], o);
   }
   const float inv = 1.f / l;
   float o[16];

@@ -213,7 +213,7 @@ __global__ void __launch_bounds__(NT) prefill_attn_kernel(
         mx = fmaxf(mx, v);
       }
 #pragma unroll
-      for (int off = 1; off < 16; off <<= 1) mx = fmaxf(mx, __shfl_xor(mx, off, 64));
+      for (int off = 1; off < 16; off <<= 1) mx = xor_max(mx, off);
       const float mnew = fmaxf(m_i[i], mx);
       const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
       alpha[i] = __builtin_amdgcn_exp2f(m_i[i] - msafe);
@@ -225,7 +225,7 @@ __global__ void __launch_bounds__(NT) prefill_attn_kernel(
         rs += p;
       }
 #pragma unroll
-      for (int off = 1; off < 16; off <<= 1) rs += __shfl_xor(rs, off, 64);
+      for (int off = 1; off < 16; off <<= 1) rs = xor_sum(rs, off);
       l_i[i] = l_i[i] * alpha[i] + rs;
       m_i[i] = mnew;
     }

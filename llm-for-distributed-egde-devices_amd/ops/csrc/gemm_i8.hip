@@ -443,8 +443,8 @@ __global__ void __launch_bounds__((NCW + NWL + NAL) * 64, 1) w8a8_gemv_ring2_ker
           h[p][q] = g / (1.f + __expf(-g)) * u;
           amax = fmaxf(amax, fabsf(h[p][q]));
         }
-      amax = fmaxf(amax, __shfl_xor(amax, 16, 64));   // the row's 64 features sit in lanes l, l ^ 16, l ^ 32, l ^ 48
-      amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+      amax = xor_max(amax, 16);   // the row's 64 features sit in lanes l, l ^ 16, l ^ 32, l ^ 48
+      amax = xor_max(amax, 32);
       amax = fmaxf(amax, 1e-8f);
       const float inv = 127.f / amax;
       if (live && lrow < Ml) {
@@ -710,8 +710,8 @@ __global__ void __launch_bounds__((RG * TG + NWL) * 64, 1) w8a8_r256_kernel(
           h[p][q] = g / (1.f + __expf(-g)) * u;
           amax = fmaxf(amax, fabsf(h[p][q]));
         }
-      amax = fmaxf(amax, __shfl_xor(amax, 16, 64));   // the row's 64 features sit in lanes l, l ^ 16, l ^ 32, l ^ 48
-      amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+      amax = xor_max(amax, 16);   // the row's 64 features sit in lanes l, l ^ 16, l ^ 32, l ^ 48
+      amax = xor_max(amax, 32);
       amax = fmaxf(amax, 1e-8f);
       const float inv = 127.f / amax;
       if (live && (PKO ? row < Mpad : lrow < Ml)) {

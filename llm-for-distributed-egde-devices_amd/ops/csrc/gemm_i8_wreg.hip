@@ -231,8 +231,8 @@ __global__ void __launch_bounds__((NTW / TPW) * 64, 1) w8a8_wreg_kernel(
         h[j][q] = g / (1.f + __expf(-g)) * u;
         amax = fmaxf(amax, fabsf(h[j][q]));
       }
-      amax = fmaxf(amax, __shfl_xor(amax, 16, 64));   // the wave's 16 features of the row: lanes l ^ 16, l ^ 32
-      amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
+      amax = xor_max(amax, 16);   // the wave's 16 features of the row: lanes l ^ 16, l ^ 32
+      amax = xor_max(amax, 32);
       if (lane < 16) xmax[wave * 128 + j * 16 + lane] = amax;
     }
     __syncthreads();

@@ -162,7 +162,7 @@ __device__ __forceinline__ void gemv_epilogue(const v4i* __restrict__ red, const
           h[o][q] = bf2f(f2bf(g));            // the unfused activation output is bf16
           float m = fabsf(h[o][q]);
 #pragma unroll
-          for (int d = 1; d < 16; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+          for (int d = 1; d < 16; d <<= 1) m = xor_max(m, d);
           if ((lane & 15) == 0) gmax[i][t][4 * (lane >> 4) + q] = m;
         }
       }
@@ -222,7 +222,7 @@ __device__ __forceinline__ void gemv_epilogue(const v4i* __restrict__ red, const
           for (int q = 0; q < 4; ++q) {
             float m = fabsf(h[o][q]);
 #pragma unroll
-            for (int d = 1; d < 16; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+            for (int d = 1; d < 16; d <<= 1) m = xor_max(m, d);
             if ((lane & 15) == 0) gmax[i][p][4 * (lane >> 4) + q] = m;
           }
         }

@@ -97,7 +97,7 @@ __global__ void __launch_bounds__(NT) llmint8_prep_kernel(const bf16_t* __restri
   for (int m = 0; m < 16; ++m) {
     float v = am[m];
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+    for (int o = 32; o > 0; o >>= 1) v = xor_max(v, o);
     if (lane == 0) rmax[m][wave] = v;
   }
   __syncthreads();
@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(256) llmint8_quant_rows_kernel(const bf16_t* _
       if (!((tk >> j) & 1u)) am = fmaxf(am, fabsf(v[j]));
   }
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o, 64));
+  for (int o = 32; o > 0; o >>= 1) am = xor_max(am, o);
   if ((tid & 63) == 0) wmax[tid >> 6] = am;
   __syncthreads();
   const float rm = fmaxf(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3])), 1e-8f);

@@ -429,7 +429,7 @@ __global__ void __launch_bounds__(NT) group_quant_kernel(const bf16_t* __restric
 #pragma unroll
   for (int j = 0; j < 8; ++j) m = fmaxf(m, fabsf(v[j]));
 #pragma unroll
-  for (int o = 1; o < 8; o <<= 1) m = fmaxf(m, __shfl_xor(m, o, 64));
+  for (int o = 1; o < 8; o <<= 1) m = xor_max(m, o);
   m = fmaxf(m, 1e-8f);
   if (!ok) return;
   const float inv = 127.f / m;

@@ -120,8 +120,8 @@ __device__ __forceinline__ bool better(float v, int i, float bv, int bi) { retur
 __device__ __forceinline__ void wave_argmax(float& v, int& idx) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(v, o, 64);
-    const int oi = __shfl_xor(idx, o, 64);
+    const float ov = lane_xor(v, o);
+    const int oi = lane_xor(idx, o);
     if (better(ov, oi, v, idx)) { v = ov; idx = oi; }
   }
 }
@@ -146,8 +146,8 @@ __device__ __forceinline__ void block_minmax_u32(uint32_t& mn, uint32_t& mx, uin
   constexpr int W = NTT / 64;
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    mn = min(mn, (uint32_t)__shfl_xor((int)mn, o, 64));
-    mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
+    mn = min(mn, (uint32_t)lane_xor((int)mn, o));
+    mx = max(mx, (uint32_t)lane_xor((int)mx, o));
   }
   const int w = threadIdx.x >> 6;
   __syncthreads();
@@ -165,7 +165,7 @@ __device__ __forceinline__ uint32_t block_max_u32(uint32_t v, uint32_t* scratch)
 
 __device__ __forceinline__ uint32_t block_sum_u32(uint32_t v, uint32_t* scratch) {
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
+  for (int o = 32; o > 0; o >>= 1) v += (uint32_t)lane_xor((int)v, o);
   __syncthreads();
   if ((threadIdx.x & 63) == 0) scratch[threadIdx.x >> 6] = v;
   __syncthreads();
@@ -262,7 +262,7 @@ __device__ __forceinline__ void rank_and_sample(const uint64_t* fc, float* fe, i
   for (int q = 0; q < PER; ++q)
     if (tid + q * NTT < n && cval(my[q]) >= kth) tot += e[q];
 #pragma unroll
-  for (int o = 32; o > 0; o >>= 1) tot += __shfl_xor(tot, o, 64);
+  for (int o = 32; o > 0; o >>= 1) tot = xor_sum(tot, o);
   if ((tid & 63) == 0) sh[1 + (tid >> 6)] = tot;
   __syncthreads();
   tot = 0.f;
@@ -443,8 +443,8 @@ __global__ void __launch_bounds__(64) argmax_merge_kernel(const uint64_t* __rest
   for (int c = threadIdx.x; c < C; c += 64) best = max(best, pc[(size_t)row * C + c]);
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) {
-    const uint64_t other = ((uint64_t)(uint32_t)__shfl_xor((int)(best >> 32), o, 64) << 32) |
-                           (uint32_t)__shfl_xor((int)(uint32_t)best, o, 64);
+    const uint64_t other = ((uint64_t)(uint32_t)lane_xor((int)(best >> 32), o) << 32) |
+                           (uint32_t)lane_xor((int)(uint32_t)best, o);
     best = max(best, other);
   }
   if (threadIdx.x == 0) {

@@ -241,7 +241,7 @@ __global__ void __launch_bounds__(NT, (DV * RH <= 4 ? (REL && DK > 2 ? 2 : 4) : 
         mx = fmaxf(mx, v);
       }
 #pragma unroll
-      for (int o_ = 1; o_ < 16; o_ <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o_, 64));
+      for (int o_ = 1; o_ < 16; o_ <<= 1) mx = xor_max(mx, o_);
       const float mnew = fmaxf(m_i[r][i], mx);
       const float msafe = (mnew == -INFINITY) ? 0.f : mnew;
       alpha[i] = __builtin_amdgcn_exp2f(m_i[r][i] - msafe);
@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(NT, (DV * RH <= 4 ? (REL && DK > 2 ? 2 : 4) : 
         rs += p;
       }
 #pragma unroll
-      for (int o_ = 1; o_ < 16; o_ <<= 1) rs += __shfl_xor(rs, o_, 64);
+      for (int o_ = 1; o_ < 16; o_ <<= 1) rs = xor_sum(rs, o_);
       l_i[r][i] = l_i[r][i] * alpha[i] + rs;
       m_i[r][i] = mnew;
     }

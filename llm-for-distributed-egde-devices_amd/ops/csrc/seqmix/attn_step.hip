@@ -72,7 +72,7 @@ __device__ __forceinline__ void halve(float (&v)[N], int& off, int lane) {
 #pragma unroll
     for (int j = 0; j < V / 2; ++j) {
       const float give = hi ? v[j] : v[j + V / 2], keep = hi ? v[j + V / 2] : v[j];
-      v[j] = keep + __shfl_xor(give, S, 64);
+      v[j] = keep + lane_xor(give, S);
     }
     off += hi ? V / 2 : 0;
     halve<V / 2, S / 2, S0>(v, off, lane);
@@ -273,11 +273,11 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
     const float sv = sk ? a.sink[hq0 + min(r, R - 1)] : -INFINITY, mw = m_s[w][r];
     float M = fmaxf(mw, sv);
 #pragma unroll
-    for (int o = SH; o < 64; o <<= 1) M = fmaxf(M, __shfl_xor(M, o, 64));
+    for (int o = SH; o < 64; o <<= 1) M = xor_max(M, o);
     const float x = mw == -INFINITY ? 0.f : exp_neg(mw - M);
     float ls = lane < NW * SH ? x * l_s[w][r] : 0.f;
 #pragma unroll
-    for (int o = SH; o < 64; o <<= 1) ls += __shfl_xor(ls, o, 64);
+    for (int o = SH; o < 64; o <<= 1) ls = xor_sum(ls, o);
     if (sk) ls += exp_neg(sv - M);
     if (lane < NW * SH) m_s[w][r] = x;
     if (lane < SH) { tot_s[0][r] = M; tot_s[1][r] = ls; }
@@ -317,9 +317,12 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) e8[e] += r < Dv ? y * uf[e] : 0.f;
     }
-    for (int o = vl; o < 64; o <<= 1)
 #pragma unroll
-      for (int e = 0; e < 8; ++e) e8[e] += __shfl_xor(e8[e], o, 64);
+    for (int o = 1; o < 64; o <<= 1)
+      if (o >= vl) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) e8[e] = xor_sum(e8[e], o);
+      }
     if (lane < vl)
 #pragma unroll
       for (int e = 0; e < 8; ++e) e_s[wave][uc + e] = e8[e];

@@ -122,8 +122,8 @@ __global__ void __launch_bounds__(N * P / 32 < 256 ? 256 : 512) delta_step_kerne
   }
 #pragma unroll
   for (int o = PG; o < 64; o <<= 1) {
-    dk.x += __shfl_xor(dk.x, o, 64); dk.y += __shfl_xor(dk.y, o, 64); dk.z += __shfl_xor(dk.z, o, 64); dk.w += __shfl_xor(dk.w, o, 64);
-    dq.x += __shfl_xor(dq.x, o, 64); dq.y += __shfl_xor(dq.y, o, 64); dq.z += __shfl_xor(dq.z, o, 64); dq.w += __shfl_xor(dq.w, o, 64);
+    dk.x = xor_sum(dk.x, o); dk.y = xor_sum(dk.y, o); dk.z = xor_sum(dk.z, o); dk.w = xor_sum(dk.w, o);
+    dq.x = xor_sum(dq.x, o); dq.y = xor_sum(dq.y, o); dq.z = xor_sum(dq.z, o); dq.w = xor_sum(dq.w, o);
   }
   if (lane < PG) {
     *reinterpret_cast<float4*>(&sk_s[wave][p0]) = dk;

@@ -326,7 +326,7 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
       float a[8], sum = 0.f, back = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) { a[i] = B_s[seg * 8 + i][nn]; sum += a[i]; }
-      const float other = __shfl_xor(sum, 32, 64);
+      const float other = lane_xor(sum, 32);
       float fwd = seg & 1 ? other : 0.f;
       back = seg & 1 ? 0.f : other;
 #pragma unroll

@@ -107,7 +107,7 @@ __global__ void __launch_bounds__(NT) moe_rows_kernel(const T* __restrict__ in, 
     moe_rows_run<T, MODE, MT, decltype(chc)::value>(wr, xr, k, acc);
     int id = 0;
     lane_sums<V, 32>(acc, id, lane);                         // lane (64 / V) v holds sum v = row MT + pair
-    const float up = __shfl_xor(acc[0], 32, 64);             // (GLU: the up row of a gate row, two rows on)
+    const float up = lane_xor(acc[0], 32);             // (GLU: the up row of a gate row, two rows on)
     const int m = id % MT, f = f0 + id / MT;
     int pm = p[0];
 #pragma unroll

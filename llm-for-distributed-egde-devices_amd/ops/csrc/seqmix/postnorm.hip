@@ -686,8 +686,8 @@ __global__ void __launch_bounds__(64) moe_topk_kernel(const float* __restrict__ 
       if (z_s[e] > best) { best = z_s[e]; bi = e; }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
+      const float ob = lane_xor(best, o);
+      const int oi = lane_xor(bi, o);
       if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
     }
     if (bi >= E) {                                           // scores that compare with nothing (NaN): keep the ids in range
@@ -757,8 +757,8 @@ __global__ void __launch_bounds__(64) route_grouped_kernel(const float* __restri
       if (c_s[e] > best) { best = c_s[e]; bi = e; }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
-      const float ob = __shfl_xor(best, o, 64);
-      const int oi = __shfl_xor(bi, o, 64);
+      const float ob = lane_xor(best, o);
+      const int oi = lane_xor(bi, o);
       if (ob > best || (ob == best && oi < bi)) { best = ob; bi = oi; }
     }
     if (bi >= E) bi = k;                                     // scores that compare with nothing (NaN): keep the ids in range

@@ -433,7 +433,7 @@ __global__ void __launch_bounds__(NT) attn_kernel(const T* __restrict__ q, const
 #pragma unroll
       for (int e = 0; e < 8; ++e)
 #pragma unroll
-        for (int o = LPK; o < 64; o <<= 1) acc[r][e] += __shfl_xor(acc[r][e], o, 64);
+        for (int o = LPK; o < 64; o <<= 1) acc[r][e] = xor_sum(acc[r][e], o);
   }
   for (int w = 0; w < NT / 64; ++w) {
     if (wave == w) {

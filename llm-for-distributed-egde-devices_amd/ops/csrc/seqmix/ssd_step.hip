@@ -56,7 +56,7 @@ __global__ void __launch_bounds__(NT) ssd_step_kernel(SsdStep a) {
 #pragma unroll
   for (int o = PG; o < 64; o <<= 1)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) y[e] += __shfl_xor(y[e], o, 64);
+    for (int e = 0; e < 4; ++e) y[e] = xor_sum(y[e], o);
   if (lane < PG) *reinterpret_cast<float4*>(&sum_s[wave][p0]) = make_float4(y[0], y[1], y[2], y[3]);
   __syncthreads();
   if (tid < P) {
