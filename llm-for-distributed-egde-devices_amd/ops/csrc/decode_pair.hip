@@ -3,11 +3,12 @@
 //   * the o projection beside the down projection, each into rows of its own (the next layer's norm adds them up).
 // What bounds a step of such a layer is not its bytes but the launches: each costs some 3.3 us of ramp, first loads and
 // reduction beside the time of its weights, and the attention's 5 us leave the memory idle.  Five launches a layer are
-// three this way.  The workgroups are the parts' own (attn_decode.h, gemv_bf16.h) with 8 waves instead of 16, one tile of 16
-// columns each: two to a CU under 128 VGPRs, so that the attention's workgroups take no CU away from the projection.
-// The attention's come first in the grid: they are the longest chains.  us a layer of Pythia-1B, fp16, one row: attention 5.3
-// and up 8.3 are 10.3 together, o 5.0 and down 10.4 are 10.9; whole answers, one row: Pythia-1B 48 tokens 33.9 -> 28.2 ms
-// (4 rows, 32 tokens 27.6 -> 22.3), Phi-2 32 tokens 57.8 -> 47.0, 64 tokens behind 200 116.6 -> 90.5.
+// three this way.  The workgroups are the parts' own (attn_decode.h, gemv_bf16.h), one tile of 16 columns each, beside the
+// attention with 8 waves instead of 16: two to a CU under 128 VGPRs, so that the attention's workgroups take no CU away from
+// the projection (with 16 waves 9.1 -> 10.7 us).  The attention's come first in the grid: they are the longest chains.  us a
+// layer, fp16, one row, before the projections requested all of a step's weights at once and now: Pythia-1B attention with up
+// 10.3 -> 9.1, o with down 10.9 -> 9.3; Phi-2 o with down 14.7 (8 waves) -> 13.5.
+// Whole answers against five launches, one row: Pythia-1B 48 tokens 33.9 -> 26.9 ms.
 #include "decode_pair.h"
 #include "gemv_bf16.h"
 
@@ -18,16 +19,26 @@ struct Proj {
   int N, K;
 };
 
-// One workgroup of a projection: as many k-pairs in flight per wave as divide its rounds evenly (8, 5 or 4: a round that runs
-// over the end loads its last k-pair again), else 2.
-template <int EPI, bool HF>
+constexpr int OW = GEMV_NW;                // waves of an o or down workgroup
+
+// One workgroup of a projection.  8 waves: as many k-pairs in flight per wave as divide its rounds evenly (8, 5 or 4: a round
+// that runs over the end loads its last k-pair again), else 2.  16 waves: 5 where that divides the rounds, else 1 (more would
+// take the registers of the CU's second workgroup: 2048 x 8192 beside 2048 x 2048 9.3 us, with 8 in flight 11.4).
+template <int NWV, int EPI, bool HF>
 __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act) {
   const int KP = p.K / 64;
   const NormIn16 none{};
-  if (KP % (8 * PW) == 0) gemv_bf16_body<PW, 1, 1, 8, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
-  else if (KP % (5 * PW) == 0) gemv_bf16_body<PW, 1, 1, 5, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
-  else if (KP % (4 * PW) == 0) gemv_bf16_body<PW, 1, 1, 4, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
-  else gemv_bf16_body<PW, 1, 1, 2, EPI, HF, 0>(bid, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none);
+#define RUN(UU, PP) gemv_tiles_body<NWV, UU, PP, EPI, HF, 0, 1>(bid, 1 << 30, p.x, p.w, p.bias, p.out, M, p.N, p.K, act, 1, nullptr, none)
+  if constexpr (NWV == GEMV_NW) {
+    if (KP % (5 * NWV) == 0) RUN(5, 0);
+    else RUN(1, 1);
+  } else {
+    if (KP % (8 * NWV) == 0) RUN(8, 0);
+    else if (KP % (5 * NWV) == 0) RUN(5, 0);
+    else if (KP % (4 * NWV) == 0) RUN(4, 0);
+    else RUN(2, 0);
+  }
+#undef RUN
 }
 
 // Three projections of the same rows (a parallel layer of attention, recurrence and feed-forward); d first, its chains are the
@@ -36,7 +47,7 @@ __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act
 template <bool HF>
 __global__ void __launch_bounds__(PW * 64, 4) rows3_kernel(Proj d, Proj o, Proj r, int M) {
   const int nd = d.N / 16, no = nd + o.N / 16, bid = blockIdx.x;
-  proj_body<EPI_OUT, HF>(bid < nd ? bid : bid < no ? bid - nd : bid - no, bid < nd ? d : bid < no ? o : r, M, 0);
+  proj_body<PW, EPI_OUT, HF>(bid < nd ? bid : bid < no ? bid - nd : bid - no, bid < nd ? d : bid < no ? o : r, M, 0);
 }
 
 template <int D, bool DIRECT, bool HF>
@@ -46,16 +57,16 @@ __global__ void __launch_bounds__(PW * 64, 4) attn_up_kernel(AttnArgs a, Proj p,
   if (bid < na) {
     attn_part<D, DIRECT, HF>(smem, bid, a);
   } else {
-    proj_body<EPI_GELU_ANY, HF>(bid - na, p, M, act);
+    proj_body<PW, EPI_GELU_ANY, HF>(bid - na, p, M, act);
   }
 }
 
 // The down projection's workgroups first: their chains are the longer ones.
 template <bool HF>
-__global__ void __launch_bounds__(PW * 64, 4) o_down_kernel(Proj o, Proj d, int M) {
+__global__ void __launch_bounds__(OW * 64) o_down_kernel(Proj o, Proj d, int M) {
   const int nd = d.N / 16, bid = blockIdx.x;
   const bool down = bid < nd;
-  proj_body<EPI_OUT, HF>(down ? bid : bid - nd, down ? d : o, M, 0);
+  proj_body<OW, EPI_OUT, HF>(down ? bid : bid - nd, down ? d : o, M, 0);
 }
 
 template <bool HF>
@@ -101,7 +112,7 @@ extern "C" int edge_o_down(const void* x, const void* wo, const void* bo, void* 
   if (M < 1 || M > 4 || N <= 0 || N % 16 != 0 || Ko <= 0 || Ko % 64 != 0 || Kd <= 0 || Kd % 64 != 0) return -2;
   const Proj o{(const bf16_t*)x, (const bf16_t*)wo, (const bf16_t*)bo, (bf16_t*)a, N, Ko};
   const Proj d{(const bf16_t*)h, (const bf16_t*)wd, (const bf16_t*)bd, (bf16_t*)y, N, Kd};
-  const dim3 grid(2 * (N / 16)), block(PW * 64);
+  const dim3 grid(2 * (N / 16)), block(OW * 64);
   if (h16) hipLaunchKernelGGL(o_down_kernel<true>, grid, block, 0, st, o, d, M);
   else hipLaunchKernelGGL(o_down_kernel<false>, grid, block, 0, st, o, d, M);
   return (int)hipGetLastError();

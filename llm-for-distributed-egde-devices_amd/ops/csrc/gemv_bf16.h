@@ -256,20 +256,172 @@ __device__ __forceinline__ void norm16_prologue(const NormIn16& na, bool wg0, in
   __syncthreads();                                        // the rows are complete in LDS
 }
 
-// One workgroup (bid) of the GEMV, NWV waves.
-template <int NWV, int MB, int NTW, int U, int EPI, bool HF, int NRM>
-__device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
-                                               const bf16_t* __restrict__ bias, bf16_t* __restrict__ out, int M, int N,
-                                               int K, int F, int S, const bf16_t* __restrict__ add, const NormIn16& na) {
-  static_assert(EPI != EPI_GLU || NTW % 2 == 0, "GLU: gate/up tile pairs");
-  static_assert(MB * NTW <= 8 && MB * (EPI == EPI_GLU ? NTW / 2 : NTW) <= NWV, "LDS reduction / output waves");
-  static_assert(NRM == 0 || (NWV == GEMV_NW && MB == 1 && NTW <= 4 && EPI != EPI_PART), "norm prologue: up to 4 rows, LDS budget");
-  __shared__ v4f red[NWV][MB * NTW][64];
-  // NRM: 8 NCH + SMAX (RMSNorm over split-K slices), + 64 for the LayerNorm of 16-bit rows
+// Workgroup bid of nwg of the GEMV of one row block (M <= 16): 16-column tiles bid, bid + nwg, ... one after the other,
+// NWV waves that split K, U k-pairs of a wave requested before the first is used.
+// What bounds it is the chain of memory round trips, so every load of a step is issued before any use (the fence: left
+// alone, the compiler moves loads behind the products and under the guards of ragged ends, two to four round trips a wave
+// instead of one), the next tile's first PRE k-pairs are requested before this one's sums meet, a wave holds one tile's
+// numbers only, so that two workgroups fit a CU, and the instructions behind the last load are few.
+// RB: groups of four rows (M <= 4 RB): a tile's rows are one number quadruple of 16 RB lanes, and the 64 lanes of one wave
+// each add up NWV RB / 4 waves' sums.
+// GLU: a tile is 8 gate columns and their 8 up columns (halves of two weight tiles, whole 128-byte lines of both).
+// NRM: the first tile's k-pairs are in flight while the norm runs; the norm runs once for all tiles.
+template <int NWV, int U, int PRE, int EPI, bool HF, int NRM, int RB>
+__device__ __forceinline__ void gemv_tiles_body(int bid, int nwg, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                const bf16_t* __restrict__ bias, bf16_t* __restrict__ out, int M, int N,
+                                                int K, int F, int S, const bf16_t* __restrict__ add, const NormIn16& na) {
+  static_assert(NRM == 0 || (NWV == GEMV_NW && RB == 1 && EPI != EPI_PART), "norm prologue: 16 waves, up to 4 rows");
   constexpr bool LN_N = NRM >= 64;
   constexpr int NCH_N = (NRM % 64) / 8, SMAX_N = LN_N ? 1 : NRM % 8;
+  constexpr int RL = 16 * RB, WG = 4 / RB;                  // lanes of a wave's rows, waves that a wave adds up side by side
+  __shared__ v4f red[2][NWV][RL];
   __shared__ __attribute__((aligned(16))) bf16_t xs[NRM > 0 ? NRM16_ROWS * NCH_N * 2048 : 8];
   __shared__ float nred[16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15;
+  const int KP = K / 64, tiles = N / 16 * (EPI == EPI_PART ? S : 1);
+  // tile tt: this lane's fragments, the wave's first k-pair and the end of the tile's k-pairs
+  const bf16_t* wp;
+  int kp, kend;
+  auto enter = [&](int tt) {
+    if constexpr (EPI == EPI_GLU) {
+      const int row = 8 * tt + (r < 8 ? r : F + r - 8);
+      wp = W + ((size_t)(row >> 4) * (2 * KP) * 64 + (lane & 48) + (row & 15)) * 8;
+    } else {
+      wp = W + ((size_t)(EPI == EPI_PART ? tt / S : tt) * (2 * KP) * 64 + lane) * 8;
+    }
+    const int ks = EPI == EPI_PART ? tt % S : 0;
+    kp = (EPI == EPI_PART ? KP * ks / S : 0) + wave;
+    kend = EPI == EPI_PART ? KP * (ks + 1) / S : KP;
+  };
+  v8s p0[PRE > 0 ? PRE : 1][2];
+  auto ahead = [&]() {
+#pragma unroll
+    for (int u = 0; u < PRE; ++u) {                          // clamped: loads never branch
+      const int k = min(kp + NWV * u, kend - 1);
+      p0[u][0] = ld_nt(wp + (size_t)k * 1024);               // tiles 2 kp, 2 kp + 1: 2 KiB contiguous
+      p0[u][1] = ld_nt(wp + (size_t)k * 1024 + 512);
+    }
+  };
+  const bf16_t* ar = (NRM > 0 ? xs : A) + (size_t)min(r, M - 1) * K + 8 * (lane >> 4);
+  int t = bid;
+  enter(t);
+  if constexpr (NRM > 0) {
+    NormRegs16<(NRM > 0 ? NCH_N : 1), (NRM > 0 ? SMAX_N : 1), LN_N> nr;
+    norm16_load(na, bid == 0, K, M, nr);
+    ahead();
+    if constexpr (LN_N) ln16_prologue<NCH_N, HF>(na, bid == 0, K, M, xs, nred, nr);
+    else norm16_prologue<NCH_N, SMAX_N, HF>(na, bid == 0, K, M, xs, nred, nr);
+  } else ahead();
+  for (int buf = 0; t < tiles; buf ^= 1) {
+    const int ks = EPI == EPI_PART ? t % S : 0, tile = EPI == EPI_PART ? t / S : t;
+    const int row0 = RB == 1 ? 0 : 4 * (lane >> 4), c = EPI == EPI_GLU ? 8 * tile + (r & 7) : 16 * tile + r;
+    v4f acc = {0.f, 0.f, 0.f, 0.f};
+    // what the writing wave adds to its sums is requested with its first weights
+    float bv = 0.f, addv[4] = {0.f, 0.f, 0.f, 0.f};
+    if (wave == 0) {
+      if (bias != nullptr && (EPI != EPI_PART || ks == 0)) bv = e2f<HF>(bias[EPI == EPI_GLU && r >= 8 ? F + c : c]);
+      if constexpr (EPI == EPI_OUT) {
+        if (add != nullptr) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) addv[q] = e2f<HF>(add[(size_t)min(row0 + q, M - 1) * N + c]);
+        }
+      }
+    }
+    if constexpr (PRE > 0) {
+      v8s a[PRE][2];
+#pragma unroll
+      for (int u = 0; u < PRE; ++u) {
+        const int k = min(kp + NWV * u, kend - 1);
+        a[u][0] = *reinterpret_cast<const v8s*>(ar + k * 64);
+        a[u][1] = *reinterpret_cast<const v8s*>(ar + k * 64 + 32);
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int u = 0; u < PRE; ++u)
+        if (kp + NWV * u < kend) {                           // wave-uniform (scalar) guard
+          acc = mfma_16<HF>(a[u][0], p0[u][0], acc);
+          acc = mfma_16<HF>(a[u][1], p0[u][1], acc);
+        }
+    }
+    for (kp += NWV * PRE; kp < kend; kp += NWV * U) {
+      v8s a[U][2], b[U][2];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = U == 1 ? kp : min(kp + u * NWV, kend - 1);
+        b[u][0] = ld_nt(wp + (size_t)k * 1024);
+        b[u][1] = ld_nt(wp + (size_t)k * 1024 + 512);
+        a[u][0] = *reinterpret_cast<const v8s*>(ar + k * 64);
+        a[u][1] = *reinterpret_cast<const v8s*>(ar + k * 64 + 32);
+      }
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (U == 1 || kp + u * NWV < kend) {
+          acc = mfma_16<HF>(a[u][0], b[u][0], acc);
+          acc = mfma_16<HF>(a[u][1], b[u][1], acc);
+        }
+    }
+    t += nwg;
+    if (t < tiles) {
+      enter(t);
+      ahead();
+    }
+    if (RB == 4 || lane < RL) red[buf][wave][lane & (RL - 1)] = acc;
+    // two buffers: the wave that reads this one has passed the next barrier before anybody writes it again
+    __syncthreads();
+    if (wave == 0) {
+      v4f s = red[buf][lane / RL][lane & (RL - 1)];
+#pragma unroll
+      for (int w = 1; w < NWV / WG; ++w) s += red[buf][WG * w + lane / RL][lane & (RL - 1)];
+      if constexpr (RB == 1) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = xor_sum(s[q], 16);
+      }
+      if constexpr (RB <= 2) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) s[q] = xor_sum(s[q], 32);
+      }
+      if constexpr (EPI == EPI_GLU) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const float g = e2f<HF>(f2e<HF>(s[q] + bv)), u = lane_xor(g, 8);
+          if (r < 8 && (RB == 4 || lane < RL) && row0 + q < M)
+            out[(size_t)(row0 + q) * F + c] = f2e<HF>(g / (1.f + __expf(-g)) * u);
+        }
+      } else if (RB == 4 || lane < RL) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int row = row0 + q;
+          float v = s[q] + bv;
+          if constexpr (EPI == EPI_PART) {
+            if (row < M) reinterpret_cast<float*>(out)[((size_t)ks * M + row) * N + c] = v;
+          } else {
+            if constexpr (EPI == EPI_GELU_TANH || EPI == EPI_GELU || EPI == EPI_GELU_ANY) {
+              const float x = e2f<HF>(f2e<HF>(v)), k0 = 0.7978845608028654f, k1 = 0.044715f;
+              if (EPI == EPI_GELU_TANH || (EPI == EPI_GELU_ANY && F == 1))
+                v = 0.5f * x * (1.f + tanhf(k0 * (x + k1 * x * x * x)));
+              else v = 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
+            } else {
+              // an addend (parallel-residual block): rnd(rnd(y) + add), the unfused add
+              if (add != nullptr) v = e2f<HF>(f2e<HF>(v)) + addv[q];
+            }
+            if (row < M) out[(size_t)row * N + c] = f2e<HF>(v);
+          }
+        }
+      }
+    }
+  }
+}
+
+// One workgroup (bid) of the GEMV of more rows: NTW tiles, MB row blocks of 16.
+template <int MB, int NTW, int U, int EPI, bool HF>
+__device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                               const bf16_t* __restrict__ bias, bf16_t* __restrict__ out, int M, int N,
+                                               int K, int F, int S, const bf16_t* __restrict__ add) {
+  constexpr int NWV = GEMV_NW;
+  static_assert(EPI != EPI_GLU || NTW % 2 == 0, "GLU: gate/up tile pairs");
+  static_assert(MB * NTW <= 8 && MB * (EPI == EPI_GLU ? NTW / 2 : NTW) <= NWV, "LDS reduction / output waves");
+  __shared__ v4f red[NWV][MB * NTW][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, kq = 8 * (lane >> 4);
   // output column of tile j for this lane (EPI_GLU: gate tiles then the matching up tiles)
@@ -290,28 +442,12 @@ __device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict
   for (int j = 0; j < NTW; ++j) wrow[j] = W + ((size_t)(min(col_of(j), N - 1) >> 4) * (2 * KP) * 64 + lane) * 8;
   const bf16_t* arow[MB];
 #pragma unroll
-  for (int mb = 0; mb < MB; ++mb) arow[mb] = (NRM > 0 ? xs : A) + (size_t)min(16 * mb + r, M - 1) * K + kq;
-  // NRM: the prologue's loads, then the first k-pair's weights, are in flight before the norm
-  // runs (a wave's loads retire in issue order: weights first would make the norm wait for them)
-  NormRegs16<(NRM > 0 ? NCH_N : 1), (NRM > 0 ? SMAX_N : 1), LN_N> nr;
-  v8s b0[NTW][2];
-  if constexpr (NRM > 0) {
-    norm16_load(na, bid == 0, K, M, nr);
-    const int k = min(kbeg + wave, kend - 1) * 64;
-#pragma unroll
-    for (int j = 0; j < NTW; ++j) {
-      b0[j][0] = ld_nt(wrow[j] + (size_t)k * 16);
-      b0[j][1] = ld_nt(wrow[j] + (size_t)k * 16 + 512);
-    }
-    if constexpr (LN_N) ln16_prologue<NCH_N, HF>(na, bid == 0, K, M, xs, nred, nr);
-    else norm16_prologue<NCH_N, SMAX_N, HF>(na, bid == 0, K, M, xs, nred, nr);
-  }
+  for (int mb = 0; mb < MB; ++mb) arow[mb] = A + (size_t)min(16 * mb + r, M - 1) * K + kq;
   v4f acc[MB][NTW];
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
     for (int j = 0; j < NTW; ++j) acc[mb][j] = v4f{0.f, 0.f, 0.f, 0.f};
-  bool first = NRM > 0;
   for (int kp = kbeg + wave; kp < kend; kp += NWV * U) {
     v8s a[U][MB][2], b[U][NTW][2];
 #pragma unroll
@@ -319,13 +455,8 @@ __device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict
       const int k = min(kp + u * NWV, kend - 1) * 64;        // clamped: loads never branch
 #pragma unroll
       for (int j = 0; j < NTW; ++j) {                        // tiles 2 kp, 2 kp + 1: 2 KiB contiguous
-        if (NRM > 0 && u == 0 && first) {
-          b[u][j][0] = b0[j][0];
-          b[u][j][1] = b0[j][1];
-        } else {
-          b[u][j][0] = ld_nt(wrow[j] + (size_t)k * 16);
-          b[u][j][1] = ld_nt(wrow[j] + (size_t)k * 16 + 512);
-        }
+        b[u][j][0] = ld_nt(wrow[j] + (size_t)k * 16);
+        b[u][j][1] = ld_nt(wrow[j] + (size_t)k * 16 + 512);
       }
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb) {
@@ -333,7 +464,6 @@ __device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict
         a[u][mb][1] = *reinterpret_cast<const v8s*>(arow[mb] + k + 32);
       }
     }
-    first = false;
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       if (kp + u * NWV < kend) {                             // wave-uniform (scalar) guard
@@ -366,7 +496,7 @@ __device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict
     if constexpr (EPI == EPI_GLU) {
       const int c1 = col_of(tw + NTW / 2);
       const v4f g4 = total(tw), u4 = total(tw + NTW / 2);
-      const float bg = bias != nullptr ? e2f<HF>(bias[c0]) : 0.f, bu = bias != nullptr ? e2f<HF>(bias[c1]) : 0.f;
+      const float bg = bias != nullptr ? e2f<HF>(bias[c0]) : 0.f, bu = bias != nullptr ? e2f<HF>(bias[min(c1, N - 1)]) : 0.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const int row = 16 * mb + 4 * (lane >> 4) + q;
@@ -389,9 +519,9 @@ __device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict
       for (int q = 0; q < 4; ++q) {
         const int row = 16 * mb + 4 * (lane >> 4) + q;
         float v = s4[q] + bv;
-        if constexpr (EPI == EPI_GELU_TANH || EPI == EPI_GELU || EPI == EPI_GELU_ANY) {
+        if constexpr (EPI == EPI_GELU_TANH || EPI == EPI_GELU) {
           const float a = e2f<HF>(f2e<HF>(v)), k0 = 0.7978845608028654f, k1 = 0.044715f;
-          if (EPI == EPI_GELU_TANH || (EPI == EPI_GELU_ANY && F == 1))
+          if (EPI == EPI_GELU_TANH)
             v = 0.5f * a * (1.f + tanhf(k0 * (a + k1 * a * a * a)));
           else v = 0.5f * a * (1.f + erff(a * 0.7071067811865476f));
         } else {

@@ -9,7 +9,8 @@
 // ((nt * K/32) + kt) * 512 elements, lane l's 8 elements = W[16 nt + (l & 15)][32 kt + 8 (l >> 4) ..]
 // — the B fragment of v_mfma_f32_16x16x32_bf16.  A wave walks K in pairs of k-steps, i.e. 2 KiB
 // of contiguous weights per tile per pair (the [N, K] layout gave each load instruction 16 rows x
-// 64 B: 36 % more bytes fetched and 2.3 TB/s on Llama-3.2-1B's gate_up).  A workgroup = 16 waves
+// 64 B: 36 % more bytes fetched and 2.3 TB/s on Llama-3.2-1B's gate_up).  Few rows run gemv_tiles_body (gemv_bf16.h):
+// one tile of a workgroup's at a time.  More rows, where a tile's reads of the rows weigh: a workgroup = 16 waves
 // on NTW 16-column tiles; wave w takes k-pairs w, w + 16, ..., keeping U pairs of weight loads in
 // flight (nontemporal: each weight byte is read once per step).  The 16 partial tiles are
 // reduced through LDS.  Rows >= M load a clamped row and are never stored.
@@ -28,23 +29,59 @@
 #include "gemv_bf16.h"
 
 namespace {
-template <int MB, int NTW, int U, int EPI, bool HF, int NRM = 0>
+template <int MB, int NTW, int U, int EPI, bool HF>
 __global__ void __launch_bounds__(GEMV_NW * 64) gemv_bf16_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                             const bf16_t* __restrict__ bias, bf16_t* __restrict__ out,
                                                             int M, int N, int K, int F, int S,
-                                                            const bf16_t* __restrict__ add, NormIn16 na) {
-  gemv_bf16_body<GEMV_NW, MB, NTW, U, EPI, HF, NRM>((int)blockIdx.x, A, W, bias, out, M, N, K, F, S, add, na);
+                                                            const bf16_t* __restrict__ add) {
+  gemv_bf16_body<MB, NTW, U, EPI, HF>((int)blockIdx.x, A, W, bias, out, M, N, K, F, S, add);
 }
 
-template <int MB, int NTW, int U, int EPI, bool HF, int NRM = 0>
+template <int MB, int NTW, int U, int EPI, bool HF>
 int launch_mb(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int F, int tiles,
-              hipStream_t st, int S, const void* add = nullptr, const NormIn16& na = NormIn16{}) {
-  const int groups = EPI == EPI_GLU ? tiles / (NTW / 2) : (tiles + NTW - 1) / NTW;
-  hipLaunchKernelGGL((gemv_bf16_kernel<MB, NTW, U, EPI, HF, NRM>), dim3(groups * S), dim3(GEMV_NW * 64), 0, st,
+              hipStream_t st, int S, const void* add = nullptr) {
+  constexpr int per = EPI == EPI_GLU ? NTW / 2 : NTW;       // output tiles a workgroup
+  const int groups = (tiles + per - 1) / per;
+  hipLaunchKernelGGL((gemv_bf16_kernel<MB, NTW, U, EPI, HF>), dim3(groups * S), dim3(GEMV_NW * 64), 0, st,
                      (const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)bias, (bf16_t*)out, M, N, K, F, S,
-                     (const bf16_t*)add, na);
+                     (const bf16_t*)add);
   return (int)hipGetLastError();
 }
+
+template <int PRE, int EPI, bool HF, int NRM, int RB>
+__global__ void __launch_bounds__(GEMV_NW * 64) gemv_tiles_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+                                                                 const bf16_t* __restrict__ bias, bf16_t* __restrict__ out,
+                                                                 int M, int N, int K, int F, int S,
+                                                                 const bf16_t* __restrict__ add, NormIn16 na) {
+  gemv_tiles_body<GEMV_NW, 1, PRE, EPI, HF, NRM, RB>((int)blockIdx.x, (int)gridDim.x, A, W, bias, out, M, N, K, F, S, add, na);
+}
+
+// Workgroups of the tiles form.  Without a norm up to 1024, two to a CU and two rounds of them: 128256 x 2048 takes 82 us on
+// 256, 77 on 512, 75.8 on 1024, 75.6 on 2048.  With a norm one to a CU (the norm's loads and sums are each workgroup's own):
+// 22016 x 4096 29.4 us on 256, 29.6 on 512, 30.9 on 1024; 6144 x 4096 (384 tiles) 10.1 on 256, 11.5 on 384.
+template <int EPI, bool HF, int NRM, int RB>
+int launch_tiles(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, hipStream_t st, int S = 1,
+                 const void* add = nullptr, const NormIn16& na = NormIn16{}) {
+  const int tiles = N / 16 * S, cap = NRM > 0 ? 256 : 1024;
+  hipLaunchKernelGGL((gemv_tiles_kernel<(NRM > 0 ? 2 : 1), EPI, HF, NRM, RB>), dim3(EPI == EPI_PART || tiles < cap ? tiles : cap),
+                     dim3(GEMV_NW * 64), 0, st, (const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)bias, (bf16_t*)out, M, N, K,
+                     EPI == EPI_GLU ? N / 2 : 0, S, (const bf16_t*)add, na);
+  return (int)hipGetLastError();
+}
+
+template <int EPI, bool HF>
+int launch_tiles_rows(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, hipStream_t st, int S = 1,
+                      const void* add = nullptr) {
+  if (M <= 4) return launch_tiles<EPI, HF, 0, 1>(A, W, bias, out, M, N, K, st, S, add);
+  if (M <= 8) return launch_tiles<EPI, HF, 0, 2>(A, W, bias, out, M, N, K, st, S, add);
+  return launch_tiles<EPI, HF, 0, 4>(A, W, bias, out, M, N, K, st, S, add);
+}
+
+// Whether the tiles form takes M rows: up to 4 always, 5 to 16 where its tiles' reads of the rows (each tile reads all of
+// them) stay small beside the weights.  us, tiles form / several tiles a workgroup: 1 row 1024 x 1024 2.7 / 3.3, 4096 x 2048 (4 rows)
+// 4.7 / 5.4, 32000 x 1024 11.8 / 12.7; 12 rows 4096 x 2048 5.3 / 6.0, 16 rows 8224 x 2048 10.5 / 12.0, 32000 x 2048 27 / 23.5;
+// SwiGLU 16384 x 2048 1 row 11.7 / 13.0, 8 rows 13.8 / 13.3.
+bool tiles_form(int M, int N, int epi) { return M <= 4 || (M <= 16 && epi != EPI_GLU && N < 16384); }
 
 // NTW / U chosen for one row block; more row blocks keep U = 2 (registers) and at most 8 / MB
 // tiles (the LDS reduction holds MB x NTW tiles of 16 waves)
@@ -67,7 +104,16 @@ int launch(const void* A, const void* W, const void* bias, void* out, int M, int
 template <bool HF>
 int gemv_run(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi, hipStream_t st,
              const void* add) {
-  if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || K <= 0) return -2;
+  if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || N <= 0 || K <= 0) return -2;
+  if (tiles_form(M, N, epi)) {
+    switch (epi) {
+      case EPI_OUT: return launch_tiles_rows<EPI_OUT, HF>(A, W, bias, out, M, N, K, st, 1, add);
+      case EPI_GLU: return N % 32 != 0 ? -2 : launch_tiles<EPI_GLU, HF, 0, 1>(A, W, bias, out, M, N, K, st);
+      case EPI_GELU_TANH: return launch_tiles_rows<EPI_GELU_TANH, HF>(A, W, bias, out, M, N, K, st);
+      case EPI_GELU: return launch_tiles_rows<EPI_GELU, HF>(A, W, bias, out, M, N, K, st);
+      default: return -2;
+    }
+  }
   const int KP = K / 64;
   const int U = KP >= 64 ? 4 : 2;                            // k-pairs in flight per wave
   if (epi == EPI_GLU) {
@@ -98,35 +144,19 @@ int gemv_run(const void* A, const void* W, const void* bias, void* out, int M, i
 }
 
 // The 16-bit GEMV over RMSNorm(sum(parts) + residual) (norm16_prologue): M <= 4, K 2048 / 4096,
-// S <= 4 slices; epi 0 (EPI_OUT) or 1 (EPI_GLU).  The geometry of gemv_run for one row block.
+// S <= 4 slices; epi 0 (EPI_OUT) or 1 (EPI_GLU).  Not taken: 3 or 4 slices of K = 4096 before 16384 outputs or more (no
+// model's projections leave that many slices; the norm is a launch of its own there).
 template <bool HF, int NRM>
 int gemv_norm_geo(const NormIn16& na, const void* W, const void* bias, void* out, int M, int N, int K, int epi,
                   hipStream_t st) {
-  const int KP = K / 64, U = KP >= 64 ? 4 : 2;
-  if (epi == EPI_GLU) {
-    const int F = N / 2, ft = F / 16;
-    if (ft >= 512) {
-      if constexpr (NRM == 20) return -2;                // 4 tiles + 3-4 held slices of K = 4096: spills
-      else return launch_mb<1, 4, 2, EPI_GLU, HF, NRM>(nullptr, W, bias, out, M, N, K, F, ft, st, 1, nullptr, na);
-    }
-    return U == 4 ? launch_mb<1, 2, 4, EPI_GLU, HF, NRM>(nullptr, W, bias, out, M, N, K, F, ft, st, 1, nullptr, na)
-                  : launch_mb<1, 2, 2, EPI_GLU, HF, NRM>(nullptr, W, bias, out, M, N, K, F, ft, st, 1, nullptr, na);
+  if (NRM == 20 && N / 16 >= 1024) return -2;
+  if constexpr (NRM < 64) {
+    if (epi == EPI_GLU) return launch_tiles<EPI_GLU, HF, NRM, 1>(nullptr, W, bias, out, M, N, K, st, 1, nullptr, na);
+  } else {
+    if (epi == EPI_GELU_TANH) return launch_tiles<EPI_GELU_TANH, HF, NRM, 1>(nullptr, W, bias, out, M, N, K, st, 1, nullptr, na);
+    if (epi == EPI_GELU) return launch_tiles<EPI_GELU, HF, NRM, 1>(nullptr, W, bias, out, M, N, K, st, 1, nullptr, na);
   }
-  const int nt = N / 16;
-#define NPICK(EP)                                                                                              \
-  if (nt >= 1024) {                                                                                            \
-    if constexpr (NRM == 20) return -2;                                                                        \
-    else return launch_mb<1, 4, 2, EP, HF, NRM>(nullptr, W, bias, out, M, N, K, 0, nt, st, 1, nullptr, na);     \
-  }                                                                                                            \
-  if (nt >= 512)                                                                                               \
-    return U == 4 ? launch_mb<1, 2, 4, EP, HF, NRM>(nullptr, W, bias, out, M, N, K, 0, nt, st, 1, nullptr, na)  \
-                  : launch_mb<1, 2, 2, EP, HF, NRM>(nullptr, W, bias, out, M, N, K, 0, nt, st, 1, nullptr, na); \
-  return U == 4 ? launch_mb<1, 1, 4, EP, HF, NRM>(nullptr, W, bias, out, M, N, K, 0, nt, st, 1, nullptr, na)    \
-                : launch_mb<1, 1, 2, EP, HF, NRM>(nullptr, W, bias, out, M, N, K, 0, nt, st, 1, nullptr, na);
-  if (epi == EPI_GELU_TANH) { NPICK(EPI_GELU_TANH) }
-  if (epi == EPI_GELU) { NPICK(EPI_GELU) }
-  NPICK(EPI_OUT)
-#undef NPICK
+  return launch_tiles<EPI_OUT, HF, NRM, 1>(nullptr, W, bias, out, M, N, K, st, 1, nullptr, na);
 }
 
 // LayerNorm prologue over 16-bit rows x (+ residual): K <= 4096 (K % 64 == 0), epi 0 / 2 / 3.
@@ -158,7 +188,8 @@ int gemv_norm_run(const NormIn16& na, const void* W, const void* bias, void* out
 template <bool HF>
 int gemv_splitk_run(const void* A, const void* W, const void* bias, float* part, int M, int N, int K, int S,
                     hipStream_t st) {
-  if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || S < 1 || S > K / 64) return -2;
+  if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || N <= 0 || S < 1 || S > K / 64) return -2;
+  if (M <= 16) return launch_tiles_rows<EPI_PART, HF>(A, W, bias, part, M, N, K, st, S);
   const int nt = N / 16, kps = K / 64 / S;
   return kps >= 64 ? launch<1, 4, EPI_PART, HF>(A, W, bias, part, M, N, K, 0, nt, st, S)
                    : launch<1, 2, EPI_PART, HF>(A, W, bias, part, M, N, K, 0, nt, st, S);
