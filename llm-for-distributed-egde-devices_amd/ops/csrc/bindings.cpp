@@ -776,6 +776,12 @@ at::Tensor w8a8_gemm_splitk(const at::Tensor& a, const at::Tensor& sa, const at:
   if (M > 128) S = edge_w8a8_rows256_splits((int)K);     // 129-256 rows: fixed per K (gemm_i8.hip rows256)
   TORCH_CHECK(M <= 128 || S > 1, "no 129-256-row split-K kernel for this K");
   if (S <= 0 && M > 64) S = 4;                           // 65-128 rows: 4 slices (gemm_i8.hip rows128)
+  if (S <= 0 && M <= 16 && mpad > 0 && N % 16 == 0) {
+    // one tile a workgroup (gemv_i8_rows.hip): two workgroups a CU, each wave a k-tile or more; us at S = 1 / 2 / 4: 4096 x 4096 5.3 / 4.7 /
+    // 7.4, 4096 x 11008 10.0 / 8.8 / 9.9, 2048 x 2048 3.4 / 3.4 / 4.1, 2048 x 8192 7.4 / 5.3 / 4.7
+    const int64_t tiles = N / 16;
+    S = std::max<int64_t>(1, std::min<int64_t>({4, (512 + tiles / 2) / tiles, KT / 16}));
+  }
   if (S <= 0) {
     const int64_t ntw = M <= 16 ? 2 : 4;                 // tiles per workgroup (gemm_i8.hip launcher)
     const int64_t groups = ((N + 15) / 16 + ntw - 1) / ntw;

@@ -978,6 +978,8 @@ int launch_out(int ntw, int un, int kw, const void* A, const float* sa, const vo
 }
 }  // namespace
 
+extern "C" int edge_w8a8_rows_splitk(const void* A, const float* sa, const void* Wp, const float* sw, const void* bias, float* part,
+                                     int M, int N, int K, int Mpad, int S, hipStream_t st);   // gemv_i8_rows.hip
 // Split-K GEMV (M <= 64, K % 64 == 0): S workgroups per 4-tile group, each reducing KT/S k-tiles
 // into fp32 partial slices part[S][M][N].  Cuts each workgroup's activation reads S-fold — at
 // decode shapes every CU re-reads the whole activation matrix from L2, and those bytes share the
@@ -996,6 +998,10 @@ extern "C" int edge_w8a8_gemm_splitk(const void* A, const float* sa, const void*
   if (M > 64) {
     const int r = launch_ring_rows128<EPI_PART>(A, sa, Wp, sw, bias, part, nullptr, M, N, K, Mpad, a_mode == A_GROUP, st, S);
     return r == -1 ? -2 : r;
+  }
+  if (a_mode == A_GROUP && M <= 16) {                       // one tile a workgroup (N % 16 == 0)
+    const int r = edge_w8a8_rows_splitk(A, sa, Wp, sw, bias, part, M, N, K, Mpad, S, st);
+    if (r != -2) return r;
   }
   // 2 tiles per workgroup for one row block, 4 for more (the binding sizes S for ~256 workgroups;
   // measured on Llama-2-7B o/down: S = 2 best at 16 rows, S = 4 at 32)
