@@ -149,12 +149,11 @@ __device__ __forceinline__ void ln16_prologue(const NormIn16& na, bool wg0, int 
       }
     }
     ss = wave_sum(ss);
+    if ((t & 63) == 0) nred[16 + 4 * row + w] = ss;         // (each reduction has words of its own: one barrier each)
   }
-  __syncthreads();                                        // every group has read its sums
-  if (act && (t & 63) == 0) nred[4 * row + w] = ss;
   __syncthreads();
   if (act) {
-    const float* gr = nred + 4 * row;
+    const float* gr = nred + 16 + 4 * row;
     const float rstd = rsqrtf(((((0.f + gr[0]) + gr[1]) + gr[2]) + gr[3]) / (float)H + na.eps);
 #pragma unroll
     for (int c = 0; c < NCH; ++c) {
@@ -276,7 +275,7 @@ __device__ __forceinline__ void gemv_tiles_body(int bid, int nwg, const bf16_t* 
   constexpr int RL = 16 * RB, WG = 4 / RB;                  // lanes of a wave's rows, waves that a wave adds up side by side
   __shared__ v4f red[2][NWV][RL];
   __shared__ __attribute__((aligned(16))) bf16_t xs[NRM > 0 ? NRM16_ROWS * NCH_N * 2048 : 8];
-  __shared__ float nred[16];
+  __shared__ float nred[32];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15;
   const int KP = K / 64, tiles = N / 16 * (EPI == EPI_PART ? S : 1);
   // tile tt: this lane's fragments, the wave's first k-pair and the end of the tile's k-pairs

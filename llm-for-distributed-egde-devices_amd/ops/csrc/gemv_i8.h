@@ -276,7 +276,7 @@ struct NormIn {
   int act = 0;                    // LLM.int8, activation chosen per launch: 1 gelu tanh, 2 gelu erf
 };
 constexpr int NRM_ROWS = 4;
-constexpr int L8_COUNT = 24;      // where l8_prologue leaves the outlier count (after 4 wave totals for each of 6 chunks)
+constexpr int L8_COUNT = 32;      // where l8_prologue leaves the outlier count (after every wave's total of every chunk)
 constexpr int L8_CMAX = 256;      // LLM.int8 outlier columns per row held in LDS (llmint8.hip's cap)
 
 // The prologue's global loads (slices, residual, gamma) are issued by norm_load BEFORE the
@@ -377,7 +377,6 @@ __device__ __forceinline__ void norm_prologue(const NormIn& na, bool wg0, int H,
     __syncthreads();
     const float* gr = nred + 4 * g;
     const float rstd = rsqrtf((((0.f + gr[0]) + gr[1]) + gr[2] + gr[3]) / (float)H + na.eps);
-    __syncthreads();
     if (act) {
 #pragma unroll
       for (int c = 0; c < NCH; ++c) {
@@ -394,12 +393,12 @@ __device__ __forceinline__ void norm_prologue(const NormIn& na, bool wg0, int H,
 #pragma unroll
         for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[c][j]));
       amax = wave_max(amax);
-      if ((t & 63) == 0) nred[4 * g + w] = amax;
+      if ((t & 63) == 0) nred[16 + 4 * g + w] = amax;     // (each reduction has words of its own: one barrier each)
     }
     __syncthreads();
     float gm = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) gm = fmaxf(gm, gr[i]);
+    for (int i = 0; i < 4; ++i) gm = fmaxf(gm, gr[16 + i]);
     gm = fmaxf(gm, 1e-8f);
     const float inv = 127.f / gm;
     if (act && t == 0) nsa[row] = gm / 127.f;
@@ -493,12 +492,10 @@ __device__ __forceinline__ void ln_prologue(const NormIn& na, bool wg0, int H, i
       }
     }
     ss = wave_sum(ss);
+    if ((t & 63) == 0) nred[16 + 4 * row + w] = ss;         // (each reduction has words of its own: one barrier each)
   }
   __syncthreads();
-  if (act && (t & 63) == 0) nred[4 * row + w] = ss;
-  __syncthreads();
-  const float rstd = rsqrtf(((((0.f + gr[0]) + gr[1]) + gr[2]) + gr[3]) / (float)H + na.eps);
-  __syncthreads();
+  const float rstd = rsqrtf(((((0.f + gr[16]) + gr[17]) + gr[18]) + gr[19]) / (float)H + na.eps);
   float amax = 0.f;
   if (act) {
 #pragma unroll
@@ -517,12 +514,12 @@ __device__ __forceinline__ void ln_prologue(const NormIn& na, bool wg0, int H, i
 #pragma unroll
       for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[c][j]));
     amax = wave_max(amax);
-    if ((t & 63) == 0) nred[4 * row + w] = amax;
+    if ((t & 63) == 0) nred[32 + 4 * row + w] = amax;
   }
   __syncthreads();
   float gm = -INFINITY;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) gm = fmaxf(gm, gr[i]);
+  for (int i = 0; i < 4; ++i) gm = fmaxf(gm, gr[32 + i]);
   gm = fmaxf(gm, 1e-8f);
   const float inv = 127.f / gm;
   if (act && t == 0) nsa[row] = gm / 127.f;
@@ -544,8 +541,7 @@ __device__ __forceinline__ void ln_prologue(const NormIn& na, bool wg0, int H, i
 }
 
 // LLM.int8 prologue (NRM >= 128, one row): llmint8.hip's decode preparation inside the GEMV, so a
-// batch-1 LLM.int8 projection is one launch instead of three (prep, GEMV, outlier add).  Threads
-// 0-255 hold the row in norm_prologue's layout (column (c 256 + t) 8 + j); columns with |x| > thr
+// batch-1 LLM.int8 projection is one launch instead of three (prep, GEMV, outlier add).  Columns with |x| > thr
 // are ranked in column order by a block prefix sum per chunk, the first L8_CMAX go to LDS (index,
 // value); the per-token absmax over the other columns, then int8 x with the taken columns zeroed.
 // The epilogue adds sum_j x[c_j] W^T[c_j][n] SCB[n] / 127 to the rounded output, in llmint8.hip's
@@ -554,20 +550,29 @@ __device__ __forceinline__ void ln_prologue(const NormIn& na, bool wg0, int H, i
 // (norm_kernel's HAS_RES path, rounded to bf16 as its output), so an LLM.int8 layer's norm is no
 // launch of its own either; workgroup 0 writes the new residual row and, when y_out is set, the
 // normalised row (for a second consumer).
-template <int NCH, int SRC>
+// Who holds the row: behind a norm threads 0-255 in norm_prologue's layout, column (c 256 + t) 8 + j (its sums' order); a row as
+// it is (ranks and maxima have no order) all threads of the workgroup, 8 columns a chunk.  Every wave of the workgroup waits for
+// this chain, so the counts and the maximum meet at one barrier: the maximum leaves out every outlier, and only a row of more than
+// L8_CMAX of them takes it again over those past the cap.  us in a graph, one row, 256 threads and three barriers /
+// now: 2560 x 10240 beside 2560 x 2560 10.5 / 8.1, 10240 x 2560 beside attention 9.5 / 8.3, 7680 x 2560 behind LayerNorm 8.3 / 7.6.
+template <int NCH, int SRC, int NW>
+constexpr int l8_chunks() { return SRC ? NCH : (NCH * 256 + NW * 64 - 1) / (NW * 64); }
+
+template <int NC, int SRC>
 struct L8Regs {
-  uint4 xv[NCH];
-  uint4 rv[SRC ? NCH : 1], gv[SRC ? NCH : 1], bv[SRC == 2 ? NCH : 1];
-  uint4 x2v[SRC == 2 ? NCH : 1], g2v[SRC == 2 ? NCH : 1], b2v[SRC == 2 ? NCH : 1];
+  uint4 xv[NC];
+  uint4 rv[SRC ? NC : 1], gv[SRC ? NC : 1], bv[SRC == 2 ? NC : 1];
+  uint4 x2v[SRC == 2 ? NC : 1], g2v[SRC == 2 ? NC : 1], b2v[SRC == 2 ? NC : 1];
 };
 
-template <int NCH, int SRC>
-__device__ __forceinline__ void l8_load(const NormIn& na, bool wg0, int H, L8Regs<NCH, SRC>& r) {
+template <int NC, int SRC, int NW>
+__device__ __forceinline__ void l8_load(const NormIn& na, bool wg0, int H, L8Regs<NC, SRC>& r) {
+  constexpr int NTH = SRC ? 256 : NW * 64;
   const int t = threadIdx.x;
-  if (t < 256) {
+  if (SRC == 0 || t < 256) {
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int e = min((c * 256 + t) * 8, H - 8);
+    for (int c = 0; c < NC; ++c) {
+      const int e = min((c * NTH + t) * 8, H - 8);
       r.xv[c] = *reinterpret_cast<const uint4*>(na.x + e);
       if constexpr (SRC > 0) {
         r.rv[c] = na.res != nullptr ? *reinterpret_cast<const uint4*>(na.res + e) : uint4{0u, 0u, 0u, 0u};
@@ -585,21 +590,23 @@ __device__ __forceinline__ void l8_load(const NormIn& na, bool wg0, int H, L8Reg
   asm volatile("" ::: "memory");                          // these loads issue before the weights
 }
 
-template <int NCH, int SRC>
+template <int NC, int SRC, int NW>
 __device__ __forceinline__ void l8_prologue(const NormIn& na, bool wg0, int H, int8_t* aq, float* nsa, float* nred, int* cols,
-                                            float* xo, int* scr, const L8Regs<NCH, SRC>& r, bf16_t* y_out) {
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
-  const bool act = t < 256;
-  float v[NCH][8];
+                                            float* xo, int* scr, const L8Regs<NC, SRC>& r, bf16_t* y_out) {
+  constexpr int NTH = SRC ? 256 : NW * 64, WV = NTH / 64;   // threads and waves that hold the row
+  static_assert(NC * WV <= L8_COUNT, "wave totals");
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
+  const bool act = SRC == 0 || w < WV;
+  float v[NC][8];
   if (act) {
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) unpack8(r.xv[c], v[c]);
+    for (int c = 0; c < NC; ++c) unpack8(r.xv[c], v[c]);
   }
   if constexpr (SRC > 0) {
     float sm = 0.f;
     if (act) {
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const int e = (c * 256 + t) * 8;
         if (e < H) {
           float rr[8];
@@ -624,7 +631,7 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, bool wg0, int H, i
       }
       if constexpr (SRC == 2) {
 #pragma unroll
-        for (int c = 0; c < NCH; ++c)
+        for (int c = 0; c < NC; ++c)
 #pragma unroll
           for (int j = 0; j < 8; ++j) sm += v[c][j];
         sm = wave_sum(sm);
@@ -635,12 +642,11 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, bool wg0, int H, i
     if constexpr (SRC == 2) {
       __syncthreads();
       mean = ((((0.f + nred[0]) + nred[1]) + nred[2]) + nred[3]) / (float)H;
-      __syncthreads();
     }
     float ss = 0.f;
     if (act) {
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const int e = (c * 256 + t) * 8;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
@@ -649,14 +655,13 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, bool wg0, int H, i
         }
       }
       ss = wave_sum(ss);
-      if (lane == 0) nred[w] = ss;
+      if (lane == 0) nred[16 + w] = ss;                     // (each reduction has words of its own: one barrier each)
     }
     __syncthreads();
-    const float rstd = rsqrtf(((((0.f + nred[0]) + nred[1]) + nred[2]) + nred[3]) / (float)H + na.eps);
-    __syncthreads();                                      // nred is reused below
+    const float rstd = rsqrtf(((((0.f + nred[16]) + nred[17]) + nred[18]) + nred[19]) / (float)H + na.eps);
     if (act) {
 #pragma unroll
-      for (int c = 0; c < NCH; ++c) {
+      for (int c = 0; c < NC; ++c) {
         const int e = (c * 256 + t) * 8;
         if (e < H) {
           float wf[8], bf[8], n1[8];
@@ -685,81 +690,90 @@ __device__ __forceinline__ void l8_prologue(const NormIn& na, bool wg0, int H, i
       }
     }
   }
-  // outliers per thread and chunk, ranked in column order: wave totals of every chunk meet in LDS at one barrier
-  uint32_t take[NCH];
-  int incl[NCH];
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    const int e = (c * 256 + (act ? t : 0)) * 8;
-    uint32_t bits = 0;
-    if (act) {
-      if (e < H) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) bits |= (fabsf(v[c][j]) > na.thr ? 1u : 0u) << j;
-      }
-    }
-    take[c] = bits;
-    incl[c] = __popc(bits);
-    // outliers are few: most waves' runs have none to rank (a plain row of two chunks is faster without the branch: 2560 x
-    // 2560 11.7 us with it, 6.0 without; 2560 x 10240 10.1 with it, 11.1 without)
-    if ((SRC == 0 && NCH <= 2) || __any(bits != 0)) {
-#pragma unroll
-      for (int o = 1; o < 64; o <<= 1) {
-        const int tt = __shfl_up(incl[c], o, 64);
-        if (lane >= o) incl[c] += tt;
-      }
-    }
-    if (act && lane == 63) scr[c * 4 + w] = incl[c];
-  }
-  __syncthreads();
-  int base = 0;                                           // outliers in the chunks before c
-#pragma unroll
-  for (int c = 0; c < NCH; ++c) {
-    const int e = (c * 256 + (act ? t : 0)) * 8;
-    const int n0 = scr[c * 4], n1 = scr[c * 4 + 1], n2 = scr[c * 4 + 2], n3 = scr[c * 4 + 3];
-    const uint32_t bits = take[c];
-    uint32_t tk = 0;
-    if (bits) {
-      int slot = base + (w > 0 ? n0 : 0) + (w > 1 ? n1 : 0) + (w > 2 ? n2 : 0) + incl[c] - __popc(bits);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {                       // (static indices: v stays in registers)
-        if ((bits >> j) & 1u) {
-          if (slot < L8_CMAX) {
-            cols[slot] = e + j;
-            xo[slot] = v[c][j];
-            tk |= 1u << j;
-          }
-          ++slot;
-        }
-      }
-    }
-    take[c] = tk;
-    base += n0 + n1 + n2 + n3;
-  }
-  if (t == 0) scr[L8_COUNT] = min(base, L8_CMAX);
+  // outliers per thread and chunk, ranked in column order, and the largest other number
+  uint32_t take[NC];
+  int incl[NC];
   float am = 0.f;
   if (act) {
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int e = (c * 256 + t) * 8;
-      if (e < H) {
+    for (int c = 0; c < NC; ++c) {
+      uint32_t bits = 0;
+      if ((c * NTH + t) * 8 < H) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-          if (!((take[c] >> j) & 1u)) am = fmaxf(am, fabsf(v[c][j]));
+        for (int j = 0; j < 8; ++j) {
+          const float a = fabsf(v[c][j]);
+          const bool out = a > na.thr;
+          bits |= (out ? 1u : 0u) << j;
+          am = fmaxf(am, out ? 0.f : a);
+        }
       }
+      take[c] = bits;
+      incl[c] = __popc(bits);
+      if (__any(bits != 0)) {                               // outliers are few: most waves have none to rank
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+          const int tt = __shfl_up(incl[c], o, 64);
+          if (lane >= o) incl[c] += tt;
+        }
+      }
+      if (lane == 63) scr[c * WV + w] = incl[c];
     }
     am = wave_max(am);
-    if (lane == 0) nred[w] = am;
+    if (lane == 0) nred[32 + w] = am;
   }
   __syncthreads();
-  const float rm = fmaxf(fmaxf(fmaxf(fmaxf(0.f, nred[0]), nred[1]), nred[2]), nred[3]);
+  int count = 0;
+#pragma unroll
+  for (int i = 0; i < NC * WV; ++i) count += scr[i];
+  if (t == 0) scr[L8_COUNT] = min(count, L8_CMAX);
+  if (act && count > 0) {
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+      if (take[c]) {
+        int slot = incl[c] - __popc(take[c]);
+        for (int i = 0; i < c * WV + w; ++i) slot += scr[i];
+        uint32_t tk = 0;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {                       // (static indices: v stays in registers)
+          if ((take[c] >> j) & 1u) {
+            if (slot < L8_CMAX) {
+              cols[slot] = (c * NTH + t) * 8 + j;
+              xo[slot] = v[c][j];
+              tk |= 1u << j;
+            }
+            ++slot;
+          }
+        }
+        take[c] = tk;
+      }
+  }
+  float rm = 0.f;
+#pragma unroll
+  for (int i = 0; i < WV; ++i) rm = fmaxf(rm, nred[32 + i]);
+  if (count > L8_CMAX) {                                    // workgroup-uniform: outliers past the cap are numbers like any
+    __syncthreads();
+    if (act) {
+#pragma unroll
+      for (int c = 0; c < NC; ++c)
+        if ((c * NTH + t) * 8 < H) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j)
+            if (!((take[c] >> j) & 1u)) am = fmaxf(am, fabsf(v[c][j]));
+        }
+      am = wave_max(am);
+      if (lane == 0) nred[32 + w] = am;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < WV; ++i) rm = fmaxf(rm, nred[32 + i]);
+  }
   const float gm = fmaxf(rm, 1e-8f);
   if (t == 0) nsa[0] = gm / 127.f;
   const float inv = 127.f / gm;
   if (act) {
 #pragma unroll
-    for (int c = 0; c < NCH; ++c) {
-      const int e = (c * 256 + t) * 8;
+    for (int c = 0; c < NC; ++c) {
+      const int e = (c * NTH + t) * 8;
       if (e < H) {
         uint32_t lo = 0, hi = 0;
 #pragma unroll
@@ -799,7 +813,7 @@ __device__ __forceinline__ void w8a8_gemv_body(int bid, const int8_t* __restrict
   __shared__ float l8_xo[L8_N ? L8_CMAX : 1];
   __shared__ int l8_scr[L8_COUNT + 1];
   __shared__ int8_t aq_l[NRM > 0 ? (L8_N ? 1 : NRM_ROWS) * NCH_N * 2048 : 16];
-  __shared__ float nsa[16], nred[16];
+  __shared__ float nsa[16], nred[48];
   constexpr bool GELUQ = EPI == EPI_GELUQT || EPI == EPI_GELUQE;
   static_assert(EPI == EPI_OUT || EPI == EPI_PART || (AMODE == A_TOKEN && (GELUQ || TPW % 2 == 0)),
                 "GLU: gate/up pairs per wave, per-token A");
@@ -884,14 +898,15 @@ __device__ __forceinline__ void w8a8_gemv_body(int bid, const int8_t* __restrict
   // NRM: the first step's weight loads go out before the norm prologue; its activations after
   NormRegs<(NRM > 0 && !LN_N && !L8_N ? NCH_N : 1), (NRM > 0 && !LN_N && !L8_N ? SMAX_N : 1)> nr;
   LnRegs<(LN_N ? NCH_N : 1)> lr;
-  L8Regs<(L8_N ? NCH_N : 1), L8S_N> l8r;
+  constexpr int L8C_N = L8_N ? l8_chunks<NCH_N, L8S_N, NW>() : 1;
+  L8Regs<L8C_N, L8S_N> l8r;
   auto nload = [&]() {
-    if constexpr (L8_N) l8_load(na, bid == 0, K, l8r);
+    if constexpr (L8_N) l8_load<L8C_N, L8S_N, NW>(na, bid == 0, K, l8r);
     else if constexpr (LN_N) ln_load(na, K, M, lr);
     else norm_load(na, K, M, nr);
   };
   auto nprologue = [&]() {
-    if constexpr (L8_N) l8_prologue(na, bid == 0, K, aq_l, nsa, nred, l8_cols, l8_xo, l8_scr, l8r, na.y_out);
+    if constexpr (L8_N) l8_prologue<L8C_N, L8S_N, NW>(na, bid == 0, K, aq_l, nsa, nred, l8_cols, l8_xo, l8_scr, l8r, na.y_out);
     else if constexpr (LN_N) ln_prologue(na, bid == 0, K, M, aq_l, nsa, nred, lr);
     else norm_prologue(na, bid == 0, K, M, aq_l, nsa, nred, nr);
   };
