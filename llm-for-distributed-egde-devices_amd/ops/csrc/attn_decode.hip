@@ -138,9 +138,9 @@ static int g_attn_unroll = 4;
 extern "C" void edge_decode_attn_unroll(int v) { g_attn_unroll = v == 8 ? 8 : 4; }
 // MHA grids below this many workgroups (batch 1: 32 on Llama-2-7B) take the double-buffered form:
 // each workgroup walks its keys in several chunks, and there the next chunk in flight beats the
-// single-buffered form's extra occupancy (tools/recipes/r4occ_b1.sh: 1 x 200 keys 8.71 -> 7.95 us,
-// batch-1 Llama-2-7B 1.960 -> 1.919 ms; 16 x 200 is slower, 16.6 vs 14.6 us).  Tune "decode_attn_small".
-static int g_attn_small_wg = 64;
+// single-buffered form's extra occupancy.  us, single / double buffered, 32 heads of 128, 41 / 141 / 251 keys: 64
+// workgroups 4.75 6.8 7.9 / 4.15 5.9 6.75, 128 5.0 7.2 8.3 / 4.7 6.3 7.8, 256 5.4 8.0 9.5 / 5.1 8.1 10.8.  Tune "decode_attn_small".
+static int g_attn_small_wg = 192;
 extern "C" void edge_decode_attn_small(int v) { g_attn_small_wg = v; }
 extern "C" void edge_decode_attn_gsplit(int v) { g_attn_gsplit = v; }
 extern "C" void edge_decode_attn_early(int v) { g_attn_early = v; }
@@ -234,7 +234,7 @@ int run_attn(const void* q, int64_t q_sb, void* k_cache, void* v_cache, int64_t 
   const int G = G0 / gs;
   const Fuse fz{pos, cs, fused ? rot : 0, q_sb, (int8_t*)out_q, out_s, Mpad, gs, g_attn_early};
   const float sl2 = scale * 1.4426950408889634f;
-  const size_t lds = (size_t)(ATTN_NW * G * D + 2 * ATTN_NW * G + 2 * G) * sizeof(float);
+  const size_t lds = (size_t)(ATTN_NW * G * D + 2 * ATTN_NW * G) * sizeof(float);
   const dim3 grid(nsplit, Hkv * gs, B);
   const bool direct = nsplit == 1;
   const bool small_grid = G0 == 1 && direct && fused && B * Hkv < g_attn_small_wg;

@@ -28,7 +28,7 @@ __device__ __forceinline__ void attn_part(float* smem, int bid, const AttnArgs& 
                                                                     a.out, a.o_sb, a.part_acc, a.part_ml, a.fz);
 }
 template <int D>
-constexpr int attn_part_lds() { return PW * D + 2 * PW + 2; }      // floats
+constexpr int attn_part_lds() { return PW * D + 2 * PW; }      // floats
 }  // namespace
 
 extern "C" int edge_decode_attn_combine(const float* part_acc, const float* part_ml, int nsplit, int B, int Hq, int D, void* out,
