@@ -2,11 +2,13 @@
 // Bound by reading W once, and below some 16 MB by the launch itself.  W stays in its [N, K] layout (no copy is made): a
 // wave takes R rows by 256 k at a time, each load one contiguous KiB of a row (with 16 rows by 16 k per load, the matrix
 // instruction's layout, the loads themselves were the bound: 1024 x 4096, launched one by one, 12.8 us against 5.9 here), the next 256 k on
-// their way meanwhile.  Few rows: KW waves of a workgroup share a row's k (until about 1024 waves are at work) and add up
+// their way meanwhile: a fence keeps the compiler from moving a load behind the products before it, and nothing past the end is
+// loaded.  Few rows: KW waves of a workgroup share a row's k (until about 2048 waves are at work: us at 1 row, 1024 / 2048 / 4096 waves,
+// 4096 x 1024 5.8 / 4.9 / 5.0, 7840 x 1024 8.4 / 7.7 / 7.2, 8192 x 2048 13.3 / 13.3 / 14.0, 2048 x 8192 14.9 / 12.5 / 12.5) and add up
 // through LDS.  All sums in a fixed order.
-// N x K at 2 rows in a graph, us, library / here: 384 x 1024 5.7 / 3.3, 1024 x 4096 9.9 / 4.1, 4096 x 1024 5.9 / 4.1, 6784 x
-// 1024 7.3 / 4.8, 8192 x 2048 13.1 / 12.2, 32000 x 2048 46 / 40 (6.6 TB/s), 128256 x 2048 187 / 167; relative error against
-// 64-bit sums 1e-7 here, 2 to 8e-7 there.
+// N x K at 2 rows in a graph, weights from memory, us, before the fence / now: 384 x 1024 3.1 / 2.9, 1024 x 4096 5.6 / 5.3, 4096 x 1024
+// 5.9 / 5.4, 7840 x 1024 8.9 / 7.8, 8192 x 2048 14.7 / 13.5, 2048 x 8192 14.7 / 12.8, 32000 x 1024 25.7 / 25.5 (5.1 TB/s); relative error
+// against 64-bit sums 1e-7 here, 2 to 8e-7 in the library's product.
 #include "common.h"
 
 namespace {
@@ -16,7 +18,7 @@ __device__ __forceinline__ void gemv_f32_body(int bid, const float* __restrict__
                                               const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K, int KW) {
   constexpr int V = MV * R;
   __shared__ float part[16 * V];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, waves = blockDim.x >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
   const int rg = wave / KW, kw = wave - rg * KW, n0 = (bid * (waves / KW) + rg) * R;
   const int C = (K + 255) / 256;
   float acc[V];
@@ -39,12 +41,14 @@ __device__ __forceinline__ void gemv_f32_body(int bid, const float* __restrict__
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[r * MV + m] = __builtin_fmaf(wv[b][r][j], xv[b][m][j], acc[r * MV + m]);
   };
-  load(0, kw);
+  // both halves' loads go out before either is used, and none past the end (a clamped one is read all the same)
+  if (kw < C) load(0, kw);
   for (int c = kw; c < C; c += 2 * KW) {
-    load(1, c + KW);
+    if (c + KW < C) load(1, c + KW);
+    asm volatile("" ::: "memory");
     use(0, c);
-    load(0, c + 2 * KW);
-    use(1, c + KW);
+    if (c + 2 * KW < C) load(0, c + 2 * KW);
+    if (c + KW < C) use(1, c + KW);
   }
   int idx = 0;
   lane_sums<V, 32>(acc, idx, lane);
@@ -83,7 +87,7 @@ __global__ void __launch_bounds__(1024) gemv_f32x3_kernel(Jobs3 a, int M) {
 int share_k(int groups, int K) {
   const int C = (K + 255) / 256;
   int KW = 1;
-  while (KW < 16 && KW * 2 <= C && groups * KW < 1024) KW *= 2;
+  while (KW < 16 && KW * 2 <= C && groups * KW < 2048) KW *= 2;
   return KW;
 }
 
@@ -112,7 +116,7 @@ void launch_f32x3(Jobs3 a, int M, hipStream_t st) {
 
 // y_j = x_j W_j^T for three projections of the same M rows' inputs, each as edge_gemv_f32 forms it: a parallel layer's three output
 // projections, whose launches' ramps and ends then overlap.  us in a graph, three launches / one, 1024 x 4096 and twice 1024 x
-// 1024: 1 row 11.9 / 7.1, 2 12.6 / 7.5, 8 14.8 / 9.5; 2048 x 8192 and twice 2048 x 2048, 2 rows 27.0 / 22.1
+// 1024: 1 row 11.9 / 6.5, 2 12.6 / 6.7; 2048 x 8192 and twice 2048 x 2048, 2 rows 27.0 / 18.3
 extern "C" int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K,
                                hipStream_t st) {
   Jobs3 a{};
