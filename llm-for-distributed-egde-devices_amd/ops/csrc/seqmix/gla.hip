@@ -253,7 +253,7 @@ __global__ void __launch_bounds__(NT) gla_chunk_scan_kernel(float* __restrict__ 
                                                             float* __restrict__ state, const int* __restrict__ seq_slot,
                                                             const int* __restrict__ seq_start, const int* __restrict__ seq_len,
                                                             int H, int N, int P) {
-  constexpr int UN = 8;
+  constexpr int UN = 16;
   const int s = blockIdx.x, h = blockIdx.y, e = blockIdx.z * NT + threadIdx.x, NP = N * P;
   if (e >= NP) return;
   const int nc = (seq_len[s] + CL - 1) / CL, n = e / P;
@@ -280,6 +280,9 @@ __global__ void __launch_bounds__(NT) gla_chunk_scan_kernel(float* __restrict__ 
 }
 
 // (3) the outputs of one chunk and 16 PT value columns.  Wave i owns the token rows of block i (16 tokens).
+// Bound by its vector instructions (5.6 k a wave, a third of them a block against itself) beside fp32 products at 40 % of their rate.
+// us, 7680 tokens, 16 heads of 128 / 128, this kernel: 288; without branches in the products 258; without a minimum a power 240; rows
+// through the LDS at the end 214.
 // FUSE: all columns of the head are here, so the norm and the gate follow.
 template <typename T, int PT, bool FUSE, bool VEC>
 __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__ u, int ld, const float* __restrict__ la,
@@ -302,7 +305,7 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
   if (c * CL >= len) return;
   const int tc = min(CL, len - c * CL), p0 = pt * CW;
   const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL;
-  const int HN = H * N, HP = H * P, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
+  const int HN = H * N, HP = H * P, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4;
   const float* sin_c = sin_ + (((size_t)chunk_base(seq_len, s) + c) * H + h) * (size_t)N * P + p0;
   const T* base = u + row0 * ld;
   const float qs = 1.f / sqrtf((float)N);
@@ -339,19 +342,20 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
     for (int kk = 0; kk < NK / 4; ++kk) {
       const int n = 4 * kk + g4;
       const float q = Q_s[t][n], bt = B_s[t][n];
+      // (no branches: every wave forms all three earlier blocks' products and counts those before its own, so that a step's
+      // reads go out together; as guarded blocks each wave waited for its LDS reads block by block)
       float tot[3], pre = 0.f;                               // whole-block decays before this wave's block
 #pragma unroll
-      for (int j = 0; j < 3; ++j) { tot[j] = j < wave ? B_s[16 * j + 15][n] : 0.f; pre += tot[j]; }
+      for (int j = 0; j < 3; ++j) { const float x = B_s[16 * j + 15][n]; tot[j] = j < wave ? x : 0.f; pre += tot[j]; }
       const float qr = q * ex2(bt), qa = q * ex2(bt + pre);
 #pragma unroll
       for (int j = 0; j < PT; ++j) o[j] = mfma4(qa, S_s[n][16 * j + l16], o[j]);
       float mid = 0.f;                                       // the blocks between j and this wave's
 #pragma unroll
-      for (int j = 2; j >= 0; --j)
-        if (j < wave) {
-          off_[j] = mfma4(qr, K_s[16 * j + l16][n] * ex2(E_s[16 * j + l16][n] + mid), off_[j]);
-          mid += tot[j];
-        }
+      for (int j = 2; j >= 0; --j) {
+        off_[j] = mfma4(j < wave ? qr : 0.f, K_s[16 * j + l16][n] * ex2(E_s[16 * j + l16][n] + mid), off_[j]);
+        mid += tot[j];
+      }
     }
     // the block against itself: lane holds (row 4 g4 + i, column l16), as the products' results lie
 #pragma unroll 2
@@ -361,8 +365,9 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
       for (int i = 0; i < 4; ++i) {
         const int r = 16 * wave + 4 * g4 + i;
         const float4 q = *reinterpret_cast<const float4*>(&Q_s[r][n]), br = *reinterpret_cast<const float4*>(&B_s[r][n]);
-        dg[i] += q.x * kv.x * ex2(fminf(br.x - bs.x, 0.f)) + q.y * kv.y * ex2(fminf(br.y - bs.y, 0.f)) +
-                 q.z * kv.z * ex2(fminf(br.z - bs.z, 0.f)) + q.w * kv.w * ex2(fminf(br.w - bs.w, 0.f));
+        // (B falls from token to token: no power of a counted pair, column <= row, grows; the others are never read)
+        dg[i] += q.x * kv.x * ex2(br.x - bs.x) + q.y * kv.y * ex2(br.y - bs.y) + q.z * kv.z * ex2(br.z - bs.z) +
+                 q.w * kv.w * ex2(br.w - bs.w);
       }
     }
   }
@@ -381,6 +386,36 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
     const float a = A_s[16 * wave + l16][4 * kk + g4];
 #pragma unroll
     for (int j = 0; j < PT; ++j) o[j] = mfma4(a, V_s[4 * kk + g4][16 * j + l16], o[j]);
+  }
+  if constexpr (FUSE && VEC) {
+    // the rows go through the LDS so that gates and results move 16 bytes a lane (one number a lane: 32 loads, 32 stores and
+    // their addresses, a quarter of the kernel's instructions)
+    float(*Y_s)[LS] = V_s;
+    __syncthreads();                                         // the values are read
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float ss = 0.f;
+#pragma unroll
+      for (int j = 0; j < PT; ++j) ss += o[j][i] * o[j][i];  // columns past P are zero
+      const float r = 1.f / sqrtf(row16_sum(ss) / (float)P + eps);
+#pragma unroll
+      for (int j = 0; j < PT; ++j) Y_s[16 * wave + 4 * g4 + i][16 * j + l16] = o[j][i] * r * norm_w[min(16 * j + l16, P - 1)];
+    }
+    __builtin_amdgcn_wave_barrier();                         // (a wave reads the rows it wrote)
+    constexpr int PER = CW / 8;
+#pragma unroll
+    for (int k = 0; k < 16 * PER / 64; ++k) {
+      const int e = lane + 64 * k, to = 16 * wave + e / PER, p = e % PER * 8;
+      if (to >= tc || p >= P) continue;
+      const size_t row = row0 + to;
+      float z[8], v[8];
+      load8<T>(u + row * ld + 2 * HN + HP + h * P + p, z);
+      load8<float>(&Y_s[to][p], v);
+#pragma unroll
+      for (int q = 0; q < 8; ++q) v[q] *= siluf_(z[q]);
+      store8<T>(out + row * HP + h * P + p, v);
+    }
+    return;
   }
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -474,7 +509,8 @@ int edge_sm_gla_chunked(const void* u, int ld, const float* a2, const float* b, 
   const bool fuse = edge_sm_gla_fused(P);
   if (!fuse && !y) return -2;
   const int ntn = (N + CL - 1) / CL, ntp = (P + CL - 1) / CL;
-  const bool vec = N % 8 == 0 && P % 8 == 0 && ld % 8 == 0 && (((uintptr_t)u | (uintptr_t)la | (uintptr_t)sloc) & 31) == 0;
+  const bool vec = N % 8 == 0 && P % 8 == 0 && ld % 8 == 0 &&
+                   (((uintptr_t)u | (uintptr_t)la | (uintptr_t)sloc | (uintptr_t)out) & 31) == 0;
 #define SM_GC(V)                                                                                                             \
   SM_T(f32, hipLaunchKernelGGL((gla_chunk_state_kernel<T, V>), dim3(max_chunks * ntn * ntp, n, H), dim3(NT),                  \
                                0, st, (const T*)u, ld, a2, b, rank, inv_tau, seq_len, seq_off,    \
