@@ -549,7 +549,7 @@ class DecoderLM(nn.Module):
             return torch.nn.functional.linear(h, self.embed)
         wp, ver = getattr(self, "_embed_wp", None), self.embed._version
         if wp is None or getattr(self, "_embed_wp_ver", -1) != ver or wp.device != self.embed.device:
-            wp = self._embed_wp = ops.pack_bf16_weight(self.embed.detach())
+            wp = self._embed_wp = ops.settle(ops.pack_bf16_weight(self.embed.detach()))
             self._embed_wp_ver = ver
         return ops.linear_bf16(h, self.embed, None, packed=wp)
 

@@ -148,7 +148,7 @@ class Linear(nn.Module):
         """The fragment-packed decode copy of the weight (``decode_weight`` without a sample input)."""
         wp, ver = getattr(self, "_wp", None), self.weight._version
         if wp is None or getattr(self, "_wp_ver", -1) != ver or wp.device != self.weight.device:
-            wp = self._wp = ops.pack_bf16_weight(self.weight.detach())
+            wp = self._wp = ops.settle(ops.pack_bf16_weight(self.weight.detach()))
             self._wp_ver = ver
         return wp
 
@@ -225,7 +225,7 @@ class Linear(nn.Module):
             return None
         wp, ver = getattr(self, "_wp", None), self.weight._version   # in-place weight edits repack
         if wp is None or getattr(self, "_wp_ver", -1) != ver or wp.device != self.weight.device:
-            wp = self._wp = ops.pack_bf16_weight(self.weight.detach())
+            wp = self._wp = ops.settle(ops.pack_bf16_weight(self.weight.detach()))
             self._wp_ver = ver
         return wp
 

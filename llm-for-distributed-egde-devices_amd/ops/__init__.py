@@ -460,6 +460,14 @@ def pack_bf16_weight(w: torch.Tensor) -> torch.Tensor:
     return w.reshape(N // 16, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().view(-1)
 
 
+def settle(t: torch.Tensor) -> torch.Tensor:
+    """Wait for the kernels that lay out a tensor that is kept (a weight's packed copy): the next call that finds it may run
+    on another stream, where nothing orders it behind them (two pipeline lanes whose first calls fall in one tick)."""
+    if t.is_cuda and not torch.cuda.is_current_stream_capturing():
+        torch.cuda.current_stream(t.device).synchronize()
+    return t
+
+
 _GEMV_EPI = {None: 0, "silu_glu": 1, "gelu_tanh": 2, "gelu": 3}
 
 

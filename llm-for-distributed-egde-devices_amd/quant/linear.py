@@ -337,8 +337,8 @@ class LLMInt8Linear(nn.Module):
 
     def _transposed(self, device):
         if self._weight_t is None or self._weight_t.device != device:
-            self._weight_t = self.weight_i8.t().contiguous()          # W^T: outlier columns as rows
             self._w_deq = self.SCB / 127.0
+            self._weight_t = ops.settle(self.weight_i8.t().contiguous())   # W^T: outlier columns as rows
 
     def _forward(self, x, glu: bool = False, act: int = 0, add: Optional[torch.Tensor] = None):
         if isinstance(x, PendingLN):
