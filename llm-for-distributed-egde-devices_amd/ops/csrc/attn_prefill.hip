@@ -107,7 +107,8 @@ __global__ void __launch_bounds__(NT) prefill_attn_kernel(
   char* v_lds = smem + G::K_BYTES;
   const int qtile = blockIdx.x, h = blockIdx.y, b = blockIdx.z;
   const int kvh = h / (Hq / Hkv);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  // (a scalar: what depends on it alone is then a branch, not a mask)
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   char* p_lds = smem + G::K_BYTES + G::V_BYTES + wave * G::P_BYTES;
   const int s0 = start_pos[b];
   const int nkeys = s0 + T;
@@ -353,7 +354,7 @@ __global__ void __launch_bounds__(FA_NT, 1) fa_kernel(
     h = (Hq & 7) == 0 ? (hr & 7) * (Hq >> 3) + (hr >> 3) : hr;
   }
   const int kvh = h / (Hq / Hkv);
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int ql = lane & 31, hf = lane >> 5;                    // query column / half of the wave
   const int s0 = start_pos[b];
   const int nkeys = s0 + T;

@@ -68,7 +68,8 @@ __global__ void __launch_bounds__(NT, (DV * RH <= 4 ? (REL && DK > 2 ? 2 : 4) : 
   const int h0 = blockIdx.y * RH, g = h0 / (H / G);
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
   const int* pt = ptab + (size_t)seq_slot[s] * ptab_ld;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g4 = lane >> 4, c16 = lane & 15;
+  // the wave's number as a scalar: what depends on it alone is then a branch or a scalar address, not a mask
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g4 = lane >> 4, c16 = lane & 15;
   char* p_lds = p_all + wave * 16 * PS * (REL ? 2 : 1);
   const int wq0 = qt * MQ + wave * 16;                       // this wave's first row inside the portion
   v8s qf[RH][DK];

@@ -82,7 +82,7 @@ __global__ void __launch_bounds__(64 * NW) decay_step_kernel(
     T* __restrict__ out, float* __restrict__ y) {
   constexpr int TH = 64 * NW, TC = 8, CW = 64 * CG, NMAX = NW * NRW;
   __shared__ float q_s[TC][NMAX], k_s[TC][NMAX], part_s[TC][NW][CW];
-  const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * CW, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * CW, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int N = a.N, P = a.P, HN = a.H * N, HP = a.H * P, v0 = 2 * HN, g0 = v0 + HP;
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
   const float d = a.dec[h];
@@ -242,7 +242,7 @@ __global__ void __launch_bounds__(NT) decay_chunk_state_kernel(const T* __restri
   stage_qk<T, CL, CL, VEC, true>(K_s, base + HN + h * N, a, seq_start[s] + c * CL, tc, n0, a.k_scale, a.dec[a.H + h], tc - 1);
   stage_plain<T, CL, CL, CL, VEC, true>(V_s, base + 2 * HN + h * P + p0, a.ld, tc, P - p0, a.silu);
   __syncthreads();
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g4 = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g4 = lane >> 4;
   v4f acc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
@@ -314,7 +314,7 @@ __global__ void __launch_bounds__(NT) decay_chunk_out_kernel(const T* __restrict
   const int N = a.N, P = a.P, HN = a.H * N, HP = a.H * P;
   const int tc = min(CL, len - c * CL), p0 = pt * CW, pos0 = seq_start[s] + c * CL;
   const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, l16 = lane & 15, g4 = lane >> 4;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g4 = lane >> 4;
   const float* sin_c = sin_ + (((size_t)chunk_base(seq_len, s) + c) * a.H + h) * (size_t)N * P + p0;
   const T* base = u + row0 * a.ld;
   const float l2 = a.dec[a.H + h];

@@ -87,7 +87,7 @@ __global__ void __launch_bounds__(NT, 2) delta_chunk_solve_kernel(const float* _
   const int t0 = (dp.c0 + c) * CL, tc = min(CL, len - t0), GN = G * N, GD = ONE ? 1 : N;
   const size_t row0 = (size_t)seq_off[s] + t0;
   cb = (cb + c) * H + h;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4;
   const float* pr = prep + row0 * prep_ld;
   const float *qb = pr + (h / (H / G)) * N, *kb = qb + GN, *gb = pr + 2 * GN + h * GD, *bb = pr + 2 * GN + H * GD + h;
   double *M = sc.M + cb * CL * NP, *U = sc.U + cb * CL * PP, *Cs = sc.Cs + cb * CL * CL, *cdec = sc.cdec + cb * NP;
@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(NT) delta_chunk_out_kernel(DeltaScratch sc, co
   const int c = blockIdx.x / ntp, t0 = (blockIdx.x % ntp) * PT, s = blockIdx.y, h = blockIdx.z, len = seq_len[s];
   size_t cb;
   if (c >= chunks_of(len, dp) || !first_chunk(seq_len, s, dp, cb)) return;
-  const int first = (dp.c0 + c) * CL, tc = min(CL, len - first), tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
+  const int first = (dp.c0 + c) * CL, tc = min(CL, len - first), tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4;
   if (16 * wave >= tc) return;
   const size_t row0 = (size_t)seq_off[s] + first;
   cb = (cb + c) * H + h;

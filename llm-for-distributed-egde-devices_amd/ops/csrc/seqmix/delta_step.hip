@@ -34,7 +34,7 @@ __global__ void __launch_bounds__(N * P / 32 < 256 ? 256 : 512) delta_step_kerne
   static_assert(2 * N + P <= NTH && N % 64 == 0 && P % 64 == 0 && N % RGS == 0 && PG <= 64, "shape");
   __shared__ __attribute__((aligned(16))) float q_s[N], k_s[N], g_s[N], v_s[P], z_s[P], sk_s[NW][P], sq_s[NW][P];
   __shared__ float ss_s[NW], kq_s;
-  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, H = a.H;
+  const int s = blockIdx.x, h = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), H = a.H;
   const int slot = a.seq_slot[s], start = a.seq_start[s];
   const size_t t = a.seq_off[s];
   const int C = 2 * H * N + H * P;

@@ -43,7 +43,7 @@ __global__ void __launch_bounds__(64 * NW) gla_step_kernel(
     float* __restrict__ y, int H, int N, int P, float inv_tau, float eps) {
   constexpr int TH = 64 * NW, TC = 8, CW = 64 * CG, NMAX = NW * NRW;
   __shared__ float q_s[TC][NMAX], k_s[TC][NMAX], a_s[TC][NMAX], part_s[TC][NW][CW];
-  const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * CW, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * CW, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
   const int HN = H * N, HP = H * P, v0 = 2 * HN, g0 = v0 + HP, d0 = g0 + HP;
   const float qs = 1.f / sqrtf((float)N);
@@ -227,7 +227,7 @@ __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict
   const size_t cb = (size_t)chunk_base(seq_len, s) + c;
   if (p0 == 0 && seg == 0 && n < N) cdec[(cb * H + h) * N + n] = ex2(end);
   __syncthreads();
-  const int lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g4 = lane >> 4;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4;
   v4f acc[4];
 #pragma unroll
   for (int j = 0; j < 4; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};

@@ -467,7 +467,7 @@ __global__ void __launch_bounds__(NT) delta_prep_kernel(const T* __restrict__ qk
                                                         const float* __restrict__ A_log, float* __restrict__ prep, int H, int G,
                                                         int N) {
   const size_t t = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, GN = G * N, HN = H * N;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), GN = G * N, HN = H * N;
   float* pr = prep + t * (2 * GN + HN + H);
   const float qs = 1.f / sqrtf((float)N);
   for (int unit = wave; unit < 2 * G; unit += NT / 64) {     // unit = (q | k, kv head): one wave each
@@ -503,7 +503,7 @@ __global__ void __launch_bounds__(NT) delta_scan_kernel(const float* __restrict_
   __shared__ __attribute__((aligned(16))) float rows_s[2][TC][3][NP];   // q | k | decay
   __shared__ float v_s[2][TC][CW], b_s[2][TC];
   const int s = blockIdx.x, h = blockIdx.y, p0 = blockIdx.z * CW, tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6, rg = lane & 15, col = wave * 4 + (lane >> 4), p = p0 + col;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), rg = lane & 15, col = wave * 4 + (lane >> 4), p = p0 + col;
   const int start = seq_start[s], len = seq_len[s], off = seq_off[s];
   if (len >= below) return;                                  // (run over chunks)
   const int g = h / (H / G), GN = G * N, HN = H * GD;
@@ -923,7 +923,7 @@ __global__ void __launch_bounds__(NT) moe_gate_up_kernel(const T* __restrict__ h
                                                          int rows_per_wg, int E, int silu, const float* __restrict__ in_w) {
   extern __shared__ __attribute__((aligned(16))) float h_s[];   // [W]
   const size_t pair = blockIdx.x, t = pair / top;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int c = tid; c < W; c += NT) h_s[c] = ldf<T>(h + t * W + c);
   __syncthreads();
   const T* wg = w_gu + (size_t)min(max(idx[pair], 0), E - 1) * 2 * ff * W;
@@ -959,7 +959,7 @@ __global__ void __launch_bounds__(NT) moe_down_kernel(const T* __restrict__ y, i
                                                       int rows_per_wg, int E) {
   extern __shared__ __attribute__((aligned(16))) float y_s[];   // [ff]
   const size_t pair = blockIdx.x;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   for (int c = tid; c < ff; c += NT) y_s[c] = ldf<T>(y + pair * ff + c);
   __syncthreads();
   const T* wd = w_down + (size_t)min(max(idx[pair], 0), E - 1) * W * ff;
@@ -1008,7 +1008,7 @@ __global__ void __launch_bounds__(NT) relu2_experts_kernel(const T* __restrict__
                                                            int sff, T* __restrict__ out, T* __restrict__ out_sh,
                                                            int rows_per_wg, int E) {
   extern __shared__ __attribute__((aligned(16))) float v_s[];
-  const int pair = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int pair = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const bool sh = pair >= routed;
   const int t = sh ? pair - routed : pair / top, f = sh ? sff : ff, K = UP ? W : f, R = UP ? f : W;
   const int r0 = blockIdx.y * rows_per_wg, r1 = min(R, r0 + rows_per_wg);

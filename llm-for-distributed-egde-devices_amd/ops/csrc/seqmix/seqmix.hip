@@ -212,7 +212,7 @@ __device__ __forceinline__ void attn_chunk(const KT* __restrict__ kbase, const K
                                            float cap = 0.f, const float* sl_s = nullptr, int dist = 0,
                                            const float* __restrict__ rel = nullptr, int rel_n = 0) {
   constexpr int AW = VEC ? 8 : DVL;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // (A) scores
   {
     float a[RMAX];
@@ -366,7 +366,7 @@ __global__ void __launch_bounds__(NT) attn_kernel(const T* __restrict__ q, const
   // more than RMAX query heads per kv head: nsp workgroups share the kv head, RMAX heads each
   const int t = blockIdx.x, g = blockIdx.y / nsp, r0 = (blockIdx.y % nsp) * RMAX;
   const int R = min(RMAX, H / G - r0), hq0 = g * (H / G) + r0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float* q_s = smem;                         // [RMAX][D]
   float* s_s = q_s + RMAX * D;               // [RMAX][KC]
   float* red = s_s + RMAX * KC;              // [RMAX][Dv]
