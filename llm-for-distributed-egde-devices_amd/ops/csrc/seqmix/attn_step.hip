@@ -9,6 +9,11 @@
 // the waves meet once, in LDS, at the end.  A workgroup's time is its vector instructions then (some 1.5 us for 128 keys and four
 // heads, 0.7 for one), so few queries run one head a workgroup; reading the next rows ahead took registers and gained nothing, and
 // an unrolled end cost 30 KB of code that every launch has to fetch (6.0 -> 18 us).
+// One head of fp32 rows takes its scores on the vector ALU: 16 products a lane and two exchanges instead of 16 matrix instructions of
+// which 15 rows in 16 are idle, and half their error (4e-7 -> 2.7e-7 of the result, against 64 bits).  us, a launch in a graph, before /
+// after: 16 heads of 64 in 4 groups, 2 tokens behind 777 (window 512, 16 blocks) 9.2 / 8.2, 8 behind 400 8.6 / 7.8; of 128, 1 behind 700 15.5 /
+// 14.6.  What is left there is the bytes of one CU: four times the keys in flight, the next rows ahead, other workgroups fetching them
+// into the L2 and 64 keys a wave at a time all gave nothing.
 // us, attn_kernel with its sum over key splits / this (bf16 but for the first): fp32, 16 heads of 64 in 4 groups, 2 tokens behind
 // 777 (window 512, 16 blocks) 15.3 / 9.9; latent rows of 160, 16 heads, 4 tokens behind 97 19.4 / 5.2; of 320, 6 behind 1100 (window 1024)
 // 35.1 / 27.0, 1 behind 7600 56 / 21; 16 heads of 128 in 4 groups, 6 in chunks of 1000 20.7 / 13.3.
@@ -40,27 +45,31 @@ struct StepArgs {
   float scale, cap, out_scale;
 };
 
-// 16 keys' rows of one wave: lane (key = lane & 15, 16-byte parts 4 c + (lane >> 4) of its row) and values (LPK lanes a key)
+// 16 keys' rows of one wave: lane (key = lane & 15, parts 4 c + (lane >> 4) of 8 numbers of its row) and values (LPK lanes a key, 8
+// numbers each).  fp32 queries: the two halves of a part are 16 (of values 4 LPK) numbers apart, so that neighbouring lanes of every
+// load read neighbouring 16 bytes (a workgroup's time is the bytes that its CU takes in, some 70 a ns)
 template <typename KT, int NC, int DVL>
 struct Tile {
   static constexpr int Q = sizeof(KT) / 2, VP = 2 * DVL;
   uint4 k[NC][Q], v[VP][Q];
 };
 
-template <typename KT, int NC, int DVL>
+template <typename KT, int NC, int DVL, bool F32>
 __device__ __forceinline__ void tile_load(Tile<KT, NC, DVL>& t, const KT* kb, const KT* vb, int row, int kld, int vld, int D, int Dv) {
   constexpr int LPK = 8 * DVL, KPR = 64 / LPK;
-  const int lane = threadIdx.x & 63, grp = lane >> 4, dp = min(lane % LPK * 8, Dv - 8);
+  const int lane = threadIdx.x & 63, grp = lane >> 4, vl = lane % LPK;
   const KT* kr = kb + (size_t)row * kld;
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int q = 0; q < Tile<KT, NC, DVL>::Q; ++q) t.k[c][q] = reinterpret_cast<const uint4*>(kr + min(32 * c + 8 * grp, D - 8))[q];
+    for (int q = 0; q < Tile<KT, NC, DVL>::Q; ++q)
+      t.k[c][q] = *reinterpret_cast<const uint4*>(F32 ? kr + min(32 * c + 16 * q + 4 * grp, D - 4) : kr + min(32 * c + 8 * grp, D - 8) + 4 * q);
 #pragma unroll
   for (int p = 0; p < Tile<KT, NC, DVL>::VP; ++p) {
-    const KT* vr = vb + (size_t)__shfl(row, p * KPR + lane / LPK, 64) * vld + dp;
+    const KT* vr = vb + (size_t)__shfl(row, p * KPR + lane / LPK, 64) * vld;
 #pragma unroll
-    for (int q = 0; q < Tile<KT, NC, DVL>::Q; ++q) t.v[p][q] = reinterpret_cast<const uint4*>(vr)[q];
+    for (int q = 0; q < Tile<KT, NC, DVL>::Q; ++q)
+      t.v[p][q] = *reinterpret_cast<const uint4*>(F32 ? vr + min(4 * (LPK * q + vl), Dv - 4) : vr + min(8 * vl, Dv - 8) + 4 * q);
   }
 }
 
@@ -109,15 +118,19 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
   const int* pt = a.ptab + (size_t)a.seq_slot[a.tok_seq[t]] * a.ptab_ld;
   // the queries as the matrix cores' rows: row = lane & 15 is head row % SH; numbers past D (or heads past R) are zero
   const T* qp = reinterpret_cast<const T*>(a.q) + ((size_t)t * a.H + hq0 + min(key % SH, R - 1)) * D;
+  constexpr bool F32 = sizeof(T) == 4, DOT = F32 && SH == 1;
   uint4 qr[NC][Tile<T, NC, DVL>::Q];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
-    for (int e = 0; e < Tile<T, NC, DVL>::Q; ++e) {
-      const int d = 32 * c + 8 * grp;
-      qr[c][e] = reinterpret_cast<const uint4*>(qp + min(d, D - 8))[e];
-      if (d >= D || (key % SH) >= R) qr[c][e] = uint4{0u, 0u, 0u, 0u};
-    }
+    for (int e = 0; e < Tile<T, NC, DVL>::Q; ++e)
+      qr[c][e] = *reinterpret_cast<const uint4*>(F32 ? qp + min(32 * c + 16 * e + 4 * grp, D - 4) : qp + min(32 * c + 8 * grp, D - 8));
+  asm volatile("" ::: "memory");        // (all on their way before one is looked at)
+#pragma unroll
+  for (int c = 0; c < NC; ++c)
+#pragma unroll
+    for (int e = 0; e < Tile<T, NC, DVL>::Q; ++e)
+      if ((F32 ? 32 * c + 16 * e + 4 * grp : 32 * c + 8 * grp) >= D || (key % SH) >= R) qr[c][e] = uint4{0u, 0u, 0u, 0u};
   float m[SH], l[SH], acc[SH * 8];
 #pragma unroll
   for (int r = 0; r < SH; ++r) { m[r] = -INFINITY; l[r] = 0.f; }
@@ -148,7 +161,7 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
 #pragma unroll 1
     for (; x0 < end; x0 += RK) {
       TL tl;
-      tile_load<KT, NC, DVL>(tl, kbase, vbase, rw, kld, vld, D, Dv);
+      tile_load<KT, NC, DVL, F32>(tl, kbase, vbase, rw, kld, vld, D, Dv);
       rw = row_of(x0 + RK);                                  // (past the end: the last key's, not used)
       v4f s2[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};     // (two sums: half the chain)
 #pragma unroll
@@ -164,10 +177,16 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
           load8<T>(reinterpret_cast<const T*>(&qr[c][0]), qf);
           load8<float>(reinterpret_cast<const float*>(&tl.k[c][0]), kf8);
 #pragma unroll
-          for (int j = 0; j < 8; ++j) s = mfma4(qf[j], in ? kf8[j] : 0.f, s);
+          for (int j = 0; j < 8; ++j) {
+            const float kx = (F32 ? 32 * c + 16 * (j / 4) + 4 * grp < D : in) ? kf8[j] : 0.f;
+            if constexpr (DOT) s[j & 3] = fmaf(qf[j], kx, s[j & 3]);
+            else s = mfma4(qf[j], kx, s);
+          }
         }
       }
-      v4f s = (s2[0] + s2[1]) * a.scale;
+      v4f s = s2[0] + s2[1];
+      if constexpr (DOT) s[0] = xor_sum(xor_sum((s[0] + s[1]) + (s[2] + s[3]), 16), 32);
+      s *= a.scale;
       shape(s, x0 + key);                                    // (s[r], r < SH: head r's score of this lane's key)
       const bool ok = x0 + key < n;
       float p[SH], mn[SH];
@@ -261,7 +280,10 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
   constexpr int VN = SH * 8 / KPR;                           // numbers a lane is left with, from off on
   const int d0 = lane % LPK * 8;
 #pragma unroll
-  for (int j = 0; j < VN; ++j) red[wave][(off + j) / 8][d0 + (off + j) % 8] = acc[j];
+  for (int j = 0; j < VN; ++j) {
+    const int e = (off + j) % 8;
+    red[wave][(off + j) / 8][F32 ? 4 * (LPK * (e / 4) + lane % LPK) + e % 4 : d0 + e] = acc[j];
+  }
   if (lane == 0) {
 #pragma unroll
     for (int r = 0; r < SH; ++r) { m_s[wave][r] = m[r]; l_s[wave][r] = l[r]; }
