@@ -58,21 +58,15 @@ class WindowPoolAttention(nn.Module):
 
     def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
         """``u`` columns [c0, ..) hold q | k | v | gate.  Returns the o-projection's output [T, W]."""
-        return self.o(self.heads(u, c0, meta, run))
-
-    def heads(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, q: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """The o-projection's input; ``q``: the rotated queries, when they and the cached rows and block means are there already."""
         s = self.spec
         nq, nk, nv, ng = s.proj_sizes
-        written = q is not None
-        if not written:
-            proj = u[:, c0:c0 + nq + nk + nv]
-            q = seqmix.rope_paged_write(proj, meta, self.rope(meta.max_keys, u.device), run.k, run.v, s.heads, s.rot_dims)
-        if s.window is not None and s.pool and not written:
+        proj = u[:, c0:c0 + nq + nk + nv]
+        q = seqmix.rope_paged_write(proj, meta, self.rope(meta.max_keys, u.device), run.k, run.v, s.heads, s.rot_dims)
+        if s.window is not None and s.pool:
             seqmix.pool_blocks(run.k, run.v, run.k_pool, run.v_pool, meta, s.pool)
         gate = u[:, c0 + nq + nk + nv:c0 + nq + nk + nv + ng] if ng else None
-        return seqmix.window_pool_attention(q, gate, run.k, run.v, run.k_pool, run.v_pool, meta, s.scale, s.window,
-                                            s.pool if s.window is not None else None)
+        return self.o(seqmix.window_pool_attention(q, gate, run.k, run.v, run.k_pool, run.v_pool, meta, s.scale, s.window,
+                                                   s.pool if s.window is not None else None))
 
 
 class SSDMixer(nn.Module):
@@ -93,17 +87,12 @@ class SSDMixer(nn.Module):
 
     def forward(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run) -> torch.Tensor:
         """``u`` columns [c0, ..) hold z | x | B | C | dt.  Returns the o-projection's output [T, W]."""
-        return self.o(self.rows(u, c0, meta, run))
-
-    def rows(self, u: torch.Tensor, c0: int, meta: seqmix.RaggedMeta, run, xbc: Optional[torch.Tensor] = None) -> torch.Tensor:
-        """The o-projection's input; ``xbc``: the convolved x | B | C rows, when they are there already."""
         s = self.spec
         inner, C = s.inner, s.conv_channels
-        if xbc is None:
-            xbc = seqmix.conv_silu(u, c0 + inner, C, self.conv_w, self.conv_b, run.conv, meta)
+        xbc = seqmix.conv_silu(u, c0 + inner, C, self.conv_w, self.conv_b, run.conv, meta)
         y = seqmix.ssd_scan(xbc, u, c0 + inner + C, self.dt_bias, self.A_log, self.D, run.ssm, meta, s.heads, s.vdim,
                             s.state, s.groups)
-        return seqmix.gated_group_norm(y, u[:, c0:c0 + inner], self.norm_w, s.norm_groups, self.eps, u.dtype)
+        return self.o(seqmix.gated_group_norm(y, u[:, c0:c0 + inner], self.norm_w, s.norm_groups, self.eps, u.dtype))
 
 
 class ParallelMixer(nn.Module):
@@ -130,6 +119,15 @@ class ParallelMixer(nn.Module):
                                        a.rot_dims, a.pool if a.window is not None and a.pool else 0, sum(a.proj_sizes) + s.inner,
                                        self.right.conv_w, self.right.conv_b, run.conv, f0, ff)
 
+    def step_heads(self, u: torch.Tensor, c0: int, meta, run, q: torch.Tensor, xbc: torch.Tensor):
+        """Both output projections' inputs from ``step_in``'s queries and x | B | C rows: the two mixers side by side."""
+        a, s, r = self.left.spec, self.right.spec, self.right
+        g0, ng = sum(a.proj_sizes[:3]), a.proj_sizes[3]
+        att, y = seqmix.attention_beside_scan(q, u[:, g0:g0 + ng] if ng else None, run.k, run.v, run.k_pool, run.v_pool, meta, a.scale,
+                                              a.window, a.pool if a.window is not None else None, xbc, u, c0 + s.inner + s.conv_channels,
+                                              r.dt_bias, r.A_log, r.D, run.ssm, s.heads, s.vdim, s.state, s.groups)
+        return att, seqmix.gated_group_norm(y, u[:, c0:c0 + s.inner], r.norm_w, s.norm_groups, r.eps, u.dtype)
+
     def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None, pre=None,
                 down: Optional[nn.Module] = None):
         """x fp32 [T, W] (residual stream, updated in place) += mixer(u) + extra.  ``nxt``: the norm that reads x next; its rows
@@ -138,7 +136,7 @@ class ParallelMixer(nn.Module):
         if pre is None:
             a, r = self.left(u, 0, meta, run), self.right(u, c0, meta, run)
         else:
-            ins = self.left.heads(u, 0, meta, run, pre[0]), self.right.rows(u, c0, meta, run, pre[1])
+            ins = self.step_heads(u, c0, meta, run, pre[0], pre[1])
             if down is not None:
                 extra, a, r = rows_together((pre[2], *ins), (down, self.left.o, self.right.o))
             else:

@@ -18,7 +18,7 @@
 // 777 (window 512, 16 blocks) 15.3 / 9.9; latent rows of 160, 16 heads, 4 tokens behind 97 19.4 / 5.2; of 320, 6 behind 1100 (window 1024)
 // 35.1 / 27.0, 1 behind 7600 56 / 21; 16 heads of 128 in 4 groups, 6 in chunks of 1000 20.7 / 13.3.
 #include "common.h"
-#include "seqmix/seqmix_common.h"
+#include "seqmix/ssd_step.h"
 
 extern "C" int edge_sm_attention_rmax(int rows, int H, int G, int D, int Dv);
 extern "C" int edge_sm_attention_splits(int rows, int G, int chunks);
@@ -100,7 +100,7 @@ __device__ __forceinline__ float exp_neg(float x) {
 }
 
 template <typename T, int NC, int DVL, int SH, bool POOL, bool EX>
-__global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
+__device__ __forceinline__ void attn_step_body(const StepArgs& a, int block) {
   constexpr int NW = STEP_NW, LPK = 8 * DVL, KPR = 64 / LPK, VP = 2 * DVL, RK = 16 * NW, DR = 64 * DVL;
   __shared__ __attribute__((aligned(16))) float p_s[NW][16][SH];
   __shared__ __attribute__((aligned(16))) float red[NW][SH][DR];
@@ -108,7 +108,7 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
   __shared__ __attribute__((aligned(16))) float y_s[EX ? DR : 1], e_s[EX ? NW : 1][EX ? MAX_VDIM : 1];
   // consecutive workgroups go to the eight dies in turn: those of one (token, kv head, part of its keys) stay on one die, where they
   // read the same rows
-  const int unit = blockIdx.x % 8 + 8 * (blockIdx.x / 8 / a.nsp), sub = blockIdx.x / 8 % a.nsp;
+  const int unit = block % 8 + 8 * (block / 8 / a.nsp), sub = block / 8 % a.nsp;
   if (unit >= a.rows * a.G * a.nsplit) return;
   const int z = unit % a.nsplit, g = unit / a.nsplit % a.G, t = unit / a.nsplit / a.G, r0 = sub * SH, D = a.D, Dv = a.Dv;
   const int R = min(SH, a.H / a.G - r0), hq0 = g * (a.H / a.G) + r0;
@@ -359,6 +359,49 @@ __global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
   }
 }
 
+template <typename T, int NC, int DVL, int SH, bool POOL, bool EX>
+__global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
+  attn_step_body<T, NC, DVL, SH, POOL, EX>(a, blockIdx.x);
+}
+
+// One head a workgroup over whole keys, beside one token of the state-space recurrence, two heads a workgroup: a parallel layer's two
+// mixers, which wait for nothing of each other and leave most of the chip idle each.  The workgroups behind those fetch: `fetch` of them
+// bring a (query, kv head) pair's keys and values into the L2 of the die whose workgroups walk them, where one CU takes in what it waits for
+// at the pace of its own misses.  us in a decode step whose weights have passed through the caches since (fp32, 16 heads of 64 in 4
+// groups, 2 tokens behind 800, window 512, 16 state heads of 64 x 64): attention 11.2 and state 4.7 in two launches (attention with the
+// fetching 9.9, with products on the vector ALU 10.8), this 9.1; a prompt of 777 and 15 such steps, four layers, 6.79 -> 6.47 ms.
+// Fetched in the launch before instead (parallel_step.hip), attention is at 9.2 alone, but that launch at 6.8 instead of 4.6.
+template <typename T, int NC, int DVL, bool POOL, int N, int P>
+__global__ void __launch_bounds__(STEP_NW * 64) attn_ssd_kernel(StepArgs a, SsdStep s, int heads, int fetch) {
+  __shared__ __attribute__((aligned(16))) float sum_s[STEP_NW * 64 / NT][NT / 64][P];
+  const int units = a.rows * a.G, own = (units + 7) / 8 * 8 * a.nsp, tid = threadIdx.x;
+  int b = blockIdx.x;
+  if (b < own) return attn_step_body<T, NC, DVL, 1, POOL, false>(a, b);
+  b -= own;
+  if (b >= heads) {                                          // (heads: a multiple of 8, and so is own: b % 8 is the die)
+    b -= heads;
+    const int unit = b % 8 + 8 * (b / 8 / fetch), part = b / 8 % fetch;
+    if (unit >= units) return;
+    const int g = unit % a.G, t = unit / a.G, i = a.tok_pos[t], jlo = a.window > 0 ? max(0, i - a.window + 1) : 0;
+    const int* pt = a.ptab + (size_t)a.seq_slot[a.tok_seq[t]] * a.ptab_ld;
+    const int kparts = a.D * (int)sizeof(T) / 16, per = kparts + a.Dv * (int)sizeof(T) / 16, n = (i - jlo + 1) * per;
+    uint32_t seen = 0;
+#pragma unroll 4
+    for (int e = part * (STEP_NW * 64) + tid; e < n; e += fetch * (STEP_NW * 64)) {
+      const int j = jlo + e / per, c = e % per;
+      const size_t row = (pt[j >> a.page_sh] << a.page_sh) + (j & (a.page - 1));
+      const T* at = c < kparts ? reinterpret_cast<const T*>(a.kp) + row * a.kld + g * a.D + c * (16 / sizeof(T))
+                               : reinterpret_cast<const T*>(a.vp) + row * a.vld + g * a.Dv + (c - kparts) * (16 / sizeof(T));
+      seen |= *reinterpret_cast<const uint32_t*>(at);
+    }
+    asm volatile("" ::"v"(seen));
+    return;
+  }
+  const int pairs = s.H / 2, q = b / pairs;
+  if (q >= a.rows) return;
+  ssd_step_body<T, N, P>(s, q, b % pairs * 2 + tid / NT, tid % NT, sum_s[tid / NT]);
+}
+
 template <typename T, int SH, bool EX>
 int run_step(const StepArgs& a, hipStream_t st) {
   const dim3 grid((a.rows * a.G * a.nsplit + 7) / 8 * 8 * a.nsp), block(STEP_NW * 64);
@@ -378,6 +421,24 @@ int run_step(const StepArgs& a, hipStream_t st) {
   else STEP(10, 4, false);
 #undef STEP
   return (int)hipGetLastError();
+}
+
+template <typename T, int NC, int DVL, bool POOL>
+int run_beside(const StepArgs& a, const SsdStep& s, int N, int P, hipStream_t st) {
+  const int units8 = (a.rows * a.G + 7) / 8, own = units8 * 8 * a.nsp, heads = (a.rows * s.H / 2 + 7) / 8 * 8;
+  const int fetch = max(0, min(12, (256 - own - heads) / (8 * units8)));    // as the chip has CUs left
+#define BESIDE(NN, PP)                                                                                                          \
+  if (N == NN && P == PP) {                                                                                                     \
+    hipLaunchKernelGGL((attn_ssd_kernel<T, NC, DVL, POOL, NN, PP>), dim3(own + heads + units8 * 8 * fetch), dim3(STEP_NW * 64), 0, st, a, \
+                       s, heads, fetch);                                                                                        \
+    return (int)hipGetLastError();                                                                                              \
+  }
+  BESIDE(64, 64)
+  BESIDE(128, 64)
+  BESIDE(64, 128)
+  BESIDE(128, 128)
+#undef BESIDE
+  return -2;
 }
 
 // Estimates in us, fitted to both kernels' times at 936 points (13 shapes of 8 to 64 heads of 32 to 320 numbers, both types, 1 to 400 rows
@@ -489,6 +550,29 @@ int edge_sm_attention_expand(const void* q, const void* gate, int gate_ld, const
                         : (f32 ? run_step<float, 4, false>(a, st) : run_step<bf16_t, 4, false>(a, st));
   if (r != 0 || nsplit == 1) return r;
   return edge_sm_attn_merge(part, gate, gate_ld, out, rows, H, G, Dv, nsp, nsplit, sh, gate_elem, out_ld, out_scale, f32, st);
+}
+
+// edge_sm_attention_step for plans of one head a workgroup over whole keys, rows of up to 128 numbers and plain scores, with
+// edge_sm_ssd_step's token of every sequence in the same launch (rows: the sequences).  -2: nothing done
+int edge_sm_attention_ssd(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb, const float* vb,
+                          const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab, int ptab_ld, void* out, int rows,
+                          int H, int G, int D, int Dv, int page, int PB, float scale, int window, int pool, int f32, int plan, int kld,
+                          int vld, const float* sink, int gate_elem, int out_ld, const void* xbc, int Cx, const void* u, int ld, int dt0,
+                          const float* dt_bias, const float* A_log, const float* Dp, float* state, const int* seq_start,
+                          const int* seq_off, float* y, int Hs, int P, int N, int groups, hipStream_t st) {
+  if (plan != 9 || rows < 1 || G < 1 || H % G || D > 128 || Dv > 128 || page < 1 || (page & (page - 1)) || (pool & (pool - 1)) ||
+      out_ld < H * Dv || ((uintptr_t)xbc | (uintptr_t)state) % 16 || Cx % 8 || groups < 1 || Hs < 2 || Hs % 2 || Hs % groups)
+    return -2;
+  const int pool_sh = window > 0 && pool > 0 ? __builtin_ctz(pool) : -1;
+  const StepArgs a{q, gate, kp, vp, kb, vb, tok_seq, tok_pos, seq_slot, ptab, out, nullptr, nullptr, sink, nullptr, nullptr, 0, rows, gate_ld,
+                   ptab_ld, H, G, D, Dv, page, __builtin_ctz(page), PB, window, pool_sh, H / G, 1, kld, vld, 0, gate_elem, 0, 0, out_ld,
+                   scale, 0.f, 1.f};
+  const SsdStep s{xbc, u, dt_bias, A_log, Dp, state, y, seq_slot, seq_start, seq_off, Cx, ld, dt0, Hs, groups};
+#define BESIDE(TT)                                                                                                     \
+  (D <= 64 && Dv <= 64 ? pool_sh >= 0 ? run_beside<TT, 2, 1, true>(a, s, N, P, st) : run_beside<TT, 2, 1, false>(a, s, N, P, st) \
+                       : pool_sh >= 0 ? run_beside<TT, 4, 2, true>(a, s, N, P, st) : run_beside<TT, 4, 2, false>(a, s, N, P, st))
+  return f32 ? BESIDE(float) : BESIDE(bf16_t);
+#undef BESIDE
 }
 
 // plan as edge_sm_attention_step_plan says, part edge_sm_attention_step_floats numbers; the rest as edge_sm_attention's

@@ -73,6 +73,12 @@ int edge_sm_attention_expand(const void* q, const void* gate, int gate_ld, const
                              int window, int pool, int f32, int plan, float* part, int kld, int vld, int chunked, float cap,
                              const float* slopes, const float* sink, int gate_elem, int keep_first, const float* rel, int rel_n,
                              int out_ld, float out_scale, const void* uv, int vdim, hipStream_t st);
+int edge_sm_attention_ssd(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb, const float* vb,
+                          const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* ptab, int ptab_ld, void* out, int rows,
+                          int H, int G, int D, int Dv, int page, int PB, float scale, int window, int pool, int f32, int plan, int kld,
+                          int vld, const float* sink, int gate_elem, int out_ld, const void* xbc, int Cx, const void* u, int ld, int dt0,
+                          const float* dt_bias, const float* A_log, const float* Dp, float* state, const int* seq_start,
+                          const int* seq_off, float* y, int Hs, int P, int N, int groups, hipStream_t st);
 int edge_sm_attention_splits(int rows, int G, int chunks);
 size_t edge_sm_attention_part_floats(int rows, int H, int G, int D, int Dv, int nsplit);
 int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp,
@@ -573,10 +579,10 @@ at::Tensor sm_conv_silu(const at::Tensor& u, int64_t c0, int64_t C, const at::Te
   return out;
 }
 
-at::Tensor sm_ssd_scan(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, const at::Tensor& dt_bias,
-                       const at::Tensor& A_log, const at::Tensor& D, at::Tensor& state, const at::Tensor& seq_slot,
-                       const at::Tensor& seq_start, const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n,
-                       int64_t Hs, int64_t P, int64_t N, int64_t groups, int64_t chunks, int64_t max_chunks, bool one) {
+// the row stride of u, with everything a recurrence over it asks of its operands
+int chk_ssd(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, const at::Tensor& dt_bias, const at::Tensor& A_log, const at::Tensor& D,
+            const at::Tensor& state, const at::Tensor& seq_slot, const at::Tensor& seq_start, const at::Tensor& seq_len,
+            const at::Tensor& seq_off, int64_t n, int64_t Hs, int64_t P, int64_t N, int64_t groups) {
   const int ld = row_ld(u, "u");
   chk_f32(dt_bias, "dt_bias");
   chk_f32(A_log, "A_log");
@@ -592,6 +598,14 @@ at::Tensor sm_ssd_scan(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, 
               "state: fp32 [slots, heads, N, vdim]");
   TORCH_CHECK(seq_slot.numel() >= n && seq_start.numel() >= n && seq_len.numel() >= n && seq_off.numel() >= n,
               "sequence metadata: [n]");
+  return ld;
+}
+
+at::Tensor sm_ssd_scan(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, const at::Tensor& dt_bias,
+                       const at::Tensor& A_log, const at::Tensor& D, at::Tensor& state, const at::Tensor& seq_slot,
+                       const at::Tensor& seq_start, const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n,
+                       int64_t Hs, int64_t P, int64_t N, int64_t groups, int64_t chunks, int64_t max_chunks, bool one) {
+  const int ld = chk_ssd(xbc, u, dt0, dt_bias, A_log, D, state, seq_slot, seq_start, seq_len, seq_off, n, Hs, P, N, groups);
   c10::hip::HIPGuardMasqueradingAsCUDA guard(xbc.device());
   auto y = at::empty({xbc.size(0), Hs * P}, xbc.options().dtype(at::kFloat));
   if (chunks > 0) {
@@ -623,6 +637,63 @@ at::Tensor sm_ssd_scan(const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, 
                          seq_start.data_ptr<int>(), seq_len.data_ptr<int>(), seq_off.data_ptr<int>(), y.data_ptr<float>(),
                          (int)n, (int)Hs, (int)P, (int)N, (int)groups, f32(xbc), stream()), "sm_ssd_scan");
   return y;
+}
+
+// a decode step's two mixers of a parallel layer in one launch: sm_attention (plain scores) and sm_ssd_scan of one token a sequence ->
+// (heads, y); nothing done where attention is not attn_step_kernel's with one head a workgroup over whole keys
+std::optional<std::tuple<at::Tensor, at::Tensor>> sm_attention_ssd(
+    const at::Tensor& q, const std::optional<at::Tensor>& gate, const at::Tensor& kp, const at::Tensor& vp, const std::optional<at::Tensor>& kb,
+    const std::optional<at::Tensor>& vb, const at::Tensor& tok_seq, const at::Tensor& tok_pos, const at::Tensor& ptab, double scale,
+    int64_t window, int64_t pool, int64_t max_keys, const at::Tensor& xbc, const at::Tensor& u, int64_t dt0, const at::Tensor& dt_bias,
+    const at::Tensor& A_log, const at::Tensor& Dp, at::Tensor& state, const at::Tensor& seq_slot, const at::Tensor& seq_start,
+    const at::Tensor& seq_len, const at::Tensor& seq_off, int64_t n, int64_t Hs, int64_t P, int64_t N, int64_t groups) {
+  const int ld = chk_ssd(xbc, u, dt0, dt_bias, A_log, Dp, state, seq_slot, seq_start, seq_len, seq_off, n, Hs, P, N, groups);
+  chk_i32(tok_seq, "tok_seq");
+  chk_i32(tok_pos, "tok_pos");
+  chk_table(ptab);
+  TORCH_CHECK(q.is_cuda() && q.dim() == 3 && q.is_contiguous() && is_act(q) && q.scalar_type() == xbc.scalar_type() &&
+                  q.device() == xbc.device(), "q: [T, H, D] beside x | B | C rows of its type");
+  const int64_t T = q.size(0), H = q.size(1), D = q.size(2);
+  TORCH_CHECK(kp.is_cuda() && vp.is_cuda() && kp.scalar_type() == q.scalar_type() && vp.scalar_type() == q.scalar_type() && kp.dim() == 4 &&
+                  vp.dim() == 4 && kp.size(3) == D && vp.size(0) == kp.size(0) && vp.size(1) == kp.size(1) && vp.size(2) == kp.size(2),
+              "pages: [pages, page, G, D] in q's dtype");
+  if (!kp.is_contiguous() || !vp.is_contiguous()) return std::nullopt;
+  const int64_t page = kp.size(1), G = kp.size(2), Dv = vp.size(3);
+  TORCH_CHECK(T == n && xbc.size(0) == n && tok_seq.numel() == T && tok_pos.numel() == T, "one token per sequence");
+  TORCH_CHECK(max_keys <= ptab.size(1) * page, "page table too short for the step");
+  int gate_ld = 0, PB = 0;
+  if (gate) {
+    gate_ld = row_ld(*gate, "gate");
+    TORCH_CHECK(gate->size(0) == T && (gate->size(1) == H * Dv || gate->size(1) == H) && gate->scalar_type() == q.scalar_type(),
+                "gate: [T, H] (one per head) or [T, H Dv] (one per coordinate)");
+  }
+  if (pool > 0 && window > 0) {
+    TORCH_CHECK(kb && vb, "pooled entries missing");
+    chk_f32(*kb, "k_pool");
+    chk_f32(*vb, "v_pool");
+    PB = (int)kb->size(1);
+    TORCH_CHECK(kb->size(0) == kp.size(0) && PB == (page + pool - 1) / pool && kb->size(2) == G && kb->size(3) == D &&
+                    vb->size(0) == kp.size(0) && vb->size(1) == PB && vb->size(2) == G && vb->size(3) == Dv,
+                "pooled entries: [pages, ceil(page / pool), G, D]");
+  }
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(q.device());
+  const int64_t vis = (window > 0 ? std::min<int64_t>(window, max_keys) : max_keys) + (PB ? max_keys / pool : 0);
+  const uintptr_t addresses = (uintptr_t)q.data_ptr() | (uintptr_t)kp.data_ptr() | (uintptr_t)vp.data_ptr() |
+                              (uintptr_t)(PB ? kb->data_ptr<float>() : nullptr) | (uintptr_t)(PB ? vb->data_ptr<float>() : nullptr);
+  const int plan = edge_sm_attention_step_plan((int)T, (int)H, (int)G, (int)D, (int)Dv, (int)kp.stride(1), (int)vp.stride(1), (int)page,
+                                               PB ? (int)pool : 0, vis, f32(q), addresses);
+  auto out = at::empty({T, H * Dv}, q.options()), y = at::empty({T, Hs * P}, q.options().dtype(at::kFloat));
+  const int rc = edge_sm_attention_ssd(
+      q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(), vp.data_ptr(), PB ? kb->data_ptr<float>() : nullptr,
+      PB ? vb->data_ptr<float>() : nullptr, tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(), ptab.data_ptr<int>(),
+      (int)ptab.stride(0), out.data_ptr(), (int)T, (int)H, (int)G, (int)D, (int)Dv, (int)page, PB, (float)scale, (int)window,
+      PB ? (int)pool : 0, f32(q), plan, (int)kp.stride(1), (int)vp.stride(1), nullptr, gate && gate->size(1) == H * Dv ? 1 : 0,
+      (int)out.stride(0), xbc.data_ptr(), (int)xbc.size(1), u.data_ptr(), ld, (int)dt0, dt_bias.data_ptr<float>(), A_log.data_ptr<float>(),
+      Dp.data_ptr<float>(), state.data_ptr<float>(), seq_start.data_ptr<int>(), seq_off.data_ptr<int>(), y.data_ptr<float>(), (int)Hs,
+      (int)P, (int)N, (int)groups, stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_attention_ssd");
+  return std::make_tuple(out, y);
 }
 
 // ---------------------------------------------------------------------------------- post-norm layers
@@ -1668,6 +1739,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_attention", &sm_attention);
   m.def("sm_conv_silu", &sm_conv_silu);
   m.def("sm_ssd_scan", &sm_ssd_scan);
+  m.def("sm_attention_ssd", &sm_attention_ssd);
   m.def("sm_embed_bigram", &sm_embed_bigram);
   m.def("sm_canon", &sm_canon);
   m.def("sm_ln_residual_taps", &sm_ln_residual_taps);

@@ -428,6 +428,22 @@ def conv_silu(u: torch.Tensor, c0: int, C: int, weight: torch.Tensor, bias: torc
 SSD_CHUNK_MIN = int(__import__("os").environ.get("EDGELLM_SSD_CHUNK_MIN", "32"))
 
 
+def attention_beside_scan(q: torch.Tensor, gate: Optional[torch.Tensor], k_pages, v_pages, k_pool, v_pool, meta: RaggedMeta, scale: float,
+                          window: Optional[int], pool: Optional[int], xbc: torch.Tensor, u: torch.Tensor, dt0: int, dt_bias, A_log, D,
+                          state: torch.Tensor, heads: int, vdim: int, N: int, groups: int):
+    """``window_pool_attention`` and ``ssd_scan`` of a step in which every sequence brings one token -> (heads, y): one launch where
+    attention takes one head a workgroup, else the two ops."""
+    if _gpu(q) and meta.max_len == 1 and meta.T == meta.n and q.dtype == xbc.dtype and min(SSD_CHUNK_MIN, ATTN_MFMA_MIN) > 1:
+        both = _ext().sm_attention_ssd(q, gate, k_pages, v_pages, k_pool if pool else None, v_pool if pool else None, meta.tok_seq,
+                                       meta.tok_pos, meta.page_table, float(scale), int(window or 0), int(pool or 0), int(meta.max_keys),
+                                       xbc, u, int(dt0), dt_bias, A_log, D, state, meta.seq_slot, meta.seq_start, meta.seq_len,
+                                       meta.seq_off, int(meta.n), int(heads), int(vdim), int(N), int(groups))
+        if both is not None:
+            return both
+    return (window_pool_attention(q, gate, k_pages, v_pages, k_pool, v_pool, meta, scale, window, pool),
+            ssd_scan(xbc, u, dt0, dt_bias, A_log, D, state, meta, heads, vdim, N, groups))
+
+
 def ssd_scan(xbc: torch.Tensor, u: torch.Tensor, dt0: int, dt_bias, A_log, D, state: torch.Tensor,
              meta: RaggedMeta, heads: int, vdim: int, N: int, groups: int) -> torch.Tensor:
     """The state-space recurrence, token by token in fp32.  xbc [T, x | B | C] (after conv + silu),
