@@ -268,7 +268,8 @@ STEP_OPS = ["embedding_scaled", "scalar_rms_norm", "relu2", "cat_cast", "combine
             "embedding_learned", "parallel_update", "glu_gelu", "moe_route_grouped", "moe_experts_shared",
             "latent_expand_write", "head_expand_gate", "gated_linear_attention", "decay_linear_attention", "softcap",
             "parallel_step_in", "combine_residual_norm", "layer_norm_residual_canon", "layer_norm_residual_norm",
-            "group_norm_residual_norm", "delta_step", "latent_attention", "moe_experts_glu_shared"]
+            "group_norm_residual_norm", "delta_step", "latent_attention", "moe_experts_glu_shared",
+            "attention_beside_scan", "layer_norm_residual_canon_route"]
 
 
 def op_times(eng: RaggedEngine, entries, close=()) -> Dict[str, float]:

@@ -134,8 +134,15 @@ class PostNormLayer(nn.Module):
         if h is None:
             h = seqmix.canon_conv(x, self.canon1, run.canon1, meta, self.dtype) if self.canon1 is not None else x.to(self.dtype)
         last = self.ff is None
-        h2 = self._join(self.norm1, x, meta, nxt if last else (self.canon2, run.canon2) if self.canon2 is not None else None,
-                        self.mix(h, meta, run))
+        y = self.mix(h, meta, run)
+        if not last and self.canon2 is not None and type(self.ff) is MoEFeedForward and unwatched(self.ff):
+            # the experts' choice with the row that it reads
+            n, f, s = self.norm1, self.ff, self.ff.spec
+            h2, choice = seqmix.layer_norm_residual_canon_route(x, y, n.weight, n.bias, n.eps, self.canon2, run.canon2, meta, self.dtype,
+                                                                f.router, s.top, s.scale, s.router, f.router_b)
+            h2 = self._join(self.norm2, x, meta, nxt, *f(h2, choice))
+            return x if nxt is None else (x, h2)
+        h2 = self._join(self.norm1, x, meta, nxt if last else (self.canon2, run.canon2) if self.canon2 is not None else None, y)
         if not last:
             shared, parts, wts = self.ff(x.to(self.dtype) if h2 is None else h2)
             h2 = self._join(self.norm2, x, meta, nxt, shared, parts, wts)

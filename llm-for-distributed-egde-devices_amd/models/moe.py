@@ -51,11 +51,12 @@ class MoEFeedForward(nn.Module):
             self.shared_gu = Linear(width, up * s.shared_ff, False, dtype, device)
             self.shared_down = Linear(s.shared_ff, width, False, dtype, device)
 
-    def forward(self, h: torch.Tensor):
+    def forward(self, h: torch.Tensor, choice=None):
         """h [T, W] -> (shared expert's output [T, W] or None, expert outputs [T, top, W], weights fp32
-        [T, top] still to be applied to them, or None when the experts ran on weighted inputs)."""
+        [T, top] still to be applied to them, or None when the experts ran on weighted inputs).  ``choice``: the experts' ids and
+        weights, when they are there already."""
         s = self.spec
-        idx, wts = seqmix.moe_route(h, self.router, s.top, s.scale, s.router, self.router_b)
+        idx, wts = seqmix.moe_route(h, self.router, s.top, s.scale, s.router, self.router_b) if choice is None else choice
         on_input = s.weight_on == "input"
         if s.shared_ff and h.shape[0] <= seqmix.MOE_GLU_SHARED_MOST and s.act == "glu_clamp" and not on_input \
                 and plain_linear(self.shared_gu) and plain_linear(self.shared_down):

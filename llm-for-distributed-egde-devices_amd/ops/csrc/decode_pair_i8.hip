@@ -2,7 +2,7 @@
 // preparation (outlier ranking and quantisation of its row) in front of its weights; side by side the
 // preparations of two overlap, and the attention's reads hide behind up's.  8 waves a workgroup, two workgroups to a CU.
 // us a layer of Phi-2: attention 5.7 and up 9.1 are 8.3 together, o 6.0 and down 10.2 are 8.1 (9.7 and 11.1 while 256 threads
-// prepared the row); whole answers against separate launches: Phi-2 32 tokens 47.8 -> 34.2 ms.
+// prepared the row); whole answers against separate launches: Phi-2 32 tokens 47.8 -> 33.6 ms.
 #include "decode_pair.h"
 #include "gemv_i8.h"
 

@@ -24,6 +24,10 @@ int edge_sm_rope_write(const void* proj, int ld, const int* tok_seq, const int* 
 int edge_sm_ln_residual_taps(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b,
                              const float* cw, float* state, const int* tok_seq, const int* tok_pos, const int* seq_slot, void* out,
                              int rows, int W, float eps, int f32, hipStream_t st);
+int edge_sm_ln_residual_taps_route(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b,
+                                   const float* cw, float* state, const int* tok_seq, const int* tok_pos, const int* seq_slot, void* out,
+                                   int rows, int W, float eps, const float* router, const float* bias, int E, int top, float scale,
+                                   int sigm, int* idx, float* wts, int f32, hipStream_t st);
 int edge_sm_ln_residual_ln(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b, float eps,
                            const float* w2, const float* b2, float eps2, void* out, int rows, int W, int f32, hipStream_t st);
 int edge_sm_group_residual_norm(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, int groups,
@@ -842,6 +846,39 @@ std::optional<at::Tensor> sm_ln_residual_taps(at::Tensor& x, const std::optional
   if (rc == -2) return std::nullopt;
   check(rc, "sm_ln_residual_taps");
   return out;
+}
+
+// sm_ln_residual_taps and sm_moe_route of its rows in one launch -> (rows, ids, weights); nothing done where it is not one
+std::optional<std::tuple<at::Tensor, at::Tensor, at::Tensor>> sm_ln_residual_taps_route(
+    at::Tensor& x, const std::optional<at::Tensor>& y, const at::Tensor& w, const at::Tensor& b, double eps,
+    const std::optional<at::Tensor>& parts, const std::optional<at::Tensor>& part_w, const at::Tensor& cw, at::Tensor& state,
+    const at::Tensor& tok_seq, const at::Tensor& tok_pos, const at::Tensor& seq_slot, bool out_f32, const at::Tensor& router, int64_t top,
+    double scale, int64_t mode, const std::optional<at::Tensor>& bias) {
+  for (const at::Tensor* f : {(const at::Tensor*)&x, &w, &b, &cw, (const at::Tensor*)&state, &router})
+    chk_f32(*f, "x, weights, state, router");
+  for (const at::Tensor* t : {&tok_seq, &tok_pos, &seq_slot}) chk_i32(*t, "metadata");
+  const int64_t T = x.size(0), W = x.size(1);
+  TORCH_CHECK(x.dim() == 2 && w.numel() == W && b.numel() == W && cw.dim() == 2 && cw.size(0) == W, "x [T, W], weights [W], taps [W, n]");
+  TORCH_CHECK(tok_seq.numel() == T && tok_pos.numel() == T, "one token per sequence");
+  TORCH_CHECK(router.dim() == 2 && router.size(1) == W && mode >= 0 && mode <= 2, "router: fp32 [E, W]");
+  if (bias) {
+    chk_f32(*bias, "bias");
+    TORCH_CHECK(bias->numel() == router.size(0), "bias: fp32 [E]");
+  }
+  const Results r = results_of(x, y, parts, part_w);
+  if (cw.size(1) != 4 || (r.is_f32 != 0) != out_f32 || top < 1 || top > router.size(0)) return std::nullopt;
+  TORCH_CHECK(state.dim() == 3 && state.size(1) == 3 && state.size(2) == W, "state: fp32 [slots, 3, W]");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(x.device());
+  auto out = at::empty({T, W}, x.options().dtype(act_type(out_f32)));
+  auto idx = at::empty({T, top}, x.options().dtype(at::kInt)), wts = at::empty({T, top}, x.options());
+  const int rc = edge_sm_ln_residual_taps_route(
+      x.data_ptr<float>(), r.y, r.parts, r.pw, r.K, w.data_ptr<float>(), b.data_ptr<float>(), cw.data_ptr<float>(),
+      state.data_ptr<float>(), tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(), out.data_ptr(), (int)T, (int)W,
+      (float)eps, router.data_ptr<float>(), bias ? bias->data_ptr<float>() : nullptr, (int)router.size(0), (int)top, (float)scale,
+      (int)mode, idx.data_ptr<int>(), wts.data_ptr<float>(), r.is_f32, stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_ln_residual_taps_route");
+  return std::make_tuple(out, idx, wts);
 }
 
 std::optional<at::Tensor> sm_ln_residual_ln(at::Tensor& x, const std::optional<at::Tensor>& y, const at::Tensor& w, const at::Tensor& b,
@@ -1743,6 +1780,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_embed_bigram", &sm_embed_bigram);
   m.def("sm_canon", &sm_canon);
   m.def("sm_ln_residual_taps", &sm_ln_residual_taps);
+  m.def("sm_ln_residual_taps_route", &sm_ln_residual_taps_route);
   m.def("sm_ln_residual_ln", &sm_ln_residual_ln);
   m.def("sm_group_residual_norm", &sm_group_residual_norm);
   m.def("sm_combine_norm", &sm_combine_norm);

@@ -16,6 +16,7 @@
 #include "seqmix/seqmix_common.h"
 #include "seqmix/delta_prep.h"
 #include "seqmix/moe_rows.h"
+#include "seqmix/route_few.h"
 #include "seqmix/row_parts.h"
 #include "seqmix/tap4.h"
 
@@ -782,28 +783,6 @@ __global__ void __launch_bounds__(64) route_grouped_kernel(const float* __restri
 // tokens, which is two workgroups a CU, and three scores a wave: us, two launches / one, 16 experts of 1024, 4 tokens 6.8 / 4.0, 64
 // 6.9 / 4.1, 512 8.4 / 5.1; 32 of 2048 7.5 / 5.6, 7.8 / 5.8, 13.2 / 10.3; grouped with a gate, 16 of 1024 7.9 / 5.3, 8.5 / 5.5, 10.1 / 7.8, 32
 // of 2048 8.6 / 7.5, 9.3 / 7.8, 14.5 / 13.5; not 64 of 4096, 4 tokens 12.1 / 22.7.
-constexpr int RF_WAVES = 16, RF_SCORES = 48;
-struct RouteFew {
-  const float *router, *bias;                                // bias: GROUPED the correction of the choice
-  int W, E, gate, groups, keep, top, sigm;
-  float scale;
-  int* idx;
-  float *wts, *gate_w;
-};
-
-// what the whole wave holds most of among lanes with v > floor: its lowest lane, -1 for none
-__device__ __forceinline__ int best_lane(float v, float floor, float& best) {
-  const bool in = v > floor;
-  float m = in ? v : -INFINITY;
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0xB1, 0xF, 0xF, false)));
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x4E, 0xF, 0xF, false)));
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x124, 0xF, 0xF, false)));
-  m = fmaxf(m, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, m), 0x128, 0xF, 0xF, false)));
-  auto row = [&](int l) { return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), l)); };
-  best = fmaxf(fmaxf(row(0), row(16)), fmaxf(row(32), row(48)));
-  return __ffsll((unsigned long long)__ballot(in && v == best)) - 1;
-}
-
 template <typename T, int EPW, bool GROUPED>
 __global__ void __launch_bounds__(RF_WAVES * 64) route_few_kernel(const T* __restrict__ h, RouteFew a) {
   __shared__ float z_s[RF_SCORES], c_s[64], g_s[64];
@@ -832,70 +811,7 @@ __global__ void __launch_bounds__(RF_WAVES * 64) route_few_kernel(const T* __res
     if (lane == 0 && e < n) z_s[e] = s + (!GROUPED && a.bias ? a.bias[e] : 0.f);
   }
   __syncthreads();
-  if (wave != 0) return;
-  const int E = a.E, top = a.top;
-  const bool live = lane < E;
-  const float z = live ? z_s[lane] : -INFINITY;
-  auto softmax = [&]() {
-    const float mx = wave_max(z), ex = live ? expf(z - mx) : 0.f;
-    return ex / wave_sum(ex);
-  };
-  float tot = 0.f, my_w = 0.f;
-  int my_i = 0;                                              // lane k keeps the k-th choice
-  if constexpr (GROUPED) {
-    const float s = softmax();
-    float c = live ? s + (a.bias ? a.bias[lane] : 0.f) : -INFINITY;
-    if (a.groups > 1) {
-      const int size = E / a.groups, g = min(lane / size, a.groups - 1);
-      c_s[lane] = c;
-      __builtin_amdgcn_wave_barrier();                       // (one wave: its LDS accesses keep their order)
-      float b = -INFINITY;
-      for (int e = g * size; e < (g + 1) * size; ++e) b = fmaxf(b, c_s[e]);
-      g_s[g] = b;
-      __builtin_amdgcn_wave_barrier();
-      int better = 0;
-      for (int o = 0; o < a.groups; ++o) better += g_s[o] > b || (g_s[o] == b && o < g);
-      if (better >= a.keep) c = -INFINITY;
-    }
-    for (int k = 0; k < top; ++k) {
-      float best;
-      int bi = best_lane(c, -INFINITY, best);
-      if (bi < 0) bi = k;                                    // scores that compare with nothing (NaN): keep the ids in range
-      const float w = __shfl(s, bi, 64);
-      if (lane == k) { my_w = w; my_i = bi; }
-      tot += w;
-      if (lane == bi) c = -INFINITY;
-    }
-    if (a.gate && lane == 0) a.gate_w[t] = sigmoidf_(z_s[E]);
-  } else {
-    float v = z;
-    if (!a.sigm) {                                           // (every lane takes part in its sums)
-      v = softmax();
-      if (!live) v = -2.f;
-    }
-    const float floor = a.sigm ? -INFINITY : -1.f, gone = a.sigm ? -INFINITY : -2.f;
-    for (int k = 0; k < top; ++k) {
-      float best;
-      int bi = best_lane(v, floor, best);
-      if (bi < 0) {
-        bi = k;
-        best = 0.f;
-      }
-      if (lane == k) { my_w = best; my_i = bi; }
-      if (lane == bi) v = gone;
-      tot += best;
-    }
-  }
-  float soft = 0.f;
-  if (!GROUPED && a.sigm == 2) {
-    const float ex = lane < top ? expf(my_w - __shfl(my_w, 0, 64)) : 0.f;
-    soft = ex / wave_sum(ex);
-  }
-  if (lane < top) {
-    a.idx[t * top + lane] = my_i;
-    a.wts[t * top + lane] = (!GROUPED && a.sigm == 2) ? soft * a.scale : (!GROUPED && a.sigm) ? sigmoidf_(my_w) * a.scale
-                                                                                             : my_w / (tot + 1e-20f) * a.scale;
-  }
+  if (wave == 0) route_choose<GROUPED>(a, z_s, c_s, g_s, t);
 }
 
 // whether one launch takes the step

@@ -12,6 +12,7 @@
 // a norm, 1024, 4 tokens 7.0 / 3.7, 2048 9.5 / 4.2, 4096 tokens 52.9 / 24.8.
 #include "common.h"
 #include "seqmix/row_parts.h"
+#include "seqmix/route_few.h"
 
 namespace {
 
@@ -20,51 +21,55 @@ __device__ __forceinline__ int col(int i, int W) { return min(((int)threadIdx.x 
 
 // x += LayerNorm(y + sum_k pw[k] parts[k]) w + b;  out = x + sum_k cw[:, k] x_(pos - 3 + k), x_pos this row and the three before it
 // the slot's tail [3][W] (zero before position 0), which moves up.  The sums are ln_residual4_kernel's and tap4_kernel's.
+constexpr int RT_MOST = 1024, RT_ROWS = 256;                // widest row and most rows with the choice of experts in the launch
 struct Taps {
   const float* w;                                            // [W, 4]
   float* state;                                              // [slots, 3, W]
   const int *tok_seq, *tok_pos, *seq_slot;
 };
-template <typename T, int CH>
-__global__ void __launch_bounds__(NT) ln_residual_taps_kernel(float* __restrict__ x, const T* __restrict__ y,
-                                                              const T* __restrict__ parts, const float* __restrict__ pw, int K,
-                                                              const float* __restrict__ w, const float* __restrict__ b, int W,
-                                                              float eps, Taps a, T* __restrict__ out) {
-  __shared__ float red[2][NT / 64];
-  const size_t t = blockIdx.x;
+// by NW waves; done(c, o): the four numbers of out from column c on
+template <typename T, int CH, int NW, typename E, typename F>
+__device__ __forceinline__ void ln_residual_taps_row(size_t t, float* __restrict__ x, const T* __restrict__ y, const T* __restrict__ parts,
+                                                     const float* __restrict__ pw, int K, const float* __restrict__ w,
+                                                     const float* __restrict__ b, int W, float eps, const Taps& a, T* __restrict__ out,
+                                                     float (*red)[NW], E&& early, F&& done) {
   const int pos = a.tok_pos[t], seq = a.tok_seq[t];
   float v[CH][4], xv[CH][4], wv[CH][4], bv[CH][4], sum = 0.f;
   float4 cw[CH][4];
-#pragma unroll
-  for (int i = 0; i < CH; ++i) {
-    const int c = col(i, W);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) v[i][e] = 0.f;
-    if (y) load4<T>(y + t * W + c, v[i]);
-    load4<float>(x + t * W + c, xv[i]);
-    load4<float>(w + c, wv[i]);
-    load4<float>(b + c, bv[i]);
-#pragma unroll
-    for (int e = 0; e < 4; ++e) cw[i][e] = *reinterpret_cast<const float4*>(a.w + (size_t)(c + e) * 4);
-  }
-  float* st = a.state + (size_t)a.seq_slot[seq] * 3 * W;
   float tail[CH][3][4];
+  const bool holds = NW == NT / 64 || __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * 256 < W;   // (a wave with part of the row)
+  float* st = a.state + (size_t)a.seq_slot[seq] * 3 * W;
+  if (holds) {
 #pragma unroll
-  for (int i = 0; i < CH; ++i)
+    for (int i = 0; i < CH; ++i) {
+      const int c = col(i, W);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) load4<float>(st + (size_t)k * W + col(i, W), tail[i][k]);
-  add_parts<T, CH>(v, parts, pw, K, t, W);
+      for (int e = 0; e < 4; ++e) v[i][e] = 0.f;
+      if (y) load4<T>(y + t * W + c, v[i]);
+      load4<float>(x + t * W + c, xv[i]);
+      load4<float>(w + c, wv[i]);
+      load4<float>(b + c, bv[i]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) cw[i][e] = *reinterpret_cast<const float4*>(a.w + (size_t)(c + e) * 4);
+    }
+#pragma unroll
+    for (int i = 0; i < CH; ++i)
+#pragma unroll
+      for (int k = 0; k < 3; ++k) load4<float>(st + (size_t)k * W + col(i, W), tail[i][k]);
+  }
+  early();
+  if (holds) add_parts<T, CH>(v, parts, pw, K, t, W);
 #pragma unroll
   for (int i = 0; i < CH; ++i)
     if (in_row(i, W)) sum += (v[i][0] + v[i][1]) + (v[i][2] + v[i][3]);
-  const float mean = row_total(sum, red[0]) / (float)W;
+  const float mean = row_total<NW>(sum, red[0]) / (float)W;
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < CH; ++i)
     if (in_row(i, W))
 #pragma unroll
       for (int e = 0; e < 4; ++e) { const float d = v[i][e] - mean; ss += d * d; }
-  const float r = 1.f / sqrtf(row_total(ss, red[1]) / (float)W + eps);
+  const float r = 1.f / sqrtf(row_total<NW>(ss, red[1]) / (float)W + eps);
 #pragma unroll
   for (int i = 0; i < CH; ++i) {
     if (!in_row(i, W)) continue;
@@ -87,7 +92,65 @@ __global__ void __launch_bounds__(NT) ln_residual_taps_kernel(float* __restrict_
     store4<float>(st + c, tail[i][1]);
     store4<float>(st + W + c, tail[i][2]);
     store4<float>(st + 2 * (size_t)W + c, xv[i]);
+    done(c, o);
   }
+}
+
+template <typename T, int CH>
+__global__ void __launch_bounds__(NT) ln_residual_taps_kernel(float* __restrict__ x, const T* __restrict__ y,
+                                                              const T* __restrict__ parts, const float* __restrict__ pw, int K,
+                                                              const float* __restrict__ w, const float* __restrict__ b, int W,
+                                                              float eps, Taps a, T* __restrict__ out) {
+  __shared__ float red[2][NT / 64];
+  ln_residual_taps_row<T, CH, NT / 64>(blockIdx.x, x, y, parts, pw, K, w, b, W, eps, a, out, red, [] {}, [](int, const float*) {});
+}
+
+// The same with the choice of the row's experts: the row stays in LDS and 16 waves form the scores of an expert each, whose router rows
+// are on their way behind the row's own (route_few_kernel's sums and choice).  us, two launches / this, rows of 1024, 16 experts, bf16: 4
+// rows 6.3 / 5.4, 64 6.6 / 5.7, 256 8.1 / 6.7; of 512, 4 rows 5.8 / 5.0; a decode of 4 sequences, 63 steps of four such layers, 14.98 -> 14.78 ms.  Two
+// scores a wave over rows of 2048 leave one CU with a router of 256 KB: 4 rows 8.6 / 10.6, 256 12.1 / 13.5, so those stay two launches.
+template <typename T>
+__global__ void __launch_bounds__(RF_WAVES * 64) ln_residual_taps_route_kernel(
+    float* __restrict__ x, const T* __restrict__ y, const T* __restrict__ parts, const float* __restrict__ pw, int K,
+    const float* __restrict__ w, const float* __restrict__ b, int W, float eps, Taps a, T* __restrict__ out, RouteFew r) {
+  constexpr int MOST = RT_MOST / 512;
+  __shared__ float red[2][RF_WAVES], z_s[RF_WAVES];
+  __shared__ __attribute__((aligned(16))) float h_s[RT_MOST];
+  const size_t t = blockIdx.x;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  float rv[MOST][8];
+  auto early = [&] {                                         // (behind the row's loads, which are waited for first)
+    asm volatile("" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < MOST; ++i)
+      load8<float>(r.router + (size_t)min(wave, r.E - 1) * W + min(i * 512 + lane * 8, W - 8), rv[i]);
+    asm volatile("" ::: "memory");
+  };
+  ln_residual_taps_row<T, 1, RF_WAVES>(t, x, y, parts, pw, K, w, b, W, eps, a, out, red, early, [&](int c, const float* o) {
+    float h[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      T v;
+      stf<T>(&v, o[e]);
+      h[e] = ldf<T>(&v);
+    }
+    store4<float>(h_s + c, h);
+  });
+  __syncthreads();
+  float acc = 0.f;
+#pragma unroll
+  for (int i = 0; i < MOST; ++i) {
+    const int c = i * 512 + lane * 8;
+    if (c >= W) break;
+    float h[8];
+    load8<float>(h_s + c, h);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc += h[j] * rv[i][j];
+  }
+  const float s = wave_sum(acc);
+  if (lane == 0 && wave < r.E) z_s[wave] = s + (r.bias ? r.bias[wave] : 0.f);
+  __syncthreads();
+  if (wave == 0) route_choose<false>(r, z_s, nullptr, nullptr, t);
 }
 
 // x += LayerNorm(y + sum_k pw[k] parts[k]) w + b;  out = LayerNorm(x) w2 + b2
@@ -298,6 +361,26 @@ int edge_sm_ln_residual_taps(float* x, const void* y, const void* parts, const f
   const Taps a{cw, state, tok_seq, tok_pos, seq_slot};
   if (f32) RN_CH(ln_residual_taps_kernel, float, x, (const float*)y, (const float*)parts, pw, K, w, b, W, eps, a, (float*)out);
   else RN_CH(ln_residual_taps_kernel, bf16_t, x, (const bf16_t*)y, (const bf16_t*)parts, pw, K, w, b, W, eps, a, (bf16_t*)out);
+  return (int)hipGetLastError();
+}
+
+// edge_sm_ln_residual_taps and edge_sm_moe_route (postnorm.hip) of its rows, up to 16 experts
+int edge_sm_ln_residual_taps_route(float* x, const void* y, const void* parts, const float* pw, int K, const float* w, const float* b,
+                                   const float* cw, float* state, const int* tok_seq, const int* tok_pos, const int* seq_slot, void* out,
+                                   int rows, int W, float eps, const float* router, const float* bias, int E, int top, float scale,
+                                   int sigm, int* idx, float* wts, int f32, hipStream_t st) {
+  if (!row_ok(W, {x, y, parts, w, b, cw, state, out, router}) || W > RT_MOST || W % 8 || rows > RT_ROWS || E < 1 || E > RF_WAVES ||
+      top < 1 || top > E)
+    return -2;
+  if (rows == 0) return 0;
+  const Taps a{cw, state, tok_seq, tok_pos, seq_slot};
+  const RouteFew r{router, bias, W, E, 0, 1, 1, top, sigm, scale, idx, wts, nullptr};
+#define RT(TT)                                                                                                               \
+  hipLaunchKernelGGL(ln_residual_taps_route_kernel<TT>, dim3(rows), dim3(RF_WAVES * 64), 0, st, x, (const TT*)y, (const TT*)parts, pw, K, w, \
+                     b, W, eps, a, (TT*)out, r)
+  if (f32) RT(float);
+  else RT(bf16_t);
+#undef RT
   return (int)hipGetLastError();
 }
 

@@ -28,14 +28,15 @@ __device__ __forceinline__ void add_parts(float (&v)[CH][4], const T* __restrict
   }
 }
 
-// sum of s over the workgroup (r: NT / 64 numbers of LDS, used once)
+// sum of s over the workgroup of NW waves (r: NW numbers of LDS, used once)
+template <int NW = NT / 64>
 __device__ __forceinline__ float row_total(float s, float* r) {
   s = wave_sum(s);
   if ((threadIdx.x & 63) == 0) r[threadIdx.x >> 6] = s;
   __syncthreads();
   float o = 0.f;
 #pragma unroll
-  for (int i = 0; i < NT / 64; ++i) o += r[i];
+  for (int i = 0; i < NW; ++i) o += r[i];
   return o;
 }
 

@@ -561,6 +561,21 @@ def layer_norm_residual_canon(x: torch.Tensor, y: Optional[torch.Tensor], weight
     return canon_conv(x, canon, state, meta, out_dtype)
 
 
+def layer_norm_residual_canon_route(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor, eps: float,
+                                    canon: torch.Tensor, state: torch.Tensor, meta: RaggedMeta, out_dtype, router: torch.Tensor, top: int,
+                                    scale: float, mode: str, router_b: Optional[torch.Tensor]):
+    """``layer_norm_residual_canon`` of y, then ``moe_route`` of its rows (one launch in steps in which every sequence brings one
+    token, where row and experts fit) -> (rows, (ids, weights))."""
+    if _gpu(x) and meta.max_len == 1:
+        r = _ext().sm_ln_residual_taps_route(x, y, weight, bias, float(eps), None, None, canon, state, meta.tok_seq, meta.tok_pos,
+                                             meta.seq_slot, out_dtype == torch.float32, router, int(top), float(scale), MOE_MODES[mode],
+                                             router_b)
+        if r is not None:
+            return r[0], (r[1], r[2])
+    h = layer_norm_residual_canon(x, y, weight, bias, eps, None, None, canon, state, meta, out_dtype)
+    return h, moe_route(h, router, top, scale, mode, router_b)
+
+
 def layer_norm_residual_norm(x: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, bias: torch.Tensor, eps: float,
                              parts: Optional[torch.Tensor], part_w: Optional[torch.Tensor], next_weight: torch.Tensor,
                              next_bias: torch.Tensor, next_eps: float, out_dtype) -> torch.Tensor:
@@ -1014,6 +1029,9 @@ def moe_route_grouped(h: torch.Tensor, router: torch.Tensor, top: int, scale: fl
     return idx.int(), w / (w.sum(-1, keepdim=True) + 1e-20) * scale, torch.sigmoid(z[:, E]) if gate else None
 
 
+MOE_MODES = {"softmax": 0, "sigmoid": 1, "top_softmax": 2}
+
+
 def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, scale: float, mode: str = "softmax",
               bias: Optional[torch.Tensor] = None):
     """Router in fp32 over h [T, W] (router fp32 [E, W], logits W_r h + ``bias`` fp32 [E]).  ``mode``
@@ -1022,8 +1040,7 @@ def moe_route(h: torch.Tensor, router: torch.Tensor, top: int, scale: float, mod
     "top_softmax": the ``top`` largest logits, softmax over those alone, times ``scale``.  Returns
     (expert ids int32 [T, top], weights fp32 [T, top]), largest first (the lower id on a tie)."""
     if _gpu(h):
-        return _ext().sm_moe_route(h, router, int(top), float(scale), {"softmax": 0, "sigmoid": 1, "top_softmax": 2}[mode],
-                                   bias)
+        return _ext().sm_moe_route(h, router, int(top), float(scale), MOE_MODES[mode], bias)
     z = h.float() @ router.float().t()
     if bias is not None:
         z = z + bias.float()
