@@ -354,7 +354,7 @@ __global__ void __launch_bounds__(FA_NT, 1) fa_kernel(
     h = (Hq & 7) == 0 ? (hr & 7) * (Hq >> 3) + (hr >> 3) : hr;
   }
   const int kvh = h / (Hq / Hkv);
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;   // (as a scalar it costs the registers that keep this from spilling)
   const int ql = lane & 31, hf = lane >> 5;                    // query column / half of the wave
   const int s0 = start_pos[b];
   const int nkeys = s0 + T;
