@@ -269,7 +269,7 @@ STEP_OPS = ["embedding_scaled", "scalar_rms_norm", "relu2", "cat_cast", "combine
             "latent_expand_write", "head_expand_gate", "gated_linear_attention", "decay_linear_attention", "softcap",
             "parallel_step_in", "combine_residual_norm", "layer_norm_residual_canon", "layer_norm_residual_norm",
             "group_norm_residual_norm", "delta_step", "latent_attention", "moe_experts_glu_shared",
-            "attention_beside_scan", "layer_norm_residual_canon_route"]
+            "attention_beside_scan", "layer_norm_residual_canon_route", "rms_norm_linear"]
 
 
 def op_times(eng: RaggedEngine, entries, close=()) -> Dict[str, float]:

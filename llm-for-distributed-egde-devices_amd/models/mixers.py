@@ -203,8 +203,7 @@ class LatentAttention(nn.Module):
         s = self.spec
         T, H = h.shape[0], s.heads
         u = self.proj_in(h)
-        cq = seqmix.rms_norm_cols(u, 0, s.q_rank, self.q_norm, self.eps, h.dtype)
-        q = self.uq(cq).view(T, H, s.dim + s.rot_dim)
+        q = seqmix.rms_norm_linear(u, self.q_norm, self.eps, self.uq).view(T, H, s.dim + s.rot_dim)
         rope = _shared_rope(self._rope, (s.rot_dims, s.rot_base, s.rot_scaling), meta.max_keys, h.device)
         qc = seqmix.latent_expand_write(u if self.own_kv else None, s.q_rank, self.kv_norm, self.eps, q, self.uk, meta, rope, run.lat,
                                         s.kv_rank, s.rot_dims)

@@ -116,6 +116,7 @@ int edge_sm_ln_residual(float* x, const void* y, const void* parts, const float*
                         int rows, int W, float eps, int f32, hipStream_t st);
 int edge_sm_rms_cols(const void* u, int ld, int c0, int C, const float* w, void* y, int rows, float eps, int f32,
                      hipStream_t st);
+int edge_sm_rms_gemv(const void* u, int ld, const float* g, const void* W, void* out, int M, int N, int K, float eps, hipStream_t st);
 int edge_sm_head_norm_gate(const float* y, const void* z, int z_ld, const float* w, void* out, int rows, int H, int P,
                            float eps, int silu, int f32, hipStream_t st);
 int edge_sm_glu_clamp(const void* u, int ld, void* y, int rows, int ff, float limit, int f32, hipStream_t st);
@@ -935,6 +936,23 @@ std::optional<at::Tensor> sm_combine_norm(at::Tensor& x, const at::Tensor& l, co
                                       out.data_ptr(), (int)x.size(0), (int)x.size(1), f32(l), stream());
   if (rc == -2) return std::nullopt;
   check(rc, "sm_combine_norm");
+  return out;
+}
+
+// sm_rms_cols of the first columns of bf16 rows, then their product with the fragment-packed W [N, K]; nothing where it is not one launch
+std::optional<at::Tensor> sm_rms_gemv(const at::Tensor& u, const at::Tensor& g, double eps, const at::Tensor& W, int64_t N) {
+  const int ld = row_ld(u, "u");
+  chk_f32(g, "weight");
+  const int64_t K = g.numel();
+  TORCH_CHECK(K > 0 && K <= u.size(1), "weight: fp32 [K], columns of u");
+  if (u.scalar_type() != at::kBFloat16 || W.scalar_type() != at::kBFloat16) return std::nullopt;
+  TORCH_CHECK(W.is_cuda() && W.is_contiguous() && W.device() == u.device() && W.numel() == N * K, "W: packed [N, K]");
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(u.device());
+  auto out = at::empty({u.size(0), N}, u.options());
+  const int rc = edge_sm_rms_gemv(u.data_ptr(), ld, g.data_ptr<float>(), W.data_ptr(), out.data_ptr(), (int)u.size(0), (int)N, (int)K,
+                                  (float)eps, stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_rms_gemv");
   return out;
 }
 
@@ -1787,6 +1805,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_layer_norm", &sm_layer_norm);
   m.def("sm_ln_residual", &sm_ln_residual);
   m.def("sm_rms_cols", &sm_rms_cols);
+  m.def("sm_rms_gemv", &sm_rms_gemv);
   m.def("sm_head_norm_gate", &sm_head_norm_gate);
   m.def("sm_glu_clamp", &sm_glu_clamp);
   m.def("sm_latent_write", &sm_latent_write);

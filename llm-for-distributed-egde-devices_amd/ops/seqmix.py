@@ -640,6 +640,22 @@ def rms_norm_cols(u: torch.Tensor, c0: int, C: int, weight: torch.Tensor, eps: f
     return (v * torch.rsqrt(v.pow(2).mean(-1, keepdim=True) + eps) * weight.float()).to(out_dtype)
 
 
+RMS_GEMV_ROWS, RMS_GEMV_K = 16, 512
+
+
+def rms_norm_linear(u: torch.Tensor, weight: torch.Tensor, eps: float, lin) -> torch.Tensor:
+    """``lin`` of ``rms_norm_cols`` of u's first columns, in u's dtype: one launch for a plain bf16 projection of few rows."""
+    C = weight.shape[0]
+    if _gpu(u) and u.dtype == torch.bfloat16 and 0 < u.shape[0] <= RMS_GEMV_ROWS and C <= RMS_GEMV_K and C % 64 == 0:
+        from ..models.layers import plain_linear
+        from . import raw_call
+        if plain_linear(lin) and lin.weight.dtype == u.dtype and lin.out_features % 16 == 0 and raw_call(u, weight, lin.weight):
+            q = _ext().sm_rms_gemv(u, weight, float(eps), lin.packed_weight(), lin.out_features)
+            if q is not None:
+                return q
+    return lin(rms_norm_cols(u, 0, C, weight, eps, u.dtype))
+
+
 def glu_clamp(u: torch.Tensor, ff: int, limit: float) -> torch.Tensor:
     """u [T, gate | up] -> g sigmoid(1.702 g) (up + 1) with g = min(gate, limit), up clamped to
     +-limit (fp32 math, stored in u's dtype)."""
