@@ -324,11 +324,14 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
     __syncthreads();
     {
       // per 16-token block and channel: B = the log decays up to and with each token, E = those after it; half a wave
-      // holds a block's first eight tokens, the other half its last eight
+      // holds a block's first eight tokens, the other half its last eight.  A decay below 2^-160 counts as that: every power over it
+      // is 0 in fp32 either way, and one of -inf (a bias of the type's lowest value) would leave -inf minus -inf between two tokens
+      // behind it
+      constexpr float GONE = -160.f;
       const int nn = tid % NK, seg = tid / NK;
       float a[8], sum = 0.f, back = 0.f;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) { a[i] = B_s[seg * 8 + i][nn]; sum += a[i]; }
+      for (int i = 0; i < 8; ++i) { const float d = B_s[seg * 8 + i][nn]; a[i] = d < GONE ? GONE : d; sum += a[i]; }
       const float other = lane_xor(sum, 32);
       float fwd = seg & 1 ? other : 0.f;
       back = seg & 1 ? 0.f : other;
