@@ -547,11 +547,15 @@ class DecoderLM(nn.Module):
         batch 1: hipBLASLt's small-M kernel ran the 525 MB head at 4.6 TB/s, 113 us per token)."""
         if not ops.bf16_gemv_ok(h, self.embed):
             return torch.nn.functional.linear(h, self.embed)
-        wp, ver = getattr(self, "_embed_wp", None), self.embed._version
-        if wp is None or getattr(self, "_embed_wp_ver", -1) != ver or wp.device != self.embed.device:
-            wp = self._embed_wp = ops.settle(ops.pack_bf16_weight(self.embed.detach()))
-            self._embed_wp_ver = ver
+        wp = ops.kept_layout(self, "_embed_laid", self.embed._version, self.embed.device,
+                             lambda: ops.pack_bf16_weight(self.embed.detach()))
         return ops.linear_bf16(h, self.embed, None, packed=wp)
+
+    @property
+    def _embed_wp(self) -> Optional[torch.Tensor]:
+        """The fragment-packed copy of the embedding, where one is kept."""
+        kept = self.__dict__.get("_embed_laid")
+        return kept and kept[3]
 
     def _b1_engine(self, ctx: AttnCtx):
         """The batch-1 persistent decode engine for this step, or None (not eligible / not batch 1)."""

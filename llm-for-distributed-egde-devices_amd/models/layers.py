@@ -146,11 +146,8 @@ class Linear(nn.Module):
 
     def packed_weight(self) -> torch.Tensor:
         """The fragment-packed decode copy of the weight (``decode_weight`` without a sample input)."""
-        wp, ver = getattr(self, "_wp", None), self.weight._version
-        if wp is None or getattr(self, "_wp_ver", -1) != ver or wp.device != self.weight.device:
-            wp = self._wp = ops.settle(ops.pack_bf16_weight(self.weight.detach()))
-            self._wp_ver = ver
-        return wp
+        w = self.weight
+        return ops.kept_layout(self, "_wp", w._version, w.device, lambda: ops.pack_bf16_weight(w.detach()))   # (in-place edits repack)
 
     def forward_norm(self, x: "PendingNorm", glu: bool = False):
         """The decode GEMV over a PendingNorm (RMSNorm in the prologue); glu: silu(gate) * up."""
@@ -223,11 +220,7 @@ class Linear(nn.Module):
         decode-sized call (before any graph capture) and kept; None when not applicable."""
         if not ops.bf16_decode_mode(x, self.weight, glu=glu, split=bool(self.split_k_out)):
             return None
-        wp, ver = getattr(self, "_wp", None), self.weight._version   # in-place weight edits repack
-        if wp is None or getattr(self, "_wp_ver", -1) != ver or wp.device != self.weight.device:
-            wp = self._wp = ops.settle(ops.pack_bf16_weight(self.weight.detach()))
-            self._wp_ver = ver
-        return wp
+        return self.packed_weight()
 
     def extra_repr(self):
         return f"{self.in_features}->{self.out_features}, bias={self.bias is not None}, {str(self.weight.dtype)[6:]}"

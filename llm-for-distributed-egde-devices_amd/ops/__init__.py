@@ -460,12 +460,54 @@ def pack_bf16_weight(w: torch.Tensor) -> torch.Tensor:
     return w.reshape(N // 16, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().view(-1)
 
 
-def settle(t: torch.Tensor) -> torch.Tensor:
-    """Wait for the kernels that lay out a tensor that is kept (a weight's packed copy): the next call that finds it may run
-    on another stream, where nothing orders it behind them (two pipeline lanes whose first calls fall in one tick)."""
-    if t.is_cuda and not torch.cuda.is_current_stream_capturing():
-        torch.cuda.current_stream(t.device).synchronize()
-    return t
+class Laid:
+    """When a layout that is kept is there: the event behind the kernels that form it, until they are done."""
+
+    def __init__(self, device: Optional[torch.device] = None):
+        self.device = device
+        self.event = torch.cuda.current_stream(device).record_event() if device is not None else None
+
+    def wait(self) -> None:
+        """Order what the current stream runs next behind them."""
+        event = self.event
+        if event is None:
+            return
+        with torch.cuda.device(self.device):
+            # (a graph cannot wait for work outside it, and its replays know nothing of that work: the host waits)
+            if _event_done(event, torch.cuda.is_current_stream_capturing()):
+                self.event = None
+            else:
+                torch.cuda.current_stream().wait_event(event)
+
+    def __reduce__(self):                       # a copy (deepcopy, pickle) is of a finished layout
+        if self.event is not None:
+            _event_done(self.event, True)
+        return Laid, ()
+
+
+def _event_done(event: torch.cuda.Event, wait: bool) -> bool:
+    from . import seqmix
+    return (ext() if available() else seqmix._ext()).event_done(event.cuda_event, wait)
+
+
+def kept_layout(owner, name: str, version, device: torch.device, make):
+    """make()'s tensors (a weight in a kernel's order), formed on the first call of a ``version`` and kept as ``owner``'s
+    attribute ``name``.  The next call that finds them may run on another stream (two pipeline lanes whose first calls fall in
+    one tick), which is ordered behind the kernels that form them; the host waits for nothing.  While a graph is recorded nothing is
+    kept: the tensors are the graph's own, its replays form them anew and nobody else may read them."""
+    kept = owner.__dict__.get(name)
+    if kept is not None and kept[1] == version and kept[2] == device:
+        if kept[0].event is not None:
+            kept[0].wait()
+        return kept[3]
+    made = make()
+    if device.type != "cuda":
+        setattr(owner, name, (Laid(), version, device, made))
+    else:
+        with torch.cuda.device(device):
+            if not torch.cuda.is_current_stream_capturing():
+                setattr(owner, name, (Laid(device), version, device, made))
+    return made
 
 
 _GEMV_EPI = {None: 0, "silu_glu": 1, "gelu_tanh": 2, "gelu": 3}

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "b1_engine.h"
+#include "event_done.h"
 #include <tuple>
 
 extern "C" {
@@ -1613,6 +1614,7 @@ int b1_lds_bytes(int D, int xqb, int sxn, int scb) { return edge_b1_lds_bytes(D,
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("event_done", &event_done, py::call_guard<py::gil_scoped_release>());
   m.def("copy_head_block", &copy_head_block, py::arg("dst"), py::arg("src"), py::arg("mode") = 0);
   m.doc() = "edgellm CDNA4 (gfx950) HIP kernels";
   m.def("b1_decode", &b1_decode);

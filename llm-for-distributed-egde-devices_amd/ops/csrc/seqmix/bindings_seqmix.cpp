@@ -8,6 +8,8 @@
 
 #include <optional>
 
+#include "event_done.h"
+
 extern "C" {
 int edge_sm_embed(const int64_t* ids, const void* table, float* out, int rows, int W, int V, float scale, int f32,
                   hipStream_t st);
@@ -1782,6 +1784,7 @@ at::Tensor sm_softcap(const at::Tensor& z, double cap) {
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  m.def("event_done", &event_done, py::call_guard<py::gil_scoped_release>());
   m.def("sm_embed", &sm_embed);
   m.def("sm_scalar_norm", &sm_scalar_norm);
   m.def("sm_relu2", &sm_relu2);

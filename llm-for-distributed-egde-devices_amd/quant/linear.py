@@ -244,6 +244,7 @@ class LLMInt8Linear(nn.Module):
     #                      (<= 16, one fused kernel, at most 256 columns) and any rows (uncapped)
     DECODE_ROWS = 16
     ONE_LAUNCH = True    # batch 1: ops/csrc/gemm_i8.hip l8_prologue (one launch per projection, K <= 12288)
+    _laid = None         # what the device-side outlier path reads (``_layouts``), formed on first use
 
     def pending_norm_ok(self, glu: bool = False):
         """Batch 1 on GPU: this projection takes the RMSNorm of a bf16 row x + residual in its one-launch
@@ -274,7 +275,6 @@ class LLMInt8Linear(nn.Module):
         self.register_buffer("w_packed", torch.zeros(nt * kt * 1024, dtype=torch.int8, device=device))
         self.register_buffer("SCB", torch.ones(out_features, dtype=torch.float32, device=device))
         self.register_buffer("bias", torch.zeros(out_features, dtype=dtype, device=device) if bias else None)
-        self._weight_t = None          # int8 W^T for the device-side outlier path (built on first use)
 
     @classmethod
     @torch.no_grad()
@@ -289,11 +289,11 @@ class LLMInt8Linear(nn.Module):
 
     @torch.no_grad()
     def _load_from_state_dict(self, *args, **kwargs):
-        self._weight_t = None          # derived device copies follow the loaded weights
+        self._laid = None              # derived device copies follow the loaded weights
         super()._load_from_state_dict(*args, **kwargs)
 
     def load_int8(self, q, scb, bias=None):
-        self._weight_t = None
+        self._laid = None
         self.weight_i8.copy_(q)
         self.w_packed.copy_(ops.pack_int8_weight(q))
         self.SCB.copy_(scb.float())
@@ -332,13 +332,29 @@ class LLMInt8Linear(nn.Module):
 
     def pair_args(self):
         """Operands of a one-row launch: threshold, packed weight, scales, bias, W^T, SCB."""
-        self._transposed(self.w_packed.device)
-        return self.threshold, self.w_packed, self._w_deq, self.bias, self._weight_t, self.SCB
+        w_deq, weight_t = self._layouts()
+        return self.threshold, self.w_packed, w_deq, self.bias, weight_t, self.SCB
 
-    def _transposed(self, device):
-        if self._weight_t is None or self._weight_t.device != device:
-            self._w_deq = self.SCB / 127.0
-            self._weight_t = ops.settle(self.weight_i8.t().contiguous())   # W^T: outlier columns as rows
+    def _layouts(self):
+        """(scales of the int8 product, int8 W^T: outlier columns as rows), kept."""
+        w = self.weight_i8
+        return ops.kept_layout(self, "_laid", 0, w.device, lambda: (self.SCB / 127.0, w.t().contiguous()))
+
+    def _transposed(self, device) -> None:
+        self._layouts()
+
+    @property
+    def _w_deq(self) -> Optional[torch.Tensor]:
+        return self._laid and self._laid[3][0]
+
+    @property
+    def _weight_t(self) -> Optional[torch.Tensor]:
+        return self._laid and self._laid[3][1]
+
+    @_weight_t.setter
+    def _weight_t(self, none) -> None:                       # (None: both are formed again)
+        assert none is None
+        self._laid = None
 
     def _forward(self, x, glu: bool = False, act: int = 0, add: Optional[torch.Tensor] = None):
         if isinstance(x, PendingLN):
@@ -347,10 +363,10 @@ class LLMInt8Linear(nn.Module):
             if (x.x.shape[0] == 1 and x.x.is_cuda and ops.gpu_path(x.x) and x.x.dtype == torch.bfloat16
                     and self._device_ok() and self.ONE_LAUNCH and K <= 4096):
                 C = ops.ext()
-                self._transposed(x.x.device)
+                w_deq, weight_t = self._layouts()
                 y = C.llmint8_gemv_norm(x.x.contiguous(), x.residual.contiguous() if x.residual is not None else None,
                                         x.weight, x.bias, x.eps, not x.rms, x.h, x.y, self.threshold, self.w_packed,
-                                        self._w_deq, self.bias, self._weight_t, self.SCB, N, glu, act, x.x2, x.y_weight, x.y_bias)
+                                        w_deq, self.bias, weight_t, self.SCB, N, glu, act, x.x2, x.y_weight, x.y_bias)
             if y is not None or glu or act:
                 return y if add is None else y + add.view_as(y)
             x = x.materialize()
@@ -363,12 +379,12 @@ class LLMInt8Linear(nn.Module):
         if x2.is_cuda and ops.gpu_path(x2) and x2.dtype == torch.bfloat16 and self._device_ok():
             # outlier columns found on the device (llmint8.hip), no host sync at any row count
             C = ops.ext()
-            self._transposed(x2.device)
+            w_deq, weight_t = self._layouts()
             x2 = x2.contiguous()
             if x2.shape[0] == 1 and K <= 12288 and K % 64 == 0 and self.ONE_LAUNCH:
                 # batch 1: outlier discovery, quantisation and the outlier part inside the GEMV
                 fuse = add is not None and not act and _epilogue_row(add, x2)
-                out = C.llmint8_gemv(x2, self.threshold, self.w_packed, self._w_deq, self.bias, self._weight_t,
+                out = C.llmint8_gemv(x2, self.threshold, self.w_packed, w_deq, self.bias, weight_t,
                                      self.SCB, N, act, add if fuse else None)
                 if out is not None:
                     return out.view(*shp, N) if fuse else plus(out.view(*shp, N))
@@ -376,12 +392,12 @@ class LLMInt8Linear(nn.Module):
                     return None
             if x2.shape[0] <= self.DECODE_ROWS:
                 q, sa, cols, xo, count = C.llmint8_prep(x2, self.threshold, self.OUTLIER_CAP)
-                out = ops.w8a8_linear(q, sa, self.w_packed, self._w_deq, self.bias, N, K)
-                C.llmint8_outlier(out, xo, cols, count, self._weight_t, self.SCB)
+                out = ops.w8a8_linear(q, sa, self.w_packed, w_deq, self.bias, N, K)
+                C.llmint8_outlier(out, xo, cols, count, weight_t, self.SCB)
             else:
                 q, sa, cols, count = C.llmint8_prep_rows(x2, self.threshold)
-                out = ops.w8a8_linear(q, sa, self.w_packed, self._w_deq, self.bias, N, K)
-                C.llmint8_outlier_rows(out, x2, cols, count, self._weight_t, self.SCB)
+                out = ops.w8a8_linear(q, sa, self.w_packed, w_deq, self.bias, N, K)
+                C.llmint8_outlier_rows(out, x2, cols, count, weight_t, self.SCB)
             return plus(out.view(*shp, N))
         cols = (x2.abs() > self.threshold).any(0).nonzero().flatten()
         w_scale = self.SCB / 127.0
