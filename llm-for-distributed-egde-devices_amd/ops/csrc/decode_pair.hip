@@ -21,9 +21,12 @@ struct Proj {
 
 constexpr int OW = GEMV_NW;                // waves of an o or down workgroup
 
-// One workgroup of a projection.  8 waves: as many k-pairs in flight per wave as divide its rounds evenly (8, 5 or 4: a round
-// that runs over the end loads its last k-pair again), else 2.  16 waves: 5 where that divides the rounds, else 1 (more would
-// take the registers of the CU's second workgroup: 2048 x 8192 beside 2048 x 2048 9.3 us, with 8 in flight 11.4).
+// One workgroup of a projection, a round's loads ahead of its products.  8 waves: 5 or 4 k-pairs of a wave a round where they divide its
+// rounds evenly (a round that runs over the end loads its last k-pair again), else 2.  Eight pairs of weights and rows are 128
+// registers by themselves: under the bound of two workgroups a CU they spill, us with 8 / 4: attention beside 16384 x 4096, 1 row
+// 32.4 / 25.5, 4 rows 36.9 / 26.2; rows3 1024 x 4096 and twice 1024 x 1024, 1 row 6.3 / 5.5, 2048 x 8192 and twice 2048 x 2048 12.5 / 11.6.
+// 16 waves: 5 where that divides the rounds, else 1 (more would take the registers of the CU's second workgroup: 2048 x 8192 beside
+// 2048 x 2048 9.3 us, with 8 in flight 11.4).
 template <int NWV, int EPI, bool HF>
 __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act) {
   const int KP = p.K / 64;
@@ -33,8 +36,7 @@ __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act
     if (KP % (5 * NWV) == 0) RUN(5, 0);
     else RUN(1, 1);
   } else {
-    if (KP % (8 * NWV) == 0) RUN(8, 0);
-    else if (KP % (5 * NWV) == 0) RUN(5, 0);
+    if (KP % (5 * NWV) == 0) RUN(5, 0);
     else if (KP % (4 * NWV) == 0) RUN(4, 0);
     else RUN(2, 0);
   }

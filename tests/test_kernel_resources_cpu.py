@@ -26,3 +26,19 @@ def test_counted_vmcnt_kernels_do_not_spill():
     spills = {f"{f}:{k}": v.get("ScratchSize", 0) for f, rep in reports.items() for k, v in rep.items()
               if v.get("ScratchSize", 0) > 0}
     assert not spills, spills
+
+
+# Kernels that ask for a round's loads in front of a fence, so that a round needs its registers at once: a spill there is a memory
+# round trip in every round (eight k-pairs under 128 registers: attention beside 16384 x 4096, 4 rows, 36.9 us, four 26.2)
+FENCED_FILES = ["decode_pair.hip", "decode_pair_i8.hip", "gemv_bf16.hip", "gemv_f32.hip", "gemv_i8_rows.hip", "seqmix/rms_gemv.hip"]
+
+
+@pytest.mark.skipif(shutil.which("/opt/rocm/bin/hipcc") is None, reason="no hipcc")
+def test_fenced_rounds_do_not_spill():
+    sys.path.insert(0, os.path.join(ROOT, "tools"))
+    from kernel_resources import resources
+    with ThreadPoolExecutor(len(FENCED_FILES)) as ex:
+        reports = dict(zip(FENCED_FILES, ex.map(lambda f: resources(os.path.join(CSRC, f)), FENCED_FILES)))
+    assert all(reports.values()), "no kernel resource remarks (compile failed?)"
+    spills = {f"{f}:{k}": v["ScratchSize"] for f, rep in reports.items() for k, v in rep.items() if v["ScratchSize"] > 0}
+    assert not spills, spills
