@@ -38,6 +38,7 @@ int edge_attn_up(const void* qkv, int64_t q_sb, void* kc, void* vc, int64_t c_sb
 int edge_o_down(const void* x, const void* wo, const void* bo, void* a, int Ko, const void* h, const void* wd,
                 const void* bd, void* y, int Kd, int M, int N, int h16, hipStream_t st);
 int edge_w8a8_gemv_norm_on();
+int edge_w8a8_rows_splits(int M, int N, int K, int S);
 int edge_w8a8_gemm_splitk(const void* A, const float* sa, const void* Wp, const float* sw, const void* bias,
                           float* part, int M, int N, int K, int KT, int a_mode, int Mpad, int S, hipStream_t st);
 int edge_act(const void* x, void* y, void* yq, float* ys, int rows, int F, int mode, int quant, int h16,
@@ -777,12 +778,7 @@ at::Tensor w8a8_gemm_splitk(const at::Tensor& a, const at::Tensor& sa, const at:
   if (M > 128) S = edge_w8a8_rows256_splits((int)K);     // 129-256 rows: fixed per K (gemm_i8.hip rows256)
   TORCH_CHECK(M <= 128 || S > 1, "no 129-256-row split-K kernel for this K");
   if (S <= 0 && M > 64) S = 4;                           // 65-128 rows: 4 slices (gemm_i8.hip rows128)
-  if (S <= 0 && M <= 16 && mpad > 0 && N % 16 == 0) {
-    // one tile a workgroup (gemv_i8_rows.hip): two workgroups a CU, each wave a k-tile or more; us at S = 1 / 2 / 4: 4096 x 4096 5.3 / 4.7 /
-    // 7.4, 4096 x 11008 10.0 / 8.8 / 9.9, 2048 x 2048 3.4 / 3.4 / 4.1, 2048 x 8192 7.4 / 5.3 / 4.7
-    const int64_t tiles = N / 16;
-    S = std::max<int64_t>(1, std::min<int64_t>({4, (512 + tiles / 2) / tiles, KT / 16}));
-  }
+  if (S <= 0 && M <= 16 && mpad > 0) S = edge_w8a8_rows_splits((int)M, (int)N, (int)K, 0);   // one tile a workgroup
   if (S <= 0) {
     const int64_t ntw = M <= 16 ? 2 : 4;                 // tiles per workgroup (gemm_i8.hip launcher)
     const int64_t groups = ((N + 15) / 16 + ntw - 1) / ntw;

@@ -7,9 +7,10 @@ from edgellm import ops
 pytestmark = pytest.mark.gpu
 
 
-# fewer k-tiles than waves, ragged rounds and parts, one tile, many tiles
+# fewer k-tiles than waves, ragged rounds and parts, one tile, many tiles, more than 16 MB whose 5 to 16 rows keep two tiles a workgroup
+# (4096 x 11008) or take one (5120 x 4160)
 @pytest.mark.parametrize("M", [1, 3, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize("N,K,S", [(16, 64, 0), (48, 1088, 3), (2064, 2560, 0), (4096, 11008, 2), (1024, 192, 3)])
+@pytest.mark.parametrize("N,K,S", [(16, 64, 0), (48, 1088, 3), (2064, 2560, 0), (4096, 11008, 2), (1024, 192, 3), (5120, 4160, 0)])
 def test_slices_sum_to_the_product(cuda, M, N, K, S):
     g = torch.Generator(device=cuda).manual_seed(M * 1009 + N + K)
     ints = lambda *s: torch.randint(-127, 128, s, generator=g, device=cuda, dtype=torch.int8)  # noqa: E731
