@@ -12,8 +12,10 @@
 // One head of fp32 rows takes its scores on the vector ALU: 16 products a lane and two exchanges instead of 16 matrix instructions of
 // which 15 rows in 16 are idle, and half their error (4e-7 -> 2.7e-7 of the result, against 64 bits).  us, a launch in a graph, before /
 // after: 16 heads of 64 in 4 groups, 2 tokens behind 777 (window 512, 16 blocks) 9.2 / 8.2, 8 behind 400 8.6 / 7.8; of 128, 1 behind 700 15.5 /
-// 14.6.  What is left there is the bytes of one CU: four times the keys in flight, the next rows ahead, other workgroups fetching them
-// into the L2 and 64 keys a wave at a time all gave nothing.
+// 14.6.  What is left there is the bytes of one CU: four times the keys in flight, the next rows ahead and 64 keys a wave at a time gave
+// nothing, other workgroups that fetch them into the L2 something where CUs are idle (attn_ssd_kernel).
+// Rows of up to 64 numbers are held to 128 registers a lane, two workgroups to a CU: four fp32 heads with blocks need one more
+// otherwise (us, 32 heads in 2 groups, 64 rows, window 512, 16 blocks, behind 800 27.4 / 22.8, 64 heads in 8, 32 rows behind 1600 30.3 / 24.6).
 // us, attn_kernel with its sum over key splits / this (bf16 but for the first): fp32, 16 heads of 64 in 4 groups, 2 tokens behind
 // 777 (window 512, 16 blocks) 15.3 / 9.9; latent rows of 160, 16 heads, 4 tokens behind 97 19.4 / 5.2; of 320, 6 behind 1100 (window 1024)
 // 35.1 / 27.0, 1 behind 7600 56 / 21; 16 heads of 128 in 4 groups, 6 in chunks of 1000 20.7 / 13.3.
@@ -118,14 +120,15 @@ __device__ __forceinline__ void attn_step_body(const StepArgs& a, int block) {
   const int* pt = a.ptab + (size_t)a.seq_slot[a.tok_seq[t]] * a.ptab_ld;
   // the queries as the matrix cores' rows: row = lane & 15 is head row % SH; numbers past D (or heads past R) are zero
   const T* qp = reinterpret_cast<const T*>(a.q) + ((size_t)t * a.H + hq0 + min(key % SH, R - 1)) * D;
-  constexpr bool F32 = sizeof(T) == 4, DOT = F32 && SH == 1;
+  // (the widest rows of four fp32 heads have no registers for either: 128 bytes a lane spilled, 40 without)
+  constexpr bool ROOM = SH == 1 || sizeof(T) == 2 || NC <= 4, F32 = sizeof(T) == 4 && ROOM, DOT = F32 && SH == 1;
   uint4 qr[NC][Tile<T, NC, DVL>::Q];
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
     for (int e = 0; e < Tile<T, NC, DVL>::Q; ++e)
-      qr[c][e] = *reinterpret_cast<const uint4*>(F32 ? qp + min(32 * c + 16 * e + 4 * grp, D - 4) : qp + min(32 * c + 8 * grp, D - 8));
-  asm volatile("" ::: "memory");        // (all on their way before one is looked at)
+      qr[c][e] = *reinterpret_cast<const uint4*>(F32 ? qp + min(32 * c + 16 * e + 4 * grp, D - 4) : qp + min(32 * c + 8 * grp, D - 8) + 4 * e);
+  if constexpr (ROOM) asm volatile("" ::: "memory");        // (all on their way before one is looked at)
 #pragma unroll
   for (int c = 0; c < NC; ++c)
 #pragma unroll
@@ -360,7 +363,7 @@ __device__ __forceinline__ void attn_step_body(const StepArgs& a, int block) {
 }
 
 template <typename T, int NC, int DVL, int SH, bool POOL, bool EX>
-__global__ void __launch_bounds__(STEP_NW * 64) attn_step_kernel(StepArgs a) {
+__global__ void __launch_bounds__(STEP_NW * 64, NC == 2 ? 4 : 2) attn_step_kernel(StepArgs a) {
   attn_step_body<T, NC, DVL, SH, POOL, EX>(a, blockIdx.x);
 }
 
@@ -442,7 +445,7 @@ int run_beside(const StepArgs& a, const SsdStep& s, int N, int P, hipStream_t st
 }
 
 // Estimates in us, fitted to both kernels' times at 936 points (13 shapes of 8 to 64 heads of 32 to 320 numbers, both types, 1 to 400 rows
-// behind 17 to 8000 keys; half of them are within 7 %): a launch, then the longer of one workgroup's chain and the chip's work per CU,
+// behind 17 to 8000 keys; half of them were within 7 %; fp32 rows of one head a workgroup have since become 5 to 11 % quicker): a launch, then the longer of one workgroup's chain and the chip's work per CU,
 // then the sum over key splits.
 constexpr double LAUNCH_US = 4.5, MERGE_US = 4.5;
 

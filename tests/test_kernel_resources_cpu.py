@@ -42,3 +42,22 @@ def test_fenced_rounds_do_not_spill():
     assert all(reports.values()), "no kernel resource remarks (compile failed?)"
     spills = {f"{f}:{k}": v["ScratchSize"] for f, rep in reports.items() for k, v in rep.items() if v["ScratchSize"] > 0}
     assert not spills, spills
+
+
+# Workgroups that a launch counts on fitting a CU twice: waves of a SIMD
+TWICE = [("gemv_i8_rows.hip", r"w8a8_rows_kernel", 8),
+         ("seqmix/attn_step.hip", r"attn_step_kernelI[ft]Li2ELi1E", 4)]     # rows of up to 64 numbers, 8 waves
+
+
+@pytest.mark.skipif(shutil.which("/opt/rocm/bin/hipcc") is None, reason="no hipcc")
+def test_two_workgroups_fit():
+    import re
+    sys.path.insert(0, os.path.join(ROOT, "tools"))
+    from kernel_resources import resources
+    with ThreadPoolExecutor(len(TWICE)) as ex:
+        reports = list(ex.map(lambda t: resources(os.path.join(CSRC, t[0])), TWICE))
+    for (f, pattern, waves), rep in zip(TWICE, reports):
+        hit = {k: v for k, v in rep.items() if re.search(pattern, k)}
+        assert hit, (f, pattern)
+        few = {k: v["Occupancy"] for k, v in hit.items() if v["Occupancy"] < waves or v["ScratchSize"] > 0}
+        assert not few, few
