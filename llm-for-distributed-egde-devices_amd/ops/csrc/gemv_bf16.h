@@ -4,7 +4,8 @@
 
 namespace {
 constexpr int EPI_OUT = 0, EPI_GLU = 1, EPI_GELU_TANH = 2, EPI_GELU = 3, EPI_PART = 4,
-              EPI_GELU_ANY = 5;               // gelu, tanh where F is 1, else erf
+              EPI_GELU_ANY = 5,               // gelu, tanh where F is 1, else erf
+              EPI_ADD = 6;                    // EPI_OUT and an addend
 constexpr int GEMV_NW = 16;
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -260,7 +261,7 @@ __device__ __forceinline__ void norm16_prologue(const NormIn16& na, bool wg0, in
 // What bounds it is the chain of memory round trips, so every load of a step is issued before any use (the fence: left
 // alone, the compiler moves loads behind the products and under the guards of ragged ends, two to four round trips a wave
 // instead of one), the next tile's first PRE k-pairs are requested before this one's sums meet, a wave holds one tile's
-// numbers only, so that two workgroups fit a CU, and the instructions behind the last load are few.
+// numbers only, so that two workgroups fit a CU (gemv_bf16.hip: without a norm), and the instructions behind the last load are few.
 // RB: groups of four rows (M <= 4 RB): a tile's rows are one number quadruple of 16 RB lanes, and the 64 lanes of one wave
 // each add up NWV RB / 4 waves' sums.
 // GLU: a tile is 8 gate columns and their 8 up columns (halves of two weight tiles, whole 128-byte lines of both).
@@ -316,14 +317,13 @@ __device__ __forceinline__ void gemv_tiles_body(int bid, int nwg, const bf16_t* 
     const int row0 = RB == 1 ? 0 : 4 * (lane >> 4), c = EPI == EPI_GLU ? 8 * tile + (r & 7) : 16 * tile + r;
     v4f acc = {0.f, 0.f, 0.f, 0.f};
     // what the writing wave adds to its sums is requested with its first weights
-    float bv = 0.f, addv[4] = {0.f, 0.f, 0.f, 0.f};
+    float bv = 0.f;
+    bf16_t addv[4] = {0, 0, 0, 0};                          // (as they are: a conversion here would wait for them here)
     if (wave == 0) {
       if (bias != nullptr && (EPI != EPI_PART || ks == 0)) bv = e2f<HF>(bias[EPI == EPI_GLU && r >= 8 ? F + c : c]);
-      if constexpr (EPI == EPI_OUT) {
-        if (add != nullptr) {
+      if constexpr (EPI == EPI_ADD) {
 #pragma unroll
-          for (int q = 0; q < 4; ++q) addv[q] = e2f<HF>(add[(size_t)min(row0 + q, M - 1) * N + c]);
-        }
+        for (int q = 0; q < 4; ++q) addv[q] = add[(size_t)min(row0 + q, M - 1) * N + c];
       }
     }
     if constexpr (PRE > 0) {
@@ -370,7 +370,8 @@ __device__ __forceinline__ void gemv_tiles_body(int bid, int nwg, const bf16_t* 
     __syncthreads();
     if (wave == 0) {
       v4f s = red[buf][lane / RL][lane & (RL - 1)];
-#pragma unroll
+      // (16 rows: five reads at a time; all 15 at once are 60 registers, the second workgroup's)
+#pragma unroll(RB == 4 ? 5 : NWV / WG)
       for (int w = 1; w < NWV / WG; ++w) s += red[buf][WG * w + lane / RL][lane & (RL - 1)];
       if constexpr (RB == 1) {
 #pragma unroll
@@ -400,9 +401,9 @@ __device__ __forceinline__ void gemv_tiles_body(int bid, int nwg, const bf16_t* 
               if (EPI == EPI_GELU_TANH || (EPI == EPI_GELU_ANY && F == 1))
                 v = 0.5f * x * (1.f + tanhf(k0 * (x + k1 * x * x * x)));
               else v = 0.5f * x * (1.f + erff(x * 0.7071067811865476f));
-            } else {
-              // an addend (parallel-residual block): rnd(rnd(y) + add), the unfused add
-              if (add != nullptr) v = e2f<HF>(f2e<HF>(v)) + addv[q];
+            } else if constexpr (EPI == EPI_ADD) {
+              // (parallel-residual block): rnd(rnd(y) + add), the unfused add
+              v = e2f<HF>(f2e<HF>(v)) + e2f<HF>(addv[q]);
             }
             if (row < M) out[(size_t)row * N + c] = f2e<HF>(v);
           }

@@ -48,8 +48,8 @@ int launch_mb(const void* A, const void* W, const void* bias, void* out, int M, 
   return (int)hipGetLastError();
 }
 
-template <int PRE, int EPI, bool HF, int NRM, int RB>
-__global__ void __launch_bounds__(GEMV_NW * 64) gemv_tiles_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+template <int PRE, int EPI, bool HF, int NRM, int RB, int TWICE>
+__global__ void __launch_bounds__(GEMV_NW * 64, TWICE ? 8 : 4) gemv_tiles_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                                  const bf16_t* __restrict__ bias, bf16_t* __restrict__ out,
                                                                  int M, int N, int K, int F, int S,
                                                                  const bf16_t* __restrict__ add, NormIn16 na) {
@@ -59,13 +59,22 @@ __global__ void __launch_bounds__(GEMV_NW * 64) gemv_tiles_kernel(const bf16_t* 
 // Workgroups of the tiles form.  Without a norm up to 1024, two to a CU and two rounds of them: 128256 x 2048 takes 82 us on
 // 256, 77 on 512, 75.8 on 1024, 75.6 on 2048.  With a norm one to a CU (the norm's loads and sums are each workgroup's own):
 // 22016 x 4096 29.4 us on 256, 29.6 on 512, 30.9 on 1024; 6144 x 4096 (384 tiles) 10.1 on 256, 11.5 on 384.
+// Two to a CU are 64 registers a lane, which the forms without a norm are held to (at 66 to 106, one to a CU: 8192 x 2048, 16 rows,
+// GELU 10.9 us, now 9.6; 6144 x 4096 16.6, 15.3).  Not with an addend of up to 256 tiles: its loads then wait for each other, and one
+// workgroup a CU is all there is (2560 x 10240 at 8 rows 13.5 us, held to 64 15.8; 8192 x 2048, 512 tiles, at 8 rows 9.5 / 8.3).
 template <int EPI, bool HF, int NRM, int RB>
 int launch_tiles(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, hipStream_t st, int S = 1,
                  const void* add = nullptr, const NormIn16& na = NormIn16{}) {
   const int tiles = N / 16 * S, cap = NRM > 0 ? 256 : 1024;
-  hipLaunchKernelGGL((gemv_tiles_kernel<(NRM > 0 ? 2 : 1), EPI, HF, NRM, RB>), dim3(EPI == EPI_PART || tiles < cap ? tiles : cap),
-                     dim3(GEMV_NW * 64), 0, st, (const bf16_t*)A, (const bf16_t*)W, (const bf16_t*)bias, (bf16_t*)out, M, N, K,
-                     EPI == EPI_GLU ? N / 2 : 0, S, (const bf16_t*)add, na);
+  const dim3 grid(EPI == EPI_PART || tiles < cap ? tiles : cap);
+#define TILES(TW)                                                                                                              \
+  hipLaunchKernelGGL((gemv_tiles_kernel<(NRM > 0 ? 2 : 1), EPI, HF, NRM, RB, TW>), grid, dim3(GEMV_NW * 64), 0, st, (const bf16_t*)A, \
+                     (const bf16_t*)W, (const bf16_t*)bias, (bf16_t*)out, M, N, K, EPI == EPI_GLU ? N / 2 : 0, S, (const bf16_t*)add, na)
+  if constexpr (EPI == EPI_ADD && RB > 1) {
+    if (tiles <= 256) TILES(0);
+    else TILES(1);
+  } else TILES(NRM == 0);
+#undef TILES
   return (int)hipGetLastError();
 }
 
@@ -78,21 +87,30 @@ int launch_tiles_rows(const void* A, const void* W, const void* bias, void* out,
 }
 
 // Whether the tiles form takes M rows: up to 4 always, 5 to 16 where its tiles' reads of the rows (each tile reads all of
-// them) stay small beside the weights.  us, tiles form / several tiles a workgroup: 1 row 1024 x 1024 2.7 / 3.3, 4096 x 2048 (4 rows)
-// 4.7 / 5.4, 32000 x 1024 11.8 / 12.7; 12 rows 4096 x 2048 5.3 / 6.0, 16 rows 8224 x 2048 10.5 / 12.0, 32000 x 2048 27 / 23.5;
-// SwiGLU 16384 x 2048 1 row 11.7 / 13.0, 8 rows 13.8 / 13.3.
-bool tiles_form(int M, int N, int epi) { return M <= 4 || (M <= 16 && epi != EPI_GLU && N < 16384); }
+// them) stay small beside the weights.  us, several tiles a workgroup / tiles form: 1 row 1024 x 1024 3.4 / 2.7, 4096 x 2048 (4 rows)
+// 5.4 / 4.7, 32000 x 1024 12.7 / 11.8; 12 rows 4096 x 2048 6.1 / 5.4, 12288 x 4096 22.4 / 19.5, 16 rows 8192 x 2048 9.2 / 9.2, 32000 x 2048
+// 23.5 / 27; SwiGLU 16384 x 2048 1 row 13.0 / 11.7, 8 rows 13.3 / 13.8.  Where two tiles a workgroup (N from 8192 on) take as many rounds of
+// the CUs and all their k-pairs in whole fours, their halved reads win from some 10 rows on: 8192 x 4096, 9 / 12 / 16 rows, 14.3 / 13.6 /
+// 14.1 against 13.7 / 13.9 / 15.5, 14336 x 8192 43.0 / 43.6 / 44.0 against 43.0 / 46 / 51.
+bool tiles_form(int M, int N, int K, int epi) {
+  if (M <= 4) return true;
+  if (M > 16 || epi == EPI_GLU || N >= 16384) return false;
+  const int nt = N / 16;
+  return M <= 10 || nt < 512 || K % 4096 != 0 || (nt + 255) / 256 < 2 * ((nt + 511) / 512);
+}
 
-// NTW / U chosen for one row block; more row blocks keep U = 2 (registers) and at most 8 / MB
-// tiles (the LDS reduction holds MB x NTW tiles of 16 waves)
+// NTW / U chosen for one row block (NTW = 1 has none: the tiles form takes those); more row blocks keep U = 2 (registers) and at
+// most 8 / MB tiles (the LDS reduction holds MB x NTW tiles of 16 waves)
 template <int NTW, int U, int EPI, bool HF>
 int launch(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int F, int tiles,
            hipStream_t st, int S = 1, const void* add = nullptr) {
   constexpr int G = EPI == EPI_GLU ? 2 : 1;                 // GLU keeps gate / up pairs
   constexpr int N2 = NTW > 4 ? 4 : (NTW < G ? G : NTW), N34 = NTW > 2 ? 2 : (NTW < G ? G : NTW);
   const int mb = (M + 15) / 16;
-  if (mb <= 1) return launch_mb<1, NTW, U, EPI, HF>(A, W, bias, out, M, N, K, F, tiles, st, S, add);
-  if (mb == 2) return launch_mb<2, N2, 2, EPI, HF>(A, W, bias, out, M, N, K, F, tiles, st, S, add);
+  if constexpr (NTW > 1) {
+    if (mb <= 1) return launch_mb<1, NTW, U, EPI, HF>(A, W, bias, out, M, N, K, F, tiles, st, S, add);
+  }
+  if (mb <= 2) return launch_mb<2, N2, 2, EPI, HF>(A, W, bias, out, M, N, K, F, tiles, st, S, add);
   if (mb == 3) return launch_mb<3, N34, 2, EPI, HF>(A, W, bias, out, M, N, K, F, tiles, st, S, add);
   return launch_mb<4, N34, 2, EPI, HF>(A, W, bias, out, M, N, K, F, tiles, st, S, add);
 }
@@ -105,41 +123,33 @@ template <bool HF>
 int gemv_run(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi, hipStream_t st,
              const void* add) {
   if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || N <= 0 || K <= 0) return -2;
-  if (tiles_form(M, N, epi)) {
+  if (tiles_form(M, N, K, epi)) {
     switch (epi) {
-      case EPI_OUT: return launch_tiles_rows<EPI_OUT, HF>(A, W, bias, out, M, N, K, st, 1, add);
+      case EPI_OUT: return add == nullptr ? launch_tiles_rows<EPI_OUT, HF>(A, W, bias, out, M, N, K, st)
+                                          : launch_tiles_rows<EPI_ADD, HF>(A, W, bias, out, M, N, K, st, 1, add);
       case EPI_GLU: return N % 32 != 0 ? -2 : launch_tiles<EPI_GLU, HF, 0, 1>(A, W, bias, out, M, N, K, st);
       case EPI_GELU_TANH: return launch_tiles_rows<EPI_GELU_TANH, HF>(A, W, bias, out, M, N, K, st);
       case EPI_GELU: return launch_tiles_rows<EPI_GELU, HF>(A, W, bias, out, M, N, K, st);
       default: return -2;
     }
   }
-  const int KP = K / 64;
-  const int U = KP >= 64 ? 4 : 2;                            // k-pairs in flight per wave
   if (epi == EPI_GLU) {
     if (N % 32 != 0) return -2;
     const int F = N / 2, ft = F / 16;
     if (ft >= 512) return launch<4, 2, EPI_GLU, HF>(A, W, bias, out, M, N, K, F, ft, st);
-    return U == 4 ? launch<2, 4, EPI_GLU, HF>(A, W, bias, out, M, N, K, F, ft, st)
-                  : launch<2, 2, EPI_GLU, HF>(A, W, bias, out, M, N, K, F, ft, st);
+    return K >= 4096 ? launch<2, 4, EPI_GLU, HF>(A, W, bias, out, M, N, K, F, ft, st)
+                     : launch<2, 2, EPI_GLU, HF>(A, W, bias, out, M, N, K, F, ft, st);
   }
   if (epi != EPI_OUT && epi != EPI_GELU_TANH && epi != EPI_GELU) return -2;
   const int nt = N / 16;
   // ~256 workgroups: one tile each below 512 tiles, then 2 or 4
-#define PICK(EP)                                                                               \
-  if (nt >= 1024) return launch<4, 2, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st);                \
-  if (nt >= 512) return U == 4 ? launch<2, 4, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st)         \
-                               : launch<2, 2, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st);        \
-  return U == 4 ? launch<1, 4, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st)                        \
-                : launch<1, 2, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st);
-  if (epi == EPI_GELU_TANH) { PICK(EPI_GELU_TANH) }
-  if (epi == EPI_GELU) { PICK(EPI_GELU) }
-  // plain output, optionally + a bf16 addend [M, N]
-  if (nt >= 1024) return launch<4, 2, EPI_OUT, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, add);
-  if (nt >= 512) return U == 4 ? launch<2, 4, EPI_OUT, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, add)
-                               : launch<2, 2, EPI_OUT, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, add);
-  return U == 4 ? launch<1, 4, EPI_OUT, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, add)
-                : launch<1, 2, EPI_OUT, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, add);
+#define PICK(EP, ADD)                                                                                       \
+  if (nt >= 1024) return launch<4, 2, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, ADD);                   \
+  if (nt >= 512) return launch<2, 4, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, ADD);                    \
+  return launch<1, 2, EP, HF>(A, W, bias, out, M, N, K, 0, nt, st, 1, ADD);
+  if (epi == EPI_GELU_TANH) { PICK(EPI_GELU_TANH, nullptr) }
+  if (epi == EPI_GELU) { PICK(EPI_GELU, nullptr) }
+  PICK(EPI_OUT, add)                                         // optionally + a bf16 addend [M, N]
 #undef PICK
 }
 
@@ -190,9 +200,7 @@ int gemv_splitk_run(const void* A, const void* W, const void* bias, float* part,
                     hipStream_t st) {
   if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || N <= 0 || S < 1 || S > K / 64) return -2;
   if (M <= 16) return launch_tiles_rows<EPI_PART, HF>(A, W, bias, part, M, N, K, st, S);
-  const int nt = N / 16, kps = K / 64 / S;
-  return kps >= 64 ? launch<1, 4, EPI_PART, HF>(A, W, bias, part, M, N, K, 0, nt, st, S)
-                   : launch<1, 2, EPI_PART, HF>(A, W, bias, part, M, N, K, 0, nt, st, S);
+  return launch<1, 2, EPI_PART, HF>(A, W, bias, part, M, N, K, 0, N / 16, st, S);
 }
 }  // namespace
 

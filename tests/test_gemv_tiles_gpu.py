@@ -20,10 +20,11 @@ def _near(y, ref, bound):
     assert bool((err <= bound).all()), float((err - bound).max())
 
 
-# K: less than a wave's k-pair each, ragged rounds, several rounds; N: one tile, ragged tiles a workgroup, over 1024 tiles
+# K: less than a wave's k-pair each, ragged rounds, several rounds; N: one tile, ragged tiles a workgroup, over 1024 tiles; 8192 x 4096 is two
+# tiles a workgroup from 11 rows on
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
-@pytest.mark.parametrize("N,K", [(16, 64), (48, 1088), (1040, 2560), (16400, 192)])
+@pytest.mark.parametrize("N,K", [(16, 64), (48, 1088), (1040, 2560), (16400, 192), (8192, 4096)])
 def test_plain_split_and_addend(cuda, dtype, M, N, K):
     x, w, b, add = _operands(cuda, dtype, M, N, K)
     wp = ops.pack_bf16_weight(w)
@@ -41,7 +42,7 @@ def test_plain_split_and_addend(cuda, dtype, M, N, K):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("M", [1, 3, 4, 6, 16])
-@pytest.mark.parametrize("N,K", [(32, 64), (1056, 1088), (16416, 192)])
+@pytest.mark.parametrize("N,K", [(32, 64), (1056, 1088), (16416, 192), (8192, 4096)])
 @pytest.mark.parametrize("epi", [1, 2, 3])
 def test_activations(cuda, dtype, M, N, K, epi):
     x, w, b, _ = _operands(cuda, dtype, M, N, K)

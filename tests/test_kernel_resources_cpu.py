@@ -45,7 +45,8 @@ def test_fenced_rounds_do_not_spill():
 
 
 # Workgroups that a launch counts on fitting a CU twice: waves of a SIMD
-TWICE = [("gemv_i8_rows.hip", r"w8a8_rows_kernel", 8),
+TWICE = [("gemv_bf16.hip", r"gemv_tiles_kernelILi1E.*Li1EEE", 8),           # (the template's last argument asks for it)
+         ("gemv_i8_rows.hip", r"w8a8_rows_kernel", 8),
          ("seqmix/attn_step.hip", r"attn_step_kernelI[ft]Li2ELi1E", 4)]     # rows of up to 64 numbers, 8 waves
 
 
