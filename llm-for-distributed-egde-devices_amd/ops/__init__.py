@@ -536,8 +536,9 @@ def raw_call(*ts: torch.Tensor) -> bool:
 
 def f32_rows_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None) -> bool:
     """Whether ``linear_bf16`` runs ``gemv_f32.hip`` for this call: dense 16-byte-aligned fp32 operands of one GPU, K % 4 == 0,
-    up to 4 rows, or up to 8 rows of at most 2^22 weights (in a graph, us at 8 rows, here / library: 1024 x 4096 6.2 / 10.0,
-    4096 x 1024 5.9 / 6.0, 6784 x 1024 8.7 / 7.3, 3000 x 12288 36 / 27; at 4 rows 5.6 / 7.3 and 24.9 / 26.4), in a ``raw_call`` (the library product serves the others)."""
+    up to 4 rows, or up to 8 rows of at most 2^22 weights (in a graph, us at 8 rows, here / library: 1024 x 4096 5.7 / 9.8,
+    4096 x 1024 5.2 / 5.9, 6784 x 1024 7.5 / 7.1, 3000 x 12288 30 / 27;
+    the last two at 4 rows 4.6 / 7.1 and 22.9 / 26.1), in a ``raw_call`` (the library product serves the others)."""
     if not (_gpu(x) and x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
         return False
     ts = (x, weight) if bias is None else (x, weight, bias)

@@ -2,13 +2,13 @@
 // Bound by reading W once, and below some 16 MB by the launch itself.  W stays in its [N, K] layout (no copy is made): a
 // wave takes R rows by 256 k at a time, each load one contiguous KiB of a row (with 16 rows by 16 k per load, the matrix
 // instruction's layout, the loads themselves were the bound: 1024 x 4096, launched one by one, 12.8 us against 5.9 here), the next 256 k on
-// their way meanwhile: a fence keeps the compiler from moving a load behind the products before it, and nothing past the end is
-// loaded.  Few rows: KW waves of a workgroup share a row's k (until about 2048 waves are at work: us at 1 row, 1024 / 2048 / 4096 waves,
+// their way meanwhile: the loop's loads stand under no guard (one that may not run is moved behind the products before it), and
+// nothing past the end is loaded, so the last two 256 k are taken behind it.  Few rows: KW waves of a workgroup share a row's k (until about 2048 waves are at work: us at 1 row, 1024 / 2048 / 4096 waves,
 // 4096 x 1024 5.8 / 4.9 / 5.0, 7840 x 1024 8.4 / 7.7 / 7.2, 8192 x 2048 13.3 / 13.3 / 14.0, 2048 x 8192 14.9 / 12.5 / 12.5) and add up
 // through LDS.  All sums in a fixed order.
-// N x K at 2 rows in a graph, weights from memory, us, before the fence / now: 384 x 1024 3.1 / 2.9, 1024 x 4096 5.6 / 5.3, 4096 x 1024
-// 5.9 / 5.4, 7840 x 1024 8.9 / 7.8, 8192 x 2048 14.7 / 13.5, 2048 x 8192 14.7 / 12.8, 32000 x 1024 25.7 / 25.5 (5.1 TB/s); relative error
-// against 64-bit sums 1e-7 here, 2 to 8e-7 in the library's product.
+// N x K at 2 rows in a graph, weights from memory, us, loads past the end / guarded behind a fence / now: 384 x 1024 3.3 / 2.8 / 2.7, 1024 x
+// 4096 5.9 / 5.5 / 5.3, 4096 x 1024 6.2 / 5.6 / 5.4, 7840 x 1024 9.3 / 8.6 / 8.0, 8192 x 2048 14.9 / 15.1 / 14.6, 2048 x 8192 14.6 / 13.7 / 13.1, 32000 x
+// 1024 25.6 / 26.9 / 25.7 (5.1 TB/s); relative error against 64-bit sums 1e-7 here, 2 to 8e-7 in the library's product.
 #include "common.h"
 
 namespace {
@@ -41,15 +41,17 @@ __device__ __forceinline__ void gemv_f32_body(int bid, const float* __restrict__
 #pragma unroll
         for (int j = 0; j < 4; ++j) acc[r * MV + m] = __builtin_fmaf(wv[b][r][j], xv[b][m][j], acc[r * MV + m]);
   };
-  // both halves' loads go out before either is used, and none past the end (a clamped one is read all the same)
-  if (kw < C) load(0, kw);
-  for (int c = kw; c < C; c += 2 * KW) {
-    if (c + KW < C) load(1, c + KW);
-    asm volatile("" ::: "memory");
+  int c = kw;
+  if (c < C) load(0, c);
+  for (; c + 2 * KW < C; c += 2 * KW) {
+    load(1, c + KW);
     use(0, c);
-    if (c + 2 * KW < C) load(0, c + 2 * KW);
-    if (c + KW < C) use(1, c + KW);
+    load(0, c + 2 * KW);
+    use(1, c + KW);
   }
+  if (c + KW < C) load(1, c + KW);
+  if (c < C) use(0, c);
+  if (c + KW < C) use(1, c + KW);
   int idx = 0;
   lane_sums<V, 32>(acc, idx, lane);
   // the first bits of the lane number chose; lanes that differ only in the others hold the same sum
@@ -115,8 +117,8 @@ void launch_f32x3(Jobs3 a, int M, hipStream_t st) {
 }  // namespace
 
 // y_j = x_j W_j^T for three projections of the same M rows' inputs, each as edge_gemv_f32 forms it: a parallel layer's three output
-// projections, whose launches' ramps and ends then overlap.  us in a graph, three launches / one, 1024 x 4096 and twice 1024 x
-// 1024: 1 row 11.9 / 6.5, 2 12.6 / 6.7; 2048 x 8192 and twice 2048 x 2048, 2 rows 27.0 / 18.3
+// projections, whose launches' ramps and ends then overlap.  us in a graph, weights from memory, three launches / one, 1024 x 4096 and
+// twice 1024 x 1024: 1 row 11.1 / 6.8, 2 11.5 / 7.0, 8 15.1 / 11.4; 2048 x 8192 and twice 2048 x 2048, 2 rows 24.0 / 18.8
 extern "C" int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K,
                                hipStream_t st) {
   Jobs3 a{};
