@@ -36,7 +36,7 @@ struct AttnExt {
 };
 
 template <int DK, int DV, int RH, bool KVS, bool EXT = false, bool REL = false>
-__global__ void __launch_bounds__(NT, (DV * RH <= 4 ? (REL && DK > 2 ? 2 : 4) : (DV * RH <= 8 ? 2 : 1))) attn_mfma_kernel(
+__global__ void __launch_bounds__(NT, (DV * RH <= 4 ? (REL && DK > 2 ? 2 : 4) : (DV * RH <= (KVS ? 12 : 8) ? 2 : 1))) attn_mfma_kernel(
     const bf16_t* __restrict__ q, const bf16_t* __restrict__ gate, int gate_ld, const bf16_t* __restrict__ kp,
     const bf16_t* __restrict__ vp, const float* __restrict__ kb, const float* __restrict__ vb,
     const int* __restrict__ seq_slot, const int* __restrict__ seq_start, const int* __restrict__ seq_len,

@@ -212,7 +212,8 @@ __device__ __forceinline__ void attn_chunk(const KT* __restrict__ kbase, const K
                                            float cap = 0.f, const float* sl_s = nullptr, int dist = 0,
                                            const float* __restrict__ rel = nullptr, int rel_n = 0) {
   constexpr int AW = VEC ? 8 : DVL;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (the wave's number as a scalar, but where that costs the scalar registers that then spill)
+  const int tid = threadIdx.x, lane = tid & 63, wave = VEC && DVL < 8 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   // (A) scores
   {
     float a[RMAX];
@@ -366,7 +367,7 @@ __global__ void __launch_bounds__(NT) attn_kernel(const T* __restrict__ q, const
   // more than RMAX query heads per kv head: nsp workgroups share the kv head, RMAX heads each
   const int t = blockIdx.x, g = blockIdx.y / nsp, r0 = (blockIdx.y % nsp) * RMAX;
   const int R = min(RMAX, H / G - r0), hq0 = g * (H / G) + r0;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int tid = threadIdx.x, lane = tid & 63, wave = VEC && DVL < 8 ? __builtin_amdgcn_readfirstlane(tid >> 6) : tid >> 6;
   float* q_s = smem;                         // [RMAX][D]
   float* s_s = q_s + RMAX * D;               // [RMAX][KC]
   float* red = s_s + RMAX * KC;              // [RMAX][Dv]
@@ -1016,7 +1017,12 @@ int edge_sm_attention(const void* q, const void* gate, int gate_ld, const void* 
   if (rmax == 0) return -3;
   const int nsp = (R + rmax - 1) / rmax;
   if (nsplit < 1 || nsplit > MAX_SPLIT || (nsplit > 1 && !part)) return -2;
-  const size_t lds = attn_lds_bytes(rmax, D, Dv);
+  size_t lds = attn_lds_bytes(rmax, D, Dv);
+  // fp32, four heads: four workgroups to a CU.  Where three take as many rounds, the fourth only slows the others in front of a last
+  // round of few: LDS for three.  us, 32 heads of 64 in 8 groups, four / three: 150 rows of 600 keys 113 / 99, 180 of 600 122 / 102, 150 of
+  // 300 64 / 58; where three take a round more, 128 rows of 300 keys 45 / 54
+  const long wgs = (long)rows * G * nsp * nsplit;
+  if (f32 && rmax == 4 && wgs > 1024 && (wgs + 1023) / 1024 == (wgs + 767) / 768) lds = max(lds, (size_t)41 * 1024);
   const bool vec = D % 8 == 0 && Dv % 8 == 0 && kld % 8 == 0 && vld % 8 == 0;
 #define SM_ATT_V(RM, DL, V)                                                                                         \
   SM_T(f32, hipLaunchKernelGGL((attn_kernel<T, RM, DL, V>), dim3(rows, G * nsp, nsplit), dim3(NT), lds, st, (const T*)q,         \

@@ -87,7 +87,8 @@ def test_splits_bias_and_view(dt):
     (torch.float32, 16, 4, 128, 128, [2000, 3]),                    # one head, split
     (torch.float32, 16, 1, 160, 128, [1300] * 12),                  # the general kernel's, split
     (torch.float32, 12, 3, 64, 64, [70] * 30),                      # four heads a workgroup, whole
-    (torch.float32, 12, 3, 64, 192, [70] * 30)])                    # the same with the widest values
+    (torch.float32, 12, 3, 64, 192, [70] * 30),                     # the same with the widest values
+    (torch.float32, 32, 8, 64, 64, [20] * 150)])                    # the general kernel's, 1200 workgroups, three to a CU
 def test_every_form_of_the_plan(dt, H, G, D, Dv, lens):
     _check(dt, lens, H, G, D, Dv, lambda q, k, v, kb, vb, m, on: S.window_pool_attention(
         q, None, k, v, None, None, m, D ** -0.5, None, None), latent=G == 1)
