@@ -25,8 +25,7 @@ constexpr int OW = GEMV_NW;                // waves of an o or down workgroup
 // rounds evenly (a round that runs over the end loads its last k-pair again), else 2.  Eight pairs of weights and rows are 128
 // registers by themselves: under the bound of two workgroups a CU they spill, us with 8 / 4: attention beside 16384 x 4096, 1 row
 // 32.4 / 25.5, 4 rows 36.9 / 26.2; rows3 1024 x 4096 and twice 1024 x 1024, 1 row 6.3 / 5.5, 2048 x 8192 and twice 2048 x 2048 12.5 / 11.6.
-// 16 waves: 5 where that divides the rounds, else 1 (more would take the registers of the CU's second workgroup: 2048 x 8192 beside
-// 2048 x 2048 9.3 us, with 8 in flight 11.4).
+// 16 waves: 5 where that divides the rounds, else 1 (2048 x 8192 beside 2048 x 2048 9.3 us, with 8 in flight 11.4).
 template <int NWV, int EPI, bool HF>
 __device__ __forceinline__ void proj_body(int bid, const Proj& p, int M, int act) {
   const int KP = p.K / 64;

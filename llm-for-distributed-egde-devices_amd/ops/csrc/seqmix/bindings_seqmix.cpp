@@ -689,6 +689,7 @@ std::optional<std::tuple<at::Tensor, at::Tensor>> sm_attention_ssd(
                               (uintptr_t)(PB ? kb->data_ptr<float>() : nullptr) | (uintptr_t)(PB ? vb->data_ptr<float>() : nullptr);
   const int plan = edge_sm_attention_step_plan((int)T, (int)H, (int)G, (int)D, (int)Dv, (int)kp.stride(1), (int)vp.stride(1), (int)page,
                                                PB ? (int)pool : 0, vis, f32(q), addresses);
+  if (plan != 9) return std::nullopt;                        // (one head a workgroup, whole keys)
   auto out = at::empty({T, H * Dv}, q.options()), y = at::empty({T, Hs * P}, q.options().dtype(at::kFloat));
   const int rc = edge_sm_attention_ssd(
       q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(), vp.data_ptr(), PB ? kb->data_ptr<float>() : nullptr,

@@ -247,7 +247,7 @@ __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict
     }
 }
 
-// (2) the state entering every chunk (written over that chunk's own contribution) and the final state; eight
+// (2) the state entering every chunk (written over that chunk's own contribution) and the final state; sixteen
 // chunks' rows are in flight at a time
 __global__ void __launch_bounds__(NT) gla_chunk_scan_kernel(float* __restrict__ sloc, const float* __restrict__ cdec,
                                                             float* __restrict__ state, const int* __restrict__ seq_slot,
