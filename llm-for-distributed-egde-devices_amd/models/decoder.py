@@ -216,6 +216,11 @@ class MLP(nn.Module):
             # W8A8 GELU MLP (Phi-2, Pythia) at decode rows: up projection + GELU + per-(token, 64)
             # int8 quantisation in one launch, consumed by the down projection's grouped-scale GEMV
             return self.down(self.up.geluq(x, self.act), add=add)
+        if type(self.up) is Linear and not down_q and self.act in ("silu_glu", "gelu_tanh", "gelu") and isinstance(x, torch.Tensor) \
+                and unwatched(self.up):
+            h = self.up.rows16(x, self.act)            # 17 to 64 rows: the activation in the product's epilogue
+            if h is not None:
+                return self.down(h, add=add)
         if self.act == "silu_glu" and type(self.up) is Linear and not down_q and not isinstance(x, QAct) \
                 and ops.bf16_gemv_ok(x, self.up.weight, glu=True):
             # bf16 decode: gate_up GEMV with the SwiGLU epilogue (one launch, gemv_bf16.hip)

@@ -1,6 +1,6 @@
 """Building blocks shared by every decoder family.
 
-``Linear`` is the bf16 projection (decode rows: ``gemv_bf16.hip`` up to 16, the bf16 ring GEMM
+``Linear`` is the bf16 projection (decode rows: ``gemv_bf16.hip`` up to 16, ``gemm_rows16.hip`` up to 64, the bf16 ring GEMM
 up to 256; otherwise hipBLASLt through ``F.linear`` — ``ops.linear_bf16``);
 quantised replacements live in ``edgellm.quant`` and expose the same interface:
 
@@ -200,6 +200,9 @@ class Linear(nn.Module):
             return self.forward_norm(x)
         if isinstance(x, QAct):
             x = (x.q.float() * x.scale[..., None]).to(self.weight.dtype)
+        y = None if self.split_k_out else self.rows16(x, add=add)
+        if y is not None:
+            return y
         wp = self.decode_weight(x)
         if self.split_k_out and wp is not None and add is None:
             K = x.shape[-1]
@@ -214,6 +217,14 @@ class Linear(nn.Module):
                                                              self.out_features, self.split_k_out), x.dtype)
         return ops.linear_bf16(x, self.weight, self.bias, packed=wp,
                                add=None if add is None else add.reshape(*x.shape[:-1], self.out_features))
+
+    def rows16(self, x, act: Optional[str] = None, add=None):
+        """17 to 64 rows in ``gemm_rows16.hip`` (``act``: the activation of the output), or None where that does not run."""
+        if not 17 * self.in_features <= x.numel() <= 64 * self.in_features or \
+                not ops.rows16_ok(x, self.weight, self.bias, act == "silu_glu"):
+            return None
+        return ops.rows16(x, self.packed_weight(), self.bias, self.out_features, act,
+                          None if add is None else add.reshape(*x.shape[:-1], self.out_features))
 
     def decode_weight(self, x, glu: bool = False) -> "Optional[torch.Tensor]":
         """Fragment-packed copy of the weight for the decode GEMV / ring GEMM, built on the first

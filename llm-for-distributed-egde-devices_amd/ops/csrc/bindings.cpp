@@ -146,6 +146,9 @@ int edge_kv_dequant(const void* src, int64_t c_sb, int64_t c_sh, const float* sc
 int edge_gemm_bf16_ring(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi, int S,
                         hipStream_t st);
 int edge_bf16_ring_splits(int N, int K);
+int edge_gemm_rows16_ok(int M, int N, int K, int epi);
+int edge_gemm_rows16(const void* x, const void* w, const void* bias, const void* add, void* out, int M, int N, int K, int epi, int S,
+                     int h16, hipStream_t st);
 int edge_bf16_ring_min_rows();
 void edge_decode_attn_gsplit(int v);
 void edge_decode_attn_small(int v);
@@ -892,8 +895,33 @@ at::Tensor gemv_bf16_splitk(const at::Tensor& x, const at::Tensor& wp, const std
   return part;
 }
 
-// bf16 decode projection at 17-256 rows on the ring2 kernel (gemm_i8.hip, bf16 operand mode) over
-// the same fragment-packed weight as gemv_bf16.  epi 0: bf16 [.., N]; 1: SwiGLU over [gate | up]
+// 16-bit projection of 17-64 rows over the fragment-packed weight (gemm_rows16.hip): epi 0 plain (+ addend), 1 SwiGLU over
+// [gate | up] (result [.., N / 2]), 2 / 3 gelu (tanh / erf).
+at::Tensor gemm_rows16(const at::Tensor& x, const at::Tensor& wp, const std::optional<at::Tensor>& bias, int64_t N, int64_t epi,
+                       const std::optional<at::Tensor>& addend) {
+  DEVICE_GUARD(x);
+  const int h16 = need16(x, "x");
+  need_same(wp, x, "weight (packed)");
+  const int64_t K = x.size(-1), M = rows_of(x);
+  TORCH_CHECK(wp.numel() == N * K, "packed weight must hold N * K elements");
+  TORCH_CHECK(((uintptr_t)x.data_ptr() | (uintptr_t)wp.data_ptr()) % 16 == 0, "gemm_rows16: 16-byte aligned operands");
+  TORCH_CHECK(M >= 17 && M <= 64 && epi >= 0 && epi <= 3, "gemm_rows16: 17-64 rows, epi 0-3");
+  if (bias) { need_same(*bias, x, "bias"); TORCH_CHECK(bias->numel() == N); }
+  if (addend) {
+    need_same(*addend, x, "addend");
+    TORCH_CHECK(epi == 0 && addend->numel() == M * N, "addend: plain output only, M * N elements");
+  }
+  auto os = x.sizes().vec();
+  os.back() = epi == 1 ? N / 2 : N;
+  auto out = at::empty(os, x.options());
+  check(edge_gemm_rows16(x.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr, addend ? addend->data_ptr() : nullptr,
+                         out.data_ptr(), (int)M, (int)N, (int)K, (int)epi, 1, h16, stream()),
+        "gemm_rows16");
+  return out;
+}
+
+// bf16 decode projection at 17-256 rows on the ring2 kernel (gemm_i8.hip, bf16 operand mode) or, where that is the quicker one,
+// gemm_rows16.hip, over the same fragment-packed weight as gemv_bf16.  epi 0: bf16 [.., N]; 1: SwiGLU over [gate | up]
 // -> bf16 [.., N / 2]; 3: split-K fp32 partial slices [S, M, N] (S = 0: the launcher's choice).
 at::Tensor gemm_bf16_ring(const at::Tensor& x, const at::Tensor& wp, const std::optional<at::Tensor>& bias, int64_t N,
                           int64_t epi, int64_t S) {
@@ -915,9 +943,15 @@ at::Tensor gemm_bf16_ring(const at::Tensor& x, const at::Tensor& wp, const std::
     out = at::empty(os, x.options());
     S = 1;
   }
-  check(edge_gemm_bf16_ring(x.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr, out.data_ptr(), (int)M,
-                            (int)N, (int)K, (int)epi, (int)S, stream()),
-        "gemm_bf16_ring");
+  const void* b = bias ? bias->data_ptr() : nullptr;
+  if ((epi == 0 || epi == 1 || epi == 3) && edge_gemm_rows16_ok((int)M, (int)N, (int)K, (int)epi) != 0 && S <= K / 64 &&
+      ((uintptr_t)x.data_ptr() | (uintptr_t)wp.data_ptr()) % 16 == 0)
+    check(edge_gemm_rows16(x.data_ptr(), wp.data_ptr(), b, nullptr, out.data_ptr(), (int)M, (int)N, (int)K, epi == 1, (int)S, 0,
+                           stream()),
+          "gemm_rows16");
+  else
+    check(edge_gemm_bf16_ring(x.data_ptr(), wp.data_ptr(), b, out.data_ptr(), (int)M, (int)N, (int)K, (int)epi, (int)S, stream()),
+          "gemm_bf16_ring");
   return out;
 }
 
@@ -1649,6 +1683,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("llmint8_outlier_rows", &llmint8_outlier_rows, "LLM.int8 outlier part for any rows, added in place");
   m.def("gemv_bf16_splitk", &gemv_bf16_splitk, "bf16 decode GEMV, split-K fp32 partial slices");
   m.def("gemm_bf16_ring", &gemm_bf16_ring, "bf16 decode GEMM, 17-256 rows (ring2 kernel, bf16 MFMA)");
+  m.def("gemm_rows16", &gemm_rows16, "16-bit projection of 17-64 rows", py::arg("x"), py::arg("wp"), py::arg("bias"), py::arg("N"),
+        py::arg("epi"), py::arg("addend") = py::none());
+  m.def("gemm_rows16_ok", [](int64_t M, int64_t N, int64_t K, int64_t epi) { return edge_gemm_rows16_ok((int)M, (int)N, (int)K, (int)epi) != 0; });
   m.def("bf16_ring_splits", [](int64_t N, int64_t K) { return (int64_t)edge_bf16_ring_splits((int)N, (int)K); });
   m.def("bf16_ring_min_rows", []() { return (int64_t)edge_bf16_ring_min_rows(); });
   m.def("gemv_bf16", &gemv_bf16, "bf16 decode GEMV (M <= 16), optional fused SwiGLU over [gate | up]", py::arg("x"),
