@@ -8,9 +8,9 @@
 //   o_t = (q_t D_t)^T S_in + sum_{s<=t} C[t, s] w_s,   C[t, s] = sum_n q_t k_s D_{s..t}
 // (1) delta_chunk_solve_kernel, parallel over chunks: A and C, then U and M with (I + A) [U | M] = [beta V | beta k D]
 //     by forward substitution over 16-token blocks (the blocks' own 16 x 16 systems inverted); also q D, k D_{..end}, D_end.
-// (2) delta_chunk_scan_kernel, chunk by chunk: W = U - M S_in and the next state, 16 value columns per workgroup.
+// (2) delta_chunk_scan_kernel, chunk by chunk: W = U - M S_in and the next state, 4 to 16 value columns per workgroup.
 // (3) delta_chunk_out_kernel, parallel over chunks: the outputs.
-// Sums, products and decays are fp64 (v_mfma_f64_16x16x4_f64 and plain FMAs); fp32 are the inputs, q D and k D_{..end}, the
+// Sums, products and decays are fp64 (v_mfma_f64_16x16x4_f64, 4x4x4_4b in (2), and plain FMAs); fp32 are the inputs, q D and k D_{..end}, the
 // states that (3) reads and the one that leaves.  In fp32 the form loses to the recurrence: with keys alike (cosine 0.98,
 // beta near 1) U and M S_in nearly cancel and the w_t of a chunk nearly add up to nothing, 1.1e-6 to 2e-6 against its 0.9e-7,
 // with random keys 1.6e-7 to 2.6e-7 against 1.1e-7.  No decay ratio is a quotient: from a token s to a later 16-token block it
@@ -21,12 +21,12 @@
 //
 // Bound: token by token, every token costs a chain of two row sums (about 530 clocks); here the chain is two products
 // and two barriers per 64 tokens, in fp64 at half the rate of fp32.  16 heads, 4096 tokens, us, token by token / this: 64 x 64
-// states 916 / 257 ((1) 115, (2) 140, (3) 37; 170 in fp32), 128 x 128 states 1512 / 527 ((2) 267, (3) 102; 373 in fp32); 512 tokens
-// 114 / 67 and 181 / 107.
+// states 916 / 198 ((1) 90, (2) 74, (3) 37), 128 x 128 states 1512 / 421; 512 tokens 114 / 56 and 181 / 86.
 #include "seqmix_common.h"
 
 namespace {
 
+typedef double v2d __attribute__((ext_vector_type(2)));
 typedef double v4d __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ v4d mfma4d(double a, double b, v4d c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 // one 16-wide block of k, 4 r + g4 of it in element r of a and b
@@ -375,18 +375,183 @@ __global__ void __launch_bounds__(NT, 2) delta_chunk_solve_kernel(const float* _
   }
 }
 
-// 4 KS waves, NP = 64 KS: wave w keeps the state rows 16 w .. of the workgroup's 16 value columns as an fp64 MFMA
-// accumulator, and computes the 16 tokens of block w % 4 of M S_in over the 64 channels of quarter w / 4 (the quarters'
-// shares meet in LDS).  The operands of the next D - 1 chunks are in registers on their way; nothing in the loop is
-// conditional, so the waits for them are counted ones.
-template <int KS, int D>
+// 4 KS waves, NP = 64 KS, 4 CS value columns a workgroup: wave w keeps the state rows 16 w .., and computes the 16 tokens of block
+// w % 4 of M S_in over the 64 channels of quarter w / 4 (the quarters' shares meet in LDS).  The next chunk's operands are requested in
+// four parts between the steps of this one (48 KiB a workgroup: asked for at once they hold up the wave that asks, 233 -> 211 us with 8
+// columns); nothing in the loop is conditional, so the waits for them are counted ones.
+// v_mfma_f64_4x4x4 does 64 operations a clock and SIMD where 16x16x4 does 32, and takes four columns, so that more CUs share a
+// head's columns.  Its four blocks take four fours of k of the same four rows: lane l, x = l >> 2, holds of row 4 g + (l & 3) the
+// numbers 4 (x & 3) + s of tile x / 4 in steps s = 0..3 (neighbours: one 32-byte load), and of the other operand that k's number in
+// column l & 3, read once for all four g.  four_sums adds up the blocks and leaves row 4 ((l >> 2) & 3) + l / 16, column l & 3.
+// 16 heads, 4096 tokens of 64 x 64 states: 140 us on 64 workgroups with 16x16x4, now 74; of 128 x 128 158 -> 64.
+__device__ __forceinline__ double mfma1d(double a, double b, double c) { return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ double lane_xor_d(double v, int o) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  return __builtin_bit_cast(double, (uint64_t)lane_xor((uint32_t)(u >> 32), o) << 32 | lane_xor((uint32_t)u, o));
+}
+__device__ __forceinline__ double four_sums(const double (&d)[4], int lane) {
+  const bool b1 = lane & 8, b0 = lane & 4;
+  const double e0 = (b1 ? d[2] : d[0]) + lane_xor_d(b1 ? d[0] : d[2], 8);
+  const double e1 = (b1 ? d[3] : d[1]) + lane_xor_d(b1 ? d[1] : d[3], 8);
+  return (b0 ? e1 : e0) + lane_xor_d(b0 ? e0 : e1, 4);
+}
+template <int KS, int CS>
 __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch sc, float* __restrict__ state,
+                                                                   const int* __restrict__ seq_slot,
+                                                                   const int* __restrict__ seq_start,
+                                                                   const int* __restrict__ seq_len, DeltaPart dp, int n, int H, int N, int P,
+                                                                   int PP) {
+  constexpr int NP = 64 * KS, PC = 4 * CS;
+  __shared__ double S_s[NP][PC], W_s[CL][PC], P_s[KS > 1 ? KS : 1][KS > 1 ? CL : 1][PC];
+  // the workgroups of a head share an L2: blocks are dealt to the eight dies in turn
+  const int nct = PP / PC, unit = ((int)blockIdx.x & 7) + 8 * (((int)blockIdx.x >> 3) / nct), ct = ((int)blockIdx.x >> 3) % nct;
+  if (unit >= n * H) return;
+  const int p0 = ct * PC, h = unit % H, s = unit / H, tid = threadIdx.x;
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 3, x = lane >> 2;
+  const int own = 4 * (x & 3) + (lane >> 4);                 // this lane's row of a wave's 16 (four_sums)
+  const int tb = wave & 3, kq = wave >> 2, n0 = 16 * wave, nc = chunks_of(seq_len[s], dp);
+  size_t cb0;
+  if (nc == 0 || !first_chunk(seq_len, s, dp, cb0)) return;
+  float* st = state + ((size_t)seq_slot[s] * H + h) * N * P;
+  const bool cont = seq_start[s] > 0 || dp.c0 > 0;
+  const int nr = n0 + own;
+  double S[CS];
+#pragma unroll
+  for (int c = 0; c < CS; ++c) {
+    const int p = p0 + 4 * c + j;
+    S[c] = (cont && nr < N && p < P) ? (double)st[(size_t)nr * P + p] : 0.;
+  }
+  struct Chunk {
+    v2d m[4][2];
+    float4 kd[4];
+    double dec, u[CS];
+  };
+  // KS > 1: a chunk's 64 x PC numbers of W are dealt to all threads
+  static_assert(KS == 1 || KS == 2, "states of up to 128 rows");
+  constexpr int UE = KS == 1 ? CS : (CL * PC + 256 * KS - 1) / (256 * KS);
+  auto wrow = [&](int i) { return KS == 1 ? 16 * tb + own : (tid + 256 * KS * i) / PC; };
+  auto wcol = [&](int i) { return KS == 1 ? 4 * i + j : (tid + 256 * KS * i) % PC; };
+  static_assert(UE <= CS, "numbers of W a thread");
+  auto load = [&](int c, Chunk& q, int part) {
+    const size_t cb = (cb0 + c) * H + h;
+    const double* mp = sc.M + cb * CL * NP + ((size_t)(tb * (NP / 16) + kq * 4 + (x >> 2)) * 16 + j) * 16 + 4 * (x & 3);
+    const float* kp = sc.Kd + cb * CL * NP + ((size_t)(wave * 4 + (x >> 2)) * 16 + j) * 16 + 4 * (x & 3);
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      if (part >= 0 && g != part) continue;
+      q.m[g][0] = *reinterpret_cast<const v2d*>(mp + g * 64);
+      q.m[g][1] = *reinterpret_cast<const v2d*>(mp + g * 64 + 2);
+      q.kd[g] = *reinterpret_cast<const float4*>(kp + g * 64);
+    }
+    if (part > 0) return;
+    q.dec = sc.cdec[cb * NP + n0 + PERM(own)];
+#pragma unroll
+    for (int i = 0; i < UE; ++i) {
+      const int r = KS == 1 ? wrow(i) : min(wrow(i), CL - 1);
+      q.u[i] = sc.U[(cb * CL + r) * PP + p0 + wcol(i)];
+    }
+  };
+  auto step = [&](int c, const Chunk& q, int cn, Chunk& qn) {
+    const size_t cb = (cb0 + c) * H + h;
+    load(cn, qn, 0);
+#pragma unroll
+    for (int i = 0; i < CS; ++i) {
+      sc.sin[cb * NP * PP + ((size_t)wave * PP + p0 + 4 * i + j) * 16 + PERM(own)] = (float)S[i];
+      S_s[nr][4 * i + j] = S[i];
+    }
+    __syncthreads();
+    double b[CS][4];
+#pragma unroll
+    for (int i = 0; i < CS; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) b[i][k] = S_s[64 * kq + 16 * (x >> 2) + 4 * k + (x & 3)][4 * i + j];
+    __builtin_amdgcn_sched_barrier(0);                       // every read on its way before the first product waits
+    load(cn, qn, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    double v[CS];
+#pragma unroll
+    for (int i = 0; i < CS; ++i) {
+      double d[4] = {0., 0., 0., 0.};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) d[g] = mfma1d(q.m[g][k >> 1][k & 1], b[i][k], d[g]);
+      v[i] = four_sums(d, lane);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    load(cn, qn, 2);
+    __builtin_amdgcn_sched_barrier(0);
+    double z[UE];
+    if constexpr (KS == 1) {
+#pragma unroll
+      for (int i = 0; i < UE; ++i) z[i] = q.u[i] - v[i];
+    } else {
+#pragma unroll
+      for (int i = 0; i < CS; ++i) P_s[kq][16 * tb + own][4 * i + j] = v[i];
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < UE; ++i) {
+        double sum = 0.;
+        const int r = min(wrow(i), CL - 1), cc = wcol(i);
+#pragma unroll
+        for (int k = 0; k < KS; ++k) sum += P_s[k][r][cc];
+        z[i] = q.u[i] - sum;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < UE; ++i) {
+      const int r = wrow(i), cc = wcol(i);
+      if (KS == 1 || r < CL) {
+        W_s[r][cc] = z[i];
+        sc.U[(cb * CL + r) * PP + p0 + cc] = z[i];
+      }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < CS; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) b[i][k] = W_s[16 * (x >> 2) + 4 * k + (x & 3)][4 * i + j];
+    __builtin_amdgcn_sched_barrier(0);
+    load(cn, qn, 3);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < CS; ++i) {
+      double d[4] = {0., 0., 0., 0.};
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const float4& f = q.kd[g];
+          d[g] = mfma1d((double)(k == 0 ? f.x : k == 1 ? f.y : k == 2 ? f.z : f.w), b[i][k], d[g]);
+        }
+      S[i] = __builtin_fma(q.dec, S[i], four_sums(d, lane));
+    }
+  };
+  Chunk even, odd;
+  load(0, even, -1);
+  int c = 0;
+  for (; c + 1 < nc; c += 2) {
+    step(c, even, c + 1, odd);
+    step(c + 1, odd, min(c + 2, nc - 1), even);              // (past the end: the last chunk again, not used)
+  }
+  if (c < nc) step(c, even, c, odd);
+#pragma unroll
+  for (int i = 0; i < CS; ++i) {
+    const int p = p0 + 4 * i + j;
+    if (nr < N && p < P) st[(size_t)nr * P + p] = (float)S[i];
+  }
+}
+
+// The same for states of 129 to 256 rows: 16 waves leave 128 registers a lane, too few for a chunk's operands on their way beside
+// another's (8 heads of 256 x 256, us for all three kernels, this form / the one above: 4096 tokens 700 / 714, six sequences of 512 419 / 689).
+// Wave w keeps the state rows 16 w .. of the workgroup's 16 value columns as a 16x16x4 accumulator.
+__global__ void __launch_bounds__(1024) delta_chunk_scan_wide_kernel(DeltaScratch sc, float* __restrict__ state,
                                                                    const int* __restrict__ seq_slot,
                                                                    const int* __restrict__ seq_start,
                                                                    const int* __restrict__ seq_len, DeltaPart dp, int H, int N, int P,
                                                                    int PP) {
-  constexpr int NP = 64 * KS, UE = 4 / KS;                   // rows of 16 numbers: four rows take each bank twice, the least
-  __shared__ double S_s[NP][16], W_s[CL][16], P_s[KS > 1 ? KS : 1][KS > 1 ? CL : 1][16];
+  constexpr int KS = 4, NP = 64 * KS;                        // rows of 16 numbers: four rows take each bank twice, the least
+  __shared__ double S_s[NP][16], W_s[CL][16], P_s[KS][CL][16];
   const int p0 = blockIdx.x * 16, h = blockIdx.y, s = blockIdx.z, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4, p = p0 + l16;
   const int tb = wave & 3, kq = wave >> 2, n0 = 16 * wave, nc = chunks_of(seq_len[s], dp);
@@ -397,12 +562,11 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
   v4d S;
 #pragma unroll
   for (int r = 0; r < 4; ++r) S[r] = (cont && n0 + 4 * r + g4 < N && p < P) ? (double)st[(size_t)(n0 + 4 * r + g4) * P + p] : 0.;
-  // this thread's numbers of a W tile, column l16: KS == 1: as the products' results lie; otherwise 4 KS waves of four rows
-  auto row = [&](int i) { return KS == 1 ? 16 * wave + 4 * i + g4 : tid / 16 + 16 * KS * i; };
+  const int row = tid / 16;                                  // this thread's number of a W tile, column l16
   struct Chunk {
     v4d m[4], dec;
     float4 kd[4];
-    double u[UE];
+    double u;
   };
   auto load = [&](int c, Chunk& x) {
     const size_t cb = (cb0 + c) * H + h;
@@ -414,8 +578,7 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
       x.kd[k] = *reinterpret_cast<const float4*>(kp + k * 256);
     }
     x.dec = *reinterpret_cast<const v4d*>(sc.cdec + cb * NP + n0 + 4 * g4);
-#pragma unroll
-    for (int i = 0; i < UE; ++i) x.u[i] = sc.U[(cb * CL + row(i)) * PP + p];
+    x.u = sc.U[(cb * CL + row) * PP + p];
   };
   auto step = [&](int c, const Chunk& x) {
     const size_t cb = (cb0 + c) * H + h;
@@ -433,27 +596,15 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
     v4d v = v4d{0., 0., 0., 0.};
 #pragma unroll
     for (int k = 0; k < 4; ++k) v = mma16(x.m[k], b[k], v);
-    double z[UE];
-    if constexpr (KS == 1) {
 #pragma unroll
-      for (int i = 0; i < UE; ++i) z[i] = x.u[i] - v[i];
-    } else {
+    for (int r = 0; r < 4; ++r) P_s[kq][16 * tb + 4 * r + g4][l16] = v[r];
+    __syncthreads();
+    double sum = 0.;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) P_s[kq][16 * tb + 4 * r + g4][l16] = v[r];
-      __syncthreads();
-#pragma unroll
-      for (int i = 0; i < UE; ++i) {
-        double sum = 0.;
-#pragma unroll
-        for (int k = 0; k < KS; ++k) sum += P_s[k][row(i)][l16];
-        z[i] = x.u[i] - sum;
-      }
-    }
-#pragma unroll
-    for (int i = 0; i < UE; ++i) {
-      W_s[row(i)][l16] = z[i];
-      sc.U[(cb * CL + row(i)) * PP + p] = z[i];
-    }
+    for (int k = 0; k < KS; ++k) sum += P_s[k][row][l16];
+    const double z = x.u - sum;
+    W_s[row][l16] = z;
+    sc.U[(cb * CL + row) * PP + p] = z;
     __syncthreads();
 #pragma unroll
     for (int k = 0; k < 4; ++k)
@@ -465,20 +616,11 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
     for (int k = 0; k < 4; ++k) a = mma16(widen(x.kd[k]), b[k], a);
     S = a;
   };
-  Chunk x[D];
-#pragma unroll
-  for (int d = 0; d < D - 1; ++d) load(min(d, nc - 1), x[d]);
-  int c0 = 0;
-  for (; c0 + D <= nc; c0 += D) {
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-      load(min(c0 + d + D - 1, nc - 1), x[(d + D - 1) % D]); // (past the end: the last chunk again, not used)
-      step(c0 + d, x[d]);
-    }
+  for (int c = 0; c < nc; ++c) {
+    Chunk x;
+    load(c, x);
+    step(c, x);
   }
-#pragma unroll
-  for (int d = 0; d < D - 1; ++d)
-    if (c0 + d < nc) step(c0 + d, x[d]);
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
     const int n = n0 + 4 * r + g4;
@@ -578,7 +720,6 @@ int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int C
   sc.Kd = sc.Qe + CH * CL * NP;
   sc.sin = sc.Kd + CH * CL * NP;
   const bool vec = N % 4 == 0 && prep_ld % 4 == 0 && ((uintptr_t)prep & 15) == 0;
-  const dim3 grid(PP / 16, H, n);                            // (a sequence's workgroups are neighbours: on all XCDs)
   const int ntp = (PP + 63) / 64;
   for (int c0 = 0; c0 < max_chunks; c0 += most) {
     const DeltaPart dp{least, c0, most, room};
@@ -592,12 +733,22 @@ int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int C
     } else if (vec) SM_DSOLVE(true, false);
     else SM_DSOLVE(false, false);
 #undef SM_DSOLVE
-#define SM_DSCAN(KS, D)                                                                                                    \
-  hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, D>), grid, dim3(256 * KS), 0, st, sc, state, seq_slot, seq_start, seq_len, \
-                     dp, H, N, P, PP)
-    if (NP == 64) SM_DSCAN(1, 3);
-    else if (NP == 128) SM_DSCAN(2, 2);
-    else SM_DSCAN(4, 1);
+    // columns a workgroup: as few fours as 256 workgroups, one a CU, leave; more share the operands' reads.  us for all three kernels,
+    // 4 / 8 / 16 columns: 16 heads of 64 x 64, 4096 tokens 198 / 211 / 283, 32 heads, four sequences of 2048 733 / 602 / 543; 16 of 128 x 128,
+    // 512 tokens 105 / 86 / 97, six sequences of 512 424 / 297 / 271
+#define SM_DSCAN(KS, CS)                                                                                                        \
+  hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, CS>), dim3((H * n + 7) / 8 * 8 * (PP / (4 * CS))), dim3(256 * KS), 0, st, sc, \
+                     state, seq_slot, seq_start, seq_len, dp, n, H, N, P, PP)
+#define SM_DCOLS(KS)                                          \
+  if (H * n * (PP / 4) <= 256) SM_DSCAN(KS, 1);               \
+  else if (H * n * (PP / 8) <= 256) SM_DSCAN(KS, 2);          \
+  else SM_DSCAN(KS, 4)
+    if (NP == 64) { SM_DCOLS(1); }
+    else if (NP == 128) { SM_DCOLS(2); }
+    else
+      hipLaunchKernelGGL(delta_chunk_scan_wide_kernel, dim3(PP / 16, H, n), dim3(1024), 0, st, sc, state, seq_slot, seq_start, seq_len, dp, H, N,
+                         P, PP);
+#undef SM_DCOLS
 #undef SM_DSCAN
     hipLaunchKernelGGL((delta_chunk_out_kernel<4>), dim3(mc * ntp, n, H), dim3(NT), 0, st, sc, seq_len, seq_off, y, dp, H, NP, P,
                        PP, ntp);

@@ -68,6 +68,23 @@ def test_chunks_against_the_recurrence(lens, starts, H, G, N, P, channel, decay,
 
 
 @gpu
+@pytest.mark.parametrize("n,H,G,N,P", [
+    (1, 16, 16, 64, 64), (1, 12, 4, 72, 80), (2, 16, 8, 33, 64), (2, 9, 3, 128, 112),    # 4 and 8 columns a workgroup
+    (5, 16, 8, 20, 80), (4, 11, 1, 100, 96), (9, 7, 7, 64, 16), (1, 1, 1, 64, 1)])       # 16; heads that do not fill the eight dies
+def test_chunks_at_every_split_of_the_columns(n, H, G, N, P, monkeypatch):
+    prep, qkv, state, meta = inputs((129, 64, 30, 70, 1, 65, 2, 128, 3)[:n], (5, 0, 1, 0, 3, 0, 0, 2, 1)[:n], H, G, N, P, True, "usual", seed=n)
+    before = state.double().cpu()
+    monkeypatch.setattr(seqmix, "DELTA_CHUNK_MIN", 1)
+    y = seqmix.delta_rule_scan(prep, qkv, state, meta, H, G, N, P).double().cpu()
+    p, v = prep.double().cpu(), qkv[:, 2 * G * N:].double().cpu().view(len(prep), H, P)
+    for slot, start, length, off in meta.host:
+        S0 = before[slot] if start > 0 else torch.zeros(H, N, P, dtype=torch.float64)
+        want, S = recurrence(p[off:off + length], v[off:off + length], S0, G, H, N, True)
+        assert (y[off:off + length].view(length, H, P) - want).norm() < TOL * want.norm()
+        assert (state[slot].double().cpu() - S).norm() < TOL * S.norm().clamp_min(1e-3)
+
+
+@gpu
 @pytest.mark.parametrize("channel", [True, False])
 @pytest.mark.parametrize("keys,decay", [("random", "usual"), ("random", "weak"), ("random", "strong"), ("alike", "none"), ("alike", "weak")])
 @pytest.mark.parametrize("H,G,N,P", [(4, 2, 64, 64), (2, 2, 128, 64), (2, 1, 200, 70)])
