@@ -216,8 +216,7 @@ class MLP(nn.Module):
             # W8A8 GELU MLP (Phi-2, Pythia) at decode rows: up projection + GELU + per-(token, 64)
             # int8 quantisation in one launch, consumed by the down projection's grouped-scale GEMV
             return self.down(self.up.geluq(x, self.act), add=add)
-        if type(self.up) is Linear and not down_q and self.act in ("silu_glu", "gelu_tanh", "gelu") and isinstance(x, torch.Tensor) \
-                and unwatched(self.up):
+        if type(self.up) is Linear and not down_q and self.act in ("silu_glu", "gelu_tanh", "gelu") and isinstance(x, torch.Tensor):
             h = self.up.rows16(x, self.act)            # 17 to 64 rows: the activation in the product's epilogue
             if h is not None:
                 return self.down(h, add=add)
@@ -554,6 +553,8 @@ class DecoderLM(nn.Module):
             return torch.nn.functional.linear(h, self.embed)
         wp = ops.kept_layout(self, "_embed_laid", self.embed._version, self.embed.device,
                              lambda: ops.pack_bf16_weight(self.embed.detach()))
+        if ops.rows16_ok(h, self.embed):
+            return ops.rows16(h, wp, None, self.embed.shape[0])
         return ops.linear_bf16(h, self.embed, None, packed=wp)
 
     @property

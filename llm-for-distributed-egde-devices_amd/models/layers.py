@@ -209,6 +209,8 @@ class Linear(nn.Module):
             if ops.bf16_decode_mode(x, self.weight, split=True) == 2:
                 # 17-256 rows: the ring GEMM's split-K slices (the launcher picks S for the shape)
                 S = int(ops.ext().bf16_ring_splits(self.out_features, K))
+                if S > 1 and self.rows16_ok(x, split=True):
+                    return PartialSum(ops.ext().gemm_rows16(x.reshape(-1, K), wp, self.bias, self.out_features, 0, S=S))
                 if S > 1:
                     return PartialSum(ops.ext().gemm_bf16_ring(x.reshape(-1, K), wp, self.bias,
                                                                self.out_features, 3, S))
@@ -218,10 +220,15 @@ class Linear(nn.Module):
         return ops.linear_bf16(x, self.weight, self.bias, packed=wp,
                                add=None if add is None else add.reshape(*x.shape[:-1], self.out_features))
 
+    def rows16_ok(self, x, glu: bool = False, split: bool = False) -> bool:
+        """Whether ``gemm_rows16.hip`` takes these rows.  Whoever watches the projection (a calibration's hooks, say) gets the
+        numbers of the kernels that serve other row counts too."""
+        return 17 * self.in_features <= x.numel() <= 64 * self.in_features and unwatched(self) and \
+            ops.rows16_ok(x, self.weight, self.bias, glu, split)
+
     def rows16(self, x, act: Optional[str] = None, add=None):
         """17 to 64 rows in ``gemm_rows16.hip`` (``act``: the activation of the output), or None where that does not run."""
-        if not 17 * self.in_features <= x.numel() <= 64 * self.in_features or \
-                not ops.rows16_ok(x, self.weight, self.bias, act == "silu_glu"):
+        if not self.rows16_ok(x, act == "silu_glu"):
             return None
         return ops.rows16(x, self.packed_weight(), self.bias, self.out_features, act,
                           None if add is None else add.reshape(*x.shape[:-1], self.out_features))

@@ -448,10 +448,10 @@ def bf16_decode_mode(x: torch.Tensor, weight: torch.Tensor, glu: bool = False, s
     return 0
 
 
-def rows16_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, glu: bool = False) -> bool:
-    """Whether ``linear_bf16`` runs ``gemm_rows16.hip`` for this call where a layer keeps its packed weight: 17 to 64 rows, bf16
-    or fp16, dense 16-byte-aligned operands of one GPU in a ``raw_call``.  Where the ring GEMM does not run (``bf16_decode_mode``
-    0) only up to K = 2048 or 2 N: longer rows over few outputs are read by few workgroups, and the library splits K (us, here /
+def rows16_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None, glu: bool = False, split: bool = False) -> bool:
+    """Whether ``gemm_rows16.hip`` (``rows16``) takes this product of a layer that keeps its packed weight: 17 to 64 rows, bf16
+    or fp16, dense 16-byte-aligned operands of one GPU in a ``raw_call``; ``split``: as fp32 slices.  Where the ring GEMM does not
+    run (``bf16_decode_mode`` 0) only up to K = 2048 or 2 N: longer rows over few outputs are read by few workgroups, and the library splits K (us, here /
     library: 2048 x 8192, 21 and 45 rows, 13.6 / 13.1 and 18.6 / 14.9; 512 x 16384 21.5 / 18.8; 4608 x 4608 15.2 / 17.8, 17.4 / 23.7)."""
     if x.dtype not in (torch.bfloat16, torch.float16) or weight.dtype != x.dtype or weight.dim() != 2 or x.dim() == 0:
         return False
@@ -465,9 +465,9 @@ def rows16_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
         return False
     if not available() and not _MAIN_EXT_REQUIRED:
         return False
-    if K > max(2048, 2 * N) and not (x.dtype == torch.bfloat16 and (glu or N >= 16384)):
+    if K > max(2048, 2 * N) and not (x.dtype == torch.bfloat16 and (glu or split or N >= 16384)):
         return False
-    return ext().gemm_rows16_ok(x.numel() // K, N, K, 1 if glu else 0)
+    return ext().gemm_rows16_ok(x.numel() // K, N, K, 3 if split else 1 if glu else 0)
 
 
 def rows16(x, packed, bias, N: int, act: Optional[str] = None, add: Optional[torch.Tensor] = None):
@@ -598,9 +598,6 @@ def linear_bf16(x, weight, bias=None, glu: bool = False, act: Optional[str] = No
         act = "silu_glu"
     assert add is None or act is None, "addend: plain outputs only"
     mode = bf16_decode_mode(x, weight, glu)
-    if (mode == 2 or (mode == 0 and packed is not None)) and (glu or act in (None, "gelu_tanh", "gelu")) and rows16_ok(x, weight, bias, glu):
-        wp = packed if packed is not None else pack_bf16_weight(weight)
-        return rows16(x, wp, bias, weight.shape[0], act, add)
     if mode == 1 or (mode == 2 and act in (None, "silu_glu")):
         wp = packed if packed is not None else pack_bf16_weight(weight)
         if mode == 1:

@@ -118,7 +118,9 @@ int edge_llmint8_o_down(const void* x, float thr_o, const void* wo, const float*
                         const float* scbo, void* a, int Ko, const void* h, float thr_d, const void* wd, const float* swd,
                         const void* bd, const void* wtd, const float* scbd, void* y, int Kd, int N, hipStream_t st);
 int edge_llmint8_prep_rows(const void* x, int M, int K, float thr, void* q, float* sa, int* cols, int* count,
-                           uint32_t* flags, uint32_t* take, hipStream_t st);
+                           uint32_t* flags, hipStream_t st);
+int edge_gemm_rows_i8(const void* A, const float* sa, const void* w, const float* sw, const void* bias, const void* add, void* out, int M,
+                      int N, int K, int act, const void* x, const int* cols, const int* count, const void* wt, const float* scb, hipStream_t st);
 int edge_llmint8_outlier_rows(void* out, const void* x, const int* cols, const int* count, const void* wt,
                               const float* scb, int M, int N, int K, hipStream_t st);
 void edge_w8a8_gemv_ntw(int ntw);
@@ -720,6 +722,19 @@ at::Tensor w8a8_gemm(const at::Tensor& a, const at::Tensor& sa, const at::Tensor
   auto os = a.sizes().vec();
   os.back() = N;
   auto out = at::empty(os, a.options().dtype(at::kBFloat16));
+  if (mpad == 0 && M >= 17 && M <= 64) {                     // (gemm_rows16.hip; -2: sizes it leaves to the kernels below)
+    if (addend) {
+      need(*addend, at::kBFloat16, "addend");
+      TORCH_CHECK(addend->numel() == M * N, "addend must hold M * N elements");
+    }
+    const int rc = edge_gemm_rows_i8(a.data_ptr(), sa.data_ptr<float>(), wp.data_ptr(), sw.data_ptr<float>(),
+                                     bias ? bias->data_ptr() : nullptr, addend ? addend->data_ptr() : nullptr, out.data_ptr(), (int)M,
+                                     (int)N, (int)K, 0, nullptr, nullptr, nullptr, nullptr, nullptr, stream());
+    if (rc != -2) {
+      check(rc, "gemm_rows_i8");
+      return out;
+    }
+  }
   if (addend) {
     need(*addend, at::kBFloat16, "addend");
     TORCH_CHECK(addend->numel() == M * N, "addend must hold M * N elements");
@@ -896,9 +911,9 @@ at::Tensor gemv_bf16_splitk(const at::Tensor& x, const at::Tensor& wp, const std
 }
 
 // 16-bit projection of 17-64 rows over the fragment-packed weight (gemm_rows16.hip): epi 0 plain (+ addend), 1 SwiGLU over
-// [gate | up] (result [.., N / 2]), 2 / 3 gelu (tanh / erf).
+// [gate | up] (result [.., N / 2]), 2 / 3 gelu (tanh / erf); S > 1 (bf16): fp32 slices [S, M, N] of the plain product.
 at::Tensor gemm_rows16(const at::Tensor& x, const at::Tensor& wp, const std::optional<at::Tensor>& bias, int64_t N, int64_t epi,
-                       const std::optional<at::Tensor>& addend) {
+                       const std::optional<at::Tensor>& addend, int64_t S) {
   DEVICE_GUARD(x);
   const int h16 = need16(x, "x");
   need_same(wp, x, "weight (packed)");
@@ -911,17 +926,18 @@ at::Tensor gemm_rows16(const at::Tensor& x, const at::Tensor& wp, const std::opt
     need_same(*addend, x, "addend");
     TORCH_CHECK(epi == 0 && addend->numel() == M * N, "addend: plain output only, M * N elements");
   }
+  TORCH_CHECK(S == 1 || (S > 1 && epi == 0 && !h16 && !addend), "gemm_rows16: slices of the plain bf16 product");
   auto os = x.sizes().vec();
   os.back() = epi == 1 ? N / 2 : N;
-  auto out = at::empty(os, x.options());
+  auto out = S > 1 ? at::empty({S, M, N}, x.options().dtype(at::kFloat)) : at::empty(os, x.options());
   check(edge_gemm_rows16(x.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr, addend ? addend->data_ptr() : nullptr,
-                         out.data_ptr(), (int)M, (int)N, (int)K, (int)epi, 1, h16, stream()),
+                         out.data_ptr(), (int)M, (int)N, (int)K, (int)epi, (int)S, h16, stream()),
         "gemm_rows16");
   return out;
 }
 
-// bf16 decode projection at 17-256 rows on the ring2 kernel (gemm_i8.hip, bf16 operand mode) or, where that is the quicker one,
-// gemm_rows16.hip, over the same fragment-packed weight as gemv_bf16.  epi 0: bf16 [.., N]; 1: SwiGLU over [gate | up]
+// bf16 decode projection at 17-256 rows on the ring2 kernel (gemm_i8.hip, bf16 operand mode) over
+// the same fragment-packed weight as gemv_bf16.  epi 0: bf16 [.., N]; 1: SwiGLU over [gate | up]
 // -> bf16 [.., N / 2]; 3: split-K fp32 partial slices [S, M, N] (S = 0: the launcher's choice).
 at::Tensor gemm_bf16_ring(const at::Tensor& x, const at::Tensor& wp, const std::optional<at::Tensor>& bias, int64_t N,
                           int64_t epi, int64_t S) {
@@ -943,15 +959,9 @@ at::Tensor gemm_bf16_ring(const at::Tensor& x, const at::Tensor& wp, const std::
     out = at::empty(os, x.options());
     S = 1;
   }
-  const void* b = bias ? bias->data_ptr() : nullptr;
-  if ((epi == 0 || epi == 1 || epi == 3) && edge_gemm_rows16_ok((int)M, (int)N, (int)K, (int)epi) != 0 && S <= K / 64 &&
-      ((uintptr_t)x.data_ptr() | (uintptr_t)wp.data_ptr()) % 16 == 0)
-    check(edge_gemm_rows16(x.data_ptr(), wp.data_ptr(), b, nullptr, out.data_ptr(), (int)M, (int)N, (int)K, epi == 1, (int)S, 0,
-                           stream()),
-          "gemm_rows16");
-  else
-    check(edge_gemm_bf16_ring(x.data_ptr(), wp.data_ptr(), b, out.data_ptr(), (int)M, (int)N, (int)K, (int)epi, (int)S, stream()),
-          "gemm_bf16_ring");
+  check(edge_gemm_bf16_ring(x.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr, out.data_ptr(), (int)M,
+                            (int)N, (int)K, (int)epi, (int)S, stream()),
+        "gemm_bf16_ring");
   return out;
 }
 
@@ -1144,12 +1154,46 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> llmint8_prep_rows(con
   auto sa = at::empty({M}, x.options().dtype(at::kFloat));
   auto cols = at::empty({K}, x.options().dtype(at::kInt));
   auto count = at::empty({1}, x.options().dtype(at::kInt));
-  auto bits = at::empty({2 * (K / 32)}, x.options().dtype(at::kInt));
+  auto bits = at::empty({K / 32}, x.options().dtype(at::kInt));
   uint32_t* flags = reinterpret_cast<uint32_t*>(bits.data_ptr<int>());
   check(edge_llmint8_prep_rows(x.data_ptr(), (int)M, (int)K, (float)thr, q.data_ptr(), sa.data_ptr<float>(),
-                               cols.data_ptr<int>(), count.data_ptr<int>(), flags, flags + K / 32, stream()),
+                               cols.data_ptr<int>(), count.data_ptr<int>(), flags, stream()),
         "llmint8_prep_rows");
   return {q, sa, cols, count};
+}
+
+// LLM.int8 product of 17-64 prepared rows (llmint8_prep_rows) with the outlier columns' part, gelu (act 1 tanh, 2 erf) of the
+// result or + an addend in one launch: bf16 [M, N], or nothing where the kernel does not take the sizes.
+std::optional<at::Tensor> llmint8_rows(const at::Tensor& q, const at::Tensor& sa, const at::Tensor& x, const at::Tensor& cols,
+                                       const at::Tensor& count, const at::Tensor& wp, const at::Tensor& sw,
+                                       const std::optional<at::Tensor>& bias, const at::Tensor& wt, const at::Tensor& scb, int64_t N,
+                                       int64_t act, const std::optional<at::Tensor>& addend) {
+  DEVICE_GUARD(q);
+  need(q, at::kChar, "q");
+  need(sa, at::kFloat, "sa");
+  need(x, at::kBFloat16, "x");
+  need(cols, at::kInt, "cols");
+  need(count, at::kInt, "count");
+  need(wt, at::kChar, "weight_t");
+  need(scb, at::kFloat, "SCB");
+  TORCH_CHECK(q.dim() == 2 && x.dim() == 2 && x.sizes() == q.sizes(), "q and x: [M, K]");
+  const int64_t M = q.size(0), K = q.size(1);
+  check_w8a8_operands(wp, sw, bias, N, K);
+  TORCH_CHECK(M >= 17 && M <= 64 && sa.numel() == M && cols.numel() >= K && count.numel() >= 1 && wt.numel() == K * N &&
+                  scb.numel() == N && act >= 0 && act <= 2,
+              "llmint8_rows: shapes");
+  if (addend) {
+    need(*addend, at::kBFloat16, "addend");
+    TORCH_CHECK(addend->numel() == M * N && act == 0, "addend: M * N elements, no activation");
+  }
+  auto out = at::empty({M, N}, x.options());
+  const int rc = edge_gemm_rows_i8(q.data_ptr(), sa.data_ptr<float>(), wp.data_ptr(), sw.data_ptr<float>(),
+                                   bias ? bias->data_ptr() : nullptr, addend ? addend->data_ptr() : nullptr, out.data_ptr(), (int)M, (int)N,
+                                   (int)K, act ? (int)act + 1 : 0, x.data_ptr(), cols.data_ptr<int>(), count.data_ptr<int>(), wt.data_ptr(),
+                                   scb.data_ptr<float>(), stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "gemm_rows_i8");
+  return out;
 }
 
 // out bf16 [M, N] += x[:, cols[:count]] . W^T[cols[:count]] * SCB / 127 (wt = int8 W^T [K, N]), in place.
@@ -1680,11 +1724,12 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("llmint8_attn_up", &llmint8_attn_up, "decode attention beside the LLM.int8 up projection of one row");
   m.def("llmint8_o_down", &llmint8_o_down, "o beside the down projection of one LLM.int8 row");
   m.def("llmint8_prep_rows", &llmint8_prep_rows, "LLM.int8 preparation for any rows (uncapped, on the device)");
+  m.def("llmint8_rows", &llmint8_rows, "LLM.int8 product of 17-64 prepared rows with its outlier columns");
   m.def("llmint8_outlier_rows", &llmint8_outlier_rows, "LLM.int8 outlier part for any rows, added in place");
   m.def("gemv_bf16_splitk", &gemv_bf16_splitk, "bf16 decode GEMV, split-K fp32 partial slices");
   m.def("gemm_bf16_ring", &gemm_bf16_ring, "bf16 decode GEMM, 17-256 rows (ring2 kernel, bf16 MFMA)");
   m.def("gemm_rows16", &gemm_rows16, "16-bit projection of 17-64 rows", py::arg("x"), py::arg("wp"), py::arg("bias"), py::arg("N"),
-        py::arg("epi"), py::arg("addend") = py::none());
+        py::arg("epi"), py::arg("addend") = py::none(), py::arg("S") = 1);
   m.def("gemm_rows16_ok", [](int64_t M, int64_t N, int64_t K, int64_t epi) { return edge_gemm_rows16_ok((int)M, (int)N, (int)K, (int)epi) != 0; });
   m.def("bf16_ring_splits", [](int64_t N, int64_t K) { return (int64_t)edge_bf16_ring_splits((int)N, (int)K); });
   m.def("bf16_ring_min_rows", []() { return (int64_t)edge_bf16_ring_min_rows(); });

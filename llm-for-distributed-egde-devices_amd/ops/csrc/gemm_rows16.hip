@@ -1,5 +1,6 @@
-// 16-bit projections of 17 to 64 rows: y[M, N] = x[M, K] . W[N, K]^T (+ bias), bf16 or fp16, over the fragment-packed weight
-// of the decode GEMV (gemv_bf16.hip).
+// Projections of 17 to 64 rows: y[M, N] = x[M, K] . W[N, K]^T (+ bias), bf16, fp16 or int8, over the fragment-packed weight of the
+// decode GEMVs (gemv_bf16.hip, gemm_i8.h: byte for byte the same tiles of 16 rows x 64 bytes, so int8 operands are read as half as
+// many 16-bit numbers).
 //
 // Bound by the weights' bytes, then by what reading the rows costs beside them.  A workgroup is 8 waves on NT tiles of 16 outputs;
 // wave w takes the k-pairs (2 KiB of a tile) w, w + 8, ... and holds one pair of each tile in flight while another is multiplied.
@@ -13,17 +14,40 @@
 //   8192 x 2048             9.0 /  9.5 / 10.7 | 11.8 / 12.0 / 12.0       2048 x 8192  13.9 / 15.8 / 22.1 | 14.1 / 16.4 / 23.0
 //   SwiGLU 22016 x 4096    33.4 / 34.1 (40: 36.1) | 39.0 / 39.5 (39.9)   16384 x 2048 14.8 / 15.5 / 17.3 | 21.7 / 21.9 / 24.0
 //   4 slices, 4096 x 4096   9.5 /  9.8 / 11.5 | 11.7 / 12.1 / 12.4       4096 x 11008 18.3 / 18.9 / 22.4 | 22.1 / 21.9 / 23.8
+// int8 (plain outputs): us, 45 rows, here | before (the decode GEMV's four row blocks; LLM.int8 with its outlier columns in a launch of
+// their own): I8_FIGURES
 #include "gemv_bf16.h"
 
 namespace {
 constexpr int GR_NW = 8;
 constexpr int ROWS_OUT = 0, ROWS_GLU = 1, ROWS_PART = 2;
+constexpr int DT_BF16 = 0, DT_FP16 = 1, DT_I8 = 2;
+constexpr int OUTLIERS = 32;                                // outlier columns in LDS at a time
 
 struct RowsArgs {
   const bf16_t *x, *w, *bias, *add;                         // bias [N], add [M, N]: may be null
   void* out;
   int M, N, K, S, act;                                      // act (ROWS_OUT): 0, or gelu of the 16-bit output (2 tanh, 3 erf)
+  // int8: scales of the rows and of the outputs; LLM.int8's columns (count null: none): x before quantisation [M, 2 K], W^T [2 K, N]
+  const float *sa, *sw;
+  const bf16_t* xo;
+  const int *cols, *count;
+  const int8_t* wt;
+  const float* scb;
 };
+template <int DT>
+struct Sum {
+  using type = v4f;
+};
+template <>
+struct Sum<DT_I8> {
+  using type = v4i;
+};
+template <int DT>
+__device__ __forceinline__ typename Sum<DT>::type rows_mma(const v8s& w, const v4i& x, const typename Sum<DT>::type& c) {
+  if constexpr (DT == DT_I8) return __builtin_amdgcn_mfma_i32_16x16x64_i8(__builtin_bit_cast(v4i, w), x, c, 0, 0, 0);
+  else return mfma_16<DT == DT_FP16>(w, __builtin_bit_cast(v8s, x), c);
+}
 
 __device__ __forceinline__ void glds16(const void* g, void* lds_base) {
   __builtin_amdgcn_global_load_lds(g, (__attribute__((address_space(3))) void*)lds_base, 16, 0, 0);
@@ -38,13 +62,16 @@ constexpr int sums_together(int MB, int NT, bool glu) {
   return c;
 }
 
-template <int MB, int NT, int EPI, bool HF>
+template <int MB, int NT, int EPI, int DT>
 __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) {
-  constexpr bool GLU = EPI == ROWS_GLU;
+  using Acc = typename Sum<DT>::type;
+  constexpr bool GLU = EPI == ROWS_GLU, HF = DT == DT_FP16, I8 = DT == DT_I8;
+  static_assert(!I8 || EPI == ROWS_OUT, "int8: plain outputs");
   constexpr int CT = sums_together(MB, NT, GLU), LOADS = 2 * MB + 2 * NT;   // of a wave and k-pair
   constexpr int XW = 2 * MB * 2048, RB = GR_NW * MB * CT * 1024, LB = GR_NW * XW > RB ? GR_NW * XW : RB;
   __shared__ __attribute__((aligned(1024))) char lds[LB];    // the waves' rows (two k-pairs each), then their sums
-  v4f (*red)[MB * CT][64] = reinterpret_cast<v4f (*)[MB * CT][64]>(lds);
+  __shared__ float xs[I8 ? OUTLIERS : 1][I8 ? 16 * MB : 1];  // outlier columns of the rows
+  Acc (*red)[MB * CT][64] = reinterpret_cast<Acc (*)[MB * CT][64]>(lds);
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r = lane & 15;
   const int M = p.M, N = p.N, K = p.K, KP = K / 64, nt = N / 16;
   const int grp = EPI == ROWS_PART ? (int)blockIdx.x / p.S : (int)blockIdx.x, ks = EPI == ROWS_PART ? (int)blockIdx.x % p.S : 0;
@@ -63,11 +90,11 @@ __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) 
   const uint32_t fr = lds_addr(xw) + (r >> 3) * 1024 + (r & 7) * 128 + (((lane >> 4) ^ (r & 7)) << 4);
   const int n = kend - kbeg > wave ? (kend - kbeg - wave + GR_NW - 1) / GR_NW : 0;   // this wave's k-pairs
 
-  v4f acc[MB][NT];
+  Acc acc[MB][NT];
 #pragma unroll
   for (int m = 0; m < MB; ++m)
 #pragma unroll
-    for (int j = 0; j < NT; ++j) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < NT; ++j) acc[m][j] = Acc{};
   v8s A[NT][2], B[NT][2];
   auto load = [&](int u, v8s (&f)[NT][2]) {                  // k-pair u of this wave
     const size_t kp = kbeg + wave + GR_NW * u;
@@ -102,7 +129,7 @@ __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) 
 #pragma unroll
       for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int m = 0; m < MB; ++m) acc[m][j] = mfma_16<HF>(f[j][s], __builtin_bit_cast(v8s, a[s][m]), acc[m][j]);
+        for (int m = 0; m < MB; ++m) acc[m][j] = rows_mma<DT>(f[j][s], a[s][m], acc[m][j]);
   };
   if (n > 0) load(0, A);
   if (n > 1) load(1, B);
@@ -129,19 +156,54 @@ __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) 
 #pragma unroll
       for (int m = 0; m < MB; ++m) red[wave][c * MB + m][lane] = acc[m][GLU ? (c & 1) * (NT / 2) + (c0 + c) / 2 : c0 + c];
     __syncthreads();
-    for (int b = wave; b < MB * CT / (GLU ? 2 : 1); b += GR_NW) {
+    constexpr int BLOCKS = MB * CT / (GLU ? 2 : 1), OWN = (BLOCKS + GR_NW - 1) / GR_NW;   // 16 x 16 outputs, of a wave
+    float extra[I8 ? OWN : 1][4];
+    bool outliers = false;
+    if constexpr (I8) {
+      const int nt_out = p.count != nullptr ? *p.count : 0;
+      outliers = nt_out > 0;
+#pragma unroll
+      for (int o = 0; o < OWN; ++o)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) extra[o][q] = 0.f;
+      for (int j0 = 0; j0 < nt_out; j0 += OUTLIERS) {        // (no such column: one load)
+        __syncthreads();
+        for (int i = threadIdx.x; i < OUTLIERS * 16 * MB; i += GR_NW * 64) {
+          const int jj = i / (16 * MB), row = i % (16 * MB);
+          xs[jj][row] = j0 + jj < nt_out && row < M ? bf2f(p.xo[(size_t)row * (2 * K) + p.cols[j0 + jj]]) : 0.f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int o = 0; o < OWN; ++o) {
+          const int b = wave + o * GR_NW, col = min(16 * (grp * NT + c0 + b / MB) + c4, N - 4);
+          if (b >= BLOCKS) continue;
+          for (int jj = 0; jj < min(OUTLIERS, nt_out - j0); ++jj) {
+            const char4 w4 = *reinterpret_cast<const char4*>(p.wt + (size_t)p.cols[j0 + jj] * N + col);
+            const float xv = xs[jj][16 * (b % MB) + r];
+            extra[o][0] += xv * (float)w4.x;
+            extra[o][1] += xv * (float)w4.y;
+            extra[o][2] += xv * (float)w4.z;
+            extra[o][3] += xv * (float)w4.w;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (int o = 0; o < OWN; ++o) {
+      const int b = wave + o * GR_NW;
+      if (b >= BLOCKS) continue;
       const int m = b % MB, c = (b / MB) * (GLU ? 2 : 1), row = 16 * m + r;
       auto total = [&](int s) {
-        v4f t = red[0][s][lane];
+        Acc t = red[0][s][lane];
 #pragma unroll
         for (int w = 1; w < GR_NW; ++w) t += red[w][s][lane];
         return t;
       };
-      const v4f s0 = total(c * MB + m);
+      const Acc s0 = total(c * MB + m);
       const int t = GLU ? grp * (NT / 2) + (c0 + c) / 2 : grp * NT + c0 + c, F = GLU ? N / 2 : N, col = 16 * t + c4;
       float v[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) v[q] = s0[q];
+      for (int q = 0; q < 4; ++q) v[q] = (float)s0[q];
       if constexpr (GLU) {
         const v4f s1 = total((c + 1) * MB + m);
         if (row >= M || t >= nt / 2) continue;
@@ -153,9 +215,18 @@ __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) 
         }
       } else {
         if (row >= M || t >= nt) continue;
-        if (p.bias != nullptr && ks == 0)
+        if constexpr (I8) {
+          const float sr = p.sa[row];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            v[q] = v[q] * sr;
+            v[q] = v[q] * p.sw[col + q] + (p.bias != nullptr ? bf2f(p.bias[col + q]) : 0.f);
+            if (outliers) v[q] = bf2f(f2bf(v[q])) + extra[o][q] * (p.scb[col + q] / 127.f);
+          }
+        } else if (p.bias != nullptr && ks == 0) {
 #pragma unroll
           for (int q = 0; q < 4; ++q) v[q] += e2f<HF>(p.bias[col + q]);
+        }
         if constexpr (EPI == ROWS_PART) {
           *reinterpret_cast<float4*>((float*)p.out + ((size_t)ks * M + row) * N + col) = float4{v[0], v[1], v[2], v[3]};
           continue;
@@ -175,36 +246,36 @@ __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) 
   }
 }
 
-template <int MB, int NT, int EPI, bool HF>
+template <int MB, int NT, int EPI, int DT>
 int launch_rows(const RowsArgs& p, hipStream_t st) {
   const int tiles = EPI == ROWS_GLU ? p.N / 32 : p.N / 16, per = EPI == ROWS_GLU ? NT / 2 : NT;
-  hipLaunchKernelGGL((gemm_rows16_kernel<MB, NT, EPI, HF>), dim3((tiles + per - 1) / per * p.S), dim3(GR_NW * 64), 0, st, p);
+  hipLaunchKernelGGL((gemm_rows16_kernel<MB, NT, EPI, DT>), dim3((tiles + per - 1) / per * p.S), dim3(GR_NW * 64), 0, st, p);
   return (int)hipGetLastError();
 }
 
 // Tiles of a workgroup: what one round of 256 of them needs, up to 4 (SwiGLU: 3 pairs; 64 rows of three pairs spill).  Outputs
 // that need more take several rounds of small workgroups, two to a CU (32000 x 4096, 18 rows, 2 / 3 / 4 / 6 tiles: 46.0 / 48.3 / 49.5 / 57.4).
-template <int MB, int EPI, bool HF>
+template <int MB, int EPI, int DT>
 int rows_dispatch(const RowsArgs& p, hipStream_t st) {
   if constexpr (EPI == ROWS_GLU) {
     const int pairs = p.N / 32;
-    if (pairs <= 256) return launch_rows<MB, 2, EPI, HF>(p, st);
+    if (pairs <= 256) return launch_rows<MB, 2, EPI, DT>(p, st);
     if constexpr (MB < 4)
-      if (pairs > 512 && pairs <= 768) return launch_rows<MB, 6, EPI, HF>(p, st);
-    return launch_rows<MB, 4, EPI, HF>(p, st);
+      if (pairs > 512 && pairs <= 768) return launch_rows<MB, 6, EPI, DT>(p, st);
+    return launch_rows<MB, 4, EPI, DT>(p, st);
   } else {
     const int tiles = p.N / 16 * p.S;
-    if (tiles <= 256) return launch_rows<MB, 1, EPI, HF>(p, st);
-    if (tiles <= 512 || (EPI == ROWS_OUT && tiles > 1024)) return launch_rows<MB, 2, EPI, HF>(p, st);
-    if (tiles <= 768) return launch_rows<MB, 3, EPI, HF>(p, st);
-    return launch_rows<MB, 4, EPI, HF>(p, st);
+    if (tiles <= 256) return launch_rows<MB, 1, EPI, DT>(p, st);
+    if (tiles <= 512 || (EPI == ROWS_OUT && tiles > 1024)) return launch_rows<MB, 2, EPI, DT>(p, st);
+    if (tiles <= 768) return launch_rows<MB, 3, EPI, DT>(p, st);
+    return launch_rows<MB, 4, EPI, DT>(p, st);
   }
 }
 
-template <int EPI, bool HF>
+template <int EPI, int DT>
 int rows_run(const RowsArgs& p, hipStream_t st) {
-  if (p.M <= 32) return rows_dispatch<2, EPI, HF>(p, st);
-  return p.M <= 48 ? rows_dispatch<3, EPI, HF>(p, st) : rows_dispatch<4, EPI, HF>(p, st);
+  if (p.M <= 32) return rows_dispatch<2, EPI, DT>(p, st);
+  return p.M <= 48 ? rows_dispatch<3, EPI, DT>(p, st) : rows_dispatch<4, EPI, DT>(p, st);
 }
 }  // namespace
 
@@ -224,8 +295,23 @@ extern "C" int edge_gemm_rows16(const void* x, const void* w, const void* bias, 
   if (edge_gemm_rows16_ok(M, N, K, S > 1 ? 3 : epi == 1 ? 1 : 0) == 0 || epi < 0 || epi > 3 || S < 1 || S > K / 64) return -2;
   if ((epi != 0 || h16) && S > 1) return -2;
   if (add != nullptr && (epi != 0 || S > 1)) return -2;
-  const RowsArgs p{(const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (const bf16_t*)add, out, M, N, K, S, epi >= 2 ? epi : 0};
-  if (S > 1) return rows_run<ROWS_PART, false>(p, st);
-  if (epi == 1) return h16 ? rows_run<ROWS_GLU, true>(p, st) : rows_run<ROWS_GLU, false>(p, st);
-  return h16 ? rows_run<ROWS_OUT, true>(p, st) : rows_run<ROWS_OUT, false>(p, st);
+  const RowsArgs p{(const bf16_t*)x, (const bf16_t*)w, (const bf16_t*)bias, (const bf16_t*)add, out, M, N, K, S, epi >= 2 ? epi : 0,
+                   nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  if (S > 1) return rows_run<ROWS_PART, DT_BF16>(p, st);
+  if (epi == 1) return h16 ? rows_run<ROWS_GLU, DT_FP16>(p, st) : rows_run<ROWS_GLU, DT_BF16>(p, st);
+  return h16 ? rows_run<ROWS_OUT, DT_FP16>(p, st) : rows_run<ROWS_OUT, DT_BF16>(p, st);
+}
+
+// int8: A [M, K] row-major with scales sa [M], w packed (K / 64 tiles a row block), scales sw [N], out bf16 [M, N] = gelu (act 2 / 3, 0:
+// none) of the rounded output, + add [M, N].  count not null: LLM.int8's outlier columns cols [*count] of x [M, K] bf16 against wt = W^T
+// [K, N], scaled by scb / 127, join the rounded product.  -2: not taken.
+extern "C" int edge_gemm_rows_i8(const void* A, const float* sa, const void* w, const float* sw, const void* bias, const void* add, void* out,
+                                 int M, int N, int K, int act, const void* x, const int* cols, const int* count, const void* wt,
+                                 const float* scb, hipStream_t st) {
+  if (K % 128 != 0 || edge_gemm_rows16_ok(M, N, K / 2, 0) == 0 || (act != 0 && act != 2 && act != 3) ||
+      ((uintptr_t)A | (uintptr_t)w) % 16 != 0 || (count != nullptr && (uintptr_t)wt % 4 != 0))
+    return -2;
+  const RowsArgs p{(const bf16_t*)A, (const bf16_t*)w, (const bf16_t*)bias, (const bf16_t*)add, out, M, N, K / 2, 1, act, sa, sw,
+                   (const bf16_t*)x, cols, count, (const int8_t*)wt, scb};
+  return rows_run<ROWS_OUT, DT_I8>(p, st);
 }

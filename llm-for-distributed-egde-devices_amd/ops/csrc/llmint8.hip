@@ -159,14 +159,23 @@ __global__ void __launch_bounds__(256) llmint8_outlier_kernel(bf16_t* __restrict
 // ---------------------------------------------------------------------------------- any rows
 // The same split for prefill-sized inputs (any M), still without a host round trip, and with no
 // cap: every column holding an |x| > threshold in any row goes to the 16-bit part, exactly the
-// bitsandbytes split.  Four launches, all of static shape:
-//   flags:   (K / 2048) x (M / 32) workgroups OR the column flags of their 32-row slab into a
-//            zeroed global bitmap (one atomic per 8 flagged columns, none for clean ones);
-//   compact: one wave turns the bitmap into the ordered column list + count (as in prep above);
-//   quant:   one workgroup per row: absmax over the kept columns, int8 with the outliers zeroed;
+// bitsandbytes split.  Launches of static shape:
+//   flags:   a bit a column: one workgroup per 64 columns, or, above FEW_ROWS rows, (K / 2048) x (M / 32) workgroups that OR the
+//            column flags of their 32-row slab into a zeroed bitmap (one atomic per 8 flagged columns, none for clean ones);
+//   quant:   one workgroup per row: absmax over the kept columns, int8 with the outliers zeroed; beside them one wave turns
+//            the bitmap into the ordered column list + count (as in prep above);
 //   outlier: 64 rows x 256 columns per workgroup: the rows' outlier values gathered from x into
 //            LDS 32 columns at a time, W^T rows read coalesced, fp32 sums, one rounding into out.
 constexpr int FR_ROWS = 32, OR_ROWS = 64, OR_COLS = 256, OR_J = 32;
+
+__device__ __forceinline__ uint32_t over(const uint4& u, float thr) {   // which of eight numbers are above the threshold
+  float v[8];
+  unpack8(u, v);
+  uint32_t bits = 0;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) bits |= (fabsf(v[j]) > thr ? 1u : 0u) << j;
+  return bits;
+}
 
 __global__ void __launch_bounds__(256) llmint8_flags_kernel(const bf16_t* __restrict__ x, int M, int K, float thr,
                                                             uint32_t* __restrict__ flags) {
@@ -174,20 +183,49 @@ __global__ void __launch_bounds__(256) llmint8_flags_kernel(const bf16_t* __rest
   if (c8 >= K) return;
   const int m0 = blockIdx.y * FR_ROWS, m1 = min(M, m0 + FR_ROWS);
   uint32_t bits = 0;
-  for (int m = m0; m < m1; ++m) {
-    float v[8];
-    unpack8(*reinterpret_cast<const uint4*>(x + (size_t)m * K + c8), v);
+  for (int m = m0; m < m1; m += 8) {                         // eight rows on their way (one by one 10 us for a slab)
+    uint4 u[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) bits |= (fabsf(v[j]) > thr ? 1u : 0u) << j;
+    for (int i = 0; i < 8; ++i) u[i] = *reinterpret_cast<const uint4*>(x + (size_t)min(m + i, m1 - 1) * K + c8);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) bits |= over(u[i], thr);
   }
   if (bits) atomicOr(&flags[c8 / 32], bits << (c8 % 32));
 }
 
-// one wave: ordered compaction of the flag bitmap (words = K / 32) into cols [count]; take = the
-// bitmap of the accepted columns (all of them here: cmax = K)
-__global__ void __launch_bounds__(64) llmint8_compact_kernel(const uint32_t* __restrict__ flags, int words, int cmax,
-                                                             uint32_t* __restrict__ take, int* __restrict__ cols,
-                                                             int* __restrict__ count) {
+// The same for up to FEW_ROWS rows without zeroed flags: a workgroup owns 64 columns of all rows (8 threads a row, 32 rows at a time) and
+// writes their two words.
+constexpr int FEW_ROWS = 1024;
+__global__ void __launch_bounds__(256) llmint8_flags_few_kernel(const bf16_t* __restrict__ x, int M, int K, float thr,
+                                                                uint32_t* __restrict__ flags) {
+  __shared__ uint32_t part[4][8];
+  const int cg = threadIdx.x & 7, rg = threadIdx.x >> 3, c8 = blockIdx.x * 64 + cg * 8, cc = min(c8, K - 8);
+  uint32_t bits = 0;
+  for (int m = rg; m < M; m += 32 * 4) {
+    uint4 u[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) u[i] = *reinterpret_cast<const uint4*>(x + (size_t)min(m + 32 * i, M - 1) * K + cc);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) bits |= over(u[i], thr);
+  }
+  bits |= lane_xor(bits, 8);
+  bits |= lane_xor(bits, 16);
+  bits |= lane_xor(bits, 32);
+  if ((threadIdx.x & 63) < 8) part[threadIdx.x >> 6][cg] = bits;
+  __syncthreads();
+  const int w = blockIdx.x * 2 + (int)threadIdx.x;
+  if (threadIdx.x < 2 && w < K / 32) {
+    uint32_t f = 0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      f |= (part[0][4 * threadIdx.x + i] | part[1][4 * threadIdx.x + i] | part[2][4 * threadIdx.x + i] | part[3][4 * threadIdx.x + i]) << (8 * i);
+    flags[w] = f;
+  }
+}
+
+// one wave: ordered compaction of the flag bitmap (words = K / 32) into cols [count]
+__device__ __forceinline__ void compact_flags(const uint32_t* __restrict__ flags, int words, int* __restrict__ cols,
+                                              int* __restrict__ count) {
   const int lane = threadIdx.x;
   int base = 0;
   for (int w0 = 0; w0 < words; w0 += 64) {
@@ -200,28 +238,27 @@ __global__ void __launch_bounds__(64) llmint8_compact_kernel(const uint32_t* __r
       if (lane >= o) incl += t;
     }
     int slot = base + incl - pc;
-    uint32_t acc = 0u, rest = f;
+    uint32_t rest = f;
     while (rest) {
-      const int b = __ffs(rest) - 1;
+      cols[slot++] = w * 32 + __ffs(rest) - 1;
       rest &= rest - 1;
-      if (slot < cmax) {
-        cols[slot] = w * 32 + b;
-        acc |= 1u << b;
-      }
-      ++slot;
     }
-    if (w < words) take[w] = acc;
     base += __shfl(incl, 63, 64);
   }
-  if (lane == 0) *count = min(base, cmax);
+  if (lane == 0) *count = base;
 }
 
-// one workgroup per row: sa[m] = absmax over the kept columns / 127, q[m] int8 (outliers zeroed)
+// one workgroup per row: sa[m] = absmax over the kept columns / 127, q[m] int8 (outliers zeroed); one more forms the column list
 __global__ void __launch_bounds__(256) llmint8_quant_rows_kernel(const bf16_t* __restrict__ x, int K,
                                                                  const uint32_t* __restrict__ take,
-                                                                 int8_t* __restrict__ q, float* __restrict__ sa) {
+                                                                 int8_t* __restrict__ q, float* __restrict__ sa, int M,
+                                                                 int* __restrict__ cols, int* __restrict__ count) {
   __shared__ float wmax[4];
   const int m = blockIdx.x, tid = threadIdx.x;
+  if (m == M) {
+    if (tid < 64) compact_flags(take, K / 32, cols, count);
+    return;
+  }
   const bf16_t* xr = x + (size_t)m * K;
   float am = 0.f;
   for (int c8 = tid * 8; c8 < K; c8 += 256 * 8) {
@@ -320,18 +357,20 @@ __global__ void __launch_bounds__(256) llmint8_clear_kernel(uint32_t* flags, int
 }
 
 // Any-rows preparation: x bf16 [M, K] (K % 32 == 0) -> q int8 [M, K] (outlier columns zeroed),
-// sa [M], cols [K] (first *count), count [1]; flags / take: scratch of K / 32 words each.
+// sa [M], cols [K] (first *count), count [1]; flags: scratch of K / 32 words.
 extern "C" int edge_llmint8_prep_rows(const void* x, int M, int K, float thr, void* q, float* sa, int* cols, int* count,
-                                      uint32_t* flags, uint32_t* take, hipStream_t st) {
+                                      uint32_t* flags, hipStream_t st) {
   if (M <= 0 || K % 32 != 0 || K <= 0) return -2;
   const int words = K / 32;
-  hipLaunchKernelGGL(llmint8_clear_kernel, dim3((words + 255) / 256), dim3(256), 0, st, flags, words);
-  hipLaunchKernelGGL(llmint8_flags_kernel, dim3((K + 2047) / 2048, (M + FR_ROWS - 1) / FR_ROWS), dim3(256), 0, st,
-                     (const bf16_t*)x, M, K, thr, flags);
-  hipLaunchKernelGGL(llmint8_compact_kernel, dim3(1), dim3(64), 0, st, (const uint32_t*)flags, words, K, take, cols,
-                     count);
-  hipLaunchKernelGGL(llmint8_quant_rows_kernel, dim3(M), dim3(256), 0, st, (const bf16_t*)x, K,
-                     (const uint32_t*)take, (int8_t*)q, sa);
+  if (M <= FEW_ROWS) {
+    hipLaunchKernelGGL(llmint8_flags_few_kernel, dim3((K + 63) / 64), dim3(256), 0, st, (const bf16_t*)x, M, K, thr, flags);
+  } else {
+    hipLaunchKernelGGL(llmint8_clear_kernel, dim3((words + 255) / 256), dim3(256), 0, st, flags, words);
+    hipLaunchKernelGGL(llmint8_flags_kernel, dim3((K + 2047) / 2048, (M + FR_ROWS - 1) / FR_ROWS), dim3(256), 0, st,
+                       (const bf16_t*)x, M, K, thr, flags);
+  }
+  hipLaunchKernelGGL(llmint8_quant_rows_kernel, dim3(M + 1), dim3(256), 0, st, (const bf16_t*)x, K, (const uint32_t*)flags,
+                     (int8_t*)q, sa, M, cols, count);
   return (int)hipGetLastError();
 }
 

@@ -22,7 +22,7 @@ import torch.nn as nn
 
 from .. import ops
 from ..ops import _ref
-from ..models.layers import GroupQuantBF16, Linear, PartialSum, PendingLN, PendingNorm, QAct
+from ..models.layers import GroupQuantBF16, Linear, PartialSum, PendingLN, PendingNorm, QAct, unwatched
 
 # Decode MLP policy (A/B on MI355X, Llama-2-7B, profiles/bench_ops_r1_gemv16.json): the gate_up
 # GEMV quantises silu(g) * u in its own epilogue (8 tiles = 64 features per workgroup) for every
@@ -321,7 +321,15 @@ class LLMInt8Linear(nn.Module):
                 and x.is_cuda and ops.gpu_path(x) and self._device_ok() and self.ONE_LAUNCH \
                 and self.in_features <= 4096:
             return self._forward(x, act=self._ACT[act])
+        if isinstance(x, torch.Tensor) and self._rows_ok(x) and unwatched(self):
+            return self._forward(x, act=self._ACT[act])
         return None
+
+    def _rows_ok(self, x: torch.Tensor) -> bool:
+        """17 to 64 bf16 rows: product, outlier columns and activation or addend in one launch (gemm_rows16.hip)."""
+        M = x.numel() // self.in_features
+        return 17 <= M <= 64 and x.dtype == torch.bfloat16 and x.is_cuda and ops.gpu_path(x) and self._device_ok() and \
+            self.in_features % 128 == 0 and ops.ext().gemm_rows16_ok(M, self.out_features, self.in_features // 2, 0)
 
     def pair_ok(self, up: bool = False) -> bool:
         """Whether this projection of one row can share a launch with another part of its block (decode_pair_i8.hip); up: as
@@ -396,6 +404,14 @@ class LLMInt8Linear(nn.Module):
                 C.llmint8_outlier(out, xo, cols, count, weight_t, self.SCB)
             else:
                 q, sa, cols, count = C.llmint8_prep_rows(x2, self.threshold)
+                if x2.shape[0] <= 64:
+                    fuse = add is not None and not act and _epilogue_row(add, x2)
+                    out = C.llmint8_rows(q, sa, x2, cols, count, self.w_packed, w_deq, self.bias, weight_t, self.SCB, N, act,
+                                         add.reshape(-1, N) if fuse else None)
+                    if out is not None:
+                        return out.view(*shp, N) if fuse else plus(out.view(*shp, N))
+                if act:
+                    return None
                 out = ops.w8a8_linear(q, sa, self.w_packed, w_deq, self.bias, N, K)
                 C.llmint8_outlier_rows(out, x2, cols, count, weight_t, self.SCB)
             return plus(out.view(*shp, N))
