@@ -200,9 +200,14 @@ class Linear(nn.Module):
             return self.forward_norm(x)
         if isinstance(x, QAct):
             x = (x.q.float() * x.scale[..., None]).to(self.weight.dtype)
-        y = None if self.split_k_out else self.rows16(x, add=add)
-        if y is not None:
-            return y
+        n, K = x.numel(), self.in_features
+        if n > ops.BF16_RING_MAX_ROWS * K:              # prompts: no kernel of few rows is looked for (25 times a step of 4 layers)
+            y = nn.functional.linear(x, self.weight, self.bias)
+            return y if add is None else y + add.reshape(y.shape)
+        if 17 * K <= n <= 64 * K and not self.split_k_out:
+            y = self.rows16(x, add=add)
+            if y is not None:
+                return y
         wp = self.decode_weight(x)
         if self.split_k_out and wp is not None and add is None:
             K = x.shape[-1]
