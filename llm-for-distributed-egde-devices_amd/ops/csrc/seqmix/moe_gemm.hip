@@ -14,7 +14,8 @@
 // 758 -> 127 us (610 TFLOP/s); 7680 x 3 of 32, 2048 -> 3072, 1679 -> 664 us (874); 512 x 4 of 32, 2048 -> 2048,
 // 1369 -> 169 us, where the experts' 805 MB (4.8 TB/s) are the bound.  At 128-row tiles the bound is the LDS: 64 B per clock and
 // CU come in and 128 are read at the full MFMA rate (tile_rows says what 256-row tiles change); 128 x 256 tiles gained 3-6 %
-// from 2048 columns on and lost below, deeper rings with one workgroup of 128 x 128 per CU lose 40 %.
+// from 2048 columns on and lost below, deeper rings with one workgroup of 128 x 128 per CU lose 40 %; a third stage for the
+// weights alone still leaves two workgroups a CU and gains 2-15 % (edge_sm_moe_gemm).
 #include "seqmix_common.h"
 
 namespace {
@@ -99,16 +100,19 @@ __device__ __forceinline__ void pin(v4i (&f)[N]) {
 //    (fp32; the unfused form rounds both halves to bf16 first).
 //  * blockIdx -> tile: each XCD takes a contiguous range of the (real) tiles, walked in groups of four row tiles
 //    column by column, so neighbours in an L2 share an expert's weights.
-template <int BM, int BN, int WM, int WN, int R, int ACT, bool GATHER>
+template <int BM, int BN, int WM, int WN, int RA, int RW, int ACT, bool GATHER>
 __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
                                                                   const int* __restrict__ rows, const int* __restrict__ tiles,
                                                                   bf16_t* __restrict__ out, int top, int N, int NW, int K,
                                                                   int grid_n, const float* __restrict__ row_w, float limit, int spread) {
   constexpr bool GLU = ACT == ACT_GLU_CLAMP || ACT == ACT_GLU_SILU;
-  constexpr int NWV = WM * WN, AP = BM / 8, BP = BN / 8, PIECES = AP + BP, PPW = PIECES / NWV, STAGE = PIECES * 1024;
+  constexpr int NWV = WM * WN, AP = BM / 8, BP = BN / 8, PA = AP / NWV, PB = BP / NWV;   // pieces of a stage, of a wave
   constexpr int MI = BM / WM / 16, NJ = BN / WN / 16;
-  static_assert(PIECES % NWV == 0 && (!GLU || NJ % 2 == 0) && R * STAGE <= 160 * 1024, "tile shape");
-  __shared__ __attribute__((aligned(1024))) int8_t ring[R * STAGE];
+  constexpr int RS = RA < RW ? RA : RW, DEEP = RA > RW ? PA : RW > RA ? PB : 0;           // pieces of the operand one stage further ahead
+  static_assert(AP % NWV == 0 && BP % NWV == 0 && (!GLU || NJ % 2 == 0) && (RA - RW) * (RA - RW) <= 1, "tile shape");
+  static_assert((RA * AP + RW * BP) * 1024 <= 160 * 1024, "LDS");
+  __shared__ __attribute__((aligned(1024))) int8_t ring[(RA * AP + RW * BP) * 1024];
+  constexpr int W0 = RA * AP * 1024;                         // the weights' stages
 
   const int nwg = tiles[0] * grid_n, orig = blockIdx.x;
   if (orig >= nwg) return;
@@ -124,9 +128,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   const int wm = wave / WN, wn = wave % WN, KT = K / 64;
   constexpr int FN = GLU ? BN / 2 : BN;                      // output columns of a block tile
   // this wave's DMA pieces p = wave + NWV i: activation rows 8 p .. (p < AP), or weight rows
-  const char* src[PPW];
+  const char* src[PA + PB];
 #pragma unroll
-  for (int i = 0; i < PPW; ++i) {
+  for (int i = 0; i < PA + PB; ++i) {
     const int p = wave + NWV * i, r = (p < AP ? p : p - AP) * 8 + (lane >> 3);
     const int ck = ((lane & 7) ^ (r & 7)) * 16;
     size_t row;
@@ -152,19 +156,24 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   // spread: column blocks and experts start at different k and go round.  In step, every workgroup reads the same 128 bytes
   // of rows 2 K bytes apart, which lie in few memory channels
   const int k0 = spread ? (tile.x * 7 + bn * 5) % KT : 0;
-  auto issue = [&](int st) {
+  auto issue = [&](int st, bool weights) {
     const int kt = min(st, KT - 1) + k0;
     const size_t ko = (size_t)(kt < KT ? kt : kt - KT) * 128;
-    int8_t* slot = ring + (st % R) * STAGE + wave * 1024;
+    int8_t* slot = ring + (weights ? W0 + (st % RW) * (BP * 1024) : (st % RA) * (AP * 1024)) + wave * 1024;
 #pragma unroll
-    for (int i = 0; i < PPW; ++i) glds16(src[i] + ko, slot + NWV * i * 1024);
+    for (int i = 0; i < (weights ? PB : PA); ++i) glds16(src[weights ? PA + i : i] + ko, slot + NWV * i * 1024);
+  };
+  // the operand that is further ahead last: its pieces may still be on their way when the other's have landed
+  auto issue_both = [&](int st) {
+    issue(RA > RW ? st + RW : st + RA, RA > RW);
+    issue(RA > RW ? st + RA : st + RW, RA <= RW);
   };
   // fragment (16 rows x 32 k of step ks): row lane & 15, chunk 4 ks + (lane >> 4)
   const uint32_t fo = lds_off(ring) + (lane & 15) * 128 + (((lane >> 4) ^ (lane & 7)) << 4);
   auto read = [&](int st, int ks, v4i (&fa)[MI], v4i (&fw)[NJ]) {
-    const uint32_t b = (fo ^ (ks << 6)) + (st % R) * STAGE;
-    lds_frags<0, MI>(b + wm * (MI * 2048), fa);
-    lds_frags<0, NJ>(b + AP * 1024 + wn * (NJ * 2048), fw);
+    const uint32_t b = fo ^ (ks << 6);
+    lds_frags<0, MI>(b + (st % RA) * (AP * 1024) + wm * (MI * 2048), fa);
+    lds_frags<0, NJ>(b + W0 + (st % RW) * (BP * 1024) + wn * (NJ * 2048), fw);
   };
   v4f acc[MI][NJ];
 #pragma unroll
@@ -189,9 +198,13 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   };
 
 #pragma unroll
-  for (int st = 0; st < R; ++st) issue(st);
+  for (int st = 0; st < RS; ++st) {
+    issue(st, RA > RW);
+    issue(st, RA <= RW);
+  }
+  if constexpr (DEEP != 0) issue(RS, RW > RA);
   v4i a0[MI], w0[NJ], a1[MI], w1[NJ];
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 1) * PPW) : "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 1) * (PA + PB) + DEEP) : "memory");
   __builtin_amdgcn_s_barrier();
   read(0, 0, a0, w0);
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -201,9 +214,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
     pin_acc();
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     if (s + 1 < KT) {
-      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((R - 2) * PPW) : "memory");   // own pieces of stage s + 1
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((RS - 2) * (PA + PB) + DEEP) : "memory");   // own pieces of stage s + 1
       __builtin_amdgcn_s_barrier();                          // stage s + 1 is there, stage s has been read by all
-      issue(s + R);
+      issue_both(s);
       read(s + 1, 0, a0, w0);
     }
     mma(a1, w1);
@@ -240,20 +253,20 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   }
 }
 
-template <int BM, int BN, int WM, int WN, int R>
+template <int BM, int BN, int WM, int WN, int RA, int RW>
 int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* rows, const int* tiles, void* y, void* out,
                 int max_tiles, int top, int W, int ff, int act, const float* row_w, float limit, int spread, hipStream_t st) {
   const dim3 blk(64 * WM * WN);
   const int up = act == ACT_RELU2 ? 1 : 2, fn = act == ACT_RELU2 ? BN : BN / 2;
   const int g1 = (ff + fn - 1) / fn, g2 = (W + BN - 1) / BN;
 #define MOE_FIRST(ACT)                                                                                                     \
-  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, ACT, true>), dim3(max_tiles * g1), blk, 0, st, (const bf16_t*)h,  \
+  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, RA, RW, ACT, true>), dim3(max_tiles * g1), blk, 0, st, (const bf16_t*)h,  \
                      (const bf16_t*)w_gu, rows, tiles, (bf16_t*)y, top, ff, up * ff, W, g1, row_w, limit, spread)
   if (act == ACT_GLU_CLAMP) MOE_FIRST(ACT_GLU_CLAMP);
   else if (act == ACT_GLU_SILU) MOE_FIRST(ACT_GLU_SILU);
   else MOE_FIRST(ACT_RELU2);
 #undef MOE_FIRST
-  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, ACT_NONE, false>), dim3(max_tiles * g2), blk, 0, st, (const bf16_t*)y,
+  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, RA, RW, ACT_NONE, false>), dim3(max_tiles * g2), blk, 0, st, (const bf16_t*)y,
                      (const bf16_t*)w_down, rows, tiles, (bf16_t*)out, top, W, W, ff, g2, nullptr, 0.f, spread);
   return (int)hipGetLastError();
 }
@@ -273,7 +286,7 @@ double expected_tiles(double R, int E, int BM) {
 // hidden behind that, or (256 rows) bound it from below.
 double tile_us(int BM, double R, int E, int W, int ff, int up) {
   //                              us a stage, a start, both launches, TB/s, whole rounds' part
-  static const double fit[3][5] = {{0.621, 4.35, 5.4, 9.36, 0.266}, {0.991, 7.2, 3.53, 13.3, 0.429}, {1.64, 16.1, 5.69, 4.04, 0.585}};
+  static const double fit[3][5] = {{0.621, 4.35, 5.4, 9.36, 0.266}, {0.96, 7.2, 3.53, 13.3, 0.48}, {1.64, 16.1, 5.69, 4.04, 0.585}};
   const double* p = fit[BM == 64 ? 0 : BM == 128 ? 1 : 2];
   const int BN = BM == 256 ? 256 : 128, slots = BM == 256 ? 256 : 512;
   const double tiles = expected_tiles(R, E, BM);
@@ -325,10 +338,19 @@ int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void
   // 3000 476 / 474; with more rows it costs 2 % (7680 tokens of 3, ff 3072: 779 / 798)
   const int spread = R <= E * 512;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(SORT_NT), 0, st, idx, R, E, BM, rows, tiles);
-  if (BM == 256) return launch_pair<256, 256, 2, 4, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  if (BM == 128) return launch_pair<128, 128, 2, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  if (BM == 64) return launch_pair<64, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  return launch_pair<32, 128, 1, 4, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  // The weights of a stage come from HBM, the rows from an L2: with a ring of three stages for the weights and two for the rows (80 KB,
+  // two workgroups of 128 x 128 a CU, or the LDS' whole 160 KB of one of 256 x 256) the weights are asked for a stage earlier and the
+  // rows' half of the LDS is not paid for.  us, two and two against two and three stages, 128 rows: 8 experts of 2048 -> 4096 (gated),
+  // 100 rows an expert 128 / 111, 250 209 / 191; 32 of 1024 -> 1024, 512 195 / 181; 16 of 1024 -> 1024, 250 77 / 71; 32 of 2048 ->
+  // 3072 (relu2), 60 181 / 170; where the experts' bytes are the bound equal (32 of 2048 -> 2048, 60 174 / 174), at the worst 3 % more
+  // (24 of 1536 -> 1536, 510 205 / 211).  256 rows: relu2, 2048 -> 3072, 510 rows 568 / 545, 720 707 / 673, 1000 916 / 878; gated, 720
+  // 632 / 619 (64 of 1024 -> 1536), 1000 912 / 904, but 375 (spread starts) 406 / 412 and 382 / 400: those keep two and two.
+  if (BM == 256 && spread && act != ACT_RELU2)
+    return launch_pair<256, 256, 2, 4, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  if (BM == 256) return launch_pair<256, 256, 2, 4, 2, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  if (BM == 128) return launch_pair<128, 128, 2, 2, 2, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  if (BM == 64) return launch_pair<64, 128, 1, 4, 3, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+  return launch_pair<32, 128, 1, 4, 3, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
 }
 
 }  // extern "C"

@@ -71,6 +71,24 @@ def test_grouped_experts_against_float64(T, top, E, W, ff, act, every_size):
 
 
 @gpu
+@pytest.mark.parametrize("T,top,E,W,ff,act", [
+    (400, 2, 8, 64, 1024, "glu_clamp"),          # 128-row tiles: one k step in the first product
+    (400, 2, 8, 1024, 64, "silu_glu"),           # one in the second
+    (400, 2, 8, 64, 1024, "relu2"),
+    (3840, 3, 48, 1024, 192, "glu_clamp"),       # three: every stage of the weights' ring once
+    (3840, 3, 48, 192, 1024, "relu2"),
+    (3200, 2, 32, 1024, 1024, "silu_glu"),       # 256-row tiles, gated, spread starts: equal rings
+    (3840, 2, 32, 1024, 1024, "relu2"),          # unequal ones: squared units
+    (2960, 2, 8, 1536, 1024, "glu_clamp")])      # and starts in step
+def test_rings_of_unequal_depth_against_float64(T, top, E, W, ff, act):
+    h, idx, w_gu, w_down, in_w = inputs(T, top, E, W, ff, act, T)
+    assert seqmix.moe_grouped(h, idx, w_gu, w_down, act, in_w)
+    got = seqmix.moe_experts(h, idx, w_gu, w_down, 1.5, act, in_w).cpu().double()
+    want = reference(h, idx, w_gu, w_down, act, 1.5, in_w)
+    assert ((got - want).norm(dim=-1) / want.norm(dim=-1).clamp_min(1e-3)).max() < 4 * TOL
+
+
+@gpu
 def test_small_experts_of_small_steps_run_by_rows():
     """Pairs times an expert's numbers on both sides of MOE_MFMA_WORK, and a step of MOE_GEMM_MIN tokens: the same result."""
     for T, W, ff, grouped in ((12, 256, 128, False), (42, 256, 128, False), (43, 256, 128, True), (64, 64, 64, True), (63, 64, 64, False)):
