@@ -671,10 +671,12 @@ def quant_per_group(x):
 # --------------------------------------------------------------------------- sampling / misc
 
 
-def _logits32(logits):
-    """The sampler reads bf16 or fp32 logits; fp16 logits (fp16 agents) are widened to fp32 first,
-    as HF's generate does before its logits processors."""
-    return logits.float() if logits.dtype == torch.float16 else logits
+def _sampler_rows(logits):
+    """The sampler widens 16-bit logits as it reads them (HF's generate does so before its logits processors); fp16 rows that
+    its 16-byte loads cannot take in place, with gaps or off their boundary, are widened first."""
+    if logits.dtype == torch.float16 and not (logits.is_contiguous() and logits.data_ptr() % 16 == 0):
+        return logits.float()
+    return logits
 
 
 def sample(logits, seen, temperature, top_k, top_p, repetition_penalty, rng: torch.Tensor,
@@ -682,14 +684,14 @@ def sample(logits, seen, temperature, top_k, top_p, repetition_penalty, rng: tor
     """Fused sampler. ``rng`` = int32 tensor [seed, step] on the logits' device (the step is
     read on device so the launch is graph-capturable)."""
     if _gpu(logits):
-        logits = _logits32(logits)
-        out = ext().sample(logits, seen, float(temperature), int(top_k or 0), float(top_p if top_p is not None else 1.0),
+        out = ext().sample(_sampler_rows(logits), seen, float(temperature), int(top_k or 0), float(top_p if top_p is not None else 1.0),
                            float(repetition_penalty), bool(do_sample), rng)
         if out.numel() > 0 or logits.shape[0] == 0:
             return out
         # top-p without top-k (or top-k > 1024): needs a full sort -> torch path on device
         seed, step = (int(v) for v in rng.tolist())
-        tok = _ref.sample(logits, seen, temperature, top_k, top_p, repetition_penalty, seed, step, do_sample)
+        full = logits.float() if logits.dtype == torch.float16 else logits
+        tok = _ref.sample(full, seen, temperature, top_k, top_p, repetition_penalty, seed, step, do_sample)
         if seen is not None:
             seen.scatter_(1, tok[:, None], 1)
         return tok
@@ -739,7 +741,7 @@ def sample_shard(logits, seen, temperature, top_k, top_p, repetition_penalty, rn
     mode = shard_mode(temperature, top_k, top_p, V, do_sample)
     assert mode >= 0, "sampling configuration does not shard over the vocabulary"
     if _gpu(logits):
-        r = ext().sample_shard(_logits32(logits), seen, float(temperature), int(top_k or 0),
+        r = ext().sample_shard(_sampler_rows(logits), seen, float(temperature), int(top_k or 0),
                                float(top_p if top_p is not None else 1.0), float(repetition_penalty),
                                bool(do_sample), rng, int(v0), int(V))
         return tuple(r) if mode == 2 else (r[0],)
@@ -823,8 +825,7 @@ def sample_advance(logits, seen, temperature, top_k, top_p, repetition_penalty, 
     sampler's last launch (one kernel boundary fewer per decode step).  ``ctr``: int32 [1] zero
     buffer the kernel uses as an arrival counter (it stays zero between calls).  Returns nxt."""
     if _gpu(logits) and FUSE_ADVANCE:
-        logits = _logits32(logits)
-        nxt = ext().sample_advance(logits, seen, float(temperature), int(top_k or 0),
+        nxt = ext().sample_advance(_sampler_rows(logits), seen, float(temperature), int(top_k or 0),
                                    float(top_p if top_p is not None else 1.0), float(repetition_penalty),
                                    bool(do_sample), rng, tok, out, step, pos, seq_lens, ctr)
         if nxt.numel() > 0 or logits.shape[0] == 0:

@@ -62,18 +62,18 @@ int edge_prefill_attn(const void* q, const void* k_cache, const void* v_cache, i
                       int causal, int h16, hipStream_t st);
 int edge_w8a8_gemm(const void* A, const float* sa, const void* Wp, const float* sw, const void* bias, void* out,
                    float* os, int M, int N, int K, int KT, int a_mode, int Mpad, int epi, hipStream_t st);
-int edge_sample(const void* logits, int is_bf16, uint8_t* seen, int B, int V, float temperature,
+int edge_sample(const void* logits, int dt, uint8_t* seen, int B, int V, float temperature,
                 float inv_temperature, float penalty, int top_k, float top_p, int do_sample, const int* rng,
                 int64_t* out_tok, void* workspace, hipStream_t st);
 size_t edge_sample_workspace(int B, int V);
 int edge_sample_shard_mode(int do_sample, float temperature, int top_k, float top_p, int V);
 int edge_sample_shard_chunks(int Vs, int V);
-int edge_sample_shard(const void* logits, int is_bf16, const uint8_t* seen, int B, int Vs, int v0, int V,
+int edge_sample_shard(const void* logits, int dt, const uint8_t* seen, int B, int Vs, int v0, int V,
                       float temperature, float inv_temperature, float penalty, int top_k, float top_p, int do_sample,
                       const int* rng, uint64_t* pc, uint32_t* pthr, hipStream_t st);
 int edge_sample_merge(const uint64_t* pc, const uint32_t* pthr, int B, int C, int V, float temperature, int top_k,
                       float top_p, int do_sample, const int* rng, int64_t* out_tok, hipStream_t st);
-int edge_sample_advance(const void* logits, int is_bf16, uint8_t* seen, int B, int V, float temperature,
+int edge_sample_advance(const void* logits, int dt, uint8_t* seen, int B, int V, float temperature,
                         float inv_temperature, float penalty, int top_k, float top_p, int do_sample, int* rng,
                         int64_t* out_tok, void* workspace, int64_t* tok, int64_t* out, int64_t out_sb, int ncols,
                         int64_t* step, int* pos, int* lens, int* ctr, hipStream_t st);
@@ -1471,15 +1471,15 @@ at::Tensor sample(const at::Tensor& logits, const std::optional<at::Tensor>& see
                   int64_t top_k, double top_p, double penalty, bool do_sample, const at::Tensor& rng) {
   DEVICE_GUARD(logits);
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && logits.dim() == 2);
-  const bool bf = logits.scalar_type() == at::kBFloat16;
-  TORCH_CHECK(bf || logits.scalar_type() == at::kFloat);
+  const int dt = logits.scalar_type() == at::kBFloat16 ? 1 : logits.scalar_type() == at::kHalf ? 2 : 0;
+  TORCH_CHECK(dt || logits.scalar_type() == at::kFloat);
   need(rng, at::kInt, "rng");
   const int64_t B = logits.size(0), V = logits.size(1);
   if (seen) { need(*seen, at::kByte, "seen"); TORCH_CHECK(seen->sizes() == logits.sizes()); }
   auto out = at::empty({B}, logits.options().dtype(at::kLong));
   auto ws = at::empty({(int64_t)edge_sample_workspace((int)B, (int)V)}, logits.options().dtype(at::kByte));
   const double inv_t = temperature > 0 ? 1.0 / temperature : 1.0;
-  const int rc = edge_sample(logits.data_ptr(), bf, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V,
+  const int rc = edge_sample(logits.data_ptr(), dt, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V,
                              (float)temperature, (float)inv_t, (float)penalty, (int)top_k, (float)top_p, do_sample,
                              rng.data_ptr<int>(), out.data_ptr<int64_t>(), ws.data_ptr(), stream());
   if (rc == -5) return at::Tensor();
@@ -1498,8 +1498,8 @@ std::optional<std::tuple<at::Tensor, at::Tensor>> sample_shard(const at::Tensor&
                                                                int64_t V) {
   DEVICE_GUARD(logits);
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && logits.dim() == 2);
-  const bool bf = logits.scalar_type() == at::kBFloat16;
-  TORCH_CHECK(bf || logits.scalar_type() == at::kFloat, "sample_shard: bf16 or fp32 logits");
+  const int dt = logits.scalar_type() == at::kBFloat16 ? 1 : logits.scalar_type() == at::kHalf ? 2 : 0;
+  TORCH_CHECK(dt || logits.scalar_type() == at::kFloat, "sample_shard: bf16, fp16 or fp32 logits");
   need(rng, at::kInt, "rng");
   const int64_t B = logits.size(0), Vs = logits.size(1);
   TORCH_CHECK(v0 >= 0 && v0 + Vs <= V, "shard outside the vocabulary");
@@ -1510,7 +1510,7 @@ std::optional<std::tuple<at::Tensor, at::Tensor>> sample_shard(const at::Tensor&
   auto pc = at::empty({B, mode == 2 ? C * 128 : C}, logits.options().dtype(at::kLong));
   auto pthr = at::empty({B, mode == 2 ? C : 0}, logits.options().dtype(at::kInt));
   const double inv_t = temperature > 0 ? 1.0 / temperature : 1.0;
-  check(edge_sample_shard(logits.data_ptr(), bf, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)Vs, (int)v0,
+  check(edge_sample_shard(logits.data_ptr(), dt, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)Vs, (int)v0,
                           (int)V, (float)temperature, (float)inv_t, (float)penalty, (int)top_k, (float)top_p, do_sample,
                           rng.data_ptr<int>(), reinterpret_cast<uint64_t*>(pc.data_ptr<int64_t>()),
                           mode == 2 ? reinterpret_cast<uint32_t*>(pthr.data_ptr<int>()) : nullptr, stream()),
@@ -1584,8 +1584,8 @@ at::Tensor sample_advance(const at::Tensor& logits, const std::optional<at::Tens
                           at::Tensor& out, at::Tensor& step, at::Tensor& pos, at::Tensor& seq_lens, at::Tensor& ctr) {
   DEVICE_GUARD(logits);
   TORCH_CHECK(logits.is_cuda() && logits.is_contiguous() && logits.dim() == 2);
-  const bool bf = logits.scalar_type() == at::kBFloat16;
-  TORCH_CHECK(bf || logits.scalar_type() == at::kFloat);
+  const int dt = logits.scalar_type() == at::kBFloat16 ? 1 : logits.scalar_type() == at::kHalf ? 2 : 0;
+  TORCH_CHECK(dt || logits.scalar_type() == at::kFloat);
   need(rng, at::kInt, "rng");
   need(tok, at::kLong, "tok");
   need(out, at::kLong, "out");
@@ -1603,7 +1603,7 @@ at::Tensor sample_advance(const at::Tensor& logits, const std::optional<at::Tens
   auto nxt = at::empty({B}, logits.options().dtype(at::kLong));
   auto ws = at::empty({(int64_t)edge_sample_workspace((int)B, (int)V)}, logits.options().dtype(at::kByte));
   const double inv_t = temperature > 0 ? 1.0 / temperature : 1.0;
-  const int rc = edge_sample_advance(logits.data_ptr(), bf, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V,
+  const int rc = edge_sample_advance(logits.data_ptr(), dt, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V,
                                      (float)temperature, (float)inv_t, (float)penalty, (int)top_k, (float)top_p,
                                      do_sample, rng.data_ptr<int>(), nxt.data_ptr<int64_t>(), ws.data_ptr(),
                                      tok.data_ptr<int64_t>(), out.data_ptr<int64_t>(), out.stride(0), (int)out.size(1),

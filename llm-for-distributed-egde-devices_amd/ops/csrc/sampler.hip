@@ -106,10 +106,30 @@ __device__ __forceinline__ uint32_t probe(uint32_t lo, uint32_t hi, int it) {
   return lo + (uint32_t)(((uint64_t)hi - lo + 1) >> 1);
 }
 
-template <bool BF16>
+// Scores as the LM head wrote them, widened where they are read (a widening launch before was 4.6 us a step of 50304 fp16 scores)
+enum { LG_FP32 = 0, LG_BF16 = 1, LG_FP16 = 2 };
+
+template <int DT>
+__device__ __forceinline__ void scores8(const void* lg, size_t e, float (&v)[8]) {
+  if constexpr (DT == LG_BF16) {
+    unpack8(*reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(lg) + e), v);
+  } else if constexpr (DT == LG_FP16) {
+    typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+    const v8h h = *reinterpret_cast<const v8h*>(reinterpret_cast<const _Float16*>(lg) + e);
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = (float)h[u];
+  } else {
+    const float4 a = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lg) + e);
+    const float4 b = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lg) + e + 4);
+    v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
+  }
+}
+
+template <int DT>
 __device__ __forceinline__ float proc(const void* lg, const uint8_t* seen, size_t base, int i, float inv_t, float pen) {
   float s;
-  if constexpr (BF16) s = bf2f(reinterpret_cast<const bf16_t*>(lg)[base + i]);
+  if constexpr (DT == LG_BF16) s = bf2f(reinterpret_cast<const bf16_t*>(lg)[base + i]);
+  else if constexpr (DT == LG_FP16) s = (float)reinterpret_cast<const _Float16*>(lg)[base + i];
   else s = reinterpret_cast<const float*>(lg)[base + i];
   if (seen != nullptr && seen[base + i]) s = s < 0.f ? s * pen : s / pen;
   return s * inv_t;
@@ -319,7 +339,7 @@ __device__ __forceinline__ void run_map(bool vec, int tid, int ept, int& o0, int
   ostr = vec ? 1 : NT;
 }
 
-template <bool BF16, int EPT>
+template <int DT, int EPT>
 __device__ __forceinline__ void load_run(const void* lg, const uint8_t* seen, size_t base, int c0, int o0, int ostr,
                                          int nvalid, bool vec, float inv_t, float pen, float (&sv)[EPT]) {
   static_assert(EPT % 8 == 0, "runs of whole 8-element groups");
@@ -328,13 +348,7 @@ __device__ __forceinline__ void load_run(const void* lg, const uint8_t* seen, si
 #pragma unroll
     for (int q = 0; q < EPT / 8; ++q) {
       float v[8];
-      if constexpr (BF16) {
-        unpack8(*reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(lg) + e0 + 8 * q), v);
-      } else {
-        const float4 a = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lg) + e0 + 8 * q);
-        const float4 b = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(lg) + e0 + 8 * q + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-      }
+      scores8<DT>(lg, e0 + 8 * q, v);
       const uint64_t sn = seen != nullptr ? *reinterpret_cast<const uint64_t*>(seen + e0 + 8 * q) : 0ull;
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
@@ -346,7 +360,7 @@ __device__ __forceinline__ void load_run(const void* lg, const uint8_t* seen, si
   } else {
 #pragma unroll
     for (int j = 0; j < EPT; ++j)
-      sv[j] = o0 + j * ostr < nvalid ? proc<BF16>(lg, seen, base, c0 + o0 + j * ostr, inv_t, pen) : -INFINITY;
+      sv[j] = o0 + j * ostr < nvalid ? proc<DT>(lg, seen, base, c0 + o0 + j * ostr, inv_t, pen) : -INFINITY;
   }
 }
 
@@ -354,7 +368,7 @@ __device__ __forceinline__ void load_run(const void* lg, const uint8_t* seen, si
 // Per-chunk best composite (value, then lower id) of the processed (MODE 1: + Gumbel noise)
 // scores -> pc[row*C + c].  v0: global token id of column 0 (a vocab shard of the LM head: the
 // noise and the composite carry global ids, so shard results merge exactly).
-template <bool BF16, int MODE, int EPT>
+template <int DT, int MODE, int EPT>
 __global__ void __launch_bounds__(NT) argmax_chunk_kernel(const void* __restrict__ logits,
                                                           const uint8_t* __restrict__ seen, int V, int C, float inv_t,
                                                           float pen, const int* __restrict__ rng,
@@ -368,7 +382,7 @@ __global__ void __launch_bounds__(NT) argmax_chunk_kernel(const void* __restrict
   int o0, ostr;
   run_map(vec != 0, (int)threadIdx.x, EPT, o0, ostr);
   float sv[EPT];
-  load_run<BF16, EPT>(logits, seen, base, c0, o0, ostr, nvalid, vec != 0, inv_t, pen, sv);
+  load_run<DT, EPT>(logits, seen, base, c0, o0, ostr, nvalid, vec != 0, inv_t, pen, sv);
   float bv = -INFINITY;
   int bi = 0x7fffffff;
 #pragma unroll
@@ -388,7 +402,7 @@ __global__ void __launch_bounds__(NT) argmax_chunk_kernel(const void* __restrict
 // pthr[row*C + c] = threshold key.  Thread t holds EPT elements of the chunk in ``run_map``'s layout:
 // [t * EPT, (t + 1) * EPT) with `vec`, else t + j * NT (strided by the block size).
 // v0: global id of column 0 (vocab shard).
-template <bool BF16, int EPT>
+template <int DT, int EPT>
 __global__ void __launch_bounds__(NT) topk_chunk_kernel(const void* __restrict__ logits,
                                                         const uint8_t* __restrict__ seen, int V, int C, float inv_t,
                                                         float pen, int top_k, uint64_t* __restrict__ pc,
@@ -406,7 +420,7 @@ __global__ void __launch_bounds__(NT) topk_chunk_kernel(const void* __restrict__
   uint32_t kmin = 0xffffffffu, kmax = 0u;
   int o0, ostr;
   run_map(vec != 0, tid, EPT, o0, ostr);
-  load_run<BF16, EPT>(logits, seen, base, c0, o0, ostr, nvalid, vec != 0, inv_t, pen, sv);
+  load_run<DT, EPT>(logits, seen, base, c0, o0, ostr, nvalid, vec != 0, inv_t, pen, sv);
 #pragma unroll
   for (int j = 0; j < EPT; ++j) {
     const int o = o0 + j * ostr;
@@ -620,7 +634,7 @@ __global__ void __launch_bounds__(NT) topk_merge_kernel(const uint64_t* __restri
 }
 
 // ---------------------------------------------------------------- single-WG fallback (large k)
-template <bool BF16>
+template <int DT>
 __global__ void __launch_bounds__(NT) topk_row_kernel(const void* __restrict__ logits, uint8_t* __restrict__ seen,
                                                       int V, float inv_t, float pen, int top_k, float top_p,
                                                       const int* rng, int64_t* __restrict__ out_tok,
@@ -636,7 +650,7 @@ __global__ void __launch_bounds__(NT) topk_row_kernel(const void* __restrict__ l
   const uint32_t seed = (uint32_t)rng[0], step = (uint32_t)rng[1];
   uint32_t kmin = 0xffffffffu, kmax = 0u;
   for (int i = tid; i < V; i += NT) {
-    const uint32_t k = f2key(proc<BF16>(logits, seen, base, i, inv_t, pen));
+    const uint32_t k = f2key(proc<DT>(logits, seen, base, i, inv_t, pen));
     kmin = min(kmin, k);
     kmax = max(kmax, k);
   }
@@ -646,7 +660,7 @@ __global__ void __launch_bounds__(NT) topk_row_kernel(const void* __restrict__ l
   for (int it = 0; it < 48 && lo < hi; ++it) {
     const uint32_t mid = probe(lo, hi, it);
     uint32_t c = 0;
-    for (int i = tid; i < V; i += NT) c += f2key(proc<BF16>(logits, seen, base, i, inv_t, pen)) >= mid;
+    for (int i = tid; i < V; i += NT) c += f2key(proc<DT>(logits, seen, base, i, inv_t, pen)) >= mid;
     c = block_sum_u32(c, red);
     if ((int)c >= top_k) {
       lo = mid;
@@ -656,7 +670,7 @@ __global__ void __launch_bounds__(NT) topk_row_kernel(const void* __restrict__ l
     }
   }
   for (int i = tid; i < V; i += NT) {
-    const float s = proc<BF16>(logits, seen, base, i, inv_t, pen);
+    const float s = proc<DT>(logits, seen, base, i, inv_t, pen);
     const bool ok = f2key(s) >= lo;
     const int slot = wave_alloc(ok, &ncand);          // divergent tail: inactive lanes are not in the ballot
     if (ok && slot < CAP) fc[slot] = ckey(s, i);
@@ -684,7 +698,7 @@ __global__ void __launch_bounds__(NT) topk_row_kernel(const void* __restrict__ l
 constexpr int NTR = 1024, NWR = NTR / 64;
 constexpr int RCAP = 256;                  // candidates ranked exactly (== FCAP)
 
-template <bool BF16, int NS>
+template <int DT, int NS>
 __global__ void __launch_bounds__(NTR) topk_rowwide_kernel(const void* __restrict__ logits,
                                                            uint8_t* __restrict__ seen, int V, float inv_t, float pen,
                                                            int top_k, float top_p, const int* rng,
@@ -706,19 +720,7 @@ __global__ void __launch_bounds__(NTR) topk_rowwide_kernel(const void* __restric
     const int e0 = (q * NTR + tid) * 8;
     if (e0 < V) {
       float v[8];
-      if constexpr (BF16) {
-        const uint4 raw = *reinterpret_cast<const uint4*>(reinterpret_cast<const bf16_t*>(logits) + base + e0);
-        const uint32_t w[4] = {raw.x, raw.y, raw.z, raw.w};
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          v[2 * u] = __uint_as_float(w[u] << 16);
-          v[2 * u + 1] = __uint_as_float(w[u] & 0xffff0000u);
-        }
-      } else {
-        const float4 a = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(logits) + base + e0);
-        const float4 b = *reinterpret_cast<const float4*>(reinterpret_cast<const float*>(logits) + base + e0 + 4);
-        v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w; v[4] = b.x; v[5] = b.y; v[6] = b.z; v[7] = b.w;
-      }
+      scores8<DT>(logits, base + e0, v);
       uint64_t sn = 0;
       if (seen != nullptr) sn = *reinterpret_cast<const uint64_t*>(seen + base + e0);
 #pragma unroll
@@ -844,7 +846,7 @@ extern "C" size_t edge_sample_workspace(int B, int V) {
 
 // mode: 0 greedy, 1 full-vocab sampling, 2 top-k(+top-p). Returns -5 when the configuration
 // needs the host fallback (top-p without top-k, or top-k beyond CAP).
-static int sample_launch(const void* logits, int is_bf16, uint8_t* seen, int B, int V, float temperature,
+static int sample_launch(const void* logits, int dt, uint8_t* seen, int B, int V, float temperature,
                          float inv_temperature, float penalty, int top_k, float top_p, int do_sample, const int* rng,
                          int64_t* out_tok, void* workspace, const Adv& adv, hipStream_t st) {
   if (B == 0) return 0;
@@ -863,22 +865,26 @@ static int sample_launch(const void* logits, int is_bf16, uint8_t* seen, int B, 
   const int vec = g_sample_vec && V % 8 == 0 && reinterpret_cast<uintptr_t>(logits) % 16 == 0 &&
                   (seen == nullptr || reinterpret_cast<uintptr_t>(seen) % 8 == 0);
   if (mode == 2 && top_k > CCAP) {
-    if (is_bf16) hipLaunchKernelGGL(topk_row_kernel<true>, dim3(B), dim3(NT), 0, st, logits, seen, V, inv_t, penalty,
-                                    top_k, top_p, rng, out_tok, adv);
-    else hipLaunchKernelGGL(topk_row_kernel<false>, dim3(B), dim3(NT), 0, st, logits, seen, V, inv_t, penalty, top_k,
-                            top_p, rng, out_tok, adv);
+#define TR(D) hipLaunchKernelGGL(topk_row_kernel<D>, dim3(B), dim3(NT), 0, st, logits, seen, V, inv_t, penalty, top_k, \
+                                 top_p, rng, out_tok, adv)
+    if (dt == LG_BF16) TR(LG_BF16);
+    else if (dt == LG_FP16) TR(LG_FP16);
+    else TR(LG_FP32);
+#undef TR
   } else if (mode == 2 && g_sample_rowwide_min > 0 && B >= g_sample_rowwide_min && V % 8 == 0 && V <= 32768) {
     const int ns = (V + NTR * 8 - 1) / (NTR * 8);
 #define RW(BF, N) hipLaunchKernelGGL((topk_rowwide_kernel<BF, N>), dim3(B), dim3(NTR), 0, st, logits, seen, V, inv_t, \
                                      penalty, top_k, top_p, rng, out_tok, adv)
-    if (is_bf16) { if (ns <= 2) RW(true, 2); else RW(true, 4); }
-    else { if (ns <= 2) RW(false, 2); else RW(false, 4); }
+    if (dt == LG_BF16) { if (ns <= 2) RW(LG_BF16, 2); else RW(LG_BF16, 4); }
+    else if (dt == LG_FP16) { if (ns <= 2) RW(LG_FP16, 2); else RW(LG_FP16, 4); }
+    else { if (ns <= 2) RW(LG_FP32, 2); else RW(LG_FP32, 4); }
 #undef RW
   } else if (mode == 2) {
 #define TC(BF, E) hipLaunchKernelGGL((topk_chunk_kernel<BF, E>), g1, dim3(NT), 0, st, logits, seen, V, C, inv_t, \
                                      penalty, top_k, pc, pthr, vec, 0)
-    if (is_bf16) { if (ept == 8) TC(true, 8); else TC(true, 16); }
-    else { if (ept == 8) TC(false, 8); else TC(false, 16); }
+    if (dt == LG_BF16) { if (ept == 8) TC(LG_BF16, 8); else TC(LG_BF16, 16); }
+    else if (dt == LG_FP16) { if (ept == 8) TC(LG_FP16, 8); else TC(LG_FP16, 16); }
+    else { if (ept == 8) TC(LG_FP32, 8); else TC(LG_FP32, 16); }
 #undef TC
     hipLaunchKernelGGL(topk_merge_kernel, dim3(B), dim3(NT), 0, st, pc, pthr, C, V, top_k, top_p, rng, seen,
                        out_tok, adv);
@@ -887,26 +893,27 @@ static int sample_launch(const void* logits, int is_bf16, uint8_t* seen, int B, 
                                                         seen, V, C, inv_t, penalty, rng, pc, vec, 0); \
                            else hipLaunchKernelGGL((argmax_chunk_kernel<BF, MD, 16>), g1, dim3(NT), 0, st, logits, seen, \
                                                    V, C, inv_t, penalty, rng, pc, vec, 0); } while (0)
-    if (is_bf16) { if (mode == 0) AC(true, 0); else AC(true, 1); }
-    else { if (mode == 0) AC(false, 0); else AC(false, 1); }
+    if (dt == LG_BF16) { if (mode == 0) AC(LG_BF16, 0); else AC(LG_BF16, 1); }
+    else if (dt == LG_FP16) { if (mode == 0) AC(LG_FP16, 0); else AC(LG_FP16, 1); }
+    else { if (mode == 0) AC(LG_FP32, 0); else AC(LG_FP32, 1); }
 #undef AC
     hipLaunchKernelGGL(argmax_merge_kernel, dim3(B), dim3(64), 0, st, pc, C, V, seen, out_tok, adv);
   }
   return (int)hipGetLastError();
 }
 
-extern "C" int edge_sample(const void* logits, int is_bf16, uint8_t* seen, int B, int V, float temperature,
+extern "C" int edge_sample(const void* logits, int dt, uint8_t* seen, int B, int V, float temperature,
                            float inv_temperature, float penalty, int top_k, float top_p, int do_sample, const int* rng,
                            int64_t* out_tok, void* workspace, hipStream_t st) {
   const Adv none{};
-  return sample_launch(logits, is_bf16, seen, B, V, temperature, inv_temperature, penalty, top_k, top_p, do_sample,
+  return sample_launch(logits, dt, seen, B, V, temperature, inv_temperature, penalty, top_k, top_p, do_sample,
                        rng, out_tok, workspace, none, st);
 }
 
 // edge_sample + edge_decode_advance (inc = 1) in the sampler's last launch: out_tok = nxt as well.
 // ctr: an int32 that is zero before the first call (each call leaves it zero); unused at B = 1.
 // rng is advanced, so it is not const here.
-extern "C" int edge_sample_advance(const void* logits, int is_bf16, uint8_t* seen, int B, int V, float temperature,
+extern "C" int edge_sample_advance(const void* logits, int dt, uint8_t* seen, int B, int V, float temperature,
                                    float inv_temperature, float penalty, int top_k, float top_p, int do_sample,
                                    int* rng, int64_t* out_tok, void* workspace, int64_t* tok, int64_t* out,
                                    int64_t out_sb, int ncols, int64_t* step, int* pos, int* lens, int* ctr,
@@ -915,7 +922,7 @@ extern "C" int edge_sample_advance(const void* logits, int is_bf16, uint8_t* see
       (B > 1 && ctr == nullptr))
     return -2;
   const Adv adv{tok, out, out_sb, ncols, step, pos, lens, ctr, rng};
-  return sample_launch(logits, is_bf16, seen, B, V, temperature, inv_temperature, penalty, top_k, top_p, do_sample,
+  return sample_launch(logits, dt, seen, B, V, temperature, inv_temperature, penalty, top_k, top_p, do_sample,
                        rng, out_tok, workspace, adv, st);
 }
 
@@ -943,7 +950,7 @@ extern "C" int edge_sample_shard_chunks(int Vs, int V) {
 }
 
 // Phase 1 over one shard: pc [B][C][CCAP] + pthr [B][C] (mode 2) or pc [B][C] (modes 0 / 1).
-extern "C" int edge_sample_shard(const void* logits, int is_bf16, const uint8_t* seen, int B, int Vs, int v0, int V,
+extern "C" int edge_sample_shard(const void* logits, int dt, const uint8_t* seen, int B, int Vs, int v0, int V,
                                  float temperature, float inv_temperature, float penalty, int top_k, float top_p,
                                  int do_sample, const int* rng, uint64_t* pc, uint32_t* pthr, hipStream_t st) {
   const int mode = shard_mode(do_sample, temperature, top_k, top_p, V);
@@ -958,16 +965,18 @@ extern "C" int edge_sample_shard(const void* logits, int is_bf16, const uint8_t*
   if (mode == 2) {
 #define TC(BF, E) hipLaunchKernelGGL((topk_chunk_kernel<BF, E>), g1, dim3(NT), 0, st, logits, seen, Vs, C, inv_t, \
                                      penalty, top_k, pc, pthr, vec, v0)
-    if (is_bf16) { if (ept == 8) TC(true, 8); else TC(true, 16); }
-    else { if (ept == 8) TC(false, 8); else TC(false, 16); }
+    if (dt == LG_BF16) { if (ept == 8) TC(LG_BF16, 8); else TC(LG_BF16, 16); }
+    else if (dt == LG_FP16) { if (ept == 8) TC(LG_FP16, 8); else TC(LG_FP16, 16); }
+    else { if (ept == 8) TC(LG_FP32, 8); else TC(LG_FP32, 16); }
 #undef TC
   } else {
 #define AC(BF, MD) do { if (ept == 8) hipLaunchKernelGGL((argmax_chunk_kernel<BF, MD, 8>), g1, dim3(NT), 0, st, logits, \
                                                         seen, Vs, C, inv_t, penalty, rng, pc, vec, v0); \
                            else hipLaunchKernelGGL((argmax_chunk_kernel<BF, MD, 16>), g1, dim3(NT), 0, st, logits, seen, \
                                                    Vs, C, inv_t, penalty, rng, pc, vec, v0); } while (0)
-    if (is_bf16) { if (mode == 0) AC(true, 0); else AC(true, 1); }
-    else { if (mode == 0) AC(false, 0); else AC(false, 1); }
+    if (dt == LG_BF16) { if (mode == 0) AC(LG_BF16, 0); else AC(LG_BF16, 1); }
+    else if (dt == LG_FP16) { if (mode == 0) AC(LG_FP16, 0); else AC(LG_FP16, 1); }
+    else { if (mode == 0) AC(LG_FP32, 0); else AC(LG_FP32, 1); }
 #undef AC
   }
   return (int)hipGetLastError();
