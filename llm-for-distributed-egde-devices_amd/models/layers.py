@@ -319,6 +319,19 @@ def plain_linear(m: nn.Module) -> bool:
     return type(m) is Linear and m.bias is None and unwatched(m)
 
 
+def rows_gated(xs, mods, z, norm_w, eps: float):
+    """``rows_together`` of fp32 rows where the last input is xs[2] silu(z), normed over the row under ``norm_w``, in the same launch;
+    None where that kernel does not run."""
+    y = xs[2]
+    if all(plain_linear(m) and not m.split_k_out for m in mods) and all(x.dim() == 2 and x.is_contiguous() for x in xs) and \
+            all(ops.f32_rows_ok(x, m.weight) for x, m in zip(xs, mods)) and z.dtype == norm_w.dtype == torch.float32 and \
+            ops.raw_call(z, norm_w) and z.shape == y.shape and z.stride(1) == 1 and z.stride(0) % 4 == 0 and norm_w.is_contiguous() and \
+            z.device == norm_w.device == y.device and (z.data_ptr() | norm_w.data_ptr()) % 16 == 0 and norm_w.numel() == y.shape[1]:
+        ws = [m.weight for m in mods]
+        return ops.ext().gemv_rows3(xs[0], ws[0], xs[1], ws[1], y, ws[2], *(m.out_features for m in mods), z, norm_w, float(eps))
+    return None
+
+
 def rows_together(xs, mods):
     """The three projections ``mods[j](xs[j])`` of the same few rows in one launch, or each by itself."""
     if all(plain_linear(m) and not m.split_k_out for m in mods) and all(x.dim() == 2 and x.is_contiguous() for x in xs):

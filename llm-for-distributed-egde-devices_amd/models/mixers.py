@@ -17,7 +17,7 @@ import torch.nn as nn
 
 from ..ops import seqmix
 from .configs import ChunkAttnSpec, DecayAttnSpec, DeltaSpec, GatedAttnSpec, GLASpec, LayerSpec, SSDSpec, WindowAttnSpec
-from .layers import Linear, plain_linear, rows_together
+from .layers import Linear, plain_linear, rows_gated, rows_together
 
 
 _ROPE_TABLES: dict = {}
@@ -120,13 +120,13 @@ class ParallelMixer(nn.Module):
                                        self.right.conv_w, self.right.conv_b, run.conv, f0, ff)
 
     def step_heads(self, u: torch.Tensor, c0: int, meta, run, q: torch.Tensor, xbc: torch.Tensor):
-        """Both output projections' inputs from ``step_in``'s queries and x | B | C rows: the two mixers side by side."""
+        """The heads of both mixers, side by side, from ``step_in``'s queries and x | B | C rows: the attention's, and the scan's before
+        their gate and norm."""
         a, s, r = self.left.spec, self.right.spec, self.right
         g0, ng = sum(a.proj_sizes[:3]), a.proj_sizes[3]
-        att, y = seqmix.attention_beside_scan(q, u[:, g0:g0 + ng] if ng else None, run.k, run.v, run.k_pool, run.v_pool, meta, a.scale,
-                                              a.window, a.pool if a.window is not None else None, xbc, u, c0 + s.inner + s.conv_channels,
-                                              r.dt_bias, r.A_log, r.D, run.ssm, s.heads, s.vdim, s.state, s.groups)
-        return att, seqmix.gated_group_norm(y, u[:, c0:c0 + s.inner], r.norm_w, s.norm_groups, r.eps, u.dtype)
+        return seqmix.attention_beside_scan(q, u[:, g0:g0 + ng] if ng else None, run.k, run.v, run.k_pool, run.v_pool, meta, a.scale,
+                                            a.window, a.pool if a.window is not None else None, xbc, u, c0 + s.inner + s.conv_channels,
+                                            r.dt_bias, r.A_log, r.D, run.ssm, s.heads, s.vdim, s.state, s.groups)
 
     def forward(self, x: torch.Tensor, u: torch.Tensor, meta, run, extra: Optional[torch.Tensor] = None, nxt=None, pre=None,
                 down: Optional[nn.Module] = None):
@@ -136,11 +136,15 @@ class ParallelMixer(nn.Module):
         if pre is None:
             a, r = self.left(u, 0, meta, run), self.right(u, c0, meta, run)
         else:
-            ins = self.step_heads(u, c0, meta, run, pre[0], pre[1])
-            if down is not None:
-                extra, a, r = rows_together((pre[2], *ins), (down, self.left.o, self.right.o))
-            else:
-                a, r = self.left.o(ins[0]), self.right.o(ins[1])
+            att, y = self.step_heads(u, c0, meta, run, pre[0], pre[1])
+            m, s = self.right, self.right.spec
+            z, outs = u[:, c0:c0 + s.inner], None
+            if down is not None and s.norm_groups == 1:
+                outs = rows_gated((pre[2], att, y), (down, self.left.o, m.o), z, m.norm_w, m.eps)
+            if outs is None:
+                y = seqmix.gated_group_norm(y, z, m.norm_w, s.norm_groups, m.eps, u.dtype)
+                outs = rows_together((pre[2], att, y), (down, self.left.o, m.o)) if down is not None else (extra, self.left.o(att), m.o(y))
+            extra, a, r = outs
         if nxt is not None:
             return seqmix.combine_residual_norm(x, a, r, self.left_out, self.right_out, self.eps, extra, nxt.weight, nxt.eps, u.dtype)
         return seqmix.combine_residual(x, a, r, self.left_out, self.right_out, self.eps, extra)

@@ -94,7 +94,8 @@ int edge_w8a8_rows256_splits(int K);
 void edge_w8a8_prefill_x32(int v);
 int edge_gemv_bf16(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi,
                    hipStream_t st, const void* add, int h16);
-int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K, hipStream_t st);
+int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K,
+                    const float* gate_z, int z_ld, const float* gate_w, float eps, hipStream_t st);
 int edge_rows3(const void* const* x, const void* const* w, void* const* y, const int* N, const int* K, int M, int h16, hipStream_t st);
 int edge_gemv_f32(const float* x, const float* W, const float* bias, float* y, int M, int N, int K, hipStream_t st);
 int edge_gemv_bf16_splitk(const void* A, const void* W, const void* bias, float* part, int M, int N, int K, int S,
@@ -856,10 +857,12 @@ at::Tensor gemv_f32(const at::Tensor& x, const at::Tensor& w, const std::optiona
 }
 
 // Three projections of the same rows in one launch: fp32 x_j [M <= 8, K_j] over weights [N_j, K_j] as they are, or 16 bits, M <= 4,
-// over packed weights of N_j K_j numbers.
+// over packed weights of N_j K_j numbers.  gate [M, K_2] (rows may lie apart) and gate_w [K_2], fp32 only: x_2 becomes
+// x_2 silu(gate), normed over the row under gate_w.
 std::tuple<at::Tensor, at::Tensor, at::Tensor> gemv_rows3(const at::Tensor& x0, const at::Tensor& w0, const at::Tensor& x1,
                                                           const at::Tensor& w1, const at::Tensor& x2, const at::Tensor& w2,
-                                                          int64_t n0, int64_t n1, int64_t n2) {
+                                                          int64_t n0, int64_t n1, int64_t n2, const std::optional<at::Tensor>& gate,
+                                                          const std::optional<at::Tensor>& gate_w, double eps) {
   DEVICE_GUARD(x0);
   const at::Tensor *x[3] = {&x0, &x1, &x2}, *w[3] = {&w0, &w1, &w2};
   const int64_t nn[3] = {n0, n1, n2}, M = x0.size(0);
@@ -884,8 +887,20 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> gemv_rows3(const at::Tensor& x0, 
     const float *xp[3], *wp[3];
     float* yp[3];
     for (int j = 0; j < 3; ++j) { xp[j] = x[j]->data_ptr<float>(); wp[j] = w[j]->data_ptr<float>(); yp[j] = y[j].data_ptr<float>(); }
-    check(edge_gemv_f32x3(xp, wp, yp, (int)M, N, K, stream()), "gemv_rows3");
+    const float* gw = nullptr;
+    int ld = 0;
+    if (gate) {
+      TORCH_CHECK(gate_w && gate->scalar_type() == at::kFloat && gate->sizes() == x2.sizes() && gate->stride(1) == 1 &&
+                      gate->stride(0) % 4 == 0 && gate->stride(0) <= INT_MAX && (uintptr_t)gate->data_ptr() % 16 == 0 &&
+                      gate->device() == x0.device(), "gate: fp32 [M, K_2], 16-byte aligned rows");
+      need(*gate_w, at::kFloat, "gate_w");
+      TORCH_CHECK(gate_w->numel() == x2.size(1) && (uintptr_t)gate_w->data_ptr() % 16 == 0 && gate_w->device() == x0.device(), "gate_w [K_2]");
+      ld = (int)gate->stride(0);
+      gw = gate_w->data_ptr<float>();
+    }
+    check(edge_gemv_f32x3(xp, wp, yp, (int)M, N, K, gate ? gate->data_ptr<float>() : nullptr, ld, gw, (float)eps, stream()), "gemv_rows3");
   } else {
+    TORCH_CHECK(!gate, "a gate needs fp32 rows");
     const void *xp[3], *wp[3];
     void* yp[3];
     for (int j = 0; j < 3; ++j) { xp[j] = x[j]->data_ptr(); wp[j] = w[j]->data_ptr(); yp[j] = y[j].data_ptr(); }
@@ -1713,7 +1728,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
         py::arg("N"), py::arg("epi"), py::arg("y_out"), py::arg("x2") = py::none(), py::arg("gamma2") = py::none(),
         py::arg("beta2") = py::none());
   m.def("decode_attn_up", &decode_attn_up, "decode attention beside the up projection of a parallel-residual block (M <= 4)");
-  m.def("gemv_rows3", &gemv_rows3, "three projections of the same rows in one launch (fp32 M <= 8, 16 bits M <= 4)");
+  m.def("gemv_rows3", &gemv_rows3, "three projections of the same rows in one launch (fp32 M <= 8, 16 bits M <= 4)", py::arg("x0"),
+        py::arg("w0"), py::arg("x1"), py::arg("w1"), py::arg("x2"), py::arg("w2"), py::arg("n0"), py::arg("n1"), py::arg("n2"),
+        py::arg("gate") = py::none(), py::arg("gate_w") = py::none(), py::arg("eps") = 0.0);
   m.def("decode_o_down", &decode_o_down, "o beside the down projection of a parallel-residual block (M <= 4)");
   m.def("w8a8_gemv_ln", &w8a8_gemv_ln, "W8A8 decode GEMV with the LayerNorm + int8 quant in its prologue (M <= 4)");
   m.def("llmint8_gemv", &llmint8_gemv, "LLM.int8 projection of one row in one launch (prep in the GEMV prologue)");

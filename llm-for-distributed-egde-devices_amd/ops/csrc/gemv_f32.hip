@@ -13,27 +13,58 @@
 
 namespace {
 
-template <int MV, int R>
+// A gated norm in front of a projection: its input is x silu(z) / rms(x silu(z)) * w over the whole row.
+struct Gate {
+  const float* z;       // [M, K], rows ld apart
+  const float* w;       // [K]
+  int ld;
+  float eps;
+};
+
+// GATED: the waves that share a row's k read all of it between them, so the row's sum of squares costs no load: they sum x silu(z) w
+// times the weights, and the sums are divided by the root mean square at the end (a launch of its own for the norm was 4.7 us of the
+// 37.7 that a layer's step of 2 rows, 1024 wide, took; this launch 7.4 us without and 7.5 with it).
+template <int MV, int R, bool GATED = false>
 __device__ __forceinline__ void gemv_f32_body(int bid, const float* __restrict__ x, const float* __restrict__ W,
-                                              const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K, int KW) {
+                                              const float* __restrict__ bias, float* __restrict__ y, int M, int N, int K, int KW,
+                                              const Gate& g = Gate{}) {
   constexpr int V = MV * R;
   __shared__ float part[16 * V];
+  __shared__ float sqs[GATED ? 16 * MV : 1];
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), waves = blockDim.x >> 6;
   const int rg = wave / KW, kw = wave - rg * KW, n0 = (bid * (waves / KW) + rg) * R;
   const int C = (K + 255) / 256;
   float acc[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) acc[i] = 0.f;
-  v4f wv[2][R], xv[2][MV];
+  v4f wv[2][R], xv[2][MV], zv[GATED ? 2 : 1][MV], gv[GATED ? 2 : 1];
+  float sq[MV];
+#pragma unroll
+  for (int m = 0; m < MV; ++m) sq[m] = 0.f;
   auto load = [&](int b, int c) {                            // rows past the last and k past the end: a clamped one
     const int k = min(min(c, C - 1) * 256 + lane * 4, K - 4);
 #pragma unroll
     for (int r = 0; r < R; ++r) wv[b][r] = *reinterpret_cast<const v4f*>(W + (size_t)min(n0 + r, N - 1) * K + k);
 #pragma unroll
     for (int m = 0; m < MV; ++m) xv[b][m] = *reinterpret_cast<const v4f*>(x + (size_t)min(m, M - 1) * K + k);
+    if constexpr (GATED) {
+#pragma unroll
+      for (int m = 0; m < MV; ++m) zv[b][m] = *reinterpret_cast<const v4f*>(g.z + (size_t)min(m, M - 1) * g.ld + k);
+      gv[b] = *reinterpret_cast<const v4f*>(g.w + k);
+    }
   };
   auto use = [&](int b, int c) {
     if (c * 256 + lane * 4 >= K) return;
+    if constexpr (GATED) {
+#pragma unroll
+      for (int m = 0; m < MV; ++m)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float v = xv[b][m][j] * (zv[b][m][j] * (1.f / (1.f + expf(-zv[b][m][j]))));
+          sq[m] = __builtin_fmaf(v, v, sq[m]);
+          xv[b][m][j] = v * gv[b][j];
+        }
+    }
 #pragma unroll
     for (int r = 0; r < R; ++r)
 #pragma unroll
@@ -57,11 +88,23 @@ __device__ __forceinline__ void gemv_f32_body(int bid, const float* __restrict__
   // the first bits of the lane number chose; lanes that differ only in the others hold the same sum
   static_assert(V <= 64, "one sum per lane");
   if (lane % (64 / V) == 0) part[wave * V + idx] = acc[0];
+  if constexpr (GATED) {
+#pragma unroll
+    for (int m = 0; m < MV; ++m) {
+      sq[m] = wave_sum(sq[m]);
+      if (lane == 0) sqs[wave * MV + m] = sq[m];
+    }
+  }
   __syncthreads();
   for (int e = tid; e < waves / KW * V; e += blockDim.x) {
     const int gq = e / V, v = e - gq * V, m = v % MV, n = (bid * (waves / KW) + gq) * R + v / MV;
     float sum = 0.f;
     for (int w = 0; w < KW; ++w) sum += part[(gq * KW + w) * V + v];
+    if constexpr (GATED) {
+      float s2 = 0.f;
+      for (int w = 0; w < KW; ++w) s2 += sqs[(gq * KW + w) * MV + m];
+      sum *= 1.f / sqrtf(s2 / (float)K + g.eps);
+    }
     if (m < M && n < N) y[(size_t)m * N + n] = sum + (bias ? bias[n] : 0.f);
   }
 }
@@ -79,9 +122,11 @@ struct Jobs3 {
   float* y[3];
   int N[3], K[3], KW[3], n[2];
 };
-template <int MV, int R>
-__global__ void __launch_bounds__(1024) gemv_f32x3_kernel(Jobs3 a, int M) {
+template <int MV, int R, bool GATED>
+__global__ void __launch_bounds__(1024) gemv_f32x3_kernel(Jobs3 a, int M, Gate g) {
   const int bid = blockIdx.x, j = bid < a.n[0] ? 0 : bid < a.n[1] ? 1 : 2;
+  if constexpr (GATED)
+    if (j == 2) return gemv_f32_body<MV, R, true>(bid - a.n[1], a.x[2], a.W[2], nullptr, a.y[2], M, a.N[2], a.K[2], a.KW[2], g);
   gemv_f32_body<MV, R>(bid - (j == 0 ? 0 : a.n[j - 1]), a.x[j], a.W[j], nullptr, a.y[j], M, a.N[j], a.K[j], a.KW[j]);
 }
 
@@ -101,7 +146,7 @@ void launch_f32(const float* x, const float* W, const float* bias, float* y, int
 }
 
 template <int MV, int R>
-void launch_f32x3(Jobs3 a, int M, hipStream_t st) {
+void launch_f32x3(Jobs3 a, int M, const Gate& g, hipStream_t st) {
   int waves = 4, blocks = 0;
   for (int j = 0; j < 3; ++j) {
     a.KW[j] = share_k((a.N[j] + R - 1) / R, a.K[j]);
@@ -112,25 +157,29 @@ void launch_f32x3(Jobs3 a, int M, hipStream_t st) {
     blocks += ((a.N[j] + R - 1) / R + per - 1) / per;
     if (j < 2) a.n[j] = blocks;
   }
-  hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R>), dim3(blocks), dim3(waves * 64), 0, st, a, M);
+  if (g.z != nullptr) hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R, true>), dim3(blocks), dim3(waves * 64), 0, st, a, M, g);
+  else hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R, false>), dim3(blocks), dim3(waves * 64), 0, st, a, M, g);
 }
 }  // namespace
 
 // y_j = x_j W_j^T for three projections of the same M rows' inputs, each as edge_gemv_f32 forms it: a parallel layer's three output
 // projections, whose launches' ramps and ends then overlap.  us in a graph, weights from memory, three launches / one, 1024 x 4096 and
 // twice 1024 x 1024: 1 row 11.1 / 6.8, 2 11.5 / 7.0, 8 15.1 / 11.4; 2048 x 8192 and twice 2048 x 2048, 2 rows 24.0 / 18.8
+// gate_z (null: none): x_2 is gated by its rows, z_ld apart, and normed under gate_w first; 16-byte aligned, z_ld % 4 == 0
 extern "C" int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K,
-                               hipStream_t st) {
+                               const float* gate_z, int z_ld, const float* gate_w, float eps, hipStream_t st) {
+  const Gate g{gate_z, gate_w, z_ld, eps};
+  if (gate_z != nullptr && (gate_w == nullptr || z_ld % 4)) return -2;
   Jobs3 a{};
   for (int j = 0; j < 3; ++j) {
     if (N[j] < 1 || K[j] < 4 || K[j] % 4) return -2;
     a.x[j] = x[j]; a.W[j] = W[j]; a.y[j] = y[j]; a.N[j] = N[j]; a.K[j] = K[j];
   }
   if (M < 1 || M > 8) return -2;
-  if (M == 1) launch_f32x3<1, 4>(a, M, st);
-  else if (M == 2) launch_f32x3<2, 4>(a, M, st);
-  else if (M <= 4) launch_f32x3<4, 4>(a, M, st);
-  else launch_f32x3<8, 2>(a, M, st);
+  if (M == 1) launch_f32x3<1, 4>(a, M, g, st);
+  else if (M == 2) launch_f32x3<2, 4>(a, M, g, st);
+  else if (M <= 4) launch_f32x3<4, 4>(a, M, g, st);
+  else launch_f32x3<8, 2>(a, M, g, st);
   return (int)hipGetLastError();
 }
 
