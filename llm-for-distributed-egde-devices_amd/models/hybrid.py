@@ -461,11 +461,16 @@ class HybridLM(nn.Module):
     def scores(self, ids: torch.Tensor, meta: seqmix.RaggedMeta, cache, rows: Optional[torch.Tensor] = None,
                taps: Optional[list] = None) -> torch.Tensor:
         """``forward`` up to the output projection's rows in the model's own type (``finish`` makes logits of them)."""
-        cfg = self.cfg
+        cfg, h_next = self.cfg, None
         if cfg.bigram:
             b = cfg.bigram
-            x0 = seqmix.embedding_bigram(ids, meta, self.embed, self.bigram, cache.prev_tok, b["buckets"], b["mul_prev"],
-                                         b["mul_cur"])
+            args = (ids, meta, self.embed, self.bigram, cache.prev_tok, b["buckets"], b["mul_prev"], b["mul_cur"])
+            first = self.layers[self.runs[0][0]] if self.runs else None
+            if meta.max_len == 1 and type(first) is PostNormLayer and first.canon1 is not None and unwatched(first) and \
+                    cfg.loop is None and not cfg.streams:    # the first layer's input with the rows that it reads
+                x0, h_next = seqmix.embedding_bigram_canon(*args, first.canon1, cache.run(0).canon1, self.dtype)
+            else:
+                x0 = seqmix.embedding_bigram(*args)
         elif cfg.pos_emb == "learned":
             x0 = seqmix.embedding_learned(ids, meta, self.embed, self.pos)
         else:
@@ -473,7 +478,6 @@ class HybridLM(nn.Module):
         x = x0.clone() if cfg.loop is not None and cfg.loop.entry != "plain" else x0
         if cfg.streams:                                  # [T, S, W]: every stream starts as the embedding rows
             x = x0[:, None, :].expand(-1, cfg.streams, -1).contiguous()
-        h_next = None
         for r, (i, t) in enumerate(self.runs):
             if t is not None and i == cfg.loop.start and cfg.loop.entry != "plain":
                 if cfg.loop.entry == "add_embed":

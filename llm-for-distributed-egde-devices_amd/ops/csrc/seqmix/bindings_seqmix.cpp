@@ -105,6 +105,9 @@ int edge_sm_ssd_chunked(const void* xbc, int Cx, const void* u, int ld, int dt0,
                         const float* A_log, const float* Dp, float* state, const int* seq_slot, const int* seq_start,
                         const int* seq_len, const int* seq_off, float* y, float* sloc, float* cdec, int n,
                         int max_chunks, int Hs, int P, int N, int groups, int f32, hipStream_t st);
+int edge_sm_embed_bigram_tap4(const int64_t* ids, const void* table, const void* bigram, int64_t* prev_tok, const int* tok_seq,
+                              const int* tok_pos, const int* seq_slot, float* x, const float* w, float* state, void* out, int rows, int W,
+                              int V, long buckets, long mul_prev, long mul_cur, int f32, hipStream_t st);
 int edge_sm_embed_bigram(const int64_t* ids, const void* table, const void* bigram, int64_t* prev_tok, const int* tok_seq,
                          const int* tok_pos, const int* seq_slot, const int* seq_start, const int* seq_len,
                          const int* seq_off, float* out, int rows, int n, int W, int V, long buckets, long mul_prev,
@@ -731,6 +734,36 @@ at::Tensor sm_embed_bigram(const at::Tensor& ids, const at::Tensor& table, const
                              out.data_ptr<float>(), (int)T, (int)n, (int)table.size(1), (int)table.size(0), (long)buckets,
                              (long)mul_prev, (long)mul_cur, f32(table), stream()), "sm_embed_bigram");
   return out;
+}
+
+// sm_embed_bigram and sm_canon of a step in which every sequence brings one token: (x fp32, rows of the table's type), or nothing where
+// the one launch does not take it.
+std::optional<std::tuple<at::Tensor, at::Tensor>> sm_embed_bigram_tap4(const at::Tensor& ids, const at::Tensor& table,
+                                                                       const at::Tensor& bigram, at::Tensor& prev_tok,
+                                                                       const at::Tensor& tok_seq, const at::Tensor& tok_pos,
+                                                                       const at::Tensor& seq_slot, int64_t buckets, int64_t mul_prev,
+                                                                       int64_t mul_cur, const at::Tensor& w, at::Tensor& state) {
+  TORCH_CHECK(ids.is_cuda() && ids.scalar_type() == at::kLong && ids.is_contiguous() && ids.dim() == 1, "ids: int64 [T]");
+  chk_act2(table, "table");
+  chk_act2(bigram, "bigram");
+  const int64_t T = ids.size(0), W = table.size(1);
+  TORCH_CHECK(bigram.scalar_type() == table.scalar_type() && bigram.size(1) == W && bigram.size(0) == buckets + 1, "bigram: [buckets + 1, W]");
+  TORCH_CHECK(prev_tok.is_cuda() && prev_tok.scalar_type() == at::kLong && prev_tok.is_contiguous(), "prev_tok: int64 [slots]");
+  for (const at::Tensor* t : {&tok_seq, &tok_pos, &seq_slot}) chk_i32(*t, "metadata");
+  TORCH_CHECK(tok_seq.numel() == T && tok_pos.numel() == T && seq_slot.numel() >= T, "metadata sizes");
+  chk_f32(w, "weight");
+  chk_f32(state, "state");
+  TORCH_CHECK(w.dim() == 2 && w.size(0) == W && state.dim() == 3 && state.size(2) == W, "weight [W, taps], state [slots, taps - 1, W]");
+  if (w.size(1) != 4 || state.size(1) != 3) return std::nullopt;
+  c10::hip::HIPGuardMasqueradingAsCUDA guard(table.device());
+  auto x = at::empty({T, W}, table.options().dtype(at::kFloat)), out = at::empty({T, W}, table.options());
+  const int rc = edge_sm_embed_bigram_tap4(ids.data_ptr<int64_t>(), table.data_ptr(), bigram.data_ptr(), prev_tok.data_ptr<int64_t>(),
+                                           tok_seq.data_ptr<int>(), tok_pos.data_ptr<int>(), seq_slot.data_ptr<int>(), x.data_ptr<float>(),
+                                           w.data_ptr<float>(), state.data_ptr<float>(), out.data_ptr(), (int)T, (int)W,
+                                           (int)table.size(0), (long)buckets, (long)mul_prev, (long)mul_cur, f32(table), stream());
+  if (rc == -2) return std::nullopt;
+  check(rc, "sm_embed_bigram_tap4");
+  return std::make_tuple(x, out);
 }
 
 at::Tensor sm_canon(const at::Tensor& x, const at::Tensor& w, at::Tensor& state, const at::Tensor& tok_seq,
@@ -1800,6 +1833,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_ssd_scan", &sm_ssd_scan);
   m.def("sm_attention_ssd", &sm_attention_ssd);
   m.def("sm_embed_bigram", &sm_embed_bigram);
+  m.def("sm_embed_bigram_tap4", &sm_embed_bigram_tap4);
   m.def("sm_canon", &sm_canon);
   m.def("sm_ln_residual_taps", &sm_ln_residual_taps);
   m.def("sm_ln_residual_taps_route", &sm_ln_residual_taps_route);

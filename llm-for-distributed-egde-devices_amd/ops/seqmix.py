@@ -502,6 +502,19 @@ def embedding_bigram(ids: torch.Tensor, meta: RaggedMeta, table: torch.Tensor, b
     return out
 
 
+def embedding_bigram_canon(ids: torch.Tensor, meta: RaggedMeta, table: torch.Tensor, bigram: torch.Tensor, prev_tok: torch.Tensor,
+                           buckets: int, mul_prev: int, mul_cur: int, weight: torch.Tensor, state: torch.Tensor, out_dtype):
+    """``embedding_bigram`` and ``canon_conv`` of its rows: (x, the convolved rows).  One launch for four taps where every sequence
+    brings one token."""
+    if _gpu(table) and meta.max_len == 1 and meta.T == meta.n and table.dtype == out_dtype:
+        both = _ext().sm_embed_bigram_tap4(ids.long().contiguous(), table, bigram, prev_tok, meta.tok_seq, meta.tok_pos, meta.seq_slot,
+                                           int(buckets), int(mul_prev), int(mul_cur), weight, state)
+        if both is not None:
+            return both
+    x = embedding_bigram(ids, meta, table, bigram, prev_tok, buckets, mul_prev, mul_cur)
+    return x, canon_conv(x, weight, state, meta, out_dtype)
+
+
 def canon_conv(x: torch.Tensor, weight: torch.Tensor, state: torch.Tensor, meta: RaggedMeta, out_dtype) -> torch.Tensor:
     """x + causal depthwise convolution of x over time, fp32 [T, W] in, ``out_dtype`` out.  weight fp32
     [W, taps] (last tap = the current token), state fp32 [slots, taps - 1, W] = each slot's last inputs
