@@ -154,30 +154,63 @@ __device__ __forceinline__ void stage_tile(float (*dst)[LDT], const T* __restric
   }
 }
 
-// (1) Sloc[n][p] = sum_s k_s[n] e^{B_end - B_s}[n] v_s[p] for one 64 x 64 tile of (n, p).  A thread computes the log2
+// stage_tile's VEC form in two halves, so that the loads run beside other work: a tile's numbers to registers (from clamped addresses:
+// rl >= 1 and cl >= 8 here), and from there to the LDS
+template <typename T, int ROWS, int COLS>
+struct TileRegs {
+  static constexpr int E = (ROWS * COLS / 8 + NT - 1) / NT;
+  float f[E][8];
+  __device__ __forceinline__ void get(const T* __restrict__ src, size_t ld, int rl, int cl) {
+    static_assert(ROWS * COLS / 8 % NT == 0, "whole rounds");
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const int e = threadIdx.x + i * NT, r = min(e / (COLS / 8), rl - 1), c = min((e % (COLS / 8)) * 8, cl - 8);
+      load8<T>(src + (size_t)r * ld + c, f[i]);
+    }
+  }
+  template <int LDT, bool SWZ = false>
+  __device__ __forceinline__ void put(float (*dst)[LDT], int rl, int cl, float mul) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const int e = threadIdx.x + i * NT, r = e / (COLS / 8), c = (e % (COLS / 8)) * 8;
+      float v[8];
+#pragma unroll
+      for (int k = 0; k < 8; ++k) v[k] = r < rl && c < cl ? f[i][k] * mul : 0.f;
+      store8<float>(&dst[r][SWZ ? c ^ ((r & 3) << 4) : c], v);
+    }
+  }
+};
+
+// (1) Sloc[n][p] = sum_s k_s[n] e^{B_end - B_s}[n] v_s[p] for one tile of 64 n and 16 PT p.  A thread computes the log2
 // decays of one key channel over a 16-token block; they go to la [rows, H N] for the outputs, the chunk's whole decay
 // e^{B_end} per key channel to cdec.  Wave w: rows 16 w .. of the tile.  The decay projection's inner rows are staged
 // RS at a time.
-template <typename T, bool VEC>
+// Bound by the chain from the loads over the decays to the products, and by its bytes.  us, 120 chunks of 16 heads of 128 / 128, 64 x 64
+// tiles 131; 64 x 128, so that a head's decays are formed once for all its columns, and keys and values on their way meanwhile 110.
+template <typename T, bool VEC, int PT>
 __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict__ u, int ld, const float* __restrict__ a2,
                                                              const float* __restrict__ b, int rank, float scale,
                                                              const int* __restrict__ seq_len, const int* __restrict__ seq_off,
                                                              float* __restrict__ sloc, float* __restrict__ cdec,
                                                              float* __restrict__ la, int H, int N, int P, int ntn, int ntp) {
   constexpr int LDT = CL;
-  constexpr int RS = 16;
+  constexpr int RS = 16, CW = 16 * PT;
   __shared__ __attribute__((aligned(16))) float d_s[RS][CL];
-  __shared__ __attribute__((aligned(16))) float K_s[CL][LDT], V_s[CL][LDT];
+  __shared__ __attribute__((aligned(16))) float K_s[CL][LDT], V_s[CL][CW];
   __shared__ float seg_s[4][CL];
   const int tile = blockIdx.x % (ntn * ntp), c = blockIdx.x / (ntn * ntp), s = blockIdx.y, h = blockIdx.z;
   const int len = seq_len[s];
   if (c * CL >= len) return;
-  const int tc = min(CL, len - c * CL), n0 = (tile / ntp) * CL, p0 = (tile % ntp) * CL;
+  const int tc = min(CL, len - c * CL), n0 = (tile / ntp) * CL, p0 = (tile % ntp) * CW;
   const size_t row0 = (size_t)seq_off[s] + (size_t)c * CL;
   const int HN = H * N, HP = H * P, tid = threadIdx.x, nn = tid & 63, seg = tid >> 6, n = n0 + nn;
   const T* base = u + row0 * ld;
-  stage_tile<T, CL, CL, LDT, VEC, true>(K_s, base + HN + h * N + n0, ld, tc, N - n0, 1.f);
-  stage_tile<T, CL, CL, LDT, VEC, true>(V_s, base + 2 * HN + h * P + p0, ld, tc, P - p0, 1.f);
+  TileRegs<T, CL, CL> rk;                                    // VEC: asked for before the decays, staged behind them
+  TileRegs<T, CL, CW> rv;
+  if constexpr (!VEC) {
+    stage_tile<T, CL, CL, LDT, VEC, true>(K_s, base + HN + h * N + n0, ld, tc, N - n0, 1.f);
+    stage_tile<T, CL, CW, CW, VEC, true>(V_s, base + 2 * HN + h * P + p0, ld, tc, P - p0, 1.f);
+  }
   float bl[16];
   {
     const int nc = min(n, N - 1);
@@ -191,6 +224,12 @@ __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict
         const int t = e / RS, r = e % RS;
         d_s[r][t] = t < tc && r0 + r < rank ? ldf<T>(base + (size_t)t * ld + 2 * HN + 2 * HP + r0 + r) : 0.f;
       }
+      if constexpr (VEC)
+        if (r0 == 0) {
+          rk.get(base + HN + h * N + n0, ld, tc, N - n0);
+          rv.get(base + 2 * HN + h * P + p0, ld, tc, P - p0);
+          asm volatile("" ::: "memory");
+        }
       __syncthreads();
       float w[RS];
 #pragma unroll
@@ -215,6 +254,10 @@ __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict
     }
     seg_s[seg][nn] = run;
   }
+  if constexpr (VEC) {
+    rk.template put<LDT, true>(K_s, tc, N - n0, 1.f);
+    rv.template put<CW, true>(V_s, tc, P - p0, 1.f);
+  }
   __syncthreads();
   float after = 0.f, end = 0.f;                              // the later blocks' decay, the chunk's
 #pragma unroll
@@ -228,18 +271,18 @@ __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict
   if (p0 == 0 && seg == 0 && n < N) cdec[(cb * H + h) * N + n] = ex2(end);
   __syncthreads();
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, g4 = lane >> 4;
-  v4f acc[4];
+  v4f acc[PT];
 #pragma unroll
-  for (int j = 0; j < 4; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < PT; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int kk = 0; kk < CL / 4; ++kk) {
     const float a = K_s[4 * kk + g4][16 * (wave ^ g4) + l16];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) acc[j] = mfma4(a, V_s[4 * kk + g4][16 * (j ^ g4) + l16], acc[j]);
+    for (int j = 0; j < PT; ++j) acc[j] = mfma4(a, V_s[4 * kk + g4][16 * (j ^ g4) + l16], acc[j]);
   }
   float* dst = sloc + (cb * H + h) * (size_t)N * P;
 #pragma unroll
-  for (int j = 0; j < 4; ++j)
+  for (int j = 0; j < PT; ++j)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
       const int r = n0 + 16 * wave + 4 * g4 + i, p = p0 + 16 * j + l16;
@@ -247,42 +290,59 @@ __global__ void __launch_bounds__(NT) gla_chunk_state_kernel(const T* __restrict
     }
 }
 
-// (2) the state entering every chunk (written over that chunk's own contribution) and the final state; sixteen
-// chunks' rows are in flight at a time
+// (2) the state entering every chunk (written over that chunk's own contribution) and the final state, V numbers a thread; the next
+// UN chunks' rows are requested before these are summed.  Bound by the rows, read and written once: 120 chunks of 16 heads of
+// 128 x 128, us, one number a thread, 16 chunks, then their sums 50; four numbers 41 (6.1 TB/s).
+template <int V>
 __global__ void __launch_bounds__(NT) gla_chunk_scan_kernel(float* __restrict__ sloc, const float* __restrict__ cdec,
                                                             float* __restrict__ state, const int* __restrict__ seq_slot,
                                                             const int* __restrict__ seq_start, const int* __restrict__ seq_len,
                                                             int H, int N, int P) {
-  constexpr int UN = 16;
-  const int s = blockIdx.x, h = blockIdx.y, e = blockIdx.z * NT + threadIdx.x, NP = N * P;
+  constexpr int UN = 8;
+  typedef float vec __attribute__((ext_vector_type(V)));
+  const int s = blockIdx.x, h = blockIdx.y, e = (blockIdx.z * NT + threadIdx.x) * V, NP = N * P;
   if (e >= NP) return;
   const int nc = (seq_len[s] + CL - 1) / CL, n = e / P;
   const size_t cb = chunk_base(seq_len, s);
-  float* st = state + ((size_t)seq_slot[s] * H + h) * NP + e;
-  float S = seq_start[s] > 0 ? *st : 0.f;
-  for (int c0 = 0; c0 < nc; c0 += UN) {
-    float own[UN], dec[UN];
+  vec* st = reinterpret_cast<vec*>(state + ((size_t)seq_slot[s] * H + h) * NP + e);
+  const size_t step = (size_t)H * NP;
+  float* p = sloc + (cb * H + h) * (size_t)NP + e;
+  const float* dp = cdec + (cb * H + h) * N + n;
+  vec S = 0.f;
+  if (seq_start[s] > 0) S = *st;
+  vec own[2][UN];
+  float dec[2][UN];
+  auto get = [&](int b, int c0) {
 #pragma unroll
     for (int i = 0; i < UN; ++i) {
-      const bool ok = c0 + i < nc;
-      own[i] = ok ? sloc[((cb + c0 + i) * H + h) * (size_t)NP + e] : 0.f;
-      dec[i] = ok ? cdec[((cb + c0 + i) * H + h) * N + n] : 1.f;
+      const int c = min(c0 + i, nc - 1);
+      own[b][i] = __builtin_nontemporal_load(reinterpret_cast<const vec*>(p + c * step));
+      dec[b][i] = dp[(size_t)c * H * N];
     }
+  };
+  auto use = [&](int b, int c0) {
 #pragma unroll
-    for (int i = 0; i < UN; ++i) {
+    for (int i = 0; i < UN; ++i)
       if (c0 + i < nc) {
-        sloc[((cb + c0 + i) * H + h) * (size_t)NP + e] = S;
-        S = dec[i] * S + own[i];
+        *reinterpret_cast<vec*>(p + (c0 + i) * step) = S;
+        S = dec[b][i] * S + own[b][i];
       }
-    }
+  };
+  get(0, 0);
+  for (int c0 = 0; c0 < nc; c0 += 2 * UN) {
+    if (c0 + UN < nc) get(1, c0 + UN);
+    use(0, c0);
+    if (c0 + 2 * UN < nc) get(0, c0 + 2 * UN);
+    use(1, c0 + UN);
   }
   *st = S;
 }
 
 // (3) the outputs of one chunk and 16 PT value columns.  Wave i owns the token rows of block i (16 tokens).
-// Bound by its vector instructions (5.6 k a wave, a third of them a block against itself) beside fp32 products at 40 % of their rate.
+// Bound by its vector instructions beside fp32 products at half their rate, with two workgroups a CU (their LDS).
 // us, 7680 tokens, 16 heads of 128 / 128, this kernel: 288; without branches in the products 258; without a minimum a power 240; rows
-// through the LDS at the end 214.
+// through the LDS at the end 198; the next channels' tiles on their way meanwhile 185; only the counted pairs of a block against itself
+// (a third of the instructions before) 172.  Half the channels at a time, which lets three workgroups on a CU, 181.
 // FUSE: all columns of the head are here, so the norm and the gate follow.
 template <typename T, int PT, bool FUSE, bool VEC>
 __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__ u, int ld, const float* __restrict__ la,
@@ -310,18 +370,47 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
   const T* base = u + row0 * ld;
   const float qs = 1.f / sqrtf((float)N);
   const int t = 16 * wave + l16;                             // this lane's token row as a product operand
-  v4f o[PT], off_[3], dg = v4f{0.f, 0.f, 0.f, 0.f};
+  v4f o[PT], off_[3];
+  // the block against itself: lane and m hold the pair (row, column <= row) that fold maps them to, row r < 8 (its columns before r) and
+  // row 15 - r (all its columns) sharing 16 lanes; the first eight rows' own columns, without a decay, are apart (lane & 7)
+  float dg[2] = {0.f, 0.f}, own = 0.f;
+  auto fold = [&](int m, int& row, int& col) {
+    const int r = g4 + 4 * m, hi = 15 - r;
+    row = l16 <= hi ? hi : r;
+    col = l16 <= hi ? l16 : 15 - l16;
+  };
 #pragma unroll
   for (int j = 0; j < PT; ++j) o[j] = v4f{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int j = 0; j < 3; ++j) off_[j] = v4f{0.f, 0.f, 0.f, 0.f};
+  TileRegs<T, CL, NK> rq, rk;
+  TileRegs<float, CL, NK> rb;
+  TileRegs<float, NK, CW> rs;
+  auto get = [&](int n0) {
+    rb.get(la + row0 * HN + h * N + n0, HN, tc, N - n0);
+    rq.get(base + h * N + n0, ld, tc, N - n0);
+    rk.get(base + HN + h * N + n0, ld, tc, N - n0);
+    rs.get(sin_c + (size_t)n0 * P, P, N - n0, P - p0);
+  };
+  if constexpr (VEC) get(0);
   for (int n0 = 0; n0 < N; n0 += NK) {
     __syncthreads();                                         // the last channels' tiles are done with
-    stage_tile<T, CL, NK, LQ, VEC>(Q_s, base + h * N + n0, ld, tc, N - n0, qs);
-    stage_tile<T, CL, NK, LQ, VEC>(K_s, base + HN + h * N + n0, ld, tc, N - n0, 1.f);
-    stage_tile<float, CL, NK, LQ, VEC>(B_s, la + row0 * HN + h * N + n0, HN, tc, N - n0, 1.f);
-    stage_tile<float, NK, CW, LS, VEC>(S_s, sin_c + (size_t)n0 * P, P, N - n0, P - p0, 1.f);
+    if constexpr (VEC) {
+      rb.template put<LQ>(B_s, tc, N - n0, 1.f);
+      rq.template put<LQ>(Q_s, tc, N - n0, qs);
+      rk.template put<LQ>(K_s, tc, N - n0, 1.f);
+      rs.template put<LS>(S_s, N - n0, P - p0, 1.f);
+    } else {
+      stage_tile<T, CL, NK, LQ, VEC>(Q_s, base + h * N + n0, ld, tc, N - n0, qs);
+      stage_tile<T, CL, NK, LQ, VEC>(K_s, base + HN + h * N + n0, ld, tc, N - n0, 1.f);
+      stage_tile<float, CL, NK, LQ, VEC>(B_s, la + row0 * HN + h * N + n0, HN, tc, N - n0, 1.f);
+      stage_tile<float, NK, CW, LS, VEC>(S_s, sin_c + (size_t)n0 * P, P, N - n0, P - p0, 1.f);
+    }
     __syncthreads();
+    if constexpr (VEC) {
+      if (n0 + NK < N) get(n0 + NK);                         // the next channels' tiles, beside this one's products
+      asm volatile("" ::: "memory");
+    }
     {
       // per 16-token block and channel: B = the log decays up to and with each token, E = those after it; half a wave
       // holds a block's first eight tokens, the other half its last eight.  A decay below 2^-160 counts as that: every power over it
@@ -360,18 +449,22 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
         mid += tot[j];
       }
     }
-    // the block against itself: lane holds (row 4 g4 + i, column l16), as the products' results lie
+    // the block against itself (B falls from token to token: no power grows)
+    int fr[2], fc[2];
+#pragma unroll
+    for (int m = 0; m < 2; ++m) { fold(m, fr[m], fc[m]); fr[m] += 16 * wave; fc[m] += 16 * wave; }
+    const int ro = 16 * wave + (lane & 7);
 #pragma unroll 2
     for (int n = 0; n < NK; n += 4) {
-      const float4 kv = *reinterpret_cast<const float4*>(&K_s[t][n]), bs = *reinterpret_cast<const float4*>(&B_s[t][n]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 16 * wave + 4 * g4 + i;
-        const float4 q = *reinterpret_cast<const float4*>(&Q_s[r][n]), br = *reinterpret_cast<const float4*>(&B_s[r][n]);
-        // (B falls from token to token: no power of a counted pair, column <= row, grows; the others are never read)
-        dg[i] += q.x * kv.x * ex2(br.x - bs.x) + q.y * kv.y * ex2(br.y - bs.y) + q.z * kv.z * ex2(br.z - bs.z) +
+      for (int m = 0; m < 2; ++m) {
+        const float4 q = *reinterpret_cast<const float4*>(&Q_s[fr[m]][n]), br = *reinterpret_cast<const float4*>(&B_s[fr[m]][n]);
+        const float4 kv = *reinterpret_cast<const float4*>(&K_s[fc[m]][n]), bs = *reinterpret_cast<const float4*>(&B_s[fc[m]][n]);
+        dg[m] += q.x * kv.x * ex2(br.x - bs.x) + q.y * kv.y * ex2(br.y - bs.y) + q.z * kv.z * ex2(br.z - bs.z) +
                  q.w * kv.w * ex2(br.w - bs.w);
       }
+      const float4 q = *reinterpret_cast<const float4*>(&Q_s[ro][n]), kv = *reinterpret_cast<const float4*>(&K_s[ro][n]);
+      own += q.x * kv.x + q.y * kv.y + q.z * kv.z + q.w * kv.w;
     }
   }
   __syncthreads();
@@ -381,8 +474,15 @@ __global__ void __launch_bounds__(NT) gla_chunk_out_kernel(const T* __restrict__
 #pragma unroll
     for (int j = 0; j < 3; ++j)
       if (j < wave) A_s[16 * wave + r][16 * j + l16] = off_[j][i];
-    A_s[16 * wave + r][16 * wave + l16] = l16 <= r ? dg[i] : 0.f;
+    if (l16 > r) A_s[16 * wave + r][16 * wave + l16] = 0.f;
   }
+#pragma unroll
+  for (int m = 0; m < 2; ++m) {
+    int row, col;
+    fold(m, row, col);
+    A_s[16 * wave + row][16 * wave + col] = dg[m];
+  }
+  if (lane < 8) A_s[16 * wave + lane][16 * wave + lane] = own;
   stage_tile<T, CL, CW, LS, VEC>(V_s, base + 2 * HN + h * P + p0, ld, tc, P - p0, 1.f);
   __syncthreads();
   for (int kk = 0; kk < 4 * (wave + 1); ++kk) {
@@ -511,18 +611,28 @@ int edge_sm_gla_chunked(const void* u, int ld, const float* a2, const float* b, 
   if (N < 1 || P < 1 || rank < 1) return -2;
   const bool fuse = edge_sm_gla_fused(P);
   if (!fuse && !y) return -2;
-  const int ntn = (N + CL - 1) / CL, ntp = (P + CL - 1) / CL;
+  const int ntn = (N + CL - 1) / CL, sw = P <= 64 ? 64 : 128, ntp = (P + sw - 1) / sw;
   const bool vec = N % 8 == 0 && P % 8 == 0 && ld % 8 == 0 &&
                    (((uintptr_t)u | (uintptr_t)la | (uintptr_t)sloc | (uintptr_t)out) & 31) == 0;
-#define SM_GC(V)                                                                                                             \
-  SM_T(f32, hipLaunchKernelGGL((gla_chunk_state_kernel<T, V>), dim3(max_chunks * ntn * ntp, n, H), dim3(NT),                  \
+#define SM_GCP(V, PT)                                                                                                             \
+  SM_T(f32, hipLaunchKernelGGL((gla_chunk_state_kernel<T, V, PT>), dim3(max_chunks * ntn * ntp, n, H), dim3(NT),                  \
                                0, st, (const T*)u, ld, a2, b, rank, inv_tau, seq_len, seq_off,    \
                                sloc, cdec, la, H, N, P, ntn, ntp))
+#define SM_GC(V)                 \
+  do {                           \
+    if (P <= 64) SM_GCP(V, 4);   \
+    else SM_GCP(V, 8);           \
+  } while (0)
   if (vec) SM_GC(true);
   else SM_GC(false);
+#undef SM_GCP
 #undef SM_GC
-  hipLaunchKernelGGL(gla_chunk_scan_kernel, dim3(n, H, (N * P + NT - 1) / NT), dim3(NT), 0, st, sloc, cdec, state, seq_slot,
-                     seq_start, seq_len, H, N, P);
+  if (P % 4 == 0 && (((uintptr_t)sloc | (uintptr_t)state) & 15) == 0)
+    hipLaunchKernelGGL(gla_chunk_scan_kernel<4>, dim3(n, H, (N * P / 4 + NT - 1) / NT), dim3(NT), 0, st, sloc, cdec, state, seq_slot,
+                       seq_start, seq_len, H, N, P);
+  else
+    hipLaunchKernelGGL(gla_chunk_scan_kernel<1>, dim3(n, H, (N * P + NT - 1) / NT), dim3(NT), 0, st, sloc, cdec, state, seq_slot,
+                       seq_start, seq_len, H, N, P);
 #define SM_GOV(PT, FUSE, V)                                                                                                  \
   SM_T(f32, hipLaunchKernelGGL((gla_chunk_out_kernel<T, PT, FUSE, V>), dim3(max_chunks * ((P + 16 * PT - 1) / (16 * PT)), n, \
                                H), dim3(NT), 0, st, (const T*)u, ld, la, seq_len, seq_off, sloc, norm_w, (T*)out, y, H, N, P, \
