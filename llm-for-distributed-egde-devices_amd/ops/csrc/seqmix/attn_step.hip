@@ -521,6 +521,12 @@ int edge_sm_attention_step_plan(int rows, int H, int G, int D, int Dv, int kld, 
   return plan;
 }
 
+// the estimate of what edge_sm_attention_step_plan would have an fp32 step run
+double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis, uintptr_t addresses) {
+  const int plan = edge_sm_attention_step_plan(rows, H, G, D, Dv, kld, vld, page, pool, vis, 1, addresses), sh = plan % 8, ns = plan / 8;
+  return plan ? step_us(1, sh, D, Dv, (long)rows * G * ((H / G + sh - 1) / sh) * ns, vis, ns) : attn_kernel_us(rows, H, G, D, Dv, vis);
+}
+
 size_t edge_sm_attention_step_floats(int rows, int H, int G, int Dv, int plan) {
   const int sh = plan % 8, nsplit = plan / 8;
   return nsplit > 1 ? (size_t)rows * G * ((H / G + sh - 1) / sh) * nsplit * sh * (Dv + 2) : 0;

@@ -94,6 +94,13 @@ int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const v
                            int pool, int kld, int vld, int chunked, float cap, const float* slopes, const float* sink,
                            int gate_elem, int keep_first, const float* rel, int rel_n, int out_ld, float out_scale,
                            hipStream_t st);
+int edge_sm_attention_f32_plan(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
+                               bool chunked, bool windowed, long vis, long mean, int want, uintptr_t addresses);
+int edge_sm_attention_f32(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb, const float* vb,
+                          const int* seq_slot, const int* seq_start, const int* seq_len, const int* seq_off, const int* ptab, int ptab_ld,
+                          void* out, int rows, int n, int H, int G, int D, int Dv, int PB, float scale, int window, int pool, int kld,
+                          int vld, int chunked, float cap, const float* slopes, const float* sink, int gate_elem, int keep_first,
+                          const float* rel, int rel_n, int out_ld, float out_scale, int ks, hipStream_t st);
 int edge_sm_conv_silu(const void* u, int ld, int c0, int C, const float* w, const float* bias, void* state,
                       const int* tok_seq, const int* tok_pos, const int* seq_slot, const int* seq_start,
                       const int* seq_len, const int* seq_off, void* out, int rows, int n, int taps, int f32,
@@ -419,8 +426,8 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
                         const std::optional<at::Tensor>& seq_off, int64_t n, int64_t qtiles, bool chunked, double softcap,
                         const std::optional<at::Tensor>& slopes, const std::optional<at::Tensor>& sink,
                         int64_t keep_first, const std::optional<at::Tensor>& rel, const std::optional<at::Tensor>& dst,
-                        double out_scale) {
-  // chunked: `window` is a chunk size (see attn_kernel); keep_first: the first tokens of a sequence that stay visible
+                        double out_scale, int64_t mean_keys) {
+  // mean_keys: as many as a row sees on average (0: not known; negative: minus the form of attn_f32.hip to take where it can); chunked: `window` is a chunk size (see attn_kernel); keep_first: the first tokens of a sequence that stay visible
   // behind a sliding window; rel [H, n]: a number per distance added to the scores; dst: where the result goes
   TORCH_CHECK(keep_first >= 0 && (keep_first == 0 || (window > 0 && !chunked)), "keep_first goes with a sliding window");
   chk_i32(tok_seq, "tok_seq");
@@ -479,14 +486,36 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
                 "out: [T, H Dv] in q's dtype");
   auto out = dst ? *dst : at::empty({T, H * Dv}, q.options());
   const int out_ld = (int)out.stride(0);
-  if (qtiles > 0 && q.scalar_type() == at::kBFloat16) {
-    // prompt portions in bf16 (qtiles = sum of ceil(len / 64)): the MFMA kernel when it takes the head sizes
+  const int64_t vis = (window > 0 ? std::min<int64_t>(window + keep_first, max_keys) : max_keys) + (PB ? max_keys / pool : 0);
+  const uintptr_t addresses = (uintptr_t)q.data_ptr() | (uintptr_t)kp.data_ptr() | (uintptr_t)vp.data_ptr() |
+                              (uintptr_t)(PB ? kb->data_ptr<float>() : nullptr) | (uintptr_t)(PB ? vb->data_ptr<float>() : nullptr);
+  if (qtiles > 0) {
+    // prompt portions (qtiles = sum of ceil(len / 64)): the matrix-core kernels when they take the head sizes
     TORCH_CHECK(seq_start && seq_len && seq_off, "sequence metadata missing");
     chk_i32(*seq_start, "seq_start");
     chk_i32(*seq_len, "seq_len");
     chk_i32(*seq_off, "seq_off");
     TORCH_CHECK(seq_start->numel() >= n && seq_len->numel() >= n && seq_off->numel() >= n && seq_slot.numel() >= n &&
                     qtiles * 64 >= T, "sequence metadata: [n]");
+  }
+  if (qtiles > 0 && f32(q)) {
+    const bool same = kp.data_ptr() == vp.data_ptr() && kld == vld;
+    const int form = edge_sm_attention_f32_plan((int)T, (int)H, (int)G, (int)D, (int)Dv, (int)kld, (int)vld, (int)page, PB ? (int)pool : 0,
+                                                out_ld, same, rel_p != nullptr, chunked || softcap > 0 || slopes_p,
+                                                window > 0 && window < max_keys, vis, mean_keys > 0 ? std::min(mean_keys, vis) : vis, mean_keys < 0 ? (int)-mean_keys : 0,
+                                                addresses | (uintptr_t)out.data_ptr());
+    if (form > 0) {
+      check(edge_sm_attention_f32(q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(), vp.data_ptr(),
+                                  PB ? kb->data_ptr<float>() : nullptr, PB ? vb->data_ptr<float>() : nullptr, seq_slot.data_ptr<int>(),
+                                  seq_start->data_ptr<int>(), seq_len->data_ptr<int>(), seq_off->data_ptr<int>(), ptab.data_ptr<int>(),
+                                  (int)ptab.stride(0), out.data_ptr(), (int)T, (int)n, (int)H, (int)G, (int)D, (int)Dv, PB, (float)scale,
+                                  (int)window, PB ? (int)pool : 0, (int)kld, (int)vld, chunked ? 1 : 0, (float)softcap, slopes_p, sink_p,
+                                  gate_elem, (int)keep_first, rel_p, rel_n, out_ld, (float)out_scale, form, stream()),
+            "sm_attention_f32");
+      return out;
+    }
+  }
+  if (qtiles > 0 && q.scalar_type() == at::kBFloat16) {
     const int rc = edge_sm_attention_mfma(q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(),
                                           vp.data_ptr(), PB ? kb->data_ptr<float>() : nullptr,
                                           PB ? vb->data_ptr<float>() : nullptr, seq_slot.data_ptr<int>(),
@@ -500,9 +529,6 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
       return out;
     }
   }
-  const int64_t vis = (window > 0 ? std::min<int64_t>(window + keep_first, max_keys) : max_keys) + (PB ? max_keys / pool : 0);
-  const uintptr_t addresses = (uintptr_t)q.data_ptr() | (uintptr_t)kp.data_ptr() | (uintptr_t)vp.data_ptr() |
-                              (uintptr_t)(PB ? kb->data_ptr<float>() : nullptr) | (uintptr_t)(PB ? vb->data_ptr<float>() : nullptr);
   // few queries over many keys (decode steps): several workgroups may share a query's keys
   int plan = edge_sm_attention_step_plan((int)T, (int)H, (int)G, (int)D, (int)Dv, (int)kld, (int)vld, (int)page,
                                          PB ? (int)pool : 0, vis, f32(q), addresses);

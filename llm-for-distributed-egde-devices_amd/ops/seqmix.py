@@ -262,6 +262,18 @@ def parallel_step_in(u: torch.Tensor, meta: RaggedMeta, rope: Optional[torch.Ten
 ATTN_MFMA_MIN = int(__import__("os").environ.get("EDGELLM_ATTN_MFMA_MIN", "16"))
 
 
+def _portions(meta: RaggedMeta, q: torch.Tensor, window: Optional[int]):
+    """What the matrix-core attention of prompt portions asks about a step: tiles of 64 query rows (0: no portion of ATTN_MFMA_MIN
+    tokens), and for fp32 how many keys a row sees on average (a portion's middle row stands for it)."""
+    if meta.max_len < ATTN_MFMA_MIN:
+        return 0, 0
+    keys = 0
+    if q.dtype == torch.float32:
+        w = window if window else 1 << 30
+        keys = sum(n * min(start + n // 2 + 1, w) for _, start, n, _ in meta.host) // max(meta.T, 1)
+    return sum((h[2] + 63) // 64 for h in meta.host), keys
+
+
 def window_pool_attention(q: torch.Tensor, gate: Optional[torch.Tensor], k_pages, v_pages, k_pool, v_pool,
                           meta: RaggedMeta, scale: float, window: Optional[int], pool: Optional[int],
                           sink: Optional[torch.Tensor] = None, keep_first: int = 0, rel: Optional[torch.Tensor] = None,
@@ -277,16 +289,14 @@ def window_pool_attention(q: torch.Tensor, gate: Optional[torch.Tensor], k_pages
     G, Dv = k_pages.shape[2], v_pages.shape[3]
     assert rel is None or not pool, "pooled blocks have no distance"
     if _gpu(q):
-        # bf16 steps with a portion of ATTN_MFMA_MIN tokens or more: the MFMA kernel (64 query rows per
-        # workgroup); decode-sized steps: attn_step.hip where its plan takes the sizes; else one workgroup per (token, kv head)
-        qtiles = 0
-        if q.dtype == torch.bfloat16 and meta.max_len >= ATTN_MFMA_MIN:
-            qtiles = sum((h[2] + 63) // 64 for h in meta.host)
+        # steps with a portion of ATTN_MFMA_MIN tokens or more: the MFMA kernels (64 query rows per
+        # workgroup; attn_f32.hip in fp32); decode-sized steps: attn_step.hip where its plan takes the sizes; else one workgroup per (token, kv head)
+        qtiles, mean = _portions(meta, q, window)
         return _ext().sm_attention(q, gate, k_pages, v_pages, k_pool if pool else None, v_pool if pool else None,
                                    meta.tok_seq, meta.tok_pos, meta.seq_slot, meta.page_table, float(scale),
                                    int(window) if window is not None else 0, int(pool or 0), int(meta.max_keys),
                                    meta.seq_start, meta.seq_len, meta.seq_off, int(meta.n), int(qtiles), False, 0.0,
-                                   None, sink, int(keep_first if window is not None else 0), rel, out, float(out_scale))
+                                   None, sink, int(keep_first if window is not None else 0), rel, out, float(out_scale), mean)
     page = meta.page
     res = torch.empty(T, H, Dv, dtype=torch.float32, device=q.device)
     R = H // G
@@ -364,13 +374,11 @@ def chunk_attention(q: torch.Tensor, gate: Optional[torch.Tensor], k_pages: torc
     T, H, D = q.shape
     G = k_pages.shape[2]
     if _gpu(q):
-        qtiles = 0
-        if q.dtype == torch.bfloat16 and meta.max_len >= ATTN_MFMA_MIN:
-            qtiles = sum((h[2] + 63) // 64 for h in meta.host)
+        qtiles, mean = _portions(meta, q, chunk)
         return _ext().sm_attention(q, gate, k_pages, k_pages, None, None, meta.tok_seq, meta.tok_pos, meta.seq_slot,
                                    meta.page_table, float(scale), int(chunk or 0), 0, int(meta.max_keys), meta.seq_start,
                                    meta.seq_len, meta.seq_off, int(meta.n), int(qtiles), True, float(softcap or 0.0),
-                                   slopes, sink, 0, None, None, 1.0)
+                                   slopes, sink, 0, None, None, 1.0, mean)
     page, R = meta.page, H // G
     out = torch.empty(T, H, D, dtype=torch.float32, device=q.device)
     for slot, start, n, off in meta.host:
