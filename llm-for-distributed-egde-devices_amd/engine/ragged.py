@@ -72,8 +72,7 @@ class _DecodeGraph:
         self.raw.copy_(hraw, non_blocking=True)
         ev.record()
         eng = self.eng
-        # a model that nobody watches is captured up to its output projection's rows: making logits of them also takes them out of
-        # the graph's memory, and every row is wanted
+        # a model that nobody watches is captured up to its output projection, which then leaves its logits outside the graph's memory
         watched = type(eng.model).forward is not HybridLM.forward or not unwatched(eng.model)
         if not self.warm:
             self.warm = True
@@ -91,7 +90,7 @@ class _DecodeGraph:
             try:
                 with torch.cuda.graph(g, pool=eng._pool):
                     self.out = eng.model(self.ids, self.meta, eng.cache) if watched else \
-                        eng.model.scores(self.ids, self.meta, eng.cache)
+                        eng.model.last_rows(self.ids, self.meta, eng.cache)
                 self.raw_out = not watched
             except Exception as e:  # noqa: BLE001 - an op that cannot be captured: this engine steps eagerly
                 from ..utils.log import get_logger
@@ -106,7 +105,7 @@ class _DecodeGraph:
                 eng._pool = g.pool()
             self.graph = g
         self.graph.replay()
-        return eng.model.finish(self.out) if self.raw_out else self.out.clone()
+        return eng.model.logits(self.out) if self.raw_out else self.out.clone()
 
 
 class RaggedEngine:

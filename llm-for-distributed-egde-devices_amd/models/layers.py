@@ -225,6 +225,15 @@ class Linear(nn.Module):
         return ops.linear_bf16(x, self.weight, self.bias, packed=wp,
                                add=None if add is None else add.reshape(*x.shape[:-1], self.out_features))
 
+    def forward_f32(self, x) -> "Optional[torch.Tensor]":
+        """Up to 16 bf16 rows' outputs as fp32 numbers straight from the GEMV (the values of ``forward`` widened), or None where that
+        does not run."""
+        K = self.in_features
+        if x.dtype != torch.bfloat16 or x.numel() > 16 * K or not plain_linear(self) or self.split_k_out or \
+                ops.bf16_decode_mode(x, self.weight) != 1 or not ops.raw_call(x, self.weight):
+            return None
+        return ops.ext().gemv_bf16(x, self.decode_weight(x), None, self.out_features, 7, None)
+
     def rows16_ok(self, x, glu: bool = False, split: bool = False) -> bool:
         """Whether ``gemm_rows16.hip`` takes these rows.  Whoever watches the projection (a calibration's hooks, say) gets the
         numbers of the kernels that serve other row counts too."""

@@ -825,7 +825,7 @@ at::Tensor gemv_bf16(const at::Tensor& x, const at::Tensor& wp, const std::optio
   if (bias) { need_same(*bias, x, "bias"); TORCH_CHECK(bias->numel() == N); }
   auto os = x.sizes().vec();
   os.back() = epi == 1 ? N / 2 : N;
-  auto out = at::empty(os, x.options());
+  auto out = at::empty(os, epi == 7 ? x.options().dtype(at::kFloat) : x.options());
   if (addend) {
     need_same(*addend, x, "addend");
     TORCH_CHECK(epi == 0 && addend->numel() == M * N, "addend: plain output only, M * N elements");

@@ -5,7 +5,8 @@
 namespace {
 constexpr int EPI_OUT = 0, EPI_GLU = 1, EPI_GELU_TANH = 2, EPI_GELU = 3, EPI_PART = 4,
               EPI_GELU_ANY = 5,               // gelu, tanh where F is 1, else erf
-              EPI_ADD = 6;                    // EPI_OUT and an addend
+              EPI_ADD = 6,                    // EPI_OUT and an addend
+              EPI_F32 = 7;                    // EPI_OUT's 16-bit numbers, stored as fp32
 constexpr int GEMV_NW = 16;
 
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
@@ -405,7 +406,11 @@ __device__ __forceinline__ void gemv_tiles_body(int bid, int nwg, const bf16_t* 
               // (parallel-residual block): rnd(rnd(y) + add), the unfused add
               v = e2f<HF>(f2e<HF>(v)) + e2f<HF>(addv[q]);
             }
-            if (row < M) out[(size_t)row * N + c] = f2e<HF>(v);
+            if constexpr (EPI == EPI_F32) {
+              if (row < M) reinterpret_cast<float*>(out)[(size_t)row * N + c] = e2f<HF>(f2e<HF>(v));
+            } else {
+              if (row < M) out[(size_t)row * N + c] = f2e<HF>(v);
+            }
           }
         }
       }
@@ -528,7 +533,11 @@ __device__ __forceinline__ void gemv_bf16_body(int bid, const bf16_t* __restrict
           // EPI_OUT with an addend (parallel-residual block): rnd(rnd(y) + add), the unfused add
           if (add != nullptr && row < M && c0 < N) v = e2f<HF>(f2e<HF>(v)) + e2f<HF>(add[(size_t)row * N + c0]);
         }
-        if (row < M && c0 < N) out[(size_t)row * N + c0] = f2e<HF>(v);
+        if constexpr (EPI == EPI_F32) {
+          if (row < M && c0 < N) reinterpret_cast<float*>(out)[(size_t)row * N + c0] = e2f<HF>(f2e<HF>(v));
+        } else {
+          if (row < M && c0 < N) out[(size_t)row * N + c0] = f2e<HF>(v);
+        }
       }
     }
   }

@@ -117,12 +117,20 @@ int launch(const void* A, const void* W, const void* bias, void* out, int M, int
 
 // W: fragment-packed bf16 (ops.pack_bf16_weight).  epi 0: out bf16 [M, N] (+ the bf16 addend `add`
 // [M, N] when not null: a parallel-residual block's other branch); epi 1 (GLU):
-// W = [gate | up] with N = 2F, out = silu(gate) * up bf16 [M, F] (F % 16 == 0); epi 2 / 3: gelu (tanh / erf) of the bf16 output.  M <= 64, K % 64 == 0,
+// W = [gate | up] with N = 2F, out = silu(gate) * up bf16 [M, F] (F % 16 == 0); epi 2 / 3: gelu (tanh / erf) of the bf16 output; epi 7: epi 0's
+// numbers as fp32 (bf16, M <= 16, no addend).  M <= 64, K % 64 == 0,
 // N % 16 == 0.  Returns -2 for shapes it does not take.
 template <bool HF>
 int gemv_run(const void* A, const void* W, const void* bias, void* out, int M, int N, int K, int epi, hipStream_t st,
              const void* add) {
   if (M <= 0 || M > 64 || K % 64 != 0 || N % 16 != 0 || N <= 0 || K <= 0) return -2;
+  if (epi == EPI_F32) {                                      // scores that a program reads in fp32: up to 16 bf16 rows, no copy behind them
+    if (HF || M > 16 || add != nullptr) return -2;
+    const int nt = N / 16;
+    if (tiles_form(M, N, K, epi)) return launch_tiles_rows<EPI_F32, false>(A, W, bias, out, M, N, K, st);
+    return nt >= 1024 ? launch_mb<1, 4, 2, EPI_F32, false>(A, W, bias, out, M, N, K, 0, nt, st, 1)
+                      : launch_mb<1, 2, 4, EPI_F32, false>(A, W, bias, out, M, N, K, 0, nt, st, 1);
+  }
   if (tiles_form(M, N, K, epi)) {
     switch (epi) {
       case EPI_OUT: return add == nullptr ? launch_tiles_rows<EPI_OUT, HF>(A, W, bias, out, M, N, K, st)
