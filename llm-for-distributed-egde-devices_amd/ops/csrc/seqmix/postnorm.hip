@@ -1031,10 +1031,12 @@ int edge_sm_canon(const float* x, int W, const float* w, float* state, const int
   if (taps < 1 || taps > 16) return -2;
   const bool one = max_len == 1 && taps > 1;                 // every sequence brings one token
   const int gy = (W + NT * 4 - 1) / (NT * 4);
-  if (tap4_ok<float>(taps, W, 0, W, x, w, state, out))
-    SM_T(f32, (launch_tap4<float, T, false>(x, W, 0, W, w, nullptr, state, tok_seq, tok_pos, seq_slot, seq_start, (T*)out, rows,
-                                            one, st)));
-  else if (W % 4 == 0)
+  if (tap4_ok<float>(taps, W, 0, W, x, w, state, out)) {
+    SM_T(f32, (launch_tap4<float, T, false>(x, W, 0, W, w, nullptr, state, tok_seq, tok_pos, seq_slot, seq_start, seq_len, seq_off, (T*)out,
+                                            rows, n, one, st)));
+    return (int)hipGetLastError();
+  }
+  if (W % 4 == 0)
     SM_T(f32, hipLaunchKernelGGL((canon_kernel<T, true>), dim3(rows, gy), dim3(NT), 0, st, x, W, w, (const float*)state,
                                  tok_seq, tok_pos, seq_slot, seq_start, seq_off, (T*)out, taps,
                                  one ? state : (float*)nullptr));

@@ -1063,10 +1063,12 @@ int edge_sm_conv_silu(const void* u, int ld, int c0, int C, const float* w, cons
   const bool one = max_len == 1 && taps > 1;                 // every sequence brings one token
   const int tokb = rows >= 64 * TOKB ? TOKB : 1;             // decode-sized steps: one token per workgroup
   const int gy = (C + NT - 1) / NT;
-  if (f32 ? tap4_ok<float>(taps, ld, c0, C, u, w, state, out) : tap4_ok<bf16_t>(taps, ld, c0, C, u, w, state, out))
-    SM_T(f32, (launch_tap4<T, T, true>((const T*)u, ld, c0, C, w, bias, (T*)state, tok_seq, tok_pos, seq_slot, seq_start,
-                                       (T*)out, rows, one, st)));
-  else if (ld % 8 == 0 && c0 % 8 == 0 && C % 8 == 0)
+  if (f32 ? tap4_ok<float>(taps, ld, c0, C, u, w, state, out) : tap4_ok<bf16_t>(taps, ld, c0, C, u, w, state, out)) {
+    SM_T(f32, (launch_tap4<T, T, true>((const T*)u, ld, c0, C, w, bias, (T*)state, tok_seq, tok_pos, seq_slot, seq_start, seq_len,
+                                       seq_off, (T*)out, rows, n, one, st)));
+    return (int)hipGetLastError();
+  }
+  if (ld % 8 == 0 && c0 % 8 == 0 && C % 8 == 0)
     SM_T(f32, hipLaunchKernelGGL((conv_kernel<T, true>), dim3((rows + tokb - 1) / tokb, (C / 8 + NT - 1) / NT), dim3(NT),
                                  0, st, (const T*)u, ld, c0, C, w, bias, (const T*)state, tok_seq, tok_pos, seq_slot,
                                  seq_start, seq_off, (T*)out, taps, one ? (T*)state : (T*)nullptr, rows, tokb));
