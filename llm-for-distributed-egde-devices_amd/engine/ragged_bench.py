@@ -261,7 +261,7 @@ def bench_hybrid(s: dict, prompt: int, batch: int, steps: int, device, cfg: Mode
 # what the layers call in ops.seqmix, each of which a breakdown names
 STEP_OPS = ["embedding_scaled", "scalar_rms_norm", "relu2", "cat_cast", "combine_residual", "gated_group_norm",
             "rope_paged_write", "pool_blocks", "window_pool_attention", "conv_silu", "ssd_scan", "linear_f32",
-            "embedding_bigram", "canon_conv", "layer_norm_rows", "layer_norm_residual", "rms_norm_cols", "glu_clamp",
+            "embedding_bigram", "embedding_bigram_canon", "canon_conv", "layer_norm_rows", "layer_norm_residual", "rms_norm_cols", "glu_clamp",
             "latent_write", "delta_prepare", "delta_rule_scan", "head_norm_gate", "moe_route", "moe_experts",
             "group_rms_norm", "group_norm_residual", "chunk_attention", "delta_prepare_head", "glu_silu",
             "hyper_read_norm", "hyper_update", "poly_norm", "qk_norm_rope_write", "unrotate_gate",
