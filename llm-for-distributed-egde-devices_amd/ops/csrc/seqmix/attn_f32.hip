@@ -323,12 +323,12 @@ double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int 
 // Waves of query rows of a group in the low bits, groups above; 0: the step is not this kernel's.  vis: the most keys that a row sees,
 // mean: as many as a row sees on average.  By estimates: an iteration is one tile of every group, its us were fitted to steps of up to six
 // portions of 16 to 600 tokens behind 0 to 1500 (112 of them, eight head shapes of 32 to 160 numbers), and the kernels before are
-// taken at 0.75 (0.65 of few heads) of theirs, whose chains they overrate; or the form that the caller wants.  Chosen so, 150 other steps took 0.71 of the time before (worst 1.1, 30 us); us before / four
+// taken at 0.75 (0.65 of few heads) of theirs, whose chains they overrate; or the form that the caller wants.  Chosen so, 150 other steps took 0.71 of the time before (worst 1.3: 191 rows of 16 heads of 128, 16 / 21); us before / four
 // waves and two groups / two and two / two and four: 16 heads of 64 in 4 groups, 2000 tokens 342 / 102 / 118 / 123, 500 behind 2000 215 /
 // 112 / 85 / 68, 100 8.8 / 10.9 / 9.2 / 9.6, 20 behind 1000 16.7 / 48 / 37 / 30; of 128, 1000 tokens 205 / 87 / 78; 16 of 160 over one
 // latent, 300 tokens 65 / 33 / 26; a group per head of 64, 2000 tokens 1115 / 102 / 117 / 122.
 // Error against 64 bits, relative: 1000 tokens 2.3e-7 before, 1.4e-7 here; 500 behind 2000 3.4e-7, 2.0e-7.
-int edge_sm_attention_f32_plan(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
+int edge_sm_attention_f32_plan(int rows, int n, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
                                bool chunked, bool windowed, long vis, long mean, int want, uintptr_t addresses) {
   if ((same ? pool > 0 || rel : chunked) || (pool & (pool - 1)) || page != FK || G < 1 || H % G || rows < 1 || kld % 4 || vld % 4 ||
       out_ld % 4 || addresses % 16)
@@ -340,9 +340,14 @@ int edge_sm_attention_f32_plan(int rows, int H, int G, int D, int Dv, int kld, i
   int plan = 0;
   const double w = (D + Dv) / 2, tiles = mean / (double)FK + 0.8, waves = rows * (double)H / 16;
   const long longest = (vis + FK - 1) / FK + (windowed ? 1 : 0);   // (a window begins inside a tile)
-  // us: an iteration; crowd: what workgroups that share a CU lose over one that has it
+  // us: an iteration; crowd: what workgroups that share a CU lose over one that has it.  Behind a window all workgroups are as long, and
+  // come in rounds of 256 (530 rows of 16 heads, window 512: 272 workgroups of two and four 44 us, 136 of four and two 34)
+  const bool even = windowed && mean * 10 >= vis * 8;
+  const int R = H / G;
   auto form = [&](int rw, int ks, double us, double crowd) {
-    const double chain = (longest + ks - 1) / ks * us, work = crowd * waves / rw / 256 * tiles / ks * us;
+    const int hw = rw == 4 && R % 4 == 0 ? 4 : R % 2 == 0 ? 2 : 1;
+    const double chain = (longest + ks - 1) / ks * us, wgs = (rows * hw / (16. * rw) + n / 2.) * (H / hw);
+    const double work = even ? ceil(wgs / 256 - 0.02) * chain : crowd * waves / rw / 256 * tiles / ks * us;
     const double t = 5.5 + (chain > work ? chain : work);
     if (t < best) { best = t; plan = rw + 8 * ks; }
   };

@@ -94,7 +94,7 @@ int edge_sm_attention_mfma(const void* q, const void* gate, int gate_ld, const v
                            int pool, int kld, int vld, int chunked, float cap, const float* slopes, const float* sink,
                            int gate_elem, int keep_first, const float* rel, int rel_n, int out_ld, float out_scale,
                            hipStream_t st);
-int edge_sm_attention_f32_plan(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
+int edge_sm_attention_f32_plan(int rows, int n, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
                                bool chunked, bool windowed, long vis, long mean, int want, uintptr_t addresses);
 int edge_sm_attention_f32(const void* q, const void* gate, int gate_ld, const void* kp, const void* vp, const float* kb, const float* vb,
                           const int* seq_slot, const int* seq_start, const int* seq_len, const int* seq_off, const int* ptab, int ptab_ld,
@@ -500,7 +500,7 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
   }
   if (qtiles > 0 && f32(q)) {
     const bool same = kp.data_ptr() == vp.data_ptr() && kld == vld;
-    const int form = edge_sm_attention_f32_plan((int)T, (int)H, (int)G, (int)D, (int)Dv, (int)kld, (int)vld, (int)page, PB ? (int)pool : 0,
+    const int form = edge_sm_attention_f32_plan((int)T, (int)n, (int)H, (int)G, (int)D, (int)Dv, (int)kld, (int)vld, (int)page, PB ? (int)pool : 0,
                                                 out_ld, same, rel_p != nullptr, chunked || softcap > 0 || slopes_p,
                                                 window > 0 && window < max_keys, vis, mean_keys > 0 ? std::min(mean_keys, vis) : vis, mean_keys < 0 ? (int)-mean_keys : 0,
                                                 addresses | (uintptr_t)out.data_ptr());
