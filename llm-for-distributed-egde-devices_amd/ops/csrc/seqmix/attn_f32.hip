@@ -331,7 +331,7 @@ double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int 
 int edge_sm_attention_f32_plan(int rows, int n, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
                                bool chunked, bool windowed, long vis, long mean, int want, uintptr_t addresses) {
   if ((same ? pool > 0 || rel : chunked) || (pool & (pool - 1)) || page != FK || G < 1 || H % G || rows < 1 || kld % 4 || vld % 4 ||
-      out_ld % 4 || addresses % 16)
+      out_ld % 4 || addresses % 16 || rows / 16 + n > 65535)   // (the grid's second number)
     return 0;
   const bool square = D == Dv && (D == 32 || D == 64 || D == 96 || D == 128);
   if (!square && !(same ? D == 160 && Dv == 128 : (D == 64 && Dv == 128) || (D == 128 && Dv == 64))) return 0;
