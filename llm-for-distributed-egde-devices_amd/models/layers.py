@@ -329,10 +329,11 @@ def plain_linear(m: nn.Module) -> bool:
 
 
 def rows_gated(xs, mods, z, norm_w, eps: float):
-    """``rows_together`` of fp32 rows where the last input is xs[2] silu(z), normed over the row under ``norm_w``, in the same launch;
-    None where that kernel does not run."""
+    """``rows_together`` of up to 4 fp32 rows where the last input is xs[2] silu(z), normed over the row under ``norm_w``, in the same launch
+    (more rows spilled the kernel's registers); None where that kernel does not run."""
     y = xs[2]
-    if all(plain_linear(m) and not m.split_k_out for m in mods) and all(x.dim() == 2 and x.is_contiguous() for x in xs) and \
+    if y.shape[0] <= 4 and all(plain_linear(m) and not m.split_k_out for m in mods) and \
+            all(x.dim() == 2 and x.is_contiguous() for x in xs) and \
             all(ops.f32_rows_ok(x, m.weight) for x, m in zip(xs, mods)) and z.dtype == norm_w.dtype == torch.float32 and \
             ops.raw_call(z, norm_w) and z.shape == y.shape and z.stride(1) == 1 and z.stride(0) % 4 == 0 and norm_w.is_contiguous() and \
             z.device == norm_w.device == y.device and (z.data_ptr() | norm_w.data_ptr()) % 16 == 0 and norm_w.numel() == y.shape[1]:

@@ -122,11 +122,12 @@ struct Jobs3 {
   float* y[3];
   int N[3], K[3], KW[3], n[2];
 };
-template <int MV, int R, bool GATED>
+// RG > 0: the last one's input is gated and normed, RG weight rows a wave (four at 4 rows spilled: 36 bytes a lane)
+template <int MV, int R, int RG>
 __global__ void __launch_bounds__(1024) gemv_f32x3_kernel(Jobs3 a, int M, Gate g) {
   const int bid = blockIdx.x, j = bid < a.n[0] ? 0 : bid < a.n[1] ? 1 : 2;
-  if constexpr (GATED)
-    if (j == 2) return gemv_f32_body<MV, R, true>(bid - a.n[1], a.x[2], a.W[2], nullptr, a.y[2], M, a.N[2], a.K[2], a.KW[2], g);
+  if constexpr (RG > 0)
+    if (j == 2) return gemv_f32_body<MV, RG, true>(bid - a.n[1], a.x[2], a.W[2], nullptr, a.y[2], M, a.N[2], a.K[2], a.KW[2], g);
   gemv_f32_body<MV, R>(bid - (j == 0 ? 0 : a.n[j - 1]), a.x[j], a.W[j], nullptr, a.y[j], M, a.N[j], a.K[j], a.KW[j]);
 }
 
@@ -145,27 +146,27 @@ void launch_f32(const float* x, const float* W, const float* bias, float* y, int
   hipLaunchKernelGGL((gemv_f32_kernel<MV, R>), dim3((groups + per - 1) / per), dim3(waves * 64), 0, st, x, W, bias, y, M, N, K, KW);
 }
 
-template <int MV, int R>
+template <int MV, int R, int RG>
 void launch_f32x3(Jobs3 a, int M, const Gate& g, hipStream_t st) {
   int waves = 4, blocks = 0;
+  auto rows = [](int j) { return j == 2 && RG > 0 ? RG : R; };
   for (int j = 0; j < 3; ++j) {
-    a.KW[j] = share_k((a.N[j] + R - 1) / R, a.K[j]);
+    a.KW[j] = share_k((a.N[j] + rows(j) - 1) / rows(j), a.K[j]);
     waves = a.KW[j] > waves ? a.KW[j] : waves;
   }
   for (int j = 0; j < 3; ++j) {
     const int per = waves / a.KW[j];
-    blocks += ((a.N[j] + R - 1) / R + per - 1) / per;
+    blocks += ((a.N[j] + rows(j) - 1) / rows(j) + per - 1) / per;
     if (j < 2) a.n[j] = blocks;
   }
-  if (g.z != nullptr) hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R, true>), dim3(blocks), dim3(waves * 64), 0, st, a, M, g);
-  else hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R, false>), dim3(blocks), dim3(waves * 64), 0, st, a, M, g);
+  hipLaunchKernelGGL((gemv_f32x3_kernel<MV, R, RG>), dim3(blocks), dim3(waves * 64), 0, st, a, M, g);
 }
 }  // namespace
 
 // y_j = x_j W_j^T for three projections of the same M rows' inputs, each as edge_gemv_f32 forms it: a parallel layer's three output
 // projections, whose launches' ramps and ends then overlap.  us in a graph, weights from memory, three launches / one, 1024 x 4096 and
 // twice 1024 x 1024: 1 row 11.1 / 6.8, 2 11.5 / 7.0, 8 15.1 / 11.4; 2048 x 8192 and twice 2048 x 2048, 2 rows 24.0 / 18.8
-// gate_z (null: none): x_2 is gated by its rows, z_ld apart, and normed under gate_w first; 16-byte aligned, z_ld % 4 == 0
+// gate_z (null: none; up to 4 rows): x_2 is gated by its rows, z_ld apart, and normed under gate_w first; 16-byte aligned, z_ld % 4 == 0
 extern "C" int edge_gemv_f32x3(const float* const* x, const float* const* W, float* const* y, int M, const int* N, const int* K,
                                const float* gate_z, int z_ld, const float* gate_w, float eps, hipStream_t st) {
   const Gate g{gate_z, gate_w, z_ld, eps};
@@ -175,11 +176,15 @@ extern "C" int edge_gemv_f32x3(const float* const* x, const float* const* W, flo
     if (N[j] < 1 || K[j] < 4 || K[j] % 4) return -2;
     a.x[j] = x[j]; a.W[j] = W[j]; a.y[j] = y[j]; a.N[j] = N[j]; a.K[j] = K[j];
   }
-  if (M < 1 || M > 8) return -2;
-  if (M == 1) launch_f32x3<1, 4>(a, M, g, st);
-  else if (M == 2) launch_f32x3<2, 4>(a, M, g, st);
-  else if (M <= 4) launch_f32x3<4, 4>(a, M, g, st);
-  else launch_f32x3<8, 2>(a, M, g, st);
+  if (M < 1 || M > (gate_z ? 4 : 8)) return -2;
+  if (gate_z != nullptr) {
+    if (M == 1) launch_f32x3<1, 4, 4>(a, M, g, st);
+    else if (M == 2) launch_f32x3<2, 4, 4>(a, M, g, st);
+    else launch_f32x3<4, 4, 2>(a, M, g, st);
+  } else if (M == 1) launch_f32x3<1, 4, 0>(a, M, g, st);
+  else if (M == 2) launch_f32x3<2, 4, 0>(a, M, g, st);
+  else if (M <= 4) launch_f32x3<4, 4, 0>(a, M, g, st);
+  else launch_f32x3<8, 2, 0>(a, M, g, st);
   return (int)hipGetLastError();
 }
 

@@ -1,12 +1,12 @@
 """The gated norm in front of the last of three projections, in their launch (gemv_f32.hip), against float64: widths beside a wave's
-256 k, every count of rows, gates that are columns of a wider row."""
+256 k, the row counts that it takes, gates that are columns of a wider row."""
 import pytest
 import torch
 
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("M", [1, 2, 3, 5, 8])
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
 @pytest.mark.parametrize("sizes", [((1024, 4096), (1024, 1024), (1024, 1024)), ((5, 4), (1, 260), (130, 1020)), ((16, 64), (3, 2052), (7, 4)),
                                    ((64, 256), (64, 256), (2048, 2048))])
 @pytest.mark.parametrize("small", [False, True])
@@ -45,3 +45,5 @@ def test_what_the_launch_takes(cuda):
     assert mixers.rows_gated((x, x, y), (m.left.o, m.left.o, m.right.o), z.t().contiguous().t(), m.right.norm_w, 1e-6) is None
     assert mixers.rows_gated((x, x, y.t().contiguous().t()), (m.left.o, m.left.o, m.right.o), z, m.right.norm_w, 1e-6) is None
     assert mixers.rows_gated((x, x, y), (m.left.o, m.left.o, m.right.o), z.bfloat16(), m.right.norm_w, 1e-6) is None
+    x5, y5, z5 = x[:1].repeat(5, 1), y[:1].repeat(5, 1), z[:1].repeat(5, 1)              # more rows: the norm in a launch of its own
+    assert mixers.rows_gated((x5, x5, y5), (m.left.o, m.left.o, m.right.o), z5, m.right.norm_w, 1e-6) is None
