@@ -328,7 +328,7 @@ __global__ void __launch_bounds__(NT) gla_chunk_scan_kernel(float* __restrict__ 
         S = dec[b][i] * S + own[b][i];
       }
   };
-  get(0, 0);
+  if (nc > 0) get(0, 0);                                     // (a portion of no token has no row to clamp to)
   for (int c0 = 0; c0 < nc; c0 += 2 * UN) {
     if (c0 + UN < nc) get(1, c0 + UN);
     use(0, c0);

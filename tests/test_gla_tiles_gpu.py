@@ -45,3 +45,20 @@ def test_chunks_at_the_edges_of_their_tiles(cuda, dt, H, N, P, rank, seqs):
     tol = 2e-6 if dt == torch.float32 else 2.0 ** -9
     assert (got - want).norm() < tol * want.norm()
     assert (state.double().cpu() - end).norm() < 2e-6 * end.norm()
+
+
+@pytest.mark.parametrize("N,P", [(64, 64), (20, 30)])        # scans of four numbers and of one
+def test_portions_without_a_token(cuda, N, P):
+    """They read no row of the chunks' states (the first one's would lie in front of them), keep a state that continues and clear one
+    that starts."""
+    H, rank, seqs = 2, 8, [(2, 5, 0), (0, 3, 130), (3, 0, 0), (1, 0, 70), (4, 9, 0)]
+    g = torch.Generator().manual_seed(N)
+    u = torch.randn(200, 2 * H * N + 2 * H * P + rank, generator=g).cuda()
+    a2, b = (torch.randn(H * N, rank, generator=g) * rank ** -0.5).cuda(), torch.randn(H * N, generator=g).cuda()
+    nw, state = (1 + 0.1 * torch.randn(P, generator=g)).cuda(), torch.randn(5, H, N, P, generator=g).cuda()
+    want, end = _reference(u, a2, b, nw, state, seqs, H, N, P, 8.0, 1e-6)
+    meta = S.RaggedMeta.build(seqs, torch.zeros(5, 1, dtype=torch.int32, device="cuda"), 64, torch.device("cuda"))
+    got = S.gated_linear_attention(u, a2, b, nw, state, meta, H, N, P, 8.0, 1e-6).double().cpu()
+    assert (got - want).norm() < 2e-6 * want.norm()
+    assert (state.double().cpu() - end).norm() < 2e-6 * end.norm()
+    assert torch.equal(state[[2, 4]].double().cpu(), end[[2, 4]]) and not state[3].any()
