@@ -15,7 +15,7 @@
 // 1369 -> 169 us, where the experts' 805 MB (4.8 TB/s) are the bound.  At 128-row tiles the bound is the LDS: 64 B per clock and
 // CU come in and 128 are read at the full MFMA rate (tile_rows says what 256-row tiles change); 128 x 256 tiles gained 3-6 %
 // from 2048 columns on and lost below, deeper rings with one workgroup of 128 x 128 per CU lose 40 %; a third stage for the
-// weights alone still leaves two workgroups a CU and gains 2-15 % (edge_sm_moe_gemm).
+// weights alone still leaves two workgroups a CU (deep_ring).
 #include "seqmix_common.h"
 
 namespace {
@@ -112,7 +112,9 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   static_assert(AP % NWV == 0 && BP % NWV == 0 && (!GLU || NJ % 2 == 0) && (RA - RW) * (RA - RW) <= 1, "tile shape");
   static_assert((RA * AP + RW * BP) * 1024 <= 160 * 1024, "LDS");
   __shared__ __attribute__((aligned(1024))) int8_t ring[(RA * AP + RW * BP) * 1024];
-  constexpr int W0 = RA * AP * 1024;                         // the weights' stages
+  // equal rings: a stage's rows and weights side by side (apart, 64-row tiles of small steps took 0.3 to 0.5 us of 21 more); else two rings
+  constexpr bool EVEN = RA == RW;
+  constexpr int W0 = (EVEN ? 1 : RA) * AP * 1024, SA = (AP + (EVEN ? BP : 0)) * 1024, SW = (BP + (EVEN ? AP : 0)) * 1024;
 
   const int nwg = tiles[0] * grid_n, orig = blockIdx.x;
   if (orig >= nwg) return;
@@ -159,7 +161,7 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   auto issue = [&](int st, bool weights) {
     const int kt = min(st, KT - 1) + k0;
     const size_t ko = (size_t)(kt < KT ? kt : kt - KT) * 128;
-    int8_t* slot = ring + (weights ? W0 + (st % RW) * (BP * 1024) : (st % RA) * (AP * 1024)) + wave * 1024;
+    int8_t* slot = ring + (weights ? W0 + (st % RW) * SW : (st % RA) * SA) + wave * 1024;
 #pragma unroll
     for (int i = 0; i < (weights ? PB : PA); ++i) glds16(src[weights ? PA + i : i] + ko, slot + NWV * i * 1024);
   };
@@ -172,8 +174,8 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   const uint32_t fo = lds_off(ring) + (lane & 15) * 128 + (((lane >> 4) ^ (lane & 7)) << 4);
   auto read = [&](int st, int ks, v4i (&fa)[MI], v4i (&fw)[NJ]) {
     const uint32_t b = fo ^ (ks << 6);
-    lds_frags<0, MI>(b + (st % RA) * (AP * 1024) + wm * (MI * 2048), fa);
-    lds_frags<0, NJ>(b + W0 + (st % RW) * (BP * 1024) + wn * (NJ * 2048), fw);
+    lds_frags<0, MI>(b + (st % RA) * SA + wm * (MI * 2048), fa);
+    lds_frags<0, NJ>(b + W0 + (st % RW) * SW + wn * (NJ * 2048), fw);
   };
   v4f acc[MI][NJ];
 #pragma unroll
@@ -253,24 +255,6 @@ __global__ void __launch_bounds__(64 * WM * WN, 2) moe_gemm_kernel(const bf16_t*
   }
 }
 
-template <int BM, int BN, int WM, int WN, int RA, int RW>
-int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* rows, const int* tiles, void* y, void* out,
-                int max_tiles, int top, int W, int ff, int act, const float* row_w, float limit, int spread, hipStream_t st) {
-  const dim3 blk(64 * WM * WN);
-  const int up = act == ACT_RELU2 ? 1 : 2, fn = act == ACT_RELU2 ? BN : BN / 2;
-  const int g1 = (ff + fn - 1) / fn, g2 = (W + BN - 1) / BN;
-#define MOE_FIRST(ACT)                                                                                                     \
-  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, RA, RW, ACT, true>), dim3(max_tiles * g1), blk, 0, st, (const bf16_t*)h,  \
-                     (const bf16_t*)w_gu, rows, tiles, (bf16_t*)y, top, ff, up * ff, W, g1, row_w, limit, spread)
-  if (act == ACT_GLU_CLAMP) MOE_FIRST(ACT_GLU_CLAMP);
-  else if (act == ACT_GLU_SILU) MOE_FIRST(ACT_GLU_SILU);
-  else MOE_FIRST(ACT_RELU2);
-#undef MOE_FIRST
-  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, RA, RW, ACT_NONE, false>), dim3(max_tiles * g2), blk, 0, st, (const bf16_t*)y,
-                     (const bf16_t*)w_down, rows, tiles, (bf16_t*)out, top, W, W, ff, g2, nullptr, 0.f, spread);
-  return (int)hipGetLastError();
-}
-
 // Row tiles of E experts that R pairs fall on at random: a normal count an expert, sum over k of P(count > k BM), the first always
 // (an expert without rows costs its launch slot too)
 double expected_tiles(double R, int E, int BM) {
@@ -280,13 +264,52 @@ double expected_tiles(double R, int E, int BM) {
   for (int k = sure + 1; k * BM < m + 5. * s; ++k) n += 0.5 * (1. + erf((m - k * BM) / (s * 1.4142135623730951)));
   return E * n;
 }
+// The weights of a stage come from HBM, the rows from an L2: a 128-row tile's ring of three stages for the weights and two for the rows
+// (80 KB, still two workgroups a CU) asks for the weights a stage earlier and does not pay for the rows' half of the LDS.  A launch of
+// one round in which CUs hold a second workgroup to wait beside (1.1 to 2.05 workgroups a CU) keeps two stages: there the third cost 1 to
+// 2 % of the launch (43 launches; at the most 8), with fewer workgroups it gained 14 to 21 % where k has more than 16 stages and 4 % below
+// (97), with more 3 to 4 % (164).  Both products, us, two stages / this: 8 experts of 3072 -> 1024 (relu2), 64 rows an expert 68 / 54; 8 of
+// 2048 -> 3072 (gated), 668 278 / 257; 24 of 1536 -> 1536 (gated), 510 290 / 278.  256-row tiles (160 KB) keep two stages: a third gained 2 to 3 %
+// at 510 rows an expert, but lost 1 to 6 % at 384 and up to 5 % above 800.
+bool deep_ring(double tiles, int columns) { return tiles * columns <= 1.1 * 256 || tiles * columns > 2.05 * 256; }
+
+template <int BM, int BN, int WM, int WN, int R, bool DEEP = false>
+int launch_pair(const void* h, const void* w_gu, const void* w_down, const int* rows, const int* tiles, void* y, void* out,
+                int max_tiles, int pairs, int E, int top, int W, int ff, int act, const float* row_w, float limit, int spread,
+                hipStream_t st) {
+  const dim3 blk(64 * WM * WN);
+  const int up = act == ACT_RELU2 ? 1 : 2, fn = act == ACT_RELU2 ? BN : BN / 2;
+  const int g1 = (ff + fn - 1) / fn, g2 = (W + BN - 1) / BN;
+  const double likely = expected_tiles(pairs, E, BM);
+#define MOE_FIRST(ACT, RW)                                                                                                 \
+  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, RW, ACT, true>), dim3(max_tiles * g1), blk, 0, st, (const bf16_t*)h,   \
+                     (const bf16_t*)w_gu, rows, tiles, (bf16_t*)y, top, ff, up * ff, W, g1, row_w, limit, spread)
+#define MOE_ACT(RW)                                           \
+  do {                                                        \
+    if (act == ACT_GLU_CLAMP) MOE_FIRST(ACT_GLU_CLAMP, RW);   \
+    else if (act == ACT_GLU_SILU) MOE_FIRST(ACT_GLU_SILU, RW); \
+    else MOE_FIRST(ACT_RELU2, RW);                            \
+  } while (0)
+#define MOE_SECOND(RW)                                                                                                          \
+  hipLaunchKernelGGL((moe_gemm_kernel<BM, BN, WM, WN, R, RW, ACT_NONE, false>), dim3(max_tiles * g2), blk, 0, st, (const bf16_t*)y, \
+                     (const bf16_t*)w_down, rows, tiles, (bf16_t*)out, top, W, W, ff, g2, nullptr, 0.f, spread)
+  if (DEEP && deep_ring(likely, g1)) MOE_ACT(R + DEEP);
+  else MOE_ACT(R);
+  if (DEEP && deep_ring(likely, g2)) MOE_SECOND(R + DEEP);
+  else MOE_SECOND(R);
+#undef MOE_FIRST
+#undef MOE_ACT
+#undef MOE_SECOND
+  return (int)hipGetLastError();
+}
+
 // us of both products with tiles of BM rows, fitted to 525 points (15 sets of 8 to 64 experts of 512 to 4096 x 512 to 4096, 26 to 1300 rows
-// an expert; half of the estimates are within 5 %): workgroups come in rounds of 512 (two to a CU; 256 of the 256-row tiles), a round
+// an expert, all with equal rings; half of the estimates are within 5 %): workgroups come in rounds of 512 (two to a CU; 256 of the 256-row tiles), a round
 // costs its 64-k stages and its start and end, and a partly filled last round more than its share; the experts' bytes are partly
 // hidden behind that, or (256 rows) bound it from below.
 double tile_us(int BM, double R, int E, int W, int ff, int up) {
   //                              us a stage, a start, both launches, TB/s, whole rounds' part
-  static const double fit[3][5] = {{0.621, 4.35, 5.4, 9.36, 0.266}, {0.96, 7.2, 3.53, 13.3, 0.48}, {1.64, 16.1, 5.69, 4.04, 0.585}};
+  static const double fit[3][5] = {{0.621, 4.35, 5.4, 9.36, 0.266}, {0.991, 7.2, 3.53, 13.3, 0.429}, {1.64, 16.1, 5.69, 4.04, 0.585}};
   const double* p = fit[BM == 64 ? 0 : BM == 128 ? 1 : 2];
   const int BN = BM == 256 ? 256 : 128, slots = BM == 256 ? 256 : 512;
   const double tiles = expected_tiles(R, E, BM);
@@ -338,19 +361,12 @@ int edge_sm_moe_gemm(const void* h, const int* idx, const void* w_gu, const void
   // 3000 476 / 474; with more rows it costs 2 % (7680 tokens of 3, ff 3072: 779 / 798)
   const int spread = R <= E * 512;
   hipLaunchKernelGGL(moe_sort_kernel, dim3(1), dim3(SORT_NT), 0, st, idx, R, E, BM, rows, tiles);
-  // The weights of a stage come from HBM, the rows from an L2: with a ring of three stages for the weights and two for the rows (80 KB,
-  // two workgroups of 128 x 128 a CU, or the LDS' whole 160 KB of one of 256 x 256) the weights are asked for a stage earlier and the
-  // rows' half of the LDS is not paid for.  us, two and two against two and three stages, 128 rows: 8 experts of 2048 -> 4096 (gated),
-  // 100 rows an expert 128 / 111, 250 209 / 191; 32 of 1024 -> 1024, 512 195 / 181; 16 of 1024 -> 1024, 250 77 / 71; 32 of 2048 ->
-  // 3072 (relu2), 60 181 / 170; where the experts' bytes are the bound equal (32 of 2048 -> 2048, 60 174 / 174), at the worst 3 % more
-  // (24 of 1536 -> 1536, 510 205 / 211).  256 rows: relu2, 2048 -> 3072, 510 rows 568 / 545, 720 707 / 673, 1000 916 / 878; gated, 720
-  // 632 / 619 (64 of 1024 -> 1536), 1000 912 / 904, but 375 (spread starts) 406 / 412 and 382 / 400: those keep two and two.
-  if (BM == 256 && spread && act != ACT_RELU2)
-    return launch_pair<256, 256, 2, 4, 2, 2>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  if (BM == 256) return launch_pair<256, 256, 2, 4, 2, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  if (BM == 128) return launch_pair<128, 128, 2, 2, 2, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  if (BM == 64) return launch_pair<64, 128, 1, 4, 3, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
-  return launch_pair<32, 128, 1, 4, 3, 3>(h, w_gu, w_down, rows, tiles, y, out, mt, top, W, ff, act, row_w, limit, spread, st);
+#define MOE_PAIR(...) launch_pair<__VA_ARGS__>(h, w_gu, w_down, rows, tiles, y, out, mt, R, E, top, W, ff, act, row_w, limit, spread, st)
+  if (BM == 256) return MOE_PAIR(256, 256, 2, 4, 2);
+  if (BM == 128) return MOE_PAIR(128, 128, 2, 2, 2, true);
+  if (BM == 64) return MOE_PAIR(64, 128, 1, 4, 3);
+  return MOE_PAIR(32, 128, 1, 4, 3);
+#undef MOE_PAIR
 }
 
 }  // extern "C"

@@ -75,10 +75,13 @@ def test_grouped_experts_against_float64(T, top, E, W, ff, act, every_size):
     (400, 2, 8, 64, 1024, "glu_clamp"),          # 128-row tiles: one k step in the first product
     (400, 2, 8, 1024, 64, "silu_glu"),           # one in the second
     (400, 2, 8, 64, 1024, "relu2"),
-    (3840, 3, 48, 1024, 192, "glu_clamp"),       # three: every stage of the weights' ring once
-    (3840, 3, 48, 192, 1024, "relu2"),
+    (3840, 3, 48, 1024, 192, "glu_clamp"),       # three in the second, every stage of the weights' ring once; the first one's rings are equal
+    (3840, 3, 48, 192, 1024, "relu2"),           # three in the first; equal rings in the second
+    (2400, 2, 8, 1024, 1024, "glu_clamp"),       # unequal, then equal
+    (1600, 2, 16, 512, 1024, "silu_glu"),        # equal, then unequal
+    (4688, 1, 8, 256, 3072, "relu2"),
     (3200, 2, 32, 1024, 1024, "silu_glu"),       # 256-row tiles, gated, spread starts: equal rings
-    (3840, 2, 32, 1024, 1024, "relu2"),          # unequal ones: squared units
+    (3840, 2, 32, 1024, 1024, "relu2"),          # squared units
     (2960, 2, 8, 1536, 1024, "glu_clamp")])      # and starts in step
 def test_rings_of_unequal_depth_against_float64(T, top, E, W, ff, act):
     h, idx, w_gu, w_down, in_w = inputs(T, top, E, W, ff, act, T)
