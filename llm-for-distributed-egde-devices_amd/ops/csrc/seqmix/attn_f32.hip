@@ -318,15 +318,16 @@ __global__ void __launch_bounds__(64 * RW * KS, 2) attn_f32_kernel(F32Attn a) {
 
 extern "C" {
 
-double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis, uintptr_t addresses);
+double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis, long mean, uintptr_t addresses);
 
 // Waves of query rows of a group in the low bits, groups above; 0: the step is not this kernel's.  vis: the most keys that a row sees,
 // mean: as many as a row sees on average.  By estimates: an iteration is one tile of every group, its us were fitted to steps of up to six
-// portions of 16 to 600 tokens behind 0 to 1500 (112 of them, eight head shapes of 32 to 160 numbers), and the kernels before are
-// taken at 0.75 (0.65 of few heads) of theirs, whose chains they overrate; or the form that the caller wants.  Chosen so, 150 other steps took 0.71 of the time before (worst 1.3: 191 rows of 16 heads of 128, 16 / 21); us before / four
-// waves and two groups / two and two / two and four: 16 heads of 64 in 4 groups, 2000 tokens 342 / 102 / 118 / 123, 500 behind 2000 215 /
-// 112 / 85 / 68, 100 8.8 / 10.9 / 9.2 / 9.6, 20 behind 1000 16.7 / 48 / 37 / 30; of 128, 1000 tokens 205 / 87 / 78; 16 of 160 over one
-// latent, 300 tokens 65 / 33 / 26; a group per head of 64, 2000 tokens 1115 / 102 / 117 / 122.
+// portions of 16 to 600 tokens behind 0 to 1500 (112 of them, eight head shapes of 32 to 160 numbers); the kernels before are taken at
+// 0.85 of theirs (edge_sm_attention_us); or the form that the caller wants.  Chosen so, 600 other steps (16 head shapes of 2 to 32 heads, 16 to 6000
+// rows, windows, pooled blocks) took 0.586 of the time before, at the worst 1.03 (two steps of 11.5 us), and 0.576 by the best form of each; at
+// 1.0 of the estimate up to 1.24.  us before / four waves and two groups / two and two / two and four: 16 heads of 64 in 4 groups, 2000
+// tokens 342 / 102 / 118 / 123, 500 behind 2000 215 / 112 / 85 / 68, 100 8.8 / 10.9 / 9.2 / 9.6, 20 behind 1000 16.7 / 48 / 37 / 30; of 128, 1000 tokens
+// 205 / 87 / 78, 191 17.1 / 23.5 / 21.2; 16 of 160 over one latent, 300 tokens 65 / 33 / 26; a group per head of 64, 2000 tokens 1115 / 102 / 117 / 122.
 // Error against 64 bits, relative: 1000 tokens 2.3e-7 before, 1.4e-7 here; 500 behind 2000 3.4e-7, 2.0e-7.
 int edge_sm_attention_f32_plan(int rows, int n, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, int out_ld, bool same, bool rel,
                                bool chunked, bool windowed, long vis, long mean, int want, uintptr_t addresses) {
@@ -336,7 +337,7 @@ int edge_sm_attention_f32_plan(int rows, int n, int H, int G, int D, int Dv, int
   const bool square = D == Dv && (D == 32 || D == 64 || D == 96 || D == 128);
   if (!square && !(same ? D == 160 && Dv == 128 : (D == 64 && Dv == 128) || (D == 128 && Dv == 64))) return 0;
   if (want) return want == 4 + 16 || want == 2 + 16 || (want == 2 + 32 && D <= 64 && Dv <= 64) ? want : 0;
-  double best = (H < 16 ? 0.65 : 0.75) * edge_sm_attention_us(rows, H, G, D, Dv, kld, vld, page, pool, mean, addresses);
+  double best = 0.85 * edge_sm_attention_us(rows, H, G, D, Dv, kld, vld, page, pool, vis, mean, addresses);
   int plan = 0;
   const double w = (D + Dv) / 2, tiles = mean / (double)FK + 0.8, waves = rows * (double)H / 16;
   const long longest = (vis + FK - 1) / FK + (windowed ? 1 : 0);   // (a window begins inside a tile)

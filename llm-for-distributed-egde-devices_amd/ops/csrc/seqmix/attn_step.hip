@@ -449,27 +449,34 @@ int run_beside(const StepArgs& a, const SsdStep& s, int N, int P, hipStream_t st
 // then the sum over key splits.
 constexpr double LAUNCH_US = 4.5, MERGE_US = 4.5;
 
+struct Cost {
+  double chain, work;
+  double us(int ns) const { return LAUNCH_US + (chain > work ? chain : work) + (ns > 1 ? MERGE_US : 0.); }
+};
 // groups workgroups of sh heads, each over its part of vis keys, 128 a round; a round's numbers count as the kernel pads them
-double step_us(int f32, int sh, int D, int Dv, long groups, long vis, int ns) {
+Cost step_cost(int f32, int sh, int D, int Dv, long groups, long vis, int ns) {
   static const double fit[2][2][5] = {{{0.57, 0.0043, 0.0017, 0.21, 0.0037}, {1.8, 0.0063, 0.0071, 0.73, 0.0053}},
                                       {{0.28, 0.0096, 0.002, 0.13, 0.01}, {1.4, 0.014, 0.0068, 0.5, 0.016}}};
   const double* p = fit[f32 ? 1 : 0][sh == 4];
   const int w = D <= 64 && Dv <= 64 ? 128 : D <= 128 && Dv <= 128 ? 256 : D <= 192 && Dv <= 128 ? 320 : 576;
-  const double rounds = (double)(((vis + 127) / 128 + ns - 1) / ns), chain = p[0] + rounds * p[1] * w;
-  const double work = groups / 256.0 * (p[2] * w + rounds * (p[3] + p[4] * w));
-  return LAUNCH_US + (chain > work ? chain : work) + (ns > 1 ? MERGE_US : 0.);
+  const double rounds = (double)(((vis + 127) / 128 + ns - 1) / ns);
+  return {p[0] + rounds * p[1] * w, groups / 256.0 * (p[2] * w + rounds * (p[3] + p[4] * w))};
+}
+double step_us(int f32, int sh, int D, int Dv, long groups, long vis, int ns) {
+  return step_cost(f32, sh, D, Dv, groups, vis, ns).us(ns);
 }
 
-// attn_kernel on fp32 rows, with the heads and splits that its own rules give it
-double attn_kernel_us(int rows, int H, int G, int D, int Dv, long vis) {
+// attn_kernel on fp32 rows, with the heads that its own rule gives it
+Cost attn_kernel_cost(int rows, int H, int G, int D, int Dv, long vis, int ns) {
   const int R = H / G, rm = edge_sm_attention_rmax(rows, H, G, D, Dv);
-  if (rm == 0) return 1e30;
-  const int ns = edge_sm_attention_splits(rows, G, (int)((vis + 255) / 256));
+  if (rm == 0) return {1e30, 1e30};
   const double chunks = (double)(((vis + 255) / 256 + ns - 1) / ns), keys = (double)vis / ns;
-  const double chain = chunks * (2.6 + 0.0099 * D * rm) + keys * (0.0019 + 2.3e-5 * Dv * rm);
-  const double work = rows * (double)G * ((R + rm - 1) / rm) * ns / 256.0 *
-                      (0.99 + keys * 1.5e-4 * (D + Dv) + chunks * 0.0068 * D * rm);
-  return LAUNCH_US + (chain > work ? chain : work) + (ns > 1 ? MERGE_US : 0.);
+  return {chunks * (2.6 + 0.0099 * D * rm) + keys * (0.0019 + 2.3e-5 * Dv * rm),
+          rows * (double)G * ((R + rm - 1) / rm) * ns / 256.0 * (0.99 + keys * 1.5e-4 * (D + Dv) + chunks * 0.0068 * D * rm)};
+}
+double attn_kernel_us(int rows, int H, int G, int D, int Dv, long vis) {
+  const int ns = edge_sm_attention_splits(rows, G, (int)((vis + 255) / 256));
+  return attn_kernel_cost(rows, H, G, D, Dv, vis, ns).us(ns);
 }
 
 }  // namespace
@@ -521,10 +528,18 @@ int edge_sm_attention_step_plan(int rows, int H, int G, int D, int Dv, int kld, 
   return plan;
 }
 
-// the estimate of what edge_sm_attention_step_plan would have an fp32 step run
-double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis, uintptr_t addresses) {
+// us of an fp32 step of portions in attn_kernel or the kernels here, as edge_sm_attention_step_plan deals it: the chain of the row that sees
+// the most keys, the work of rows that see `mean`.  Workgroups of several rounds overlap the two: attn_kernel's shares were fitted to 454
+// steps of 1 to 9 portions (2 to 32 heads of 32 to 160 numbers; rms 12 %; the larger of the two, as above, is up to three times too much).
+double edge_sm_attention_us(int rows, int H, int G, int D, int Dv, int kld, int vld, int page, int pool, long vis, long mean, uintptr_t addresses) {
   const int plan = edge_sm_attention_step_plan(rows, H, G, D, Dv, kld, vld, page, pool, vis, 1, addresses), sh = plan % 8, ns = plan / 8;
-  return plan ? step_us(1, sh, D, Dv, (long)rows * G * ((H / G + sh - 1) / sh) * ns, vis, ns) : attn_kernel_us(rows, H, G, D, Dv, vis);
+  if (plan) {
+    const long groups = (long)rows * G * ((H / G + sh - 1) / sh) * ns;
+    return Cost{step_cost(1, sh, D, Dv, groups, vis, ns).chain, step_cost(1, sh, D, Dv, groups, mean, ns).work}.us(ns);
+  }
+  const int parts = edge_sm_attention_splits(rows, G, (int)((vis + 255) / 256));
+  return 4. + 0.7 * attn_kernel_cost(rows, H, G, D, Dv, vis, parts).chain + 0.4 * attn_kernel_cost(rows, H, G, D, Dv, mean, parts).work +
+         (parts > 1 ? MERGE_US : 0.);
 }
 
 size_t edge_sm_attention_step_floats(int rows, int H, int G, int Dv, int plan) {

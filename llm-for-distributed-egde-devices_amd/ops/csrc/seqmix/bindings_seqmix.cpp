@@ -1860,6 +1860,10 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("sm_attention_ssd", &sm_attention_ssd);
   m.def("sm_embed_bigram", &sm_embed_bigram);
   m.def("sm_embed_bigram_tap4", &sm_embed_bigram_tap4);
+  // which form of attn_f32.hip a step of dense rows takes (0: none; windowed: a window shorter than vis keys), for want the forced one
+  m.def("sm_attention_f32_plan", [](int rows, int n, int H, int G, int D, int Dv, bool same, bool windowed, int64_t vis, int64_t mean, int want) {
+    return edge_sm_attention_f32_plan(rows, n, H, G, D, Dv, G * D, same ? G * D : G * Dv, 64, 0, H * Dv, same, false, false, windowed, vis, mean, want, 0);
+  });
   m.def("sm_canon", &sm_canon);
   m.def("sm_ln_residual_taps", &sm_ln_residual_taps);
   m.def("sm_ln_residual_taps_route", &sm_ln_residual_taps_route);
