@@ -24,7 +24,7 @@ struct F32Attn {
 
 constexpr int FK = 64;                                       // keys of a tile: one page
 
-// LDS of a group of four waves, in floats: the key and the value tile, or at the end its sums
+// LDS of a group of RW waves, in floats: the key and the value tile, or at the end its sums
 template <int D, int Dv, bool KVS, int RW>
 constexpr int group_floats() {
   constexpr int tile = FK * (D + 4) + (KVS ? 0 : FK * Dv), sums = (Dv / 4 + 2) * 64 * RW;

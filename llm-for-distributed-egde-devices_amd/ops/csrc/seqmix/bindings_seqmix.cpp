@@ -427,7 +427,7 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
                         const std::optional<at::Tensor>& slopes, const std::optional<at::Tensor>& sink,
                         int64_t keep_first, const std::optional<at::Tensor>& rel, const std::optional<at::Tensor>& dst,
                         double out_scale, int64_t mean_keys) {
-  // mean_keys: as many as a row sees on average (0: not known; negative: minus the form of attn_f32.hip to take where it can); chunked: `window` is a chunk size (see attn_kernel); keep_first: the first tokens of a sequence that stay visible
+  // mean_keys: as many as a row sees on average (0: not known; negative: minus the form of attn_f32.hip to take, which must fit); chunked: `window` is a chunk size (see attn_kernel); keep_first: the first tokens of a sequence that stay visible
   // behind a sliding window; rel [H, n]: a number per distance added to the scores; dst: where the result goes
   TORCH_CHECK(keep_first >= 0 && (keep_first == 0 || (window > 0 && !chunked)), "keep_first goes with a sliding window");
   chk_i32(tok_seq, "tok_seq");
@@ -504,6 +504,7 @@ at::Tensor sm_attention(const at::Tensor& q, const std::optional<at::Tensor>& ga
                                                 out_ld, same, rel_p != nullptr, chunked || softcap > 0 || slopes_p,
                                                 window > 0 && window < max_keys, vis, mean_keys > 0 ? std::min(mean_keys, vis) : vis, mean_keys < 0 ? (int)-mean_keys : 0,
                                                 addresses | (uintptr_t)out.data_ptr());
+    TORCH_CHECK(form > 0 || mean_keys >= 0, "attn_f32.hip has no such form for this step");
     if (form > 0) {
       check(edge_sm_attention_f32(q.data_ptr(), gate ? gate->data_ptr() : nullptr, gate_ld, kp.data_ptr(), vp.data_ptr(),
                                   PB ? kb->data_ptr<float>() : nullptr, PB ? vb->data_ptr<float>() : nullptr, seq_slot.data_ptr<int>(),
