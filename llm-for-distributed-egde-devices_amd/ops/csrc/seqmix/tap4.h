@@ -68,7 +68,13 @@ __global__ void __launch_bounds__(NT) tap4_kernel(const TI* __restrict__ u, int 
   if (ENDS && t0 < 0) {
     const int s = blockIdx.x, start = seq_start[s], len = seq_len[s], off = seq_off[s];
     TI* const tail = state + (size_t)seq_slot[s] * 3 * C + c;
-    if (len < 1) return;
+    if (len < 1) {                                           // (no rows: of the tail, what lies in front of the sequence is cleared)
+      const float none[CV] = {};
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (start - 3 + k < 0) keep(tail + (size_t)k * C, none);
+      return;
+    }
     float v[9][CV];                                          // the old tail, the first three rows, the last three
 #pragma unroll
     for (int k = 0; k < 3; ++k) {

@@ -45,3 +45,23 @@ def test_tap4(step, dt, op, C, taps, c0):
     # a handful of fp32 products and sums of size <= 20 (2^-24 each), silu's expf, then one rounding to the output type
     tol = 1e-5 + (2.0 ** -8 if dt == torch.bfloat16 else 1e-5) * ref.abs()
     assert ((got.cpu().float() - ref).abs() <= tol).all()
+
+
+@pytest.mark.parametrize("rows", [30, 600])
+@pytest.mark.parametrize("op,dt", [("silu", torch.bfloat16), ("silu", torch.float32), ("plain", torch.float32)])
+def test_portions_without_a_token(op, dt, rows):
+    """They clear what lies in front of their sequence's start, keep the rest of the tail, and change nothing for the others."""
+    dev, C = torch.device("cuda:0"), 1032
+    full, empty = [(0, 4, rows), (4, 0, 2)], [(2, 0, 0), (0, 4, rows), (1, 1, 0), (5, 9, 0), (4, 0, 2), (3, 2, 0)]
+    g = torch.Generator().manual_seed(rows)
+    u, w, b = torch.randn(rows + 2, C, generator=g).to(dt).to(dev), torch.randn(C, 4, generator=g).to(dev), torch.randn(C, generator=g).to(dev)
+    kept = torch.randn(6, 3, C, generator=g).to(dt).to(dev)
+    res = []
+    for seqs in (full, empty):
+        meta, state = S.RaggedMeta.build(seqs, torch.zeros(6, 1, dtype=torch.int32, device=dev), 64, dev), kept.clone()
+        y = S.conv_silu(u, 0, C, w, b, state, meta) if op == "silu" else S.canon_conv(u, w, state, meta, dt)
+        res.append((y, state))
+    assert torch.equal(res[0][0], res[1][0]) and torch.equal(res[0][1][[0, 4]], res[1][1][[0, 4]])
+    state = res[1][1]
+    assert not state[2].any() and not state[1, :2].any() and not state[3, 0].any()
+    assert torch.equal(state[5], kept[5]) and torch.equal(state[1, 2], kept[1, 2]) and torch.equal(state[3, 1:], kept[3, 1:])
