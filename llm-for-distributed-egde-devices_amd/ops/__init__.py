@@ -472,7 +472,8 @@ def rows16_ok(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor
 
 def rows16(x, packed, bias, N: int, act: Optional[str] = None, add: Optional[torch.Tensor] = None):
     """``gemm_rows16.hip`` for a call that ``rows16_ok`` lets pass; ``act``: None, "silu_glu", "gelu_tanh" or "gelu"."""
-    joins = add is not None and add.dtype == x.dtype and add.shape == x.shape[:-1] + (N,) and add.is_contiguous() and raw_call(add)
+    joins = add is not None and add.dtype == x.dtype and add.device == x.device and add.shape == x.shape[:-1] + (N,) and \
+        add.is_contiguous() and raw_call(add)
     y = ext().gemm_rows16(x, packed, bias, N, _GEMV_EPI[act], add if joins else None)
     return y if add is None or joins else y + add
 

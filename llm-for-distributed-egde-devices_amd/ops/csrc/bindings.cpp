@@ -199,6 +199,7 @@ int need16(const at::Tensor& t, const char* name, bool contiguous = true) {
 void need_same(const at::Tensor& t, const at::Tensor& like, const char* name) {
   TORCH_CHECK(t.scalar_type() == like.scalar_type(), name, " has dtype ", t.scalar_type(), ", expected ",
               like.scalar_type());
+  TORCH_CHECK(t.device() == like.device(), name, " is on ", t.device(), ", expected ", like.device());
 }
 
 // ---------------------------------------------------------------------------------- norms
