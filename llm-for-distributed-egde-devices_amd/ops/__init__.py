@@ -602,7 +602,9 @@ def linear_bf16(x, weight, bias=None, glu: bool = False, act: Optional[str] = No
     if mode == 1 or (mode == 2 and act in (None, "silu_glu")):
         wp = packed if packed is not None else pack_bf16_weight(weight)
         if mode == 1:
-            return ext().gemv_bf16(x, wp, bias, weight.shape[0], _GEMV_EPI[act], add)
+            joins = add is None or (add.is_contiguous() and raw_call(add))       # (strides, gradients and transforms: an op of its own)
+            y = ext().gemv_bf16(x, wp, bias, weight.shape[0], _GEMV_EPI[act], add if joins else None)
+            return y if joins else y + add
         y = ext().gemm_bf16_ring(x, wp, bias, weight.shape[0], 1 if glu else 0, 0)
         return y if add is None else y + add
     if mode == 2:           # GELU MLPs: ring GEMM, then the activation kernel

@@ -829,7 +829,7 @@ at::Tensor gemv_bf16(const at::Tensor& x, const at::Tensor& wp, const std::optio
   auto out = at::empty(os, epi == 7 ? x.options().dtype(at::kFloat) : x.options());
   if (addend) {
     need_same(*addend, x, "addend");
-    TORCH_CHECK(epi == 0 && addend->numel() == M * N, "addend: plain output only, M * N elements");
+    TORCH_CHECK(epi == 0 && addend->numel() == M * N && addend->is_contiguous(), "addend: plain output only, M * N elements, dense");
   }
   check(edge_gemv_bf16(x.data_ptr(), wp.data_ptr(), bias ? bias->data_ptr() : nullptr, out.data_ptr(), (int)M, (int)N,
                        (int)K, (int)epi, stream(), addend ? addend->data_ptr() : nullptr, h16),
@@ -940,7 +940,7 @@ at::Tensor gemm_rows16(const at::Tensor& x, const at::Tensor& wp, const std::opt
   if (bias) { need_same(*bias, x, "bias"); TORCH_CHECK(bias->numel() == N); }
   if (addend) {
     need_same(*addend, x, "addend");
-    TORCH_CHECK(epi == 0 && addend->numel() == M * N, "addend: plain output only, M * N elements");
+    TORCH_CHECK(epi == 0 && addend->numel() == M * N && addend->is_contiguous(), "addend: plain output only, M * N elements, dense");
   }
   TORCH_CHECK(S == 1 || (S > 1 && epi == 0 && !h16 && !addend), "gemm_rows16: slices of the plain bf16 product");
   auto os = x.sizes().vec();
