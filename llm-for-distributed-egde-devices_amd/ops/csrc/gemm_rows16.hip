@@ -55,6 +55,30 @@ __device__ __forceinline__ void glds16(const void* g, void* lds_base) {
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
   return (uint32_t)(uintptr_t)((__attribute__((address_space(3))) const void*)p);
 }
+// A k-pair's rows from the LDS, MB 16-row blocks and two halves, and the wait for them in one block: between a read and its wait the
+// compiler would take the registers as written.  (Plain loads would wait for the LDS-DMA in flight.)
+template <int MB>
+__device__ __forceinline__ void read_rows(uint32_t b0, uint32_t b1, v4i (&a)[2][MB]) {
+  static_assert(MB >= 2 && MB <= 4, "17 to 64 rows");
+  if constexpr (MB == 2)
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\t"
+                 "ds_read_b128 %2, %4 offset:2048\n\tds_read_b128 %3, %5 offset:2048\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[1][0]), "=&v"(a[0][1]), "=&v"(a[1][1]) : "v"(b0), "v"(b1) : "memory");
+  else if constexpr (MB == 3)
+    asm volatile("ds_read_b128 %0, %6\n\tds_read_b128 %1, %7\n\t"
+                 "ds_read_b128 %2, %6 offset:2048\n\tds_read_b128 %3, %7 offset:2048\n\t"
+                 "ds_read_b128 %4, %6 offset:4096\n\tds_read_b128 %5, %7 offset:4096\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[1][0]), "=&v"(a[0][1]), "=&v"(a[1][1]), "=&v"(a[0][2]), "=&v"(a[1][2])
+                 : "v"(b0), "v"(b1) : "memory");
+  else
+    asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\t"
+                 "ds_read_b128 %2, %8 offset:2048\n\tds_read_b128 %3, %9 offset:2048\n\t"
+                 "ds_read_b128 %4, %8 offset:4096\n\tds_read_b128 %5, %9 offset:4096\n\t"
+                 "ds_read_b128 %6, %8 offset:6144\n\tds_read_b128 %7, %9 offset:6144\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(a[0][0]), "=&v"(a[1][0]), "=&v"(a[0][1]), "=&v"(a[1][1]), "=&v"(a[0][2]), "=&v"(a[1][2]), "=&v"(a[0][3]),
+                   "=&v"(a[1][3])
+                 : "v"(b0), "v"(b1) : "memory");
+}
 // tiles whose sums meet at a time: at most 128 KiB of them, gate and up tiles together
 constexpr int sums_together(int MB, int NT, bool glu) {
   int c = NT;
@@ -113,17 +137,7 @@ __global__ void __launch_bounds__(GR_NW * 64, 2) gemm_rows16_kernel(RowsArgs p) 
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     v4i a[2][MB];
     const uint32_t b0 = fr + (u & 1) * (XW / 2), b1 = b0 ^ 64;
-#pragma unroll
-    for (int m = 0; m < MB; ++m) {
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(a[0][m]) : "v"(b0), "n"(m * 2048));
-      asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(a[1][m]) : "v"(b1), "n"(m * 2048));
-    }
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");       // (read: the next load may overwrite them)
-#pragma unroll
-    for (int m = 0; m < MB; ++m) {
-      asm volatile("" : "+v"(a[0][m]));
-      asm volatile("" : "+v"(a[1][m]));
-    }
+    read_rows<MB>(b0, b1, a);                                // (all there: the next load may overwrite them)
 #pragma unroll
     for (int s = 0; s < 2; ++s)
 #pragma unroll
