@@ -403,8 +403,10 @@ __global__ void __launch_bounds__(256 * KS) delta_chunk_scan_kernel(DeltaScratch
                                                                    int PP) {
   constexpr int NP = 64 * KS, PC = 4 * CS;
   __shared__ double S_s[NP][PC], W_s[CL][PC], P_s[KS > 1 ? KS : 1][KS > 1 ? CL : 1][PC];
-  // the workgroups of a head share an L2: blocks are dealt to the eight dies in turn
-  const int nct = PP / PC, unit = ((int)blockIdx.x & 7) + 8 * (((int)blockIdx.x >> 3) / nct), ct = ((int)blockIdx.x >> 3) % nct;
+  // the workgroups of a head share an L2: blocks are dealt to the eight dies in turn, every other eight heads half a round further (of four
+  // heads, long and short sequences in turn fell on four dies each: 16 sequences of 35 to 863, 64 x 128 states, 140 / 125 us)
+  const int nct = PP / PC, oct = ((int)blockIdx.x >> 3) / nct, ct = ((int)blockIdx.x >> 3) % nct;
+  const int unit = (((int)blockIdx.x + 4 * oct) & 7) + 8 * oct;
   if (unit >= n * H) return;
   const int p0 = ct * PC, h = unit % H, s = unit / H, tid = threadIdx.x;
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane & 3, x = lane >> 2;
@@ -733,22 +735,24 @@ int edge_sm_delta_chunked(const float* prep, int prep_ld, const void* qkv, int C
     } else if (vec) SM_DSOLVE(true, false);
     else SM_DSOLVE(false, false);
 #undef SM_DSOLVE
-    // columns a workgroup: as few fours as 256 workgroups, one a CU, leave; more share the operands' reads.  us for all three kernels,
-    // 4 / 8 / 16 columns: 16 heads of 64 x 64, 4096 tokens 198 / 211 / 283, 32 heads, four sequences of 2048 733 / 602 / 543; 16 of 128 x 128,
-    // 512 tokens 105 / 86 / 97, six sequences of 512 424 / 297 / 271
+    // columns a workgroup: as few fours as 256 workgroups, one a CU, leave; more share the operands' reads.  States of up to 64 rows stop at
+    // 8: their 16 columns (four waves) step no quicker than the 16x16x4 form did, and behind uneven portions, whose longest is the launch,
+    // cost up to 12 % more than 8.  us for all three kernels, 4 / 8 / 16 columns: 16 heads of 64 x 64, 4096 tokens 198 / 211 / 283, 12 heads, eight
+    // sequences of 24 to 1344 189 / 174 / 194, 32 heads, four of 2048 502 / 502 / 507; 16 of 128 x 128, 512 tokens 105 / 86 / 97, two sequences of 1386
+    // 401 / 296 / 277, six of 512 230 / 231 / 231.  101 steps of up to 40 sequences: 0.953 of that form's time, at the worst 1.05
+    // (eight sequences of 83 to 1325, 4 heads of 64 x 128, 151 / 159).
 #define SM_DSCAN(KS, CS)                                                                                                        \
   hipLaunchKernelGGL((delta_chunk_scan_kernel<KS, CS>), dim3((H * n + 7) / 8 * 8 * (PP / (4 * CS))), dim3(256 * KS), 0, st, sc, \
                      state, seq_slot, seq_start, seq_len, dp, n, H, N, P, PP)
-#define SM_DCOLS(KS)                                          \
-  if (H * n * (PP / 4) <= 256) SM_DSCAN(KS, 1);               \
-  else if (H * n * (PP / 8) <= 256) SM_DSCAN(KS, 2);          \
-  else SM_DSCAN(KS, 4)
-    if (NP == 64) { SM_DCOLS(1); }
-    else if (NP == 128) { SM_DCOLS(2); }
+    const int fours = H * n * (PP / 4) <= 256 ? 1 : H * n * (PP / 8) <= 256 ? 2 : 4;
+    if (NP == 64 && fours == 1) SM_DSCAN(1, 1);
+    else if (NP == 64) SM_DSCAN(1, 2);
+    else if (NP == 128 && fours == 1) SM_DSCAN(2, 1);
+    else if (NP == 128 && fours == 2) SM_DSCAN(2, 2);
+    else if (NP == 128) SM_DSCAN(2, 4);
     else
       hipLaunchKernelGGL(delta_chunk_scan_wide_kernel, dim3(PP / 16, H, n), dim3(1024), 0, st, sc, state, seq_slot, seq_start, seq_len, dp, H, N,
                          P, PP);
-#undef SM_DCOLS
 #undef SM_DSCAN
     hipLaunchKernelGGL((delta_chunk_out_kernel<4>), dim3(mc * ntp, n, H), dim3(NT), 0, st, sc, seq_len, seq_off, y, dp, H, NP, P,
                        PP, ntp);

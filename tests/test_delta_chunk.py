@@ -70,7 +70,7 @@ def test_chunks_against_the_recurrence(lens, starts, H, G, N, P, channel, decay,
 @gpu
 @pytest.mark.parametrize("n,H,G,N,P", [
     (1, 16, 16, 64, 64), (1, 12, 4, 72, 80), (2, 16, 8, 33, 64), (2, 9, 3, 128, 112),    # 4 and 8 columns a workgroup
-    (5, 16, 8, 20, 80), (4, 11, 1, 100, 96), (9, 7, 7, 64, 16), (1, 1, 1, 64, 1)])       # 16; heads that do not fill the eight dies
+    (5, 16, 8, 20, 80), (4, 11, 1, 100, 96), (9, 7, 7, 64, 16), (1, 1, 1, 64, 1)])       # 8, 16, 4; heads that do not fill the eight dies
 def test_chunks_at_every_split_of_the_columns(n, H, G, N, P, monkeypatch):
     prep, qkv, state, meta = inputs((129, 64, 30, 70, 1, 65, 2, 128, 3)[:n], (5, 0, 1, 0, 3, 0, 0, 2, 1)[:n], H, G, N, P, True, "usual", seed=n)
     before = state.double().cpu()
