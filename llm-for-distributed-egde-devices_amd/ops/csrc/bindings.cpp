@@ -1495,9 +1495,13 @@ at::Tensor sample(const at::Tensor& logits, const std::optional<at::Tensor>& see
   auto out = at::empty({B}, logits.options().dtype(at::kLong));
   auto ws = at::empty({(int64_t)edge_sample_workspace((int)B, (int)V)}, logits.options().dtype(at::kByte));
   const double inv_t = temperature > 0 ? 1.0 / temperature : 1.0;
-  const int rc = edge_sample(logits.data_ptr(), dt, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V,
-                             (float)temperature, (float)inv_t, (float)penalty, (int)top_k, (float)top_p, do_sample,
-                             rng.data_ptr<int>(), out.data_ptr<int64_t>(), ws.data_ptr(), stream());
+  auto run = [&](const at::Tensor& lg, int type) {
+    return edge_sample(lg.data_ptr(), type, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V, (float)temperature, (float)inv_t,
+                       (float)penalty, (int)top_k, (float)top_p, do_sample, rng.data_ptr<int>(), out.data_ptr<int64_t>(), ws.data_ptr(),
+                       stream());
+  };
+  int rc = run(logits, dt);
+  if (rc == -6) rc = run(logits.to(at::kFloat), 0);
   if (rc == -5) return at::Tensor();
   check(rc, "sample");
   return out;
@@ -1619,12 +1623,15 @@ at::Tensor sample_advance(const at::Tensor& logits, const std::optional<at::Tens
   auto nxt = at::empty({B}, logits.options().dtype(at::kLong));
   auto ws = at::empty({(int64_t)edge_sample_workspace((int)B, (int)V)}, logits.options().dtype(at::kByte));
   const double inv_t = temperature > 0 ? 1.0 / temperature : 1.0;
-  const int rc = edge_sample_advance(logits.data_ptr(), dt, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V,
-                                     (float)temperature, (float)inv_t, (float)penalty, (int)top_k, (float)top_p,
-                                     do_sample, rng.data_ptr<int>(), nxt.data_ptr<int64_t>(), ws.data_ptr(),
-                                     tok.data_ptr<int64_t>(), out.data_ptr<int64_t>(), out.stride(0), (int)out.size(1),
-                                     step.data_ptr<int64_t>(), pos.data_ptr<int>(), seq_lens.data_ptr<int>(),
-                                     ctr.data_ptr<int>(), stream());
+  auto run = [&](const at::Tensor& lg, int type) {
+    return edge_sample_advance(lg.data_ptr(), type, seen ? seen->data_ptr<uint8_t>() : nullptr, (int)B, (int)V, (float)temperature,
+                               (float)inv_t, (float)penalty, (int)top_k, (float)top_p, do_sample, rng.data_ptr<int>(),
+                               nxt.data_ptr<int64_t>(), ws.data_ptr(), tok.data_ptr<int64_t>(), out.data_ptr<int64_t>(), out.stride(0),
+                               (int)out.size(1), step.data_ptr<int64_t>(), pos.data_ptr<int>(), seq_lens.data_ptr<int>(),
+                               ctr.data_ptr<int>(), stream());
+  };
+  int rc = run(logits, dt);
+  if (rc == -6) rc = run(logits.to(at::kFloat), 0);
   if (rc == -5) return at::Tensor();
   check(rc, "sample_advance");
   return nxt;

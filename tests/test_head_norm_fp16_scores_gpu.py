@@ -31,6 +31,33 @@ def test_fp16_scores_draw_what_their_fp32_values_do(cuda, B, V, top_k, top_p, do
     assert torch.equal(a, b) and torch.equal(seen, seen2)      # widening is exact
 
 
+@pytest.mark.parametrize("top_k", [128, 129, 1000])            # the last two: widened in front of a row's many passes
+def test_fp16_scores_of_a_decode_step(cuda, top_k):
+    """The sampler with the step's bookkeeping behind it, eager and in a graph."""
+    from edgellm import ops
+    B, V = 3, 4096
+    x = (torch.randn(B, V, generator=torch.Generator().manual_seed(top_k)) * 4).half().cuda()
+
+    def state():
+        z = lambda n, t: torch.zeros(n, dtype=t, device="cuda")
+        return dict(seen=z((B, V), torch.uint8), rng=torch.tensor([5, 0], dtype=torch.int32, device="cuda"), tok=z(B, torch.long),
+                    out=z((B, 8), torch.long), step=z(1, torch.long), pos=z(B, torch.int32), lens=z(B, torch.int32), ctr=z(1, torch.int32))
+
+    def step(s, lg):
+        return ops.sample_advance(lg, s["seen"], 0.8, top_k, 0.95, 1.1, s["rng"], s["tok"], s["out"], s["step"], s["pos"], s["lens"], s["ctr"])
+    a, b, c, wide = state(), state(), state(), x.float()
+    for _ in range(4):
+        assert torch.equal(step(a, x), step(b, wide))
+    g = torch.cuda.CUDAGraph()
+    step(state(), x)
+    with torch.cuda.graph(g):
+        step(c, x)
+    for _ in range(4):
+        g.replay()
+    for k in a:
+        assert torch.equal(a[k], b[k]) and torch.equal(a[k], c[k]), k
+
+
 @pytest.mark.parametrize("family,dtype", [("gpt_neox", torch.float16), ("phi", torch.bfloat16)])
 @pytest.mark.parametrize("rows", [1, 4])
 def test_head_takes_both_branches(cuda, family, dtype, rows, monkeypatch):
