@@ -241,7 +241,8 @@ class Linear(nn.Module):
             ops.rows16_ok(x, self.weight, self.bias, glu, split)
 
     def rows16(self, x, act: Optional[str] = None, add=None):
-        """17 to 64 rows in ``gemm_rows16.hip`` (``act``: the activation of the output), or None where that does not run."""
+        """17 to 64 rows in ``gemm_rows16.hip`` (``act``: the activation of the output), or None where that does not run.  Reads the packed
+        copy that the decode GEMVs keep; a layer without one yet forms it here (as many bytes as the weight)."""
         if not self.rows16_ok(x, act == "silu_glu"):
             return None
         return ops.rows16(x, self.packed_weight(), self.bias, self.out_features, act,
