@@ -47,7 +47,7 @@ __global__ void prev_token_kernel(const int64_t* __restrict__ ids, int64_t* __re
                                   const int* __restrict__ seq_slot, const int* __restrict__ seq_len,
                                   const int* __restrict__ seq_off, int n) {
   const int s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < n) prev_tok[seq_slot[s]] = ids[seq_off[s] + seq_len[s] - 1];
+  if (s < n && seq_len[s] > 0) prev_tok[seq_slot[s]] = ids[seq_off[s] + seq_len[s] - 1];
 }
 
 // A step in which every sequence brings one token: the embedding, the slot's previous token and the first layer's input convolution

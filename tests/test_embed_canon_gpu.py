@@ -32,3 +32,14 @@ def test_one_launch(cuda, dt, W, taps, seqs, monkeypatch):
     want = S.embedding_bigram(ids, meta, table, big, p2, B, 3, 11)
     assert torch.equal(x, want) and torch.equal(prev, p2)
     assert torch.equal(h, S.canon_conv(want, w, s2, meta, dt)) and torch.equal(state.nan_to_num(7.0), s2.nan_to_num(7.0))
+
+
+def test_a_portion_without_a_token_keeps_its_previous_one(cuda):
+    """It has no last token to read, in front of the step's first or another sequence's."""
+    g, V, B, W = torch.Generator().manual_seed(0), 33, 13, 64
+    seqs = [(2, 5, 0), (0, 3, 4), (3, 9, 0), (1, 0, 2)]
+    meta = S.RaggedMeta.build(seqs, torch.zeros(4, 1, dtype=torch.int32, device="cuda"), 64, torch.device("cuda"))
+    table, big = (torch.randn(n, W, generator=g).cuda() for n in (V, B + 1))
+    prev, ids = torch.tensor([7, 8, 9, 10]).cuda(), torch.randint(0, V, (6,), generator=g).cuda()
+    S.embedding_bigram(ids, meta, table, big, prev, B, 3, 11)
+    assert prev.tolist() == [int(ids[3]), int(ids[5]), 9, 10]
